@@ -578,13 +578,7 @@ int fsvd_lowrank_expand_heads_multi(const fsvd_expand_desc* desc, int n, const v
                       d.dst_rows, B, M, d.heads, Dh, d.R, dtype};
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (expand_multi_apply(a, n)) {
-    // the single-expansion checks (head_dim, alignment) hold for every descriptor: expand_tiles_apply covers strides
-    // and rank, the pointers are checked here
-    bool ok = true;
-    for (int k = 0; k < n; ++k) ok = ok && ((reinterpret_cast<uintptr_t>(a[k].p) | reinterpret_cast<uintptr_t>(a[k].u)) & 15) == 0 && (a[k].sp_h % 8) == 0;
-    if (ok) return launch_expand_multi(a, n, st);
-  }
+  if (expand_multi_apply(a, n)) return launch_expand_multi(a, n, st);
   for (int k = 0; k < n; ++k) {
     const int rc = launch_expand(a[k], st);
     if (rc != kOk) return rc;

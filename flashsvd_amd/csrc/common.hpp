@@ -155,6 +155,31 @@ __device__ __forceinline__ float wave_max(float v) {
   return fmaxf(fmaxf(a, b), fmaxf(c, d));
 }
 
+// Eight consecutive 16-bit elements at any element's address as one 16-byte load (the hardware takes unaligned ones).
+typedef uint32_t u32x4_any_t __attribute__((ext_vector_type(4), aligned(2)));
+// The same for a piece that may reach past the end of its row: `left` elements of the row from `p` on, zero past them
+// (none at all for left <= 0).  Nothing outside the row is read: the load takes the row's last eight elements instead and
+// the piece is shifted out of them; a row of fewer than eight elements (K) is read element by element.
+__device__ __forceinline__ u32x4_t load_masked_piece(const uint16_t* p, int left, int K) {
+  if (K < 8) {
+    uint32_t w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int e = 0; e < 7; ++e)
+      if (e < left) w[e >> 1] |= (uint32_t)p[e] << (16 * (e & 1));
+    return u32x4_t{w[0], w[1], w[2], w[3]};
+  }
+  const int back = max(8 - left, 0);             // elements the load starts before the piece
+  const u32x4_t q = *reinterpret_cast<const u32x4_any_t*>(p - back);
+  const int ws = back >> 1;
+  const uint32_t z = 0u;
+  uint32_t w[5] = {ws == 0 ? q.x : ws == 1 ? q.y : ws == 2 ? q.z : ws == 3 ? q.w : z, ws == 0 ? q.y : ws == 1 ? q.z : ws == 2 ? q.w : z,
+                   ws == 0 ? q.z : ws == 1 ? q.w : z, ws == 0 ? q.w : z, z};
+  const bool odd = back & 1;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = odd ? (w[i] >> 16) | (w[i + 1] << 16) : w[i];
+  return u32x4_t{w[0], w[1], w[2], w[3]};
+}
+
 // Cross-workgroup hand-off without L2 write-back/invalidate fences: producers use write-through
 // (agent-scope) stores, wait until the memory system has acknowledged them, then signal through an
 // agent-scope atomic; consumers read with agent-scope loads.  A workgroup-scope release fence does

@@ -178,6 +178,8 @@ bool gemm_tiles_apply(const MfmaArgs& a);                                   // m
 int launch_gemm_tiles(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
 bool gemm_rows_apply(const MfmaArgs& a);                                    // mfma_gemm.hip: 5..127 rows, K split
 int launch_gemm_rows(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
+bool gemm_ragged_apply(const MfmaArgs& a);                                  // mfma_gemm.hip: any K, rows that start anywhere
+int launch_gemm_ragged(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
 
 int launch_linear(const LinearArgs& a, int cfg, hipStream_t st);
 // matrix-core path for 5+ rows (mfma_gemv.hip); launch_linear / launch_swiglu route to it when cfg == 0

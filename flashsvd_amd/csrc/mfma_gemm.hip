@@ -13,6 +13,7 @@
 // head expansion of the prompt pass (RoPE, store into the query buffer or the cache rows).  Few tiles or a very long K:
 // K split over workgroups, partial tiles added in a fixed order by the last arrival.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -44,11 +45,17 @@ struct ExpandEpi {
 // gate partners through LDS once, before the SwiGLU epilogue.  8, single matrix: waves 4-7 take the second half of the
 // k slices of every step and hand their sums to waves 0-3 through LDS at the end.
 // PF > 0: register sets in flight; PF < 0: loads straight into LDS with -PF stages.
-template <int DT, bool DUAL, int WTM, int WT, int PF, bool EXPAND, int BK, int NW>
+// RAG: rows that start anywhere and any K, not only whole steps of aligned rows -- the ranks that a parameter ratio
+// leaves (1492, 1638, ...).  The pieces of a row are still one 16-byte load each: the hardware takes them at any element's
+// address.  The K steps that are whole run as they do otherwise; what is left of K is one more step behind the loop, its
+// pieces masked to the row (zero past its end), so nothing is read outside the operands.
+template <int DT, bool DUAL, int WTM, int WT, int PF, bool EXPAND, int BK, int NW, bool RAG = false>
 __device__ __forceinline__ void gemm_tiles_body(const MfmaArgs& a, const ExpandEpi& ep, const int tile_m, const int tile_n) {
   typedef E16<DT> E;
   typedef typename E::frag_t frag_t;
   static_assert(!EXPAND || (!DUAL && WT == 4), "head expansion takes whole 128-wide heads");
+  static_assert(!RAG || PF > 0, "ragged rows are staged through registers");
+  typedef typename std::conditional<RAG, u32x4_any_t, u32x4_t>::type piece_t;
   static_assert(NW == 4 || (NW == 8 && DUAL && WT == 4 && WTM == 4) || (NW == 8 && !DUAL && !EXPAND && BK >= 64),
                 "eight waves: the split form of the 128 x 128 pair tile, or two halves of every K step of a single matrix");
   constexpr int kGT = NW * 64;
@@ -79,7 +86,8 @@ __device__ __forceinline__ void gemm_tiles_body(const MfmaArgs& a, const ExpandE
   const int ksteps_all = a.K / BK;
   const int kper = (ksteps_all + (int)gridDim.z - 1) / (int)gridDim.z;
   const int kbeg = min((int)blockIdx.z * kper, ksteps_all);
-  const int ksteps = max(1, min(kper, ksteps_all - kbeg));   // a share past the end re-reads the last step and adds zero
+  // a share past the end re-reads the last step and adds zero (ragged: it walks no step)
+  const int ksteps = max(RAG ? 0 : 1, min(kper, ksteps_all - kbeg));
   const bool kdead = kbeg >= ksteps_all;
 
   // global -> register staging: a tile row is CPR 16-byte pieces; NP pieces per thread and operand
@@ -121,11 +129,11 @@ __device__ __forceinline__ void gemm_tiles_body(const MfmaArgs& a, const ExpandE
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
 #pragma unroll
-      for (int j = 0; j < NPX; ++j) rx[set][m][j] = *reinterpret_cast<const u32x4_t*>(gx[m][j] + k);
+      for (int j = 0; j < NPX; ++j) rx[set][m][j] = *reinterpret_cast<const piece_t*>(gx[m][j] + k);
 #pragma unroll
       // plain loads: the other row tiles resident on this XCD read the same W tile out of its L2 (a streaming hint
       // gives the lines up early: 10..25 % slower at 512 rows and more)
-      for (int j = 0; j < NP; ++j) rw[set][m][j] = *reinterpret_cast<const u32x4_t*>(gw[m][j] + k);
+      for (int j = 0; j < NP; ++j) rw[set][m][j] = *reinterpret_cast<const piece_t*>(gw[m][j] + k);
     }
   };
   auto store_lds = [&](int set, int stage) {
@@ -173,7 +181,7 @@ __device__ __forceinline__ void gemm_tiles_body(const MfmaArgs& a, const ExpandE
 #pragma unroll
     for (int s0 = 0; s0 < NS - 1; ++s0) issue_direct(s0, s0);
     __builtin_amdgcn_s_waitcnt(kWaitOpen);
-  } else {
+  } else if (!RAG || ksteps > 0) {
 #pragma unroll
     for (int u = 0; u < PFR; ++u) load_regs(u, u);
     store_lds(0, 0);
@@ -243,6 +251,39 @@ __device__ __forceinline__ void gemm_tiles_body(const MfmaArgs& a, const ExpandE
     }
   }
 
+  // what is left of K behind the whole steps, taken by the last share
+  if (RAG && a.K % BK != 0 && blockIdx.z == gridDim.z - 1) {
+    const int k = ksteps_all * BK, left = a.K - k - g_chunk * 8;     // elements of the row from this thread's piece on
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+#pragma unroll
+      for (int j = 0; j < NPX; ++j) rx[0][m][j] = load_masked_piece(gx[m][j] + k, left, a.K);
+#pragma unroll
+      for (int j = 0; j < NP; ++j) rw[0][m][j] = load_masked_piece(gw[m][j] + k, left, a.K);
+    }
+    store_lds(0, 0);                    // the loop ended with a barrier (or did not run): nobody reads the stages
+    __syncthreads();
+    constexpr int Q = KHALF ? BK / 64 : (BK / 32) * NMA;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int kk = KHALF ? mat * (BK / 64) + q : q / NMA, m = SPLIT ? mat : (KHALF ? 0 : q % NMA);
+      const int fcol = (((kk * 4) ^ fr_hi) + fr_lo) * 8;
+      frag_t fx[WTM], fw[WT];
+#pragma unroll
+      for (int i = 0; i < WTM; ++i) fx[i] = *reinterpret_cast<const frag_t*>(lds + m * kTileX + (wm * 16 * WTM + i * 16 + lr) * kGLd + fcol);
+#pragma unroll
+      for (int i = 0; i < WT; ++i) {
+        const int wrow = EXPAND ? (i < 2 ? wn * 32 + i * 16 : 64 + wn * 32 + (i - 2) * 16) : wn * 16 * WT + i * 16;
+        fw[i] = *reinterpret_cast<const frag_t*>(lds + NM * kTileX + m * kTileW + (wrow + lr) * kGLd + fcol);
+      }
+#pragma unroll
+      for (int i = 0; i < WTM; ++i)
+#pragma unroll
+        for (int j = 0; j < WT; ++j) acc[q % NMA][i][j] = E::mfma(fw[j], fx[i], acc[q % NMA][i][j]);
+    }
+    __syncthreads();
+  }
+
   if (KHALF) {
     gm_f32x4_t* ex = reinterpret_cast<gm_f32x4_t*>(gm_smem);     // [WTM*WT][256] 16-byte words, inside the stages
     __syncthreads();                                             // every wave has finished reading the last stage
@@ -278,7 +319,7 @@ __device__ __forceinline__ void gemm_tiles_body(const MfmaArgs& a, const ExpandE
 #pragma unroll
         for (int j = 0; j < WT; ++j) {
           if (!writer) break;
-          const gm_f32x4_t v = kdead ? gm_f32x4_t{0.f, 0.f, 0.f, 0.f} : acc[m][i][j];
+          const gm_f32x4_t v = !RAG && kdead ? gm_f32x4_t{0.f, 0.f, 0.f, 0.f} : acc[m][i][j];
           unsigned long long* dst = reinterpret_cast<unsigned long long*>(mine + ((m * WTM + i) * WT + j) * kGT + tid);
           __hip_atomic_store(dst, ((unsigned long long)__float_as_uint(v[1]) << 32) | __float_as_uint(v[0]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           __hip_atomic_store(dst + 1, ((unsigned long long)__float_as_uint(v[3]) << 32) | __float_as_uint(v[2]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -472,28 +513,30 @@ __device__ __forceinline__ void tile_of_workgroup(int NT, int MT, int& tile_m, i
   tile_m = band * 8 + tb - tile_n * bh;
 }
 
-template <int DT, bool DUAL, int WTM, int WT, int PF, bool EXPAND, int BK, int NW>
+template <int DT, bool DUAL, int WTM, int WT, int PF, bool EXPAND, int BK, int NW, bool RAG = false>
 __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void gemm_tiles_kernel(MfmaArgs a, ExpandEpi ep) {
   int tile_m, tile_n;
   tile_of_workgroup(gridDim.x, gridDim.y, tile_m, tile_n);
-  gemm_tiles_body<DT, DUAL, WTM, WT, PF, EXPAND, BK, NW>(a, ep, tile_m, tile_n);
+  gemm_tiles_body<DT, DUAL, WTM, WT, PF, EXPAND, BK, NW, RAG>(a, ep, tile_m, tile_n);
 }
 
 // up to three head expansions of the same token rows (q, k, v of a prompt pass) in one launch: column tile = one head
 // of one of them.  At 512 rows a single expansion has one workgroup per compute unit and waits on its own loads; the
 // three together give every compute unit three.
 struct ExpandBatch { MfmaArgs a[3]; ExpandEpi ep[3]; int first_head[4]; };
-template <int DT, int WTM>
+template <int DT, int WTM, bool RAG = false>
 __global__ __launch_bounds__(kGT4, 2) void expand_multi_kernel(ExpandBatch eb) {
   int tile_m, tile_n;
   tile_of_workgroup(gridDim.x, gridDim.y, tile_m, tile_n);
   const int k = tile_n >= eb.first_head[2] ? 2 : (tile_n >= eb.first_head[1] ? 1 : 0);
-  gemm_tiles_body<DT, false, WTM, 4, 2, true, kGBK, 4>(eb.a[k], eb.ep[k], tile_m, tile_n - eb.first_head[k]);
+  gemm_tiles_body<DT, false, WTM, 4, 2, true, kGBK, 4, RAG>(eb.a[k], eb.ep[k], tile_m, tile_n - eb.first_head[k]);
 }
 
-bool gemm_tiles_apply(const MfmaArgs& a) {
-  return a.B >= 128 && (a.K % kGBK) == 0 && (a.ldw % 8) == 0 && (a.ldx % 8) == 0 && (a.up_off % 8) == 0;
+static bool at16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+static bool aligned_rows(const MfmaArgs& a) {
+  return (a.ldw % 8) == 0 && (a.ldx % 8) == 0 && (a.up_off % 8) == 0 && at16(a.x) && at16(a.W) && (a.W2 == nullptr || at16(a.W2));
 }
+bool gemm_tiles_apply(const MfmaArgs& a) { return a.B >= 128 && (a.K % kGBK) == 0 && aligned_rows(a); }
 
 // K split for a grid of `tiles` workgroups: enough shares to give every compute unit two workgroups, at least four
 // K steps per share, and only as many as the registered workspace holds (1 = no split)
@@ -519,7 +562,7 @@ static int pick_ksplit_prompt(int64_t tiles, int ksteps, int K, size_t floats_pe
   return z > 1 ? fit_ksplit(z, tiles, ksteps, floats_per_share, ws, 8) : 1;
 }
 
-template <int DT, bool DUAL, int WTM, int WT, int BK, int NW = 4, int PFSEL = 99>
+template <int DT, bool DUAL, int WTM, int WT, int BK, int NW = 4, int PFSEL = 99, bool RAG = false>
 static int launch_gemm_tiles_t(const MfmaArgs& a0, hipStream_t st, const char* who) {
   static bool granted = false;
   constexpr int BM = 32 * WTM, BN = 32 * WT;
@@ -529,7 +572,7 @@ static int launch_gemm_tiles_t(const MfmaArgs& a0, hipStream_t st, const char* w
   constexpr int PF = PFSEL != 99 ? PFSEL : (!DUAL && WT == 2 && WTM == 2 && BK == 64) ? 4 : 2;
   const size_t lds = (size_t)(PF < 0 ? -PF : 2) * (DUAL ? 2 : 1) * (BM + BN) * kGLd * 2;
   if (lds > 64 * 1024 && !granted) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_tiles_kernel<DT, DUAL, WTM, WT, PF, false, BK, NW>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_tiles_kernel<DT, DUAL, WTM, WT, PF, false, BK, NW, RAG>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) { set_last_error("%s: cannot reserve %zu bytes of LDS: %s", who, lds, hipGetErrorString(e)); return kErrLaunch; }
     granted = true;
@@ -546,7 +589,7 @@ static int launch_gemm_tiles_t(const MfmaArgs& a0, hipStream_t st, const char* w
   a.ws_part = ws.part;
   a.ws_count = ws.count;
   grid.z = a.ksplit;
-  hipLaunchKernelGGL((gemm_tiles_kernel<DT, DUAL, WTM, WT, PF, false, BK, NW>), grid, dim3(NW * 64), lds, st, a, ExpandEpi{});
+  hipLaunchKernelGGL((gemm_tiles_kernel<DT, DUAL, WTM, WT, PF, false, BK, NW, RAG>), grid, dim3(NW * 64), lds, st, a, ExpandEpi{});
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }
   return kOk;
@@ -613,14 +656,39 @@ int launch_gemm_rows(const MfmaArgs& a, bool dual, hipStream_t st, const char* w
   return a.dt == 1 ? launch_gemm_rows_dt<1>(a, dual, st, who) : launch_gemm_rows_dt<0>(a, dual, st, who);
 }
 
-// head expansion of the prefill on the tiled kernel: 128 token rows and more, head_dim 128, rank a multiple of 64,
-// coefficients shared by the heads
-bool expand_tiles_apply(const ExpandArgs& a) {
-  return a.Dh == 128 && (int64_t)a.B * a.M >= 128 && (a.R % kGBK) == 0 && a.sp_h == 0 && (a.sp_b % 8) == 0 && (a.sp_m % 8) == 0 &&
-         (a.ldu % 8) == 0;
+// Rows or row lengths that the kernels above cannot take (K off the 64 grid, up to 32 rows off the 32 grid, or rows off the
+// 16-byte grid): three rows and more.  They ran on the vector kernels, which multiply every weight row with every row of x
+// out of LDS, four rows at a time, and load such rows element by element: the gate / up pair of the 7B shape at rank 1492
+// and 333 rows 3655 -> 93 us, down_u 656 -> 22 us (rank 1536: 64 and 16 us; the rest is misaligned pieces that straddle
+// cache lines).  With K a multiple of 32 only (33 to 127 rows; slices of 64 rows read the weights again for each) the pair
+// at rank 1504 and 64 rows 68 -> 42 us.
+bool gemm_ragged_apply(const MfmaArgs& a) {
+  if (a.B < 3) return false;
+  return !aligned_rows(a) || (a.K % (a.B > 32 ? kGBK : 32)) != 0;
+}
+template <int DT>
+static int launch_gemm_ragged_dt(const MfmaArgs& a, bool dual, hipStream_t st, const char* who) {
+  if (a.B < 128) return dual ? launch_gemm_tiles_t<DT, true, 1, 2, 64, 4, 2, true>(a, st, who) : launch_gemm_tiles_t<DT, false, 1, 2, 64, 4, 2, true>(a, st, who);
+  const int64_t big = (int64_t)((a.N + 127) / 128) * ((a.B + 127) / 128);
+  if (dual) return big >= 512 ? launch_gemm_tiles_t<DT, true, 4, 4, 64, 8, 2, true>(a, st, who) : launch_gemm_tiles_t<DT, true, 2, 2, 64, 4, 2, true>(a, st, who);
+  return big >= 256 ? launch_gemm_tiles_t<DT, false, 4, 4, 64, 4, 2, true>(a, st, who) : launch_gemm_tiles_t<DT, false, 2, 2, 64, 4, 4, true>(a, st, who);
+}
+int launch_gemm_ragged(const MfmaArgs& a, bool dual, hipStream_t st, const char* who) {
+  return a.dt == 1 ? launch_gemm_ragged_dt<1>(a, dual, st, who) : launch_gemm_ragged_dt<0>(a, dual, st, who);
 }
 
-template <int DT, int WTM>
+// head expansion of the prefill on the tiled kernel: 128 token rows and more, head_dim 128, rank a multiple of 64,
+// coefficients shared by the heads
+static bool expand_aligned(const ExpandArgs& a) {
+  return (a.R % kGBK) == 0 && (a.sp_b % 8) == 0 && (a.sp_m % 8) == 0 && (a.ldu % 8) == 0 && at16(a.p) && at16(a.u);
+}
+// any rank and rows that start anywhere, from 16 token rows on (q, k and v of 32 heads at rank 1024: one launch of 13.7 to
+// 16 us at 16 to 64 rows, three launches of one wave per 32 rows and head 80 to 95 us)
+bool expand_tiles_apply(const ExpandArgs& a) {
+  return a.Dh == 128 && a.R > 0 && a.heads > 0 && a.sp_h == 0 && (int64_t)a.B * a.M >= 16;
+}
+
+template <int DT, int WTM, bool RAG>
 static int launch_expand_tiles_t(const ExpandArgs& a, hipStream_t st) {
   const char* who = "fsvd_lowrank_expand_heads";
   static bool granted = false;
@@ -629,7 +697,7 @@ static int launch_expand_tiles_t(const ExpandArgs& a, hipStream_t st) {
   constexpr int BM = 32 * WTM;
   const size_t lds = (size_t)2 * (BM + 128) * kGLd * 2;
   if (!granted) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_tiles_kernel<DT, false, WTM, 4, PF, true, kGBK, 4>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_tiles_kernel<DT, false, WTM, 4, PF, true, kGBK, 4, RAG>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) { set_last_error("%s: cannot reserve %zu bytes of LDS: %s", who, lds, hipGetErrorString(e)); return kErrLaunch; }
     granted = true;
@@ -638,20 +706,20 @@ static int launch_expand_tiles_t(const ExpandArgs& a, hipStream_t st) {
   MfmaArgs g{a.p, 0, 0, a.u, nullptr, a.ldu, a.bias, nullptr, 0, a.y, 0, rows, a.heads * 128, a.R, 0};
   ExpandEpi ep{a.cos, a.sin, a.rope_len, a.positions, a.M, a.sp_b, a.sp_m, a.sy_b, a.sy_m, a.sy_h, a.dst_by_position, a.dst_rows};
   const dim3 grid(a.heads, (rows + BM - 1) / BM);
-  hipLaunchKernelGGL((gemm_tiles_kernel<DT, false, WTM, 4, PF, true, kGBK, 4>), grid, dim3(kGT4), lds, st, g, ep);
+  hipLaunchKernelGGL((gemm_tiles_kernel<DT, false, WTM, 4, PF, true, kGBK, 4, RAG>), grid, dim3(kGT4), lds, st, g, ep);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }
   return kOk;
 }
 
-template <int DT, int WTM>
+template <int DT, int WTM, bool RAG>
 static int launch_expand_multi_t(const ExpandArgs* d, int n, hipStream_t st) {
   const char* who = "fsvd_lowrank_expand_heads_multi";
   static bool granted = false;
   constexpr int BM = 32 * WTM;
   const size_t lds = (size_t)2 * (BM + 128) * kGBK * 2;
   if (!granted) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&expand_multi_kernel<DT, WTM>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&expand_multi_kernel<DT, WTM, RAG>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) { set_last_error("%s: cannot reserve %zu bytes of LDS: %s", who, lds, hipGetErrorString(e)); return kErrLaunch; }
     granted = true;
   }
@@ -668,7 +736,7 @@ static int launch_expand_multi_t(const ExpandArgs* d, int n, hipStream_t st) {
   eb.first_head[3] = heads;
   for (int k = n; k < 3; ++k) eb.first_head[k] = heads;    // unused sets start past the last head
   const dim3 grid(heads, (rows + BM - 1) / BM);
-  hipLaunchKernelGGL((expand_multi_kernel<DT, WTM>), grid, dim3(kGT4), lds, st, eb);
+  hipLaunchKernelGGL((expand_multi_kernel<DT, WTM, RAG>), grid, dim3(kGT4), lds, st, eb);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }
   return kOk;
@@ -681,19 +749,28 @@ bool expand_multi_apply(const ExpandArgs* d, int n) {
     if (!expand_tiles_apply(d[k]) || d[k].B != d[0].B || d[k].M != d[0].M || d[k].dt != d[0].dt) return false;
   return true;
 }
+template <int DT>
+static int launch_expand_multi_dt(const ExpandArgs* d, int n, bool aligned, bool wide, hipStream_t st) {
+  if (!aligned) return wide ? launch_expand_multi_t<DT, 4, true>(d, n, st) : launch_expand_multi_t<DT, 2, true>(d, n, st);
+  return wide ? launch_expand_multi_t<DT, 4, false>(d, n, st) : launch_expand_multi_t<DT, 2, false>(d, n, st);
+}
 int launch_expand_multi(const ExpandArgs* d, int n, hipStream_t st) {
   int heads = 0;
-  for (int k = 0; k < n; ++k) heads += d[k].heads;
-  const int64_t big = (int64_t)heads * (((int64_t)d[0].B * d[0].M + 127) / 128);
-  if (d[0].dt == 1) return big >= 384 ? launch_expand_multi_t<1, 4>(d, n, st) : launch_expand_multi_t<1, 2>(d, n, st);
-  return big >= 384 ? launch_expand_multi_t<0, 4>(d, n, st) : launch_expand_multi_t<0, 2>(d, n, st);
+  bool aligned = true;
+  for (int k = 0; k < n; ++k) { heads += d[k].heads; aligned = aligned && expand_aligned(d[k]); }
+  const bool wide = (int64_t)heads * (((int64_t)d[0].B * d[0].M + 127) / 128) >= 384;
+  return d[0].dt == 1 ? launch_expand_multi_dt<1>(d, n, aligned, wide, st) : launch_expand_multi_dt<0>(d, n, aligned, wide, st);
 }
 
+template <int DT>
+static int launch_expand_tiles_dt(const ExpandArgs& a, bool wide, hipStream_t st) {
+  if (!expand_aligned(a)) return wide ? launch_expand_tiles_t<DT, 4, true>(a, st) : launch_expand_tiles_t<DT, 2, true>(a, st);
+  return wide ? launch_expand_tiles_t<DT, 4, false>(a, st) : launch_expand_tiles_t<DT, 2, false>(a, st);
+}
 int launch_expand_tiles(const ExpandArgs& a, hipStream_t st) {
   // a column tile is always one head; 128 token rows per workgroup when that gives every compute unit two tiles, else 64
-  const int64_t big = (int64_t)a.heads * (((int64_t)a.B * a.M + 127) / 128);
-  if (a.dt == 1) return big >= 384 ? launch_expand_tiles_t<1, 4>(a, st) : launch_expand_tiles_t<1, 2>(a, st);
-  return big >= 384 ? launch_expand_tiles_t<0, 4>(a, st) : launch_expand_tiles_t<0, 2>(a, st);
+  const bool wide = (int64_t)a.heads * (((int64_t)a.B * a.M + 127) / 128) >= 384;
+  return a.dt == 1 ? launch_expand_tiles_dt<1>(a, wide, st) : launch_expand_tiles_dt<0>(a, wide, st);
 }
 
 }  // namespace fsvd

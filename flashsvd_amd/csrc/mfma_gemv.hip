@@ -29,7 +29,13 @@ template <class F>
 __device__ __forceinline__ F ldx_frag(const uint16_t* p) {
   return __builtin_bit_cast(F, *(gp16_t)(uintptr_t)p);
 }
-
+// the same at any element's address
+typedef const __attribute__((address_space(1))) u32x4_any_t* gpany_t;
+template <class F, bool NT>
+__device__ __forceinline__ F ld_any_frag(const uint16_t* p) {
+  const gpany_t g = (gpany_t)(uintptr_t)p;
+  return __builtin_bit_cast(F, (u32x4_t)(NT ? __builtin_nontemporal_load(g) : *g));
+}
 
 // the waves' partial tiles through LDS, added in wave order, then the epilogue of the vector kernels
 template <int DT, int NB, bool DUAL, int KS>
@@ -137,7 +143,8 @@ __device__ __forceinline__ void mfma_finish_split(const MfmaArgs& a, float (*red
 
 // NB: 16-row batch tiles (B <= 16 * NB); KS: waves that split K for one 16-row weight tile, so a workgroup
 // of 8 waves covers 8 / KS weight tiles
-template <int DT, int NB, bool DUAL, int KS>
+// RAG: any K, rows that start anywhere
+template <int DT, int NB, bool DUAL, int KS, bool RAG = false>
 __global__ __launch_bounds__(kMfThreads) void mfma_linear_kernel(MfmaArgs a) {
   typedef E16<DT> E;
   typedef typename E::frag_t frag_t;
@@ -147,7 +154,7 @@ __global__ __launch_bounds__(kMfThreads) void mfma_linear_kernel(MfmaArgs a) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
   const int rt = wave / KS, ks = wave % KS;
   const int n0 = (blockIdx.x * RT + rt) * 16;
-  const int ksteps = a.K >> 5;
+  const int ksteps = RAG ? (a.K + 31) >> 5 : a.K >> 5;
   // the KS waves of a weight tile take the k-steps in turn (wave ks: steps ks, ks + KS, ...), so that together they read
   // KS * 64 contiguous bytes of every row at a time; s counts this wave's own steps
   const int s0 = 0, s1 = (ksteps - ks + KS - 1) / KS;
@@ -168,9 +175,18 @@ __global__ __launch_bounds__(kMfThreads) void mfma_linear_kernel(MfmaArgs a) {
   const frag_t zero = __builtin_bit_cast(frag_t, u32x4_t{0u, 0u, 0u, 0u});
   for (int s = s0; s < s1; s += UN) {
     frag_t fa0[UN], fa1[UN], fb0[UN][NB], fb1[UN][NB];
+    // ragged: the trip that reaches past the last whole step masks its pieces (the same for every lane of the wave)
+    const bool masked = RAG && __builtin_amdgcn_readfirstlane(((min(s + UN, s1) - 1) * KS + ks + 1) << 5) > a.K;
 #pragma unroll
     for (int j = 0; j < UN; ++j) {
       const int k = (min(s + j, s1 - 1) * KS + ks) << 5;
+      if (RAG) {
+        static_assert(!RAG || (!DUAL && NB == 1), "the ragged form is built for up to 16 rows of a single matrix");
+        const int left = a.K - k - lg * 8;
+        fa0[j] = masked ? __builtin_bit_cast(frag_t, load_masked_piece(w0 + k, left, a.K)) : ld_any_frag<frag_t, true>(w0 + k);
+        fb0[j][0] = masked ? __builtin_bit_cast(frag_t, load_masked_piece(xr[0] + k, left, a.K)) : ld_any_frag<frag_t, false>(xr[0] + k);
+        continue;
+      }
       fa0[j] = ldw_frag<frag_t>(w0 + k);
       if (DUAL) fa1[j] = ldw_frag<frag_t>(w1 + k);
 #pragma unroll
@@ -517,11 +533,12 @@ static int launch_mfma_resident(const MfmaArgs& a, hipStream_t st, const char* w
   return a.B <= 16 ? launch_mfma_resident_nb<DT, DUAL, 1>(a, st, who) : launch_mfma_resident_nb<DT, DUAL, 2>(a, st, who);
 }
 
-template <int DT, int NB, bool DUAL>
+template <int DT, int NB, bool DUAL, bool RAG = false>
 static void launch_mfma_ks(const MfmaArgs& a, int ks, hipStream_t st) {
   const int tiles = (a.N + 15) / 16;
   const dim3 block(kMfThreads);
-  if (ks == 2) hipLaunchKernelGGL((mfma_linear_kernel<DT, NB, DUAL, 2>), dim3((tiles + 3) / 4), block, 0, st, a);
+  if (RAG) hipLaunchKernelGGL((mfma_linear_kernel<DT, NB, DUAL, 8, RAG>), dim3(tiles), block, 0, st, a);
+  else if (ks == 2) hipLaunchKernelGGL((mfma_linear_kernel<DT, NB, DUAL, 2>), dim3((tiles + 3) / 4), block, 0, st, a);
   else if (ks == 4) hipLaunchKernelGGL((mfma_linear_kernel<DT, NB, DUAL, 4>), dim3((tiles + 1) / 2), block, 0, st, a);
   else hipLaunchKernelGGL((mfma_linear_kernel<DT, NB, DUAL, 8>), dim3(tiles), block, 0, st, a);
 }
@@ -614,6 +631,16 @@ static int launch_mfma(const MfmaArgs& a0, hipStream_t st, const char* who) {
   int ks = 8;
   for (int c = 2; c <= 8; c *= 2)
     if ((tiles * c + 7) / 8 >= 256 && ksteps / c >= 4) { ks = c; break; }
+  // any K, rows that start anywhere: the tiled kernel, except that up to 16 rows of a single matrix run here (4096 x 1492 at
+  // 4 / 16 rows 8.5 / 9.7 us against 11.0 / 11.3; at 23 rows 11.5 both; the gate / up pair 11008 x 1492 at 4 / 16 rows is
+  // 36 / 43 us here and 35 / 36 there)
+  if (gemm_ragged_apply(a0)) {
+    if (DUAL || a0.B > 16) return launch_gemm_ragged(a0, DUAL, st, who);
+    launch_mfma_ks<DT, 1, false, true>(a0, 8, st);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }
+    return kOk;
+  }
   // many rows (prefill): the tiled kernel reads every weight once per 128 rows instead of once per 64
   if (gemm_tiles_apply(a0)) return launch_gemm_tiles(a0, DUAL, st, who);
   // a batch of rows: 32-row tiles with K split over workgroups, when the caller has registered a workspace — from 33
@@ -650,21 +677,14 @@ static int launch_mfma(const MfmaArgs& a0, hipStream_t st, const char* who) {
   return kOk;
 }
 
-static inline bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
-
 // true when the matrix-core path applies (the caller then skips the vector kernel)
-bool mfma_linear_applies(const LinearArgs& a) {
-  return a.B >= 3 && a.norm_w == nullptr && (a.K % 32) == 0 && (a.ldw % 8) == 0 && (a.ldx % 8) == 0 && al16(a.W) && al16(a.x);
-}
+bool mfma_linear_applies(const LinearArgs& a) { return a.B >= 3 && a.norm_w == nullptr; }
 int launch_linear_mfma(const LinearArgs& a, hipStream_t st) {
   MfmaArgs m{a.x, a.ldx, 0, a.W, nullptr, a.ldw, a.bias, a.res, a.ldres, a.y, a.ldy, a.B, a.N, a.K, 0};
   m.dt = a.dt;
   return a.dt == 1 ? launch_mfma<1, false>(m, st, "fsvd_linear") : launch_mfma<0, false>(m, st, "fsvd_linear");
 }
-bool mfma_swiglu_applies(const SwigluArgs& a) {
-  return a.B >= 3 && (a.R % 32) == 0 && (a.ldw % 8) == 0 && (a.ldp % 8) == 0 && (a.up_off % 8) == 0 && al16(a.gate_u) &&
-         al16(a.up_u) && al16(a.p);
-}
+bool mfma_swiglu_applies(const SwigluArgs& a) { return a.B >= 3; }
 int launch_swiglu_mfma(const SwigluArgs& a, hipStream_t st) {
   MfmaArgs m{a.p, a.ldp, a.up_off, a.gate_u, a.up_u, a.ldw, nullptr, nullptr, 0, a.h, a.ldh, a.B, a.D, a.R, a.mode};
   m.dt = a.dt;

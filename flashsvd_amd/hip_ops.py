@@ -144,7 +144,7 @@ def _linear_impl(x, weight, bias, norm_weight, eps, residual, out, cfg):
     lib = _lib.load()
     if B >= 3:
         ensure_split_workspace(x.device)
-    if norm_weight is not None and B >= 3 and cfg == 0 and K % 32 == 0:
+    if norm_weight is not None and B >= 3 and cfg == 0:
         # three rows and more run on the matrix cores, which take the activations as they are: normalise once
         # up front (same rounding points as the fused prologue)
         x2 = _rmsnorm_impl(x2, norm_weight, eps, None)

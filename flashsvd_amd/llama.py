@@ -383,7 +383,7 @@ class SVD_LlamaAttention(nn.Module):
     def prefill_tokens(self, x: torch.Tensor, cache, cache_position=None, *, norm_weight=None, eps: float = 1e-6,
                        residual: Optional[torch.Tensor] = None) -> torch.Tensor:
         """Causal full-sequence pass; T tokens are appended at start..start+T-1.
-        head_dim 128 with ranks that are multiples of 8 takes the matrix-core route (q/k/v rebuilt once
+        head_dim 128 takes the matrix-core route (q/k/v rebuilt once
         per token with the rotation fused, then causal flash attention over the cache).  Other shapes
         (or FLASHSVD_AMD_PREFILL=decode) reuse the decode kernels: the T tokens of one sequence are the
         kernel's batch rows, all bound to the same cache row (batch stride 0), token t written at
@@ -412,7 +412,7 @@ class SVD_LlamaAttention(nn.Module):
             p = hip_ops.linear(x, self._packed_qkv_v, norm_weight=norm_weight, eps=eps)   # [B,T,Rtot]
             wq, wk, wv = self.q_u_proj.weight, self.k_u_proj.weight, self.v_u_proj.weight
         rq, rk, rv = self._qkv_rank_tuple()
-        mfma_ok = Dh == 128 and rq % 8 == 0 and rk % 8 == 0 and rv % 8 == 0 and T >= 16 \
+        mfma_ok = Dh == 128 and T >= 16 \
             and os.getenv("FLASHSVD_AMD_PREFILL", "mfma").strip().lower() != "decode"
         a = torch.empty(B, T, H * Dh, device=x.device, dtype=x.dtype)
         if mfma_ok:

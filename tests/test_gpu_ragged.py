@@ -1,0 +1,71 @@
+"""Projections and head expansions whose rank or row length is no multiple of the matrix-core steps, or whose rows start
+off the 16-byte grid (three rows and more): edges of K steps (one element below and above a multiple of 64, less than one
+step), of row and column tiles, K split over workgroups, against the CPU oracle."""
+import pytest
+import torch
+
+from oracle import flashsvd_oracle as O
+from tests.util import assert_close_bf16, bounds, rand_bf16
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,N,K", [(3, 17, 1), (3, 64, 7), (5, 130, 63), (16, 100, 65), (40, 515, 1492), (127, 33, 2049), (128, 65, 63),
+                                   (130, 129, 1638), (129, 4100, 1025), (300, 257, 96), (1030, 4096, 130)])
+def test_linear_any_k(B, N, K):
+    from flashsvd_amd import hip_ops
+    x, w = rand_bf16(B, K, seed=1), rand_bf16(N, K, std=K ** -0.5, seed=2)
+    res, bias = rand_bf16(B, N, seed=3), rand_bf16(N, seed=4)
+    y = hip_ops.linear(x.cuda(), w.cuda(), bias.cuda(), residual=res.cuda())
+    ref = res + O.lin(x, w, bias)
+    assert_close_bf16(y, ref, f"linear {B}x{N}x{K}", **bounds(ref))
+
+
+@pytest.mark.parametrize("off", [1, 2, 4])
+@pytest.mark.parametrize("B", [4, 200])
+def test_linear_rows_off_the_grid(B, off):
+    """K is a whole number of steps, the rows of x and W start ``off`` elements past a 16-byte boundary."""
+    from flashsvd_amd import hip_ops
+    x, w = rand_bf16(B, 136, seed=1).cuda(), rand_bf16(96, 136, std=0.1, seed=2).cuda()
+    y = hip_ops.linear(x[:, off:off + 128], w[:, off:off + 128])
+    assert_close_bf16(y, O.lin(x[:, off:off + 128].cpu(), w[:, off:off + 128].cpu()), f"offset {off}")
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("B,D,R", [(3, 100, 52), (33, 1376, 375), (128, 130, 1), (200, 688, 100), (1040, 8200, 67)])
+def test_swiglu_any_rank(B, D, R, mode):
+    from flashsvd_amd import hip_ops
+    p = rand_bf16(B, 2 * R, seed=1)
+    gu, uu = rand_bf16(D, R, std=R ** -0.5, seed=2), rand_bf16(D, R, std=R ** -0.5, seed=3)
+    h = hip_ops.swiglu_linear(p.cuda(), gu.cuda(), uu.cuda(), up_off=R, mode=mode)
+    g, u = p[:, :R].float() @ gu.float().t(), p[:, R:].float() @ uu.float().t()
+    if mode == 0:
+        ref = torch.nn.functional.silu(g.to(torch.bfloat16)) * u.to(torch.bfloat16)
+    else:
+        ref = ((g * torch.sigmoid(g)) * u).to(torch.bfloat16)
+    assert_close_bf16(h, ref, f"swiglu {B}x{D}x{R}", **bounds(ref))
+
+
+@pytest.mark.parametrize("B,T,R", [(1, 16, 1), (2, 37, 52), (1, 130, 1638), (2, 333, 65)])
+def test_head_expansion_any_rank(B, T, R):
+    """q with the rotation and v without, as one launch and as two, at positions behind a cached prefix."""
+    from flashsvd_amd import hip_ops
+    H, Hk, Dh = 4, 2, 128
+    p = rand_bf16(B, T, 2 * R, seed=1)
+    qu, vu = rand_bf16(H * Dh, R, std=R ** -0.5, seed=2), rand_bf16(Hk * Dh, R, std=R ** -0.5, seed=3)
+    cos, sin = O.rope_tables(T + 9, Dh, dtype=torch.bfloat16)
+    pos = torch.full((B,), 9, dtype=torch.int32)
+    q = torch.zeros(B, T, H, Dh, dtype=torch.bfloat16, device="cuda")
+    v = torch.zeros(B, T + 9, Hk, Dh, dtype=torch.bfloat16, device="cuda")
+    pc = p.cuda()
+    items = [dict(p=pc[..., :R], u=qu.cuda(), num_heads=H, out=q, rotate=True),
+             dict(p=pc[..., R:], u=vu.cuda(), num_heads=Hk, out=v, dst_by_position=True)]
+    kw = dict(head_dim=Dh, cos=cos.cuda(), sin=sin.cuda(), positions=pos.cuda())
+    hip_ops.lowrank_expand_heads_multi(items, **kw)
+    ref_q = O.apply_rope(O.lin(p[..., :R], qu).view(B, T, H, Dh), cos[9:, None], sin[9:, None])
+    ref_v = O.lin(p[..., R:], vu).view(B, T, Hk, Dh)
+    assert_close_bf16(q, ref_q, "q", **bounds(ref_q))
+    assert_close_bf16(v[:, 9:], ref_v, "v", **bounds(ref_v))
+    q2 = torch.zeros_like(q)
+    hip_ops.lowrank_expand_heads(pc[..., :R], qu.cuda(), num_heads=H, out=q2, **kw)
+    assert torch.equal(q, q2)
