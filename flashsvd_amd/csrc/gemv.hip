@@ -640,6 +640,24 @@ int launch_swiglu(const SwigluArgs& a, int cfg, hipStream_t st) {
   return a.dt == 1 ? launch_swiglu_t<1>(a, cfg, st) : launch_swiglu_t<0>(a, cfg, st);
 }
 
+// the head expansion of the prompt pass with one token per batch row: q to its buffer, k and v to the cache rows
+static int launch_qkv_tiles(const QkvArgs& a, hipStream_t st) {
+  ExpandArgs d[3];
+  for (int i = 0; i < 3; ++i) {
+    ExpandArgs& e = d[i];
+    e = ExpandArgs{};
+    e.p = a.p + (i == 0 ? 0 : (i == 1 ? a.Rq : a.Rq + a.Rk)); e.sp_b = a.ldp;
+    e.u = i == 0 ? a.q_u : (i == 1 ? a.k_u : a.v_u); e.ldu = i == 0 ? a.ldq : (i == 1 ? a.ldk : a.ldv);
+    if (i < 2) { e.cos = a.cos; e.sin = a.sin; e.rope_len = a.rope_len; }
+    e.positions = a.positions;
+    e.y = i == 0 ? a.q_out : (i == 1 ? a.k_cache : a.v_cache);
+    e.sy_b = i == 0 ? (int64_t)a.H * a.Dh : a.sc_b; e.sy_m = i == 0 ? 0 : a.sc_s; e.sy_h = i == 0 ? a.Dh : a.sc_h;
+    e.dst_by_position = i > 0; e.dst_rows = i == 0 ? 1 : a.S;
+    e.B = a.B; e.M = 1; e.heads = i == 0 ? a.H : a.Hk; e.Dh = a.Dh; e.R = i == 0 ? a.Rq : (i == 1 ? a.Rk : a.Rv); e.dt = a.dt;
+  }
+  return launch_expand_multi(d, 3, st);
+}
+
 template <int DT, int BATCH, bool VEC>
 static int launch_qkv_b(const QkvArgs& a, int cfg, hipStream_t st) {
   const int Rq8 = (a.Rq + 7) & ~7, Rk8 = (a.Rk + 7) & ~7, Rv8 = (a.Rv + 7) & ~7;
@@ -688,6 +706,10 @@ static int launch_qkv_t(const QkvArgs& a, int cfg, hipStream_t st) {
 int launch_qkv(const QkvArgs& a, int cfg, hipStream_t st) {
   const int rc = check_qkv(a);
   if (rc != kOk) return rc;
+  if (cfg == 0 && qkv_mfma_applies(a)) return launch_qkv_mfma(a, st);
+  // the tiled head expansion with one token per row takes the other batches: more tokens, or ranks and rows off the grid
+  // (64 tokens at rank 1024 206 -> 16 us, 4 tokens at rank 1001 30 -> 20 us)
+  if (cfg == 0 && a.B >= 3 && a.Dh == 128) return launch_qkv_tiles(a, st);
   return a.dt == 1 ? launch_qkv_t<1>(a, cfg, st) : launch_qkv_t<0>(a, cfg, st);
 }
 

@@ -478,6 +478,136 @@ __global__ __launch_bounds__(kMfThreads) void mfma_resident_kernel(MfmaArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// Head expansion of a batch of decoded tokens, 3..32 rows: q, k and v from their rank coefficients, rotate-half RoPE on q
+// and k, k and v into the cache rows (the rounding points of qkv_rope_append_kernel).  The weight stream is the one of
+// mfma_stream_kernel's pair form, the pair being rows d .. d + 15 and d + Dh/2 .. of one head, which the rotation mixes and
+// which share their activation fragments: a workgroup per pair of tiles (384 at the 7B shape, two to a compute unit), K
+// split over its eight waves.  Bound by the launch-to-drain chain (two chunks per wave at rank 1024) more than by the
+// 25 MB it streams.  The vector kernel takes four rows at a time, so at 16 rows it reads the bases four times over and
+// multiplies out of LDS: 17.6 / 31.6 / 60.2 / 115 us at 3 / 8 / 16 / 32 tokens of the 7B shape, 6.8 / 7.2 / 7.8 / 9.6 here.
+// ---------------------------------------------------------------------------------------------
+template <int DT, int NB>
+__global__ __launch_bounds__(kMfThreads) void mfma_qkv_kernel(QkvArgs a) {
+  typedef E16<DT> E;
+  typedef typename E::frag_t frag_t;
+  typedef StreamShape<true> SS;
+  constexpr int CKB = SS::CKB, kStage = SS::kStage, D = 2;
+  constexpr int PPR = CKB / 16, KST = CKB / 64, RPI = 64 / PPR, NI = 16 / RPI;
+  constexpr int kGroup = 2 * NI + KST * NB;       // loads per chunk: weight pieces into LDS, activation fragments into registers
+  extern __shared__ __align__(16) unsigned char st_smem[];     // [8 waves][D][kStage]; the partial tiles at the end
+  float* red = reinterpret_cast<float*>(st_smem);              // [8][2][NB][4][kResPitch]
+  constexpr int kRedWave = 2 * NB * 4 * kResPitch;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
+  const int half = a.Dh >> 1, per_head = half >> 4;
+  const int hh = blockIdx.x / per_head, d0 = (blockIdx.x - hh * per_head) * 16;
+  const int kind = hh < a.H ? 0 : (hh < a.H + a.Hk ? 1 : 2);
+  const int head = kind == 0 ? hh : (kind == 1 ? hh - a.H : hh - a.H - a.Hk);
+  const int K = kind == 0 ? a.Rq : (kind == 1 ? a.Rk : a.Rv);
+  const int64_t ldw = kind == 0 ? a.ldq : (kind == 1 ? a.ldk : a.ldv);
+  const uint16_t* W = (kind == 0 ? a.q_u : (kind == 1 ? a.k_u : a.v_u)) + (int64_t)(head * a.Dh + d0) * ldw;
+  const uint16_t* x = a.p + (kind == 0 ? 0 : (kind == 1 ? a.Rq : a.Rq + a.Rk));
+  unsigned char* ring = st_smem + (size_t)wave * D * kStage;
+  const int nchunk = K / (CKB / 2);
+  const int cw = max(0, (nchunk - wave + kMfWaves - 1) / kMfWaves);   // this wave's chunks: wave, wave + 8, ...
+  typedef const __attribute__((address_space(1))) void* gptr_t;
+  typedef __attribute__((address_space(3))) void* lptr_t;
+  const int lrow = lane / PPR, lpc = lane % PPR;
+  const uint16_t* wsrc[2][NI];
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int q = 0; q < NI; ++q) {
+      const int row = q * RPI + lrow;
+      wsrc[m][q] = W + (int64_t)(m * half + row) * ldw + ((lpc ^ (row % PPR)) * 8);
+    }
+  const uint16_t* xsrc[NB];
+#pragma unroll
+  for (int t = 0; t < NB; ++t) xsrc[t] = x + (int64_t)min(t * 16 + lr, a.B - 1) * a.ldp + lg * 8;
+  frag_t xf[D][KST][NB];
+  const auto issue = [&](int c, int slot) {        // one chunk's loads stay together: the wait below counts them in order
+    const int k0 = (c * kMfWaves + wave) * (CKB / 2);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int q = 0; q < NI; ++q)
+        __builtin_amdgcn_global_load_lds((gptr_t)(wsrc[m][q] + k0), (lptr_t)(ring + slot * kStage + m * 16 * CKB + q * 1024), 16, 0, 2);
+#pragma unroll
+    for (int s = 0; s < KST; ++s)
+#pragma unroll
+      for (int t = 0; t < NB; ++t) xf[slot][s][t] = ldx_frag<frag_t>(xsrc[t] + k0 + s * 32);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  f32x4_t acc[2][NB];
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int t = 0; t < NB; ++t) acc[m][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  constexpr int kW0 = (7 << 4) | (15 << 8);
+  static_assert(kGroup < 16, "one group of loads fits the low bits of the wait");
+  if (cw > 0) issue(0, 0);
+  for (int c0 = 0; c0 < cw; c0 += D) {
+#pragma unroll
+    for (int u = 0; u < D; ++u) {
+      const int c = c0 + u;
+      if (c >= cw) break;
+      if (c + 1 < cw) {
+        issue(c + 1, (u + 1) % D);
+        __builtin_amdgcn_s_waitcnt(kW0 | kGroup);
+      } else {
+        __builtin_amdgcn_s_waitcnt(kW0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s = 0; s < KST; ++s)
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          const frag_t wf = *reinterpret_cast<const frag_t*>(ring + u * kStage + m * 16 * CKB + lr * CKB + (((s * 4 + lg) ^ (lr % PPR)) * 16));
+#pragma unroll
+          for (int t = 0; t < NB; ++t) acc[m][t] = E::mfma(wf, xf[u][s][t], acc[m][t]);
+        }
+    }
+  }
+  __syncthreads();                                 // every wave is done with its ring: the partial tiles take its place
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int t = 0; t < NB; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) red[wave * kRedWave + ((m * NB + t) * 4 + i) * kResPitch + lane] = acc[m][t][i];
+  __syncthreads();
+  // a thread per rotation pair, 16 consecutive lanes on 16 consecutive dimensions of one token; the waves' sums in wave order
+  const int nn = tid & 15, b = tid >> 4;
+  if (b >= a.B || b >= 16 * NB) return;
+  const int ro = ((b >> 4) * 4 + (nn & 3)) * kResPitch + (nn >> 2) * 16 + (b & 15);
+  float x0 = 0.f, x1 = 0.f;
+#pragma unroll
+  for (int w = 0; w < kMfWaves; ++w) {
+    x0 += red[w * kRedWave + ro];
+    x1 += red[w * kRedWave + NB * 4 * kResPitch + ro];
+  }
+  const int d = d0 + nn, pos = a.positions[b];
+  x0 = E::rnd(x0);
+  x1 = E::rnd(x1);
+  if (kind != 2 && a.cos) {
+    const int tp = min(max(pos, 0), a.rope_len - 1);
+    const float c = E::val(a.cos[(int64_t)tp * half + d]), s = E::val(a.sin[(int64_t)tp * half + d]);
+    const float r0 = E::rnd(E::rnd(x0 * c) - E::rnd(x1 * s));
+    const float r1 = E::rnd(E::rnd(x1 * c) + E::rnd(x0 * s));
+    x0 = r0; x1 = r1;
+  }
+  uint16_t* dst;
+  if (kind == 0) {
+    dst = a.q_out + ((int64_t)b * a.H + head) * a.Dh + d;
+  } else {
+    if (pos < 0 || pos >= a.S) return;
+    dst = (kind == 1 ? a.k_cache : a.v_cache) + (int64_t)b * a.sc_b + (int64_t)pos * a.sc_s + (int64_t)head * a.sc_h + d;
+  }
+  dst[0] = (uint16_t)E::bits(x0);
+  dst[half] = (uint16_t)E::bits(x1);
+}
+
 static int compute_units() {
   static int cus[16] = {0};
   int dev = 0;
@@ -675,6 +805,36 @@ static int launch_mfma(const MfmaArgs& a0, hipStream_t st, const char* who) {
     if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }
   }
   return kOk;
+}
+
+static inline bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+template <int DT, int NB>
+static int launch_qkv_mfma_t(const QkvArgs& a, hipStream_t st) {
+  const char* who = "fsvd_qkv_rope_append";
+  constexpr size_t ring = (size_t)kMfWaves * 2 * StreamShape<true>::kStage, parked = (size_t)kMfWaves * 2 * NB * 4 * kResPitch * sizeof(float);
+  constexpr size_t lds = ring > parked ? ring : parked;
+  if (lds > 64 * 1024) {
+    static bool granted = false;
+    if (!granted) {
+      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&mfma_qkv_kernel<DT, NB>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      if (e != hipSuccess) { set_last_error("%s: cannot reserve %zu bytes of LDS: %s", who, lds, hipGetErrorString(e)); return kErrLaunch; }
+      granted = true;
+    }
+  }
+  hipLaunchKernelGGL((mfma_qkv_kernel<DT, NB>), dim3((a.H + 2 * a.Hk) * (a.Dh / 32)), dim3(kMfThreads), lds, st, a);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }
+  return kOk;
+}
+// 3..32 tokens, ranks of whole chunks, a head of whole tile pairs
+bool qkv_mfma_applies(const QkvArgs& a) {
+  return a.B >= 3 && a.B <= 32 && a.Dh % 32 == 0 && a.Rq % 64 == 0 && a.Rk % 64 == 0 && a.Rv % 64 == 0 && a.ldp % 8 == 0 && a.ldq % 8 == 0 &&
+         a.ldk % 8 == 0 && a.ldv % 8 == 0 && al16(a.p) && al16(a.q_u) && al16(a.k_u) && al16(a.v_u);
+}
+int launch_qkv_mfma(const QkvArgs& a, hipStream_t st) {
+  if (a.B <= 16) return a.dt == 1 ? launch_qkv_mfma_t<1, 1>(a, st) : launch_qkv_mfma_t<0, 1>(a, st);
+  return a.dt == 1 ? launch_qkv_mfma_t<1, 2>(a, st) : launch_qkv_mfma_t<0, 2>(a, st);
 }
 
 // true when the matrix-core path applies (the caller then skips the vector kernel)
