@@ -36,8 +36,10 @@ __device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) {
 }
 // value after one bf16 rounding
 __device__ __forceinline__ float round_bf16(float f) { return bf16_bits_to_f32(f32_to_bf16_bits(f)); }
+// two roundings in one instruction (V_CVT_PK_BF16_F32; rounding each by itself and joining the halves takes four)
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-  return f32_to_bf16_bits(lo) | (f32_to_bf16_bits(hi) << 16);
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{lo, hi}, bf16x2_t));
 }
 
 // acc += a.lo*b.lo + a.hi*b.hi with fp32 accumulation (V_DOT2_F32_BF16)
@@ -104,7 +106,9 @@ template <> struct E16<1> {
     return static_cast<uint32_t>(__builtin_bit_cast(unsigned short, static_cast<_Float16>(f)));
   }
   static __device__ __forceinline__ float rnd(float f) { return (float)static_cast<_Float16>(f); }
-  static __device__ __forceinline__ uint32_t pack2(float l, float h) { return bits(l) | (bits(h) << 16); }
+  static __device__ __forceinline__ uint32_t pack2(float l, float h) {
+    return __builtin_bit_cast(uint32_t, f16x2_t{static_cast<_Float16>(l), static_cast<_Float16>(h)});
+  }
   // V_DOT2_F32_F16
   static __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float acc) {
     return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, a), __builtin_bit_cast(f16x2_t, b), acc, false);

@@ -178,6 +178,11 @@ bool gemm_tiles_apply(const MfmaArgs& a);                                   // m
 int launch_gemm_tiles(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
 bool gemm_rows_apply(const MfmaArgs& a);                                    // mfma_gemm.hip: 5..127 rows, K split
 int launch_gemm_rows(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
+int compute_units();                                                         // of the current device, 0 when it cannot be asked
+bool gemm_big_apply(const MfmaArgs& a, bool dual);                          // mfma_big.hip: 256 x 256 tiles
+int launch_gemm_big(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
+bool expand_big_apply(const ExpandArgs* d, int n);
+int launch_expand_big(const ExpandArgs* d, int n, hipStream_t st);
 bool gemm_ragged_apply(const MfmaArgs& a);                                  // mfma_gemm.hip: any K, rows that start anywhere
 int launch_gemm_ragged(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
 

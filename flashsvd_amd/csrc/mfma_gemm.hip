@@ -598,7 +598,8 @@ static int launch_gemm_tiles_t(const MfmaArgs& a0, hipStream_t st, const char* w
 template <int DT>
 static int launch_gemm_tiles_dt(const MfmaArgs& a, bool dual, hipStream_t st, const char* who) {
   const int64_t big = (int64_t)((a.N + 127) / 128) * ((a.B + 127) / 128);
-  // Forms by tile count (measured on the projections of the 7B shape at 128..4096 rows).  The pair kernel: the
+  // Forms by tile count, for what the 256 x 256 tiles of mfma_big.hip leave (too few tiles for them, the pair with the
+  // gate kept in fp32, outputs off the 16-byte grid) (measured on the projections of the 7B shape at 128..4096 rows).  The pair kernel: the
   // eight-wave 128 x 128 form from two big tiles per compute unit on, else 64 x 64.  A single matrix: 128 x 128 from
   // 448 big tiles on, 128 x 64 from 256 on, else 64 x 64 — in K steps of 64 with a deep register pipeline when there
   // are more of those than the chip holds at once (320), in steps of 128 (half as many barriers) when there are fewer:
@@ -615,10 +616,6 @@ static int launch_gemm_tiles_dt(const MfmaArgs& a, bool dual, hipStream_t st, co
   // a single matrix with more than one big tile per compute unit: loads straight into LDS, two stages (the second and
   // third workgroup of a compute unit cover the one-step load distance; 5..8 % faster than the register pipeline with
   // weights that come from HBM, and slower than it below these tile counts)
-  // many tiles per compute unit (long prompts): 128 x 256 tiles, a wave on 64 x 128 of it -- a third fewer fragment
-  // reads from LDS per product; K steps of 32 keep two workgroups per compute unit (16384 rows of the 7B shape at
-  // ratio 0.8: 1..6 % faster per projection, same results bit for bit)
-  if (big >= 2048) return launch_gemm_tiles_t<DT, false, 4, 8, 32, 4, -2>(a, st, who);
   if (big >= 448) return launch_gemm_tiles_t<DT, false, 4, 4, 64, 4, -2>(a, st, who);
   if (big >= 320) return launch_gemm_tiles_t<DT, false, 4, 2, 64, 4, -2>(a, st, who);
   // about one tile per compute unit: eight waves on a 128 x 128 or 128 x 64 tile, each half of them on half of the k
@@ -755,6 +752,7 @@ static int launch_expand_multi_dt(const ExpandArgs* d, int n, bool aligned, bool
   return wide ? launch_expand_multi_t<DT, 4, false>(d, n, st) : launch_expand_multi_t<DT, 2, false>(d, n, st);
 }
 int launch_expand_multi(const ExpandArgs* d, int n, hipStream_t st) {
+  if (expand_big_apply(d, n)) return launch_expand_big(d, n, st);
   int heads = 0;
   bool aligned = true;
   for (int k = 0; k < n; ++k) { heads += d[k].heads; aligned = aligned && expand_aligned(d[k]); }
@@ -768,6 +766,7 @@ static int launch_expand_tiles_dt(const ExpandArgs& a, bool wide, hipStream_t st
   return wide ? launch_expand_tiles_t<DT, 4, false>(a, st) : launch_expand_tiles_t<DT, 2, false>(a, st);
 }
 int launch_expand_tiles(const ExpandArgs& a, hipStream_t st) {
+  if (expand_big_apply(&a, 1)) return launch_expand_big(&a, 1, st);
   // a column tile is always one head; 128 token rows per workgroup when that gives every compute unit two tiles, else 64
   const bool wide = (int64_t)a.heads * (((int64_t)a.B * a.M + 127) / 128) >= 384;
   return a.dt == 1 ? launch_expand_tiles_dt<1>(a, wide, st) : launch_expand_tiles_dt<0>(a, wide, st);

@@ -608,7 +608,7 @@ __global__ __launch_bounds__(kMfThreads) void mfma_qkv_kernel(QkvArgs a) {
   dst[half] = (uint16_t)E::bits(x1);
 }
 
-static int compute_units() {
+int compute_units() {
   static int cus[16] = {0};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 16) return 0;
@@ -772,6 +772,7 @@ static int launch_mfma(const MfmaArgs& a0, hipStream_t st, const char* who) {
     return kOk;
   }
   // many rows (prefill): the tiled kernel reads every weight once per 128 rows instead of once per 64
+  if (gemm_big_apply(a0, DUAL)) return launch_gemm_big(a0, DUAL, st, who);
   if (gemm_tiles_apply(a0)) return launch_gemm_tiles(a0, DUAL, st, who);
   // a batch of rows: 32-row tiles with K split over workgroups, when the caller has registered a workspace — from 33
   // rows on (up to 32 rows the streaming form is faster: 12.3 / 25.3 / 6.7 us against 13.4 / 28.8 / 8.8 us on the wide
