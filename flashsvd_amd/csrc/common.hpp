@@ -184,6 +184,14 @@ __device__ __forceinline__ u32x4_t load_masked_piece(const uint16_t* p, int left
   return u32x4_t{w[0], w[1], w[2], w[3]};
 }
 
+// 16 bytes per lane from p + lane offset + uniform offset straight to LDS (lane i lands 16 i bytes past dst)
+__device__ __forceinline__ void buffer_to_lds(const uint16_t* p, unsigned char* dst, uint32_t lane_off, int off) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p), 0, 0xffffffffu, 0x00020000u);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)dst, 16, (int)lane_off, off, 0, 0);
+#endif
+}
+
 // Cross-workgroup hand-off without L2 write-back/invalidate fences: producers use write-through
 // (agent-scope) stores, wait until the memory system has acknowledged them, then signal through an
 // agent-scope atomic; consumers read with agent-scope loads.  A workgroup-scope release fence does

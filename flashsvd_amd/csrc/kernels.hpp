@@ -171,6 +171,15 @@ struct MfmaArgs {
   int ksplit; float* ws_part; int32_t* ws_count;
   int dt = 0;
 };
+// epilogue of a head expansion (mfma_gemm.hip, mfma_mid.hip)
+struct ExpandEpi {
+  const uint16_t* cos; const uint16_t* sin; int rope_len;
+  const int32_t* positions;
+  int M;                                   // tokens per batch row (x row r = batch r / M, token r % M)
+  int64_t sp_b, sp_m;                      // strides of the coefficient rows
+  int64_t sy_b, sy_m, sy_h;                // destination strides
+  int dst_by_position, dst_rows;
+};
 // caller-owned scratch of the current device for the K-split projections (null when none is registered)
 struct SplitWorkspace { float* part; size_t part_floats; int32_t* count; int ncount; };
 SplitWorkspace split_workspace();                                            // capi.hip
@@ -183,6 +192,10 @@ bool gemm_big_apply(const MfmaArgs& a, bool dual);                          // m
 int launch_gemm_big(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
 bool expand_big_apply(const ExpandArgs* d, int n);
 int launch_expand_big(const ExpandArgs* d, int n, hipStream_t st);
+bool gemm_mid_apply(const MfmaArgs& a, bool dual);                          // mfma_mid.hip: about one tile per compute unit
+int launch_gemm_mid(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
+bool expand_mid_apply(const ExpandArgs* d, int n);
+int launch_expand_mid(const ExpandArgs* d, int n, hipStream_t st);
 bool gemm_ragged_apply(const MfmaArgs& a);                                  // mfma_gemm.hip: any K, rows that start anywhere
 int launch_gemm_ragged(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
 

@@ -56,14 +56,6 @@ struct BigProblem {
 };
 struct BigArgs { BigProblem p[3]; int first_tile[4]; int rows, nt; };   // column tiles of problem i: [first_tile[i], first_tile[i + 1])
 
-// 16 bytes per lane from p + lane offset + uniform offset straight to LDS (lane i lands 16 i bytes past dst)
-__device__ __forceinline__ void buffer_to_lds(const uint16_t* p, unsigned char* dst, uint32_t lane_off, int off) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p), 0, 0xffffffffu, 0x00020000u);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)dst, 16, (int)lane_off, off, 0, 0);
-#endif
-}
-
 // two tiles' words of a row of 16 lanes become consecutive words: lanes of even rows get columns 4 r .. 4 r + 7 of tile a,
 // lanes of odd rows of tile b (r the row below), see store_pair
 __device__ __forceinline__ void swap_rows(uint32_t& a, uint32_t& b) {
@@ -409,7 +401,7 @@ bool expand_big_apply(const ExpandArgs* d, int n) {
     if (a.sp_b < 0 || a.sp_m < 0 || ((a.B - 1) * a.sp_b + (a.M - 1) * a.sp_m + a.R) * 2 >= (int64_t)4 << 30 || !below4g((int64_t)a.heads * 128, a.ldu)) return false;
     tiles += (a.heads + 1) / 2;
   }
-  return big_worth((int64_t)d[0].B * d[0].M, tiles, 55);
+  return big_worth((int64_t)d[0].B * d[0].M, tiles, 65);   // q, k and v of 32 heads at 1024 rows (75 %) 42 against 44 us of 64-row tiles, at 1536 (56 %) 77 against 69
 }
 int launch_expand_big(const ExpandArgs* d, int n, hipStream_t st) {
   BigArgs a{};

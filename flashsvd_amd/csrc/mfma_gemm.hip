@@ -30,14 +30,6 @@ constexpr int kGBK = 64;            // K per step (the small tile takes 128 when
 // EXPAND: the head-expansion form of the prefill (y = P . u^T per head, then rotate-half RoPE at the token's position
 // and a store into the query buffer or the cache rows): a column tile is one 128-wide head, and a wave takes columns
 // [32 wn, 32 wn + 32) and [64 + 32 wn, 64 + 32 wn + 32) of it so that d and d + 64 of a rotation pair sit in one lane
-struct ExpandEpi {
-  const uint16_t* cos; const uint16_t* sin; int rope_len;
-  const int32_t* positions;
-  int M;                                   // tokens per batch row (x row r = batch r / M, token r % M)
-  int64_t sp_b, sp_m;                      // strides of the coefficient rows
-  int64_t sy_b, sy_m, sy_h;                // destination strides
-  int dst_by_position, dst_rows;
-};
 
 // NW: waves per workgroup.  4: a wave owns a 16 WTM x 16 WT block of the output tile (both matrices of the gate / up
 // pair).  8, pair (128 x 128 only): waves 0-3 accumulate the gate matrix and waves 4-7 the up matrix of the same
@@ -524,12 +516,12 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void gemm_tiles_kernel(Mf
 // of one of them.  At 512 rows a single expansion has one workgroup per compute unit and waits on its own loads; the
 // three together give every compute unit three.
 struct ExpandBatch { MfmaArgs a[3]; ExpandEpi ep[3]; int first_head[4]; };
-template <int DT, int WTM, bool RAG = false>
+template <int DT, int WTM>
 __global__ __launch_bounds__(kGT4, 2) void expand_multi_kernel(ExpandBatch eb) {
   int tile_m, tile_n;
   tile_of_workgroup(gridDim.x, gridDim.y, tile_m, tile_n);
   const int k = tile_n >= eb.first_head[2] ? 2 : (tile_n >= eb.first_head[1] ? 1 : 0);
-  gemm_tiles_body<DT, false, WTM, 4, 2, true, kGBK, 4, RAG>(eb.a[k], eb.ep[k], tile_m, tile_n - eb.first_head[k]);
+  gemm_tiles_body<DT, false, WTM, 4, 2, true, kGBK, 4, true>(eb.a[k], eb.ep[k], tile_m, tile_n - eb.first_head[k]);
 }
 
 static bool at16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -598,31 +590,21 @@ static int launch_gemm_tiles_t(const MfmaArgs& a0, hipStream_t st, const char* w
 template <int DT>
 static int launch_gemm_tiles_dt(const MfmaArgs& a, bool dual, hipStream_t st, const char* who) {
   const int64_t big = (int64_t)((a.N + 127) / 128) * ((a.B + 127) / 128);
-  // Forms by tile count, for what the 256 x 256 tiles of mfma_big.hip leave (too few tiles for them, the pair with the
-  // gate kept in fp32, outputs off the 16-byte grid) (measured on the projections of the 7B shape at 128..4096 rows).  The pair kernel: the
-  // eight-wave 128 x 128 form from two big tiles per compute unit on, else 64 x 64.  A single matrix: 128 x 128 from
-  // 448 big tiles on, 128 x 64 from 256 on, else 64 x 64 — in K steps of 64 with a deep register pipeline when there
-  // are more of those than the chip holds at once (320), in steps of 128 (half as many barriers) when there are fewer:
-  // with one workgroup or less per compute unit and a long K only loads issued several steps ahead hide the latency.
-  // The pair at four big tiles per compute unit and more: four waves with both accumulator sets, K steps of 32
-  // loaded straight into LDS (two workgroups per compute unit; 243 -> 214 us at 2048 rows of the 7B MLP)
-  if (dual && big >= 1024) return launch_gemm_tiles_t<DT, true, 4, 4, 32, 4, -2>(a, st, who);
-  if (dual && big >= 512) return launch_gemm_tiles_t<DT, true, 4, 4, 64, 8>(a, st, who);
-  // two and a half to four 64 x 128 tiles per compute unit: that tile, K steps of 32 straight into LDS, three
-  // workgroups per compute unit (7B MLP at 512 rows 83 -> 77 us, at 768 rows 114 -> 110; slower outside this range)
-  const int64_t wide = (int64_t)((a.N + 127) / 128) * ((a.B + 63) / 64);
-  if (dual && wide >= 640 && wide <= 1100) return launch_gemm_tiles_t<DT, true, 2, 4, 32, 4, -2>(a, st, who);
-  if (dual) return launch_gemm_tiles_t<DT, true, 2, 2, 64>(a, st, who);
+  // Forms by tile count, for what the other two tiled kernels leave (mfma_mid.hip: about one tile per compute unit; mfma_big.hip:
+  // many), measured on the projections of the 7B shape at 128..4096 rows.  The pair reaches this kernel with few tiles, or
+  // with operands of 4 GiB and more.  A single matrix: 128 x 128 from 448 big tiles on, 128 x 64 from 256 on, else 64 x 64 —
+  // in K steps of 64 with a deep register pipeline when there are more of those than the chip holds at once (320), in
+  // steps of 128 (half as many barriers) when there are fewer: with one workgroup or less per compute unit and a long K
+  // only loads issued several steps ahead hide the latency.
+  if (dual) return big >= 512 ? launch_gemm_tiles_t<DT, true, 4, 4, 64, 8, 2, true>(a, st, who) : launch_gemm_tiles_t<DT, true, 2, 2, 64>(a, st, who);
   // a single matrix with more than one big tile per compute unit: loads straight into LDS, two stages (the second and
   // third workgroup of a compute unit cover the one-step load distance; 5..8 % faster than the register pipeline with
   // weights that come from HBM, and slower than it below these tile counts)
   if (big >= 448) return launch_gemm_tiles_t<DT, false, 4, 4, 64, 4, -2>(a, st, who);
   if (big >= 320) return launch_gemm_tiles_t<DT, false, 4, 2, 64, 4, -2>(a, st, who);
-  // about one tile per compute unit: eight waves on a 128 x 128 or 128 x 64 tile, each half of them on half of the k
-  // slices of a step, so that a workgroup alone on its compute unit still runs two waves per SIMD (rank projections at
-  // 512 rows 36 -> 29 us, at 1024 rows 50 -> 43; down_v at 2048 rows 131 -> 109; with fewer tiles than ~0.6 per
-  // compute unit the 64 x 64 tiles below win, with more the four-wave forms that share a compute unit)
-  if (big >= 144 && big <= 256) return launch_gemm_tiles_t<DT, false, 4, 4, 64, 8>(a, st, who);
+  // K of 8192 and more with about one 128 x 64 tile per compute unit: eight waves, each half of them on half of the k slices
+  // of a step, so that a workgroup alone on its compute unit still runs two waves per SIMD (1536 x 11008 at 1024 rows 72 us,
+  // three stages of loads straight into LDS 73)
   if (big >= 256) return launch_gemm_tiles_t<DT, false, 4, 2, 64>(a, st, who);
   const int64_t half = (int64_t)((a.N + 63) / 64) * ((a.B + 127) / 128);
   if (half >= 160 && half <= 256 && (a.K % 128) == 0) return launch_gemm_tiles_t<DT, false, 4, 2, 128, 8>(a, st, who);
@@ -674,27 +656,23 @@ int launch_gemm_ragged(const MfmaArgs& a, bool dual, hipStream_t st, const char*
   return a.dt == 1 ? launch_gemm_ragged_dt<1>(a, dual, st, who) : launch_gemm_ragged_dt<0>(a, dual, st, who);
 }
 
-// head expansion of the prefill on the tiled kernel: 128 token rows and more, head_dim 128, rank a multiple of 64,
-// coefficients shared by the heads
-static bool expand_aligned(const ExpandArgs& a) {
-  return (a.R % kGBK) == 0 && (a.sp_b % 8) == 0 && (a.sp_m % 8) == 0 && (a.ldu % 8) == 0 && at16(a.p) && at16(a.u);
-}
+// Head expansions that neither mfma_big.hip nor mfma_mid.hip takes: head_dim 128, coefficients shared by the heads,
 // any rank and rows that start anywhere, from 16 token rows on (q, k and v of 32 heads at rank 1024: one launch of 13.7 to
 // 16 us at 16 to 64 rows, three launches of one wave per 32 rows and head 80 to 95 us)
 bool expand_tiles_apply(const ExpandArgs& a) {
   return a.Dh == 128 && a.R > 0 && a.heads > 0 && a.sp_h == 0 && (int64_t)a.B * a.M >= 16;
 }
 
-template <int DT, int WTM, bool RAG>
+template <int DT, int WTM>
 static int launch_expand_tiles_t(const ExpandArgs& a, hipStream_t st) {
   const char* who = "fsvd_lowrank_expand_heads";
   static bool granted = false;
-  constexpr int PF = 2;   // register pipeline (loads straight into LDS were slower here: 0.92 -> 1.03 ms at 8 x 2048 rows)
+  constexpr int PF = 2;
   constexpr int kGLd = kGBK;
   constexpr int BM = 32 * WTM;
   const size_t lds = (size_t)2 * (BM + 128) * kGLd * 2;
   if (!granted) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_tiles_kernel<DT, false, WTM, 4, PF, true, kGBK, 4, RAG>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_tiles_kernel<DT, false, WTM, 4, PF, true, kGBK, 4, true>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) { set_last_error("%s: cannot reserve %zu bytes of LDS: %s", who, lds, hipGetErrorString(e)); return kErrLaunch; }
     granted = true;
@@ -703,20 +681,20 @@ static int launch_expand_tiles_t(const ExpandArgs& a, hipStream_t st) {
   MfmaArgs g{a.p, 0, 0, a.u, nullptr, a.ldu, a.bias, nullptr, 0, a.y, 0, rows, a.heads * 128, a.R, 0};
   ExpandEpi ep{a.cos, a.sin, a.rope_len, a.positions, a.M, a.sp_b, a.sp_m, a.sy_b, a.sy_m, a.sy_h, a.dst_by_position, a.dst_rows};
   const dim3 grid(a.heads, (rows + BM - 1) / BM);
-  hipLaunchKernelGGL((gemm_tiles_kernel<DT, false, WTM, 4, PF, true, kGBK, 4, RAG>), grid, dim3(kGT4), lds, st, g, ep);
+  hipLaunchKernelGGL((gemm_tiles_kernel<DT, false, WTM, 4, PF, true, kGBK, 4, true>), grid, dim3(kGT4), lds, st, g, ep);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }
   return kOk;
 }
 
-template <int DT, int WTM, bool RAG>
+template <int DT, int WTM>
 static int launch_expand_multi_t(const ExpandArgs* d, int n, hipStream_t st) {
   const char* who = "fsvd_lowrank_expand_heads_multi";
   static bool granted = false;
   constexpr int BM = 32 * WTM;
   const size_t lds = (size_t)2 * (BM + 128) * kGBK * 2;
   if (!granted) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&expand_multi_kernel<DT, WTM, RAG>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&expand_multi_kernel<DT, WTM>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) { set_last_error("%s: cannot reserve %zu bytes of LDS: %s", who, lds, hipGetErrorString(e)); return kErrLaunch; }
     granted = true;
   }
@@ -733,7 +711,7 @@ static int launch_expand_multi_t(const ExpandArgs* d, int n, hipStream_t st) {
   eb.first_head[3] = heads;
   for (int k = n; k < 3; ++k) eb.first_head[k] = heads;    // unused sets start past the last head
   const dim3 grid(heads, (rows + BM - 1) / BM);
-  hipLaunchKernelGGL((expand_multi_kernel<DT, WTM, RAG>), grid, dim3(kGT4), lds, st, eb);
+  hipLaunchKernelGGL((expand_multi_kernel<DT, WTM>), grid, dim3(kGT4), lds, st, eb);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }
   return kOk;
@@ -746,30 +724,23 @@ bool expand_multi_apply(const ExpandArgs* d, int n) {
     if (!expand_tiles_apply(d[k]) || d[k].B != d[0].B || d[k].M != d[0].M || d[k].dt != d[0].dt) return false;
   return true;
 }
-template <int DT>
-static int launch_expand_multi_dt(const ExpandArgs* d, int n, bool aligned, bool wide, hipStream_t st) {
-  if (!aligned) return wide ? launch_expand_multi_t<DT, 4, true>(d, n, st) : launch_expand_multi_t<DT, 2, true>(d, n, st);
-  return wide ? launch_expand_multi_t<DT, 4, false>(d, n, st) : launch_expand_multi_t<DT, 2, false>(d, n, st);
-}
 int launch_expand_multi(const ExpandArgs* d, int n, hipStream_t st) {
   if (expand_big_apply(d, n)) return launch_expand_big(d, n, st);
+  if (expand_mid_apply(d, n)) return launch_expand_mid(d, n, st);
   int heads = 0;
-  bool aligned = true;
-  for (int k = 0; k < n; ++k) { heads += d[k].heads; aligned = aligned && expand_aligned(d[k]); }
+  for (int k = 0; k < n; ++k) heads += d[k].heads;
   const bool wide = (int64_t)heads * (((int64_t)d[0].B * d[0].M + 127) / 128) >= 384;
-  return d[0].dt == 1 ? launch_expand_multi_dt<1>(d, n, aligned, wide, st) : launch_expand_multi_dt<0>(d, n, aligned, wide, st);
+  if (d[0].dt == 1) return wide ? launch_expand_multi_t<1, 4>(d, n, st) : launch_expand_multi_t<1, 2>(d, n, st);
+  return wide ? launch_expand_multi_t<0, 4>(d, n, st) : launch_expand_multi_t<0, 2>(d, n, st);
 }
 
-template <int DT>
-static int launch_expand_tiles_dt(const ExpandArgs& a, bool wide, hipStream_t st) {
-  if (!expand_aligned(a)) return wide ? launch_expand_tiles_t<DT, 4, true>(a, st) : launch_expand_tiles_t<DT, 2, true>(a, st);
-  return wide ? launch_expand_tiles_t<DT, 4, false>(a, st) : launch_expand_tiles_t<DT, 2, false>(a, st);
-}
 int launch_expand_tiles(const ExpandArgs& a, hipStream_t st) {
   if (expand_big_apply(&a, 1)) return launch_expand_big(&a, 1, st);
+  if (expand_mid_apply(&a, 1)) return launch_expand_mid(&a, 1, st);
   // a column tile is always one head; 128 token rows per workgroup when that gives every compute unit two tiles, else 64
   const bool wide = (int64_t)a.heads * (((int64_t)a.B * a.M + 127) / 128) >= 384;
-  return a.dt == 1 ? launch_expand_tiles_dt<1>(a, wide, st) : launch_expand_tiles_dt<0>(a, wide, st);
+  if (a.dt == 1) return wide ? launch_expand_tiles_t<1, 4>(a, st) : launch_expand_tiles_t<1, 2>(a, st);
+  return wide ? launch_expand_tiles_t<0, 4>(a, st) : launch_expand_tiles_t<0, 2>(a, st);
 }
 
 }  // namespace fsvd

@@ -772,6 +772,7 @@ static int launch_mfma(const MfmaArgs& a0, hipStream_t st, const char* who) {
     return kOk;
   }
   // many rows (prefill): the tiled kernel reads every weight once per 128 rows instead of once per 64
+  if (gemm_mid_apply(a0, DUAL)) return launch_gemm_mid(a0, DUAL, st, who);
   if (gemm_big_apply(a0, DUAL)) return launch_gemm_big(a0, DUAL, st, who);
   if (gemm_tiles_apply(a0)) return launch_gemm_tiles(a0, DUAL, st, who);
   // a batch of rows: 32-row tiles with K split over workgroups, when the caller has registered a workspace — from 33
