@@ -17,7 +17,7 @@ def dtype_code(t: torch.Tensor) -> int:
 
 
 def stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def scratch(device: torch.device, nbytes: int, tag: str) -> torch.Tensor:

@@ -127,9 +127,10 @@ def _run_fast(p_up_2d, p_gate_2d, GateU, UpU, DownV, DownU, b2):
     else:
         p = torch.cat([p_gate_2d, p_up_2d], dim=1)
     gate_u, up_u = linear_layout_of(GateU), linear_layout_of(UpU)          # [D, R]
-    h = hip_ops.swiglu_linear(p, gate_u, up_u, up_off=R, mode=1)           # h = round(silu(g32) * u32), dual_split_triton.py:207
-    s = hip_ops.linear(h, linear_layout_of(DownV))                        # S: fp32 sum over D, one rounding (:719-720)
-    return hip_ops.linear(s, linear_layout_of(DownU), None if b2 is None else b2.to(s.dtype).contiguous())
+    # inside the operator flashsvd_hip::mlp_dual_split: its steps do not go through the dispatcher again
+    h = hip_ops._swiglu_linear_impl(p, gate_u, up_u, R, 1, None, 0)        # h = round(silu(g32) * u32), dual_split_triton.py:207
+    s = hip_ops._linear_impl(h, linear_layout_of(DownV), None, None, 0.0, None, None, 0)       # S: fp32 sum over D, one rounding (:719-720)
+    return hip_ops._linear_impl(s, linear_layout_of(DownU), None if b2 is None else b2.to(s.dtype).contiguous(), None, 0.0, None, None, 0)
 
 
 def _run_impl(p_up_2d, p_gate_2d, GateU, UpU, DownV, DownU, b2, variant, BD, partials_fp32, s_out):
