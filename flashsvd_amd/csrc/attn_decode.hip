@@ -31,6 +31,42 @@ __device__ __forceinline__ void decode_work_item(int B, int H, int nsplit, int& 
 __device__ __forceinline__ void st_agent(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ float ld_agent(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
+// dimensions d and d + half of the new row of (b, hk): k_new rotated at position pos (fp32 math, one rounding), v_new as it is
+template <int DT, class Args>
+__device__ __forceinline__ void append_pair(const Args& a, int half, int b, int hk, int pos, int d) {
+  typedef E16<DT> E;
+  const uint16_t* kp = a.k_new + (int64_t)b * a.sk_b + (int64_t)hk * a.sk_h;
+  const uint16_t* vp = a.v_new + (int64_t)b * a.sv_b + (int64_t)hk * a.sv_h;
+  float x0 = E::val(kp[d]), x1 = E::val(kp[d + half]);
+  if (a.cos) {
+    const int tp = min(pos, a.rope_len - 1);
+    const float c = E::val(a.cos[(int64_t)tp * half + d]);
+    const float s = E::val(a.sin[(int64_t)tp * half + d]);
+    const float r0 = x0 * c - x1 * s, r1 = x0 * s + x1 * c;
+    x0 = r0; x1 = r1;
+  }
+  const int64_t off = (int64_t)b * a.sc_b + (int64_t)pos * a.sc_s + (int64_t)hk * a.sc_h;
+  uint16_t* kc = const_cast<uint16_t*>(a.k_cache) + off;
+  uint16_t* vc = const_cast<uint16_t*>(a.v_cache) + off;
+  kc[d] = (uint16_t)E::bits(x0);
+  kc[d + half] = (uint16_t)E::bits(x1);
+  vc[d] = vp[d];
+  vc[d + half] = vp[d + half];
+}
+
+// The new row of a sequence is its last key: the workgroup whose keys [k0, k1) end with it writes it before it reads them.
+// Only where no other workgroup reads the row (append_in_kernel).  Against a launch of its own for the append: 16 sequences of
+// up to 4001 keys, 32 heads over 8, 53.5 -> 50.1 us, 64 x 1000 49.8 -> 48.0, 16 x 1000 with 32 kv heads 49.6 -> 46.9.
+template <int DT, int DH>
+__device__ __forceinline__ void append_own_row(const AttnDecodeArgs& a, int b, int hk, int k0, int k1) {
+  if (a.k_new == nullptr) return;
+  const int pos = a.seqlens[b];
+  if (pos < k0 || pos >= k1) return;               // the same for the whole workgroup; k1 <= S
+  if (threadIdx.x < DH / 2) append_pair<DT>(a, DH / 2, b, hk, pos, threadIdx.x);
+  wait_stores_acked();
+  __syncthreads();
+}
+
 template <int DT, int DH, int U>
 __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArgs a) {
   typedef E16<DT> E;
@@ -52,6 +88,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
   per = (per + KPB - 1) / KPB * KPB;
   const int k0 = min(s * per, n_keys);
   const int k1 = min(n_keys, k0 + per);
+  append_own_row<DT, DH>(a, b, hk, k0, k1);
 
   // query chunk (optionally rotated at position seqlens[b], fp32 math, one rounding)
   const uint16_t* qp = a.q + (int64_t)b * a.sq_b + (int64_t)h * a.sq_h;
@@ -199,8 +236,8 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
 // At two workgroups per compute unit the vector work of G heads (about 900 instructions per wave and pass) is as long as
 // the loads, so the two run at the same time: the K rows of a pass are replaced by the next pass's as soon as they are
 // scored, the V rows as soon as they are added up.  The heads leave together: one fold through LDS, one arrival, one merge
-// (head by head it was four hand-offs in a row).  Same bits.  With the append launch, 32 query heads over 8 kv heads: 16 x
-// up to 4001 keys 61.4 -> 53.5 us (4.3 TB/s), 64 x 1000 52.9 -> 49.8, 40 x 1500 68.1 -> 65.1.
+// (head by head it was four hand-offs in a row).  Same bits.  With an append launch before it, 32 query heads over 8 kv heads:
+// 16 x up to 4001 keys 61.4 -> 53.5 us (4.3 TB/s), 64 x 1000 52.9 -> 49.8, 40 x 1500 68.1 -> 65.1.
 template <int DT, int DH, int U, int G>
 __global__ __launch_bounds__(kAttnThreads) void attn_decode_gqa_kernel(AttnDecodeArgs a) {
   typedef E16<DT> E;
@@ -221,6 +258,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_gqa_kernel(AttnDecod
   per = (per + KPB - 1) / KPB * KPB;
   const int k0 = min(s * per, n_keys);
   const int k1 = min(n_keys, k0 + per);
+  append_own_row<DT, DH>(a, b, hk, k0, k1);
 
   if (tid < G * (DH / 2)) {
     const int g = tid / (DH / 2), d = tid % (DH / 2);
@@ -401,31 +439,16 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_gqa_kernel(AttnDecod
   if (tid == 0) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// rotate k_new at position seqlens[b] (fp32 math, one rounding) and write k/v into the caches
+// the appends of a call whose rows more than one workgroup reads
 template <int DT>
 __global__ __launch_bounds__(256) void kv_append_kernel(KvAppendArgs a) {
-  typedef E16<DT> E;
   const int half = a.Dh >> 1;
   const int total = a.B * a.Hk * half;
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
     const int d = i % half, hk = (i / half) % a.Hk, b = i / (half * a.Hk);
     const int pos = a.seqlens[b];
     if (pos < 0 || pos >= a.S) continue;
-    const uint16_t* kp = a.k_new + (int64_t)b * a.sk_b + (int64_t)hk * a.sk_h;
-    const uint16_t* vp = a.v_new + (int64_t)b * a.sv_b + (int64_t)hk * a.sv_h;
-    float x0 = E::val(kp[d]), x1 = E::val(kp[d + half]);
-    if (a.cos) {
-      const int tp = min(pos, a.rope_len - 1);
-      const float c = E::val(a.cos[(int64_t)tp * half + d]);
-      const float s = E::val(a.sin[(int64_t)tp * half + d]);
-      const float r0 = x0 * c - x1 * s, r1 = x0 * s + x1 * c;
-      x0 = r0; x1 = r1;
-    }
-    const int64_t off = (int64_t)b * a.sc_b + (int64_t)pos * a.sc_s + (int64_t)hk * a.sc_h;
-    a.k_cache[off + d] = (uint16_t)E::bits(x0);
-    a.k_cache[off + d + half] = (uint16_t)E::bits(x1);
-    a.v_cache[off + d] = vp[d];
-    a.v_cache[off + d + half] = vp[d + half];
+    append_pair<DT>(a, half, b, hk, pos, d);
   }
 }
 
@@ -440,7 +463,15 @@ static void launch_attn_decode_t(const AttnDecodeArgs& a, int G, hipStream_t st)
   else hipLaunchKernelGGL((attn_decode_kernel<DT, 64, 4>), grid, dim3(kAttnThreads), 0, st, a);
 }
 
-int launch_attn_decode(const AttnDecodeArgs& a, hipStream_t st) {
+// true when the appended row of (b, hk) is read by one workgroup alone: all query heads of the kv head in one workgroup, and
+// cache rows of different sequences and heads that do not overlap (sequences bound to one cache row see each other's new
+// tokens, which takes a launch before this one)
+static bool append_in_kernel(const AttnDecodeArgs& a, int G) {
+  return a.H / a.Hk == G && a.sc_h >= a.Dh && a.sc_s >= (a.Hk - 1) * a.sc_h + a.Dh && (a.B == 1 || a.sc_b >= a.S * a.sc_s);
+}
+
+int launch_attn_decode(const AttnDecodeArgs& args, hipStream_t st) {
+  AttnDecodeArgs a = args;
   if (a.dt != 0 && a.dt != 1) { set_last_error("fsvd_attn_decode_densekv: dtype code %d (bf16 = 0 and fp16 = 1 are served)", a.dt); return kErrBadDtype; }
   if (a.B <= 0 || a.H <= 0 || a.Hk <= 0 || a.H % a.Hk != 0 || a.S <= 0 || a.nsplit <= 0) {
     set_last_error("fsvd_attn_decode_densekv: bad shape B=%d H=%d Hk=%d S=%d nsplit=%d", a.B, a.H, a.Hk, a.S, a.nsplit);
@@ -466,6 +497,13 @@ int launch_attn_decode(const AttnDecodeArgs& a, hipStream_t st) {
   if (a.Dh == 128) {
     if (rep % 4 == 0 && (int64_t)a.B * (a.H / 4) * a.nsplit >= 512) G = 4;
     else if (rep % 2 == 0 && (int64_t)a.B * (a.H / 2) * a.nsplit >= 512) G = 2;
+  }
+  if (a.k_new && !append_in_kernel(a, G)) {
+    const KvAppendArgs ka{a.k_new, a.v_new, a.sk_b, a.sk_h, a.sv_b, a.sv_h, const_cast<uint16_t*>(a.k_cache), const_cast<uint16_t*>(a.v_cache),
+                          a.sc_b, a.sc_s, a.sc_h, a.seqlens, a.cos, a.sin, a.rope_len, a.B, a.Hk, a.Dh, a.S, a.dt};
+    const int rc = launch_kv_append(ka, st);
+    if (rc != kOk) return rc;
+    a.k_new = nullptr;
   }
   if (a.dt == 1) launch_attn_decode_t<1>(a, G, st);
   else launch_attn_decode_t<0>(a, G, st);

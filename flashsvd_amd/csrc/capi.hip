@@ -201,16 +201,9 @@ int fsvd_attn_decode_densekv(const void* q, int64_t sq_b, int64_t sq_h, void* k_
     ws_count = static_cast<int32_t*>(workspace);
     ws_part = reinterpret_cast<float*>(static_cast<char*>(workspace) + kAttnCounterBytes);
   }
-  if (k_new) {
-    KvAppendArgs ka{cu16(k_new), cu16(v_new), sk_b, sk_h, sv_b, sv_h, u16(k_cache), u16(v_cache), sc_b, sc_s, sc_h,
-                    cache_seqlens, cu16(cos), cu16(sin), rope_len, B, Hk, Dh, S, dtype};
-    int rc = launch_kv_append(ka, st);
-    if (rc != kOk) return rc;
-    seqlen_add = 1;
-  }
-  AttnDecodeArgs a{cu16(q), sq_b, sq_h, cu16(k_cache), cu16(v_cache), sc_b, sc_s, sc_h, cache_seqlens, seqlen_add,
+  AttnDecodeArgs a{cu16(q), sq_b, sq_h, cu16(k_cache), cu16(v_cache), sc_b, sc_s, sc_h, cache_seqlens, k_new ? 1 : seqlen_add,
                    cu16(cos), cu16(sin), rope_len, u16(out), so_b, so_h, ws_part, ws_count, B, H, Hk, Dh, S, nsplit,
-                   scale > 0.f ? scale : 1.0f / sqrtf((float)Dh), dtype};
+                   scale > 0.f ? scale : 1.0f / sqrtf((float)Dh), dtype, cu16(k_new), cu16(v_new), sk_b, sk_h, sv_b, sv_h};
   return launch_attn_decode(a, st);
 }
 

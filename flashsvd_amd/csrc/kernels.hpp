@@ -61,6 +61,9 @@ struct AttnDecodeArgs {
   int B, H, Hk, Dh, S, nsplit;
   float scale;
   int dt = 0;
+  // rows to append at position seqlens[b], [B, Hk, Dh] (seqlen_add is 1 then)
+  const uint16_t* k_new = nullptr; const uint16_t* v_new = nullptr;
+  int64_t sk_b = 0, sk_h = 0, sv_b = 0, sv_h = 0;
 };
 
 struct KvAppendArgs {

@@ -45,3 +45,52 @@ def test_grouped_decode_attention(ops, dtype, B, H, Hk, nsplit, lens):
             assert_close_bf16(out[b], _reference(q[b], kc[b], vc[b], n), f"sequence {b}, {n} keys")
         else:
             assert torch.all(out[b] == 0)
+
+
+def _pair_of_caches(B, S, Hk, dtype):
+    """The same values with the rows of a token together (a workgroup may append its own row) and with the rows of a head
+    together (the append is a launch of its own)."""
+    kc, vc = (rand_bf16(B, S, Hk, 128, seed=i).to(dtype).cuda() for i in (3, 4))
+    return (kc, vc), tuple(t.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3) for t in (kc, vc))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,Hk,nsplit,lens", [(2, 8, 8, 1, (0, 128)), (3, 16, 16, 4, (63, 64, 300)), (16, 32, 8, 4, (0, 1, 127, 128, 511, 512, 400)),
+                                                (64, 32, 8, 1, (0, 15, 128, 255)), (16, 32, 16, 2, (31, 32, 33, 256)), (32, 16, 2, 4, (5, 64, 130)),
+                                                (1, 32, 8, 3, (47,))])
+@pytest.mark.parametrize("rotate", [True, False])
+def test_append_in_the_attention_launch(ops, dtype, B, H, Hk, nsplit, lens, rotate):
+    """New rows at split and pass borders, at the first and the last row of the cache and past its end (dropped): the caches
+    and results are those of an append launched before the attention, bit for bit."""
+    S = max(lens) + 1
+    lens = torch.tensor([lens[b % len(lens)] for b in range(B)], dtype=torch.int32)
+    if B > 2:
+        lens[-1] = S                                            # no room: nothing is written, all S rows are attended to
+    cos, sin = (rand_bf16(S + 1, 64, seed=i).to(dtype).cuda() for i in (6, 7)) if rotate else (None, None)
+    q, kn, vn = (rand_bf16(B, h, 128, seed=i).to(dtype).cuda() for i, h in ((0, H), (1, Hk), (2, Hk)))
+    results = []
+    for kc, vc in _pair_of_caches(B, S, Hk, dtype):
+        for _ in range(2):                                      # a second call finds the row there already
+            out = ops.attn_decode_densekv(q, kc, vc, lens.cuda(), k_new=kn, v_new=vn, cos=cos, sin=sin, nsplit=nsplit)
+        results.append((out, kc, vc))
+    for got, want in zip(*results):
+        assert torch.equal(got, want)
+    if not rotate:
+        for b in range(min(B, 4)):
+            n = min(int(lens[b]) + 1, S)
+            if lens[b] < S:
+                assert torch.equal(results[0][1][b, n - 1], kn[b]) and torch.equal(results[0][2][b, n - 1], vn[b])
+            kc, vc = (t[b].cpu() for t in results[0][1:])
+            assert_close_bf16(results[0][0][b], _reference(q[b].cpu(), kc, vc, n), f"sequence {b}")
+
+
+def test_sequences_bound_to_one_cache_row_see_each_other(ops):
+    """Three tokens of one sequence as three batch rows over one cache: each attends to the rows that the others append."""
+    H, S, n = 8, 64, 20
+    kc, vc = (rand_bf16(1, S, H, 128, seed=i).cuda() for i in (3, 4))
+    q, kn, vn = (rand_bf16(3, H, 128, seed=i).cuda() for i in (0, 1, 2))
+    lens = torch.tensor([n, n + 1, n + 2], dtype=torch.int32).cuda()
+    out = ops.attn_decode_densekv(q, kc.expand(3, S, H, 128), vc.expand(3, S, H, 128), lens, k_new=kn, v_new=vn, nsplit=2)
+    assert torch.equal(kc[0, n:n + 3], kn) and torch.equal(vc[0, n:n + 3], vn)
+    for b in range(3):
+        assert_close_bf16(out[b], _reference(q[b].cpu(), kc[0].cpu(), vc[0].cpu(), n + 1 + b), f"token {b}")
