@@ -40,7 +40,7 @@ constexpr int kGBK = 64;            // K per step (the small tile takes 128 when
 // RAG: rows that start anywhere and any K, not only whole steps of aligned rows -- the ranks that a parameter ratio
 // leaves (1492, 1638, ...).  The pieces of a row are still one 16-byte load each: the hardware takes them at any element's
 // address.  The K steps that are whole run as they do otherwise; what is left of K is one more step behind the loop, its
-// pieces masked to the row (zero past its end), so nothing is read outside the operands.
+// pieces masked to the row (zero past its end), so nothing is read outside the operands.  Never split over workgroups.
 template <int DT, bool DUAL, int WTM, int WT, int PF, bool EXPAND, int BK, int NW, bool RAG = false>
 __device__ __forceinline__ void gemm_tiles_body(const MfmaArgs& a, const ExpandEpi& ep, const int tile_m, const int tile_n) {
   typedef E16<DT> E;
@@ -76,10 +76,10 @@ __device__ __forceinline__ void gemm_tiles_body(const MfmaArgs& a, const ExpandE
   const int m0 = tile_m * kGBM, n0 = tile_n * kGBN;
   // this workgroup's share of the K steps (all of them unless K is split over gridDim.z)
   const int ksteps_all = a.K / BK;
-  const int kper = (ksteps_all + (int)gridDim.z - 1) / (int)gridDim.z;
-  const int kbeg = min((int)blockIdx.z * kper, ksteps_all);
-  // a share past the end re-reads the last step and adds zero (ragged: it walks no step)
-  const int ksteps = max(RAG ? 0 : 1, min(kper, ksteps_all - kbeg));
+  const int kper = RAG ? ksteps_all : (ksteps_all + (int)gridDim.z - 1) / (int)gridDim.z;
+  const int kbeg = RAG ? 0 : min((int)blockIdx.z * kper, ksteps_all);
+  // a share past the end re-reads the last step and adds zero (ragged: a short K has no whole step)
+  const int ksteps = RAG ? ksteps_all : max(1, min(kper, ksteps_all - kbeg));
   const bool kdead = kbeg >= ksteps_all;
 
   // global -> register staging: a tile row is CPR 16-byte pieces; NP pieces per thread and operand
@@ -243,8 +243,8 @@ __device__ __forceinline__ void gemm_tiles_body(const MfmaArgs& a, const ExpandE
     }
   }
 
-  // what is left of K behind the whole steps, taken by the last share
-  if (RAG && a.K % BK != 0 && blockIdx.z == gridDim.z - 1) {
+  // what is left of K behind the whole steps
+  if (RAG && a.K % BK != 0) {
     const int k = ksteps_all * BK, left = a.K - k - g_chunk * 8;     // elements of the row from this thread's piece on
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
@@ -296,7 +296,7 @@ __device__ __forceinline__ void gemm_tiles_body(const MfmaArgs& a, const ExpandE
   const bool writer = !KHALF || mat == 0;   // waves 4-7 of the halved form keep the barriers below company and store nothing
   // K split: park the partial tile (thread-major 16-byte words, coalesced), count arrivals; the last workgroup of a
   // tile adds all partials in split order (its own included, so the sum does not depend on who came last)
-  if (WTM <= 2 && gridDim.z > 1) {         // only the 32- and 64-row tiles are ever launched with a split
+  if (!RAG && WTM <= 2 && gridDim.z > 1) { // only the 32- and 64-row tiles are ever launched with a split
     constexpr int WPT = NMA * WTM * WT;                          // 16-byte words per thread
     const int tile = blockIdx.y * gridDim.x + blockIdx.x;
     gm_f32x4_t* part = reinterpret_cast<gm_f32x4_t*>(a.ws_part) + (size_t)tile * gridDim.z * WPT * kGT;
@@ -311,7 +311,7 @@ __device__ __forceinline__ void gemm_tiles_body(const MfmaArgs& a, const ExpandE
 #pragma unroll
         for (int j = 0; j < WT; ++j) {
           if (!writer) break;
-          const gm_f32x4_t v = !RAG && kdead ? gm_f32x4_t{0.f, 0.f, 0.f, 0.f} : acc[m][i][j];
+          const gm_f32x4_t v = kdead ? gm_f32x4_t{0.f, 0.f, 0.f, 0.f} : acc[m][i][j];
           unsigned long long* dst = reinterpret_cast<unsigned long long*>(mine + ((m * WTM + i) * WT + j) * kGT + tid);
           __hip_atomic_store(dst, ((unsigned long long)__float_as_uint(v[1]) << 32) | __float_as_uint(v[0]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           __hip_atomic_store(dst + 1, ((unsigned long long)__float_as_uint(v[3]) << 32) | __float_as_uint(v[2]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -574,8 +574,10 @@ static int launch_gemm_tiles_t(const MfmaArgs& a0, hipStream_t st, const char* w
   const SplitWorkspace ws = split_workspace();
   constexpr size_t share = (size_t)(DUAL && NW == 4 ? 2 : 1) * WTM * WT * 4 * NW * 64;   // floats one workgroup parks
   // the 32-row tiles split K whenever that fills the chip; 64 x 64 prompt tiles only where measured to pay; larger
-  // tiles never (parking and re-reading the partial tiles costs what the extra workgroups gain)
-  if (WTM == 1) a.ksplit = pick_ksplit((int64_t)grid.x * grid.y, a.K / BK, share, ws);
+  // tiles never (parking and re-reading the partial tiles costs what the extra workgroups gain), ragged rows never (calls
+  // that need no workspace stay independent of the stream they run on)
+  if (RAG) a.ksplit = 1;
+  else if (WTM == 1) a.ksplit = pick_ksplit((int64_t)grid.x * grid.y, a.K / BK, share, ws);
   else if (WTM == 2 && !DUAL) a.ksplit = pick_ksplit_prompt((int64_t)grid.x * grid.y, a.K / BK, a.K, share, ws);
   else a.ksplit = 1;
   a.ws_part = ws.part;
@@ -645,12 +647,20 @@ bool gemm_ragged_apply(const MfmaArgs& a) {
   if (a.B < 3) return false;
   return !aligned_rows(a) || (a.K % (a.B > 32 ? kGBK : 32)) != 0;
 }
+// Forms without a split over workgroups: with up to about one 32 x 64 tile per compute unit the K steps of 128 are halved between
+// two groups of waves.  us with weights from HBM, such tiles in steps of 64 by four waves / these: 4096 x 1492 at 33, 64, 127
+// rows 12.7 / 11.1, 13.6 / 12.0, 13.4 / 11.7, 1492 x 4104 27.4 / 19.4, 28.9 / 21.7, 28.1 / 21.0, 64 x 64 tiles alike: 4096 x 1492 at
+// 333, 500 rows 21.5 / 19.9, 23.7 / 22.0, 1492 x 4104 26.4 / 22.8, 32.5 / 26.1.  The pair at 3, 16, 64, 127 rows: 11008 x 1492
+// 24.7, 27.1, 43.4, 55.1 (with a split over three workgroups, which has to park partial tiles, 33.1, 34.6, 41.0, 54.8).
 template <int DT>
 static int launch_gemm_ragged_dt(const MfmaArgs& a, bool dual, hipStream_t st, const char* who) {
-  if (a.B < 128) return dual ? launch_gemm_tiles_t<DT, true, 1, 2, 64, 4, 2, true>(a, st, who) : launch_gemm_tiles_t<DT, false, 1, 2, 64, 4, 2, true>(a, st, who);
   const int64_t big = (int64_t)((a.N + 127) / 128) * ((a.B + 127) / 128);
-  if (dual) return big >= 512 ? launch_gemm_tiles_t<DT, true, 4, 4, 64, 8, 2, true>(a, st, who) : launch_gemm_tiles_t<DT, true, 2, 2, 64, 4, 2, true>(a, st, who);
-  return big >= 256 ? launch_gemm_tiles_t<DT, false, 4, 4, 64, 4, 2, true>(a, st, who) : launch_gemm_tiles_t<DT, false, 2, 2, 64, 4, 4, true>(a, st, who);
+  if (dual) {
+    if (a.B < 128) return launch_gemm_tiles_t<DT, true, 1, 2, 64, 4, 2, true>(a, st, who);
+    return big >= 512 ? launch_gemm_tiles_t<DT, true, 4, 4, 64, 8, 2, true>(a, st, who) : launch_gemm_tiles_t<DT, true, 2, 2, 64, 4, 2, true>(a, st, who);
+  }
+  if ((int64_t)((a.N + 63) / 64) * ((a.B + 31) / 32) <= 256) return launch_gemm_tiles_t<DT, false, 1, 2, 128, 8, 2, true>(a, st, who);
+  return big >= 256 ? launch_gemm_tiles_t<DT, false, 4, 4, 64, 4, 2, true>(a, st, who) : launch_gemm_tiles_t<DT, false, 2, 2, 128, 8, 2, true>(a, st, who);
 }
 int launch_gemm_ragged(const MfmaArgs& a, bool dual, hipStream_t st, const char* who) {
   return a.dt == 1 ? launch_gemm_ragged_dt<1>(a, dual, st, who) : launch_gemm_ragged_dt<0>(a, dual, st, who);

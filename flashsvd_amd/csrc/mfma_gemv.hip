@@ -181,10 +181,15 @@ __global__ __launch_bounds__(kMfThreads) void mfma_linear_kernel(MfmaArgs a) {
     for (int j = 0; j < UN; ++j) {
       const int k = (min(s + j, s1 - 1) * KS + ks) << 5;
       if (RAG) {
-        static_assert(!RAG || (!DUAL && NB == 1), "the ragged form is built for up to 16 rows of a single matrix");
         const int left = a.K - k - lg * 8;
         fa0[j] = masked ? __builtin_bit_cast(frag_t, load_masked_piece(w0 + k, left, a.K)) : ld_any_frag<frag_t, true>(w0 + k);
-        fb0[j][0] = masked ? __builtin_bit_cast(frag_t, load_masked_piece(xr[0] + k, left, a.K)) : ld_any_frag<frag_t, false>(xr[0] + k);
+        if (DUAL) fa1[j] = masked ? __builtin_bit_cast(frag_t, load_masked_piece(w1 + k, left, a.K)) : ld_any_frag<frag_t, true>(w1 + k);
+#pragma unroll
+        for (int t = 0; t < NB; ++t) {
+          const uint16_t* x0 = xr[t] + k;
+          fb0[j][t] = masked ? __builtin_bit_cast(frag_t, load_masked_piece(x0, left, a.K)) : ld_any_frag<frag_t, false>(x0);
+          if (DUAL) fb1[j][t] = masked ? __builtin_bit_cast(frag_t, load_masked_piece(x0 + a.up_off, left, a.K)) : ld_any_frag<frag_t, false>(x0 + a.up_off);
+        }
         continue;
       }
       fa0[j] = ldw_frag<frag_t>(w0 + k);
@@ -753,6 +758,17 @@ static int launch_mfma_stream_split(const MfmaArgs& a0, int z, hipStream_t st, c
   return kOk;
 }
 
+// Ragged rows, up to 32 of them, on a workgroup per 16 weight rows (K split over its eight waves): single matrices of fewer
+// than 8192 rows, and pairs of up to 4096 and a rank of 512 and more.  us with weights from HBM, here / on the tiles of
+// mfma_gemm.hip, at 3, 16, 17, 32 rows: 4096 x 1492 8.2 / 11.1, 9.4 / 11.6, 10.3 / 11.6, 12.1 / 12.3; 1492 x 4104 10.8 / 19.5,
+// 13.5 / 20.8, 15.2 / 20.8, 19.0 / 22.6; 11008 x 1001 12.9 / 10.5, 16.6 / 11.9, 18.7 / 11.0, 23.6 / 11.6; the pair 4096 x 1001
+// 13.5 / 17.4, 15.1 / 17.6, 17.5 / 17.8, 19.3 / 19.2, 5504 x 746 14.7 / 13.5, 17.3 / 13.9, 24.4 / 14.0, 1376 x 375 10.7 / 9.1.
+template <bool DUAL>
+static bool ragged_waves_apply(const MfmaArgs& a) {
+  if (a.B > 32) return false;
+  return DUAL ? a.N <= 4096 && a.K >= 512 : a.N < 8192;
+}
+
 template <int DT, bool DUAL>
 static int launch_mfma(const MfmaArgs& a0, hipStream_t st, const char* who) {
   // K is split over as few waves as still give every compute unit a workgroup: long slices amortise the
@@ -761,12 +777,11 @@ static int launch_mfma(const MfmaArgs& a0, hipStream_t st, const char* who) {
   int ks = 8;
   for (int c = 2; c <= 8; c *= 2)
     if ((tiles * c + 7) / 8 >= 256 && ksteps / c >= 4) { ks = c; break; }
-  // any K, rows that start anywhere: the tiled kernel, except that up to 16 rows of a single matrix run here (4096 x 1492 at
-  // 4 / 16 rows 8.5 / 9.7 us against 11.0 / 11.3; at 23 rows 11.5 both; the gate / up pair 11008 x 1492 at 4 / 16 rows is
-  // 36 / 43 us here and 35 / 36 there)
+  // any K, rows that start anywhere: in the kernel above without a workspace, or on tiles that are never split
   if (gemm_ragged_apply(a0)) {
-    if (DUAL || a0.B > 16) return launch_gemm_ragged(a0, DUAL, st, who);
-    launch_mfma_ks<DT, 1, false, true>(a0, 8, st);
+    if (!ragged_waves_apply<DUAL>(a0)) return launch_gemm_ragged(a0, DUAL, st, who);
+    if (a0.B <= 16) launch_mfma_ks<DT, 1, DUAL, true>(a0, 8, st);
+    else launch_mfma_ks<DT, 2, DUAL, true>(a0, 8, st);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }
     return kOk;

@@ -75,8 +75,8 @@ _SPLIT_WS_MAX = 1 << 30
 
 
 def ensure_split_workspace(device: torch.device, min_bytes: int = 0) -> bool:
-    """Register, once per device, the scratch the library's K-split projections (3..127 rows) work in.  The library
-    allocates nothing itself; this hands it 64 MiB of torch memory, or ``min_bytes`` rounded up to a power of two (up to
+    """Register, once per device, the scratch the library's K-split projections (three rows and more, K a multiple of 64 and
+    rows on the 16-byte grid; others run without it) work in.  The library allocates nothing itself; this hands it 64 MiB of torch memory, or ``min_bytes`` rounded up to a power of two (up to
     1 GiB) when a caller needs more: a larger buffer then replaces the registered one (a doubling each time at least, so
     a growing demand costs a logarithmic number of replacements), and the old one is kept alive until
     ``release_split_workspace`` because graphs captured earlier hold its address.  ``FLASHSVD_AMD_SPLITK=0`` keeps the

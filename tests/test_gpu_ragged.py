@@ -69,3 +69,53 @@ def test_head_expansion_any_rank(B, T, R):
     q2 = torch.zeros_like(q)
     hip_ops.lowrank_expand_heads(pc[..., :R], qu.cuda(), num_heads=H, out=q2, **kw)
     assert torch.equal(q, q2)
+
+
+# pairs and single matrices of 3 to 500 rows, from less than one K step to a long K; every form that ragged rows take
+_INDEPENDENT = [("pair", 4, 11008, 1492), ("pair", 40, 5504, 746), ("pair", 20, 2048, 1001), ("pair", 130, 1376, 375),
+                ("single", 5, 1492, 4104), ("single", 30, 100, 4000), ("single", 40, 1536, 4100), ("single", 100, 515, 1492),
+                ("single", 128, 1000, 2050), ("single", 200, 300, 8200), ("single", 500, 1492, 4104)]
+
+
+def _ragged_call(kind, B, N, K, seed):
+    from flashsvd_amd import hip_ops
+    if kind == "pair":
+        p, gu, uu = rand_bf16(B, 2 * K, seed=seed).cuda(), rand_bf16(N, K, std=K ** -0.5, seed=seed + 1).cuda(), rand_bf16(N, K, std=K ** -0.5, seed=seed + 2).cuda()
+        return lambda: hip_ops.swiglu_linear(p, gu, uu, up_off=K)
+    x, w = rand_bf16(B, K, seed=seed).cuda(), rand_bf16(N, K, std=K ** -0.5, seed=seed + 1).cuda()
+    return lambda: hip_ops.linear(x, w)
+
+
+@pytest.mark.parametrize("kind,B,N,K", _INDEPENDENT)
+def test_ragged_rows_leave_the_shared_workspace_alone(kind, B, N, K):
+    """One workspace serves a device, so whatever uses it is bound to one stream; ragged rows do not use it."""
+    from flashsvd_amd import hip_ops
+    assert hip_ops.ensure_split_workspace(torch.device("cuda", 0))
+    ws = hip_ops._SPLIT_WS[0]
+    call = _ragged_call(kind, B, N, K, seed=1)
+    torch.cuda.synchronize()
+    partials = ws[64 << 10:]                            # behind the arrival counters, which are zero between calls
+    partials.fill_(0x5a)
+    call()
+    torch.cuda.synchronize()
+    untouched, at_rest = int((partials != 0x5a).sum()) == 0, int(ws[:64 << 10].sum()) == 0
+    assert untouched and at_rest
+
+
+def test_ragged_rows_on_two_streams():
+    """The same projections issued on two streams at once give the bits that each gives alone."""
+    calls = [_ragged_call(*c, seed=10 * i) for i, c in enumerate(_INDEPENDENT)]
+    alone = [c() for c in calls]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for _ in range(5):
+        got = [[], []]
+        for i in range(len(calls)):
+            for s, st in enumerate(streams):            # the two streams are at different calls at any time
+                with torch.cuda.stream(st):
+                    j = (i + s * 3) % len(calls)
+                    got[s].append((j, calls[j]()))
+        torch.cuda.synchronize()
+        for s in range(2):
+            for j, y in got[s]:
+                assert torch.equal(y, alone[j]), f"{_INDEPENDENT[j]} on stream {s}"
