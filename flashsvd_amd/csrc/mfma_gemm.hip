@@ -608,6 +608,8 @@ static int launch_gemm_tiles_dt(const MfmaArgs& a, bool dual, hipStream_t st, co
   // of a step, so that a workgroup alone on its compute unit still runs two waves per SIMD (1536 x 11008 at 1024 rows 72 us,
   // three stages of loads straight into LDS 73)
   if (big >= 256) return launch_gemm_tiles_t<DT, false, 4, 2, 64>(a, st, who);
+  // mfma_mid.hip takes these where its 32-bit offsets reach; operands past them stay on unsplit 128 x 128 tiles
+  if (big >= 144) return launch_gemm_tiles_t<DT, false, 4, 4, 64, 4, 2, true>(a, st, who);
   const int64_t half = (int64_t)((a.N + 63) / 64) * ((a.B + 127) / 128);
   if (half >= 160 && half <= 256 && (a.K % 128) == 0) return launch_gemm_tiles_t<DT, false, 4, 2, 128, 8>(a, st, who);
   const int64_t small = (int64_t)((a.N + 63) / 64) * ((a.B + 63) / 64);
