@@ -96,6 +96,7 @@ WBITS_Q4_FP16 = -4
 SIGNATURES = {
     "fsvd_version": (c_int, []),
     "fsvd_last_error": (c_char_p, []),
+    "fsvd_last_form": (c_char_p, []),
     "fsvd_linear": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_float, c_void_p, c_int64,
                             c_void_p, c_int64, c_int, c_int, c_int, c_int, c_int, c_void_p]),
     "fsvd_linear_rankkv_append": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_float, c_void_p, c_int64, c_int, c_int, c_int, c_int,

@@ -11,6 +11,8 @@
 
 namespace fsvd {
 static thread_local char g_last_error[512] = "";
+static thread_local const char* g_last_form = "";
+void set_last_form(const char* name) { g_last_form = name; }
 void set_last_error(const char* fmt, ...) {
   va_list ap;
   va_start(ap, fmt);
@@ -50,6 +52,7 @@ extern "C" {
 
 int fsvd_version(void) { return 102; }
 const char* fsvd_last_error(void) { return g_last_error; }
+const char* fsvd_last_form(void) { return g_last_form; }
 
 int fsvd_set_workspace(void* ws, size_t bytes, void* stream) {
   const char* fn = "fsvd_set_workspace";

@@ -20,6 +20,7 @@ enum Status : int {
 };
 
 void set_last_error(const char* fmt, ...);
+void set_last_form(const char* name);   // of static storage: what fsvd_last_form() reports
 
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));

@@ -596,6 +596,7 @@ int launch_linear(const LinearArgs& a, int cfg, hipStream_t st) {
     return launch_linear_mfma(a, st);
   }
   if (a.K > 32768) { set_last_error("fsvd_linear: K=%d exceeds the 32768 LDS staging limit", a.K); return kErrBadShape; }
+  set_last_form("vector");
   return a.dt == 1 ? launch_linear_t<1>(a, cfg, st) : launch_linear_t<0>(a, cfg, st);
 }
 
@@ -637,6 +638,7 @@ int launch_swiglu(const SwigluArgs& a, int cfg, hipStream_t st) {
   if (a.dt != 0 && a.dt != 1) { set_last_error("fsvd_swiglu_linear: dtype code %d (bf16 = 0 and fp16 = 1 are served)", a.dt); return kErrBadDtype; }
   if (cfg == 0 && mfma_swiglu_applies(a)) return launch_swiglu_mfma(a, st);
   if (a.R > 16384) { set_last_error("fsvd_swiglu_linear: R=%d exceeds 16384", a.R); return kErrBadShape; }
+  set_last_form("vector pair");
   return a.dt == 1 ? launch_swiglu_t<1>(a, cfg, st) : launch_swiglu_t<0>(a, cfg, st);
 }
 
@@ -710,6 +712,7 @@ int launch_qkv(const QkvArgs& a, int cfg, hipStream_t st) {
   // the tiled head expansion with one token per row takes the other batches: more tokens, or ranks and rows off the grid
   // (64 tokens at rank 1024 206 -> 16 us, 4 tokens at rank 1001 30 -> 20 us)
   if (cfg == 0 && a.B >= 3 && a.Dh == 128) return launch_qkv_tiles(a, st);
+  set_last_form("vector q k v");
   return a.dt == 1 ? launch_qkv_t<1>(a, cfg, st) : launch_qkv_t<0>(a, cfg, st);
 }
 

@@ -356,6 +356,7 @@ static int launch_big_t(const BigArgs& a, hipStream_t st, const char* who) {
     granted = true;
   }
   const int tiles = a.nt * ((a.rows + kBigT - 1) / kBigT);
+  set_last_form(EPI == kBigPair ? "256 x 256 pair" : (EPI == kBigHeads ? "256 x 256 heads" : "256 x 256"));
   hipLaunchKernelGGL((gemm_big_kernel<DT, EPI>), dim3(std::min(tiles, compute_units())), dim3(kBigThreads), lds, st, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }

@@ -13,6 +13,7 @@
 // head expansion of the prompt pass (RoPE, store into the query buffer or the cache rows).  Few tiles or a very long K:
 // K split over workgroups, partial tiles added in a fixed order by the last arrival.
 #include <algorithm>
+#include <string>
 #include <type_traits>
 
 #include "common.hpp"
@@ -583,6 +584,8 @@ static int launch_gemm_tiles_t(const MfmaArgs& a0, hipStream_t st, const char* w
   a.ws_part = ws.part;
   a.ws_count = ws.count;
   grid.z = a.ksplit;
+  static const std::string form = (RAG ? "any rows " : "tiles ") + std::to_string(BM) + " x " + std::to_string(BN) + (DUAL ? " pair" : "");
+  set_last_form(form.c_str());
   hipLaunchKernelGGL((gemm_tiles_kernel<DT, DUAL, WTM, WT, PF, false, BK, NW, RAG>), grid, dim3(NW * 64), lds, st, a, ExpandEpi{});
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }
@@ -693,6 +696,7 @@ static int launch_expand_tiles_t(const ExpandArgs& a, hipStream_t st) {
   MfmaArgs g{a.p, 0, 0, a.u, nullptr, a.ldu, a.bias, nullptr, 0, a.y, 0, rows, a.heads * 128, a.R, 0};
   ExpandEpi ep{a.cos, a.sin, a.rope_len, a.positions, a.M, a.sp_b, a.sp_m, a.sy_b, a.sy_m, a.sy_h, a.dst_by_position, a.dst_rows};
   const dim3 grid(a.heads, (rows + BM - 1) / BM);
+  set_last_form(WTM == 4 ? "tiles 128 x 128 heads" : "tiles 64 x 128 heads");
   hipLaunchKernelGGL((gemm_tiles_kernel<DT, false, WTM, 4, PF, true, kGBK, 4, true>), grid, dim3(kGT4), lds, st, g, ep);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }
@@ -723,6 +727,7 @@ static int launch_expand_multi_t(const ExpandArgs* d, int n, hipStream_t st) {
   eb.first_head[3] = heads;
   for (int k = n; k < 3; ++k) eb.first_head[k] = heads;    // unused sets start past the last head
   const dim3 grid(heads, (rows + BM - 1) / BM);
+  set_last_form(WTM == 4 ? "tiles 128 x 128 heads" : "tiles 64 x 128 heads");
   hipLaunchKernelGGL((expand_multi_kernel<DT, WTM>), grid, dim3(kGT4), lds, st, eb);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }

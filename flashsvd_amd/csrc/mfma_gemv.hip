@@ -651,6 +651,7 @@ static int launch_mfma_resident_t(const MfmaArgs& a, hipStream_t st, const char*
     granted = true;
   }
   const int G = std::min(compute_units(), (a.N + 15) / 16);
+  set_last_form(DUAL ? "resident pair" : "resident");
   hipLaunchKernelGGL((mfma_resident_kernel<DT, DUAL, NB, CW, D>), dim3(G), dim3(kMfThreads), lds, st, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }
@@ -672,6 +673,7 @@ template <int DT, int NB, bool DUAL, bool RAG = false>
 static void launch_mfma_ks(const MfmaArgs& a, int ks, hipStream_t st) {
   const int tiles = (a.N + 15) / 16;
   const dim3 block(kMfThreads);
+  set_last_form(RAG ? (DUAL ? "any rows 16 pair" : "any rows 16") : (DUAL ? "rows 16 pair" : "rows 16"));
   if (RAG) hipLaunchKernelGGL((mfma_linear_kernel<DT, NB, DUAL, 8, RAG>), dim3(tiles), block, 0, st, a);
   else if (ks == 2) hipLaunchKernelGGL((mfma_linear_kernel<DT, NB, DUAL, 2>), dim3((tiles + 3) / 4), block, 0, st, a);
   else if (ks == 4) hipLaunchKernelGGL((mfma_linear_kernel<DT, NB, DUAL, 4>), dim3((tiles + 1) / 2), block, 0, st, a);
@@ -696,6 +698,7 @@ static int launch_mfma_stream_d(const MfmaArgs& a, int ks, hipStream_t st, const
     return granted[i] = true;
   };
   const dim3 block(kMfThreads);
+  set_last_form(DUAL ? "stream pair" : "stream");
   if (ks == 2) {
     if (!grant(reinterpret_cast<const void*>(&mfma_stream_kernel<DT, DUAL, 2, D, NB>), 0)) return kErrLaunch;
     hipLaunchKernelGGL((mfma_stream_kernel<DT, DUAL, 2, D, NB>), dim3((tiles + 3) / 4), block, lds, st, a);
@@ -752,6 +755,7 @@ static int launch_mfma_stream_split(const MfmaArgs& a0, int z, hipStream_t st, c
   a.ksplit = z;
   a.ws_part = ws.part;
   a.ws_count = ws.count;
+  set_last_form("stream split");
   hipLaunchKernelGGL((mfma_stream_kernel<DT, false, 8, D, NB, true>), dim3((a.N + 15) / 16, z), dim3(kMfThreads), lds, st, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }
@@ -839,6 +843,7 @@ static int launch_qkv_mfma_t(const QkvArgs& a, hipStream_t st) {
       granted = true;
     }
   }
+  set_last_form("stream q k v");
   hipLaunchKernelGGL((mfma_qkv_kernel<DT, NB>), dim3((a.H + 2 * a.Hk) * (a.Dh / 32)), dim3(kMfThreads), lds, st, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }

@@ -14,6 +14,7 @@
 // of every 128 of K and hand their sums to waves 0-3 through LDS at the end; sums run over K in the order of the forms of
 // mfma_gemm.hip.  The gate / up pair runs its two products one after the other over the same tile.
 #include <algorithm>
+#include <string>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -286,6 +287,8 @@ static int launch_mid_t(MidArgs& m, hipStream_t st, const char* who) {
   }
   if (EPI != kMidHeads) m.nt = (m.a[0].N + BN - 1) / BN;
   const int64_t tiles = (int64_t)m.nt * ((m.a[0].B + BM - 1) / BM);
+  static const std::string form = "ring " + std::to_string(BM) + " x " + std::to_string(BN) + (EPI == kMidPair ? " pair" : (EPI == kMidHeads ? " heads" : ""));
+  set_last_form(form.c_str());
   hipLaunchKernelGGL((gemm_mid_kernel<DT, EPI, WM, WN, TM, TN, KH, NS>), dim3((unsigned)tiles), dim3(kMidThreads), lds, st, m);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }

@@ -456,6 +456,7 @@ int launch_expand(const ExpandArgs& a, hipStream_t st) {
     return kErrBadAlign;
   }
   const int T = a.B * a.M;
+  set_last_form("rows 128 heads");
   if (a.dt == 1) hipLaunchKernelGGL(lowrank_expand_kernel<1>, dim3((T + 127) / 128, a.heads), dim3(kPfThreads), 0, st, a);
   else hipLaunchKernelGGL(lowrank_expand_kernel<0>, dim3((T + 127) / 128, a.heads), dim3(kPfThreads), 0, st, a);
   hipError_t e = hipGetLastError();

@@ -38,6 +38,9 @@ extern "C" {
 
 int fsvd_version(void);
 const char* fsvd_last_error(void);
+/* Which kernel form the last projection, gate / up pair, q / k / v expansion or head expansion that this thread issued took
+ * ("256 x 256 pair", "ring 128 x 64", "vector", ...): for tests and measurements; the names are no part of the interface. */
+const char* fsvd_last_form(void);
 
 /* Optional scratch for the projections (fsvd_linear, fsvd_swiglu_linear) of 17..127 rows, of 3..16 rows when the matrix has
  * fewer than 2048 rows, and of 128 rows and more where a single matrix has few output tiles or K >= 8192, each for K a

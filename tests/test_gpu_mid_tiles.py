@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from tests.test_gpu_big_tiles import _check, _rand
+from tests.util import form_taken
 
 pytestmark = pytest.mark.gpu
 
@@ -72,3 +73,29 @@ def test_head_expansion(B, T, H, Hk, R):
         n = min(T, k.shape[1] - s0)
         _check(k[b, s0:s0 + n], rope((p[b, :, R:].float() @ ku.float().t()).bfloat16().view(T, Hk, Dh))[:n], f"k of row {b}")
         assert not k[b, :s0].any()
+
+
+# every tiling by name, each with a partial last row and column tile
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,N,K,form", [(200, 4035, 256, "ring 64 x 64"), (333, 3077, 128, "ring 128 x 64"), (1000, 4009, 192, "ring 128 x 128")])
+def test_linear_forms(B, N, K, form, dtype):
+    from flashsvd_amd import hip_ops
+    x, w = _rand(B, K, seed=1, dtype=dtype), _rand(N, K, std=K ** -0.5, seed=2, dtype=dtype)
+    bias, res = _rand(N, seed=3, dtype=dtype), _rand(B, N, seed=4, dtype=dtype)
+    y = hip_ops.linear(x, w, bias, residual=res)
+    assert form_taken() == form
+    _check(y, (((x.float() @ w.float().t()) + bias.float()).to(dtype).float() + res.float()).to(dtype), form)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,D,R,form", [(333, 11005, 128, "ring 128 x 192 pair"), (154, 11005, 192, "ring 64 x 192 pair")])
+def test_pair_forms(B, D, R, form, dtype):
+    from flashsvd_amd import hip_ops
+    p = _rand(B, 2 * R, seed=1, dtype=dtype)
+    gu, uu = _rand(D, R, std=R ** -0.5, seed=2, dtype=dtype), _rand(D, R, std=R ** -0.5, seed=3, dtype=dtype)
+    g, u = p[:, :R].float() @ gu.float().t(), p[:, R:].float() @ uu.float().t()
+    for mode in (0, 1):
+        ref = torch.nn.functional.silu(g.to(dtype)) * u.to(dtype) if mode == 0 else ((g * torch.sigmoid(g)) * u).to(dtype)
+        h = hip_ops.swiglu_linear(p, gu, uu, up_off=R, mode=mode)
+        assert form_taken() == form
+        _check(h, ref, f"mode {mode}")

@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from oracle import flashsvd_oracle as O
-from tests.util import assert_close_bf16, bounds, rand_bf16
+from tests.util import assert_close_bf16, bounds, form_taken, rand_bf16
 
 pytestmark = pytest.mark.gpu
 
@@ -39,3 +39,25 @@ def test_qkv_batch(B, H, Hk, Dh, Rq, Rk, Rv, rope):
         kc[b, at[b]] = 0
         vc[b, at[b]] = 0
     assert not kc.any() and not vc.any()                 # nothing else in the caches was touched
+
+
+@pytest.mark.parametrize("B,H,Hk,Dh,R,form", [
+    (3, 4, 2, 128, 64, "stream q k v"), (17, 4, 4, 64, 576, "stream q k v"), (33, 2, 2, 128, 128, "ring 64 x 128 heads"),
+    (5, 2, 2, 128, 65, "tiles 64 x 128 heads"), (4, 2, 2, 64, 100, "vector q k v")])
+def test_qkv_batch_float16(B, H, Hk, Dh, R, form):
+    from flashsvd_amd import hip_ops
+    from tests.test_gpu_ragged import _close16, _rand16
+    S = 50
+    p = _rand16(B, 3 * R, seed=1)
+    qu, ku, vu = (_rand16(h * Dh, R, std=R ** -0.5, seed=2 + i) for i, h in enumerate((H, Hk, Hk)))
+    cos, sin = O.rope_tables(S, Dh, dtype=torch.float16)
+    pos = torch.tensor([(7 * b + 5) % S for b in range(B)], dtype=torch.int32)
+    kc, vc = (torch.zeros(B, S, Hk, Dh, dtype=torch.float16, device="cuda") for _ in range(2))
+    q = hip_ops.qkv_rope_append(p.cuda(), qu.cuda(), ku.cuda(), vu.cuda(), cos.cuda(), sin.cuda(), pos.cuda(), kc, vc,
+                                num_heads=H, num_kv_heads=Hk, head_dim=Dh)
+    assert form_taken() == form
+    at, rows = pos.long(), torch.arange(B)
+    rot = lambda x: O.apply_rope(x, cos[at][:, None], sin[at][:, None])
+    _close16(q, rot(O.lin(p[:, :R], qu).view(B, H, Dh)), "q")
+    _close16(kc.cpu()[rows, at], rot(O.lin(p[:, R:2 * R], ku).view(B, Hk, Dh)), "k rows")
+    _close16(vc.cpu()[rows, at], O.lin(p[:, 2 * R:], vu).view(B, Hk, Dh), "v rows")

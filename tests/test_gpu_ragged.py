@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from oracle import flashsvd_oracle as O
-from tests.util import assert_close_bf16, bounds, rand_bf16
+from tests.util import assert_close_bf16, bounds, form_taken, rand_bf16
 
 pytestmark = pytest.mark.gpu
 
@@ -119,3 +119,76 @@ def test_ragged_rows_on_two_streams():
         for s in range(2):
             for j, y in got[s]:
                 assert torch.equal(y, alone[j]), f"{_INDEPENDENT[j]} on stream {s}"
+
+
+def _rand16(*shape, std=1.0, seed=0):
+    return (torch.randn(*shape, generator=torch.Generator().manual_seed(seed), dtype=torch.float32) * std).to(torch.float16)
+
+
+def _close16(got, ref, what):
+    """A quarter of the bf16 bounds: float16 has three more mantissa bits (two of its ulps where max|ref| is 2 and more)."""
+    m = float(ref.float().abs().max())
+    assert got.dtype == torch.float16
+    assert_close_bf16(got, ref, what, abs_tol=5e-3 if m < 2.0 else 2.0 * m * 2.0 ** -10, rel_tol=2.5e-3)
+
+
+@pytest.mark.parametrize("B,N,K,form", [
+    (16, 4097, 1492, "any rows 16"), (31, 4097, 1003, "any rows 16"), (12, 8200, 333, "any rows 32 x 64"), (100, 3970, 1492, "any rows 32 x 64"),
+    (500, 4097, 333, "any rows 64 x 64"), (1030, 4096, 130, "any rows 128 x 128")])
+def test_linear_forms(B, N, K, form):
+    """Every form that ragged rows of a single matrix take, in both element types."""
+    from flashsvd_amd import hip_ops
+    for rand, close in ((rand_bf16, lambda y, r, w: assert_close_bf16(y, r, w, **bounds(r))), (_rand16, _close16)):
+        x, w, bias, res = rand(B, K, seed=1), rand(N, K, std=K ** -0.5, seed=2), rand(N, seed=3), rand(B, N, seed=4)
+        y = hip_ops.linear(x.cuda(), w.cuda(), bias.cuda(), residual=res.cuda())
+        assert form_taken() == form
+        close(y, res + O.lin(x, w, bias), form)
+
+
+@pytest.mark.parametrize("B,D,R,form", [
+    (16, 1000, 517, "any rows 16 pair"), (30, 4090, 517, "any rows 16 pair"), (33, 1000, 517, "any rows 32 x 64 pair"), (5, 5000, 130, "any rows 32 x 64 pair"),
+    (200, 4090, 67, "any rows 64 x 64 pair"), (1040, 8200, 67, "any rows 128 x 128 pair")])
+def test_pair_forms(B, D, R, form):
+    from flashsvd_amd import hip_ops
+    for rand, close in ((rand_bf16, lambda y, r, w: assert_close_bf16(y, r, w, **bounds(r))), (_rand16, _close16)):
+        p, gu, uu = rand(B, 2 * R, seed=1), rand(D, R, std=R ** -0.5, seed=2), rand(D, R, std=R ** -0.5, seed=3)
+        g, u = p[:, :R].float() @ gu.float().t(), p[:, R:].float() @ uu.float().t()
+        for mode in (0, 1):
+            ref = torch.nn.functional.silu(g.to(p.dtype)) * u.to(p.dtype) if mode == 0 else ((g * torch.sigmoid(g)) * u).to(p.dtype)
+            h = hip_ops.swiglu_linear(p.cuda(), gu.cuda(), uu.cuda(), up_off=R, mode=mode)
+            assert form_taken() == form
+            close(h, ref, f"{form}, mode {mode}")
+
+
+@pytest.mark.parametrize("B,K", [(3, 33), (5, 262), (40, 1001), (150, 100), (9, 4104)])
+def test_norm_in_front_of_a_ragged_projection(B, K):
+    """RMSNorm with its own rounding in front of a projection whose K is no multiple of 32."""
+    from flashsvd_amd import hip_ops
+    for rand, close in ((rand_bf16, lambda y, r, w: assert_close_bf16(y, r, w, **bounds(r))), (_rand16, _close16)):
+        x, w, nw = rand(B, K, seed=1), rand(300, K, std=K ** -0.5, seed=2), rand(K, seed=3) * 0.1 + 1
+        y = hip_ops.linear(x.cuda(), w.cuda(), norm_weight=nw.cuda(), eps=1e-6)
+        close(y, O.lin(O.rms_norm(x, nw, 1e-6), w), f"{B} x {K}")
+
+
+def test_longest_rows():
+    """K past what the vector kernels stage in LDS."""
+    from flashsvd_amd import hip_ops
+    x, w = rand_bf16(3, 33001, seed=1), rand_bf16(20, 33001, std=33001 ** -0.5, seed=2)
+    ref = O.lin(x, w)
+    assert_close_bf16(hip_ops.linear(x.cuda(), w.cuda()), ref, "linear", **bounds(ref))
+
+
+@pytest.mark.parametrize("B,T,R", [(2, 37, 52), (1, 333, 65)])
+def test_head_expansion_any_rank_float16(B, T, R):
+    from flashsvd_amd import hip_ops
+    H, Hk, Dh = 4, 2, 128
+    p, qu, vu = _rand16(B, T, 2 * R, seed=1), _rand16(H * Dh, R, std=R ** -0.5, seed=2), _rand16(Hk * Dh, R, std=R ** -0.5, seed=3)
+    cos, sin = O.rope_tables(T + 9, Dh, dtype=torch.float16)
+    q, v = torch.zeros(B, T, H, Dh, dtype=torch.float16, device="cuda"), torch.zeros(B, T + 9, Hk, Dh, dtype=torch.float16, device="cuda")
+    pc = p.cuda()
+    hip_ops.lowrank_expand_heads_multi([dict(p=pc[..., :R], u=qu.cuda(), num_heads=H, out=q, rotate=True),
+                                        dict(p=pc[..., R:], u=vu.cuda(), num_heads=Hk, out=v, dst_by_position=True)],
+                                       head_dim=Dh, cos=cos.cuda(), sin=sin.cuda(), positions=torch.full((B,), 9, dtype=torch.int32, device="cuda"))
+    assert form_taken() == "tiles 64 x 128 heads"
+    _close16(q, O.apply_rope(O.lin(p[..., :R], qu).view(B, T, H, Dh), cos[9:, None], sin[9:, None]), "q")
+    _close16(v[:, 9:], O.lin(p[..., R:], vu).view(B, T, Hk, Dh), "v")

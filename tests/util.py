@@ -58,3 +58,9 @@ def bounds(ref):
     1.5e-2, so the absolute bound becomes two ulps at max|ref|."""
     m = float(ref.float().abs().max())
     return dict(abs_tol=2e-2 if m < 2.0 else 2.0 * m * 2.0 ** -7, rel_tol=1e-2)
+
+
+def form_taken():
+    """The kernel form that the last projection or head expansion of this thread took (fsvd_last_form)."""
+    from flashsvd_amd import _lib
+    return _lib.load().fsvd_last_form().decode()
