@@ -559,6 +559,7 @@ int fsvd_lowrank_expand_heads_multi(const fsvd_expand_desc* desc, int n, const v
   const char* fn = "fsvd_lowrank_expand_heads_multi";
   FSVD_REQUIRE_PTR(desc, fn);
   if (n < 1 || n > 3) { set_last_error("%s: %d descriptors (1..3)", fn, n); return kErrBadShape; }
+  if (dtype != 0 && dtype != 1) { set_last_error("%s: dtype code %d (bf16 = 0 and fp16 = 1 are served)", fn, dtype); return kErrBadDtype; }
   if ((cos == nullptr) != (sin == nullptr) || (cos && rope_len <= 0)) { set_last_error("%s: cos/sin must both be set with rope_len > 0", fn); return kErrBadShape; }
   ExpandArgs a[3];
   for (int k = 0; k < n; ++k) {

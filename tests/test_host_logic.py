@@ -45,6 +45,21 @@ def test_null_pointer_and_shape_errors_come_back_as_status_codes():
         _lib.check("fsvd_linear", -1)
 
 
+@pytest.mark.parametrize("tokens", [1, 16, 200])
+def test_expansions_of_one_call_refuse_other_element_types(tokens):
+    """FSVD_FP32 is no type of the head expansions, whatever kernel the token count would select."""
+    from flashsvd_amd import _lib
+    lib = _lib.load()
+    buf = ctypes.create_string_buffer(64)  # never dereferenced: the type check comes first
+    p = ctypes.addressof(buf)
+    descs = (_lib.ExpandDesc * 2)()
+    for d in descs:
+        d.p, d.sp_b, d.sp_m, d.u, d.ldu, d.y, d.sy_b, d.sy_m, d.sy_h = p, 64 * tokens, 64, p, 64, p, 256 * tokens, 256, 128
+        d.heads, d.R, d.dst_rows = 2, 64, tokens
+    rc = lib.fsvd_lowrank_expand_heads_multi(descs, 2, None, None, 0, None, 1, tokens, 128, 2, None)
+    assert rc == -3 and b"dtype code 2" in lib.fsvd_last_error()
+
+
 # ------------------------------------------------------------------ runtime flags
 def test_configure_runtime_flashsvd_snapshot():
     from flashsvd_amd import api
