@@ -671,11 +671,13 @@ int launch_gemm_ragged(const MfmaArgs& a, bool dual, hipStream_t st, const char*
   return a.dt == 1 ? launch_gemm_ragged_dt<1>(a, dual, st, who) : launch_gemm_ragged_dt<0>(a, dual, st, who);
 }
 
-// Head expansions that neither mfma_big.hip nor mfma_mid.hip takes: head_dim 128, coefficients shared by the heads,
-// any rank and rows that start anywhere, from 16 token rows on (q, k and v of 32 heads at rank 1024: one launch of 13.7 to
-// 16 us at 16 to 64 rows, three launches of one wave per 32 rows and head 80 to 95 us)
+// Head expansions of head_dim 128 whose coefficients the heads share, at any rank and with rows that start anywhere: from 16
+// token rows on (q, k and v of 32 heads at rank 1024: one launch of 13.7 to 16 us at 16 to 64 rows, three launches of one wave
+// per 32 rows and head 80 to 95 us), and with fewer rows where lowrank_expand_kernel cannot take them, so that a rank or an
+// address is accepted or refused alike at every row count.
 bool expand_tiles_apply(const ExpandArgs& a) {
-  return a.Dh == 128 && a.R > 0 && a.heads > 0 && a.sp_h == 0 && (int64_t)a.B * a.M >= 16;
+  const bool on_grid = a.R % 8 == 0 && a.sp_b % 8 == 0 && a.sp_m % 8 == 0 && a.ldu % 8 == 0 && at16(a.p) && at16(a.u);
+  return a.Dh == 128 && a.R > 0 && a.heads > 0 && a.B > 0 && a.M > 0 && a.sp_h == 0 && ((int64_t)a.B * a.M >= 16 || !on_grid);
 }
 
 template <int DT, int WTM>

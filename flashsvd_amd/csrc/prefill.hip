@@ -448,8 +448,8 @@ int launch_expand(const ExpandArgs& a, hipStream_t st) {
   if (a.dt != 0 && a.dt != 1) { set_last_error("%s: dtype code %d (bf16 = 0 and fp16 = 1 are served)", fn, a.dt); return kErrBadDtype; }
   if (a.B <= 0 || a.M <= 0 || a.heads <= 0 || a.R <= 0) { set_last_error("%s: empty shape", fn); return kErrBadShape; }
   if (a.Dh != 128) { set_last_error("%s: head_dim %d is not 128", fn, a.Dh); return kErrBadShape; }
-  if (expand_tiles_apply(a)) return launch_expand_tiles(a, st);   // the LDS-tiled kernel: long prompts, ranks and rows off the 16-byte grid
-  if (a.R % 8) { set_last_error("%s: rank %d is not a multiple of 8; pad the factors", fn, a.R); return kErrBadShape; }
+  if (expand_tiles_apply(a)) return launch_expand_tiles(a, st);   // the LDS-tiled kernels
+  if (a.R % 8) { set_last_error("%s: rank %d is not a multiple of 8 (coefficients of their own per head); pad the factors", fn, a.R); return kErrBadShape; }
   const auto mis = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) != 0; };
   if (mis(a.p) || mis(a.u) || (a.sp_b % 8) || (a.sp_m % 8) || (a.sp_h % 8) || (a.ldu % 8)) {
     set_last_error("%s: coefficient / factor pointers and strides must be 16-byte aligned", fn);

@@ -267,7 +267,8 @@ int fsvd_rankkv_append(const void* pk, int64_t ldpk, const void* pv, int64_t ldp
  *   stored at row = m (dst_by_position = 0: a query buffer [B,M,H,Dh]) or row = positions[b]+m
  *   (dst_by_position = 1: the dense KV cache [B,S,Hk,Dh]; rows outside [0,dst_rows) are dropped).
  *   P is [B,M,heads,R] with sp_h = 0 for coefficients shared by all heads; u is the nn.Linear-layout
- *   u_proj weight [heads*Dh, R] (per-head basis V[h][r][d] = u[h*Dh+d][r]).  bf16, Dh = 128, R % 8 == 0.
+ *   u_proj weight [heads*Dh, R] (per-head basis V[h][r][d] = u[h*Dh+d][r]).  Dh = 128.  With sp_h = 0 any R and rows that
+ *   start anywhere; coefficients per head (sp_h != 0) take R % 8 == 0 and pointers and strides on the 16-byte grid.
  *
  * fsvd_attn_prefill: out[b,m,h,:] = softmax_n(q[b,m,h,:] . k[b,n,hk,:] * scale + masks) v[b,n,hk,:]
  *   over keys n < q_pos0[b] + M, causal (n <= q_pos0[b] + m) when causal != 0; pad_mask [B,keys] (0 =
@@ -279,8 +280,8 @@ int fsvd_lowrank_expand_heads(const void* p, int64_t sp_b, int64_t sp_m, int64_t
                               int B, int M, int heads, int Dh, int R, int dtype, void* stream);
 /* The q, k and v expansions of one prompt pass in one call: the same results as `n` calls of
  * fsvd_lowrank_expand_heads on the same token rows (one per descriptor; `rotate` selects whether that one gets the
- * rotation), and a single launch when every one of them takes the tiled kernel (128 token rows and more, rank a
- * multiple of 64, coefficients shared by the heads).  The reference computes all three inside one kernel as well
+ * rotation), and a single launch when every one of them takes the tiled kernels (coefficients shared by the heads, 16
+ * token rows and more, or a rank or rows off the 16-byte grid).  The reference computes all three inside one kernel as well
  * (rope_sdpa.py:67-248 takes Pq/Vq, Pk/Vk, Pv/Vv together).  n = 1..3. */
 typedef struct fsvd_expand_desc {
   const void* p; int64_t sp_b, sp_m, sp_h;   /* rank coefficients [B,M,(heads),R] */

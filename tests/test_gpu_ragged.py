@@ -46,7 +46,7 @@ def test_swiglu_any_rank(B, D, R, mode):
     assert_close_bf16(h, ref, f"swiglu {B}x{D}x{R}", **bounds(ref))
 
 
-@pytest.mark.parametrize("B,T,R", [(1, 16, 1), (2, 37, 52), (1, 130, 1638), (2, 333, 65)])
+@pytest.mark.parametrize("B,T,R", [(1, 16, 1), (2, 37, 52), (1, 130, 1638), (2, 333, 65), (1, 1, 52), (1, 15, 52), (3, 4, 65)])
 def test_head_expansion_any_rank(B, T, R):
     """q with the rotation and v without, as one launch and as two, at positions behind a cached prefix."""
     from flashsvd_amd import hip_ops
