@@ -534,7 +534,6 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_vec_kernel(const uint16_t* _
 // ---------------------------------------------------------------------------------------
 // host-side launchers
 // ---------------------------------------------------------------------------------------
-static inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 #define FSVD_CHECK_LAUNCH(name)                                             \
   do {                                                                      \

@@ -183,6 +183,9 @@ struct ExpandEpi {
   int64_t sy_b, sy_m, sy_h;                // destination strides
   int dst_by_position, dst_rows;
 };
+inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+// byte offsets of `rows` rows of stride ld fit the 32 unsigned bits of a buffer load
+inline bool below_4gib(int64_t rows, int64_t ld) { return ld >= 0 && rows * ld * 2 < (int64_t)4 << 30; }
 // caller-owned scratch of the current device for the K-split projections (null when none is registered)
 struct SplitWorkspace { float* part; size_t part_floats; int32_t* count; int ncount; };
 SplitWorkspace split_workspace();                                            // capi.hip

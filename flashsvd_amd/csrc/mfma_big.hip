@@ -57,7 +57,7 @@ struct BigProblem {
 struct BigArgs { BigProblem p[3]; int first_tile[4]; int rows, nt; };   // column tiles of problem i: [first_tile[i], first_tile[i + 1])
 
 // two tiles' words of a row of 16 lanes become consecutive words: lanes of even rows get columns 4 r .. 4 r + 7 of tile a,
-// lanes of odd rows of tile b (r the row below), see store_pair
+// lanes of odd rows of tile b (r the row below): 8-byte pieces of two neighbouring tiles leave as 16-byte stores
 __device__ __forceinline__ void swap_rows(uint32_t& a, uint32_t& b) {
   const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
   a = r[0];
@@ -343,9 +343,6 @@ __global__ __launch_bounds__(kBigThreads, 2) void gemm_big_kernel(BigArgs args) 
   if (wm == 0) barrier();                            // the other group's last turn
 }
 
-static bool big16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
-static bool below4g(int64_t rows, int64_t ld) { return ld >= 0 && rows * ld * 2 < (int64_t)4 << 30; }
-
 template <int DT, int EPI>
 static int launch_big_t(const BigArgs& a, hipStream_t st, const char* who) {
   static bool granted = false;
@@ -367,8 +364,8 @@ static int launch_big_t(const BigArgs& a, hipStream_t st, const char* who) {
 // smaller tiles of mfma_gemm.hip, which leave fewer compute units idle, are ahead.  us per call, those tiles -> this kernel:
 // 320 tiles (8192 x 2432 x 11008, 62 % full) 557 -> 486, 448 (16384 x 1664 x 4096, 87 %) 269 -> 193, 160 (5000 x 2048 x 2048,
 // 62 %) 68 -> 46, 256 (4096 x 4096 x 4096) 158 -> 105; 128 tiles (2048 x 4096 x 4096, 50 %) 80 -> 97, 96 tiles (4096 x 1536 x
-// 11008, 37 %) 181 -> 243.  The gate / up pair (11008 x 1536) at 2048 / 1024 / 768 rows (67 / 67 / 50 %) 208 -> 194, 124 -> 98,
-// 113 -> 98; at 512 rows (34 %) 75 -> 98.
+// 11008, 37 %) 181 -> 243.  The gate / up pair comes here where mfma_mid.hip needs more than twice the rounds (its 128 x 192 tiles
+// take half as long): 1280 rows of 11008 x 1536 (84 % of one round) 101 here and 130 there.
 static bool big_worth(int64_t rows, int64_t col_tiles, int share) {
   const int64_t tiles = ((rows + kBigT - 1) / kBigT) * col_tiles, cu = compute_units();
   return rows >= kBigT && cu > 0 && tiles * 100 >= share * cu * ((tiles + cu - 1) / cu);
@@ -377,8 +374,8 @@ static bool big_worth(int64_t rows, int64_t col_tiles, int share) {
 bool gemm_big_apply(const MfmaArgs& a, bool dual) {
   if (dual && a.mode != 0) return false;             // the fused rounding keeps the gate in fp32
   return big_worth(a.B, (a.N + kBigT - 1) / kBigT, dual ? 50 : 55) && a.K > 0 && a.K % 64 == 0 && a.ldx % 8 == 0 && a.ldw % 8 == 0 && a.ldy % 8 == 0 && a.up_off % 8 == 0 &&
-         big16(a.x) && big16(a.W) && (!dual || big16(a.W2)) && big16(a.y) && (a.res == nullptr || (big16(a.res) && a.ldres % 8 == 0)) &&
-         below4g(a.B, a.ldx) && below4g(a.N, a.ldw);
+         aligned16(a.x) && aligned16(a.W) && (!dual || aligned16(a.W2)) && aligned16(a.y) && (a.res == nullptr || (aligned16(a.res) && a.ldres % 8 == 0)) &&
+         below_4gib(a.B, a.ldx) && below_4gib(a.N, a.ldw);
 }
 int launch_gemm_big(const MfmaArgs& m, bool dual, hipStream_t st, const char* who) {
   BigArgs a{};
@@ -396,10 +393,10 @@ bool expand_big_apply(const ExpandArgs* d, int n) {
   for (int i = 0; i < n; ++i) {
     const ExpandArgs& a = d[i];
     const auto al8 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7) == 0; };
-    if (a.R % 64 || a.sp_b % 8 || a.sp_m % 8 || a.ldu % 8 || a.sy_b % 8 || a.sy_m % 8 || a.sy_h % 8 || !big16(a.p) || !big16(a.u) || !big16(a.y) ||
+    if (a.R % 64 || a.sp_b % 8 || a.sp_m % 8 || a.ldu % 8 || a.sy_b % 8 || a.sy_m % 8 || a.sy_h % 8 || !aligned16(a.p) || !aligned16(a.u) || !aligned16(a.y) ||
         (a.cos && !(al8(a.cos) && al8(a.sin))))
       return false;
-    if (a.sp_b < 0 || a.sp_m < 0 || ((a.B - 1) * a.sp_b + (a.M - 1) * a.sp_m + a.R) * 2 >= (int64_t)4 << 30 || !below4g((int64_t)a.heads * 128, a.ldu)) return false;
+    if (a.sp_b < 0 || a.sp_m < 0 || ((a.B - 1) * a.sp_b + (a.M - 1) * a.sp_m + a.R) * 2 >= (int64_t)4 << 30 || !below_4gib((int64_t)a.heads * 128, a.ldu)) return false;
     tiles += (a.heads + 1) / 2;
   }
   return big_worth((int64_t)d[0].B * d[0].M, tiles, 65);   // q, k and v of 32 heads at 1024 rows (75 %) 42 against 44 us of 64-row tiles, at 1536 (56 %) 77 against 69

@@ -1,9 +1,11 @@
-// Prefill projections: y[M, N] = epilogue(x[M, K] . W[N, K]^T) for 128 rows and more, on the matrix cores.
+// Projections y[M, N] = epilogue(x[M, K] . W[N, K]^T) on the matrix cores that neither mfma_mid.hip (about one tile per compute
+// unit) nor mfma_big.hip (many) takes: prompts with few output tiles or a very long K, 17 to 127 rows with K split, rows and
+// row lengths off the grid from three rows on, and head expansions of such ranks.
 //
 // Both operands are K-contiguous, which is the layout V_MFMA_F32_16X16X32_BF16 wants for its two inputs (each lane
 // holds 8 consecutive k of one row).  A workgroup of four or eight waves owns a 128 x 128, 128 x 64 or 64 x 64 output
 // tile (32 x 64 below 128 rows) — the launcher picks by how many tiles the problem has for 256 compute units — and walks
-// K in steps of 32, 64 or 128 through two LDS stages (the 16-byte pieces of a row swizzled so that the fragment reads of
+// K in steps of 64 or 128 through two LDS stages (the 16-byte pieces of a row swizzled so that the fragment reads of
 // 16 consecutive rows fall on different banks).  Two ways to fill a stage: global loads that run two to four steps
 // ahead in registers and are written to the idle stage one step before their products (few workgroups per compute
 // unit, long K: latency-bound), or loads that write LDS themselves one step ahead (no staging registers, no LDS write
@@ -13,7 +15,6 @@
 // head expansion of the prompt pass (RoPE, store into the query buffer or the cache rows).  Few tiles or a very long K:
 // K split over workgroups, partial tiles added in a fixed order by the last arrival.
 #include <algorithm>
-#include <string>
 #include <type_traits>
 
 #include "common.hpp"
@@ -24,7 +25,7 @@ namespace fsvd {
 typedef float gm_f32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kGT4 = 256;           // threads of the four-wave form: 2 x 2 waves
-constexpr int kGBK = 64;            // K per step (the small tile takes 128 when K allows: half as many barriers)
+constexpr int kGBK = 64;            // K per step (the small tiles take 128 when K allows: half as many barriers)
 
 // WT: 16 x 16 accumulator tiles per wave and dimension: 4 -> 128 x 128 per workgroup, 2 -> 64 x 64 (problems with
 // few output tiles, where more workgroups matter more than reuse)
@@ -49,7 +50,7 @@ __device__ __forceinline__ void gemm_tiles_body(const MfmaArgs& a, const ExpandE
   static_assert(!EXPAND || (!DUAL && WT == 4), "head expansion takes whole 128-wide heads");
   static_assert(!RAG || PF > 0, "ragged rows are staged through registers");
   typedef typename std::conditional<RAG, u32x4_any_t, u32x4_t>::type piece_t;
-  static_assert(NW == 4 || (NW == 8 && DUAL && WT == 4 && WTM == 4) || (NW == 8 && !DUAL && !EXPAND && BK >= 64),
+  static_assert(NW == 4 || (NW == 8 && DUAL && WT == 4 && WTM == 4) || (NW == 8 && !DUAL && !EXPAND),
                 "eight waves: the split form of the 128 x 128 pair tile, or two halves of every K step of a single matrix");
   constexpr int kGT = NW * 64;
   constexpr bool SPLIT = NW == 8 && DUAL;
@@ -91,9 +92,8 @@ __device__ __forceinline__ void gemm_tiles_body(const MfmaArgs& a, const ExpandE
   // below (lane = row % 16 + 16 * piece) touch every bank once per group, which row padding of 16 bytes does not
   // achieve (two lanes per bank, half the read rate).  RPP and the fragment row bases are multiples of CPR, so the
   // swizzle term of a thread never changes.
-  // (Rows of 64 bytes, K steps of 32: four rows span the banks once, and the term is (-(r / 4)) % 4 instead.)
-  static_assert(RPP % 16 == 0 && CPR >= 4 && CPR <= 16, "swizzle term must be constant per thread");
-  const auto swz = [](int r) { return CPR == 4 ? ((-(r >> 2)) & 3) : r % CPR; };
+  static_assert(RPP % 16 == 0 && (CPR == 8 || CPR == 16), "swizzle term must be constant per thread");
+  const auto swz = [](int r) { return r % CPR; };
   const int st_chunk = ld_chunk ^ swz(ld_row);
   // direct form: lane i of a load instruction lands at 16 i bytes past the instruction's LDS base, i.e. at piece
   // ld_chunk of its row, so it fetches the piece that belongs there
@@ -525,9 +525,8 @@ __global__ __launch_bounds__(kGT4, 2) void expand_multi_kernel(ExpandBatch eb) {
   gemm_tiles_body<DT, false, WTM, 4, 2, true, kGBK, 4, true>(eb.a[k], eb.ep[k], tile_m, tile_n - eb.first_head[k]);
 }
 
-static bool at16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 static bool aligned_rows(const MfmaArgs& a) {
-  return (a.ldw % 8) == 0 && (a.ldx % 8) == 0 && (a.up_off % 8) == 0 && at16(a.x) && at16(a.W) && (a.W2 == nullptr || at16(a.W2));
+  return (a.ldw % 8) == 0 && (a.ldx % 8) == 0 && (a.up_off % 8) == 0 && aligned16(a.x) && aligned16(a.W) && (a.W2 == nullptr || aligned16(a.W2));
 }
 bool gemm_tiles_apply(const MfmaArgs& a) { return a.B >= 128 && (a.K % kGBK) == 0 && aligned_rows(a); }
 
@@ -554,6 +553,29 @@ static int pick_ksplit_prompt(int64_t tiles, int ksteps, int K, size_t floats_pe
   if (K >= 8192 && tiles < 512) z = std::max(z, (int)((768 + tiles - 1) / tiles));
   return z > 1 ? fit_ksplit(z, tiles, ksteps, floats_per_share, ws, 8) : 1;
 }
+
+// "tiles 64 x 128", "any rows 32 x 64 pair", ... made by the compiler: an entry point neither allocates nor throws
+template <int BM, int BN, bool DUAL, bool RAG>
+struct TileForm {
+  struct Text { char s[32]; };
+  static constexpr Text make() {
+    Text t{};
+    int n = 0;
+    const auto word = [&](const char* w) { for (; *w; ++w) t.s[n++] = *w; };
+    const auto number = [&](int v) {
+      if (v >= 100) t.s[n++] = (char)('0' + v / 100);
+      t.s[n++] = (char)('0' + v / 10 % 10);
+      t.s[n++] = (char)('0' + v % 10);
+    };
+    word(RAG ? "any rows " : "tiles ");
+    number(BM);
+    word(" x ");
+    number(BN);
+    if (DUAL) word(" pair");
+    return t;
+  }
+  static constexpr Text name = make();
+};
 
 template <int DT, bool DUAL, int WTM, int WT, int BK, int NW = 4, int PFSEL = 99, bool RAG = false>
 static int launch_gemm_tiles_t(const MfmaArgs& a0, hipStream_t st, const char* who) {
@@ -584,8 +606,7 @@ static int launch_gemm_tiles_t(const MfmaArgs& a0, hipStream_t st, const char* w
   a.ws_part = ws.part;
   a.ws_count = ws.count;
   grid.z = a.ksplit;
-  static const std::string form = (RAG ? "any rows " : "tiles ") + std::to_string(BM) + " x " + std::to_string(BN) + (DUAL ? " pair" : "");
-  set_last_form(form.c_str());
+  set_last_form(TileForm<BM, BN, DUAL, RAG>::name.s);
   hipLaunchKernelGGL((gemm_tiles_kernel<DT, DUAL, WTM, WT, PF, false, BK, NW, RAG>), grid, dim3(NW * 64), lds, st, a, ExpandEpi{});
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }
@@ -595,24 +616,23 @@ static int launch_gemm_tiles_t(const MfmaArgs& a0, hipStream_t st, const char* w
 template <int DT>
 static int launch_gemm_tiles_dt(const MfmaArgs& a, bool dual, hipStream_t st, const char* who) {
   const int64_t big = (int64_t)((a.N + 127) / 128) * ((a.B + 127) / 128);
-  // Forms by tile count, for what the other two tiled kernels leave (mfma_mid.hip: about one tile per compute unit; mfma_big.hip:
-  // many), measured on the projections of the 7B shape at 128..4096 rows.  The pair reaches this kernel with few tiles, or
-  // with operands of 4 GiB and more.  A single matrix: 128 x 128 from 448 big tiles on, 128 x 64 from 256 on, else 64 x 64 —
-  // in K steps of 64 with a deep register pipeline when there are more of those than the chip holds at once (320), in
-  // steps of 128 (half as many barriers) when there are fewer: with one workgroup or less per compute unit and a long K
-  // only loads issued several steps ahead hide the latency.
+  // Forms by tile count, for what the other two tiled kernels leave, measured on the projections of the 7B shape at 128..4096
+  // rows.  The pair reaches this kernel with few tiles, or with operands of 4 GiB and more.  A single matrix: 128 x 128 from 448
+  // big tiles on, 128 x 64 from 256 on, else 64 x 64 — in K steps of 64 with a deep register pipeline when there are more of
+  // those than the chip holds at once (320), in steps of 128 (half as many barriers) when there are fewer: with one
+  // workgroup or less per compute unit and a long K only loads issued several steps ahead hide the latency.
   if (dual) return big >= 512 ? launch_gemm_tiles_t<DT, true, 4, 4, 64, 8, 2, true>(a, st, who) : launch_gemm_tiles_t<DT, true, 2, 2, 64>(a, st, who);
   // a single matrix with more than one big tile per compute unit: loads straight into LDS, two stages (the second and
   // third workgroup of a compute unit cover the one-step load distance; 5..8 % faster than the register pipeline with
   // weights that come from HBM, and slower than it below these tile counts)
   if (big >= 448) return launch_gemm_tiles_t<DT, false, 4, 4, 64, 4, -2>(a, st, who);
   if (big >= 320) return launch_gemm_tiles_t<DT, false, 4, 2, 64, 4, -2>(a, st, who);
-  // K of 8192 and more with about one 128 x 64 tile per compute unit: eight waves, each half of them on half of the k slices
-  // of a step, so that a workgroup alone on its compute unit still runs two waves per SIMD (1536 x 11008 at 1024 rows 72 us,
-  // three stages of loads straight into LDS 73)
   if (big >= 256) return launch_gemm_tiles_t<DT, false, 4, 2, 64>(a, st, who);
   // mfma_mid.hip takes these where its 32-bit offsets reach; operands past them stay on unsplit 128 x 128 tiles
   if (big >= 144) return launch_gemm_tiles_t<DT, false, 4, 4, 64, 4, 2, true>(a, st, who);
+  // K of 8192 and more with about one 128 x 64 tile per compute unit: eight waves, each half of them on half of the k slices
+  // of a step, so that a workgroup alone on its compute unit still runs two waves per SIMD (1536 x 11008 at 1024 rows 72 us,
+  // three stages of loads straight into LDS 73)
   const int64_t half = (int64_t)((a.N + 63) / 64) * ((a.B + 127) / 128);
   if (half >= 160 && half <= 256 && (a.K % 128) == 0) return launch_gemm_tiles_t<DT, false, 4, 2, 128, 8>(a, st, who);
   const int64_t small = (int64_t)((a.N + 63) / 64) * ((a.B + 63) / 64);
@@ -676,7 +696,7 @@ int launch_gemm_ragged(const MfmaArgs& a, bool dual, hipStream_t st, const char*
 // per 32 rows and head 80 to 95 us), and with fewer rows where lowrank_expand_kernel cannot take them, so that a rank or an
 // address is accepted or refused alike at every row count.
 bool expand_tiles_apply(const ExpandArgs& a) {
-  const bool on_grid = a.R % 8 == 0 && a.sp_b % 8 == 0 && a.sp_m % 8 == 0 && a.ldu % 8 == 0 && at16(a.p) && at16(a.u);
+  const bool on_grid = a.R % 8 == 0 && a.sp_b % 8 == 0 && a.sp_m % 8 == 0 && a.ldu % 8 == 0 && aligned16(a.p) && aligned16(a.u);
   return a.Dh == 128 && a.R > 0 && a.heads > 0 && a.B > 0 && a.M > 0 && a.sp_h == 0 && ((int64_t)a.B * a.M >= 16 || !on_grid);
 }
 

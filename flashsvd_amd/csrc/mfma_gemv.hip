@@ -828,8 +828,6 @@ static int launch_mfma(const MfmaArgs& a0, hipStream_t st, const char* who) {
   return kOk;
 }
 
-static inline bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
-
 template <int DT, int NB>
 static int launch_qkv_mfma_t(const QkvArgs& a, hipStream_t st) {
   const char* who = "fsvd_qkv_rope_append";
@@ -852,7 +850,7 @@ static int launch_qkv_mfma_t(const QkvArgs& a, hipStream_t st) {
 // 3..32 tokens, ranks of whole chunks, a head of whole tile pairs
 bool qkv_mfma_applies(const QkvArgs& a) {
   return a.B >= 3 && a.B <= 32 && a.Dh % 32 == 0 && a.Rq % 64 == 0 && a.Rk % 64 == 0 && a.Rv % 64 == 0 && a.ldp % 8 == 0 && a.ldq % 8 == 0 &&
-         a.ldk % 8 == 0 && a.ldv % 8 == 0 && al16(a.p) && al16(a.q_u) && al16(a.k_u) && al16(a.v_u);
+         a.ldk % 8 == 0 && a.ldv % 8 == 0 && aligned16(a.p) && aligned16(a.q_u) && aligned16(a.k_u) && aligned16(a.v_u);
 }
 int launch_qkv_mfma(const QkvArgs& a, hipStream_t st) {
   if (a.B <= 16) return a.dt == 1 ? launch_qkv_mfma_t<1, 1>(a, st) : launch_qkv_mfma_t<0, 1>(a, st);

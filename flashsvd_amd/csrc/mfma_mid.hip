@@ -295,8 +295,6 @@ static int launch_mid_t(MidArgs& m, hipStream_t st, const char* who) {
   return kOk;
 }
 
-static bool mid16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
-static bool mid_below4g(int64_t rows, int64_t ld) { return ld >= 0 && rows * ld * 2 < (int64_t)4 << 30; }
 // share (percent) of its last round of one tile per compute unit and all before it that a tiling fills
 static int64_t mid_tiles(const MfmaArgs& a, int bm, int bn) { return (int64_t)((a.N + bn - 1) / bn) * ((a.B + bm - 1) / bm); }
 static int64_t mid_rounds(int64_t tiles) { return (tiles + compute_units() - 1) / compute_units(); }
@@ -315,9 +313,10 @@ enum MidForm { kMidNone = 0, kMid128x192, kMid64x192, kMid128x64Halves, kMid64x6
 // them (4096 x 1024 at 333 / 512 rows 12.3 -> 10.2, 12.9 -> 11.3, 3072 x 4096 at 420 29.3 -> 25.9), then 64 x 64 (4096 x 1024 at 154
 // rows 8.5 -> 7.5, 1536 x 2048 at 256 15.4 -> 12.1; 64 to 128 tiles only for a short K, beyond that a K split over workgroups wins:
 // 4096 x 4096 at 128 rows 18.0 against 21.9).  A K of 8192 and more is better split as well (1536 x 11008 at 512 rows 47, here 51).
+// The counts are those of 256 compute units, the rules fractions of them.
 static MidForm mid_form(const MfmaArgs& a, bool dual) {
-  if (a.B < 128 || compute_units() <= 0 || a.K < 64 || a.K % 64 || a.ldx % 8 || a.ldw % 8 || a.up_off % 8 || !mid16(a.x) || !mid16(a.W) ||
-      (dual && !mid16(a.W2)) || !mid_below4g(a.B, a.ldx) || !mid_below4g(a.N, a.ldw))
+  if (a.B < 128 || compute_units() <= 0 || a.K < 64 || a.K % 64 || a.ldx % 8 || a.ldw % 8 || a.up_off % 8 || !aligned16(a.x) || !aligned16(a.W) ||
+      (dual && !aligned16(a.W2)) || !below_4gib(a.B, a.ldx) || !below_4gib(a.N, a.ldw))
     return kMidNone;
   if (dual) {
     const int64_t t = mid_tiles(a, 128, 192);
@@ -325,11 +324,11 @@ static MidForm mid_form(const MfmaArgs& a, bool dual) {
     if (mid_fills(t, 55)) return kMid128x192;
     return mid_fills(mid_tiles(a, 64, 192), 60) ? kMid64x192 : kMidNone;
   }
-  const int64_t big = mid_tiles(a, 128, 128), half = mid_tiles(a, 128, 64), small = mid_tiles(a, 64, 64);
-  if (big >= 144 && big <= 256) return kMid128x128;
+  const int64_t big = mid_tiles(a, 128, 128), half = mid_tiles(a, 128, 64), small = mid_tiles(a, 64, 64), cu = compute_units();
+  if (big * 16 >= cu * 9 && big <= cu) return kMid128x128;
   if (a.K % 128 || a.K >= 8192) return kMidNone;
-  if (half > 128 && half <= 256) return kMid128x64Halves;
-  return small <= 256 && (small > 128 || (small >= 64 && a.K <= 2048)) ? kMid64x64Halves : kMidNone;
+  if (half * 2 > cu && half <= cu) return kMid128x64Halves;
+  return small <= cu && (small * 2 > cu || (small * 4 >= cu && a.K <= 2048)) ? kMid64x64Halves : kMidNone;
 }
 bool gemm_mid_apply(const MfmaArgs& a, bool dual) { return mid_form(a, dual) != kMidNone; }
 
@@ -355,8 +354,8 @@ int launch_gemm_mid(const MfmaArgs& a, bool dual, hipStream_t st, const char* wh
 bool expand_mid_apply(const ExpandArgs* d, int n) {
   for (int k = 0; k < n; ++k) {
     const ExpandArgs& a = d[k];
-    if (a.R < 64 || a.R % 64 || a.sp_b % 8 || a.sp_m % 8 || a.ldu % 8 || !mid16(a.p) || !mid16(a.u) || a.sp_b < 0 || a.sp_m < 0 ||
-        ((a.B - 1) * a.sp_b + (a.M - 1) * a.sp_m + a.R) * 2 >= (int64_t)4 << 30 || !mid_below4g((int64_t)a.heads * 128, a.ldu))
+    if (a.R < 64 || a.R % 64 || a.sp_b % 8 || a.sp_m % 8 || a.ldu % 8 || !aligned16(a.p) || !aligned16(a.u) || a.sp_b < 0 || a.sp_m < 0 ||
+        ((a.B - 1) * a.sp_b + (a.M - 1) * a.sp_m + a.R) * 2 >= (int64_t)4 << 30 || !below_4gib((int64_t)a.heads * 128, a.ldu))
       return false;
   }
   return true;

@@ -484,15 +484,16 @@ static int launch_prefill_attn_form(const PrefillAttnArgs& a, hipStream_t st) {
 
 template <int DT>
 static int launch_prefill_attn_t(const PrefillAttnArgs& a, hipStream_t st) {
-  // 128 query rows per workgroup when that gives every compute unit work, else 64 (half the rows per wave)
-  if ((int64_t)((a.M + 127) / 128) * a.H * a.B >= 384) return launch_prefill_attn_form<DT, 2, 1>(a, st);
+  // 128 query rows per workgroup from 1.5 workgroups per compute unit on, else 64 (half the rows per wave)
+  const int64_t cu = compute_units();
+  if ((int64_t)((a.M + 127) / 128) * a.H * a.B * 2 >= cu * 3) return launch_prefill_attn_form<DT, 2, 1>(a, st);
   // chunks of up to one 64-row workgroup per compute unit: three groups of waves share its key tiles (four spill); prompts of
   // up to ~1.5: two.  us with one / two / three groups: 512 rows of 32 heads (256 workgroups) 17.1 / 15.3 / 15.7, the same behind 1000
   // tokens 42.7 / 34.0 / 31.7, two chunks of 77 rows behind 1411 tokens (128) 42.0 / 33.4 / 30.5; 700 rows (352) 26.5 / 23.2 /
   // 23.4, 1024 rows (512) 37.3 / 38.9 / 37.7
   const int64_t tiles = (int64_t)((a.M + 63) / 64) * a.H * a.B;
-  if (tiles <= 256 && a.M < 128) return launch_prefill_attn_form<DT, 1, 3>(a, st);
-  if (tiles <= 384) return launch_prefill_attn_form<DT, 1, 2>(a, st);
+  if (tiles <= cu && a.M < 128) return launch_prefill_attn_form<DT, 1, 3>(a, st);
+  if (tiles * 2 <= cu * 3) return launch_prefill_attn_form<DT, 1, 2>(a, st);
   return launch_prefill_attn_form<DT, 1, 1>(a, st);
 }
 

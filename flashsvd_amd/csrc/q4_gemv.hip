@@ -240,7 +240,6 @@ int launch_dequant_q4(const uint8_t* qw, int64_t ldq, const uint16_t* sc, const 
   return kOk;
 }
 
-static inline bool q4_al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 size_t q4_lds_bytes(int batch, int nmat, int K, int rows_per_wg) {
   const size_t ppr = (size_t)K / 32, cpr = ppr / 8;
@@ -289,9 +288,9 @@ int launch_linear_q4(const Q4Args& a0, hipStream_t st) {
   if (a0.ldq < a0.K / 2 || (a0.ldq % 16) || (a0.ldx % 8) || (a0.up_off % 8)) { set_last_error("%s: row strides must keep 16-byte alignment", fn); return kErrBadAlign; }
   for (int m = 0; m < a0.nmat; ++m) {
     if (!a0.qw[m] || !a0.sc[m] || !a0.zr[m]) { set_last_error("%s: null weight, scale or zero pointer", fn); return kErrNullPtr; }
-    if (!q4_al16(a0.qw[m])) { set_last_error("%s: packed weights must be 16-byte aligned", fn); return kErrBadAlign; }
+    if (!aligned16(a0.qw[m])) { set_last_error("%s: packed weights must be 16-byte aligned", fn); return kErrBadAlign; }
   }
-  if (!q4_al16(a0.x) || (a0.norm_w && !q4_al16(a0.norm_w))) { set_last_error("%s: activations / norm weight must be 16-byte aligned", fn); return kErrBadAlign; }
+  if (!aligned16(a0.x) || (a0.norm_w && !aligned16(a0.norm_w))) { set_last_error("%s: activations / norm weight must be 16-byte aligned", fn); return kErrBadAlign; }
   const int ppr = a0.K / 32;
   // at least one piece per thread, at least twice as many weight bytes as staged activation bytes
   int rows = (a0.N + 511) / 512;

@@ -221,10 +221,9 @@ def test_swiglu_wide_matrix_resident_form(ops, B, D, R, mode):
     assert torch.equal(h, ops.swiglu_linear(p.cuda(), gu.cuda(), uu.cuda(), up_off=R, mode=mode)), "repeat differs"
 
 
-# ---- 128 rows and more (prefill): the tiled matrix-core kernel (csrc/mfma_gemm.hip) behind the same entry points
-#      (shapes chosen to reach every tile form: 64 x 64 in K steps of 64 / 128, 128 x 64 and 128 x 128 with four and with
-#      eight waves, 128 x 256 from 2048 big tiles on, loads through registers and straight into LDS, ragged edges in rows
-#      and columns)
+# ---- 128 rows and more (prefill): the tiled matrix-core kernels (csrc/mfma_gemm.hip, mfma_mid.hip, mfma_big.hip) behind the same
+#      entry points, at whole and partial tiles, few and many of them, short and long K (the forms by name:
+#      test_gpu_mid_tiles.py, test_gpu_big_tiles.py, test_gpu_ragged.py)
 @pytest.mark.parametrize("B,N,K", [(512, 3072, 4096), (128, 128, 64), (200, 1000, 1536), (129, 130, 192), (384, 1536, 11008),
                                    (1024, 64, 1024), (500, 3050, 1152), (1000, 3000, 1088), (1024, 3072, 1024), (2048, 4096, 256),
                                    (2040, 2900, 192), (1150, 4090, 320), (4096, 8192, 64), (4100, 8200, 96)])
