@@ -186,6 +186,22 @@ struct ExpandEpi {
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 // byte offsets of `rows` rows of stride ld fit the 32 unsigned bits of a buffer load
 inline bool below_4gib(int64_t rows, int64_t ld) { return ld >= 0 && rows * ld * 2 < (int64_t)4 << 30; }
+// "tiles 64 x 128", "ring 128 x 192 pair", ... for set_last_form, made by the compiler: an entry point neither allocates nor throws
+struct FormText { char s[32]; };
+constexpr FormText form_text(const char* head, int bm, int bn, const char* tail) {
+  FormText t{};
+  int n = 0;
+  for (; *head; ++head) t.s[n++] = *head;
+  for (int part = 0; part < 2; ++part) {
+    const int v = part ? bn : bm;
+    if (part) { t.s[n++] = ' '; t.s[n++] = 'x'; t.s[n++] = ' '; }
+    if (v >= 100) t.s[n++] = static_cast<char>('0' + v / 100);
+    t.s[n++] = static_cast<char>('0' + v / 10 % 10);
+    t.s[n++] = static_cast<char>('0' + v % 10);
+  }
+  for (; *tail; ++tail) t.s[n++] = *tail;
+  return t;
+}
 // caller-owned scratch of the current device for the K-split projections (null when none is registered)
 struct SplitWorkspace { float* part; size_t part_floats; int32_t* count; int ncount; };
 SplitWorkspace split_workspace();                                            // capi.hip

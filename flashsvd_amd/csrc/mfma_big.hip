@@ -1,19 +1,20 @@
 // Projections of long prompts: 256 x 256 output tiles, one workgroup of eight waves per compute unit that walks its share of
 // the tiles.
 //
-// What bounds a large product on this chip is power: under a stream of matrix products the clock settles at 1.4 to 1.75 GHz,
-// and every byte that has to be moved to feed the products costs both cycles and clock.  So the tile is the largest that one
-// compute unit can hold.  A wave owns 128 x 64 of it (16 x 16 x 32 products, 128 accumulators): a K slice of 32 costs 12
-// fragment reads from LDS for 32 products, two thirds of what a 64 x 64 block costs.  K goes in steps of 64, i.e. whole
+// What bounds a large product on this chip is cycles and clock alike: under a stream of these products the clock stays at 1.95 to
+// 2.2 GHz (1.65 in the first milliseconds of a burst), the matrix cores are busy in 50 to 63 % of the cycles (counters), and
+// every byte that has to be moved to feed the products costs both.  So the tile is the largest that one compute unit can
+// hold.  A wave owns 128 x 64 of it (16 x 16 x 32 products, 128 accumulators): a K slice of 32 costs 12 fragment reads
+// from LDS for 32 products, two thirds of what a 64 x 64 block costs.  K goes in steps of 64, i.e. whole
 // 128-byte cache lines of every operand row (in steps of 32 every line crossed from L2 twice, because the L1 does not keep
 // its other half until the next step: the loads alone then took 430 us of a 546 us product).  Loads write LDS directly, one
 // step ahead into the other of two stages (two steps ahead for x, 160 KB of LDS: no faster).
 //
 // The two waves of a SIMD alternate: waves 0-3 (the upper half of the tile) read the fragments of a slice while waves 4-7
 // multiply theirs, then the other way round, a bare barrier between the turns (published as "ping-pong" scheduling for this
-// family of chips) and the multiplying wave at raised priority (12 % slower without).  Of the 2048 cycles of products in a
-// step it reaches 2900 with the loads and 2200 without them; four waves of 128 x 128, which read a third less from LDS,
-// came to 2570 to 2860.
+// family of chips) and the multiplying wave at raised priority (12 % slower without).  A step, 2048
+// cycles of products, takes 3260 to 3340 with its share of the epilogue (a single matrix, K = 4096 and 1664; 4040 for the pair);
+// four waves of 128 x 128, which read a third less from LDS, were no faster.
 //
 // The walk over the tiles is one stream: the first stage of the next tile is requested during the last step of this one, and
 // a finished tile leaves from the accumulators (pairs of 8-byte pieces become 16-byte ones by a row swap between lanes)

@@ -554,29 +554,6 @@ static int pick_ksplit_prompt(int64_t tiles, int ksteps, int K, size_t floats_pe
   return z > 1 ? fit_ksplit(z, tiles, ksteps, floats_per_share, ws, 8) : 1;
 }
 
-// "tiles 64 x 128", "any rows 32 x 64 pair", ... made by the compiler: an entry point neither allocates nor throws
-template <int BM, int BN, bool DUAL, bool RAG>
-struct TileForm {
-  struct Text { char s[32]; };
-  static constexpr Text make() {
-    Text t{};
-    int n = 0;
-    const auto word = [&](const char* w) { for (; *w; ++w) t.s[n++] = *w; };
-    const auto number = [&](int v) {
-      if (v >= 100) t.s[n++] = (char)('0' + v / 100);
-      t.s[n++] = (char)('0' + v / 10 % 10);
-      t.s[n++] = (char)('0' + v % 10);
-    };
-    word(RAG ? "any rows " : "tiles ");
-    number(BM);
-    word(" x ");
-    number(BN);
-    if (DUAL) word(" pair");
-    return t;
-  }
-  static constexpr Text name = make();
-};
-
 template <int DT, bool DUAL, int WTM, int WT, int BK, int NW = 4, int PFSEL = 99, bool RAG = false>
 static int launch_gemm_tiles_t(const MfmaArgs& a0, hipStream_t st, const char* who) {
   static bool granted = false;
@@ -606,7 +583,8 @@ static int launch_gemm_tiles_t(const MfmaArgs& a0, hipStream_t st, const char* w
   a.ws_part = ws.part;
   a.ws_count = ws.count;
   grid.z = a.ksplit;
-  set_last_form(TileForm<BM, BN, DUAL, RAG>::name.s);
+  static constexpr FormText form = form_text(RAG ? "any rows " : "tiles ", BM, BN, DUAL ? " pair" : "");
+  set_last_form(form.s);
   hipLaunchKernelGGL((gemm_tiles_kernel<DT, DUAL, WTM, WT, PF, false, BK, NW, RAG>), grid, dim3(NW * 64), lds, st, a, ExpandEpi{});
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }

@@ -2,19 +2,18 @@
 // per output tile, operand rows straight into a ring of three to five LDS stages.
 //
 // Up to a few tiles per compute unit neither form beside this one fits: the two-stage tiles of mfma_gemm.hip rely on a second
-// workgroup of the compute unit to cover a load distance of one step and wait out most of it (1900 cycles per 128 of K of a
-// 128 x 64 tile whose products take 512), and the 256 x 256 tiles of mfma_big.hip leave compute units idle.  So the tile is
-// chosen to give nearly every compute unit one, and loads run two to four steps ahead of the products behind a counted
-// wait (a bare barrier, no fence).  The fragments of a slice are read while the slice before it multiplies; what is left as
-// the bound is LDS traffic: a 128 x 192 step of 64 writes 40 KB and reads 112 KB of fragments for 768 cycles of products and
-// takes about 1700 cycles (the pair 512 x 11008 x 1536 82 -> 49 us, 0.71 PFLOP/s; accumulators that a condition inside the loop
-// may move cost another 10 us of register copies, hence two walks).
+// workgroup of the compute unit to cover a load distance of one step and wait out most of it, and the 256 x 256 tiles of
+// mfma_big.hip leave compute units idle.  So the tile is chosen to give nearly every compute unit one, and loads run two to
+// four steps ahead of the products behind a counted wait (a bare barrier, no fence).  The fragments of a slice are read while
+// the slice before it multiplies; what is left as the bound is LDS traffic: a 128 x 192 step of 64 writes 40 KB and reads
+// 112 KB of fragments for 768 cycles of products and takes about 2400 cycles, first loads and epilogue included (the pair
+// 512 x 11008 x 1536 82 -> 49 us, 0.71 PFLOP/s; accumulators that a condition inside the loop may move cost another 10 us
+// of register copies, hence two walks).
 //
 // LDS rows are 128 bytes (64 of K), their eight 16-byte pieces XOR-swizzled by row % 8.  KH = 2: waves 4-7 take the second half
 // of every 128 of K and hand their sums to waves 0-3 through LDS at the end; sums run over K in the order of the forms of
 // mfma_gemm.hip.  The gate / up pair runs its two products one after the other over the same tile.
 #include <algorithm>
-#include <string>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -287,17 +286,17 @@ static int launch_mid_t(MidArgs& m, hipStream_t st, const char* who) {
   }
   if (EPI != kMidHeads) m.nt = (m.a[0].N + BN - 1) / BN;
   const int64_t tiles = (int64_t)m.nt * ((m.a[0].B + BM - 1) / BM);
-  static const std::string form = "ring " + std::to_string(BM) + " x " + std::to_string(BN) + (EPI == kMidPair ? " pair" : (EPI == kMidHeads ? " heads" : ""));
-  set_last_form(form.c_str());
+  static constexpr FormText form = form_text("ring ", BM, BN, EPI == kMidPair ? " pair" : (EPI == kMidHeads ? " heads" : ""));
+  set_last_form(form.s);
   hipLaunchKernelGGL((gemm_mid_kernel<DT, EPI, WM, WN, TM, TN, KH, NS>), dim3((unsigned)tiles), dim3(kMidThreads), lds, st, m);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }
   return kOk;
 }
 
-// share (percent) of its last round of one tile per compute unit and all before it that a tiling fills
 static int64_t mid_tiles(const MfmaArgs& a, int bm, int bn) { return (int64_t)((a.N + bn - 1) / bn) * ((a.B + bm - 1) / bm); }
 static int64_t mid_rounds(int64_t tiles) { return (tiles + compute_units() - 1) / compute_units(); }
+// true when a tiling fills `share` percent of its rounds of one tile per compute unit
 static bool mid_fills(int64_t tiles, int share) { return tiles * 100 >= share * compute_units() * mid_rounds(tiles); }
 
 enum MidForm { kMidNone = 0, kMid128x192, kMid64x192, kMid128x64Halves, kMid64x64Halves, kMid128x128 };

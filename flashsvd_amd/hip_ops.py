@@ -118,7 +118,9 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
            norm_weight: Optional[torch.Tensor] = None, eps: float = 1e-6,
            residual: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None, cfg: int = 0) -> torch.Tensor:
     """out = (residual +) linear(rmsnorm?(x), weight, bias); weight is nn.Linear layout [N, K].
-    Dispatches to the custom operator flashsvd_hip::linear (``.out`` when ``out`` is given)."""
+    Dispatches to the custom operator flashsvd_hip::linear (``.out`` when ``out`` is given).  From three rows on, with K a
+    multiple of 64 and rows on the 16-byte grid, the call may split K through the device's one scratch buffer
+    (``ensure_split_workspace``): such calls are to be ordered on one stream."""
     if out is None:
         return _OPS.linear.default(x, weight, bias, norm_weight, float(eps), residual, int(cfg))
     return _OPS.linear.out(x, weight, bias, norm_weight, float(eps), residual, int(cfg), out=out)
@@ -207,7 +209,8 @@ def _linear_rankkv_append_impl(x, weight, pk_cache, pv_cache, positions, rq, rk,
 def swiglu_linear(p: torch.Tensor, gate_u: torch.Tensor, up_u: torch.Tensor, *, up_off: int, mode: int = 0,
                   out: Optional[torch.Tensor] = None, cfg: int = 0) -> torch.Tensor:
     """h = silu(p[..., :R] @ gate_u.T) * (p[..., up_off:up_off+R] @ up_u.T); gate_u/up_u are [D, R].
-    Custom operator flashsvd_hip::swiglu_linear."""
+    Custom operator flashsvd_hip::swiglu_linear.  3 to 127 rows with R a multiple of 64 on the 16-byte grid may split R
+    through the device's one scratch buffer, as :func:`linear` does."""
     if out is None:
         return _OPS.swiglu_linear.default(p, gate_u, up_u, int(up_off), int(mode), int(cfg))
     return _OPS.swiglu_linear.out(p, gate_u, up_u, int(up_off), int(mode), int(cfg), out=out)

@@ -71,14 +71,15 @@ int fsvd_set_workspace(void* ws, size_t bytes, void* stream);
  * `hidden @ packed_qkv_rank` (benchmark/attn/decode_compare.py:1538), `o_u_proj(o_v_proj(.))`
  * (utils/model_utils.py:332-341), `up_v_proj/gate_v_proj` (benchmark/mlp/bench_svd_llama_decode_graph.py:133),
  * phase-2 `matmul(S, DownU)` (kernels/mlp/decode/dual_split_triton.py:719-721) and RMSNorm
- * (benchmark/mlp/bench_svd_llama_decode_graph.py:78-83).  cfg = 0 picks the tiling. */
+ * (benchmark/mlp/bench_svd_llama_decode_graph.py:78-83).  cfg = 0 picks the tiling.  K <= 32768 for one or two rows, with
+ * norm_w and with cfg != 0 (the kernels that keep x in LDS); any K otherwise. */
 int fsvd_linear(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* bias,
                 const void* norm_w, float eps, const void* res, int64_t ldres,
                 void* y, int64_t ldy, int B, int N, int K, int cfg, int dtype, void* stream);
 
 /* h[b,n] = silu(gate_u[n,:] . p[b,0:R]) * (up_u[n,:] . p[b,up_off:up_off+R]),  gate_u/up_u [D,R].
  * mode 0 rounds like a chain of bf16 nn.Linear modules, mode 1 like the fused reference kernel
- * (h = bf16(silu(g32)*u32), kernels/mlp/decode/dual_split_triton.py:207). */
+ * (h = bf16(silu(g32)*u32), kernels/mlp/decode/dual_split_triton.py:207).  R <= 16384 for one or two rows and with cfg != 0. */
 int fsvd_swiglu_linear(const void* p, int64_t ldp, int64_t up_off, const void* gate_u, const void* up_u,
                        int64_t ldw, void* h, int64_t ldh, int B, int D, int R, int mode, int cfg, int dtype, void* stream);
 
