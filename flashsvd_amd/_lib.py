@@ -149,6 +149,9 @@ SIGNATURES = {
     "fsvd_decode_step_workgroups": (c_int, []),
     "fsvd_decode_step_prepare": (c_int, [c_void_p, c_int, c_int]),
     "fsvd_decode_step_validate": (c_int, [c_void_p, c_int, c_int]),
+    "fsvd_decode_step_set_state": (c_int, [c_void_p, c_int64, ctypes.c_int32, c_void_p]),
+    "fsvd_greedy_token": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_void_p]),
+    "fsvd_set_token_rows": (c_int, [c_void_p, c_void_p, c_void_p, ctypes.c_int32, c_int, c_void_p]),
     "fsvd_set_workspace": (c_int, [c_void_p, c_size_t, c_void_p]),
     "fsvd_decode_step": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_int, c_void_p]),
     "fsvd_decode_step_trace": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_size_t, c_int, c_void_p]),

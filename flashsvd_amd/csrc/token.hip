@@ -1,0 +1,121 @@
+// The few words of state between two decoded tokens: the greedy token of every row and its next position, and the state that a
+// caller sets before a step.  Each was a chain of library launches around a step that is itself a chain of launches: at one
+// sequence and 32000 logits the library's argmax took 13.0 us, the copy of its result and the position increment 6 with their
+// gaps, for 64 KB that one compute unit reads in about one; setting the resident step's state took three 4-byte copies of 3 to
+// 6 us each.  A token of a one-block model 69.5 -> 57.8 us, of 8 layers of the 7B shape with int4 factors 486 -> 440, of 32 with
+// 16-bit factors 1966 -> 1921, of sixteen sequences over 4 layers 596 -> 584.
+#include "common.hpp"
+#include "../../include/flashsvd_hip.h"
+
+namespace fsvd {
+
+constexpr int kPickThreads = 1024, kPickLoads = 4;
+
+// 16-bit patterns as integers in the order of their values: NaN above everything, the two zeros equal
+template <int DT>
+__device__ __forceinline__ uint32_t order_key(uint32_t p) {
+  const uint32_t mag = p & 0x7fffu;
+  if (mag > (DT == 1 ? 0x7c00u : 0x7f80u)) return 0x10000u;
+  if (mag == 0) return 0x8000u;
+  return (p & 0x8000u) ? 0xffffu - p : p | 0x8000u;
+}
+
+// One workgroup per row: the row is requested in rounds of four 16-byte pieces per thread (32768 elements), so what it takes is
+// one round trip and 60 GB/s of one compute unit.  Ties go to the lowest index and NaN counts as the largest value, as
+// torch.argmax has it.
+template <int DT>
+__global__ __launch_bounds__(kPickThreads) void greedy_token_kernel(const uint16_t* __restrict__ logits, int64_t ld, int64_t* __restrict__ tokens,
+                                                                   int64_t ldt, int32_t* __restrict__ positions, int V) {
+  const uint16_t* row = logits + (int64_t)blockIdx.x * ld;
+  const int tid = threadIdx.x, pieces = V >> 3;
+  uint32_t best = 0, at = 0x7fffffffu;
+  const auto take = [&](uint32_t p, uint32_t i) {
+    const uint32_t k = order_key<DT>(p);
+    if (k > best) { best = k; at = i; }                // a thread meets its elements in ascending order
+  };
+  for (int c0 = 0; c0 < pieces; c0 += kPickThreads * kPickLoads) {
+    u32x4_t v[kPickLoads];
+#pragma unroll
+    for (int j = 0; j < kPickLoads; ++j) v[j] = *reinterpret_cast<const u32x4_any_t*>(row + (int64_t)min(c0 + j * kPickThreads + tid, pieces - 1) * 8);
+#pragma unroll
+    for (int j = 0; j < kPickLoads; ++j) {
+      const int c = c0 + j * kPickThreads + tid;
+      if (c >= pieces) break;
+      const uint32_t w[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) take((w[e >> 1] >> (16 * (e & 1))) & 0xffffu, c * 8 + e);
+    }
+  }
+  if (pieces * 8 + tid < V) take(row[pieces * 8 + tid], pieces * 8 + tid);
+  unsigned long long m = ((unsigned long long)best << 32) | (0xffffffffu - at);
+#pragma unroll
+  for (int o = 32; o; o >>= 1) {
+    const unsigned long long other = __shfl_xor(m, o);
+    m = other > m ? other : m;
+  }
+  __shared__ unsigned long long red[kPickThreads / kWave];
+  if ((tid & 63) == 0) red[tid >> 6] = m;
+  __syncthreads();
+  if (tid == 0) {
+#pragma unroll
+    for (int i = 1; i < kPickThreads / kWave; ++i) m = red[i] > m ? red[i] : m;
+    tokens[(int64_t)blockIdx.x * ldt] = (int64_t)(0xffffffffu - (uint32_t)m);
+    if (positions) positions[blockIdx.x] += 1;
+  }
+}
+
+__global__ void step_state_kernel(fsvd_step_state* st, int64_t token, int32_t pos) {
+  st->pos = pos;
+  st->step = 0;
+  st->token = token;
+}
+
+__global__ void token_rows_kernel(int64_t* tokens, const int64_t* src, int32_t* positions, int32_t pos, int B) {
+  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= B) return;
+  tokens[b] = src[b];
+  positions[b] = pos;
+}
+
+static int launched(const char* fn) {
+  const hipError_t e = hipGetLastError();
+  if (e == hipSuccess) return kOk;
+  set_last_error("%s: launch failed: %s", fn, hipGetErrorString(e));
+  return kErrLaunch;
+}
+
+}  // namespace fsvd
+
+using namespace fsvd;
+
+extern "C" {
+
+int fsvd_greedy_token(const void* logits, int64_t ld, int64_t* tokens, int64_t ldt, int32_t* positions, int B, int V, int dtype, void* stream) {
+  const char* fn = "fsvd_greedy_token";
+  if (logits == nullptr || tokens == nullptr) { set_last_error("%s: argument %s is NULL", fn, logits == nullptr ? "logits" : "tokens"); return kErrNullPtr; }
+  if (B <= 0 || V <= 0) { set_last_error("%s: empty shape (B = %d, V = %d)", fn, B, V); return kErrBadShape; }
+  if (dtype != 0 && dtype != 1) { set_last_error("%s: dtype code %d (bf16 = 0 and fp16 = 1 are served)", fn, dtype); return kErrBadDtype; }
+  if ((reinterpret_cast<uintptr_t>(logits) & 1) != 0) { set_last_error("%s: logits must be 2-byte aligned", fn); return kErrBadAlign; }
+  const auto* x = static_cast<const uint16_t*>(logits);
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  if (dtype == 1) hipLaunchKernelGGL(greedy_token_kernel<1>, dim3(B), dim3(kPickThreads), 0, st, x, ld, tokens, ldt, positions, V);
+  else hipLaunchKernelGGL(greedy_token_kernel<0>, dim3(B), dim3(kPickThreads), 0, st, x, ld, tokens, ldt, positions, V);
+  return launched(fn);
+}
+
+int fsvd_decode_step_set_state(fsvd_step_state* state, int64_t token, int32_t position, void* stream) {
+  const char* fn = "fsvd_decode_step_set_state";
+  if (state == nullptr) { set_last_error("%s: argument state is NULL", fn); return kErrNullPtr; }
+  hipLaunchKernelGGL(step_state_kernel, dim3(1), dim3(1), 0, static_cast<hipStream_t>(stream), state, token, position);
+  return launched(fn);
+}
+
+int fsvd_set_token_rows(int64_t* tokens, const int64_t* src, int32_t* positions, int32_t position, int B, void* stream) {
+  const char* fn = "fsvd_set_token_rows";
+  if (tokens == nullptr || src == nullptr || positions == nullptr) { set_last_error("%s: a buffer is NULL", fn); return kErrNullPtr; }
+  if (B <= 0) { set_last_error("%s: empty shape (B = %d)", fn, B); return kErrBadShape; }
+  hipLaunchKernelGGL(token_rows_kernel, dim3((B + 255) / 256), dim3(256), 0, static_cast<hipStream_t>(stream), tokens, src, positions, position, B);
+  return launched(fn);
+}
+
+}  // extern "C"

@@ -58,11 +58,15 @@ class GraphedDecoder:
         self.warmup = int(warmup)
 
     def _step(self):
+        from . import hip_ops
         logits, hidden = self.model.decode_step(self.tokens, self.cache, self.positions, rope=self.rope,
                                                 attn_ws=self.attn_ws, nsplit=self.nsplit, return_hidden=True)
-        nxt = logits[:, -1, :].argmax(dim=-1, keepdim=True)
-        self.tokens.copy_(nxt)
-        self.positions.add_(1)
+        last = logits[:, -1, :]
+        if last.dtype in (torch.bfloat16, torch.float16) and last.stride(1) == 1:
+            hip_ops.greedy_token_(last, self.tokens, self.positions)
+        else:
+            self.tokens.copy_(last.argmax(dim=-1, keepdim=True))
+            self.positions.add_(1)
         return logits, hidden
 
     def eager_step(self):
@@ -90,10 +94,15 @@ class GraphedDecoder:
         torch.cuda.synchronize()
 
     def set_state(self, tokens: torch.Tensor, position: int) -> None:
+        from . import hip_ops
         if position < 0 or position >= self.cache.max_cache_len:
             raise IndexError(f"decode position {position} outside the cache (max {self.cache.max_cache_len})")
-        self.tokens.copy_(tokens.reshape(self.B, 1))
-        self.positions.fill_(int(position))
+        ids = tokens.reshape(self.B, 1)
+        if ids.dtype == torch.long and ids.device == self.tokens.device and ids.is_contiguous():
+            hip_ops.set_token_rows_(self.tokens, ids, self.positions, int(position))
+        else:
+            self.tokens.copy_(ids)
+            self.positions.fill_(int(position))
         self._host_pos = int(position)
 
     def step(self) -> torch.Tensor:

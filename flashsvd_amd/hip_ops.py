@@ -471,6 +471,43 @@ def _attn_decode_densekv_impl(q, k_cache, v_cache, cache_seqlens, k_new, v_new, 
     return out
 
 
+def greedy_token_(logits: torch.Tensor, tokens: torch.Tensor, positions: Optional[torch.Tensor] = None) -> None:
+    """``tokens[b] = logits[b].argmax()`` (ties to the lowest index, NaN above everything) and ``positions[b] += 1`` in one
+    launch; logits [B, V] with unit inner stride, tokens int64 [B, 1] or [B], positions int32 [B].  Custom operator
+    flashsvd_hip::greedy_token_ (tokens and positions are mutated arguments)."""
+    _OPS.greedy_token_.default(logits, tokens, positions)
+
+
+def _greedy_token_impl(logits, tokens, positions):
+    _, code = _elem(logits, "logits")
+    if logits.dim() != 2 or logits.stride(1) != 1:
+        raise ValueError(f"logits must be [B, V] with unit inner stride, got {tuple(logits.shape)} strides {logits.stride()}")
+    B, V = logits.shape
+    _need(tokens, "tokens", dtype=torch.long)
+    if tokens.numel() != B or tokens.shape[0] != B:
+        raise ValueError(f"tokens must hold {B} rows of one id, got {tuple(tokens.shape)}")
+    if positions is not None:
+        _need(positions, "positions", dtype=torch.int32)
+        if positions.shape != (B,) or not positions.is_contiguous():
+            raise ValueError(f"positions must be a contiguous [{B}] tensor")
+    rc = _lib.load().fsvd_greedy_token(logits.data_ptr(), logits.stride(0), tokens.data_ptr(), tokens.stride(0), _ptr(positions), B, V, code,
+                                       _stream())
+    _lib.check("fsvd_greedy_token", rc)
+
+
+def set_token_rows_(tokens: torch.Tensor, src: torch.Tensor, positions: torch.Tensor, position: int) -> None:
+    """``tokens.copy_(src)`` and ``positions.fill_(position)`` in one launch (contiguous int64 / int64 / int32 of the same
+    number of rows on one device)."""
+    _need(tokens, "tokens", dtype=torch.long)
+    _need(src, "src", dtype=torch.long)
+    _need(positions, "positions", dtype=torch.int32)
+    if not (tokens.is_contiguous() and src.is_contiguous() and positions.is_contiguous() and tokens.numel() == src.numel() == positions.numel()):
+        raise ValueError("tokens, src and positions must be contiguous and of one length")
+    with torch.cuda.device(tokens.device):
+        rc = _lib.load().fsvd_set_token_rows(tokens.data_ptr(), src.data_ptr(), positions.data_ptr(), int(position), tokens.numel(), _stream())
+    _lib.check("fsvd_set_token_rows", rc)
+
+
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """w * bf16(x * rsqrt(mean(x^2) + eps)); custom operator flashsvd_hip::rmsnorm."""
     return _OPS.rmsnorm.default(x, weight, float(eps)) if out is None else _OPS.rmsnorm.out(x, weight, float(eps), out=out)

@@ -504,10 +504,11 @@ class PersistentDecoder:
         if position < 0 or position >= self.S:
             raise IndexError(f"decode position {position} outside the cache (max {self.S})")
         tok = int(token.reshape(-1)[0].item()) if torch.is_tensor(token) else int(token)
-        st = self.state
-        st[2] = int(position)
-        st[3] = 0
-        st.view(torch.int64)[2] = tok
+        if not -(1 << 63) <= tok < 1 << 63:
+            raise RuntimeError(f"token {tok} does not fit 64 bits")
+        with torch.cuda.device(self.state.device):
+            _lib.check("fsvd_decode_step_set_state",
+                       self.lib.fsvd_decode_step_set_state(self.state.data_ptr(), tok, int(position), torch.cuda.current_stream().cuda_stream))
         self._host_pos = int(position)
         self._host_steps = 0
 

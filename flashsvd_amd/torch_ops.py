@@ -8,6 +8,7 @@ tensors.  ``flashsvd_amd.hip_ops`` and the modules under ``flashsvd_amd.kernels`
   linear / linear.out                 fsvd_linear            rank projections, factor pairs, fused RMSNorm / residual
   swiglu_linear / .out                fsvd_swiglu_linear     gate_u / up_u pair + SwiGLU
   rmsnorm / .out                      fsvd_rmsnorm
+  greedy_token_                       fsvd_greedy_token      argmax of every row + position increment
   qkv_rope_append / .out              fsvd_qkv_rope_append   head expansion + RoPE + dense-cache append
   attn_decode_densekv / .out          fsvd_attn_decode_densekv(_static)   the flash_attn_with_kvcache role
   attn_decode_rankkv / .out           fsvd_attn_decode_rankkv             decode over the rank-space cache
@@ -92,6 +93,15 @@ _define("rmsnorm(Tensor x, Tensor weight, float eps=1e-6) -> Tensor", _rmsnorm,
         lambda x, weight, eps=1e-6: torch.empty_like(x, memory_format=torch.contiguous_format))
 _define("rmsnorm.out(Tensor x, Tensor weight, float eps=1e-6, *, Tensor(a!) out) -> Tensor(a!)", _rmsnorm_out,
         lambda *a, out, **k: out)
+
+
+# ------------------------------------------------------------------ greedy token of every row
+def _greedy_token(logits, tokens, positions=None):
+    from . import hip_ops
+    hip_ops._greedy_token_impl(logits, tokens, positions)
+
+
+_define("greedy_token_(Tensor logits, Tensor(a!) tokens, Tensor(b!)? positions=None) -> ()", _greedy_token, lambda *a, **k: None)
 
 
 # ------------------------------------------------------------------ q / k / v expansion + RoPE + cache append
@@ -243,5 +253,5 @@ _define("mlp_dual_split(Tensor PUp, Tensor PGate, Tensor GateU, Tensor UpU, Tens
         PUp.new_empty((PUp.shape[0], DownU.shape[1])))
 
 ops = getattr(torch.ops, NS)
-OP_NAMES = ("linear", "swiglu_linear", "rmsnorm", "qkv_rope_append", "attn_decode_densekv", "attn_decode_rankkv", "rankkv_append", "linear_rankkv_append",
+OP_NAMES = ("linear", "swiglu_linear", "rmsnorm", "greedy_token_", "qkv_rope_append", "attn_decode_densekv", "attn_decode_rankkv", "rankkv_append", "linear_rankkv_append",
             "lowrank_expand_heads", "rope_attn_prefill", "reconstruct_qkv_token", "xw_linear", "mlp_dual_split")

@@ -160,6 +160,14 @@ int fsvd_attn_decode_densekv_static(const void* q, int64_t sq_b, int64_t sq_h,
 int fsvd_rmsnorm(const void* x, int64_t ldx, const void* w, float eps, void* y, int64_t ldy, int rows, int K, int dtype,
                  void* stream);
 
+/* tokens[b * ldt] = the greedy token of row b of logits [B, V] (rows ld elements apart, at any element's address): the lowest
+ * index of the largest value, NaN above everything, as torch.argmax has it.  positions, when given: positions[b] += 1. */
+int fsvd_greedy_token(const void* logits, int64_t ld, int64_t* tokens, int64_t ldt, int32_t* positions, int B, int V, int dtype,
+                      void* stream);
+/* tokens[b] = src[b], positions[b] = position for b < B, in one launch. */
+int fsvd_set_token_rows(int64_t* tokens, const int64_t* src, int32_t* positions, int32_t position, int B, void* stream);
+
+
 /* ---------------------------------------------------------------------------------------------
  * Reference operand layouts ("x @ W", W is [K, N]).  dtype is FSVD_BF16 / FSVD_FP16 / FSVD_FP32;
  * accumulation is fp32 with one rounding at the store.  Workspaces: bytes from the matching
@@ -426,6 +434,9 @@ typedef struct fsvd_step_state {
   int32_t err_wg;     /* workgroup that raised err                                                            */
   int32_t spin_limit; /* polls before a workgroup gives up; 0 = default (about a second)                       */
 } fsvd_step_state;
+
+/* Next input token and its position (state->pos, ->token; ->step = 0) in one launch on `stream`. */
+int fsvd_decode_step_set_state(fsvd_step_state* state, int64_t token, int32_t position, void* stream);
 
 /* Workgroups the step kernel runs with on the current device (one per compute unit), or 0 with fsvd_last_error() when
  * the device cannot hold one workgroup of the kernel per compute unit (the grid must be co-resident: workgroups wait
