@@ -86,6 +86,26 @@ class StepState(ctypes.Structure):
                 ("token", c_int64), ("err_wg", ctypes.c_int32), ("spin_limit", ctypes.c_int32)]
 
 
+class MlpBlock(ctypes.Structure):
+    """fsvd_mlp_block."""
+    _fields_ = [("x", c_void_p), ("ldx", c_int64), ("norm_w", c_void_p), ("xn", c_void_p), ("gu_v", c_void_p), ("ldgv", c_int64),
+                ("p", c_void_p), ("ldp", c_int64), ("up", c_void_p), ("gate_u", c_void_p), ("up_u", c_void_p), ("ldu", c_int64),
+                ("h", c_void_p), ("down_v", c_void_p), ("ldv", c_int64), ("s", c_void_p), ("down_u", c_void_p), ("ldd", c_int64),
+                ("bias", c_void_p), ("res", c_void_p), ("ldres", c_int64), ("y", c_void_p), ("ldy", c_int64), ("eps", c_float),
+                *((n, ctypes.c_int32) for n in ("B", "K", "R", "D", "Rd", "N", "mode", "dtype"))]
+
+
+class AttnBlock(ctypes.Structure):
+    """fsvd_attn_block."""
+    _fields_ = [("x", c_void_p), ("ldx", c_int64), ("norm_w", c_void_p), ("xn", c_void_p), ("qkv_v", c_void_p), ("ldqkv", c_int64),
+                ("p", c_void_p), ("q_u", c_void_p), ("k_u", c_void_p), ("v_u", c_void_p), ("ldq", c_int64), ("ldk", c_int64), ("ldvu", c_int64),
+                ("cos", c_void_p), ("sin", c_void_p), ("k_cache", c_void_p), ("v_cache", c_void_p), ("sc_b", c_int64), ("sc_s", c_int64),
+                ("sc_h", c_int64), ("q", c_void_p), ("a", c_void_p), ("o_v", c_void_p), ("ldov", c_int64), ("o_v_bias", c_void_p),
+                ("po", c_void_p), ("o_u", c_void_p), ("ldou", c_int64), ("o_u_bias", c_void_p), ("res", c_void_p), ("ldres", c_int64),
+                ("y", c_void_p), ("ldy", c_int64), ("eps", c_float),
+                *((n, ctypes.c_int32) for n in ("B", "M", "K", "Rq", "Rk", "Rv", "H", "Hk", "Dh", "S", "start", "rope_len", "Ro", "N", "dtype"))]
+
+
 PH_EMBED, PH_GEMV, _PH_RESERVED, PH_ATTN, PH_MERGE, PH_ARGMAX = range(6)
 EP_STORE, EP_RESID, EP_SWIGLU, EP_LOGITS, EP_F32 = range(5)
 PF_NOWAIT, PF_STAGE2, PF_SPLIT, PF_LEAD = 1, 2, 4, 8
@@ -152,6 +172,8 @@ SIGNATURES = {
     "fsvd_decode_step_set_state": (c_int, [c_void_p, c_int64, ctypes.c_int32, c_void_p]),
     "fsvd_greedy_token": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_void_p]),
     "fsvd_set_token_rows": (c_int, [c_void_p, c_void_p, c_void_p, ctypes.c_int32, c_int, c_void_p]),
+    "fsvd_mlp_block_run": (c_int, [ctypes.POINTER(MlpBlock), c_void_p]),
+    "fsvd_attn_block_prefill": (c_int, [ctypes.POINTER(AttnBlock), c_void_p]),
     "fsvd_set_workspace": (c_int, [c_void_p, c_size_t, c_void_p]),
     "fsvd_decode_step": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_int, c_void_p]),
     "fsvd_decode_step_trace": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_size_t, c_int, c_void_p]),

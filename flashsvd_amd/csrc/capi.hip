@@ -595,6 +595,97 @@ int fsvd_attn_prefill(const void* q, int64_t sq_b, int64_t sq_m, int64_t sq_h, c
   return launch_prefill_attn(a, static_cast<hipStream_t>(stream));
 }
 
+// one projection of a block: contiguous rows in and out unless said otherwise
+static int block_linear(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* bias, const void* norm_w, float eps, const void* res,
+                        int64_t ldres, void* y, int64_t ldy, int B, int N, int K, int dtype, void* stream) {
+  return fsvd_linear(x, ldx, W, ldw, bias, norm_w, eps, res, ldres, y, ldy, B, N, K, 0, dtype, stream);
+}
+// the rank projection in front of a block: three rows and more are normalised once up front, fewer in the projection's own launch
+static int block_input(const void* x, int64_t ldx, const void* norm_w, float eps, void* xn, const void* W, int64_t ldw, void* p, int64_t ldp, int B,
+                       int N, int K, int dtype, const char* fn, void* stream) {
+  if (norm_w != nullptr && B >= 3) {
+    FSVD_REQUIRE_PTR(xn, fn);
+    const int rc = fsvd_rmsnorm(x, ldx, norm_w, eps, xn, K, B, K, dtype, stream);
+    if (rc != kOk) return rc;
+    x = xn; ldx = K; norm_w = nullptr;
+  }
+  return block_linear(x, ldx, W, ldw, nullptr, norm_w, eps, nullptr, 0, p, ldp, B, N, K, dtype, stream);
+}
+
+int fsvd_mlp_block_run(const fsvd_mlp_block* d, void* stream) {
+  const char* fn = "fsvd_mlp_block_run";
+  FSVD_REQUIRE_PTR(d, fn);
+  const fsvd_mlp_block& b = *d;
+  FSVD_REQUIRE_PTR(b.p, fn); FSVD_REQUIRE_PTR(b.gate_u, fn); FSVD_REQUIRE_PTR(b.up_u, fn); FSVD_REQUIRE_PTR(b.h, fn);
+  FSVD_REQUIRE_PTR(b.down_v, fn); FSVD_REQUIRE_PTR(b.s, fn); FSVD_REQUIRE_PTR(b.down_u, fn); FSVD_REQUIRE_PTR(b.y, fn);
+  if (b.R <= 0 || b.ldp < (b.up ? b.R : 2 * (int64_t)b.R) || b.ldu < b.R || (b.mode != 0 && b.mode != 1) || (b.x && b.up)) {
+    set_last_error("%s: inconsistent layout (ldp=%lld R=%d ldu=%lld mode=%d)", fn, (long long)b.ldp, b.R, (long long)b.ldu, b.mode);
+    return kErrBadShape;
+  }
+  int rc;
+  if (b.x != nullptr) {
+    FSVD_REQUIRE_PTR(b.gu_v, fn);
+    rc = block_input(b.x, b.ldx, b.norm_w, b.eps, b.xn, b.gu_v, b.ldgv, b.p, b.ldp, b.B, 2 * b.R, b.K, b.dtype, fn, stream);
+    if (rc != kOk) return rc;
+  }
+  // the two sets of coefficients may be tensors of their own: a signed distance in elements
+  const int64_t bytes = b.up ? (int64_t)(reinterpret_cast<intptr_t>(b.up) - reinterpret_cast<intptr_t>(b.p)) : 2 * (int64_t)b.R;
+  if (bytes & 1) { set_last_error("%s: coefficients at an odd address", fn); return kErrBadAlign; }
+  SwigluArgs a{cu16(b.p), b.ldp, bytes / 2, cu16(b.gate_u), cu16(b.up_u), b.ldu, u16(b.h), b.D, b.B, b.D, b.R, b.mode, b.dtype};
+  rc = launch_swiglu(a, 0, static_cast<hipStream_t>(stream));
+  if (rc != kOk) return rc;
+  rc = block_linear(b.h, b.D, b.down_v, b.ldv, nullptr, nullptr, 0.f, nullptr, 0, b.s, b.Rd, b.B, b.Rd, b.D, b.dtype, stream);
+  if (rc != kOk) return rc;
+  return block_linear(b.s, b.Rd, b.down_u, b.ldd, b.bias, nullptr, 0.f, b.res, b.ldres, b.y, b.ldy, b.B, b.N, b.Rd, b.dtype, stream);
+}
+
+int fsvd_attn_block_prefill(const fsvd_attn_block* d, void* stream) {
+  const char* fn = "fsvd_attn_block_prefill";
+  FSVD_REQUIRE_PTR(d, fn);
+  const fsvd_attn_block& b = *d;
+  FSVD_REQUIRE_PTR(b.x, fn); FSVD_REQUIRE_PTR(b.qkv_v, fn); FSVD_REQUIRE_PTR(b.p, fn); FSVD_REQUIRE_PTR(b.q_u, fn); FSVD_REQUIRE_PTR(b.k_u, fn);
+  FSVD_REQUIRE_PTR(b.v_u, fn); FSVD_REQUIRE_PTR(b.cos, fn); FSVD_REQUIRE_PTR(b.sin, fn); FSVD_REQUIRE_PTR(b.k_cache, fn); FSVD_REQUIRE_PTR(b.v_cache, fn);
+  FSVD_REQUIRE_PTR(b.q, fn); FSVD_REQUIRE_PTR(b.a, fn); FSVD_REQUIRE_PTR(b.o_v, fn); FSVD_REQUIRE_PTR(b.po, fn); FSVD_REQUIRE_PTR(b.o_u, fn);
+  FSVD_REQUIRE_PTR(b.y, fn);
+  if (b.dtype != 0 && b.dtype != 1) { set_last_error("%s: dtype code %d (bf16 = 0 and fp16 = 1 are served)", fn, b.dtype); return kErrBadDtype; }
+  const int64_t rows64 = (int64_t)b.B * b.M;
+  if (b.B <= 0 || b.M <= 0 || rows64 > 0x7fffffff || b.start < 0 || b.S <= 0 || (int64_t)b.start + b.M > b.S || b.rope_len <= 0 || b.Rq <= 0 || b.Rk <= 0 ||
+      b.Rv <= 0 || b.H <= 0 || b.Hk <= 0 || b.H % b.Hk || b.Dh <= 0 || b.ldq < b.Rq || b.ldk < b.Rk || b.ldvu < b.Rv || b.sc_h < b.Dh) {
+    set_last_error("%s: bad shape (B=%d M=%d start=%d S=%d ranks %d, %d, %d, heads %d, %d)", fn, b.B, b.M, b.start, b.S, b.Rq, b.Rk, b.Rv, b.H, b.Hk);
+    return kErrBadShape;
+  }
+  const int rows = (int)rows64, Rt = b.Rq + b.Rk + b.Rv, w = b.H * b.Dh;
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  int rc = block_input(b.x, b.ldx, b.norm_w, b.eps, b.xn, b.qkv_v, b.ldqkv, b.p, Rt, rows, Rt, b.K, b.dtype, fn, stream);
+  if (rc != kOk) return rc;
+  const auto expansion = [&](int at, const void* u, int64_t ldu, int R, int heads, bool rotate, void* y, int64_t sy_b, int64_t sy_m, int64_t sy_h, int by_pos, int dst) {
+    ExpandArgs e{cu16(b.p) + at, (int64_t)b.M * Rt, Rt, 0, cu16(u), ldu, nullptr, rotate ? cu16(b.cos) : nullptr, rotate ? cu16(b.sin) : nullptr, b.rope_len,
+                 nullptr, u16(y), sy_b, sy_m, sy_h, by_pos, dst, b.B, b.M, heads, b.Dh, R, b.dtype};
+    e.pos0 = b.start;
+    return e;
+  };
+  const ExpandArgs e[3] = {expansion(0, b.q_u, b.ldq, b.Rq, b.H, true, b.q, (int64_t)b.M * w, w, b.Dh, 0, b.M),
+                           expansion(b.Rq, b.k_u, b.ldk, b.Rk, b.Hk, true, b.k_cache, b.sc_b, b.sc_s, b.sc_h, 1, b.S),
+                           expansion(b.Rq + b.Rk, b.v_u, b.ldvu, b.Rv, b.Hk, false, b.v_cache, b.sc_b, b.sc_s, b.sc_h, 1, b.S)};
+  if (expand_multi_apply(e, 3)) {
+    rc = launch_expand_multi(e, 3, st);
+    if (rc != kOk) return rc;
+  } else {
+    for (int k = 0; k < 3; ++k) {
+      rc = launch_expand(e[k], st);
+      if (rc != kOk) return rc;
+    }
+  }
+  PrefillAttnArgs t{cu16(b.q), (int64_t)b.M * w, w, b.Dh, cu16(b.k_cache), cu16(b.v_cache), b.sc_b, b.sc_s, b.sc_h, nullptr, nullptr, 0, nullptr, 0, 0,
+                    u16(b.a), (int64_t)b.M * w, w, b.Dh, b.B, b.M, b.H, b.Hk, b.Dh, b.S, 1, 1.0f / sqrtf((float)b.Dh), b.dtype};
+  t.pos0 = b.start;
+  rc = launch_prefill_attn(t, st);
+  if (rc != kOk) return rc;
+  rc = block_linear(b.a, w, b.o_v, b.ldov, b.o_v_bias, nullptr, 0.f, nullptr, 0, b.po, b.Ro, rows, b.Ro, w, b.dtype, stream);
+  if (rc != kOk) return rc;
+  return block_linear(b.po, b.Ro, b.o_u, b.ldou, b.o_u_bias, nullptr, 0.f, b.res, b.ldres, b.y, b.ldy, rows, b.N, b.Ro, b.dtype, stream);
+}
+
 int fsvd_decode_step_workgroups(void) { return decode_step_workgroups(); }
 
 int fsvd_decode_step_prepare(fsvd_phase* phases_host, int nphase, int workgroups) {

@@ -142,6 +142,7 @@ struct ExpandArgs {
   int dst_rows;                                     // rows the destination has (bounds check)
   int B, M, heads, Dh, R;
   int dt = 0;
+  int pos0 = 0;                                     // position of token 0 of every row where positions is null
 };
 struct PrefillAttnArgs {
   const uint16_t* q; int64_t sq_b, sq_m, sq_h;      // [B,M,H,Dh], rotated
@@ -153,6 +154,7 @@ struct PrefillAttnArgs {
   int B, M, H, Hk, Dh, S, causal;
   float scale;
   int dt = 0;
+  int pos0 = 0;                                     // position of query row 0 where q_pos0 is null
 };
 int launch_expand(const ExpandArgs& a, hipStream_t st);
 bool expand_tiles_apply(const ExpandArgs& a);                               // mfma_gemm.hip
@@ -182,6 +184,7 @@ struct ExpandEpi {
   int64_t sp_b, sp_m;                      // strides of the coefficient rows
   int64_t sy_b, sy_m, sy_h;                // destination strides
   int dst_by_position, dst_rows;
+  int pos0;
 };
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 // byte offsets of `rows` rows of stride ld fit the 32 unsigned bits of a buffer load

@@ -53,7 +53,7 @@ struct BigProblem {
   const uint16_t* cos; const uint16_t* sin; int rope_len;
   const int32_t* positions;
   int M; int64_t sp_b, sp_m, sy_b, sy_m, sy_h;
-  int dst_by_position, dst_rows;
+  int dst_by_position, dst_rows, pos0;
 };
 struct BigArgs { BigProblem p[3]; int first_tile[4]; int rows, nt; };   // column tiles of problem i: [first_tile[i], first_tile[i + 1])
 
@@ -219,7 +219,7 @@ __global__ __launch_bounds__(kBigThreads, 2) void gemm_big_kernel(BigArgs args) 
         for (int i = 0; i < 8; ++i) {
           const int m = cur.m0 + wm * 128 + i * 16 + lr;
           const int mc = min(m, args.rows - 1), b = mc / a.M, tok = mc - b * a.M;
-          const int pos = (a.positions ? a.positions[b] : 0) + tok;
+          const int pos = (a.positions ? a.positions[b] : a.pos0) + tok;
           const int tp = min(max(pos, 0), a.rope_len - 1);
           uint32_t o[2][2][2];                       // [half][tile j][word]
 #pragma unroll
@@ -410,7 +410,7 @@ int launch_expand_big(const ExpandArgs* d, int n, hipStream_t st) {
     BigProblem& p = a.p[i];
     p.x = e.p; p.W = e.u; p.ldw = e.ldu; p.bias = e.bias; p.y = e.y; p.N = e.heads * 128; p.K = e.R;
     p.cos = e.cos; p.sin = e.sin; p.rope_len = e.rope_len; p.positions = e.positions; p.M = e.M; p.sp_b = e.sp_b; p.sp_m = e.sp_m;
-    p.sy_b = e.sy_b; p.sy_m = e.sy_m; p.sy_h = e.sy_h; p.dst_by_position = e.dst_by_position; p.dst_rows = e.dst_rows;
+    p.sy_b = e.sy_b; p.sy_m = e.sy_m; p.sy_h = e.sy_h; p.dst_by_position = e.dst_by_position; p.dst_rows = e.dst_rows; p.pos0 = e.pos0;
     a.first_tile[i] = tiles;
     tiles += (e.heads + 1) / 2;
   }

@@ -394,7 +394,7 @@ __device__ __forceinline__ void gemm_tiles_body(const MfmaArgs& a, const ExpandE
     if (m >= a.B) continue;
     if (EXPAND) {
       const int b = m / ep.M, t = m - b * ep.M;
-      const int pos = (ep.positions ? ep.positions[b] : 0) + t;
+      const int pos = (ep.positions ? ep.positions[b] : ep.pos0) + t;
       const int slot = ep.dst_by_position ? pos : t;
       if (slot < 0 || slot >= ep.dst_rows) continue;   // outside the destination: dropped
       const int head = tile_n;
@@ -694,7 +694,7 @@ static int launch_expand_tiles_t(const ExpandArgs& a, hipStream_t st) {
   }
   const int rows = a.B * a.M;
   MfmaArgs g{a.p, 0, 0, a.u, nullptr, a.ldu, a.bias, nullptr, 0, a.y, 0, rows, a.heads * 128, a.R, 0};
-  ExpandEpi ep{a.cos, a.sin, a.rope_len, a.positions, a.M, a.sp_b, a.sp_m, a.sy_b, a.sy_m, a.sy_h, a.dst_by_position, a.dst_rows};
+  ExpandEpi ep{a.cos, a.sin, a.rope_len, a.positions, a.M, a.sp_b, a.sp_m, a.sy_b, a.sy_m, a.sy_h, a.dst_by_position, a.dst_rows, a.pos0};
   const dim3 grid(a.heads, (rows + BM - 1) / BM);
   set_last_form(WTM == 4 ? "tiles 128 x 128 heads" : "tiles 64 x 128 heads");
   hipLaunchKernelGGL((gemm_tiles_kernel<DT, false, WTM, 4, PF, true, kGBK, 4, true>), grid, dim3(kGT4), lds, st, g, ep);
@@ -720,7 +720,7 @@ static int launch_expand_multi_t(const ExpandArgs* d, int n, hipStream_t st) {
   for (int k = 0; k < 3; ++k) {
     const ExpandArgs& a = d[k < n ? k : n - 1];
     eb.a[k] = MfmaArgs{a.p, 0, 0, a.u, nullptr, a.ldu, a.bias, nullptr, 0, a.y, 0, rows, a.heads * 128, a.R, 0};
-    eb.ep[k] = ExpandEpi{a.cos, a.sin, a.rope_len, a.positions, a.M, a.sp_b, a.sp_m, a.sy_b, a.sy_m, a.sy_h, a.dst_by_position, a.dst_rows};
+    eb.ep[k] = ExpandEpi{a.cos, a.sin, a.rope_len, a.positions, a.M, a.sp_b, a.sp_m, a.sy_b, a.sy_m, a.sy_h, a.dst_by_position, a.dst_rows, a.pos0};
     eb.first_head[k] = heads;
     if (k < n) heads += a.heads;
   }

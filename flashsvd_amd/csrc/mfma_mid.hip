@@ -178,7 +178,7 @@ __global__ __launch_bounds__(kMidThreads, 2) void gemm_mid_kernel(MidArgs args) 
     if (m >= a.B) continue;
     if constexpr (HEADS) {
       const int b = m / ep.M, tok = m - b * ep.M;
-      const int pos = (ep.positions ? ep.positions[b] : 0) + tok;
+      const int pos = (ep.positions ? ep.positions[b] : ep.pos0) + tok;
       const int slot = ep.dst_by_position ? pos : tok;
       if (slot < 0 || slot >= ep.dst_rows) continue;             // outside the destination: dropped
       uint16_t* dst = a.y + (int64_t)b * ep.sy_b + (int64_t)slot * ep.sy_m + (int64_t)head * ep.sy_h;
@@ -366,7 +366,7 @@ int launch_expand_mid(const ExpandArgs* d, int n, hipStream_t st) {
   for (int k = 0; k < n; ++k) {
     const ExpandArgs& a = d[k];
     m.a[k] = MfmaArgs{a.p, 0, 0, a.u, nullptr, a.ldu, a.bias, nullptr, 0, a.y, 0, rows, a.heads * 128, a.R, 0};
-    m.ep[k] = ExpandEpi{a.cos, a.sin, a.rope_len, a.positions, a.M, a.sp_b, a.sp_m, a.sy_b, a.sy_m, a.sy_h, a.dst_by_position, a.dst_rows};
+    m.ep[k] = ExpandEpi{a.cos, a.sin, a.rope_len, a.positions, a.M, a.sp_b, a.sp_m, a.sy_b, a.sy_m, a.sy_h, a.dst_by_position, a.dst_rows, a.pos0};
     m.first_head[k] = heads;
     heads += a.heads;
   }

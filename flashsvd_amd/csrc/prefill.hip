@@ -80,7 +80,7 @@ __global__ __launch_bounds__(kPfThreads) void lowrank_expand_kernel(ExpandArgs a
       const int r = row0 + mi * 16 + lg * 4 + i;
       if (r >= T) continue;
       const int b = r / a.M, m = r % a.M;
-      const int pos = (a.positions ? a.positions[b] : 0) + m;
+      const int pos = (a.positions ? a.positions[b] : a.pos0) + m;
       float x[NT];
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(kPfThreads * NG, NG == 1 ? 2 : 1) void attn_prefill
   const int hk = h / (a.H / a.Hk);
   const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;   // thread and wave within the group
   const int lr = lane & 15, lg = lane >> 4;
-  const int q0 = a.q_pos0 ? a.q_pos0[b] : 0;
+  const int q0 = a.q_pos0 ? a.q_pos0[b] : a.pos0;
   const int m_base = mt * BM + wave * QW;
   const int n_keys_all = max(1, min(q0 + a.M, a.S));
 

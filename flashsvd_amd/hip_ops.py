@@ -594,6 +594,135 @@ def _lowrank_expand_heads_impl(p, u, num_heads, head_dim, out, cos, sin, positio
     return out
 
 
+def _weights2d(dt, **ts) -> None:
+    for nm, t in ts.items():
+        _need(t, nm, dtype=dt)
+        if t.dim() != 2 or t.stride(1) != 1:
+            raise ValueError(f"{nm} must be a 2-d weight with unit inner stride, got {tuple(t.shape)} strides {t.stride()}")
+
+
+def _row_vector(dt, t, n: int, nm: str) -> Optional[int]:
+    if t is None:
+        return None
+    _need(t, nm, dtype=dt)
+    if t.shape != (n,) or not t.is_contiguous():
+        raise ValueError(f"{nm} must be a contiguous [{n}] tensor")
+    return t.data_ptr()
+
+
+def _residual_rows(dt, t, B: int, N: int):
+    """(tensor to keep alive, address, row stride) of a residual of B rows of N."""
+    if t is None:
+        return None, None, 0
+    _need(t, "residual", dtype=dt)
+    t, p, ld, rows, cols = _row_operand(t, "residual")
+    if rows != B or cols != N:
+        raise ValueError(f"residual shape {tuple(t.shape)} does not match output [{B}, {N}]")
+    return t, p, ld
+
+
+def _buffers(dt, device, *counts):
+    """One allocation for the intermediates of a block: (tensor, addresses), each 512-byte aligned as an allocation of its own."""
+    ends, n = [], 0
+    for c in counts:
+        ends.append(n)
+        n += (c + 255) // 256 * 256
+    buf = torch.empty(max(n, 1), dtype=dt, device=device)
+    base = buf.data_ptr()
+    return buf, [base + 2 * e for e in ends]
+
+
+def lowrank_mlp(x: torch.Tensor, gu_v: torch.Tensor, gate_u: torch.Tensor, up_u: torch.Tensor, down_v: torch.Tensor, down_u: torch.Tensor, *,
+                norm_weight: Optional[torch.Tensor] = None, eps: float = 1e-6, residual: Optional[torch.Tensor] = None, mode: int = 0) -> torch.Tensor:
+    """(residual +) down_u(down_v(silu(gate_u g) * up_u u)) with [g | u] = gu_v norm(x): the launches of :func:`linear`,
+    :func:`swiglu_linear` and twice :func:`linear` issued by one native call.  Custom operator flashsvd_hip::lowrank_mlp."""
+    return _OPS.lowrank_mlp.default(x, gu_v, gate_u, up_u, down_v, down_u, norm_weight, float(eps), residual, int(mode))
+
+
+def _lowrank_mlp_impl(x, gu_v, gate_u, up_u, down_v, down_u, norm_weight, eps, residual, mode):
+    dt, code = _elem(x, "x")
+    _weights2d(dt, gu_v=gu_v, gate_u=gate_u, up_u=up_u, down_v=down_v, down_u=down_u)
+    (two_r, K), (D, R), (Rd, Dv), (N, Ru) = gu_v.shape, gate_u.shape, down_v.shape, down_u.shape
+    if two_r != 2 * R or up_u.shape != gate_u.shape or up_u.stride() != gate_u.stride() or Dv != D or Ru != Rd or x.shape[-1] != K:
+        raise ValueError(f"factors do not match: x [.., {x.shape[-1]}], gu_v {tuple(gu_v.shape)}, gate_u {tuple(gate_u.shape)}, up_u {tuple(up_u.shape)}, "
+                         f"down_v {tuple(down_v.shape)}, down_u {tuple(down_u.shape)}")
+    nw = _row_vector(dt, norm_weight, K, "norm_weight")
+    x2, xp, ldx, B, _ = _row_operand(x, "x")
+    out = torch.empty(*x.shape[:-1], N, device=x.device, dtype=dt)
+    keep, rp, ldr = _residual_rows(dt, residual, B, N)
+    if B >= 3:
+        ensure_split_workspace(x.device)
+    # the normalised rows are read by the rank projection only: the down projection's coefficients take their place
+    buf, (xs, p, h) = _buffers(dt, x.device, max(B * K if nw and B >= 3 else 0, B * Rd), B * two_r, B * D)
+    b = _lib.MlpBlock(xp, ldx, nw, xs, gu_v.data_ptr(), gu_v.stride(0), p, two_r, None, gate_u.data_ptr(), up_u.data_ptr(), gate_u.stride(0),
+                      h, down_v.data_ptr(), down_v.stride(0), xs, down_u.data_ptr(), down_u.stride(0), None, rp, ldr, out.data_ptr(), N,
+                      float(eps), B, K, R, D, Rd, N, int(mode), code)
+    _lib.check("fsvd_mlp_block_run", _lib.load().fsvd_mlp_block_run(b, _stream()))
+    return out
+
+
+def _mlp_from_coefficients(pg, pu, gate_u, up_u, down_v, down_u, bias, mode):
+    """The same from gate and up coefficients [B, R] of one row stride, which may be tensors of their own."""
+    dt, code = _elem(pg, "pg")
+    _weights2d(dt, gate_u=gate_u, up_u=up_u, down_v=down_v, down_u=down_u, pg=pg, pu=pu)
+    (D, R), (Rd, Dv), (N, Ru) = gate_u.shape, down_v.shape, down_u.shape
+    if pg.shape != pu.shape or pg.stride() != pu.stride() or pg.shape[1] != R or up_u.shape != gate_u.shape or up_u.stride() != gate_u.stride() \
+            or Dv != D or Ru != Rd:
+        raise ValueError("coefficients and factors do not match")
+    B = pg.shape[0]
+    bp = _row_vector(dt, bias, N, "bias")
+    out = torch.empty(B, N, device=pg.device, dtype=dt)
+    if B >= 3:
+        ensure_split_workspace(pg.device)
+    buf, (h, s) = _buffers(dt, pg.device, B * D, B * Rd)
+    b = _lib.MlpBlock(None, 0, None, None, None, 0, pg.data_ptr(), pg.stride(0), pu.data_ptr(), gate_u.data_ptr(), up_u.data_ptr(), gate_u.stride(0),
+                      h, down_v.data_ptr(), down_v.stride(0), s, down_u.data_ptr(), down_u.stride(0), bp, None, 0, out.data_ptr(), N,
+                      0.0, B, 0, R, D, Rd, N, int(mode), code)
+    _lib.check("fsvd_mlp_block_run", _lib.load().fsvd_mlp_block_run(b, _stream()))
+    return out
+
+
+def lowrank_attn_prefill(x: torch.Tensor, qkv_v: torch.Tensor, q_u: torch.Tensor, k_u: torch.Tensor, v_u: torch.Tensor, o_v: torch.Tensor,
+                         o_u: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, *, start: int,
+                         num_heads: int, num_kv_heads: int, norm_weight: Optional[torch.Tensor] = None, eps: float = 1e-6,
+                         residual: Optional[torch.Tensor] = None, o_v_bias: Optional[torch.Tensor] = None,
+                         o_u_bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """The attention half of a prompt pass over the dense cache: x [B, T, K] at positions start .. start + T - 1, keys and values
+    into the cache rows of those positions, (residual +) o_u(o_v(attention)).  The launches of :func:`linear`,
+    :func:`lowrank_expand_heads_multi`, :func:`attn_prefill` and twice :func:`linear` issued by one native call.  Custom
+    operator flashsvd_hip::lowrank_attn_prefill (the caches are mutated arguments)."""
+    return _OPS.lowrank_attn_prefill.default(x, qkv_v, q_u, k_u, v_u, o_v, o_u, k_cache, v_cache, cos, sin, int(start), int(num_heads),
+                                             int(num_kv_heads), norm_weight, float(eps), residual, o_v_bias, o_u_bias)
+
+
+def _lowrank_attn_prefill_impl(x, qkv_v, q_u, k_u, v_u, o_v, o_u, k_cache, v_cache, cos, sin, start, num_heads, num_kv_heads, norm_weight, eps,
+                               residual, o_v_bias, o_u_bias):
+    dt, code = _elem(x, "x")
+    _weights2d(dt, qkv_v=qkv_v, q_u=q_u, k_u=k_u, v_u=v_u, o_v=o_v, o_u=o_u)
+    _need(k_cache, "k_cache", dtype=dt); _need(v_cache, "v_cache", dtype=dt)
+    if x.dim() != 3 or k_cache.dim() != 4 or k_cache.shape != v_cache.shape or k_cache.stride() != v_cache.stride() or k_cache.stride(3) != 1:
+        raise ValueError("x must be [B, T, K] and the caches matching [B, S, Hk, Dh] with unit inner stride")
+    H, Hk = int(num_heads), int(num_kv_heads)
+    (B, T, K), (_, S, hk, Dh) = x.shape, k_cache.shape
+    (Rt, Kw), (qn, rq), (kn, rk), (vn, rv), (Ro, w), (N, Ru) = (t.shape for t in (qkv_v, q_u, k_u, v_u, o_v, o_u))
+    if k_cache.shape[0] < B or hk != Hk or qn != H * Dh or kn != Hk * Dh or vn != Hk * Dh or Rt != rq + rk + rv or Kw != K or w != H * Dh or Ru != Ro:
+        raise ValueError("factors and caches do not match")
+    rope_len = _rope_tables(cos, sin, Dh, dt)
+    nw, bv, bu = _row_vector(dt, norm_weight, K, "norm_weight"), _row_vector(dt, o_v_bias, Ro, "o_v_bias"), _row_vector(dt, o_u_bias, N, "o_u_bias")
+    x2, xp, ldx, rows, _ = _row_operand(x, "x")
+    out = torch.empty(B, T, N, device=x.device, dtype=dt)
+    keep, rp, ldr = _residual_rows(dt, residual, rows, N)
+    if rows >= 3:
+        ensure_split_workspace(x.device)
+    buf, (xs, p, q, a) = _buffers(dt, x.device, max(rows * K if nw and rows >= 3 else 0, rows * Ro), rows * Rt, rows * w, rows * w)
+    b = _lib.AttnBlock(xp, ldx, nw, xs, qkv_v.data_ptr(), qkv_v.stride(0), p, q_u.data_ptr(), k_u.data_ptr(), v_u.data_ptr(), q_u.stride(0),
+                       k_u.stride(0), v_u.stride(0), cos.data_ptr(), sin.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0),
+                       k_cache.stride(1), k_cache.stride(2), q, a, o_v.data_ptr(), o_v.stride(0), bv, xs, o_u.data_ptr(), o_u.stride(0), bu,
+                       rp, ldr, out.data_ptr(), N, float(eps), B, T, K, rq, rk, rv, H, Hk, Dh, S, int(start), rope_len, Ro, N, code)
+    _lib.check("fsvd_attn_block_prefill", _lib.load().fsvd_attn_block_prefill(b, _stream()))
+    return out
+
+
 def prefill_head_groups(B: int, M: int, n_ctx: int, H: int, Hk: int, Dh: int, itemsize: int = 2) -> int:
     """How many kv heads (with their query heads) the expand-then-attend prompt pass takes at a time.
 

@@ -119,18 +119,14 @@ def _fast_path_ok(p_up_2d, p_gate_2d, GateU, UpU, DownV, DownU, variant, partial
 def _run_fast(p_up_2d, p_gate_2d, GateU, UpU, DownV, DownU, b2):
     from .. import hip_ops
     from ._common import linear_layout_of
-    T, R = p_up_2d.shape
-    # the coefficient rows as one [T, 2R] buffer [PGate | PUp]: adjacent views of such a packed tensor are used in place,
-    # anything else (separate tensors, the [PUp | PGate] order of the pcat_s variant) is packed by one small copy
-    if p_up_2d.data_ptr() == p_gate_2d.data_ptr() + R * 2 and p_up_2d.stride(0) == p_gate_2d.stride(0) >= 2 * R:
-        p = p_gate_2d.as_strided((T, 2 * R), (p_gate_2d.stride(0), 1))
-    else:
-        p = torch.cat([p_gate_2d, p_up_2d], dim=1)
-    gate_u, up_u = linear_layout_of(GateU), linear_layout_of(UpU)          # [D, R]
-    # inside the operator flashsvd_hip::mlp_dual_split: its steps do not go through the dispatcher again
-    h = hip_ops._swiglu_linear_impl(p, gate_u, up_u, R, 1, None, 0)        # h = round(silu(g32) * u32), dual_split_triton.py:207
-    s = hip_ops._linear_impl(h, linear_layout_of(DownV), None, None, 0.0, None, None, 0)       # S: fp32 sum over D, one rounding (:719-720)
-    return hip_ops._linear_impl(s, linear_layout_of(DownU), None if b2 is None else b2.to(s.dtype).contiguous(), None, 0.0, None, None, 0)
+    # inside the operator flashsvd_hip::mlp_dual_split: its launches are issued by one native call, the coefficients taken where
+    # they are (separate tensors, adjacent views of a packed one in either order); rows of different strides, and rows off the
+    # 16-byte grid of the kernels, are copied
+    if p_up_2d.stride(0) != p_gate_2d.stride(0) or p_up_2d.stride(0) % 8 or (p_up_2d.data_ptr() | p_gate_2d.data_ptr()) % 16:
+        p_up_2d, p_gate_2d = (t.clone(memory_format=torch.contiguous_format) for t in (p_up_2d, p_gate_2d))
+    # h = round(silu(g32) * u32), dual_split_triton.py:207; S: fp32 sum over D, one rounding (:719-720)
+    return hip_ops._mlp_from_coefficients(p_gate_2d, p_up_2d, linear_layout_of(GateU), linear_layout_of(UpU), linear_layout_of(DownV),
+                                          linear_layout_of(DownU), None if b2 is None else b2.to(p_up_2d.dtype).contiguous(), 1)
 
 
 def _run_impl(p_up_2d, p_gate_2d, GateU, UpU, DownV, DownU, b2, variant, BD, partials_fp32, s_out):

@@ -402,7 +402,19 @@ class SVD_LlamaAttention(nn.Module):
         kc, vc = cache.key_cache[self.layer_idx], cache.value_cache[self.layer_idx]
         rope = cache.get_rope_tables(seqlen=cache.max_cache_len, head_dim=Dh, device=x.device, dtype=x.dtype)
         from .quant import PackedQuantLinear, apply_linear, is_quantized
-        if is_quantized(*self._factor_modules()):
+        quantized = is_quantized(*self._factor_modules())
+        mfma_ok = Dh == 128 and T >= 16 \
+            and os.getenv("FLASHSVD_AMD_PREFILL", "mfma").strip().lower() != "decode"
+        if mfma_ok and not quantized:
+            # the matrix-core route below, its launches issued by one native call
+            out = hip_ops.lowrank_attn_prefill(
+                x, self._packed_qkv_v, self.q_u_proj.weight, self.k_u_proj.weight, self.v_u_proj.weight, self.o_v_proj.weight,
+                self.o_u_proj.weight, kc, vc, rope[0], rope[1], start=start, num_heads=H, num_kv_heads=Hk, norm_weight=norm_weight, eps=eps,
+                residual=residual, o_v_bias=getattr(self.o_v_proj, "bias", None), o_u_bias=getattr(self.o_u_proj, "bias", None))
+            cache._layer_initialized[self.layer_idx] = True
+            cache._note_seen(self.layer_idx, T, cache_position)
+            return out
+        if quantized:
             # int4 factors: rank projections module by module, head bases expanded to bf16 for this call
             xn = x if norm_weight is None else hip_ops.rmsnorm(x, norm_weight, eps)
             p = torch.cat([apply_linear(m, xn) for m in (self.q_v_proj, self.k_v_proj, self.v_v_proj)], dim=-1)
@@ -412,8 +424,6 @@ class SVD_LlamaAttention(nn.Module):
             p = hip_ops.linear(x, self._packed_qkv_v, norm_weight=norm_weight, eps=eps)   # [B,T,Rtot]
             wq, wk, wv = self.q_u_proj.weight, self.k_u_proj.weight, self.v_u_proj.weight
         rq, rk, rv = self._qkv_rank_tuple()
-        mfma_ok = Dh == 128 and T >= 16 \
-            and os.getenv("FLASHSVD_AMD_PREFILL", "mfma").strip().lower() != "decode"
         a = torch.empty(B, T, H * Dh, device=x.device, dtype=x.dtype)
         if mfma_ok:
             # matrix-core route: q/k/v rebuilt once per token with the rotation fused (k, v land in the
@@ -617,12 +627,9 @@ class SVD_LlamaMLP(nn.Module):
         if is_quantized(*self._factor_modules()):
             return self._run_quantized(x, norm_weight=norm_weight, eps=eps, residual=residual, mode=mode)
         self._ensure_runtime_state()
-        r = self.gate_v_proj.out_features
-        p = hip_ops.linear(x, self._packed_gu_v, norm_weight=norm_weight, eps=eps)      # [.., 2R] = [PGate | PUp]
-        h = hip_ops.swiglu_linear(p, self.gate_u_proj.weight, self.up_u_proj.weight, up_off=r,
-                                  mode=mlp_rounding_mode() if mode is None else mode)
-        s = hip_ops.linear(h, self.down_v_proj.weight)
-        return hip_ops.linear(s, self.down_u_proj.weight, residual=residual)
+        return hip_ops.lowrank_mlp(x, self._packed_gu_v, self.gate_u_proj.weight, self.up_u_proj.weight, self.down_v_proj.weight,
+                                   self.down_u_proj.weight, norm_weight=norm_weight, eps=eps, residual=residual,
+                                   mode=mlp_rounding_mode() if mode is None else mode)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         _require_gpu(x, "SVD_LlamaMLP")

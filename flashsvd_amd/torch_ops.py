@@ -8,6 +8,8 @@ tensors.  ``flashsvd_amd.hip_ops`` and the modules under ``flashsvd_amd.kernels`
   linear / linear.out                 fsvd_linear            rank projections, factor pairs, fused RMSNorm / residual
   swiglu_linear / .out                fsvd_swiglu_linear     gate_u / up_u pair + SwiGLU
   rmsnorm / .out                      fsvd_rmsnorm
+  lowrank_mlp                         fsvd_mlp_block_run     norm + rank projection + SwiGLU pair + down projection
+  lowrank_attn_prefill                fsvd_attn_block_prefill   the attention half of a prompt pass over the dense cache
   greedy_token_                       fsvd_greedy_token      argmax of every row + position increment
   qkv_rope_append / .out              fsvd_qkv_rope_append   head expansion + RoPE + dense-cache append
   attn_decode_densekv / .out          fsvd_attn_decode_densekv(_static)   the flash_attn_with_kvcache role
@@ -93,6 +95,30 @@ _define("rmsnorm(Tensor x, Tensor weight, float eps=1e-6) -> Tensor", _rmsnorm,
         lambda x, weight, eps=1e-6: torch.empty_like(x, memory_format=torch.contiguous_format))
 _define("rmsnorm.out(Tensor x, Tensor weight, float eps=1e-6, *, Tensor(a!) out) -> Tensor(a!)", _rmsnorm_out,
         lambda *a, out, **k: out)
+
+
+# ------------------------------------------------------------------ the two halves of a layer, one native call each
+def _lowrank_mlp(x, gu_v, gate_u, up_u, down_v, down_u, norm_weight=None, eps=1e-6, residual=None, mode=0):
+    from . import hip_ops
+    return hip_ops._lowrank_mlp_impl(x, gu_v, gate_u, up_u, down_v, down_u, norm_weight, eps, residual, mode)
+
+
+_define("lowrank_mlp(Tensor x, Tensor gu_v, Tensor gate_u, Tensor up_u, Tensor down_v, Tensor down_u, Tensor? norm_weight=None, "
+        "float eps=1e-6, Tensor? residual=None, int mode=0) -> Tensor", _lowrank_mlp,
+        lambda x, gu_v, gate_u, up_u, down_v, down_u, *a, **k: x.new_empty((*x.shape[:-1], down_u.shape[0])))
+
+
+def _lowrank_attn_prefill(x, qkv_v, q_u, k_u, v_u, o_v, o_u, k_cache, v_cache, cos, sin, start, num_heads, num_kv_heads, norm_weight=None,
+                          eps=1e-6, residual=None, o_v_bias=None, o_u_bias=None):
+    from . import hip_ops
+    return hip_ops._lowrank_attn_prefill_impl(x, qkv_v, q_u, k_u, v_u, o_v, o_u, k_cache, v_cache, cos, sin, start, num_heads, num_kv_heads,
+                                              norm_weight, eps, residual, o_v_bias, o_u_bias)
+
+
+_define("lowrank_attn_prefill(Tensor x, Tensor qkv_v, Tensor q_u, Tensor k_u, Tensor v_u, Tensor o_v, Tensor o_u, Tensor(a!) k_cache, "
+        "Tensor(b!) v_cache, Tensor cos, Tensor sin, int start, int num_heads, int num_kv_heads, Tensor? norm_weight=None, float eps=1e-6, "
+        "Tensor? residual=None, Tensor? o_v_bias=None, Tensor? o_u_bias=None) -> Tensor", _lowrank_attn_prefill,
+        lambda x, qkv_v, q_u, k_u, v_u, o_v, o_u, *a, **k: x.new_empty((*x.shape[:-1], o_u.shape[0])))
 
 
 # ------------------------------------------------------------------ greedy token of every row
@@ -253,5 +279,5 @@ _define("mlp_dual_split(Tensor PUp, Tensor PGate, Tensor GateU, Tensor UpU, Tens
         PUp.new_empty((PUp.shape[0], DownU.shape[1])))
 
 ops = getattr(torch.ops, NS)
-OP_NAMES = ("linear", "swiglu_linear", "rmsnorm", "greedy_token_", "qkv_rope_append", "attn_decode_densekv", "attn_decode_rankkv", "rankkv_append", "linear_rankkv_append",
+OP_NAMES = ("linear", "swiglu_linear", "rmsnorm", "greedy_token_", "lowrank_mlp", "lowrank_attn_prefill", "qkv_rope_append", "attn_decode_densekv", "attn_decode_rankkv", "rankkv_append", "linear_rankkv_append",
             "lowrank_expand_heads", "rope_attn_prefill", "reconstruct_qkv_token", "xw_linear", "mlp_dual_split")

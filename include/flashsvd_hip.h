@@ -310,6 +310,52 @@ int fsvd_attn_prefill(const void* q, int64_t sq_b, int64_t sq_m, int64_t sq_h,
                       void* out, int64_t so_b, int64_t so_m, int64_t so_h,
                       int B, int M, int H, int Hk, int Dh, int S, int causal, float scale, int dtype, void* stream);
 
+/* ---- two halves of a layer over a block of rows, one call each: the launches of the single entry points, back to back -----------
+ * Every intermediate is the caller's, [rows, width] contiguous of the element type, 16-byte aligned. */
+typedef struct fsvd_mlp_block {
+  const void* x; int64_t ldx;          /* [B, K]; NULL: p and up hold the coefficients already                            */
+  const void* norm_w;                  /* RMSNorm weight of x or NULL                                                     */
+  void* xn;                            /* [B, K] for the normalised rows (may be NULL without norm_w or below 3 rows)     */
+  const void* gu_v; int64_t ldgv;      /* [2R, K]: rank projections of gate and up                                        */
+  void* p; int64_t ldp;                /* [B, >= R] gate coefficients, ...                                                */
+  const void* up;                      /* ... up coefficients with the same row stride; NULL: at column R of p            */
+  const void* gate_u; const void* up_u; int64_t ldu;   /* [D, R]                                                          */
+  void* h;                             /* [B, D]                                                                          */
+  const void* down_v; int64_t ldv;     /* [Rd, D]                                                                         */
+  void* s;                             /* [B, Rd]; may share memory with xn                                               */
+  const void* down_u; int64_t ldd;     /* [N, Rd]                                                                         */
+  const void* bias;                    /* [N] or NULL                                                                     */
+  const void* res; int64_t ldres;      /* [B, N] or NULL                                                                  */
+  void* y; int64_t ldy;                /* [B, N]                                                                          */
+  float eps;
+  int32_t B, K, R, D, Rd, N, mode, dtype;
+} fsvd_mlp_block;
+/* y = (res +) down_u(down_v(silu(gate_u pg) * up_u pu)) (+ bias), [pg | pu] = gu_v norm(x): fsvd_rmsnorm, fsvd_linear,
+ * fsvd_swiglu_linear, fsvd_linear, fsvd_linear. */
+int fsvd_mlp_block_run(const fsvd_mlp_block* b, void* stream);
+
+typedef struct fsvd_attn_block {
+  const void* x; int64_t ldx;          /* [B * M, K]                                                                      */
+  const void* norm_w; void* xn;        /* as above                                                                        */
+  const void* qkv_v; int64_t ldqkv;    /* [Rq + Rk + Rv, K]                                                               */
+  void* p;                             /* [B * M, Rq + Rk + Rv]                                                           */
+  const void* q_u; const void* k_u; const void* v_u; int64_t ldq, ldk, ldvu;   /* [H Dh, Rq], [Hk Dh, Rk], [Hk Dh, Rv]    */
+  const void* cos; const void* sin;    /* [rope_len, Dh / 2]                                                              */
+  void* k_cache; void* v_cache; int64_t sc_b, sc_s, sc_h;       /* [>= B, S, Hk, Dh]; rows start .. start + M - 1 written  */
+  void* q; void* a;                    /* [B * M, H, Dh] each                                                             */
+  const void* o_v; int64_t ldov; const void* o_v_bias;          /* [Ro, H Dh]                                             */
+  void* po;                            /* [B * M, Ro]; may share memory with xn                                           */
+  const void* o_u; int64_t ldou; const void* o_u_bias;          /* [N, Ro]                                                */
+  const void* res; int64_t ldres;
+  void* y; int64_t ldy;                /* [B * M, N]                                                                      */
+  float eps;
+  int32_t B, M, K, Rq, Rk, Rv, H, Hk, Dh, S, start, rope_len, Ro, N, dtype;
+} fsvd_attn_block;
+/* The attention half of a prompt pass over the dense cache, M tokens of B sequences from position `start` on: fsvd_rmsnorm,
+ * fsvd_linear, fsvd_lowrank_expand_heads_multi, fsvd_attn_prefill (causal), fsvd_linear, fsvd_linear. */
+int fsvd_attn_block_prefill(const fsvd_attn_block* b, void* stream);
+
+
 /* ---------------------------------------------------------------------------------------------
  * Persistent decode step (batch 1): ONE launch walks a caller-built list of phases — embedding row,
  * low-rank projections with fused RMSNorm / residual / SwiGLU, q/k/v head expansion with RoPE and
