@@ -92,7 +92,8 @@ class MlpBlock(ctypes.Structure):
                 ("p", c_void_p), ("ldp", c_int64), ("up", c_void_p), ("gate_u", c_void_p), ("up_u", c_void_p), ("ldu", c_int64),
                 ("h", c_void_p), ("down_v", c_void_p), ("ldv", c_int64), ("s", c_void_p), ("down_u", c_void_p), ("ldd", c_int64),
                 ("bias", c_void_p), ("res", c_void_p), ("ldres", c_int64), ("y", c_void_p), ("ldy", c_int64), ("eps", c_float),
-                *((n, ctypes.c_int32) for n in ("B", "K", "R", "D", "Rd", "N", "mode", "dtype"))]
+                *((n, ctypes.c_int32) for n in ("B", "K", "R", "D", "Rd", "N", "mode", "dtype")),
+                ("scratch", c_void_p), ("scratch_bytes", c_size_t)]
 
 
 class AttnBlock(ctypes.Structure):
@@ -103,7 +104,8 @@ class AttnBlock(ctypes.Structure):
                 ("sc_h", c_int64), ("q", c_void_p), ("a", c_void_p), ("o_v", c_void_p), ("ldov", c_int64), ("o_v_bias", c_void_p),
                 ("po", c_void_p), ("o_u", c_void_p), ("ldou", c_int64), ("o_u_bias", c_void_p), ("res", c_void_p), ("ldres", c_int64),
                 ("y", c_void_p), ("ldy", c_int64), ("eps", c_float),
-                *((n, ctypes.c_int32) for n in ("B", "M", "K", "Rq", "Rk", "Rv", "H", "Hk", "Dh", "S", "start", "rope_len", "Ro", "N", "dtype"))]
+                *((n, ctypes.c_int32) for n in ("B", "M", "K", "Rq", "Rk", "Rv", "H", "Hk", "Dh", "S", "start", "rope_len", "Ro", "N", "dtype")),
+                ("scratch", c_void_p), ("scratch_bytes", c_size_t)]
 
 
 PH_EMBED, PH_GEMV, _PH_RESERVED, PH_ATTN, PH_MERGE, PH_ARGMAX = range(6)
@@ -119,6 +121,9 @@ SIGNATURES = {
     "fsvd_last_form": (c_char_p, []),
     "fsvd_linear": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_float, c_void_p, c_int64,
                             c_void_p, c_int64, c_int, c_int, c_int, c_int, c_int, c_void_p]),
+    "fsvd_linear_scratch_bytes": (c_size_t, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int, c_int, c_int]),
+    "fsvd_linear_scratch": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_float, c_void_p, c_int64,
+                                    c_void_p, c_int64, c_int, c_int, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p]),
     "fsvd_linear_rankkv_append": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_float, c_void_p, c_int64, c_int, c_int, c_int, c_int,
                                           c_int, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int, c_int, c_void_p]),
     "fsvd_swiglu_linear": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_void_p, c_int64,
@@ -172,6 +177,8 @@ SIGNATURES = {
     "fsvd_decode_step_set_state": (c_int, [c_void_p, c_int64, ctypes.c_int32, c_void_p]),
     "fsvd_greedy_token": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_void_p]),
     "fsvd_set_token_rows": (c_int, [c_void_p, c_void_p, c_void_p, ctypes.c_int32, c_int, c_void_p]),
+    "fsvd_mlp_block_scratch_bytes": (c_size_t, [ctypes.POINTER(MlpBlock)]),
+    "fsvd_attn_block_scratch_bytes": (c_size_t, [ctypes.POINTER(AttnBlock)]),
     "fsvd_mlp_block_run": (c_int, [ctypes.POINTER(MlpBlock), c_void_p]),
     "fsvd_attn_block_prefill": (c_int, [ctypes.POINTER(AttnBlock), c_void_p]),
     "fsvd_set_workspace": (c_int, [c_void_p, c_size_t, c_void_p]),

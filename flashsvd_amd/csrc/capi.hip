@@ -70,16 +70,41 @@ int fsvd_set_workspace(void* ws, size_t bytes, void* stream) {
   return kOk;
 }
 
-int fsvd_linear(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* bias, const void* norm_w, float eps,
-                const void* res, int64_t ldres, void* y, int64_t ldy, int B, int N, int K, int cfg, int dtype, void* stream) {
-  FSVD_REQUIRE_PTR(x, "fsvd_linear"); FSVD_REQUIRE_PTR(W, "fsvd_linear"); FSVD_REQUIRE_PTR(y, "fsvd_linear");
-  if (ldx < K || ldw < K || ldy < N || (res && ldres < N)) {
-    set_last_error("fsvd_linear: leading dimension smaller than the row (ldx=%lld ldw=%lld ldy=%lld ldres=%lld K=%d N=%d)",
-                   (long long)ldx, (long long)ldw, (long long)ldy, (long long)ldres, K, N);
+static int linear_args(LinearArgs& a, const char* fn) {
+  if (a.ldx < a.K || a.ldw < a.K || a.ldy < a.N || (a.res && a.ldres < a.N)) {
+    set_last_error("%s: leading dimension smaller than the row (ldx=%lld ldw=%lld ldy=%lld ldres=%lld K=%d N=%d)", fn,
+                   (long long)a.ldx, (long long)a.ldw, (long long)a.ldy, (long long)a.ldres, a.K, a.N);
     return kErrBadShape;
   }
+  return kOk;
+}
+
+int fsvd_linear(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* bias, const void* norm_w, float eps,
+                const void* res, int64_t ldres, void* y, int64_t ldy, int B, int N, int K, int cfg, int dtype, void* stream) {
+  return fsvd_linear_scratch(x, ldx, W, ldw, bias, norm_w, eps, res, ldres, y, ldy, B, N, K, cfg, dtype, nullptr, 0, stream);
+}
+
+constexpr size_t kShareScratchBytes = (size_t)64 << 20;
+size_t fsvd_linear_scratch_bytes(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* res, int64_t ldres, const void* y, int64_t ldy,
+                                 int B, int N, int K) {
+  if (B < 128 || N <= 0 || K <= 0) return 0;
+  LinearArgs a{cu16(x), ldx, cu16(W), ldw, nullptr, nullptr, 0.f, cu16(res), ldres, const_cast<uint16_t*>(cu16(y)), ldy, B, N, K, 0};
+  return linear_scratch_floats(a, kShareScratchBytes / sizeof(float)) * sizeof(float);
+}
+
+int fsvd_linear_scratch(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* bias, const void* norm_w, float eps,
+                        const void* res, int64_t ldres, void* y, int64_t ldy, int B, int N, int K, int cfg, int dtype,
+                        void* scratch, size_t scratch_bytes, void* stream) {
+  const char* fn = "fsvd_linear";
+  FSVD_REQUIRE_PTR(x, fn); FSVD_REQUIRE_PTR(W, fn); FSVD_REQUIRE_PTR(y, fn);
   LinearArgs a{cu16(x), ldx, cu16(W), ldw, cu16(bias), cu16(norm_w), eps, cu16(res), ldres, u16(y), ldy, B, N, K, dtype};
-  return launch_linear(a, cfg, static_cast<hipStream_t>(stream));
+  if (scratch != nullptr) {
+    if ((reinterpret_cast<uintptr_t>(scratch) & 15) != 0) { set_last_error("%s: scratch must be 16-byte aligned", fn); return kErrBadAlign; }
+    a.scratch = static_cast<float*>(scratch);
+    a.scratch_floats = std::min(scratch_bytes, kShareScratchBytes) / sizeof(float);
+  }
+  const int rc = linear_args(a, fn);
+  return rc != kOk ? rc : launch_linear(a, cfg, static_cast<hipStream_t>(stream));
 }
 
 int fsvd_linear_rankkv_append(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* norm_w, float eps, void* y, int64_t ldy,
@@ -597,19 +622,19 @@ int fsvd_attn_prefill(const void* q, int64_t sq_b, int64_t sq_m, int64_t sq_h, c
 
 // one projection of a block: contiguous rows in and out unless said otherwise
 static int block_linear(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* bias, const void* norm_w, float eps, const void* res,
-                        int64_t ldres, void* y, int64_t ldy, int B, int N, int K, int dtype, void* stream) {
-  return fsvd_linear(x, ldx, W, ldw, bias, norm_w, eps, res, ldres, y, ldy, B, N, K, 0, dtype, stream);
+                        int64_t ldres, void* y, int64_t ldy, int B, int N, int K, int dtype, void* scratch, size_t scratch_bytes, void* stream) {
+  return fsvd_linear_scratch(x, ldx, W, ldw, bias, norm_w, eps, res, ldres, y, ldy, B, N, K, 0, dtype, scratch, scratch_bytes, stream);
 }
 // the rank projection in front of a block: three rows and more are normalised once up front, fewer in the projection's own launch
 static int block_input(const void* x, int64_t ldx, const void* norm_w, float eps, void* xn, const void* W, int64_t ldw, void* p, int64_t ldp, int B,
-                       int N, int K, int dtype, const char* fn, void* stream) {
+                       int N, int K, int dtype, void* scratch, size_t scratch_bytes, const char* fn, void* stream) {
   if (norm_w != nullptr && B >= 3) {
     FSVD_REQUIRE_PTR(xn, fn);
     const int rc = fsvd_rmsnorm(x, ldx, norm_w, eps, xn, K, B, K, dtype, stream);
     if (rc != kOk) return rc;
     x = xn; ldx = K; norm_w = nullptr;
   }
-  return block_linear(x, ldx, W, ldw, nullptr, norm_w, eps, nullptr, 0, p, ldp, B, N, K, dtype, stream);
+  return block_linear(x, ldx, W, ldw, nullptr, norm_w, eps, nullptr, 0, p, ldp, B, N, K, dtype, scratch, scratch_bytes, stream);
 }
 
 int fsvd_mlp_block_run(const fsvd_mlp_block* d, void* stream) {
@@ -625,7 +650,7 @@ int fsvd_mlp_block_run(const fsvd_mlp_block* d, void* stream) {
   int rc;
   if (b.x != nullptr) {
     FSVD_REQUIRE_PTR(b.gu_v, fn);
-    rc = block_input(b.x, b.ldx, b.norm_w, b.eps, b.xn, b.gu_v, b.ldgv, b.p, b.ldp, b.B, 2 * b.R, b.K, b.dtype, fn, stream);
+    rc = block_input(b.x, b.ldx, b.norm_w, b.eps, b.xn, b.gu_v, b.ldgv, b.p, b.ldp, b.B, 2 * b.R, b.K, b.dtype, b.scratch, b.scratch_bytes, fn, stream);
     if (rc != kOk) return rc;
   }
   // the two sets of coefficients may be tensors of their own: a signed distance in elements
@@ -634,9 +659,31 @@ int fsvd_mlp_block_run(const fsvd_mlp_block* d, void* stream) {
   SwigluArgs a{cu16(b.p), b.ldp, bytes / 2, cu16(b.gate_u), cu16(b.up_u), b.ldu, u16(b.h), b.D, b.B, b.D, b.R, b.mode, b.dtype};
   rc = launch_swiglu(a, 0, static_cast<hipStream_t>(stream));
   if (rc != kOk) return rc;
-  rc = block_linear(b.h, b.D, b.down_v, b.ldv, nullptr, nullptr, 0.f, nullptr, 0, b.s, b.Rd, b.B, b.Rd, b.D, b.dtype, stream);
+  rc = block_linear(b.h, b.D, b.down_v, b.ldv, nullptr, nullptr, 0.f, nullptr, 0, b.s, b.Rd, b.B, b.Rd, b.D, b.dtype, b.scratch, b.scratch_bytes, stream);
   if (rc != kOk) return rc;
-  return block_linear(b.s, b.Rd, b.down_u, b.ldd, b.bias, nullptr, 0.f, b.res, b.ldres, b.y, b.ldy, b.B, b.N, b.Rd, b.dtype, stream);
+  return block_linear(b.s, b.Rd, b.down_u, b.ldd, b.bias, nullptr, 0.f, b.res, b.ldres, b.y, b.ldy, b.B, b.N, b.Rd, b.dtype, b.scratch, b.scratch_bytes, stream);
+}
+
+// (the normalised rows stand in for x: what counts is where they lie and how far apart)
+size_t fsvd_mlp_block_scratch_bytes(const fsvd_mlp_block* d) {
+  if (d == nullptr) return 0;
+  const fsvd_mlp_block& b = *d;
+  const bool norm = b.norm_w != nullptr && b.B >= 3;
+  size_t n = b.x ? fsvd_linear_scratch_bytes(norm ? b.xn : b.x, norm ? b.K : b.ldx, b.gu_v, b.ldgv, nullptr, 0, b.p, b.ldp, b.B, 2 * b.R, b.K) : 0;
+  n = std::max(n, fsvd_linear_scratch_bytes(b.h, b.D, b.down_v, b.ldv, nullptr, 0, b.s, b.Rd, b.B, b.Rd, b.D));
+  return std::max(n, fsvd_linear_scratch_bytes(b.s, b.Rd, b.down_u, b.ldd, b.res, b.ldres, b.y, b.ldy, b.B, b.N, b.Rd));
+}
+
+size_t fsvd_attn_block_scratch_bytes(const fsvd_attn_block* d) {
+  if (d == nullptr) return 0;
+  const fsvd_attn_block& b = *d;
+  const int64_t rows = (int64_t)b.B * b.M;
+  if (rows <= 0 || rows > 0x7fffffff) return 0;
+  const bool norm = b.norm_w != nullptr && rows >= 3;
+  const int Rt = b.Rq + b.Rk + b.Rv, w = b.H * b.Dh;
+  size_t n = fsvd_linear_scratch_bytes(norm ? b.xn : b.x, norm ? b.K : b.ldx, b.qkv_v, b.ldqkv, nullptr, 0, b.p, Rt, (int)rows, Rt, b.K);
+  n = std::max(n, fsvd_linear_scratch_bytes(b.a, w, b.o_v, b.ldov, nullptr, 0, b.po, b.Ro, (int)rows, b.Ro, w));
+  return std::max(n, fsvd_linear_scratch_bytes(b.po, b.Ro, b.o_u, b.ldou, b.res, b.ldres, b.y, b.ldy, (int)rows, b.N, b.Ro));
 }
 
 int fsvd_attn_block_prefill(const fsvd_attn_block* d, void* stream) {
@@ -656,7 +703,7 @@ int fsvd_attn_block_prefill(const fsvd_attn_block* d, void* stream) {
   }
   const int rows = (int)rows64, Rt = b.Rq + b.Rk + b.Rv, w = b.H * b.Dh;
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  int rc = block_input(b.x, b.ldx, b.norm_w, b.eps, b.xn, b.qkv_v, b.ldqkv, b.p, Rt, rows, Rt, b.K, b.dtype, fn, stream);
+  int rc = block_input(b.x, b.ldx, b.norm_w, b.eps, b.xn, b.qkv_v, b.ldqkv, b.p, Rt, rows, Rt, b.K, b.dtype, b.scratch, b.scratch_bytes, fn, stream);
   if (rc != kOk) return rc;
   const auto expansion = [&](int at, const void* u, int64_t ldu, int R, int heads, bool rotate, void* y, int64_t sy_b, int64_t sy_m, int64_t sy_h, int by_pos, int dst) {
     ExpandArgs e{cu16(b.p) + at, (int64_t)b.M * Rt, Rt, 0, cu16(u), ldu, nullptr, rotate ? cu16(b.cos) : nullptr, rotate ? cu16(b.sin) : nullptr, b.rope_len,
@@ -681,9 +728,9 @@ int fsvd_attn_block_prefill(const fsvd_attn_block* d, void* stream) {
   t.pos0 = b.start;
   rc = launch_prefill_attn(t, st);
   if (rc != kOk) return rc;
-  rc = block_linear(b.a, w, b.o_v, b.ldov, b.o_v_bias, nullptr, 0.f, nullptr, 0, b.po, b.Ro, rows, b.Ro, w, b.dtype, stream);
+  rc = block_linear(b.a, w, b.o_v, b.ldov, b.o_v_bias, nullptr, 0.f, nullptr, 0, b.po, b.Ro, rows, b.Ro, w, b.dtype, b.scratch, b.scratch_bytes, stream);
   if (rc != kOk) return rc;
-  return block_linear(b.po, b.Ro, b.o_u, b.ldou, b.o_u_bias, nullptr, 0.f, b.res, b.ldres, b.y, b.ldy, rows, b.N, b.Ro, b.dtype, stream);
+  return block_linear(b.po, b.Ro, b.o_u, b.ldou, b.o_u_bias, nullptr, 0.f, b.res, b.ldres, b.y, b.ldy, rows, b.N, b.Ro, b.dtype, b.scratch, b.scratch_bytes, stream);
 }
 
 int fsvd_decode_step_workgroups(void) { return decode_step_workgroups(); }

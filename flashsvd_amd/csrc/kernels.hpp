@@ -22,6 +22,7 @@ struct LinearArgs {
   int64_t app_sb[2] = {0, 0}, app_ss[2] = {0, 0};
   int app_n0[2] = {0, 0}, app_n[2] = {0, 0};
   int app_S = 0;
+  float* scratch = nullptr; size_t scratch_floats = 0;   // this call's own, for the K shares of long prompt rows (fsvd_linear_scratch)
 };
 
 struct SwigluArgs {
@@ -175,6 +176,7 @@ struct MfmaArgs {
   // fp32 partial tiles and one arrival counter per tile; the last workgroup to arrive adds the partials in order
   int ksplit; float* ws_part; int32_t* ws_count;
   int dt = 0;
+  float* scratch = nullptr; size_t scratch_floats = 0;   // this call's own (K shares of mfma_mid.hip)
 };
 // epilogue of a head expansion (mfma_gemm.hip, mfma_mid.hip)
 struct ExpandEpi {
@@ -210,6 +212,7 @@ struct SplitWorkspace { float* part; size_t part_floats; int32_t* count; int nco
 SplitWorkspace split_workspace();                                            // capi.hip
 bool gemm_tiles_apply(const MfmaArgs& a);                                   // mfma_gemm.hip: 128 rows and more
 int launch_gemm_tiles(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
+int gemm_tiles_shares(const MfmaArgs& a, int* unit);
 bool gemm_rows_apply(const MfmaArgs& a);                                    // mfma_gemm.hip: 5..127 rows, K split
 int launch_gemm_rows(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
 int compute_units();                                                         // of the current device, 0 when it cannot be asked
@@ -219,6 +222,8 @@ bool expand_big_apply(const ExpandArgs* d, int n);
 int launch_expand_big(const ExpandArgs* d, int n, hipStream_t st);
 bool gemm_mid_apply(const MfmaArgs& a, bool dual);                          // mfma_mid.hip: about one tile per compute unit
 int launch_gemm_mid(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
+size_t gemm_share_floats(MfmaArgs a, size_t cap);
+size_t linear_scratch_floats(const LinearArgs& a, size_t cap);              // mfma_gemv.hip
 bool expand_mid_apply(const ExpandArgs* d, int n);
 int launch_expand_mid(const ExpandArgs* d, int n, hipStream_t st);
 bool gemm_ragged_apply(const MfmaArgs& a);                                  // mfma_gemm.hip: any K, rows that start anywhere

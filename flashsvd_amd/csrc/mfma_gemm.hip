@@ -546,12 +546,23 @@ static int pick_ksplit(int64_t tiles, int ksteps, size_t floats_per_share, const
 // units idle (up to 128 tiles: two workgroups per tile-starved pair of compute units) or walks a very long K with at
 // most two workgroups per compute unit (down_v of the 7B MLP, K = 11008).  Measured at 128..1024 rows with weights from
 // HBM: o_v 18 -> 12..15 us, down_v 51 -> 25 (128 rows), 32 (256), 46 (512), 92 -> 76 (1024); everything else is as fast
-// or faster unsplit.
+// or faster unsplit.  (Calls with scratch of their own take the shares of mfma_mid.hip for such a K: 20, 24, 36, 47.)
 static int pick_ksplit_prompt(int64_t tiles, int ksteps, int K, size_t floats_per_share, const SplitWorkspace& ws) {
   int z = 1;
   if (tiles <= 128) z = (int)((256 + tiles - 1) / tiles);
   if (K >= 8192 && tiles < 512) z = std::max(z, (int)((768 + tiles - 1) / tiles));
   return z > 1 ? fit_ksplit(z, tiles, ksteps, floats_per_share, ws, 8) : 1;
+}
+
+// how a K of 8192 and more would be cut over the 64 x 64 tiles with scratch at hand: shares, and the K steps of 64 in their unit (1 share:
+// another tile takes the shape)
+int gemm_tiles_shares(const MfmaArgs& a, int* unit) {
+  const auto count = [&](int bm, int bn) { return (int64_t)((a.N + bn - 1) / bn) * ((a.B + bm - 1) / bm); };
+  const int64_t big = count(128, 128), half = count(128, 64), small = count(64, 64);
+  if (big >= 144 || (half >= 160 && half <= 256 && a.K % 128 == 0)) return 1;
+  *unit = small < 320 && a.K % 128 == 0 ? 2 : 1;
+  const SplitWorkspace plenty{reinterpret_cast<float*>(16), ~(size_t)0, nullptr, 1 << 30};      // only counted with
+  return pick_ksplit_prompt(small, a.K / (64 * *unit), a.K, 0, plenty);
 }
 
 template <int DT, bool DUAL, int WTM, int WT, int BK, int NW = 4, int PFSEL = 99, bool RAG = false>

@@ -859,9 +859,19 @@ int launch_qkv_mfma(const QkvArgs& a, hipStream_t st) {
 
 // true when the matrix-core path applies (the caller then skips the vector kernel)
 bool mfma_linear_applies(const LinearArgs& a) { return a.B >= 3 && a.norm_w == nullptr; }
-int launch_linear_mfma(const LinearArgs& a, hipStream_t st) {
+static MfmaArgs mfma_args(const LinearArgs& a) {
   MfmaArgs m{a.x, a.ldx, 0, a.W, nullptr, a.ldw, a.bias, a.res, a.ldres, a.y, a.ldy, a.B, a.N, a.K, 0};
   m.dt = a.dt;
+  m.scratch = a.scratch;
+  m.scratch_floats = a.scratch_floats;
+  return m;
+}
+size_t linear_scratch_floats(const LinearArgs& a, size_t cap) {
+  const MfmaArgs m = mfma_args(a);
+  return mfma_linear_applies(a) && !gemm_ragged_apply(m) ? gemm_share_floats(m, cap) : 0;
+}
+int launch_linear_mfma(const LinearArgs& a, hipStream_t st) {
+  const MfmaArgs m = mfma_args(a);
   return a.dt == 1 ? launch_mfma<1, false>(m, st, "fsvd_linear") : launch_mfma<0, false>(m, st, "fsvd_linear");
 }
 bool mfma_swiglu_applies(const SwigluArgs& a) { return a.B >= 3; }

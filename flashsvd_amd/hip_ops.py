@@ -160,8 +160,14 @@ def _linear_impl(x, weight, bias, norm_weight, eps, residual, out, cfg):
         # up front (same rounding points as the fused prologue)
         x2, xp, ldx, _, _ = _row_operand(_rmsnorm_impl(x2, norm_weight, eps, None), "x")
         norm_weight = None
-    rc = lib.fsvd_linear(xp, ldx, weight.data_ptr(), weight.stride(0), _ptr(bias), _ptr(norm_weight),
-                         float(eps), rp, ldr, op, ldo, B, N, K, int(cfg), code, _stream())
+    wp, ldw = weight.data_ptr(), weight.stride(0)
+    scratch, nbytes = None, 0
+    if B >= 128 and K >= 4096 and cfg == 0:
+        nbytes = lib.fsvd_linear_scratch_bytes(xp, ldx, wp, ldw, rp, ldr, op, ldo, B, N, K)
+        if nbytes:
+            scratch = torch.empty(nbytes, dtype=torch.uint8, device=x.device)      # of this call and stream
+    rc = lib.fsvd_linear_scratch(xp, ldx, wp, ldw, _ptr(bias), _ptr(norm_weight), float(eps), rp, ldr, op, ldo, B, N, K, int(cfg), code,
+                                 _ptr(scratch), nbytes, _stream())
     _lib.check("fsvd_linear", rc)
     return out
 
@@ -632,6 +638,16 @@ def _buffers(dt, device, *counts):
     return buf, [base + 2 * e for e in ends]
 
 
+def _block_scratch(b, device, nbytes_of):
+    """Scratch of this call and stream for the K shares of a block's projections; the tensor to keep alive."""
+    n = nbytes_of(b)
+    if not n:
+        return None
+    t = torch.empty(n, dtype=torch.uint8, device=device)
+    b.scratch, b.scratch_bytes = t.data_ptr(), n
+    return t
+
+
 def lowrank_mlp(x: torch.Tensor, gu_v: torch.Tensor, gate_u: torch.Tensor, up_u: torch.Tensor, down_v: torch.Tensor, down_u: torch.Tensor, *,
                 norm_weight: Optional[torch.Tensor] = None, eps: float = 1e-6, residual: Optional[torch.Tensor] = None, mode: int = 0) -> torch.Tensor:
     """(residual +) down_u(down_v(silu(gate_u g) * up_u u)) with [g | u] = gu_v norm(x): the launches of :func:`linear`,
@@ -657,6 +673,7 @@ def _lowrank_mlp_impl(x, gu_v, gate_u, up_u, down_v, down_u, norm_weight, eps, r
     b = _lib.MlpBlock(xp, ldx, nw, xs, gu_v.data_ptr(), gu_v.stride(0), p, two_r, None, gate_u.data_ptr(), up_u.data_ptr(), gate_u.stride(0),
                       h, down_v.data_ptr(), down_v.stride(0), xs, down_u.data_ptr(), down_u.stride(0), None, rp, ldr, out.data_ptr(), N,
                       float(eps), B, K, R, D, Rd, N, int(mode), code)
+    scratch = _block_scratch(b, x.device, _lib.load().fsvd_mlp_block_scratch_bytes) if B >= 128 and max(K, D, Rd) >= 4096 else None
     _lib.check("fsvd_mlp_block_run", _lib.load().fsvd_mlp_block_run(b, _stream()))
     return out
 
@@ -678,6 +695,7 @@ def _mlp_from_coefficients(pg, pu, gate_u, up_u, down_v, down_u, bias, mode):
     b = _lib.MlpBlock(None, 0, None, None, None, 0, pg.data_ptr(), pg.stride(0), pu.data_ptr(), gate_u.data_ptr(), up_u.data_ptr(), gate_u.stride(0),
                       h, down_v.data_ptr(), down_v.stride(0), s, down_u.data_ptr(), down_u.stride(0), bp, None, 0, out.data_ptr(), N,
                       0.0, B, 0, R, D, Rd, N, int(mode), code)
+    scratch = _block_scratch(b, pg.device, _lib.load().fsvd_mlp_block_scratch_bytes) if B >= 128 and max(D, Rd) >= 4096 else None
     _lib.check("fsvd_mlp_block_run", _lib.load().fsvd_mlp_block_run(b, _stream()))
     return out
 
@@ -719,6 +737,7 @@ def _lowrank_attn_prefill_impl(x, qkv_v, q_u, k_u, v_u, o_v, o_u, k_cache, v_cac
                        k_u.stride(0), v_u.stride(0), cos.data_ptr(), sin.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0),
                        k_cache.stride(1), k_cache.stride(2), q, a, o_v.data_ptr(), o_v.stride(0), bv, xs, o_u.data_ptr(), o_u.stride(0), bu,
                        rp, ldr, out.data_ptr(), N, float(eps), B, T, K, rq, rk, rv, H, Hk, Dh, S, int(start), rope_len, Ro, N, code)
+    scratch = _block_scratch(b, x.device, _lib.load().fsvd_attn_block_scratch_bytes) if rows >= 128 and max(K, w, Ro) >= 4096 else None
     _lib.check("fsvd_attn_block_prefill", _lib.load().fsvd_attn_block_prefill(b, _stream()))
     return out
 

@@ -76,6 +76,16 @@ int fsvd_set_workspace(void* ws, size_t bytes, void* stream);
 int fsvd_linear(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* bias,
                 const void* norm_w, float eps, const void* res, int64_t ldres,
                 void* y, int64_t ldy, int B, int N, int K, int cfg, int dtype, void* stream);
+/* fsvd_linear with scratch of the call's own: 128 rows and more of a long K (4096 and more) then run in shares of K over
+ * workgroups whose fp32 sums lie there, where that is faster.  fsvd_linear_scratch_bytes tells how much such a call can use
+ * (0: none, and `scratch` may be NULL; reads no memory, at most 64 MiB); with less, or with NULL, the call runs with fewer
+ * shares or as fsvd_linear.  The buffer (device memory, 16-byte aligned, contents don't matter) is the call's until the
+ * stream has run it, so calls with buffers of their own are independent on any streams. */
+size_t fsvd_linear_scratch_bytes(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* res, int64_t ldres, const void* y,
+                                 int64_t ldy, int B, int N, int K);
+int fsvd_linear_scratch(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* bias, const void* norm_w, float eps,
+                        const void* res, int64_t ldres, void* y, int64_t ldy, int B, int N, int K, int cfg, int dtype,
+                        void* scratch, size_t scratch_bytes, void* stream);
 
 /* h[b,n] = silu(gate_u[n,:] . p[b,0:R]) * (up_u[n,:] . p[b,up_off:up_off+R]),  gate_u/up_u [D,R].
  * mode 0 rounds like a chain of bf16 nn.Linear modules, mode 1 like the fused reference kernel
@@ -329,10 +339,12 @@ typedef struct fsvd_mlp_block {
   void* y; int64_t ldy;                /* [B, N]                                                                          */
   float eps;
   int32_t B, K, R, D, Rd, N, mode, dtype;
+  void* scratch; size_t scratch_bytes; /* for the projections, as in fsvd_linear_scratch, or NULL                         */
 } fsvd_mlp_block;
 /* y = (res +) down_u(down_v(silu(gate_u pg) * up_u pu)) (+ bias), [pg | pu] = gu_v norm(x): fsvd_rmsnorm, fsvd_linear,
  * fsvd_swiglu_linear, fsvd_linear, fsvd_linear. */
 int fsvd_mlp_block_run(const fsvd_mlp_block* b, void* stream);
+size_t fsvd_mlp_block_scratch_bytes(const fsvd_mlp_block* b);          /* what `scratch` can be used for, reads no device memory */
 
 typedef struct fsvd_attn_block {
   const void* x; int64_t ldx;          /* [B * M, K]                                                                      */
@@ -350,10 +362,12 @@ typedef struct fsvd_attn_block {
   void* y; int64_t ldy;                /* [B * M, N]                                                                      */
   float eps;
   int32_t B, M, K, Rq, Rk, Rv, H, Hk, Dh, S, start, rope_len, Ro, N, dtype;
+  void* scratch; size_t scratch_bytes;
 } fsvd_attn_block;
 /* The attention half of a prompt pass over the dense cache, M tokens of B sequences from position `start` on: fsvd_rmsnorm,
  * fsvd_linear, fsvd_lowrank_expand_heads_multi, fsvd_attn_prefill (causal), fsvd_linear, fsvd_linear. */
 int fsvd_attn_block_prefill(const fsvd_attn_block* b, void* stream);
+size_t fsvd_attn_block_scratch_bytes(const fsvd_attn_block* b);
 
 
 /* ---------------------------------------------------------------------------------------------

@@ -1,0 +1,90 @@
+"""Projections of a long K in shares over workgroups (csrc/mfma_mid.hip) at the edges of their tilings: partial row and column
+tiles, shares of unequal length, strided and odd rows, bias and residual, against the same product in fp32; and the two-stage
+ring of the head expansions at its shortest rank."""
+import pytest
+import torch
+
+from tests import test_gpu_mid_tiles as mid
+from tests.test_gpu_big_tiles import _check, _rand
+from tests.util import form_taken
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,N,K,form", [
+    (128, 1536, 11008, "shares 64 x 128"), (191, 1027, 8256, "shares 64 x 128"), (130, 3001, 4096, "shares 64 x 128"),
+    (193, 1030, 8192, "shares 128 x 128"), (333, 3070, 4160, "shares 128 x 128"),
+    (512, 1500, 5504, "shares 256 x 128"), (769, 1533, 8320, "shares 128 x 128"), (1000, 1533, 8320, "shares 256 x 128"), (2047, 2390, 8192, "shares 256 x 128"),
+    (512, 1536, 11008, "shares 128 x 128"), (420, 3072, 4096, "ring 128 x 64"), (512, 4096, 4096, "ring 128 x 64"), (127, 3072, 4096, "tiles 32 x 64"),
+])
+def test_linear(B, N, K, form, dtype):
+    from flashsvd_amd import hip_ops
+    x, w = _rand(B, K + 8, seed=1, dtype=dtype)[:, 8:], _rand(N, K + 16, std=K ** -0.5, seed=2, dtype=dtype)[:, :K]
+    bias, res = _rand(N, seed=3, dtype=dtype), _rand(B, N + 1, seed=4, dtype=dtype)[:, 1:]
+    ref = x.float() @ w.float().t()
+    y = hip_ops.linear(x, w)
+    assert form_taken() == form
+    _check(y, ref.to(dtype), "plain")
+    ref = ((ref + bias.float()).to(dtype).float() + res.float()).to(dtype)
+    out = torch.full((B + 1, N + 3), 7.0, device="cuda", dtype=dtype)                 # rows and columns around the output stay as they are
+    hip_ops.linear(x, w, bias, residual=res, out=out[:B, 1:N + 1])
+    _check(out[:B, 1:N + 1], ref, "bias, residual, odd output")
+    assert bool((out[B] == 7).all()) and bool((out[:, 0] == 7).all()) and bool((out[:, N + 1:] == 7).all())
+    assert torch.equal(y, hip_ops.linear(x, w)), "repeat differs"
+
+
+def test_calls_on_two_streams_are_independent():
+    """Each call's sums lie in scratch of its own, the registered buffer stays as it is."""
+    from flashsvd_amd import hip_ops
+    xs = [_rand(333, 8192, seed=s) for s in (1, 2)]
+    ws = [_rand(1536, 8192, std=8192 ** -0.5, seed=s) for s in (3, 4)]
+    assert hip_ops.ensure_split_workspace(xs[0].device)
+    partials = hip_ops._SPLIT_WS[0][64 << 10:]
+    partials.fill_(0x5a)
+    want = [hip_ops.linear(x, w) for x, w in zip(xs, ws)]
+    assert int((partials != 0x5a).sum()) == 0
+    streams = [torch.cuda.Stream() for _ in xs]
+    torch.cuda.synchronize()
+    got = [[], []]
+    for _ in range(20):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                got[i].append(hip_ops.linear(xs[i], ws[i]))
+    torch.cuda.synchronize()
+    for i in (0, 1):
+        assert all(torch.equal(g, want[i]) for g in got[i])
+
+
+def test_a_buffer_that_is_too_small_means_fewer_shares():
+    from flashsvd_amd import _lib, hip_ops
+    lib = _lib.load()
+    x, w = _rand(333, 8192, seed=1), _rand(1536, 8192, std=8192 ** -0.5, seed=2)
+    y = torch.empty(333, 1536, dtype=torch.bfloat16, device="cuda")
+    args = (x.data_ptr(), 8192, w.data_ptr(), 8192, None, None, 0.0, None, 0, y.data_ptr(), 1536, 333, 1536, 8192, 0, 0)
+    full = lib.fsvd_linear_scratch_bytes(x.data_ptr(), 8192, w.data_ptr(), 8192, None, 0, y.data_ptr(), 1536, 333, 1536, 8192)
+    ref = (x.float() @ w.float().t()).bfloat16()
+    for nbytes in (full, full - 1, full // 3, 1 << 16, 0):
+        scratch = torch.full((nbytes + 4096,), 0x5a, dtype=torch.uint8, device="cuda")
+        rc = lib.fsvd_linear_scratch(*args, scratch.data_ptr(), nbytes, hip_ops._stream())
+        assert rc == 0
+        _check(y, ref, f"{nbytes} bytes")
+        assert bool((scratch[nbytes:] == 0x5a).all())
+
+
+@pytest.mark.parametrize("B,T,H,Hk,R", [(1, 520, 32, 32, 64), (3, 400, 20, 10, 128)])
+def test_head_expansion_in_two_stages(B, T, H, Hk, R):
+    mid.test_head_expansion(B, T, H, Hk, R)
+    assert form_taken().startswith("ring 64 x 128")
+
+
+def test_blocks_hand_their_projections_scratch():
+    from flashsvd_amd import hip_ops as ops
+    B, K, R, D = 333, 4096, 1500, 8192                                     # both long projections in shares
+    x, gu_v, dv, du = _rand(B, K, seed=1), _rand(2 * R, K, std=K ** -0.5, seed=2), _rand(R, D, std=D ** -0.5, seed=5), _rand(K, R, std=R ** -0.5, seed=6)
+    gu, uu = _rand(D, R, std=R ** -0.5, seed=3), _rand(D, R, std=R ** -0.5, seed=4)
+    p = ops.linear(x, gu_v)
+    assert form_taken().startswith("shares")
+    s = ops.linear(ops.swiglu_linear(p, gu, uu, up_off=R), dv)
+    assert form_taken().startswith("shares")
+    assert torch.equal(ops.lowrank_mlp(x, gu_v, gu, uu, dv, du, residual=x), ops.linear(s, du, residual=x))
