@@ -501,7 +501,10 @@ int launch_gemm_mid(const MfmaArgs& a, bool dual, hipStream_t st, const char* wh
 
 // Head expansions that the 256 x 256 tiles do not take: 64 rows of a head per tile, two workgroups per compute unit (us for q, k
 // and v of 32 heads at rank 1024, 64- or 128-row tiles of two stages -> this kernel: 16 rows 11.8 -> 10.6, 154 19.2 -> 15.6, 512
-// 30.1 -> 25.7, 768 41.8 -> 37.1; with 8 kv heads at 333 18.6 -> 15.3; 128 or 256 rows per tile: 30.6, 28.1 at 512).
+// 30.1 -> 25.7, 768 41.8 -> 37.1; with 8 kv heads at 333 18.6 -> 15.3; 128 or 256 rows per tile: 30.6, 28.1 at 512).  More than two tiles
+// per compute unit: two stages instead of three, so that three workgroups fit one (three / two stages with weights from HBM: 333 and
+// 512 rows of 96 heads at rank 1024 27.1 / 25.2, 29.9 / 28.3, at 1664 37.9 / 35.8, 42.7 / 39.4, 768 and 1024 rows of 48 heads at 512
+// 18.4 / 16.8, 20.5 / 18.3; with fewer tiles the longer distance wins: 154 rows of 96 heads 18.0 / 20.0, 77 13.1 / 17.5).
 bool expand_mid_apply(const ExpandArgs* d, int n) {
   for (int k = 0; k < n; ++k) {
     const ExpandArgs& a = d[k];
@@ -525,6 +528,9 @@ int launch_expand_mid(const ExpandArgs* d, int n, hipStream_t st) {
   for (int k = n; k < 4; ++k) m.first_head[k] = heads;
   m.nt = heads;
   const char* who = "fsvd_lowrank_expand_heads";
+  // more than two tiles per compute unit: a ring of two stages, so that three workgroups share one
+  if ((int64_t)heads * ((rows + 63) / 64) > 2 * compute_units())
+    return d[0].dt == 1 ? launch_mid_t<1, kMidHeads, 4, 2, 1, 4, 1, 2>(m, st, who) : launch_mid_t<0, kMidHeads, 4, 2, 1, 4, 1, 2>(m, st, who);
   return d[0].dt == 1 ? launch_mid_t<1, kMidHeads, 4, 2, 1, 4, 1, 3>(m, st, who) : launch_mid_t<0, kMidHeads, 4, 2, 1, 4, 1, 3>(m, st, who);
 }
 
