@@ -608,6 +608,12 @@ int fsvd_lowrank_expand_heads_multi(const fsvd_expand_desc* desc, int n, const v
   return kOk;
 }
 
+int fsvd_rope_tables(const int64_t* positions, const float* inv_freq, void* cos_out, void* sin_out, int64_t rows, int half, int dtype, void* stream) {
+  const char* fn = "fsvd_rope_tables";
+  FSVD_REQUIRE_PTR(positions, fn); FSVD_REQUIRE_PTR(inv_freq, fn); FSVD_REQUIRE_PTR(cos_out, fn); FSVD_REQUIRE_PTR(sin_out, fn);
+  return launch_rope_tables(positions, inv_freq, u16(cos_out), u16(sin_out), rows, half, dtype, static_cast<hipStream_t>(stream));
+}
+
 int fsvd_attn_prefill(const void* q, int64_t sq_b, int64_t sq_m, int64_t sq_h, const void* k, const void* v, int64_t sk_b,
                       int64_t sk_s, int64_t sk_h, const int32_t* q_pos0, const uint8_t* pad_mask, int64_t spm_b,
                       const float* add_mask, int64_t sam_b, int64_t sam_q, void* out, int64_t so_b, int64_t so_m, int64_t so_h,

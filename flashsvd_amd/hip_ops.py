@@ -796,6 +796,27 @@ def lowrank_expand_heads_multi(items, *, head_dim: int, cos: Optional[torch.Tens
     _lib.check("fsvd_lowrank_expand_heads_multi", rc)
 
 
+def rope_tables(position_ids: torch.Tensor, inv_freq: torch.Tensor, dtype: torch.dtype):
+    """cos, sin [rows, half] of ``position_ids.float() * inv_freq`` (contiguous int64 and fp32 tensors), rounded to ``dtype``,
+    in one launch.  Custom operator flashsvd_hip::rope_tables."""
+    return _OPS.rope_tables.default(position_ids, inv_freq, dtype)
+
+
+def _rope_tables_impl(position_ids, inv_freq, dtype):
+    code = _ELEM_CODES.get(dtype)
+    if code is None:
+        raise ValueError(f"rotation tables are torch.bfloat16 or torch.float16, got {dtype}")
+    _need(position_ids, "position_ids", dtype=torch.long); _need(inv_freq, "inv_freq", dtype=torch.float32)
+    if not position_ids.is_contiguous() or inv_freq.dim() != 1 or not inv_freq.is_contiguous():
+        raise ValueError("position_ids and inv_freq must be contiguous, inv_freq one-dimensional")
+    rows, half = position_ids.numel(), inv_freq.numel()
+    cos = torch.empty(rows, half, dtype=dtype, device=position_ids.device)
+    sin = torch.empty_like(cos)
+    _lib.check("fsvd_rope_tables", _lib.load().fsvd_rope_tables(position_ids.data_ptr(), inv_freq.data_ptr(), cos.data_ptr(), sin.data_ptr(), rows,
+                                                                half, code, _stream()))
+    return cos, sin
+
+
 def attn_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, q_pos0: Optional[torch.Tensor] = None, causal: bool = True,
                  pad_mask: Optional[torch.Tensor] = None, add_mask: Optional[torch.Tensor] = None,
                  out: Optional[torch.Tensor] = None, softmax_scale: Optional[float] = None) -> torch.Tensor:

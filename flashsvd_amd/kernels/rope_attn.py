@@ -55,7 +55,7 @@ class FlashSVDRoPEAttention(nn.Module):
         self.causal = True   # decoder-only
 
     def _tables(self, B: int, M: int, dh: int, position_ids, device, dtype):
-        """Per-token cos/sin rows [rows, dh/2] and the row offset of each batch entry."""
+        """Per-token cos/sin rows [rows, dh/2] and the row offset of each batch entry (None: they share the rows)."""
         if position_ids is None:
             position_ids = torch.arange(M, device=device, dtype=torch.long).unsqueeze(0)
         if position_ids.dim() == 1:
@@ -65,6 +65,10 @@ class FlashSVDRoPEAttention(nn.Module):
         if position_ids.shape[0] not in (1, B):
             raise ValueError(f"position_ids batch dim {position_ids.shape[0]} != B {B}")
         inv = getattr(self.rotary_emb, "inv_freq", None)
+        if torch.is_tensor(inv) and inv.dim() == 1 and inv.numel() == dh // 2 and inv.dtype == torch.float32 and inv.is_contiguous() \
+                and position_ids.dtype == torch.long and position_ids.is_contiguous() and inv.device == position_ids.device == device:
+            cos, sin = hip_ops.rope_tables(position_ids, inv, dtype)
+            return cos, sin, None if position_ids.shape[0] == 1 else torch.arange(B, dtype=torch.int32, device=device) * M
         if inv is not None:
             ang = position_ids.to(device=device, dtype=torch.float32)[..., None] * inv.to(device=device, dtype=torch.float32)
             cos, sin = torch.cos(ang).to(dtype), torch.sin(ang).to(dtype)          # [Bpos, M, dh/2]
@@ -78,7 +82,7 @@ class FlashSVDRoPEAttention(nn.Module):
                     cos, sin = cos[:, 0], sin[:, 0]
             cos, sin = cos[..., : dh // 2].to(dtype), sin[..., : dh // 2].to(dtype)
         shared = cos.shape[0] == 1
-        offs = torch.zeros(B, dtype=torch.int32, device=device) if shared else \
+        offs = None if shared else \
             torch.arange(B, dtype=torch.int32, device=device) * M
         return cos.reshape(-1, dh // 2).contiguous(), sin.reshape(-1, dh // 2).contiguous(), offs
 
@@ -116,7 +120,7 @@ class FlashSVDRoPEAttention(nn.Module):
         pad = add = None
         if attention_mask is not None:
             if attention_mask.dim() == 2:
-                pad = (attention_mask != 0).to(torch.uint8).contiguous()
+                pad = (attention_mask != 0).contiguous().view(torch.uint8)
             elif attention_mask.dim() == 4:
                 add = attention_mask[:, 0].to(torch.float32).expand(B, M, M).contiguous()
             else:

@@ -10,6 +10,7 @@ tensors.  ``flashsvd_amd.hip_ops`` and the modules under ``flashsvd_amd.kernels`
   rmsnorm / .out                      fsvd_rmsnorm
   lowrank_mlp                         fsvd_mlp_block_run     norm + rank projection + SwiGLU pair + down projection
   lowrank_attn_prefill                fsvd_attn_block_prefill   the attention half of a prompt pass over the dense cache
+  rope_tables                         fsvd_rope_tables
   greedy_token_                       fsvd_greedy_token      argmax of every row + position increment
   qkv_rope_append / .out              fsvd_qkv_rope_append   head expansion + RoPE + dense-cache append
   attn_decode_densekv / .out          fsvd_attn_decode_densekv(_static)   the flash_attn_with_kvcache role
@@ -119,6 +120,20 @@ _define("lowrank_attn_prefill(Tensor x, Tensor qkv_v, Tensor q_u, Tensor k_u, Te
         "Tensor(b!) v_cache, Tensor cos, Tensor sin, int start, int num_heads, int num_kv_heads, Tensor? norm_weight=None, float eps=1e-6, "
         "Tensor? residual=None, Tensor? o_v_bias=None, Tensor? o_u_bias=None) -> Tensor", _lowrank_attn_prefill,
         lambda x, qkv_v, q_u, k_u, v_u, o_v, o_u, *a, **k: x.new_empty((*x.shape[:-1], o_u.shape[0])))
+
+
+# ------------------------------------------------------------------ rotation tables of given positions
+def _rope_tables(position_ids, inv_freq, dtype):
+    from . import hip_ops
+    return hip_ops._rope_tables_impl(position_ids, inv_freq, dtype)
+
+
+def _rope_tables_fake(position_ids, inv_freq, dtype):
+    shape = (position_ids.numel(), inv_freq.numel())
+    return inv_freq.new_empty(shape, dtype=dtype), inv_freq.new_empty(shape, dtype=dtype)
+
+
+_define("rope_tables(Tensor position_ids, Tensor inv_freq, ScalarType dtype) -> (Tensor, Tensor)", _rope_tables, _rope_tables_fake)
 
 
 # ------------------------------------------------------------------ greedy token of every row
@@ -279,5 +294,5 @@ _define("mlp_dual_split(Tensor PUp, Tensor PGate, Tensor GateU, Tensor UpU, Tens
         PUp.new_empty((PUp.shape[0], DownU.shape[1])))
 
 ops = getattr(torch.ops, NS)
-OP_NAMES = ("linear", "swiglu_linear", "rmsnorm", "greedy_token_", "lowrank_mlp", "lowrank_attn_prefill", "qkv_rope_append", "attn_decode_densekv", "attn_decode_rankkv", "rankkv_append", "linear_rankkv_append",
+OP_NAMES = ("linear", "swiglu_linear", "rmsnorm", "greedy_token_", "lowrank_mlp", "lowrank_attn_prefill", "rope_tables", "qkv_rope_append", "attn_decode_densekv", "attn_decode_rankkv", "rankkv_append", "linear_rankkv_append",
             "lowrank_expand_heads", "rope_attn_prefill", "reconstruct_qkv_token", "xw_linear", "mlp_dual_split")
