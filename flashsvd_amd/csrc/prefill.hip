@@ -130,8 +130,10 @@ __global__ __launch_bounds__(kPfThreads) void lowrank_expand_kernel(ExpandArgs a
 //     roundings are packed two to an instruction, and the key padding mask is one 64-bit word per tile: a tile without a
 //     masked key runs unmasked, one without a visible key is skipped.  All of it gives the bits of the plain
 //     formula (one multiply-add in front of the exponential instruction and row sums left to the end would save another 4 %).
-//     Measured before -> after: 8 x 2048 tokens of 32 heads 758 -> 602 us (457 TFLOP/s), 4 x 1024 tokens 161 -> 122, with a
-//     padding mask 215 -> 120; 512 tokens 19.0 -> 16.0.  Below 128 rows a kernel without shared
+//     Measured before -> after: 8 x 2048 tokens of 32 heads 758 -> 602 us, 4 x 1024 tokens 161 -> 122, with a
+//     padding mask 215 -> 120; 512 tokens 19.0 -> 16.0.  Then, with every XCD starting the long tiles of all its heads first instead of
+//     head by head (on average 1.2 of two possible waves were resident per SIMD): 576 -> 506 us (543 TFLOP/s), 122 -> 85, padded
+//     121 -> 83; one sequence of 1024 / 2048 tokens 43 -> 36, 121 -> 97, 700 behind 1000 72 -> 63.  Below 128 rows a kernel without shared
 //     tiles ran: two chunks of 77 rows behind 1411 tokens (32 / 8 heads) 181 -> 31 us.  Two LDS stages instead of one, raised
 //     priority around the products and scalar address parts were built and gave nothing: two workgroups share a compute
 //     unit, and each covers the other's waits.
@@ -178,11 +180,23 @@ __global__ __launch_bounds__(kPfThreads * NG, NG == 1 ? 2 : 1) void attn_prefill
   uint16_t (*Ks)[KSTR] = reinterpret_cast<uint16_t (*)[KSTR]>(gsm);                                   // [BN][KSTR]
   uint16_t (*Vt)[VSTR] = reinterpret_cast<uint16_t (*)[VSTR]>(gsm + (size_t)BN * KSTR * 2);            // [DH][VSTR]
 
-  // the query tiles of a head (and the heads of a kv head) run on one XCD, so its K and V come out of one L2; under
-  // a causal mask the last tiles, which see the most keys, start first
-  const int MT = gridDim.x;
-  const int t = xcd_run_index(blockIdx.x + MT * (blockIdx.y + gridDim.y * blockIdx.z), MT * gridDim.y * gridDim.z);
-  const int mt = a.causal ? MT - 1 - t % MT : t % MT, h = (t / MT) % (int)gridDim.y, b = t / (MT * (int)gridDim.y);
+  // The query tiles of a head (and the heads of a kv head) run on one XCD, so its K and V come out of one L2; the sequences of
+  // a batch, which padding makes unequal, are spread over all of them.  Under a causal mask the last tiles see the most keys:
+  // every XCD starts those of all its heads first, so that the short ones fill the end of the launch, and the tiles of a head
+  // walk its keys side by side.
+  const int MT = gridDim.x, HB = gridDim.y * gridDim.z, id = blockIdx.x + MT * (blockIdx.y + gridDim.y * blockIdx.z);
+  int mt, hb;
+  if (HB % 8 == 0) {
+    const int per = HB >> 3, r = id >> 3;
+    mt = r / per;
+    hb = (id & 7) * per + r - mt * per;
+  } else {
+    const int t = xcd_run_index(id, MT * HB);
+    hb = t / MT;
+    mt = t - hb * MT;
+  }
+  if (a.causal) mt = MT - 1 - mt;
+  const int h = hb / (int)gridDim.z, b = hb - h * (int)gridDim.z;
   const int hk = h / (a.H / a.Hk);
   const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;   // thread and wave within the group
   const int lr = lane & 15, lg = lane >> 4;
