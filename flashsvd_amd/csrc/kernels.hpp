@@ -224,6 +224,8 @@ int launch_expand_big(const ExpandArgs* d, int n, hipStream_t st);
 bool gemm_mid_apply(const MfmaArgs& a, bool dual);                          // mfma_mid.hip: about one tile per compute unit
 int launch_gemm_mid(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
 size_t gemm_share_floats(MfmaArgs a, size_t cap);
+bool gemm_mid_ragged_apply(const MfmaArgs& a, bool dual);                    // mfma_mid.hip: 128 rows and more, any K and rows
+int launch_mid_ragged(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
 size_t linear_scratch_floats(const LinearArgs& a, size_t cap);              // mfma_gemv.hip
 bool expand_mid_apply(const ExpandArgs* d, int n);
 int launch_expand_mid(const ExpandArgs* d, int n, hipStream_t st);

@@ -666,8 +666,10 @@ bool gemm_ragged_apply(const MfmaArgs& a) {
 // rows 12.7 / 11.1, 13.6 / 12.0, 13.4 / 11.7, 1492 x 4104 27.4 / 19.4, 28.9 / 21.7, 28.1 / 21.0, 64 x 64 tiles alike: 4096 x 1492 at
 // 333, 500 rows 21.5 / 19.9, 23.7 / 22.0, 1492 x 4104 26.4 / 22.8, 32.5 / 26.1.  The pair at 3, 16, 64, 127 rows: 11008 x 1492
 // 24.7, 27.1, 43.4, 55.1 (with a split over three workgroups, which has to park partial tiles, 33.1, 34.6, 41.0, 54.8).
+// From 128 rows on the tiles of mfma_mid.hip take what gives about every compute unit one (or several rounds of the pair's).
 template <int DT>
 static int launch_gemm_ragged_dt(const MfmaArgs& a, bool dual, hipStream_t st, const char* who) {
+  if (gemm_mid_ragged_apply(a, dual)) return launch_mid_ragged(a, dual, st, who);
   const int64_t big = (int64_t)((a.N + 127) / 128) * ((a.B + 127) / 128);
   if (dual) {
     if (a.B < 128) return launch_gemm_tiles_t<DT, true, 1, 2, 64, 4, 2, true>(a, st, who);

@@ -32,11 +32,15 @@ struct MidArgs {
   int shares, per; float* part;                      // kMidShare: workgroups per tile, the K steps of each (the last one may have fewer), their sums
 };
 
-template <int DT, int EPI, int WM, int WN, int TM, int TN, int KH, int NS>
+// RAG: any K, rows that start anywhere (plain and pair).  Loads that write LDS themselves want aligned addresses, so the pieces go
+// through registers, two steps ahead of the two LDS stages; the steps past the last whole one are masked to the row, an even
+// number of steps in all, so that stage and register set of a step are known to the compiler.
+template <int DT, int EPI, int WM, int WN, int TM, int TN, int KH, int NS, bool RAG = false>
 __global__ __launch_bounds__(kMidThreads, 2) void gemm_mid_kernel(MidArgs args) {
   typedef E16<DT> E;
   typedef typename E::frag_t frag_t;
   static_assert(WM * WN * KH == 8, "eight waves");
+  static_assert(!RAG || (KH == 1 && NS == 2 && (EPI == kMidPlain || EPI == kMidPair)), "ragged rows: two stages, plain and pair");
   constexpr bool PAIR = EPI == kMidPair, HEADS = EPI == kMidHeads, SHARE = EPI == kMidShare;
   constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN, LX = BM / 64, LW = BN / 64, LOADS = KH * (LX + LW);
   static_assert(BM % 64 == 0 && BN % 64 == 0 && (!HEADS || (BN == 128 && TN % 2 == 0)), "whole groups of rows per load");
@@ -73,7 +77,7 @@ __global__ __launch_bounds__(kMidThreads, 2) void gemm_mid_kernel(MidArgs args) 
 #pragma unroll
   for (int j = 0; j < LW; ++j) wo[j] = (uint32_t)(min(n0 + lrow + 64 * j, a.N - 1) * a.ldw * 2) + lpiece;
   const int first = SHARE ? share * args.per : 0, k0 = first * 128 * KH;          // this share's first K step, and its place in a row
-  const int ksteps = SHARE ? min(args.per, a.K / 64 - first) : a.K / (64 * KH), total = (PAIR ? 2 : 1) * ksteps;
+  const int ksteps = SHARE ? min(args.per, a.K / 64 - first) : (RAG ? (a.K + 127) / 128 * 2 : a.K / (64 * KH)), total = (PAIR ? 2 : 1) * ksteps;
   const uint32_t my_rows = (uint32_t)__builtin_amdgcn_readfirstlane(wave) * 1024;
   const auto issue = [&](int s, int stage) {
     const bool second = PAIR && s >= ksteps;
@@ -120,17 +124,73 @@ __global__ __launch_bounds__(kMidThreads, 2) void gemm_mid_kernel(MidArgs args) 
       for (int j = 0; j < TN; ++j) acc[i][j] = E::mfma(f.w[j], f.x[i], acc[i][j]);
     __builtin_amdgcn_sched_barrier(0);
   };
+  u32x4_t rx[RAG ? 2 : 1][LX], rw[RAG ? 2 : 1][LW];    // ragged: the pieces of steps s + 2 and s + 3
+  const auto fetch = [&](int set, int s) {
+    const bool second = PAIR && s >= ksteps;
+    const int k = (second ? s - ksteps : s) * 64;
+    const char* xb = reinterpret_cast<const char*>(a.x + (second ? a.up_off : 0) + k);
+    const char* wb = reinterpret_cast<const char*>((second ? a.W2 : a.W) + k);
+    if (k + 64 <= a.K) {
 #pragma unroll
-  for (int s = 0; s < NS; ++s)
-    if (s < total) issue(s, s);
+      for (int j = 0; j < LX; ++j) rx[set][j] = *reinterpret_cast<const u32x4_any_t*>(xb + xo[j]);
+#pragma unroll
+      for (int j = 0; j < LW; ++j) rw[set][j] = *reinterpret_cast<const u32x4_any_t*>(wb + wo[j]);
+    } else {
+      const int left = a.K - k - lpiece / 2;
+#pragma unroll
+      for (int j = 0; j < LX; ++j) rx[set][j] = load_masked_piece(reinterpret_cast<const uint16_t*>(xb + xo[j]), left, a.K);
+#pragma unroll
+      for (int j = 0; j < LW; ++j) rw[set][j] = load_masked_piece(reinterpret_cast<const uint16_t*>(wb + wo[j]), left, a.K);
+    }
+  };
+  const auto park = [&](int set, int st) {
+    unsigned char* dst = mid_smem + st * kStage + tid * 16;
+#pragma unroll
+    for (int j = 0; j < LX; ++j) *reinterpret_cast<u32x4_t*>(dst + j * 64 * kMidRow) = rx[set][j];
+#pragma unroll
+    for (int j = 0; j < LW; ++j) *reinterpret_cast<u32x4_t*>(dst + (BM + j * 64) * kMidRow) = rw[set][j];
+  };
   constexpr int kW1 = (NS - 1) * LOADS, kW2 = (NS - 2) * LOADS;
-  if (total >= NS) __builtin_amdgcn_s_waitcnt(0x0f70 | (kW1 & 15) | ((kW1 >> 4) << 14));
-  else __builtin_amdgcn_s_waitcnt(0x0f70);
+  if constexpr (RAG) {
+    fetch(0, 0);
+    fetch(1, 1);
+    park(0, 0);
+    park(1, 1);
+    if (total > 2) {
+      fetch(0, 2);
+      fetch(1, 3);
+    }
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+  } else {
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+      if (s < total) issue(s, s);
+    if (total >= NS) __builtin_amdgcn_s_waitcnt(0x0f70 | (kW1 & 15) | ((kW1 >> 4) << 14));
+    else __builtin_amdgcn_s_waitcnt(0x0f70);
+  }
   barrier();
   Frags f0, f1;
   read(f0, 0, 0);
   int stage = 0;
   const auto walk = [&](const int begin, const int end) {
+    if constexpr (RAG) {
+      for (int s0 = begin; s0 < end; s0 += 2) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const int s = s0 + u;
+          read(f1, u, 1);
+          multiply(f0);
+          // the stage is read to its end and the other one written by this wave; behind the barrier by all of them
+          __builtin_amdgcn_s_waitcnt(0xc07f);
+          barrier();
+          if (s + 1 < total) read(f0, u ^ 1, 0);
+          if (s + 2 < total) park(u, u);
+          if (s + 4 < total) fetch(u, s + 4);
+          multiply(f1);
+        }
+      }
+      return;
+    }
     for (int s = begin; s < end; ++s) {
       read(f1, stage, 1);
       multiply(f0);
@@ -288,21 +348,21 @@ __global__ __launch_bounds__(kMidThreads, 2) void gemm_mid_kernel(MidArgs args) 
   }
 }
 
-template <int DT, int EPI, int WM, int WN, int TM, int TN, int KH, int NS>
+template <int DT, int EPI, int WM, int WN, int TM, int TN, int KH, int NS, bool RAG = false>
 static int launch_mid_t(MidArgs& m, hipStream_t st, const char* who) {
   static bool granted = false;
   constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN;
   constexpr size_t lds = (size_t)NS * KH * (BM + BN) * kMidRow;
   if (!granted) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_mid_kernel<DT, EPI, WM, WN, TM, TN, KH, NS>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_mid_kernel<DT, EPI, WM, WN, TM, TN, KH, NS, RAG>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) { set_last_error("%s: cannot reserve %zu bytes of LDS: %s", who, lds, hipGetErrorString(e)); return kErrLaunch; }
     granted = true;
   }
   if (EPI != kMidHeads) m.nt = (m.a[0].N + BN - 1) / BN;
   const int64_t tiles = (int64_t)m.nt * ((m.a[0].B + BM - 1) / BM);
-  static constexpr FormText form = form_text("ring ", BM, BN, EPI == kMidPair ? " pair" : (EPI == kMidHeads ? " heads" : ""));
+  static constexpr FormText form = form_text(RAG ? "any ring " : "ring ", BM, BN, EPI == kMidPair ? " pair" : (EPI == kMidHeads ? " heads" : ""));
   set_last_form(form.s);
-  hipLaunchKernelGGL((gemm_mid_kernel<DT, EPI, WM, WN, TM, TN, KH, NS>), dim3((unsigned)tiles), dim3(kMidThreads), lds, st, m);
+  hipLaunchKernelGGL((gemm_mid_kernel<DT, EPI, WM, WN, TM, TN, KH, NS, RAG>), dim3((unsigned)tiles), dim3(kMidThreads), lds, st, m);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }
   return kOk;
@@ -497,6 +557,41 @@ int launch_gemm_mid(const MfmaArgs& a, bool dual, hipStream_t st, const char* wh
   const ShareForm f = dual ? ShareForm{0, 0, 0} : share_form(a);
   if (f.shares > 0) return a.dt == 1 ? launch_share_dt<1>(a, f, st, who) : launch_share_dt<0>(a, f, st, who);
   return a.dt == 1 ? launch_gemm_mid_dt<1>(a, dual, st, who) : launch_gemm_mid_dt<0>(a, dual, st, who);
+}
+
+// Ragged rows of 128 and more.  us with weights from HBM, the two-stage tiles of mfma_gemm.hip -> this:
+// The pair by the fills of the aligned one: 128 x 192 tiles, 11008 x 1492 at 333 / 512 / 768 / 1024 / 1500 rows 82 -> 65, 126 -> 67, 151 ->
+// 125, 172 -> 125, 240 -> 185, 5504 x 746 at 768 / 1024 57 -> 38, 68 -> 39; 64 x 192, 11008 x 1492 at 154 / 200 56 -> 52, 56 -> 50 (128 rows, 116
+// tiles, 52 against 57), 5504 x 746 at 333 / 512 32 -> 28, 42 -> 30 (aligned rows, 1536 and 768: 48, 49, 84, 92 and 28, 29).  What is left of
+// the difference is pieces that straddle cache lines and their way through registers.
+// A single matrix: 128 x 128 tiles for 144 to 256 of them, 4096 x 1492 at 768 / 1024 rows 30 -> 27, 33 -> 27, 3000 x 1001 at 768 25 -> 19,
+// 2048 x 746 at 1500 18 -> 13 (more than a round of them, 1500 x 4096 x 1492, 42 against 50); 64 x 128 likewise, 4096 x 1492 at 512
+// 22 -> 20, 3000 x 1001 at 333 / 512 17 -> 14, 19 -> 14, 2048 x 746 at 768 / 1024 12 -> 10, 13 -> 10, above a K of 2048 from seven eighths of
+// a round on (4096 x 2390 at 512 rows, 256 tiles, 31 -> 30; at 333, 192 tiles, 27 against 28).
+enum RagForm { kRagNone = 0, kRag128x192, kRag64x192, kRag128x128, kRag64x128 };
+static RagForm mid_ragged_form(const MfmaArgs& a, bool dual) {
+  const int64_t cu = compute_units();
+  if (a.B < 128 || cu <= 0 || a.K < 128 || !below_4gib(a.B, a.ldx) || !below_4gib(a.N, a.ldw)) return kRagNone;     // two whole steps at least
+  if (dual) return mid_fills(mid_tiles(a, 128, 192), 55) ? kRag128x192 : (mid_fills(mid_tiles(a, 64, 192), 60) ? kRag64x192 : kRagNone);
+  const auto about_one = [&](int64_t t) { return t * 16 >= cu * 9 && t <= cu; };
+  if (about_one(mid_tiles(a, 128, 128))) return kRag128x128;
+  const int64_t t = mid_tiles(a, 64, 128);
+  return about_one(t) && (a.K <= 2048 || t * 8 >= cu * 7) ? kRag64x128 : kRagNone;
+}
+bool gemm_mid_ragged_apply(const MfmaArgs& a, bool dual) { return mid_ragged_form(a, dual) != kRagNone; }
+template <int DT>
+static int launch_mid_ragged_dt(const MfmaArgs& a, bool dual, hipStream_t st, const char* who) {
+  MidArgs m{};
+  m.a[0] = a;
+  switch (mid_ragged_form(a, dual)) {
+    case kRag128x192: return launch_mid_t<DT, kMidPair, 2, 4, 4, 3, 1, 2, true>(m, st, who);
+    case kRag64x192: return launch_mid_t<DT, kMidPair, 2, 4, 2, 3, 1, 2, true>(m, st, who);
+    case kRag128x128: return launch_mid_t<DT, kMidPlain, 2, 4, 4, 2, 1, 2, true>(m, st, who);
+    default: return launch_mid_t<DT, kMidPlain, 2, 4, 2, 2, 1, 2, true>(m, st, who);
+  }
+}
+int launch_mid_ragged(const MfmaArgs& a, bool dual, hipStream_t st, const char* who) {
+  return a.dt == 1 ? launch_mid_ragged_dt<1>(a, dual, st, who) : launch_mid_ragged_dt<0>(a, dual, st, who);
 }
 
 // Head expansions that the 256 x 256 tiles do not take: 64 rows of a head per tile, two workgroups per compute unit (us for q, k
