@@ -14,15 +14,45 @@ namespace fsvd {
 constexpr int kAttnThreads = 256;
 constexpr int kMaxKeysPerSplit = 1 << 20;  // the key loop is streamed; only a sanity bound
 
+// Workgroup -> key range s of query head (or head group) h of sequence b.  Consecutive workgroup ids go round-robin over the 8
+// XCDs: the ranges of one head (which meet again in the merge) run on the same XCD, the first range of all its heads before
+// the second of any, so that workgroups without a range, which leave at once, are the last ones (between the others they left
+// the compute units unevenly loaded: 16 x 1000 keys 93 us, now 49).  With head_dim 128 an XCD takes some heads of every sequence,
+// not every head of some: sequences of 1 to 2000 keys, 8 x 32 heads, 41 -> 28 us, 64 x up to 300 34.9 -> 29.6.  With
+// head_dim 64 the pieces of a row that an XCD then reads are too small for that (64 x 1000 keys 98.7 -> 105).
+// Each range starts at another pair, so that a long sequence's ranges don't meet on one compute unit.
+template <int DH>
 __device__ __forceinline__ void decode_work_item(int B, int H, int nsplit, int& b, int& h, int& s) {
-  // Consecutive workgroup ids go round-robin over the 8 XCDs; remap so that the splits of one
-  // head (which meet again in the merge) run on the same XCD and share its L2.
-  const int total = B * H * nsplit;
-  int id = blockIdx.x;
-  if ((total & 7) == 0) id = (id & 7) * (total >> 3) + (id >> 3);
-  s = id % nsplit;
-  h = (id / nsplit) % H;
-  b = id / (nsplit * H);
+  const int pairs = B * H;
+  const bool by_xcd = (pairs & 7) == 0;
+  const int per = by_xcd ? pairs >> 3 : pairs, xcd = by_xcd ? blockIdx.x & 7 : 0;
+  const int id = by_xcd ? blockIdx.x >> 3 : blockIdx.x;
+  s = id / per;
+  const int local = (id - s * per + s * max(1, per / nsplit)) % per;
+  if (DH == 128 && (H & 7) == 0) {
+    const int heads = H >> 3;
+    h = xcd * heads + local % heads;
+    b = local / heads;
+  } else {
+    const int pair = xcd * per + local;
+    h = pair % H;
+    b = pair / H;
+  }
+}
+
+// Key ranges that a sequence of n keys is cut into, at most nsplit (what the scratch holds): known from the length alone, so
+// the same launch serves a cache that is nearly empty and one that is full; the other workgroups of (b, h) leave at once.
+// A range holds at least one pass of 128 keys.  Where the heads of all sequences fill the chip by themselves (one query head per
+// workgroup, 256 pairs and more) ranges only even out sequences of different lengths: from 2 keys a pair on, and an odd count
+// (the starts of two or four equal ranges lie a power of two apart, and their workgroups ask the same memory channels at the
+// same time).  Both sides with 32 heads: 16 x 1000 keys 53.0 us in four ranges, 49.3 in one (in a cache of 1024 rows 67.2,
+// 51.7), 32 x 1000 94.3 and 92.0, 8 x 1 to 2000 33.8 in eight and 27.2 in up to three; one sequence of 300 keys in a cache of
+// 4096 rows 13.0 in 32, 6.7 in three.
+template <int G>
+__device__ __forceinline__ int key_ranges(const AttnDecodeArgs& a, int n_keys) {
+  int n = min(a.nsplit, (n_keys + 127) >> 7);
+  if (G == 1 && a.B * a.H >= 256) n = min(n, (n_keys / (2 * a.B * a.H)) | 1);
+  return max(1, n);
 }
 
 // coherent (L2-bypassing) scalar accessors for the cross-workgroup partials: the producers write
@@ -79,12 +109,14 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
   __shared__ int last_flag;
 
   int b, h, s;
-  decode_work_item(a.B, a.H, a.nsplit, b, h, s);
+  decode_work_item<DH>(a.B, a.H, a.nsplit, b, h, s);
   const int tid = threadIdx.x;
   const int hk = h / (a.H / a.Hk);
   int n_keys = a.seqlens[b] + a.seqlen_add;
   n_keys = max(0, min(n_keys, a.S));
-  int per = (n_keys + a.nsplit - 1) / a.nsplit;
+  const int ranges = key_ranges<1>(a, n_keys);
+  if (s >= ranges) return;
+  int per = (n_keys + ranges - 1) / ranges;
   per = (per + KPB - 1) / KPB * KPB;
   const int k0 = min(s * per, n_keys);
   const int k1 = min(n_keys, k0 + per);
@@ -179,7 +211,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
   }
 
   uint16_t* outp = a.out + (int64_t)b * a.so_b + (int64_t)h * a.so_h;
-  if (a.nsplit == 1) {
+  if (ranges == 1) {
     if (tid < DH) outp[tid] = (uint16_t)E::bits(l > 0.f ? o / l : 0.f);
     return;
   }
@@ -191,7 +223,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
   __syncthreads();
   if (tid == 0) {
     const int old = __hip_atomic_fetch_add(&a.ws_count[b * a.H + h], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    last_flag = (old == a.nsplit - 1);
+    last_flag = (old == ranges - 1);
   }
   __syncthreads();
   if (!last_flag) return;
@@ -201,26 +233,26 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
     // made this merge a third of the kernel at eight splits); the splits are added in order
     constexpr int SU = 8;
     float M = -INFINITY;
-    for (int i0 = 0; i0 < a.nsplit; i0 += SU) {
+    for (int i0 = 0; i0 < ranges; i0 += SU) {
       float mi[SU];
 #pragma unroll
-      for (int u = 0; u < SU; ++u) mi[u] = ld_agent(part_ws + (int64_t)min(i0 + u, a.nsplit - 1) * (DH + 2) + DH);
+      for (int u = 0; u < SU; ++u) mi[u] = ld_agent(part_ws + (int64_t)min(i0 + u, ranges - 1) * (DH + 2) + DH);
 #pragma unroll
       for (int u = 0; u < SU; ++u) M = fmaxf(M, mi[u]);
     }
     float num = 0.f, den = 0.f;
-    for (int i0 = 0; i0 < a.nsplit; i0 += SU) {
+    for (int i0 = 0; i0 < ranges; i0 += SU) {
       float mi[SU], oi[SU], li[SU];
 #pragma unroll
       for (int u = 0; u < SU; ++u) {
-        const float* pw = part_ws + (int64_t)min(i0 + u, a.nsplit - 1) * (DH + 2);
+        const float* pw = part_ws + (int64_t)min(i0 + u, ranges - 1) * (DH + 2);
         mi[u] = ld_agent(pw + DH);
         oi[u] = ld_agent(pw + tid);
         li[u] = ld_agent(pw + DH + 1);
       }
 #pragma unroll
       for (int u = 0; u < SU; ++u) {
-        const float w = (i0 + u >= a.nsplit || mi[u] == -INFINITY) ? 0.f : __expf(mi[u] - M);
+        const float w = (i0 + u >= ranges || mi[u] == -INFINITY) ? 0.f : __expf(mi[u] - M);
         num += w * oi[u];
         den += w * li[u];
       }
@@ -249,12 +281,14 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_gqa_kernel(AttnDecod
   __shared__ int last_flag;
 
   int b, hg, s;
-  decode_work_item(a.B, a.H / G, a.nsplit, b, hg, s);
+  decode_work_item<DH>(a.B, a.H / G, a.nsplit, b, hg, s);
   const int tid = threadIdx.x;
   const int h0 = hg * G, hk = h0 / (a.H / a.Hk);
   int n_keys = a.seqlens[b] + a.seqlen_add;
   n_keys = max(0, min(n_keys, a.S));
-  int per = (n_keys + a.nsplit - 1) / a.nsplit;
+  const int ranges = key_ranges<G>(a, n_keys);
+  if (s >= ranges) return;
+  int per = (n_keys + ranges - 1) / ranges;
   per = (per + KPB - 1) / KPB * KPB;
   const int k0 = min(s * per, n_keys);
   const int k1 = min(n_keys, k0 + per);
@@ -370,7 +404,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_gqa_kernel(AttnDecod
     for (int j = 0; j < KPB; ++j) o[i] += accs[g][j * DH + d];
   }
   const auto leave = [&](int i, float v) { a.out[(int64_t)b * a.so_b + (int64_t)(h0 + g0 + i * GS) * a.so_h + d] = (uint16_t)E::bits(v); };
-  if (a.nsplit == 1) {
+  if (ranges == 1) {
 #pragma unroll
     for (int i = 0; i < NG; ++i) leave(i, l[i] > 0.f ? o[i] / l[i] : 0.f);
     return;
@@ -394,7 +428,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_gqa_kernel(AttnDecod
   int* count = &a.ws_count[b * a.H + h0];          // one arrival per split for the whole group
   if (tid == 0) {
     const int old = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    last_flag = (old == a.nsplit - 1);
+    last_flag = (old == ranges - 1);
   }
   __syncthreads();
   if (!last_flag) return;
@@ -403,24 +437,24 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_gqa_kernel(AttnDecod
   float M[NG], num[NG], den[NG];
 #pragma unroll
   for (int i = 0; i < NG; ++i) { M[i] = -INFINITY; num[i] = 0.f; den[i] = 0.f; }
-  for (int i0 = 0; i0 < a.nsplit; i0 += SU) {
+  for (int i0 = 0; i0 < ranges; i0 += SU) {
     float mi[NG][SU];
 #pragma unroll
     for (int i = 0; i < NG; ++i)
 #pragma unroll
-      for (int u = 0; u < SU; ++u) mi[i][u] = ld_agent(part_ws + (g0 + i * GS) * head_ws + (int64_t)min(i0 + u, a.nsplit - 1) * (DH + 2) + DH);
+      for (int u = 0; u < SU; ++u) mi[i][u] = ld_agent(part_ws + (g0 + i * GS) * head_ws + (int64_t)min(i0 + u, ranges - 1) * (DH + 2) + DH);
 #pragma unroll
     for (int i = 0; i < NG; ++i)
 #pragma unroll
       for (int u = 0; u < SU; ++u) M[i] = fmaxf(M[i], mi[i][u]);
   }
-  for (int i0 = 0; i0 < a.nsplit; i0 += SU) {
+  for (int i0 = 0; i0 < ranges; i0 += SU) {
     float mi[NG][SU], oi[NG][SU], li[NG][SU];
 #pragma unroll
     for (int i = 0; i < NG; ++i)
 #pragma unroll
       for (int u = 0; u < SU; ++u) {
-        const float* pw = part_ws + (g0 + i * GS) * head_ws + (int64_t)min(i0 + u, a.nsplit - 1) * (DH + 2);
+        const float* pw = part_ws + (g0 + i * GS) * head_ws + (int64_t)min(i0 + u, ranges - 1) * (DH + 2);
         mi[i][u] = ld_agent(pw + DH);
         oi[i][u] = ld_agent(pw + d);
         li[i][u] = ld_agent(pw + DH + 1);
@@ -429,7 +463,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_gqa_kernel(AttnDecod
     for (int i = 0; i < NG; ++i)
 #pragma unroll
       for (int u = 0; u < SU; ++u) {
-        const float w = (i0 + u >= a.nsplit || mi[i][u] == -INFINITY) ? 0.f : __expf(mi[i][u] - M[i]);
+        const float w = (i0 + u >= ranges || mi[i][u] == -INFINITY) ? 0.f : __expf(mi[i][u] - M[i]);
         num[i] += w * oi[i][u];
         den[i] += w * li[i][u];
       }
@@ -457,7 +491,8 @@ size_t attn_decode_ws_floats(int B, int H, int nsplit, int Dh) { return (size_t)
 template <int DT>
 static void launch_attn_decode_t(const AttnDecodeArgs& a, int G, hipStream_t st) {
   dim3 grid(a.B * (a.H / G) * a.nsplit);
-  if (G == 4) hipLaunchKernelGGL((attn_decode_gqa_kernel<DT, 128, 8, 4>), grid, dim3(kAttnThreads), 0, st, a);
+  if (G == 4 && a.Dh == 64) hipLaunchKernelGGL((attn_decode_gqa_kernel<DT, 64, 4, 4>), grid, dim3(kAttnThreads), 0, st, a);
+  else if (G == 4) hipLaunchKernelGGL((attn_decode_gqa_kernel<DT, 128, 8, 4>), grid, dim3(kAttnThreads), 0, st, a);
   else if (G == 2) hipLaunchKernelGGL((attn_decode_gqa_kernel<DT, 128, 8, 2>), grid, dim3(kAttnThreads), 0, st, a);
   else if (a.Dh == 128) hipLaunchKernelGGL((attn_decode_kernel<DT, 128, 8>), grid, dim3(kAttnThreads), 0, st, a);
   else hipLaunchKernelGGL((attn_decode_kernel<DT, 64, 4>), grid, dim3(kAttnThreads), 0, st, a);
@@ -494,9 +529,9 @@ int launch_attn_decode(const AttnDecodeArgs& args, hipStream_t st) {
   // per group of query heads
   const int rep = a.H / a.Hk;
   int G = 1;
-  if (a.Dh == 128) {
-    if (rep % 4 == 0 && (int64_t)a.B * (a.H / 4) * a.nsplit >= 512) G = 4;
-    else if (rep % 2 == 0 && (int64_t)a.B * (a.H / 2) * a.nsplit >= 512) G = 2;
+  if (rep % 4 == 0 && (int64_t)a.B * (a.H / 4) * a.nsplit >= 512) G = 4;
+  else if (a.Dh == 128) {
+    if (rep % 2 == 0 && (int64_t)a.B * (a.H / 2) * a.nsplit >= 512) G = 2;
   }
   if (a.k_new && !append_in_kernel(a, G)) {
     const KvAppendArgs ka{a.k_new, a.v_new, a.sk_b, a.sk_h, a.sv_b, a.sv_h, const_cast<uint16_t*>(a.k_cache), const_cast<uint16_t*>(a.v_cache),
