@@ -14,44 +14,58 @@ namespace fsvd {
 constexpr int kAttnThreads = 256;
 constexpr int kMaxKeysPerSplit = 1 << 20;  // the key loop is streamed; only a sanity bound
 
-// Workgroup -> key range s of query head (or head group) h of sequence b.  Consecutive workgroup ids go round-robin over the 8
-// XCDs: the ranges of one head (which meet again in the merge) run on the same XCD, the first range of all its heads before
-// the second of any, so that workgroups without a range, which leave at once, are the last ones (between the others they left
-// the compute units unevenly loaded: 16 x 1000 keys 93 us, now 49).  With head_dim 128 an XCD takes some heads of every sequence,
-// not every head of some: sequences of 1 to 2000 keys, 8 x 32 heads, 41 -> 28 us, 64 x up to 300 34.9 -> 29.6.  With
-// head_dim 64 the pieces of a row that an XCD then reads are too small for that (64 x 1000 keys 98.7 -> 105).
-// Each range starts at another pair, so that a long sequence's ranges don't meet on one compute unit.
+// Workgroup -> key range s of query head (or head group) h of sequence b, len = seqlens[b].  Consecutive workgroup ids go
+// round-robin over the 8 XCDs: the ranges of one head (which meet again in the merge) run on the same XCD, the first range of all
+// its heads before the second of any, so that workgroups without a range, which leave at once, are the last ones (between the
+// others they left the compute units unevenly loaded: 16 x 1000 keys 93 us).
+// Up to 64 sequences with head_dim 128, 1024 pairs (four per compute unit; beyond, the order of dispatch evens things out, and
+// 48 x 500 keys of 32 heads are 68 us this way, 71 the other): an XCD takes some heads of every sequence, not every head of some, the
+// sequences longest first, and every other 32 workgroups of an XCD (one per compute unit) in reverse, so that the ranges of a
+// long and of a short sequence share a compute unit.  Without -> with, 32 heads: 16 x 1 to 1000 keys 31.4 -> 27.0 us, 32 x 1 to
+// 1000 55.6 -> 46.2, 16 x 4000 175.6 -> 171.2; 64 x 1 to 1000, four heads a group, 42.7 -> 32.8.  With head_dim 64 the pieces of
+// a row that an XCD then reads are too small (64 x 1000 keys 98.7 -> 105).
 template <int DH>
-__device__ __forceinline__ void decode_work_item(int B, int H, int nsplit, int& b, int& h, int& s) {
+__device__ __forceinline__ void decode_work_item(const int32_t* seqlens, int B, int H, int& b, int& h, int& s, int& len) {
   const int pairs = B * H;
   const bool by_xcd = (pairs & 7) == 0;
   const int per = by_xcd ? pairs >> 3 : pairs, xcd = by_xcd ? blockIdx.x & 7 : 0;
-  const int id = by_xcd ? blockIdx.x >> 3 : blockIdx.x;
-  s = id / per;
-  const int local = (id - s * per + s * max(1, per / nsplit)) % per;
-  if (DH == 128 && (H & 7) == 0) {
-    const int heads = H >> 3;
-    h = xcd * heads + local % heads;
-    b = local / heads;
+  int id = by_xcd ? blockIdx.x >> 3 : blockIdx.x;
+  if (DH == 128 && (H & 7) == 0 && B <= 64 && pairs <= 1024) {
+    if ((id & 32) && (id | 31) < (int)(gridDim.x >> 3)) id ^= 31;
+    s = id / per;
+    id -= s * per;
+    const int heads = H >> 3, lane = threadIdx.x & 63;
+    h = xcd * heads + id % heads;
+    const int n = seqlens[min(lane, B - 1)];
+    int rank = 0;                     // of this lane's sequence, longest first
+    for (int u = 0; u < B; ++u) {
+      const int nu = __builtin_amdgcn_readlane(n, u);
+      rank += nu > n || (nu == n && u < lane);
+    }
+    b = __builtin_ctzll(__ballot(lane < B && rank == id / heads));
+    len = __builtin_amdgcn_readlane(n, b);
   } else {
-    const int pair = xcd * per + local;
+    s = id / per;
+    const int turn = max(1, per * pairs / (int)gridDim.x);     // a range later: another compute unit
+    const int pair = xcd * per + (id - s * per + s * turn) % per;
     h = pair % H;
     b = pair / H;
+    len = seqlens[b];
   }
 }
 
 // Key ranges that a sequence of n keys is cut into, at most nsplit (what the scratch holds): known from the length alone, so
 // the same launch serves a cache that is nearly empty and one that is full; the other workgroups of (b, h) leave at once.
 // A range holds at least one pass of 128 keys.  Where the heads of all sequences fill the chip by themselves (one query head per
-// workgroup, 256 pairs and more) ranges only even out sequences of different lengths: from 2 keys a pair on, and an odd count
-// (the starts of two or four equal ranges lie a power of two apart, and their workgroups ask the same memory channels at the
-// same time).  Both sides with 32 heads: 16 x 1000 keys 53.0 us in four ranges, 49.3 in one (in a cache of 1024 rows 67.2,
-// 51.7), 32 x 1000 94.3 and 92.0, 8 x 1 to 2000 33.8 in eight and 27.2 in up to three; one sequence of 300 keys in a cache of
-// 4096 rows 13.0 in 32, 6.7 in three.
-template <int G>
+// workgroup, 256 pairs and more) ranges only even out sequences of different lengths: from 2 keys a pair on (one with head_dim 64,
+// whose sequences stay on one XCD), and an odd count (the starts of two or four equal ranges lie a power of two apart, and
+// their workgroups ask the same memory channels at the same time).  Both sides with 32 heads: 16 x 1000 keys 55.1 us in four
+// ranges, 46.9 in one (in a cache of 1024 rows 67.2, 48.9), 32 x 1000 95.6 and 88.4, 16 x 750 to 1000 47.7 and 42.7; one sequence
+// of 300 keys in a cache of 4096 rows 13.0 in 32, 6.6 in three.
+template <int DH, int G>
 __device__ __forceinline__ int key_ranges(const AttnDecodeArgs& a, int n_keys) {
   int n = min(a.nsplit, (n_keys + 127) >> 7);
-  if (G == 1 && a.B * a.H >= 256) n = min(n, (n_keys / (2 * a.B * a.H)) | 1);
+  if (G == 1 && a.B * a.H >= 256) n = min(n, (n_keys / (DH / 64 * a.B * a.H)) | 1);
   return max(1, n);
 }
 
@@ -88,9 +102,8 @@ __device__ __forceinline__ void append_pair(const Args& a, int half, int b, int 
 // Only where no other workgroup reads the row (append_in_kernel).  Against a launch of its own for the append: 16 sequences of
 // up to 4001 keys, 32 heads over 8, 53.5 -> 50.1 us, 64 x 1000 49.8 -> 48.0, 16 x 1000 with 32 kv heads 49.6 -> 46.9.
 template <int DT, int DH>
-__device__ __forceinline__ void append_own_row(const AttnDecodeArgs& a, int b, int hk, int k0, int k1) {
+__device__ __forceinline__ void append_own_row(const AttnDecodeArgs& a, int b, int hk, int pos, int k0, int k1) {
   if (a.k_new == nullptr) return;
-  const int pos = a.seqlens[b];
   if (pos < k0 || pos >= k1) return;               // the same for the whole workgroup; k1 <= S
   if (threadIdx.x < DH / 2) append_pair<DT>(a, DH / 2, b, hk, pos, threadIdx.x);
   wait_stores_acked();
@@ -108,26 +121,26 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
   __shared__ float red[2][4];
   __shared__ int last_flag;
 
-  int b, h, s;
-  decode_work_item<DH>(a.B, a.H, a.nsplit, b, h, s);
+  int b, h, s, len;
+  decode_work_item<DH>(a.seqlens, a.B, a.H, b, h, s, len);
   const int tid = threadIdx.x;
   const int hk = h / (a.H / a.Hk);
-  int n_keys = a.seqlens[b] + a.seqlen_add;
+  int n_keys = len + a.seqlen_add;
   n_keys = max(0, min(n_keys, a.S));
-  const int ranges = key_ranges<1>(a, n_keys);
+  const int ranges = key_ranges<DH, 1>(a, n_keys);
   if (s >= ranges) return;
   int per = (n_keys + ranges - 1) / ranges;
   per = (per + KPB - 1) / KPB * KPB;
   const int k0 = min(s * per, n_keys);
   const int k1 = min(n_keys, k0 + per);
-  append_own_row<DT, DH>(a, b, hk, k0, k1);
+  append_own_row<DT, DH>(a, b, hk, len, k0, k1);
 
   // query chunk (optionally rotated at position seqlens[b], fp32 math, one rounding)
   const uint16_t* qp = a.q + (int64_t)b * a.sq_b + (int64_t)h * a.sq_h;
   if (tid < DH / 2) {
     float x0 = E::val(qp[tid]), x1 = E::val(qp[tid + DH / 2]);
     if (a.cos) {
-      const int tp = min(max(a.seqlens[b], 0), a.rope_len - 1);
+      const int tp = min(max(len, 0), a.rope_len - 1);
       const float c = E::val(a.cos[(int64_t)tp * (DH / 2) + tid]);
       const float sn = E::val(a.sin[(int64_t)tp * (DH / 2) + tid]);
       const float r0 = x0 * c - x1 * sn, r1 = x0 * sn + x1 * c;
@@ -280,26 +293,26 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_gqa_kernel(AttnDecod
   __shared__ float red[2][4][G], sums[4][G];
   __shared__ int last_flag;
 
-  int b, hg, s;
-  decode_work_item<DH>(a.B, a.H / G, a.nsplit, b, hg, s);
+  int b, hg, s, len;
+  decode_work_item<DH>(a.seqlens, a.B, a.H / G, b, hg, s, len);
   const int tid = threadIdx.x;
   const int h0 = hg * G, hk = h0 / (a.H / a.Hk);
-  int n_keys = a.seqlens[b] + a.seqlen_add;
+  int n_keys = len + a.seqlen_add;
   n_keys = max(0, min(n_keys, a.S));
-  const int ranges = key_ranges<G>(a, n_keys);
+  const int ranges = key_ranges<DH, G>(a, n_keys);
   if (s >= ranges) return;
   int per = (n_keys + ranges - 1) / ranges;
   per = (per + KPB - 1) / KPB * KPB;
   const int k0 = min(s * per, n_keys);
   const int k1 = min(n_keys, k0 + per);
-  append_own_row<DT, DH>(a, b, hk, k0, k1);
+  append_own_row<DT, DH>(a, b, hk, len, k0, k1);
 
   if (tid < G * (DH / 2)) {
     const int g = tid / (DH / 2), d = tid % (DH / 2);
     const uint16_t* qp = a.q + (int64_t)b * a.sq_b + (int64_t)(h0 + g) * a.sq_h;
     float x0 = E::val(qp[d]), x1 = E::val(qp[d + DH / 2]);
     if (a.cos) {
-      const int tp = min(max(a.seqlens[b], 0), a.rope_len - 1);
+      const int tp = min(max(len, 0), a.rope_len - 1);
       const float c = E::val(a.cos[(int64_t)tp * (DH / 2) + d]);
       const float sn = E::val(a.sin[(int64_t)tp * (DH / 2) + d]);
       const float r0 = x0 * c - x1 * sn, r1 = x0 * sn + x1 * c;
