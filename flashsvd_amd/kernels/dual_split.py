@@ -120,9 +120,10 @@ def _run_fast(p_up_2d, p_gate_2d, GateU, UpU, DownV, DownU, b2):
     from .. import hip_ops
     from ._common import linear_layout_of
     # inside the operator flashsvd_hip::mlp_dual_split: its launches are issued by one native call, the coefficients taken where
-    # they are (separate tensors, adjacent views of a packed one in either order); rows of different strides, and rows off the
-    # 16-byte grid of the kernels, are copied
-    if p_up_2d.stride(0) != p_gate_2d.stride(0) or p_up_2d.stride(0) % 8 or (p_up_2d.data_ptr() | p_gate_2d.data_ptr()) % 16:
+    # they are (separate tensors, adjacent views of a packed one in either order); rows of different strides, rows that overlap (an
+    # expanded row among them), and rows off the 16-byte grid of the kernels, are copied
+    ld = p_up_2d.stride(0)
+    if ld != p_gate_2d.stride(0) or ld < p_up_2d.shape[1] or ld % 8 or (p_up_2d.data_ptr() | p_gate_2d.data_ptr()) % 16:
         p_up_2d, p_gate_2d = (t.clone(memory_format=torch.contiguous_format) for t in (p_up_2d, p_gate_2d))
     # h = round(silu(g32) * u32), dual_split_triton.py:207; S: fp32 sum over D, one rounding (:719-720)
     return hip_ops._mlp_from_coefficients(p_gate_2d, p_up_2d, linear_layout_of(GateU), linear_layout_of(UpU), linear_layout_of(DownV),

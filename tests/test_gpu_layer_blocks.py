@@ -76,3 +76,15 @@ def test_refusals():
              o_u=_rand(64, 16, seed=3))
     with pytest.raises((ValueError, RuntimeError)):                        # past the end of the cache
         ops.lowrank_attn_prefill(_rand(1, 16, 64, seed=1), **w, k_cache=k, v_cache=k.clone(), cos=cs, sin=cs, start=5, num_heads=1, num_kv_heads=1)
+
+
+def test_dual_split_operator_takes_rows_of_any_stride():
+    """The operator's coefficient rows may be one row expanded, overlap, or start off the 16-byte grid."""
+    T, R, D, N = 5, 64, 128, 96
+    w = [_rand(*s, std=s[0] ** -0.5, seed=i) for i, s in enumerate(((R, D), (R, D), (D, R), (R, N)))]
+    base = _rand(T * (R + 8) + 8, seed=9)
+    from flashsvd_amd.torch_ops import ops as registered
+    for size, start in ((0, 0), (8, 0), (R, 1), (R + 3, 0), (R + 8, 8)):
+        pu, pg = base.as_strided((T, R), (size, 1), start), base.flip(0).as_strided((T, R), (size, 1), start)
+        got, want = (registered.mlp_dual_split(u, g, *w, None, 2, 64, True, None) for u, g in ((pu, pg), (pu.clone(memory_format=torch.contiguous_format), pg.clone(memory_format=torch.contiguous_format))))
+        assert torch.equal(got, want)
