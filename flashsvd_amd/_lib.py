@@ -155,6 +155,8 @@ SIGNATURES = {
     "fsvd_attn_decode_rankkv_scores_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),
     "fsvd_rankkv_append": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p,
                                    c_int, c_int, c_int, c_int, c_void_p]),
+    "fsvd_rankkv_fill": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_int, c_int,
+                                 c_int, c_int, c_int, c_int, c_void_p]),
     "fsvd_lowrank_expand_heads": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int,
                                           c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_int, c_int, c_int, c_int, c_int,
                                           c_int, c_int, c_void_p]),

@@ -129,6 +129,8 @@ struct RankDecodeArgs {
 };
 size_t rank_decode_scores_floats(int B, int H, int S, int64_t spv_h);
 int launch_rank_decode(const RankDecodeArgs& a, hipStream_t st);
+int launch_rankkv_fill(const uint16_t* pk, int64_t spk_r, const uint16_t* pv, int64_t spv_r, uint16_t* pkc, int64_t spk_b, int64_t spk_s, uint16_t* pvc,
+                       int64_t spv_b, int64_t spv_s, int start, int B, int T, int Rk, int Rv, hipStream_t st);
 int launch_rankkv_append(const uint16_t* pk, int64_t ldpk, const uint16_t* pv, int64_t ldpv, uint16_t* pkc, int64_t spk_b, int64_t spk_s,
                          uint16_t* pvc, int64_t spv_b, int64_t spv_s, const int32_t* positions, int B, int S, int Rk, int Rv, hipStream_t st);
 

@@ -166,6 +166,40 @@ def _rankkv_append_impl(pk, pv, pk_cache, pv_cache, positions):
     check("fsvd_rankkv_append", rc)
 
 
+def rankkv_fill(p: torch.Tensor, pk_cache: torch.Tensor, pv_cache: torch.Tensor, start: int) -> None:
+    """pk_cache[:B, start:start + T] and pv_cache[:B, start:start + T] from the last Rk + Rv columns of the packed coefficients p
+    [B, T, R*] (FlashSVDLegacySparseKVCache.update, runtime/cache/attn_legacy_sparse_kv.py:113-169).  Rows and caches of one 16-bit
+    type on the 16-byte grid take one launch (custom operator flashsvd_hip::rankkv_fill), others two copies."""
+    B, T, w = p.shape
+    rk, rv = pk_cache.shape[2], pv_cache.shape[2]
+    grid = w | rk | rv | pk_cache.stride(0) | pk_cache.stride(1) | pv_cache.stride(0) | pv_cache.stride(1)
+    if B * T and p.is_contiguous() and p.dtype in (torch.bfloat16, torch.float16) and p.dtype == pk_cache.dtype == pv_cache.dtype and grid % 8 == 0 \
+            and pk_cache.stride(2) == pv_cache.stride(2) == 1 and pk_cache.stride(1) >= rk and pv_cache.stride(1) >= rv \
+            and p.device == pk_cache.device == pv_cache.device and (p.data_ptr() | pk_cache.data_ptr() | pv_cache.data_ptr()) % 16 == 0:
+        _OPS.rankkv_fill.default(p, pk_cache, pv_cache, int(start))
+        return
+    pk_cache[:B, start:start + T] = p[..., w - rk - rv:w - rv]
+    pv_cache[:B, start:start + T] = p[..., w - rv:]
+
+
+def _rankkv_fill_impl(p, pk_cache, pv_cache, start):
+    for t, nm in ((p, "p"), (pk_cache, "pk_cache"), (pv_cache, "pv_cache")):
+        if not t.is_cuda or t.dtype not in (torch.bfloat16, torch.float16) or t.dtype != p.dtype or t.device != p.device:
+            raise ValueError(f"{nm} must be a bfloat16 or float16 GPU tensor of the rows' type and device")
+        if t.dim() != 3 or t.stride(2) != 1:
+            raise ValueError(f"{nm} must have three axes, the last with unit stride")
+    if not p.is_contiguous():
+        raise ValueError("p must be contiguous")
+    B, T, w = p.shape
+    rk, rv, S = pk_cache.shape[2], pv_cache.shape[2], pk_cache.shape[1]
+    if rk + rv > w or pk_cache.shape[0] < B or pv_cache.shape[0] < B or pv_cache.shape[1] != S:
+        raise ValueError(f"shapes do not agree: p {tuple(p.shape)} caches {tuple(pk_cache.shape)} / {tuple(pv_cache.shape)}")
+    base = p.data_ptr()
+    rc = _lib.load().fsvd_rankkv_fill(base + 2 * (w - rk - rv), w, base + 2 * (w - rv), w, pk_cache.data_ptr(), pk_cache.stride(0), pk_cache.stride(1),
+                                      pv_cache.data_ptr(), pv_cache.stride(0), pv_cache.stride(1), int(start), B, T, S, rk, rv, stream())
+    check("fsvd_rankkv_fill", rc)
+
+
 def flashsvd_attn_decode_packed(factors: DecodePackedFactors, cos_half: Optional[torch.Tensor], sin_half: Optional[torch.Tensor], *,
                                 seqlen_k: Optional[int] = None, causal: bool = True, split_k: int = 512, bn: int = 64,
                                 br: int = 64, num_warps_stage1: int = 4, num_stages_stage1: int = 2, num_warps_stage2: int = 4,
@@ -201,4 +235,4 @@ def flashsvd_attn_decode_packed(factors: DecodePackedFactors, cos_half: Optional
 
 flashsvd_attn_decode_packed_v1 = flashsvd_attn_decode_packed
 
-__all__ = ["DecodePackedFactors", "flashsvd_attn_decode_packed", "flashsvd_attn_decode_packed_v1", "rank_decode", "rankkv_append"]
+__all__ = ["DecodePackedFactors", "flashsvd_attn_decode_packed", "flashsvd_attn_decode_packed_v1", "rank_decode", "rankkv_append", "rankkv_fill"]

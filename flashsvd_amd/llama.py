@@ -458,7 +458,7 @@ def _prefill_tokens_rank(self, x, cache, cache_position=None, *, norm_weight=Non
     (kernels/attn/prefill/rope_sdpa.py:133-199).  Other shapes (or FLASHSVD_AMD_PREFILL=decode) use the decode kernel:
     the tokens of a sequence are its batch rows bound to one cache row (batch stride 0) with key counts start+t+1, K
     tiles rebuilt per query — short prompts only."""
-    from .kernels.rank_decode import rank_decode
+    from .kernels.rank_decode import rank_decode, rankkv_fill
     from .quant import is_quantized
     if is_quantized(*self._factor_modules()):
         raise NotImplementedError("the rank-space cache reads bf16 head bases; int4 factors decode through the dense cache")
@@ -472,8 +472,7 @@ def _prefill_tokens_rank(self, x, cache, cache_position=None, *, norm_weight=Non
     pkc, pvc = cache.key_cache[self.layer_idx], cache.value_cache[self.layer_idx]
     rope = cache.get_rope_tables(seqlen=cache.max_cache_len, head_dim=Dh, device=x.device, dtype=x.dtype)
     p = hip_ops.linear(x, self._packed_qkv_v, norm_weight=norm_weight, eps=eps)           # [B,T,R*]
-    pkc[:B, start:start + T] = p[..., rq:rq + rk]
-    pvc[:B, start:start + T] = p[..., rq + rk:]
+    rankkv_fill(p, pkc, pvc, start)
     cache._layer_initialized[self.layer_idx] = True
     cache._note_seen(self.layer_idx, T, cache_position)
     a = torch.empty(B, T, H * Dh, device=x.device, dtype=x.dtype)
@@ -488,8 +487,7 @@ def _prefill_tokens_rank(self, x, cache, cache_position=None, *, norm_weight=Non
         q = torch.empty(B, T, gk * G, Dh, device=x.device, dtype=x.dtype)
         kt = torch.empty(B, n_ctx, gk, Dh, device=x.device, dtype=x.dtype)
         vt = torch.empty_like(kt)
-        zero = torch.zeros(B, device=x.device, dtype=torch.int32)
-        pos_q = torch.full((B,), start, device=x.device, dtype=torch.int32)
+        pos_q = torch.full((B,), start, device=x.device, dtype=torch.int32) if start else None      # None: position 0
         wq, wk, wv = self.q_u_proj.weight, self.k_u_proj.weight, self.v_u_proj.weight
         av = a.view(B, T, H, Dh)
         for k0 in range(0, Hk, gk):
@@ -502,13 +500,13 @@ def _prefill_tokens_rank(self, x, cache, cache_position=None, *, norm_weight=Non
                     [dict(p=p[..., :rq], u=wqg, num_heads=nq, out=qg, rotate=True),
                      dict(p=p[..., rq:rq + rk], u=wkg, num_heads=nk, out=kg, rotate=True),
                      dict(p=p[..., rq + rk:], u=wvg, num_heads=nk, out=vg)],
-                    head_dim=Dh, cos=rope[0], sin=rope[1], positions=zero)
+                    head_dim=Dh, cos=rope[0], sin=rope[1])
             else:
                 hip_ops.lowrank_expand_heads(p[..., :rq], wqg, num_heads=nq, head_dim=Dh, out=qg, cos=rope[0], sin=rope[1], positions=pos_q)
                 hip_ops.lowrank_expand_heads_multi(
                     [dict(p=pkc[:B, :n_ctx], u=wkg, num_heads=nk, out=kg, rotate=True),
                      dict(p=pvc[:B, :n_ctx], u=wvg, num_heads=nk, out=vg)],
-                    head_dim=Dh, cos=rope[0], sin=rope[1], positions=zero)
+                    head_dim=Dh, cos=rope[0], sin=rope[1])
             hip_ops.attn_prefill(qg, kg, vg, q_pos0=pos_q, causal=True, out=av[:, :, k0 * G:k1 * G])
         po = hip_ops.linear(a, self.o_v_proj.weight)
         return hip_ops.linear(po, self.o_u_proj.weight, residual=residual)

@@ -16,6 +16,7 @@ tensors.  ``flashsvd_amd.hip_ops`` and the modules under ``flashsvd_amd.kernels`
   attn_decode_densekv / .out          fsvd_attn_decode_densekv(_static)   the flash_attn_with_kvcache role
   attn_decode_rankkv / .out           fsvd_attn_decode_rankkv             decode over the rank-space cache
   rankkv_append                       fsvd_rankkv_append
+  rankkv_fill                         fsvd_rankkv_fill
   lowrank_expand_heads                fsvd_lowrank_expand_heads           prompt-pass head expansion (+ RoPE)
   rope_attn_prefill / .out            fsvd_attn_prefill                   causal prompt attention
   reconstruct_qkv_token               fsvd_reconstruct_qkv_token          reference-layout current-token q / k / v
@@ -232,6 +233,14 @@ _define("rankkv_append(Tensor pk, Tensor pv, Tensor(a!) pk_cache, Tensor(b!) pv_
         lambda *a, **k: None)
 
 
+def _rankkv_fill(p, pk_cache, pv_cache, start):
+    from .kernels import rank_decode as RD
+    RD._rankkv_fill_impl(p, pk_cache, pv_cache, start)
+
+
+_define("rankkv_fill(Tensor p, Tensor(a!) pk_cache, Tensor(b!) pv_cache, int start) -> ()", _rankkv_fill, lambda *a, **k: None)
+
+
 # ------------------------------------------------------------------ prompt pass
 def _expand(p, u, num_heads, head_dim, out, cos=None, sin=None, positions=None, bias=None, dst_by_position=False, head_stride=None):
     from . import hip_ops
@@ -294,5 +303,5 @@ _define("mlp_dual_split(Tensor PUp, Tensor PGate, Tensor GateU, Tensor UpU, Tens
         PUp.new_empty((PUp.shape[0], DownU.shape[1])))
 
 ops = getattr(torch.ops, NS)
-OP_NAMES = ("linear", "swiglu_linear", "rmsnorm", "greedy_token_", "lowrank_mlp", "lowrank_attn_prefill", "rope_tables", "qkv_rope_append", "attn_decode_densekv", "attn_decode_rankkv", "rankkv_append", "linear_rankkv_append",
+OP_NAMES = ("linear", "swiglu_linear", "rmsnorm", "greedy_token_", "lowrank_mlp", "lowrank_attn_prefill", "rope_tables", "qkv_rope_append", "attn_decode_densekv", "attn_decode_rankkv", "rankkv_append", "rankkv_fill", "linear_rankkv_append",
             "lowrank_expand_heads", "rope_attn_prefill", "reconstruct_qkv_token", "xw_linear", "mlp_dual_split")

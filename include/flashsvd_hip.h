@@ -278,6 +278,12 @@ int fsvd_rankkv_append(const void* pk, int64_t ldpk, const void* pv, int64_t ldp
                        void* pk_cache, int64_t spk_b, int64_t spk_s, void* pv_cache, int64_t spv_b, int64_t spv_s,
                        const int32_t* positions, int B, int S, int Rk, int Rv, void* stream);
 
+/* The coefficients of a prompt: pk_cache[b, start + t, :] = pk[(b * T + t) * spk_r ..] and the same for pv, for all B sequences and T
+ * tokens (FlashSVDLegacySparseKVCache.update, runtime/cache/attn_legacy_sparse_kv.py:113-169), one launch.  16-bit patterns;
+ * start + T <= S, the caches' rows; ranks multiples of 8; pointers and strides 16-byte aligned. */
+int fsvd_rankkv_fill(const void* pk, int64_t spk_r, const void* pv, int64_t spv_r, void* pk_cache, int64_t spk_b, int64_t spk_s,
+                     void* pv_cache, int64_t spv_b, int64_t spv_s, int start, int B, int T, int S, int Rk, int Rv, void* stream);
+
 /* Full-sequence low-rank RoPE attention = the role of the fused Triton kernel flashsvd_rope_sdpa
  * (kernels/attn/prefill/rope_sdpa.py:67-248, wrapper FlashSVDRoPEAttention :254-427), as two launches:
  *

@@ -377,3 +377,24 @@ def test_decode_driver_serves_the_rank_space_cache(monkeypatch):
         lo = ref_logits[0, same].float()
         assert float(lo[ref[same]] - lo[got[same]]) <= 2e-2 * float(lo.abs().max()), f"{got} vs {ref}"
     assert same >= 3, f"{got} vs {ref}"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,T,start,rq,rk,rv", [(1, 1, 0, 8, 8, 8), (2, 17, 3, 64, 520, 256), (3, 5, 0, 40, 1664, 2048), (2, 9, 4, 6, 8, 8), (2, 9, 4, 8, 12, 4)])
+def test_rankkv_fill_matches_copies(RD, B, T, start, rq, rk, rv, dtype):
+    """Rows of one piece to several rounds of a wave, a last workgroup that is not full, rows off the grid; nothing beside them is written."""
+    S = start + T + 2
+    p = torch.randn(B, T, rq + rk + rv, device="cuda").to(dtype)
+    caches = [torch.full((B + 1, S, r), 7.0, device="cuda", dtype=dtype) for r in (rk, rv)]
+    want = [c.clone() for c in caches]
+    want[0][:B, start:start + T], want[1][:B, start:start + T] = p[..., rq:rq + rk], p[..., rq + rk:]
+    RD.rankkv_fill(p, *caches, start)
+    assert torch.equal(caches[0], want[0]) and torch.equal(caches[1], want[1])
+    if rk % 8 == 0 and rq % 8 == 0:
+        with pytest.raises((ValueError, RuntimeError)):                    # past the end of the caches
+            torch.ops.flashsvd_hip.rankkv_fill(p, *caches, start + 3)
+    wide = [torch.full((B + 1, S + 1, r + 8), 7.0, device="cuda", dtype=dtype) for r in (rk, rv)]
+    views = [w[:, 1:, :r] for w, r in zip(wide, (rk, rv))]
+    RD.rankkv_fill(p, *views, start)
+    for v, c, w in zip(views, want, wide):
+        assert torch.equal(v, c) and bool((w[:, 0] == 7).all()) and bool((w[..., v.shape[2]:] == 7).all())
