@@ -314,15 +314,14 @@ typedef struct fsvd_expand_desc {
   const void* bias;                          /* [heads*Dh] or NULL */
   void* y; int64_t sy_b, sy_m, sy_h;         /* destination [B, rows, heads, Dh] */
   int32_t heads, R;
-  int32_t rotate;                            /* cos_out / sin_out [rows, half] = cos / sin of (float)positions[row] * inv_freq[i], rounded once to `dtype`. */
-int fsvd_rope_tables(const int64_t* positions, const float* inv_freq, void* cos_out, void* sin_out, int64_t rows, int half, int dtype,
-                     void* stream);
-
-/* 1: rotate-half RoPE with the call's cos / sin */
+  int32_t rotate;                            /* 1: rotate-half RoPE with the call's cos / sin */
   int32_t dst_by_position, dst_rows, rsv0;
 } fsvd_expand_desc;
 int fsvd_lowrank_expand_heads_multi(const fsvd_expand_desc* desc, int n, const void* cos, const void* sin, int rope_len,
                                     const int32_t* positions, int B, int M, int Dh, int dtype, void* stream);
+/* cos_out / sin_out [rows, half] = cos / sin of (float)positions[row] * inv_freq[i], rounded once to `dtype`. */
+int fsvd_rope_tables(const int64_t* positions, const float* inv_freq, void* cos_out, void* sin_out, int64_t rows, int half, int dtype,
+                     void* stream);
 int fsvd_attn_prefill(const void* q, int64_t sq_b, int64_t sq_m, int64_t sq_h,
                       const void* k, const void* v, int64_t sk_b, int64_t sk_s, int64_t sk_h,
                       const int32_t* q_pos0, const uint8_t* pad_mask, int64_t spm_b,

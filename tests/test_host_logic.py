@@ -3,6 +3,7 @@ loads and exports every symbol the header declares (no kernel is launched here).
 import ctypes
 import os
 import re
+import subprocess
 from pathlib import Path
 from types import SimpleNamespace
 
@@ -28,6 +29,23 @@ def test_library_exports_every_declared_symbol():
     assert lib.fsvd_attn_decode_workspace_bytes(1, 32, 128, 8) == 256 * 1024 + 32 * 8 * 130 * 4
     assert lib.fsvd_attn_decode_workspace_bytes(0, 32, 128, 8) == 0
     assert lib.fsvd_mlp_dual_split_workspace_bytes(1, 1536, 11008, 4096, 0, 128) > 64 * 1024 + 11008 * 2 + 1536 * 4
+
+
+@pytest.mark.parametrize("compiler,std,suffix", [("gcc", "c11", ".c"), ("g++", "c++17", ".cpp")])
+def test_header_compiles_and_declares_every_entry_point(tmp_path, compiler, std, suffix):
+    """The public header by itself, as C and as C++: every entry point can be named and the structures have the sizes that are
+    passed to the library from Python."""
+    from flashsvd_amd import _lib
+    structs = {"fsvd_expand_desc": _lib.ExpandDesc, "fsvd_mlp_block": _lib.MlpBlock, "fsvd_attn_block": _lib.AttnBlock,
+               "fsvd_step_state": _lib.StepState, "fsvd_phase": _lib.Phase}
+    lines = ['#include "flashsvd_hip.h"', "typedef void (*entry)(void);"]
+    lines += [f"entry e{i} = (entry)&{name};" for i, name in enumerate(sorted(_lib.SIGNATURES))]
+    lines += [f"typedef char size_of_{c}[sizeof({c}) == {ctypes.sizeof(py)} ? 1 : -1];" for c, py in structs.items()]
+    src = tmp_path / ("use" + suffix)
+    src.write_text("\n".join(lines) + "\n")
+    r = subprocess.run([compiler, f"-std={std}", "-Wall", "-Werror", "-Wno-cast-function-type", "-fsyntax-only", f"-I{ROOT / 'include'}", str(src)],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
 
 
 def test_null_pointer_and_shape_errors_come_back_as_status_codes():
