@@ -74,13 +74,18 @@ _SPLIT_WS_OLD: dict = {}                  # device index -> replaced buffers: gr
 _SPLIT_WS_MAX = 1 << 30
 
 
+def _splitk_enabled() -> bool:
+    """``FLASHSVD_AMD_SPLITK=0``: no call gets scratch to split K in, neither the device's nor one of its own."""
+    return os.environ.get("FLASHSVD_AMD_SPLITK", "1") != "0"
+
+
 def ensure_split_workspace(device: torch.device, min_bytes: int = 0) -> bool:
     """Register, once per device, the scratch the library's K-split projections (three rows and more, K a multiple of 64 and
     rows on the 16-byte grid; others run without it) work in.  The library allocates nothing itself; this hands it 64 MiB of torch memory, or ``min_bytes`` rounded up to a power of two (up to
     1 GiB) when a caller needs more: a larger buffer then replaces the registered one (a doubling each time at least, so
     a growing demand costs a logarithmic number of replacements), and the old one is kept alive until
     ``release_split_workspace`` because graphs captured earlier hold its address.  ``FLASHSVD_AMD_SPLITK=0`` keeps the
-    library without scratch; so does a first call made under stream capture (an allocation there would belong to the
+    library without scratch (and the calls of 128 rows and more without scratch of their own); so does a first call made under stream capture (an allocation there would belong to the
     graph's pool), and a registered buffer is never replaced under capture.  Launches that use the scratch must be
     ordered on one stream per device.  Returns whether a buffer of at least ``min_bytes`` is registered."""
     idx = device.index if device.index is not None else torch.cuda.current_device()
@@ -88,7 +93,7 @@ def ensure_split_workspace(device: torch.device, min_bytes: int = 0) -> bool:
     have = _SPLIT_WS.get(idx)
     if have is not None and have.numel() >= need:
         return True
-    if os.environ.get("FLASHSVD_AMD_SPLITK", "1") == "0" or torch.cuda.is_current_stream_capturing() or need > _SPLIT_WS_MAX:
+    if not _splitk_enabled() or torch.cuda.is_current_stream_capturing() or need > _SPLIT_WS_MAX:
         return have is not None and min_bytes <= 0
     if need > _SPLIT_WS_BYTES:
         need = min(_SPLIT_WS_MAX, 1 << (need - 1).bit_length())
@@ -162,7 +167,7 @@ def _linear_impl(x, weight, bias, norm_weight, eps, residual, out, cfg):
         norm_weight = None
     wp, ldw = weight.data_ptr(), weight.stride(0)
     scratch, nbytes = None, 0
-    if B >= 128 and K >= 4096 and cfg == 0:
+    if B >= 128 and K >= 4096 and cfg == 0 and _splitk_enabled():
         nbytes = lib.fsvd_linear_scratch_bytes(xp, ldx, wp, ldw, rp, ldr, op, ldo, B, N, K)
         if nbytes:
             scratch = torch.empty(nbytes, dtype=torch.uint8, device=x.device)      # of this call and stream
@@ -640,7 +645,7 @@ def _buffers(dt, device, *counts):
 
 def _block_scratch(b, device, nbytes_of):
     """Scratch of this call and stream for the K shares of a block's projections; the tensor to keep alive."""
-    n = nbytes_of(b)
+    n = nbytes_of(b) if _splitk_enabled() else 0
     if not n:
         return None
     t = torch.empty(n, dtype=torch.uint8, device=device)

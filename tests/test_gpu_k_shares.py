@@ -1,6 +1,8 @@
 """Projections of a long K in shares over workgroups (csrc/mfma_mid.hip) at the edges of their tilings: partial row and column
 tiles, shares of unequal length, strided and odd rows, bias and residual, against the same product in fp32; and the two-stage
 ring of the head expansions at its shortest rank."""
+import os
+
 import pytest
 import torch
 
@@ -88,3 +90,37 @@ def test_blocks_hand_their_projections_scratch():
     s = ops.linear(ops.swiglu_linear(p, gu, uu, up_off=R), dv)
     assert form_taken().startswith("shares")
     assert torch.equal(ops.lowrank_mlp(x, gu_v, gu, uu, dv, du, residual=x), ops.linear(s, du, residual=x))
+
+
+def test_the_switch_keeps_every_call_unsplit():
+    """FLASHSVD_AMD_SPLITK=0 with no buffer registered: single projections and those of both blocks run in one share each."""
+    from flashsvd_amd import hip_ops as ops
+    B, K, R, D, H = 333, 4096, 1500, 8192, 64
+    x, gu_v, dv, du = _rand(B, K, seed=1), _rand(2 * R, K, std=K ** -0.5, seed=2), _rand(R, D, std=D ** -0.5, seed=5), _rand(K, R, std=R ** -0.5, seed=6)
+    gu, uu = _rand(D, R, std=R ** -0.5, seed=3), _rand(D, R, std=R ** -0.5, seed=4)
+    pg, pu = _rand(B, 1504, seed=7)[:, :R], _rand(B, 1504, seed=8)[:, :R]
+    qkv_v, ov, ou = _rand(3 * 64, K, std=K ** -0.5, seed=9), _rand(R, H * 128, std=(H * 128) ** -0.5, seed=10), _rand(K, R, std=R ** -0.5, seed=11)
+    qu, ku, vu = (_rand(H * 128, 64, std=0.125, seed=12 + i) for i in range(3))
+    cos, sin = _rand(B, 64, seed=15), _rand(B, 64, seed=16)
+    k, v = torch.zeros(1, B, H, 128, device="cuda", dtype=torch.bfloat16), torch.zeros(1, B, H, 128, device="cuda", dtype=torch.bfloat16)
+
+    def long(a, w):
+        y = ops.linear(a, w)
+        assert not form_taken().startswith("shares"), form_taken()
+        return y
+
+    os.environ["FLASHSVD_AMD_SPLITK"] = "0"
+    ops.release_split_workspace(x.device)
+    try:
+        y = long(ops.swiglu_linear(long(x, gu_v), gu, uu, up_off=R), dv)
+        assert torch.equal(ops.lowrank_mlp(x, gu_v, gu, uu, dv, du, residual=x), ops.linear(y, du, residual=x))
+        y = long(ops.swiglu_linear(torch.cat([pg, pu], 1), gu, uu, up_off=R, mode=1), dv)
+        assert torch.equal(ops._mlp_from_coefficients(pg, pu, gu, uu, dv, du, None, 1), ops.linear(y, du))
+        got = ops.lowrank_attn_prefill(x[None], qkv_v, qu, ku, vu, ov, ou, k, v, cos, sin, start=0, num_heads=H, num_kv_heads=H)
+        p = long(x, qkv_v)
+        q = ops.lowrank_expand_heads(p[None, :, :64], qu, num_heads=H, head_dim=128, out=torch.empty_like(k), cos=cos, sin=sin)
+        a = ops.attn_prefill(q, k, v, causal=True)
+        assert torch.equal(got[0], ops.linear(long(a.view(B, -1), ov), ou))
+    finally:
+        del os.environ["FLASHSVD_AMD_SPLITK"]
+        assert ops.ensure_split_workspace(x.device)
