@@ -7,6 +7,7 @@
 // with write-through stores; the last workgroup to arrive for a (b,h) merges the partials in
 // split order, so the result does not depend on arrival order.
 #include "common.hpp"
+#include "decode_map.hpp"
 #include "kernels.hpp"
 
 namespace fsvd {
@@ -14,59 +15,25 @@ namespace fsvd {
 constexpr int kAttnThreads = 256;
 constexpr int kMaxKeysPerSplit = 1 << 20;  // the key loop is streamed; only a sanity bound
 
-// Workgroup -> key range s of query head (or head group) h of sequence b, len = seqlens[b].  Consecutive workgroup ids go
-// round-robin over the 8 XCDs: the ranges of one head (which meet again in the merge) run on the same XCD, the first range of all
-// its heads before the second of any, so that workgroups without a range, which leave at once, are the last ones (between the
-// others they left the compute units unevenly loaded: 16 x 1000 keys 93 us).
-// Up to 64 sequences with head_dim 128, 1024 pairs (four per compute unit; beyond, the order of dispatch evens things out, and
-// 48 x 500 keys of 32 heads are 68 us this way, 71 the other): an XCD takes some heads of every sequence, not every head of some, the
-// sequences longest first, and every other 32 workgroups of an XCD (one per compute unit) in reverse, so that the ranges of a
-// long and of a short sequence share a compute unit.  Without -> with, 32 heads: 16 x 1 to 1000 keys 31.4 -> 27.0 us, 32 x 1 to
-// 1000 55.6 -> 46.2, 16 x 4000 175.6 -> 171.2; 64 x 1 to 1000, four heads a group, 42.7 -> 32.8.  With head_dim 64 the pieces of
-// a row that an XCD then reads are too small (64 x 1000 keys 98.7 -> 105).
+// The range, head (or head group) and sequence of this workgroup (decode_map.hpp), len = seqlens[b].
 template <int DH>
 __device__ __forceinline__ void decode_work_item(const int32_t* seqlens, int B, int H, int& b, int& h, int& s, int& len) {
-  const int pairs = B * H;
-  const bool by_xcd = (pairs & 7) == 0;
-  const int per = by_xcd ? pairs >> 3 : pairs, xcd = by_xcd ? blockIdx.x & 7 : 0;
-  int id = by_xcd ? blockIdx.x >> 3 : blockIdx.x;
-  if (DH == 128 && (H & 7) == 0 && B <= 64 && pairs <= 1024) {
-    if ((id & 32) && (id | 31) < (int)(gridDim.x >> 3)) id ^= 31;
-    s = id / per;
-    id -= s * per;
-    const int heads = H >> 3, lane = threadIdx.x & 63;
-    h = xcd * heads + id % heads;
-    const int n = seqlens[min(lane, B - 1)];
+  const DecodeSlot slot = decode_slot(DH, blockIdx.x, gridDim.x, B, H);
+  s = slot.s;
+  h = slot.h;
+  if (decode_by_length(DH, B, H)) {
+    const int lane = threadIdx.x & 63, n = seqlens[min(lane, B - 1)];
     int rank = 0;                     // of this lane's sequence, longest first
     for (int u = 0; u < B; ++u) {
       const int nu = __builtin_amdgcn_readlane(n, u);
       rank += nu > n || (nu == n && u < lane);
     }
-    b = __builtin_ctzll(__ballot(lane < B && rank == id / heads));
+    b = __builtin_ctzll(__ballot(lane < B && rank == slot.seq));
     len = __builtin_amdgcn_readlane(n, b);
   } else {
-    s = id / per;
-    const int turn = max(1, per * pairs / (int)gridDim.x);     // a range later: another compute unit
-    const int pair = xcd * per + (id - s * per + s * turn) % per;
-    h = pair % H;
-    b = pair / H;
+    b = slot.seq;
     len = seqlens[b];
   }
-}
-
-// Key ranges that a sequence of n keys is cut into, at most nsplit (what the scratch holds): known from the length alone, so
-// the same launch serves a cache that is nearly empty and one that is full; the other workgroups of (b, h) leave at once.
-// A range holds at least one pass of 128 keys.  Where the heads of all sequences fill the chip by themselves (one query head per
-// workgroup, 256 pairs and more) ranges only even out sequences of different lengths: from 2 keys a pair on (one with head_dim 64,
-// whose sequences stay on one XCD), and an odd count (the starts of two or four equal ranges lie a power of two apart, and
-// their workgroups ask the same memory channels at the same time).  Both sides with 32 heads: 16 x 1000 keys 55.1 us in four
-// ranges, 46.9 in one (in a cache of 1024 rows 67.2, 48.9), 32 x 1000 95.6 and 88.4, 16 x 750 to 1000 47.7 and 42.7; one sequence
-// of 300 keys in a cache of 4096 rows 13.0 in 32, 6.6 in three.
-template <int DH, int G>
-__device__ __forceinline__ int key_ranges(const AttnDecodeArgs& a, int n_keys) {
-  int n = min(a.nsplit, (n_keys + 127) >> 7);
-  if (G == 1 && a.B * a.H >= 256) n = min(n, (n_keys / (DH / 64 * a.B * a.H)) | 1);
-  return max(1, n);
 }
 
 // coherent (L2-bypassing) scalar accessors for the cross-workgroup partials: the producers write
@@ -127,7 +94,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
   const int hk = h / (a.H / a.Hk);
   int n_keys = len + a.seqlen_add;
   n_keys = max(0, min(n_keys, a.S));
-  const int ranges = key_ranges<DH, 1>(a, n_keys);
+  const int ranges = decode_ranges(DH, 1, a.B, a.H, a.nsplit, n_keys);
   if (s >= ranges) return;
   int per = (n_keys + ranges - 1) / ranges;
   per = (per + KPB - 1) / KPB * KPB;
@@ -301,7 +268,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_gqa_kernel(AttnDecod
   const int h0 = hg * G, hk = h0 / (a.H / a.Hk);
   int n_keys = len + a.seqlen_add;
   n_keys = max(0, min(n_keys, a.S));
-  const int ranges = key_ranges<DH, G>(a, n_keys);
+  const int ranges = decode_ranges(DH, G, a.B, a.H, a.nsplit, n_keys);
   if (s >= ranges) return;
   int per = (n_keys + ranges - 1) / ranges;
   per = (per + KPB - 1) / KPB * KPB;

@@ -19,7 +19,8 @@ def _reference(q, kc, vc, n):
 @pytest.mark.parametrize("B,H,Hk,Dh,nsplit,lens", [
     (1, 8, 8, 128, 40, (128,)), (1, 8, 8, 128, 40, (129,)), (2, 5, 5, 64, 7, (255, 700)), (3, 8, 2, 128, 5, (0, 1, 641)),  # one pass and more
     (8, 32, 32, 128, 8, (511, 512, 1023, 1024, 1535, 1536, 0, 1)), (8, 32, 32, 64, 2, (1024, 1100, 30)),                 # from 2 keys a pair
-    (17, 16, 16, 128, 3, (1087, 1088, 64)), (64, 16, 16, 128, 2, (9, 300, 300, 17, 140)), (65, 8, 8, 128, 2, (300, 17)), (33, 9, 9, 64, 3, (593, 594, 595)),                                         # odd batches and heads
+    (17, 16, 16, 128, 3, (1087, 1088, 64)), (64, 16, 16, 128, 2, (9, 300, 300, 17, 140)), (65, 8, 8, 128, 2, (300, 17)), (33, 9, 9, 64, 3, (593, 594, 595)),
+    (48, 32, 32, 128, 2, (300, 17, 129)), (4, 12, 12, 128, 3, (300, 40)),                                                   # odd batches and heads, more than 1024 pairs
     (64, 32, 8, 64, 1, (1, 31, 32, 127, 128, 129, 0, 300)), (16, 32, 8, 64, 4, (511, 512, 513, 40, 0)), (4, 64, 8, 64, 9, (3, 1160))])  # groups of 64
 def test_ranges_follow_the_length(dtype, B, H, Hk, Dh, nsplit, lens):
     from flashsvd_amd import hip_ops as ops
@@ -32,30 +33,8 @@ def test_ranges_follow_the_length(dtype, B, H, Hk, Dh, nsplit, lens):
     other = ops.attn_decode_densekv(qd, kd, vd, nd.flip(0), nsplit=nsplit, workspace=ws)        # other ranges over the same scratch
     assert torch.equal(out, ops.attn_decode_densekv(qd, kd, vd, nd, nsplit=nsplit, workspace=ws))
     for got, length in ((out, n), (other, n.flip(0))):
-        for b in {*range(min(B, 8)), B - 1}:
+        for b in range(B):
             if int(length[b]):
                 assert_close_bf16(got[b], _reference(q[b], kc[b], vc[b], int(length[b])), f"sequence {b}, {int(length[b])} keys")
             else:
                 assert torch.all(got[b] == 0)
-
-
-def test_every_range_has_one_workgroup():
-    """The assignment of workgroups, as the kernel computes it, covers (sequence, head, range) once."""
-    for B, H, Dh, nsplit in [(1, 8, 128, 32), (16, 8, 128, 4), (8, 32, 128, 8), (3, 5, 64, 7), (8, 12, 64, 3), (2, 12, 128, 5), (1, 1, 64, 9),
-                             (7, 16, 128, 9), (64, 16, 128, 2), (48, 32, 128, 1), (5, 24, 128, 3)]:
-        pairs = B * H
-        xcds = 8 if pairs % 8 == 0 else 1
-        per, seen, blocks = pairs // xcds, set(), pairs * nsplit
-        by_length = sorted(range(B), key=lambda b: (-(b * 7 % 5), b))
-        for block in range(blocks):
-            xcd, i = block % xcds, block // xcds
-            if Dh == 128 and H % 8 == 0 and B <= 64 and pairs <= 1024:
-                if i & 32 and (i | 31) < blocks // 8:
-                    i ^= 31
-                s, i = divmod(i, per)
-                seen.add((by_length[i // (H // 8)], xcd * (H // 8) + i % (H // 8), s))
-            else:
-                s, i = divmod(i, per)
-                pair = xcd * per + (i + s * max(1, per * pairs // blocks)) % per
-                seen.add((pair // H, pair % H, s))
-        assert seen == {(b, h, s) for b in range(B) for h in range(H) for s in range(nsplit)}
