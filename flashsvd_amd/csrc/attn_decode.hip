@@ -17,8 +17,8 @@ constexpr int kMaxKeysPerSplit = 1 << 20;  // the key loop is streamed; only a s
 
 // The range, head (or head group) and sequence of this workgroup (decode_map.hpp), len = seqlens[b].
 template <int DH>
-__device__ __forceinline__ void decode_work_item(const int32_t* seqlens, int B, int H, int& b, int& h, int& s, int& len) {
-  const DecodeSlot slot = decode_slot(DH, blockIdx.x, gridDim.x, B, H);
+__device__ __forceinline__ void decode_work_item(const int32_t* seqlens, int B, int H, int nsplit, int& b, int& h, int& s, int& len) {
+  const DecodeSlot slot = decode_slot(DH, blockIdx.x, B, H, nsplit);
   s = slot.s;
   h = slot.h;
   if (decode_by_length(DH, B, H)) {
@@ -89,7 +89,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
   __shared__ int last_flag;
 
   int b, h, s, len;
-  decode_work_item<DH>(a.seqlens, a.B, a.H, b, h, s, len);
+  decode_work_item<DH>(a.seqlens, a.B, a.H, a.nsplit, b, h, s, len);
   const int tid = threadIdx.x;
   const int hk = h / (a.H / a.Hk);
   int n_keys = len + a.seqlen_add;
@@ -263,7 +263,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_gqa_kernel(AttnDecod
   __shared__ int last_flag;
 
   int b, hg, s, len;
-  decode_work_item<DH>(a.seqlens, a.B, a.H / G, b, hg, s, len);
+  decode_work_item<DH>(a.seqlens, a.B, a.H / G, a.nsplit, b, hg, s, len);
   const int tid = threadIdx.x;
   const int h0 = hg * G, hk = h0 / (a.H / a.Hk);
   int n_keys = len + a.seqlen_add;

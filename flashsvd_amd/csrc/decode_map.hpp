@@ -8,7 +8,7 @@ namespace fsvd {
 // the batch, longest first (equal lengths in their order).
 struct DecodeSlot { int s, h, seq; };
 
-// Workgroup `block` of `blocks` = B * H * (ranges at most); H counts the head groups where a workgroup takes a group.
+// Workgroup `block` of B * H * nsplit; H counts the head groups where a workgroup takes a group.
 // Consecutive workgroup ids go round-robin over the 8 XCDs: the ranges of one head (which meet again in the merge) run on the same
 // XCD, the first range of all its heads before the second of any, so that workgroups without a range, which leave at once, are the
 // last ones (between the others they left the compute units unevenly loaded: 16 x 1000 keys 93 us).
@@ -20,18 +20,18 @@ struct DecodeSlot { int s, h, seq; };
 // a row that an XCD then reads are too small (64 x 1000 keys 98.7 -> 105).
 constexpr bool decode_by_length(int head_dim, int B, int H) { return head_dim == 128 && H % 8 == 0 && B <= 64 && B * H <= 1024; }
 
-constexpr DecodeSlot decode_slot(int head_dim, int block, int blocks, int B, int H) {
+constexpr DecodeSlot decode_slot(int head_dim, int block, int B, int H, int nsplit) {
   const int pairs = B * H;
   const bool by_xcd = pairs % 8 == 0;
   const int per = by_xcd ? pairs >> 3 : pairs, xcd = by_xcd ? block & 7 : 0;
   int id = by_xcd ? block >> 3 : block;
   if (decode_by_length(head_dim, B, H)) {
-    if ((id & 32) && (id | 31) < (blocks >> 3)) id ^= 31;
+    if ((id & 32) && (id | 31) < per * nsplit) id ^= 31;
     const int s = id / per, heads = H >> 3;
     id -= s * per;
     return DecodeSlot{s, xcd * heads + id % heads, id / heads};
   }
-  const int s = id / per, share = per * pairs / blocks, turn = share > 1 ? share : 1;     // a range later: another compute unit
+  const int s = id / per, share = per / nsplit, turn = share > 1 ? share : 1;     // a range later: another compute unit
   const int pair = xcd * per + (id - s * per + s * turn) % per;
   return DecodeSlot{s, pair % H, pair / H};
 }
