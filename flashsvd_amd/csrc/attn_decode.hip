@@ -18,19 +18,22 @@ constexpr int kMaxKeysPerSplit = 1 << 20;  // the key loop is streamed; only a s
 // The range, head (or head group) and sequence of this workgroup (decode_map.hpp), len = seqlens[b].
 template <int DH>
 __device__ __forceinline__ void decode_work_item(const int32_t* seqlens, int B, int H, int nsplit, int& b, int& h, int& s, int& len) {
-  const DecodeSlot slot = decode_slot(DH, blockIdx.x, B, H, nsplit);
-  s = slot.s;
-  h = slot.h;
   if (decode_by_length(DH, B, H)) {
-    const int lane = threadIdx.x & 63, n = seqlens[min(lane, B - 1)];
+    const int lane = threadIdx.x & 63, n = seqlens[min(lane, B - 1)];     // on its way during the divisions
+    const DecodeSlot slot = decode_slot_by_length(blockIdx.x, B, H, nsplit);
     int rank = 0;                     // of this lane's sequence, longest first
     for (int u = 0; u < B; ++u) {
       const int nu = __builtin_amdgcn_readlane(n, u);
       rank += nu > n || (nu == n && u < lane);
     }
+    s = slot.s;
+    h = slot.h;
     b = __builtin_ctzll(__ballot(lane < B && rank == slot.seq));
     len = __builtin_amdgcn_readlane(n, b);
   } else {
+    const DecodeSlot slot = decode_slot_by_pair(blockIdx.x, B, H, nsplit);
+    s = slot.s;
+    h = slot.h;
     b = slot.seq;
     len = seqlens[b];
   }

@@ -20,17 +20,20 @@ struct DecodeSlot { int s, h, seq; };
 // a row that an XCD then reads are too small (64 x 1000 keys 98.7 -> 105).
 constexpr bool decode_by_length(int head_dim, int B, int H) { return head_dim == 128 && H % 8 == 0 && B <= 64 && B * H <= 1024; }
 
-constexpr DecodeSlot decode_slot(int head_dim, int block, int B, int H, int nsplit) {
+// (pairs that are a multiple of 8, as H is)
+constexpr DecodeSlot decode_slot_by_length(int block, int B, int H, int nsplit) {
+  const int per = (B * H) >> 3, heads = H >> 3;
+  int id = block >> 3;
+  if ((id & 32) && (id | 31) < per * nsplit) id ^= 31;
+  const int s = id / per;
+  id -= s * per;
+  return DecodeSlot{s, (block & 7) * heads + id % heads, id / heads};
+}
+
+constexpr DecodeSlot decode_slot_by_pair(int block, int B, int H, int nsplit) {
   const int pairs = B * H;
-  const bool by_xcd = pairs % 8 == 0;
-  const int per = by_xcd ? pairs >> 3 : pairs, xcd = by_xcd ? block & 7 : 0;
-  int id = by_xcd ? block >> 3 : block;
-  if (decode_by_length(head_dim, B, H)) {
-    if ((id & 32) && (id | 31) < per * nsplit) id ^= 31;
-    const int s = id / per, heads = H >> 3;
-    id -= s * per;
-    return DecodeSlot{s, xcd * heads + id % heads, id / heads};
-  }
+  const bool by_xcd = (pairs & 7) == 0;
+  const int per = by_xcd ? pairs >> 3 : pairs, xcd = by_xcd ? block & 7 : 0, id = by_xcd ? block >> 3 : block;
   const int s = id / per, share = per / nsplit, turn = share > 1 ? share : 1;     // a range later: another compute unit
   const int pair = xcd * per + (id - s * per + s * turn) % per;
   return DecodeSlot{s, pair % H, pair / H};

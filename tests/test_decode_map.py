@@ -16,7 +16,7 @@ int main(int argc, char** argv) {
     const int dh = atoi(argv[i]), B = atoi(argv[i + 1]), H = atoi(argv[i + 2]), nsplit = atoi(argv[i + 3]), blocks = B * H * nsplit;
     std::vector<int> seen((size_t)blocks);
     for (int id = 0; id < blocks; ++id) {
-      const DecodeSlot t = decode_slot(dh, id, B, H, nsplit);
+      const DecodeSlot t = decode_by_length(dh, B, H) ? decode_slot_by_length(id, B, H, nsplit) : decode_slot_by_pair(id, B, H, nsplit);
       if (t.s < 0 || t.s >= nsplit || t.h < 0 || t.h >= H || t.seq < 0 || t.seq >= B) { printf("%d %d %d %d: workgroup %d outside\n", dh, B, H, nsplit, id); return 1; }
       if (seen[((size_t)t.seq * H + t.h) * nsplit + t.s]++) { printf("%d %d %d %d: workgroup %d takes a part twice\n", dh, B, H, nsplit, id); return 1; }
     }
@@ -54,7 +54,6 @@ def test_assignment_of_many_pairs_is_a_constant_expression(tmp_path):
         for s in range(nsplit):
             first, xcds = s * per, 8 if B * H % 8 == 0 else 1
             pair = s * max(1, per // nsplit) % per
-            for dh in (64, 128):
-                asserts.append(f"constexpr auto t{len(asserts)} = decode_slot({dh}, {first * xcds}, {B}, {H}, {nsplit});\n"
-                               f"static_assert(t{len(asserts)}.s == {s} && t{len(asserts)}.h == {pair % H} && t{len(asserts)}.seq == {pair // H});")
+            asserts.append(f"constexpr auto t{len(asserts)} = decode_slot_by_pair({first * xcds}, {B}, {H}, {nsplit});\n"
+                           f"static_assert(t{len(asserts)}.s == {s} && t{len(asserts)}.h == {pair % H} && t{len(asserts)}.seq == {pair // H});")
     _build(tmp_path, '#include "decode_map.hpp"\nusing namespace fsvd;\n' + "\n".join(asserts) + "\nint main() { return 0; }\n")
