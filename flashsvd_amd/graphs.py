@@ -99,7 +99,7 @@ class GraphedDecoder:
             raise IndexError(f"decode position {position} outside the cache (max {self.cache.max_cache_len})")
         ids = tokens.reshape(self.B, 1)
         if ids.dtype == torch.long and ids.device == self.tokens.device and ids.is_contiguous():
-            hip_ops.set_token_rows_(self.tokens, ids, self.positions, int(position))
+            hip_ops._set_token_rows_impl(self.tokens, ids, self.positions, int(position))     # host code: not through the dispatcher
         else:
             self.tokens.copy_(ids)
             self.positions.fill_(int(position))

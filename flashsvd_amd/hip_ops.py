@@ -508,10 +508,16 @@ def _greedy_token_impl(logits, tokens, positions):
 
 def set_token_rows_(tokens: torch.Tensor, src: torch.Tensor, positions: torch.Tensor, position: int) -> None:
     """``tokens.copy_(src)`` and ``positions.fill_(position)`` in one launch (contiguous int64 / int64 / int32 of the same
-    number of rows on one device)."""
+    number of rows on one device).  Custom operator flashsvd_hip::set_token_rows_ (tokens and positions are mutated arguments)."""
+    _OPS.set_token_rows_.default(tokens, src, positions, int(position))
+
+
+def _set_token_rows_impl(tokens, src, positions, position):
     _need(tokens, "tokens", dtype=torch.long)
     _need(src, "src", dtype=torch.long)
     _need(positions, "positions", dtype=torch.int32)
+    if not tokens.device == src.device == positions.device:
+        raise ValueError(f"tokens, src and positions must be on one device, got {tokens.device}, {src.device} and {positions.device}")
     if not (tokens.is_contiguous() and src.is_contiguous() and positions.is_contiguous() and tokens.numel() == src.numel() == positions.numel()):
         raise ValueError("tokens, src and positions must be contiguous and of one length")
     with torch.cuda.device(tokens.device):

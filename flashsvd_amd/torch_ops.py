@@ -12,6 +12,7 @@ tensors.  ``flashsvd_amd.hip_ops`` and the modules under ``flashsvd_amd.kernels`
   lowrank_attn_prefill                fsvd_attn_block_prefill   the attention half of a prompt pass over the dense cache
   rope_tables                         fsvd_rope_tables
   greedy_token_                       fsvd_greedy_token      argmax of every row + position increment
+  set_token_rows_                     fsvd_set_token_rows    token and position of every row
   qkv_rope_append / .out              fsvd_qkv_rope_append   head expansion + RoPE + dense-cache append
   attn_decode_densekv / .out          fsvd_attn_decode_densekv(_static)   the flash_attn_with_kvcache role
   attn_decode_rankkv / .out           fsvd_attn_decode_rankkv             decode over the rank-space cache
@@ -144,6 +145,14 @@ def _greedy_token(logits, tokens, positions=None):
 
 
 _define("greedy_token_(Tensor logits, Tensor(a!) tokens, Tensor(b!)? positions=None) -> ()", _greedy_token, lambda *a, **k: None)
+
+
+def _set_token_rows(tokens, src, positions, position):
+    from . import hip_ops
+    hip_ops._set_token_rows_impl(tokens, src, positions, position)
+
+
+_define("set_token_rows_(Tensor(a!) tokens, Tensor src, Tensor(b!) positions, int position) -> ()", _set_token_rows, lambda *a, **k: None)
 
 
 # ------------------------------------------------------------------ q / k / v expansion + RoPE + cache append
@@ -303,5 +312,5 @@ _define("mlp_dual_split(Tensor PUp, Tensor PGate, Tensor GateU, Tensor UpU, Tens
         PUp.new_empty((PUp.shape[0], DownU.shape[1])))
 
 ops = getattr(torch.ops, NS)
-OP_NAMES = ("linear", "swiglu_linear", "rmsnorm", "greedy_token_", "lowrank_mlp", "lowrank_attn_prefill", "rope_tables", "qkv_rope_append", "attn_decode_densekv", "attn_decode_rankkv", "rankkv_append", "rankkv_fill", "linear_rankkv_append",
+OP_NAMES = ("linear", "swiglu_linear", "rmsnorm", "greedy_token_", "set_token_rows_", "lowrank_mlp", "lowrank_attn_prefill", "rope_tables", "qkv_rope_append", "attn_decode_densekv", "attn_decode_rankkv", "rankkv_append", "rankkv_fill", "linear_rankkv_append",
             "lowrank_expand_heads", "rope_attn_prefill", "reconstruct_qkv_token", "xw_linear", "mlp_dual_split")

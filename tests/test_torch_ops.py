@@ -4,6 +4,8 @@ through these operators, and by torch.library.opcheck in the GPU part below."""
 import pytest
 import torch
 
+import flashsvd_amd.torch_ops  # noqa: F401  (registers the operators, whichever test runs first)
+
 BF16 = torch.bfloat16
 
 
@@ -55,6 +57,19 @@ def test_host_tensors_raise_value_error_through_the_dispatcher():
         hip_ops.linear(torch.zeros(1, 64, dtype=BF16), torch.zeros(8, 64, dtype=BF16))
     with pytest.raises(ValueError, match="GPU tensor"):
         torch.ops.flashsvd_hip.rmsnorm(torch.zeros(1, 64, dtype=BF16), torch.ones(64, dtype=BF16))
+
+
+def test_token_rows_are_an_operator_of_one_device():
+    """set_token_rows_ writes through raw addresses: it declares what it writes, and refuses tensors of another device."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from flashsvd_amd import hip_ops
+    schema = str(torch.ops.flashsvd_hip.set_token_rows_.default._schema)
+    assert "Tensor(a!) tokens" in schema and "Tensor(b!) positions" in schema
+    with FakeTensorMode():
+        on = lambda dtype, i: torch.empty(4, dtype=dtype, device=f"cuda:{i}")
+        for devices in ((0, 1, 0), (0, 0, 1), (1, 0, 0)):
+            with pytest.raises(ValueError, match="one device"):
+                hip_ops._set_token_rows_impl(*(on(dt, i) for dt, i in zip((torch.long, torch.long, torch.int32), devices)), 3)
 
 
 @pytest.mark.gpu
