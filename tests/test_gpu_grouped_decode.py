@@ -47,29 +47,32 @@ def test_grouped_decode_attention(ops, dtype, B, H, Hk, nsplit, lens):
             assert torch.all(out[b] == 0)
 
 
-def _pair_of_caches(B, S, Hk, dtype):
+def _pair_of_caches(B, S, Hk, Dh, dtype):
     """The same values with the rows of a token together (a workgroup may append its own row) and with the rows of a head
     together (the append is a launch of its own)."""
-    kc, vc = (rand_bf16(B, S, Hk, 128, seed=i).to(dtype).cuda() for i in (3, 4))
+    kc, vc = (rand_bf16(B, S, Hk, Dh, seed=i).to(dtype).cuda() for i in (3, 4))
     return (kc, vc), tuple(t.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3) for t in (kc, vc))
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("B,H,Hk,nsplit,lens", [(2, 8, 8, 1, (0, 128)), (3, 16, 16, 4, (63, 64, 300)), (16, 32, 8, 4, (0, 1, 127, 128, 511, 512, 400)),
-                                                (64, 32, 8, 1, (0, 15, 128, 255)), (16, 32, 16, 2, (31, 32, 33, 256)), (32, 16, 2, 4, (5, 64, 130)),
-                                                (1, 32, 8, 3, (47,))])
+@pytest.mark.parametrize("B,H,Hk,Dh,nsplit,lens", [(2, 8, 8, 128, 1, (0, 128)), (3, 16, 16, 128, 4, (63, 64, 300)), (16, 32, 8, 128, 4, (0, 1, 127, 128, 511, 512, 400)),
+                                                   (64, 32, 8, 128, 1, (0, 15, 128, 255)), (16, 32, 16, 128, 2, (31, 32, 33, 256)), (32, 16, 2, 128, 4, (5, 64, 130)),
+                                                   (1, 32, 8, 128, 3, (47,)),
+                                                   # four heads of 64 per workgroup, which append in the launch; eight per kv head, which do not; one
+                                                   (64, 32, 8, 64, 1, (0, 31, 32, 127, 128, 255)), (16, 32, 8, 64, 4, (0, 1, 127, 128, 256, 511, 512, 400)),
+                                                   (32, 16, 2, 64, 4, (5, 64, 130)), (3, 8, 8, 64, 2, (63, 64, 300))])
 @pytest.mark.parametrize("rotate", [True, False])
-def test_append_in_the_attention_launch(ops, dtype, B, H, Hk, nsplit, lens, rotate):
+def test_append_in_the_attention_launch(ops, dtype, B, H, Hk, Dh, nsplit, lens, rotate):
     """New rows at split and pass borders, at the first and the last row of the cache and past its end (dropped): the caches
     and results are those of an append launched before the attention, bit for bit."""
     S = max(lens) + 1
     lens = torch.tensor([lens[b % len(lens)] for b in range(B)], dtype=torch.int32)
     if B > 2:
         lens[-1] = S                                            # no room: nothing is written, all S rows are attended to
-    cos, sin = (rand_bf16(S + 1, 64, seed=i).to(dtype).cuda() for i in (6, 7)) if rotate else (None, None)
-    q, kn, vn = (rand_bf16(B, h, 128, seed=i).to(dtype).cuda() for i, h in ((0, H), (1, Hk), (2, Hk)))
+    cos, sin = (rand_bf16(S + 1, Dh // 2, seed=i).to(dtype).cuda() for i in (6, 7)) if rotate else (None, None)
+    q, kn, vn = (rand_bf16(B, h, Dh, seed=i).to(dtype).cuda() for i, h in ((0, H), (1, Hk), (2, Hk)))
     results = []
-    for kc, vc in _pair_of_caches(B, S, Hk, dtype):
+    for kc, vc in _pair_of_caches(B, S, Hk, Dh, dtype):
         for _ in range(2):                                      # a second call finds the row there already
             out = ops.attn_decode_densekv(q, kc, vc, lens.cuda(), k_new=kn, v_new=vn, cos=cos, sin=sin, nsplit=nsplit)
         results.append((out, kc, vc))
