@@ -13,7 +13,9 @@
 namespace fsvd {
 
 constexpr int kAttnThreads = 256;
-constexpr int kMaxKeysPerSplit = 1 << 20;  // the key loop is streamed; only a sanity bound
+// cache rows for each range that the caller has scratch for: a bound on what a call may ask, not on what a workgroup walks (a
+// sequence may be cut into fewer ranges than that, decode_map.hpp; the key loop is streamed)
+constexpr int kMaxRowsPerRange = 1 << 20;
 
 // The range, head (or head group) and sequence of this workgroup (decode_map.hpp), len = seqlens[b].
 template <int DH>
@@ -500,8 +502,8 @@ int launch_attn_decode(const AttnDecodeArgs& args, hipStream_t st) {
   if (a.Dh != 64 && a.Dh != 128) { set_last_error("fsvd_attn_decode_densekv: head_dim %d not in {64,128}", a.Dh); return kErrBadShape; }
   const int kpb = kAttnThreads / (a.Dh / 8);
   const int per = ((a.S + a.nsplit - 1) / a.nsplit + kpb - 1) / kpb * kpb;
-  if (per > kMaxKeysPerSplit) {
-    set_last_error("fsvd_attn_decode_densekv: %d keys per split exceeds %d; raise nsplit", per, kMaxKeysPerSplit);
+  if (per > kMaxRowsPerRange) {
+    set_last_error("fsvd_attn_decode_densekv: a cache of %d rows for %d key ranges (nsplit): at most %d rows a range", a.S, a.nsplit, kMaxRowsPerRange);
     return kErrBadShape;
   }
   if ((a.sc_s % 8) || (a.sc_h % 8) || (a.sc_b % 8) || (reinterpret_cast<uintptr_t>(a.k_cache) & 15) ||

@@ -63,6 +63,18 @@ def test_null_pointer_and_shape_errors_come_back_as_status_codes():
         _lib.check("fsvd_linear", -1)
 
 
+def test_decode_attention_names_the_bound_on_cache_rows():
+    """Rows of the cache per key range that there is scratch for, whatever a sequence is cut into."""
+    from flashsvd_amd import _lib
+    lib = _lib.load()
+    buf = ctypes.create_string_buffer(64)  # never dereferenced: the shape check fails first
+    p = ctypes.addressof(buf)
+    S = (1 << 20) + 1
+    rc = lib.fsvd_attn_decode_densekv(p, 1024, 128, p, p, S * 1024, 1024, 128, None, 0, 0, None, 0, 0, p, 0, None, None, 0, p, 1024, 128, None, 0,
+                                      1, 8, 8, 128, S, 1, 0.0, 0, None)
+    assert rc == -1 and f"a cache of {S} rows for 1 key ranges (nsplit): at most {1 << 20} rows a range".encode() in lib.fsvd_last_error()
+
+
 @pytest.mark.parametrize("tokens", [1, 16, 200])
 def test_expansions_of_one_call_refuse_other_element_types(tokens):
     """FSVD_FP32 is no type of the head expansions, whatever kernel the token count would select."""
