@@ -507,15 +507,18 @@ static MidForm mid_form(const MfmaArgs& a, bool dual) {
 // from 385 on where they pad no more rows than 128 x 128 do (768 rows of 1536 x 11008 40 us against 45), else 128 x 128 (256 rows 24
 // against 27).  us with weights from HBM, what runs otherwise -> this:
 // K of 8192 and more, always: 1536 x 11008 (64-row tiles of two stages whose last workgroup adds the shares) at 128 / 154 / 256 / 333 /
-// 512 / 768 / 1024 rows 24 -> 20, 30 -> 24, 32 -> 24, 41 -> 28, 45 -> 36, 63 -> 45, 67 -> 47 (up to 768 with the cut that the 64-row
-// tiles have: as many shares as the chip has room for took 19, 20, 23, 26, 32, 39); 1536 x 8192 at 1536 / 2048 (ring of 128 x
-// 128) 71 -> 53, 74 -> 69; 2390 x 11008 at 2048 (128 x 64 tiles; one share) 194 -> 161.
-// From 4096 on, where the ring's tiles keep the compute units less busy: `area` counts a workgroup's outputs, so
-// shares * area(ring) / area(share) is how much more of the chip works here, and adding up the shares has to come out of it.
-// 1.5 times: 128 x 4992 x 4096 22.1 -> 19.6, 333 x 3072 x 4096 25.2 -> 23.7, 768 x 3072 x 4096 38.7 -> 34.8, 1536 x 1500 x 5504 51 -> 41,
-// 640 x 2048 x 5504 36 -> 28; 1.25 times, full: 512 x 3072 x 4096 28.9 -> 27.7 (not taken), 768 x 2048 x 5504 36 -> 32, 1024 x 1500 x 5504 37 -> 32; 1.25
-// times, a quarter padding: 420 x 3072 x 4096 24 against 28 here, 200 x 3072 x 4096 17.0 against 19.5; adding the shares of a K of
-// 4096 leaves 4 % of the latter gain, so those keep the ring; alike: 512 x 4096 x 4096 30.9 against 31.8.  No ring: 128 x 3072 x 4096 21 -> 16, 154 x 2048 x 5504 22 -> 17.
+// 512 / 768 / 1024 rows 24 -> 20, 30 -> 24, 32 -> 24, 41 -> 28, 45 -> 36, 63 -> 45, 67 -> 47; 1536 x 8192 at 1536 / 2048 (ring of 128 x
+// 128) 71 -> 53, 74 -> 69; 2390 x 11008 at 2048 (128 x 64 tiles; one share) 194 -> 161.  Where no ring takes the shape and 64- or 128-row
+// tiles fill 70 percent of the compute units with it, K is cut as the 64 x 64 tiles cut it, whose bits those rows had before; as many shares
+// as the chip has room for took 19, 20, 23, 26, 32, 39 at the first six of these row counts.
+// K of 4096 to 8191: adding up the shares has to come out of the compute units that work here and not under the ring, i.e. out of
+// gain = shares * area(ring tile) / area(tile), where area counts a workgroup's outputs.
+//   gain 1.5: 128 x 4992 x 4096 22.1 -> 19.6, 333 x 3072 x 4096 25.2 -> 23.7, 768 x 3072 x 4096 38.7 -> 34.8, 1536 x 1500 x 5504 51 -> 41, 640 x 2048 x
+//     5504 36 -> 28.  Taken: from 1.4 on.
+//   gain 1.25, outputs for 90 percent of the compute units and more: 768 x 2048 x 5504 36 -> 32, 1024 x 1500 x 5504 37 -> 32; at a K of 4096, where
+//     the sum weighs more, only 4 percent (512 x 3072 x 4096 28.9 -> 27.7).  Taken: from 1.2 on with a K of 5120 and more.
+//   gain 1.25, a quarter of it padding: 420 x 3072 x 4096 24 -> 28, 200 x 3072 x 4096 17.0 -> 19.5; gain 1: 512 x 4096 x 4096 30.9 -> 31.8.  Not taken.
+//   no ring to compare with: from three shares over 3/16 of the compute units on: 128 x 3072 x 4096 21 -> 16, 154 x 2048 x 5504 22 -> 17.
 struct ShareForm { int bm, shares, per; };
 static ShareForm share_form(const MfmaArgs& a) {
   const ShareForm none{0, 0, 0};

@@ -1,9 +1,10 @@
 // The few words of state between two decoded tokens: the greedy token of every row and its next position, and the state that a
-// caller sets before a step.  Each was a chain of library launches around a step that is itself a chain of launches: at one
-// sequence and 32000 logits the library's argmax took 13.0 us, the copy of its result and the position increment 6 with their
-// gaps, for 64 KB that one compute unit reads in about one; setting the resident step's state took three 4-byte copies of 3 to
-// 6 us each.  A token of a one-block model 69.5 -> 57.8 us, of 8 layers of the 7B shape with int4 factors 486 -> 440, of 32 with
-// 16-bit factors 1966 -> 1921, of sixteen sequences over 4 layers 596 -> 584.
+// caller sets before a step, one launch each instead of a chain of library launches.
+//   greedy token, one sequence of 32000 logits, on every token of the graph engine: the library's argmax took 13.0 us, the copy of its
+//     result and the position increment 6 with their gaps; this takes 5.9, bound by the one compute unit that reads the row.
+//   state, once per prompt in a generation: three 4-byte copies of 3 to 6 us each in front of the resident step, two in front of a
+//     graph -> one launch.  The steps advance their own state, so a generated token gains nothing from it; a program that sets the
+//     state before every token of the resident step saves 46 us on each.
 #include "common.hpp"
 #include "../../include/flashsvd_hip.h"
 
@@ -21,7 +22,7 @@ __device__ __forceinline__ uint32_t order_key(uint32_t p) {
 }
 
 // One workgroup per row: the row is requested in rounds of four 16-byte pieces per thread (32768 elements), so what it takes is
-// one round trip and 60 GB/s of one compute unit.  Ties go to the lowest index and NaN counts as the largest value, as
+// one round trip per round and the 60 GB/s of one compute unit.  Ties go to the lowest index and NaN counts as the largest value, as
 // torch.argmax has it.
 template <int DT>
 __global__ __launch_bounds__(kPickThreads) void greedy_token_kernel(const uint16_t* __restrict__ logits, int64_t ld, int64_t* __restrict__ tokens,
