@@ -852,6 +852,9 @@ def _attn_prefill_impl(q, k, v, q_pos0, causal, pad_mask, add_mask, out, softmax
         out = torch.empty(B, M, H, Dh, device=q.device, dtype=dt)
     _need(out, "out", dtype=dt)
     spm = sam_b = sam_q = 0
+    for t, nm in ((pad_mask, "pad_mask"), (add_mask, "add_mask")):
+        if t is not None and t.device != q.device:
+            raise ValueError(f"{nm} must be on the device of q, {q.device}, got {t.device}")
     if pad_mask is not None:
         if pad_mask.dtype != torch.uint8 or pad_mask.dim() != 2 or pad_mask.shape[0] != B or pad_mask.stride(1) != 1:
             raise ValueError("pad_mask must be uint8 [B, keys]")

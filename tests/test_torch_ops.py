@@ -72,6 +72,18 @@ def test_token_rows_are_an_operator_of_one_device():
                 hip_ops._set_token_rows_impl(*(on(dt, i) for dt, i in zip((torch.long, torch.long, torch.int32), devices)), 3)
 
 
+def test_prompt_attention_refuses_masks_of_another_device():
+    """The kernel reads the masks through raw addresses: one that was left on the host is refused, not read."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from flashsvd_amd import hip_ops
+    with FakeTensorMode():
+        q, kv = torch.empty(2, 9, 4, 128, dtype=BF16, device="cuda:0"), torch.empty(2, 9, 4, 128, dtype=BF16, device="cuda:0")
+        for device in ("cpu", "cuda:1"):
+            for pad, add in ((torch.empty(2, 9, dtype=torch.uint8, device=device), None), (None, torch.empty(2, 9, 9, device=device))):
+                with pytest.raises(ValueError, match="on the device of q"):
+                    hip_ops._attn_prefill_impl(q, kv, kv, None, True, pad, add, None, None)
+
+
 @pytest.mark.gpu
 def test_opcheck_and_fake_tensor_tracing_on_the_device():
     """torch.library.opcheck (schema and fake-tensor consistency against the real kernels) on the hot operators, and a
