@@ -538,7 +538,7 @@ def run_dense(args):
 
 
 def run_dense_step(args):
-    """The same 7B shape with DENSE bf16 weights through this build's own engine: the resident step kernel walking
+    """The same 7B shape with DENSE bf16 weights through this package's own engine: the resident step kernel walking
     [q;k;v] projection -> attention -> merge -> o projection -> gate/up pair + SwiGLU -> down projection per layer
     (flashsvd_amd.step.DenseStepDecoder).  Same kernel, same hand-off and attention phase as the low-rank step: the
     like-for-like comparator for "the same model run as dense bf16 on the same GPU"."""
@@ -885,7 +885,7 @@ def run_cpu_baseline():
 def main():
     args = _parse()
     if args.gpus != 1:
-        print(f"bench.py: this build measures one GPU only (got --gpus {args.gpus}); no multi-GPU path exists", file=sys.stderr)
+        print(f"bench.py: this benchmark measures one GPU only (got --gpus {args.gpus}); no multi-GPU path exists", file=sys.stderr)
         sys.exit(2)
     import torch
     if not torch.cuda.is_available():
@@ -969,7 +969,7 @@ def main():
         line["dense_bf16"] = {
             "tok_s": best, "ms_per_step": 1e3 / best, "speedup_lowrank_vs_dense": lr["tok_s"] / best,
             "comparator": "resident step kernel over dense weights" if ds["tok_s"] >= dn["tok_s"] else "torch.matmul graph",
-            "resident_step": dict(ds, how="same shape, dense bf16 weights, this build's resident step kernel (q;k;v projection, attention, "
+            "resident_step": dict(ds, how="same shape, dense bf16 weights, this package's resident step kernel (q;k;v projection, attention, "
                                           "o projection, gate/up pair + SwiGLU, down projection per layer), one launch per token"),
             "torch_graph": dict(dn, how="same shape, dense bf16 weights, torch.matmul (hipBLASLt) projections, torch elementwise ops, "
                                         "same attention kernel, one HIP graph per token"),

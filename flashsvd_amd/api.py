@@ -175,7 +175,7 @@ def _manual_llama_decode_step(model, input_ids: torch.Tensor, *, past_key_values
 
 def _build_generation_cache(model, *, prompt_len: int, max_new_tokens: int, batch_size: int, device):
     """(cache, use_manual_decode).  The dense FlashSVD cache is used when the dense-attention decode
-    route or the dense-KV baseline is switched on; this build has no other cache for its modules."""
+    route or the dense-KV baseline is switched on; the package has no other cache for its modules."""
     from .runtime.cache import FlashSVDLegacySparseKVCache, FlashSVDV15DenseKVCache
     dtype = next(iter(model.parameters())).dtype
     use_flash = _env_truthy("FLASH_SVD_ENABLE_DENSE_ATTN_DECODE") and not _env_truthy("SVDLLM_FLASH_FALLBACK")
@@ -263,7 +263,7 @@ def decode_kvcache_eval(model, *, prompt_len: int = 2048, new_tokens: int = 128,
 
     Cache choice as in utils/evaluator.py:352-388: ``lowrank_cache`` decodes over the rank-space cache
     (FlashSVDLegacySparseKVCache: per-layer, possibly unequal q/k/v ranks, shaped at the first write), otherwise the
-    dense cache (this build has no third, HF-static one, so ``flashsvd_dense_cache`` left unset means "dense unless
+    dense cache (the package has no third, HF-static one, so ``flashsvd_dense_cache`` left unset means "dense unless
     lowrank_cache").  Two modes switched on together raise, as there."""
     from .graphs import GraphedDecoder
     from .runtime.cache import FlashSVDLegacySparseKVCache, FlashSVDV15DenseKVCache

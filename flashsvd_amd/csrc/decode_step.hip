@@ -128,7 +128,7 @@ struct GemvCtx {
 };
 // wbits of an int4 phase: 4 with bf16 activations, FSVD_WBITS_Q4_FP16 with float16 ones
 __host__ __device__ __forceinline__ bool is_q4_bits(int wbits) { return wbits == 4 || wbits == FSVD_WBITS_Q4_FP16; }
-// QB: the wbits value of an int4 phase in this build of the kernel (one compare on the walk)
+// QB: the wbits value of an int4 phase in this instance of the kernel (one compare on the walk)
 template <bool Q4, int QB>
 __device__ __forceinline__ void gemv_ctx(uint32_t dv, int w, GemvCtx& c) {
   c.K = DF_I(dv, K);

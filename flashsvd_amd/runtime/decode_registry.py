@@ -83,7 +83,7 @@ def flash_attn_with_kvcache(q, k_cache, v_cache, k=None, v=None, rotary_cos=None
 
 
 def get_flash_attn_with_kvcache():
-    """The attend-with-append callable of this build (never None: it does not depend on flash-attn)."""
+    """The attend-with-append callable of this package (never None: it does not depend on flash-attn)."""
     return flash_attn_with_kvcache
 
 
