@@ -7,7 +7,6 @@
 // with write-through stores; the last workgroup to arrive for a (b,h) merges the partials in
 // split order, so the result does not depend on arrival order.
 #include "common.hpp"
-#include "decode_map.hpp"
 #include "kernels.hpp"
 
 namespace fsvd {
@@ -17,28 +16,44 @@ constexpr int kAttnThreads = 256;
 // sequence may be cut into fewer ranges than that, decode_map.hpp; the key loop is streamed)
 constexpr int kMaxRowsPerRange = 1 << 20;
 
-// The range, head (or head group) and sequence of this workgroup (decode_map.hpp), len = seqlens[b].
-template <int DH>
-__device__ __forceinline__ void decode_work_item(const int32_t* seqlens, int B, int H, int nsplit, int& b, int& h, int& s, int& len) {
-  if (decode_by_length(DH, B, H)) {
-    const int lane = threadIdx.x & 63, n = seqlens[min(lane, B - 1)];     // on its way during the divisions
-    const DecodeSlot slot = decode_slot_by_length(blockIdx.x, B, H, nsplit);
-    int rank = 0;                     // of this lane's sequence, longest first
-    for (int u = 0; u < B; ++u) {
-      const int nu = __builtin_amdgcn_readlane(n, u);
-      rank += nu > n || (nu == n && u < lane);
+// The range, head (or head group, H of them) and sequence of this workgroup, len = seqlens[b] and the number of ranges of that
+// sequence.  Five to 64 sequences: a wave has all their lengths, and all workgroups come to the same assignment.  Up to four take the
+// first ranges first whatever their lengths (what the lengths would tell comes 0.2 us later, 3 percent of 129 keys), as long as that leaves
+// the heads of a kv head together (28 heads over four, 1500 keys 11.7 -> 14.1).
+__device__ __forceinline__ int decode_keys(const AttnDecodeArgs& a, int len) { return max(0, min(len + a.seqlen_add, a.S)); }
+__device__ __forceinline__ void decode_work_item(const AttnDecodeArgs& a, int H, int& b, int& h, int& s, int& len, int& ranges) {
+  DecodeSlot slot;
+  int one_below = a.plan.one_below;
+  const bool sorts = a.plan.by_length > 0.f;
+  if (a.B > 4 && a.B <= 64 && (a.nsplit > 1 || sorts)) {
+    const int lane = threadIdx.x & 63, n = a.seqlens[min(lane, a.B - 1)];     // lanes past the last sequence repeat it
+    slot = decode_slot_by_range(blockIdx.x, a.B, H, a.nsplit);
+    asm volatile("" : "+s"(slot.s), "+s"(slot.h), "+s"(slot.seq));      // the divisions while the lengths are on their way
+    const float keys = (float)decode_keys(a, n), longest = wave_max(keys);
+    float mean = 0.f;
+    if (sorts || a.plan.one_if_even) mean = wave_sum(lane < a.B ? keys : 0.f) / a.B;
+    if (longest >= (float)one_below || (a.plan.one_if_even && longest > 1.5f * mean)) one_below = 0;
+    const float uneven = longest >= kDecodeLong ? a.plan.by_length : a.plan.by_length_short;
+    if (sorts && uneven > 0.f && longest > uneven * mean) {
+      slot = decode_slot_by_length(blockIdx.x, a.B, H, a.nsplit);
+      int rank = 0;                     // of this lane's sequence, longest first
+      for (int u = 0; u < a.B; ++u) {
+        const int nu = __builtin_amdgcn_readlane(n, u);
+        rank += nu > n || (nu == n && u < lane);
+      }
+      slot.seq = __builtin_ctzll(__ballot(lane < a.B && rank == slot.seq));
+    } else if (2 * decode_ranges(one_below, a.nsplit, (int)longest) <= a.nsplit) {
+      slot = decode_slot_by_pair(blockIdx.x, a.B, H, a.nsplit);
     }
-    s = slot.s;
-    h = slot.h;
-    b = __builtin_ctzll(__ballot(lane < B && rank == slot.seq));
-    len = __builtin_amdgcn_readlane(n, b);
+    len = __builtin_amdgcn_readlane(n, slot.seq);
   } else {
-    const DecodeSlot slot = decode_slot_by_pair(blockIdx.x, B, H, nsplit);
-    s = slot.s;
-    h = slot.h;
-    b = slot.seq;
-    len = seqlens[b];
+    slot = (a.B <= 4 && a.B * H % 8 == 0) || one_below > 0 ? decode_slot_by_pair(blockIdx.x, a.B, H, a.nsplit) : decode_slot_by_range(blockIdx.x, a.B, H, a.nsplit);
+    len = a.seqlens[slot.seq];
   }
+  b = slot.seq;
+  h = slot.h;
+  s = slot.s;
+  ranges = decode_ranges(one_below, a.nsplit, decode_keys(a, len));
 }
 
 // coherent (L2-bypassing) scalar accessors for the cross-workgroup partials: the producers write
@@ -82,8 +97,9 @@ __device__ __forceinline__ void append_own_row(const AttnDecodeArgs& a, int b, i
   __syncthreads();
 }
 
+// (head_dim 64 would fit eight waves on a SIMD, all of up to 2048 workgroups at once: 16 x 4000 keys of 32 heads 111.8 us, with seven 105.5)
 template <int DT, int DH, int U>
-__global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArgs a) {
+__global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(1, DH == 64 ? 7 : 8))) void attn_decode_kernel(AttnDecodeArgs a) {
   typedef E16<DT> E;
   constexpr int LPK = DH / 8;                 // lanes that share one key (8 bf16 each)
   constexpr int KPB = kAttnThreads / LPK;     // keys per block pass
@@ -93,14 +109,12 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
   __shared__ float red[2][4];
   __shared__ int last_flag;
 
-  int b, h, s, len;
-  decode_work_item<DH>(a.seqlens, a.B, a.H, a.nsplit, b, h, s, len);
+  int b, h, s, len, ranges;
+  decode_work_item(a, a.H, b, h, s, len, ranges);
+  if (s >= ranges) return;
   const int tid = threadIdx.x;
   const int hk = h / (a.H / a.Hk);
-  int n_keys = len + a.seqlen_add;
-  n_keys = max(0, min(n_keys, a.S));
-  const int ranges = decode_ranges(DH, 1, a.B, a.H, a.nsplit, n_keys);
-  if (s >= ranges) return;
+  const int n_keys = decode_keys(a, len);
   int per = (n_keys + ranges - 1) / ranges;
   per = (per + KPB - 1) / KPB * KPB;
   const int k0 = min(s * per, n_keys);
@@ -267,14 +281,12 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_gqa_kernel(AttnDecod
   __shared__ float red[2][4][G], sums[4][G];
   __shared__ int last_flag;
 
-  int b, hg, s, len;
-  decode_work_item<DH>(a.seqlens, a.B, a.H / G, a.nsplit, b, hg, s, len);
+  int b, hg, s, len, ranges;
+  decode_work_item(a, a.H / G, b, hg, s, len, ranges);
+  if (s >= ranges) return;
   const int tid = threadIdx.x;
   const int h0 = hg * G, hk = h0 / (a.H / a.Hk);
-  int n_keys = len + a.seqlen_add;
-  n_keys = max(0, min(n_keys, a.S));
-  const int ranges = decode_ranges(DH, G, a.B, a.H, a.nsplit, n_keys);
-  if (s >= ranges) return;
+  const int n_keys = decode_keys(a, len);
   int per = (n_keys + ranges - 1) / ranges;
   per = (per + KPB - 1) / KPB * KPB;
   const int k0 = min(s * per, n_keys);
@@ -520,6 +532,7 @@ int launch_attn_decode(const AttnDecodeArgs& args, hipStream_t st) {
   else if (a.Dh == 128) {
     if (rep % 2 == 0 && (int64_t)a.B * (a.H / 2) * a.nsplit >= 512) G = 2;
   }
+  a.plan = decode_plan(a.Dh, G, a.B, a.H, a.Hk, a.nsplit);
   if (a.k_new && !append_in_kernel(a, G)) {
     const KvAppendArgs ka{a.k_new, a.v_new, a.sk_b, a.sk_h, a.sv_b, a.sv_h, const_cast<uint16_t*>(a.k_cache), const_cast<uint16_t*>(a.v_cache),
                           a.sc_b, a.sc_s, a.sc_h, a.seqlens, a.cos, a.sin, a.rope_len, a.B, a.Hk, a.Dh, a.S, a.dt};

@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "decode_map.hpp"
+
 namespace fsvd {
 
 struct LinearArgs {
@@ -65,6 +67,7 @@ struct AttnDecodeArgs {
   // rows to append at position seqlens[b], [B, Hk, Dh] (seqlen_add is 1 then)
   const uint16_t* k_new = nullptr; const uint16_t* v_new = nullptr;
   int64_t sk_b = 0, sk_h = 0, sv_b = 0, sv_h = 0;
+  DecodePlan plan{0, 0, 0.f, 0.f};
 };
 
 struct KvAppendArgs {

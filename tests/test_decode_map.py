@@ -11,20 +11,39 @@ PROGRAM = r"""
 #include <vector>
 #include "decode_map.hpp"
 using namespace fsvd;
+template <class F>
+bool every_part(F slot, const char* how, int B, int H, int nsplit) {
+  std::vector<int> seen((size_t)B * H * nsplit);
+  for (int id = 0; id < B * H * nsplit; ++id) {
+    const DecodeSlot t = slot(id, B, H, nsplit);
+    if (t.s < 0 || t.s >= nsplit || t.h < 0 || t.h >= H || t.seq < 0 || t.seq >= B || seen[((size_t)t.seq * H + t.h) * nsplit + t.s]++) {
+      printf("%d %d %d %s: workgroup %d is outside or takes a part twice\n", B, H, nsplit, how, id);
+      return false;
+    }
+  }
+  return true;
+}
 int main(int argc, char** argv) {
   for (int i = 1; i + 3 < argc; i += 4) {
-    const int dh = atoi(argv[i]), B = atoi(argv[i + 1]), H = atoi(argv[i + 2]), nsplit = atoi(argv[i + 3]), blocks = B * H * nsplit;
-    std::vector<int> seen((size_t)blocks);
-    for (int id = 0; id < blocks; ++id) {
-      const DecodeSlot t = decode_by_length(dh, B, H) ? decode_slot_by_length(id, B, H, nsplit) : decode_slot_by_pair(id, B, H, nsplit);
-      if (t.s < 0 || t.s >= nsplit || t.h < 0 || t.h >= H || t.seq < 0 || t.seq >= B) { printf("%d %d %d %d: workgroup %d outside\n", dh, B, H, nsplit, id); return 1; }
-      if (seen[((size_t)t.seq * H + t.h) * nsplit + t.s]++) { printf("%d %d %d %d: workgroup %d takes a part twice\n", dh, B, H, nsplit, id); return 1; }
-    }
-    for (int group : {1, 2, 4})
-      for (int n = 0; n < 5000; n += 1 + n / 50) {
-        const int r = decode_ranges(dh, group, B, H, nsplit, n);
-        if (r < 1 || r > nsplit || (r > 1 && (r - 1) * 128 >= n)) { printf("%d %d %d %d: %d keys in %d ranges\n", dh, B, H, nsplit, n, r); return 1; }
+    const int dh = atoi(argv[i]), B = atoi(argv[i + 1]), H = atoi(argv[i + 2]), nsplit = atoi(argv[i + 3]);
+    if (B * H % 8 == 0 && H % 8 == 0 && !every_part(decode_slot_by_length, "by length", B, H, nsplit)) return 1;
+    if (!every_part(decode_slot_by_pair, "by pair", B, H, nsplit) || !every_part(decode_slot_by_range, "by range", B, H, nsplit)) return 1;
+    for (int hk : {1, 2, H}) {
+      if (H % hk) continue;
+      for (int group : {1, 2, 4}) {
+        if (H / hk % group) continue;
+        const DecodePlan p = decode_plan(dh, group, B, H, hk, nsplit);
+        const int heads = H / group, same = H / hk / group;
+        // by length only what a wave can sort, and never a kv head on two XCDs
+        if (p.by_length > 0.f && (B < 5 || B > 64 || heads % 8 || heads / 8 % same)) { printf("%d %d %d %d over %d: by length\n", dh, B, H, nsplit, hk); return 1; }
+        // one range each only where that makes full rounds of workgroups
+        if (p.one_below && (B * heads < 256 || (B * heads + 255) / 256 * 256 * 9 > B * heads * 10)) { printf("%d %d %d %d over %d: one range\n", dh, B, H, nsplit, hk); return 1; }
+        for (int n = 0; n < 5000; n += 1 + n / 50) {
+          const int r = decode_ranges(p.one_below, nsplit, n);
+          if (r < 1 || r > nsplit || (r > 1 && (r - 1) * 128 >= n)) { printf("%d %d %d %d: %d keys in %d ranges\n", dh, B, H, nsplit, n, r); return 1; }
+        }
       }
+    }
   }
   return 0;
 }
@@ -45,6 +64,20 @@ def test_every_range_has_one_workgroup(tmp_path):
     assert r.returncode == 0, r.stdout
 
 
+def test_what_the_shape_decides(tmp_path):
+    """The query heads of a kv head stay on one XCD; a second round of workgroups that is nearly empty is no reason for one range."""
+    _build(tmp_path, """#include "decode_map.hpp"
+using namespace fsvd;
+static_assert(decode_plan(128, 1, 48, 16, 2, 2).by_length == 0.f && decode_plan(128, 1, 5, 16, 4, 16).by_length == 0.f);
+static_assert(decode_plan(128, 1, 16, 32, 32, 4).by_length < 1.1f && decode_plan(128, 4, 64, 32, 8, 1).by_length == 1.5f);
+static_assert(decode_plan(128, 2, 24, 32, 8, 2).by_length == 0.f && decode_plan(64, 1, 16, 32, 32, 4).by_length == 0.f);
+static_assert(decode_plan(128, 1, 24, 12, 12, 7).one_below == 0 && decode_plan(64, 1, 24, 12, 12, 7).one_below == 0);
+static_assert(decode_plan(128, 1, 16, 32, 32, 4).one_below == 1536 && decode_plan(64, 1, 16, 16, 16, 3).one_below == 512);
+static_assert(decode_plan(128, 1, 16, 32, 32, 1).one_below == 0 && decode_plan(128, 4, 64, 32, 8, 2).one_below == 0);
+int main() { return 0; }
+""")
+
+
 def test_assignment_of_many_pairs_is_a_constant_expression(tmp_path):
     """131072 (sequence, head) pairs and more: the arithmetic stays within 32 bits (a constant expression that overflows does not
     compile), and the ranges of a pair go an equal share of an XCD's workgroups apart."""
@@ -55,5 +88,7 @@ def test_assignment_of_many_pairs_is_a_constant_expression(tmp_path):
             first, xcds = s * per, 8 if B * H % 8 == 0 else 1
             pair = s * max(1, per // nsplit) % per
             asserts.append(f"constexpr auto t{len(asserts)} = decode_slot_by_pair({first * xcds}, {B}, {H}, {nsplit});\n"
+                           f"constexpr auto r{len(asserts)} = decode_slot_by_range({first}, {B}, {H}, {nsplit});\n"
+                           f"constexpr auto p{len(asserts)} = decode_plan(64, 1, {B}, {H}, {H}, {nsplit});\n"
                            f"static_assert(t{len(asserts)}.s == {s} && t{len(asserts)}.h == {pair % H} && t{len(asserts)}.seq == {pair // H});")
     _build(tmp_path, '#include "decode_map.hpp"\nusing namespace fsvd;\n' + "\n".join(asserts) + "\nint main() { return 0; }\n")
