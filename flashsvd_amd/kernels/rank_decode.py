@@ -169,15 +169,23 @@ def _rankkv_append_impl(pk, pv, pk_cache, pv_cache, positions):
 def rankkv_fill(p: torch.Tensor, pk_cache: torch.Tensor, pv_cache: torch.Tensor, start: int) -> None:
     """pk_cache[:B, start:start + T] and pv_cache[:B, start:start + T] from the last Rk + Rv columns of the packed coefficients p
     [B, T, R*] (FlashSVDLegacySparseKVCache.update, runtime/cache/attn_legacy_sparse_kv.py:113-169).  Rows and caches of one 16-bit
-    type on the 16-byte grid take one launch (custom operator flashsvd_hip::rankkv_fill), others two copies."""
+    type on the 16-byte grid, whose rows lie apart, take one launch (custom operator flashsvd_hip::rankkv_fill), others two copies."""
+    B, T, w = p.shape
+    (_, S, rk), rv = pk_cache.shape, pv_cache.shape[2]
+    grid = w | rk | rv
+    one = B * T > 0 and p.is_cuda and p.is_contiguous() and p.dtype in (torch.bfloat16, torch.float16) and pv_cache.shape[1] == S
+    for t, r in ((pk_cache, rk), (pv_cache, rv)):
+        grid |= t.stride(0) | t.stride(1)
+        one = one and t.dtype == p.dtype and t.device == p.device and t.stride(2) == 1 and t.stride(1) >= r and (B == 1 or t.stride(0) >= S * t.stride(1))
+    if one and grid % 8 == 0:                          # (whether they start on the grid is known inside the operator)
+        _OPS.rankkv_fill.default(p, pk_cache, pv_cache, int(start))
+    else:
+        _rankkv_copies(p, pk_cache, pv_cache, int(start))
+
+
+def _rankkv_copies(p, pk_cache, pv_cache, start):
     B, T, w = p.shape
     rk, rv = pk_cache.shape[2], pv_cache.shape[2]
-    grid = w | rk | rv | pk_cache.stride(0) | pk_cache.stride(1) | pv_cache.stride(0) | pv_cache.stride(1)
-    if B * T and p.is_contiguous() and p.dtype in (torch.bfloat16, torch.float16) and p.dtype == pk_cache.dtype == pv_cache.dtype and grid % 8 == 0 \
-            and pk_cache.stride(2) == pv_cache.stride(2) == 1 and pk_cache.stride(1) >= rk and pv_cache.stride(1) >= rv \
-            and p.device == pk_cache.device == pv_cache.device and (p.data_ptr() | pk_cache.data_ptr() | pv_cache.data_ptr()) % 16 == 0:
-        _OPS.rankkv_fill.default(p, pk_cache, pv_cache, int(start))
-        return
     pk_cache[:B, start:start + T] = p[..., w - rk - rv:w - rv]
     pv_cache[:B, start:start + T] = p[..., w - rv:]
 
@@ -195,6 +203,8 @@ def _rankkv_fill_impl(p, pk_cache, pv_cache, start):
     if rk + rv > w or pk_cache.shape[0] < B or pv_cache.shape[0] < B or pv_cache.shape[1] != S:
         raise ValueError(f"shapes do not agree: p {tuple(p.shape)} caches {tuple(pk_cache.shape)} / {tuple(pv_cache.shape)}")
     base = p.data_ptr()
+    if start >= 0 and start + T <= S and (base | pk_cache.data_ptr() | pv_cache.data_ptr()) % 16:
+        return _rankkv_copies(p, pk_cache, pv_cache, start)
     rc = _lib.load().fsvd_rankkv_fill(base + 2 * (w - rk - rv), w, base + 2 * (w - rv), w, pk_cache.data_ptr(), pk_cache.stride(0), pk_cache.stride(1),
                                       pv_cache.data_ptr(), pv_cache.stride(0), pv_cache.stride(1), int(start), B, T, S, rk, rv, stream())
     check("fsvd_rankkv_fill", rc)

@@ -398,3 +398,7 @@ def test_rankkv_fill_matches_copies(RD, B, T, start, rq, rk, rv, dtype):
     RD.rankkv_fill(p, *views, start)
     for v, c, w in zip(views, want, wide):
         assert torch.equal(v, c) and bool((w[:, 0] == 7).all()) and bool((w[..., v.shape[2]:] == 7).all())
+    off = [torch.full((B + 1, S, r + 8), 7.0, device="cuda", dtype=dtype) for r in (rk, rv)]
+    RD.rankkv_fill(p, *(o[..., 4:4 + r] for o, r in zip(off, (rk, rv))), start)                  # strides on the grid, addresses off it
+    for o, c, r in zip(off, want, (rk, rv)):
+        assert torch.equal(o[..., 4:4 + r], c) and bool((o[..., :4] == 7).all()) and bool((o[..., 4 + r:] == 7).all())

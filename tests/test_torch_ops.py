@@ -84,6 +84,34 @@ def test_prompt_attention_refuses_masks_of_another_device():
                     hip_ops._attn_prefill_impl(q, kv, kv, None, True, pad, add, None, None)
 
 
+def test_prompt_coefficients_without_addresses_and_into_any_pair_of_caches():
+    """The route of rankkv_fill is known from shapes and strides (a traced tensor has no address); caches of unequal length
+    and caches that overlap are not for the kernel."""
+    import warnings
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from flashsvd_amd.kernels.rank_decode import rankkv_fill
+
+    class Names(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func.name())
+            return func(*args, **(kwargs or {}))
+
+    with FakeTensorMode(), warnings.catch_warnings():
+        warnings.simplefilter("error")
+        new = lambda *s: torch.empty(*s, dtype=BF16, device="cuda:0")
+        p, rows = new(2, 9, 192), new(2, 32, 64)
+        for pk, pv, in_one in ((rows, new(2, 32, 64), True), (rows, new(2, 40, 64), False), (rows, new(1, 32, 64).expand(2, 32, 64), False),
+                               (new(2, 32, 72)[..., 8:], rows, True), (new(32, 2, 64).transpose(0, 1), rows, False)):
+            seen = []
+            with Names():
+                try:
+                    rankkv_fill(p, pk, pv, 0)
+                except RuntimeError:
+                    assert not in_one                          # copies refuse to write rows that overlap
+            assert ("flashsvd_hip::rankkv_fill" in seen) == in_one, (pk.shape, pk.stride(), pv.shape, pv.stride())
+
+
 @pytest.mark.gpu
 def test_opcheck_and_fake_tensor_tracing_on_the_device():
     """torch.library.opcheck (schema and fake-tensor consistency against the real kernels) on the hot operators, and a
