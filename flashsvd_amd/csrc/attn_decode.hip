@@ -23,18 +23,24 @@ constexpr int kMaxRowsPerRange = 1 << 20;
 __device__ __forceinline__ int decode_keys(const AttnDecodeArgs& a, int len) { return max(0, min(len + a.seqlen_add, a.S)); }
 __device__ __forceinline__ void decode_work_item(const AttnDecodeArgs& a, int H, int& b, int& h, int& s, int& len, int& ranges) {
   DecodeSlot slot;
+  asm volatile("" :: "s"(a.q), "s"(a.seqlen_add));   // the lines of the arguments that are needed behind the lengths, along with the others
   int one_below = a.plan.one_below;
   const bool sorts = a.plan.by_length > 0.f;
   if (a.B > 4 && a.B <= 64 && (a.nsplit > 1 || sorts)) {
     const int lane = threadIdx.x & 63, n = a.seqlens[min(lane, a.B - 1)];     // lanes past the last sequence repeat it
     slot = decode_slot_by_range(blockIdx.x, a.B, H, a.nsplit);
     asm volatile("" : "+s"(slot.s), "+s"(slot.h), "+s"(slot.seq));      // the divisions while the lengths are on their way
-    const float keys = (float)decode_keys(a, n), longest = wave_max(keys);
-    float mean = 0.f;
-    if (sorts || a.plan.one_if_even) mean = wave_sum(lane < a.B ? keys : 0.f) / a.B;
-    if (longest >= (float)one_below || (a.plan.one_if_even && longest > 1.5f * mean)) one_below = 0;
-    const float uneven = longest >= kDecodeLong ? a.plan.by_length : a.plan.by_length_short;
-    if (sorts && uneven > 0.f && longest > uneven * mean) {
+    const int keys = decode_keys(a, n);
+    const auto any_from = [&](int k) { return __ballot(keys >= k) != 0; };
+    const float uneven = any_from(kDecodeLong) ? a.plan.by_length : (any_from(kDecodeShort) ? a.plan.by_length_short : 0.f);
+    if (any_from(one_below)) one_below = 0;
+    bool by_length = uneven == kDecodeAlways;
+    if ((sorts && uneven > kDecodeAlways) || (one_below > 0 && a.plan.one_if_even)) {
+      const float longest = wave_max((float)keys), mean = wave_sum(lane < a.B ? (float)keys : 0.f) / a.B;
+      if (a.plan.one_if_even && longest > 1.5f * mean) one_below = 0;
+      by_length |= uneven > 0.f && longest > uneven * mean;
+    }
+    if (by_length) {
       slot = decode_slot_by_length(blockIdx.x, a.B, H, a.nsplit);
       int rank = 0;                     // of this lane's sequence, longest first
       for (int u = 0; u < a.B; ++u) {
@@ -42,7 +48,7 @@ __device__ __forceinline__ void decode_work_item(const AttnDecodeArgs& a, int H,
         rank += nu > n || (nu == n && u < lane);
       }
       slot.seq = __builtin_ctzll(__ballot(lane < a.B && rank == slot.seq));
-    } else if (2 * decode_ranges(one_below, a.nsplit, (int)longest) <= a.nsplit) {
+    } else if (one_below > 0 || !any_from(128 * (a.nsplit >> 1) + 1)) {          // at least half of the ranges have no keys
       slot = decode_slot_by_pair(blockIdx.x, a.B, H, a.nsplit);
     }
     len = __builtin_amdgcn_readlane(n, slot.seq);

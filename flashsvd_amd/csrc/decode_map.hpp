@@ -9,11 +9,12 @@ namespace fsvd {
 struct DecodeSlot { int s, h, seq; };
 
 // What a call's shape leaves open until the lengths are known in the kernel.
-constexpr float kDecodeLong = 1000.f;
+constexpr int kDecodeLong = 1000, kDecodeShort = 257;
+constexpr float kDecodeAlways = 1.f;
 struct DecodePlan {
   int one_below;       // sequences of fewer keys run in one range (0: none does)
   int one_if_even;     // ... only while the longest is at most 1.5 times the mean
-  float by_length, by_length_short;     // sequences by length where the longest exceeds this many times the mean (0: never); below kDecodeLong keys
+  float by_length, by_length_short;     // sequences by length where the longest exceeds this many times the mean (0: never); from kDecodeLong, kDecodeShort keys on
 };
 
 // B sequences, H query heads over Hk, `group` heads per workgroup, at most nsplit ranges; a pair is a (sequence, group).  Measured per
@@ -25,14 +26,18 @@ struct DecodePlan {
 // channels at the same time: 16 x 1000 keys of 32 heads 55.1 -> 46.9, 16 x 300 of 16 heads of 64 10.2 -> 8.7.  A single round of fewer
 // than 512 pairs of uneven sequences has nothing that evens it out (16 x up to 1000 keys of 16 heads in one range 23.3, in ranges 20.4).
 // By length: head_dim 128, up to 64 sequences and 1024 pairs (four per compute unit; beyond, the order of dispatch evens things out: 48 x 500
-// keys of 32 heads 68 in that order, 71 by length).  An XCD takes some heads of every sequence instead of every head of some, so the query heads of
-// a kv head have to stay together (eight heads over one kv head apart: 48 x 500 keys 18.7 -> 27.1), and its pieces of a row get short: with
-// four kv heads of an XCD (1 KB) it pays for long sequences that differ at all (16 x 750 to 1000 keys 47.0 -> 44.4, but 12 x 375 to 500 22.6 ->
-// 23.8), with fewer where the longest is 1.5 times the mean (64 x 1 to 1000 keys of four heads a group 45.7 -> 36.0, but 48 x 375 to 500,
-// two heads a group, 28.0 -> 30.4, and 64 x 125, 15.0 -> 17.7).  Groups: an even number of rounds, since every other one runs backwards
-// (24 x up to 900 keys in three 24.1 -> 26.9).  No groups and two kv heads of an XCD: long ones (5 x up to 2000 keys 16.1 -> 12.8,
-// 6 x up to 900 11.4 -> 12.0) or 512 pairs, one: 512 pairs (64 x up to 1000 33.1 -> 32.0, 32 x up to 600 13.9 -> 15.4).  With head_dim 64 the
-// pieces are too short (64 x 1000 keys 98.7 -> 105), and up to four sequences leave nothing to sort.
+// keys of 32 heads 68 in that order, 71 by length).  An XCD takes some heads of every sequence instead of every head of some.
+//   A sequence of kDecodeLong keys and more: always, the reversed rounds and the eight XCDs share what there is more evenly even where
+//     all are alike (16 x 3000 to 4001 keys of 32 heads over 8 51.0 -> 49.0, 33 x up to 4001 128 -> 78, 8 x 4001 over 16 58 -> 47, 5 x 2000 to 4001 of 40
+//     heads over 8 46 -> 39); with one kv head of an XCD and a last round that is not full only where the longest is 1.2 times the
+//     mean (14 x 4001 keys of 64 heads over 8 96 -> 109).
+//   Shorter ones, from three passes of keys on (60 x up to 150 keys 13.1 -> 18.6): where the longest is 1.5 times the mean (40 x up to
+//     900 keys of 32 heads over 8 33.8 -> 25.7, but 48 x 375 to 500, two heads a group, 28.0 -> 30.4), in groups not over a full odd number of rounds,
+//     since every other one runs backwards (24 x up to 900 keys in three 24.1 -> 26.9), without groups with four kv heads of an XCD (1 KB of a
+//     row) or 512 pairs (64 x up to 1000 33.1 -> 32.0, 32 x up to 600 with fewer 13.9 -> 15.4).
+//   The query heads of a kv head on different XCDs read it twice (eight over one: 48 x 500 keys 18.7 -> 27.1, 48 x up to 2500 in two ranges
+//     37 -> 56): only long and uneven ones for which there are no ranges (36 x up to 1500 keys of 32 heads over 4 46 -> 33).
+// With head_dim 64 the pieces are too short (64 x 1000 keys 98.7 -> 105), and up to four sequences leave nothing to sort.
 constexpr DecodePlan decode_plan(int head_dim, int group, int B, int H, int Hk, int nsplit) {
   const int heads = H / group, same_kv = H / Hk / group;
   const long pairs = (long)B * heads, rounds = (pairs + 255) / 256, all_rounds = (pairs * nsplit + 255) / 256;
@@ -42,13 +47,11 @@ constexpr DecodePlan decode_plan(int head_dim, int group, int B, int H, int Hk, 
     p.one_below = full < most ? full : most;
     p.one_if_even = head_dim == 128 && pairs < 512;
   }
-  if (head_dim == 128 && heads % 8 == 0 && B > 4 && B <= 64 && pairs <= 1024 && heads / 8 % same_kv == 0) {
-    const int kv_heads = heads / 8 / same_kv;           // of an XCD
-    if (group > 1 ? all_rounds % 2 == 0 : (kv_heads >= 2 || pairs >= 512)) {
-      const bool wide = group == 1 && kv_heads >= 4;
-      p.by_length = wide ? 1.05f : 1.5f;
-      p.by_length_short = group > 1 || wide || pairs >= 512 ? 1.5f : 0.f;
-    }
+  if (head_dim == 128 && heads % 8 == 0 && B > 4 && B <= 64 && pairs <= 1024) {
+    const int kv_heads = heads / 8 % same_kv == 0 ? heads / 8 / same_kv : 0;           // of an XCD
+    const bool full = pairs * nsplit * 10 >= all_rounds * 256 * 9;
+    p.by_length = kv_heads == 0 ? (nsplit == 1 ? 1.5f : 0.f) : (full || kv_heads >= 2 ? kDecodeAlways : 1.2f);
+    if (kv_heads > 0 && (group > 1 ? !full || all_rounds % 2 == 0 : kv_heads >= 4 || pairs >= 512)) p.by_length_short = 1.5f;
   }
   return p;
 }
@@ -66,31 +69,30 @@ constexpr int decode_ranges(int one_below, int nsplit, int n_keys) {
 // By length: an XCD takes some heads of every sequence, the sequences longest first, and every other 32 workgroups of an XCD (one per
 // compute unit) in reverse, so that the ranges of a long and of a short sequence share a compute unit (pairs that are a multiple of 8, as H is).
 constexpr DecodeSlot decode_slot_by_length(int block, int B, int H, int nsplit) {
-  const int per = (B * H) >> 3, heads = H >> 3;
-  int id = block >> 3;
+  const unsigned per = (unsigned)(B * H) >> 3, heads = (unsigned)H >> 3;
+  unsigned id = (unsigned)block >> 3;
   if ((id & 32) && (id | 31) < per * nsplit) id ^= 31;
-  const int s = id / per;
-  id -= s * per;
-  return DecodeSlot{s, (block & 7) * heads + id % heads, id / heads};
+  const unsigned s = id / per, at = id - s * per, seq = at / heads;
+  return DecodeSlot{(int)s, (int)((block & 7) * heads + at - seq * heads), (int)seq};
 }
 
 // The first range of all heads of an XCD before the second of any, where half of the ranges and more have no keys: those workgroups, which
 // leave at once, are the last ones (between the others they left the compute units unevenly loaded: 16 x 1000 keys in one range 93 us).
 constexpr DecodeSlot decode_slot_by_pair(int block, int B, int H, int nsplit) {
-  const int pairs = B * H;
+  const unsigned pairs = B * H;
   const bool by_xcd = (pairs & 7) == 0;
-  const int per = by_xcd ? pairs >> 3 : pairs, xcd = by_xcd ? block & 7 : 0, id = by_xcd ? block >> 3 : block;
-  const int s = id / per, share = per / nsplit, turn = share > 1 ? share : 1;     // a range later: another compute unit
-  const int pair = xcd * per + (id - s * per + s * turn) % per;
-  return DecodeSlot{s, pair % H, pair / H};
+  const unsigned per = by_xcd ? pairs >> 3 : pairs, xcd = by_xcd ? block & 7 : 0, id = by_xcd ? block >> 3 : block;
+  const unsigned s = id / per, share = per / (unsigned)nsplit, turn = share > 1 ? share : 1;     // a range later: another compute unit
+  const unsigned pair = xcd * per + (id - s * per + s * turn) % per, seq = pair / (unsigned)H;
+  return DecodeSlot{(int)s, (int)(pair - seq * H), (int)seq};
 }
 
 // The ranges of a head side by side, where most of them have keys (first ranges first: 5 x 2000 keys of 8 heads 13.1 -> 14.0 us, 8 x up to
 // 500 of 16 heads of 64 8.0 -> 8.5).
 constexpr DecodeSlot decode_slot_by_range(int block, int B, int H, int nsplit) {
-  const int total = B * H * nsplit, id = (total & 7) == 0 ? (block & 7) * (total >> 3) + (block >> 3) : block;
-  const int pair = id / nsplit;
-  return DecodeSlot{id - pair * nsplit, pair % H, pair / H};
+  const unsigned total = (unsigned)(B * H) * nsplit, id = (total & 7) == 0 ? (block & 7) * (total >> 3) + ((unsigned)block >> 3) : block;
+  const unsigned pair = id / (unsigned)nsplit, seq = pair / (unsigned)H;
+  return DecodeSlot{(int)(id - pair * nsplit), (int)(pair - seq * H), (int)seq};
 }
 
 }  // namespace fsvd

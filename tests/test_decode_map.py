@@ -34,8 +34,8 @@ int main(int argc, char** argv) {
         if (H / hk % group) continue;
         const DecodePlan p = decode_plan(dh, group, B, H, hk, nsplit);
         const int heads = H / group, same = H / hk / group;
-        // by length only what a wave can sort, and never a kv head on two XCDs
-        if (p.by_length > 0.f && (B < 5 || B > 64 || heads % 8 || heads / 8 % same)) { printf("%d %d %d %d over %d: by length\n", dh, B, H, nsplit, hk); return 1; }
+        // by length only what a wave can sort; a kv head on two XCDs only for long sequences without ranges
+        if (p.by_length > 0.f && (B < 5 || B > 64 || heads % 8 || (heads / 8 % same && (nsplit > 1 || p.by_length_short > 0.f)))) { printf("%d %d %d %d over %d: by length\n", dh, B, H, nsplit, hk); return 1; }
         // one range each only where that makes full rounds of workgroups
         if (p.one_below && (B * heads < 256 || (B * heads + 255) / 256 * 256 * 9 > B * heads * 10)) { printf("%d %d %d %d over %d: one range\n", dh, B, H, nsplit, hk); return 1; }
         for (int n = 0; n < 5000; n += 1 + n / 50) {
@@ -65,12 +65,15 @@ def test_every_range_has_one_workgroup(tmp_path):
 
 
 def test_what_the_shape_decides(tmp_path):
-    """The query heads of a kv head stay on one XCD; a second round of workgroups that is nearly empty is no reason for one range."""
+    """The query heads of a kv head stay on one XCD where there are ranges; a second round of workgroups that is nearly empty is no reason for one range."""
     _build(tmp_path, """#include "decode_map.hpp"
 using namespace fsvd;
-static_assert(decode_plan(128, 1, 48, 16, 2, 2).by_length == 0.f && decode_plan(128, 1, 5, 16, 4, 16).by_length == 0.f);
-static_assert(decode_plan(128, 1, 16, 32, 32, 4).by_length < 1.1f && decode_plan(128, 4, 64, 32, 8, 1).by_length == 1.5f);
-static_assert(decode_plan(128, 2, 24, 32, 8, 2).by_length == 0.f && decode_plan(64, 1, 16, 32, 32, 4).by_length == 0.f);
+static_assert(decode_plan(128, 1, 48, 16, 2, 2).by_length == 0.f && decode_plan(128, 2, 48, 16, 2, 2).by_length == 0.f);
+static_assert(decode_plan(128, 2, 36, 32, 4, 1).by_length == 1.5f && decode_plan(128, 2, 36, 32, 4, 1).by_length_short == 0.f);
+static_assert(decode_plan(128, 4, 16, 32, 8, 4).by_length == kDecodeAlways && decode_plan(128, 1, 5, 40, 8, 10).by_length == kDecodeAlways);
+static_assert(decode_plan(128, 4, 14, 64, 8, 2).by_length == 1.2f && decode_plan(128, 4, 64, 32, 8, 1).by_length_short == 1.5f);
+static_assert(decode_plan(128, 2, 24, 32, 8, 2).by_length_short == 0.f && decode_plan(128, 2, 40, 32, 8, 1).by_length_short == 1.5f);
+static_assert(decode_plan(64, 1, 16, 32, 32, 4).by_length == 0.f && decode_plan(128, 1, 4, 32, 32, 4).by_length == 0.f);
 static_assert(decode_plan(128, 1, 24, 12, 12, 7).one_below == 0 && decode_plan(64, 1, 24, 12, 12, 7).one_below == 0);
 static_assert(decode_plan(128, 1, 16, 32, 32, 4).one_below == 1536 && decode_plan(64, 1, 16, 16, 16, 3).one_below == 512);
 static_assert(decode_plan(128, 1, 16, 32, 32, 1).one_below == 0 && decode_plan(128, 4, 64, 32, 8, 2).one_below == 0);
