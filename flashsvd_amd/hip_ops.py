@@ -697,6 +697,8 @@ def _mlp_from_coefficients(pg, pu, gate_u, up_u, down_v, down_u, bias, mode):
     if pg.shape != pu.shape or pg.stride() != pu.stride() or pg.shape[1] != R or up_u.shape != gate_u.shape or up_u.stride() != gate_u.stride() \
             or Dv != D or Ru != Rd:
         raise ValueError("coefficients and factors do not match")
+    if pg.device != pu.device:
+        raise ValueError(f"gate and up coefficients must be on one device, got {pg.device} and {pu.device}")
     B = pg.shape[0]
     bp = _row_vector(dt, bias, N, "bias")
     out = torch.empty(B, N, device=pg.device, dtype=dt)

@@ -112,6 +112,16 @@ def test_prompt_coefficients_without_addresses_and_into_any_pair_of_caches():
             assert ("flashsvd_hip::rankkv_fill" in seen) == in_one, (pk.shape, pk.stride(), pv.shape, pv.stride())
 
 
+def test_coefficients_of_different_devices_are_refused():
+    """The dual-split MLP reads both sets of coefficients through raw addresses, one as a distance from the other."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from flashsvd_amd import hip_ops
+    with FakeTensorMode():
+        t = lambda *s, i=0: torch.empty(*s, dtype=BF16, device=f"cuda:{i}")
+        with pytest.raises(ValueError, match="one device"):
+            hip_ops._mlp_from_coefficients(t(4, 64), t(4, 64, i=1), t(128, 64), t(128, 64), t(64, 128), t(32, 64), None, 1)
+
+
 @pytest.mark.gpu
 def test_opcheck_and_fake_tensor_tracing_on_the_device():
     """torch.library.opcheck (schema and fake-tensor consistency against the real kernels) on the hot operators, and a
