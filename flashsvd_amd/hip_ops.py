@@ -501,6 +501,8 @@ def _greedy_token_impl(logits, tokens, positions):
         _need(positions, "positions", dtype=torch.int32)
         if positions.shape != (B,) or not positions.is_contiguous():
             raise ValueError(f"positions must be a contiguous [{B}] tensor")
+    if logits.device != tokens.device or (positions is not None and positions.device != tokens.device):
+        raise ValueError("logits, tokens and positions must be on one device")
     rc = _lib.load().fsvd_greedy_token(logits.data_ptr(), logits.stride(0), tokens.data_ptr(), tokens.stride(0), _ptr(positions), B, V, code,
                                        _stream())
     _lib.check("fsvd_greedy_token", rc)
@@ -822,6 +824,8 @@ def _rope_tables_impl(position_ids, inv_freq, dtype):
     _need(position_ids, "position_ids", dtype=torch.long); _need(inv_freq, "inv_freq", dtype=torch.float32)
     if not position_ids.is_contiguous() or inv_freq.dim() != 1 or not inv_freq.is_contiguous():
         raise ValueError("position_ids and inv_freq must be contiguous, inv_freq one-dimensional")
+    if position_ids.device != inv_freq.device:
+        raise ValueError(f"position_ids and inv_freq must be on one device, got {position_ids.device} and {inv_freq.device}")
     rows, half = position_ids.numel(), inv_freq.numel()
     cos = torch.empty(rows, half, dtype=dtype, device=position_ids.device)
     sin = torch.empty_like(cos)

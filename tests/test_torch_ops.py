@@ -72,6 +72,19 @@ def test_token_rows_are_an_operator_of_one_device():
                 hip_ops._set_token_rows_impl(*(on(dt, i) for dt, i in zip((torch.long, torch.long, torch.int32), devices)), 3)
 
 
+def test_greedy_tokens_and_rotation_tables_are_of_one_device():
+    """Both take raw addresses; as tensor operations a table of two devices was refused."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from flashsvd_amd import hip_ops
+    with FakeTensorMode():
+        on = lambda i, dtype, *s: torch.empty(*s, dtype=dtype, device=f"cuda:{i}")
+        for a, b, c in ((0, 0, 1), (0, 1, 0), (1, 0, 0)):
+            with pytest.raises(ValueError, match="one device"):
+                hip_ops._greedy_token_impl(on(a, BF16, 4, 100), on(b, torch.long, 4, 1), on(c, torch.int32, 4))
+        with pytest.raises(ValueError, match="one device"):
+            hip_ops._rope_tables_impl(on(0, torch.long, 9), on(1, torch.float32, 64), BF16)
+
+
 def test_prompt_attention_refuses_masks_of_another_device():
     """The kernel reads the masks through raw addresses: one that was left on the host is refused, not read."""
     from torch._subclasses.fake_tensor import FakeTensorMode
