@@ -2,7 +2,7 @@
 
 TEST INFRASTRUCTURE ONLY.  Nothing in the shipped package imports this file; it is
 used by ``tests/``, by ``__graft_entry__.smoke()`` and by the ``cpu_baseline`` leg of
-``bench.py`` as the checker / the reported CPU figure, never as the product path.
+``bench.py``, as what results are compared with and as the reported CPU figure, never as the product path.
 
 It is a plain PyTorch-on-CPU restatement (no custom kernels) of the algorithms the
 reference implements with Triton kernels, cuBLAS calls and flash-attn, with every

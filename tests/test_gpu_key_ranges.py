@@ -21,6 +21,9 @@ def _reference(q, kc, vc, n):
     (8, 32, 32, 128, 8, (511, 512, 1023, 1024, 1535, 1536, 0, 1)), (8, 32, 32, 64, 2, (1024, 1100, 30)),                 # from 2 keys a pair
     (17, 16, 16, 128, 3, (1087, 1088, 64)), (64, 16, 16, 128, 2, (9, 300, 300, 17, 140)), (65, 8, 8, 128, 2, (300, 17)), (33, 9, 9, 64, 3, (593, 594, 595)),
     (48, 32, 32, 128, 2, (300, 17, 129)), (4, 12, 12, 128, 3, (300, 40)),                                                   # odd batches and heads, more than 1024 pairs
+    # longest first, a group of heads per workgroup: around 1000 keys, alike and not, a last round that is not full, without ranges on more than one XCD, around 257 keys
+    (16, 32, 8, 128, 4, (999, 1000, 1024, 3)), (14, 64, 8, 128, 2, (1000, 830, 999)), (14, 64, 8, 128, 2, (1024, 300, 0)), (5, 40, 8, 128, 10, (1001, 1, 130)),
+    (36, 32, 4, 128, 1, (1100, 9, 300)), (36, 32, 4, 128, 1, (999, 9, 300)), (40, 32, 8, 128, 1, (257, 20, 90)), (40, 32, 8, 128, 1, (256, 20, 90)),
     (64, 32, 8, 64, 1, (1, 31, 32, 127, 128, 129, 0, 300)), (16, 32, 8, 64, 4, (511, 512, 513, 40, 0)), (4, 64, 8, 64, 9, (3, 1160))])  # groups of 64
 def test_ranges_follow_the_length(dtype, B, H, Hk, Dh, nsplit, lens):
     from flashsvd_amd import hip_ops as ops
