@@ -182,7 +182,7 @@ struct MfmaArgs {
   // fp32 partial tiles and one arrival counter per tile; the last workgroup to arrive adds the partials in order
   int ksplit; float* ws_part; int32_t* ws_count;
   int dt = 0;
-  float* scratch = nullptr; size_t scratch_floats = 0;   // this call's own (K shares of mfma_mid.hip)
+  float* scratch = nullptr; size_t scratch_floats = 0;   // this call's own (K shares of mfma_quad.hip)
 };
 // epilogue of a head expansion (mfma_gemm.hip, mfma_mid.hip)
 struct ExpandEpi {
@@ -194,7 +194,7 @@ struct ExpandEpi {
   int dst_by_position, dst_rows;
   int pos0;
 };
-inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+__host__ __device__ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 // byte offsets of `rows` rows of stride ld fit the 32 unsigned bits of a buffer load
 inline bool below_4gib(int64_t rows, int64_t ld) { return ld >= 0 && rows * ld * 2 < (int64_t)4 << 30; }
 // "tiles 64 x 128", "ring 128 x 192 pair", ... for set_last_form, made by the compiler: an entry point neither allocates nor throws
@@ -218,7 +218,6 @@ struct SplitWorkspace { float* part; size_t part_floats; int32_t* count; int nco
 SplitWorkspace split_workspace();                                            // capi.hip
 bool gemm_tiles_apply(const MfmaArgs& a);                                   // mfma_gemm.hip: 128 rows and more
 int launch_gemm_tiles(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
-int gemm_tiles_shares(const MfmaArgs& a, int* unit);
 bool gemm_rows_apply(const MfmaArgs& a);                                    // mfma_gemm.hip: 5..127 rows, K split
 int launch_gemm_rows(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
 int compute_units();                                                         // of the current device, 0 when it cannot be asked
@@ -226,6 +225,14 @@ bool gemm_big_apply(const MfmaArgs& a, bool dual);                          // m
 int launch_gemm_big(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
 bool expand_big_apply(const ExpandArgs* d, int n);
 int launch_expand_big(const ExpandArgs* d, int n, hipStream_t st);
+bool gemm_quad_apply(const MfmaArgs& a, bool dual);                         // mfma_quad.hip: prompts, K of five steps and more
+int launch_gemm_quad(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
+bool expand_quad_apply(const ExpandArgs* d, int n);                         // mfma_quad_heads.hip
+int launch_expand_quad(const ExpandArgs* d, int n, hipStream_t st);
+struct RingRule { int area; bool halves; };                                  // outputs of a ring tile (0: no ring), K halved between waves
+RingRule gemm_mid_rule(const MfmaArgs& a);
+int gemm_tiles_cut(const MfmaArgs& a);                                      // mfma_gemm.hip: steps of 64 in a K range, 0 where K is not cut
+int gemm_tiles_shares(const MfmaArgs& a, int* unit);
 bool gemm_mid_apply(const MfmaArgs& a, bool dual);                          // mfma_mid.hip: about one tile per compute unit
 int launch_gemm_mid(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
 size_t gemm_share_floats(MfmaArgs a, size_t cap);

@@ -565,6 +565,17 @@ int gemm_tiles_shares(const MfmaArgs& a, int* unit) {
   return pick_ksplit_prompt(small, a.K / (64 * *unit), a.K, 0, plenty);
 }
 
+// Steps of 64 in a range of K where the 64 x 64 tiles cut a K below 8192 (0: they do not); a caller that takes over their shapes adds the
+// ranges up in the same order.
+int gemm_tiles_cut(const MfmaArgs& a) {
+  const auto count = [&](int bm, int bn) { return (int64_t)((a.N + bn - 1) / bn) * ((a.B + bm - 1) / bm); };
+  const int64_t small = count(64, 64);
+  if (count(128, 128) >= 144 || a.K >= 8192) return 0;
+  const int unit = small < 320 && a.K % 128 == 0 ? 2 : 1, steps = a.K / (64 * unit);
+  const int z = pick_ksplit_prompt(small, steps, a.K, (size_t)64 * 64, split_workspace());
+  return z > 1 ? (steps + z - 1) / z * unit : 0;
+}
+
 template <int DT, bool DUAL, int WTM, int WT, int BK, int NW = 4, int PFSEL = 99, bool RAG = false>
 static int launch_gemm_tiles_t(const MfmaArgs& a0, hipStream_t st, const char* who) {
   static bool granted = false;
@@ -755,6 +766,7 @@ bool expand_multi_apply(const ExpandArgs* d, int n) {
   return true;
 }
 int launch_expand_multi(const ExpandArgs* d, int n, hipStream_t st) {
+  if (expand_quad_apply(d, n)) return launch_expand_quad(d, n, st);
   if (expand_big_apply(d, n)) return launch_expand_big(d, n, st);
   if (expand_mid_apply(d, n)) return launch_expand_mid(d, n, st);
   int heads = 0;
@@ -765,6 +777,7 @@ int launch_expand_multi(const ExpandArgs* d, int n, hipStream_t st) {
 }
 
 int launch_expand_tiles(const ExpandArgs& a, hipStream_t st) {
+  if (expand_quad_apply(&a, 1)) return launch_expand_quad(&a, 1, st);
   if (expand_big_apply(&a, 1)) return launch_expand_big(&a, 1, st);
   if (expand_mid_apply(&a, 1)) return launch_expand_mid(&a, 1, st);
   // a column tile is always one head; 128 token rows per workgroup when that gives every compute unit two tiles, else 64

@@ -21,7 +21,7 @@
 
 namespace fsvd {
 
-enum MidEpi { kMidPlain = 0, kMidPair = 1, kMidHeads = 2, kMidShare = 3 };
+enum MidEpi { kMidPlain = 0, kMidPair = 1, kMidHeads = 2 };
 constexpr int kMidThreads = 512, kMidRow = 128;
 
 struct MidArgs {
@@ -29,7 +29,6 @@ struct MidArgs {
   ExpandEpi ep[3];
   int first_head[4];
   int nt;                                            // column tiles
-  int shares, per; float* part;                      // kMidShare: workgroups per tile, the K steps of each (the last one may have fewer), their sums
 };
 
 // RAG: any K, rows that start anywhere (plain and pair).  Loads that write LDS themselves want aligned addresses, so the pieces go
@@ -41,7 +40,7 @@ __global__ __launch_bounds__(kMidThreads, 2) void gemm_mid_kernel(MidArgs args) 
   typedef typename E::frag_t frag_t;
   static_assert(WM * WN * KH == 8, "eight waves");
   static_assert(!RAG || (KH == 1 && NS == 2 && (EPI == kMidPlain || EPI == kMidPair)), "ragged rows: two stages, plain and pair");
-  constexpr bool PAIR = EPI == kMidPair, HEADS = EPI == kMidHeads, SHARE = EPI == kMidShare;
+  constexpr bool PAIR = EPI == kMidPair, HEADS = EPI == kMidHeads;
   constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN, LX = BM / 64, LW = BN / 64, LOADS = KH * (LX + LW);
   static_assert(BM % 64 == 0 && BN % 64 == 0 && (!HEADS || (BN == 128 && TN % 2 == 0)), "whole groups of rows per load");
   constexpr int kHalf = (BM + BN) * kMidRow, kStage = KH * kHalf;
@@ -51,9 +50,7 @@ __global__ __launch_bounds__(kMidThreads, 2) void gemm_mid_kernel(MidArgs args) 
   const int wm = __builtin_amdgcn_readfirstlane(wi / WN), wn = __builtin_amdgcn_readfirstlane(wi % WN);
 
   // every XCD takes one contiguous run of tiles, the row tiles of a column one after the other: W crosses from HBM once
-  // (a K range of all tiles before the next range, so that an XCD reads few ranges of the operands)
-  const int tiles = SHARE ? gridDim.x / args.shares : gridDim.x, MT = tiles / args.nt, run = xcd_run_index(blockIdx.x, gridDim.x);
-  const int share = SHARE ? run / tiles : 0, t = run - share * tiles;
+  const int MT = gridDim.x / args.nt, t = xcd_run_index(blockIdx.x, gridDim.x);
   const int tn = t / MT, m0 = (t - tn * MT) * BM;
   const int pi = !HEADS ? 0 : (tn >= args.first_head[2] ? 2 : (tn >= args.first_head[1] ? 1 : 0));
   const MfmaArgs& a = args.a[pi];
@@ -76,14 +73,13 @@ __global__ __launch_bounds__(kMidThreads, 2) void gemm_mid_kernel(MidArgs args) 
   }
 #pragma unroll
   for (int j = 0; j < LW; ++j) wo[j] = (uint32_t)(min(n0 + lrow + 64 * j, a.N - 1) * a.ldw * 2) + lpiece;
-  const int first = SHARE ? share * args.per : 0, k0 = first * 128 * KH;          // this share's first K step, and its place in a row
-  const int ksteps = SHARE ? min(args.per, a.K / 64 - first) : (RAG ? (a.K + 127) / 128 * 2 : a.K / (64 * KH)), total = (PAIR ? 2 : 1) * ksteps;
+  const int ksteps = RAG ? (a.K + 127) / 128 * 2 : a.K / (64 * KH), total = (PAIR ? 2 : 1) * ksteps;
   const uint32_t my_rows = (uint32_t)__builtin_amdgcn_readfirstlane(wave) * 1024;
   const auto issue = [&](int s, int stage) {
     const bool second = PAIR && s >= ksteps;
     const uint16_t* xb = a.x + (second ? a.up_off : 0);
     const uint16_t* wb = second ? a.W2 : a.W;
-    const int k = k0 + (second ? s - ksteps : s) * 128 * KH;
+    const int k = (second ? s - ksteps : s) * 128 * KH;
 #pragma unroll
     for (int h = 0; h < KH; ++h) {
       unsigned char* dst = mid_smem + stage * kStage + h * kHalf + my_rows;
@@ -258,15 +254,6 @@ __global__ __launch_bounds__(kMidThreads, 2) void gemm_mid_kernel(MidArgs args) 
       for (int j = 0; j < TN; ++j) acc[i][j] += ex[(i * TN + j) * 256 + (tid & 255)];
   }
 
-  if constexpr (SHARE) {                               // the sums as they lie in the accumulators, for share_sum_kernel
-    f32x4_t* mine = reinterpret_cast<f32x4_t*>(args.part) + ((size_t)t * args.shares + share) * TM * TN * kMidThreads + tid;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) mine[(i * TN + j) * kMidThreads] = acc[i][j];
-    return;
-  }
-
   // ---- element e of lane (lr, lg) of tile (i, j): row i * 16 + lr, column j * 16 + lg * 4 + e; four consecutive columns of a
   // row per lane (8-byte accesses where the addresses allow)
   const auto al8 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7) == 0; };
@@ -394,79 +381,6 @@ static int launch_mid_t(MidArgs& m, hipStream_t st, const char* who) {
   return kOk;
 }
 
-// The shares of every tile, added in their order, and the epilogue of a single matrix: one thread per four columns of a row, as the
-// accumulators hold them.  A launch of its own: the shares need no counters, and all compute units add (the last workgroup of
-// each tile adding by itself took 4.7 us longer at 512 x 1536 x 11008, 48 tiles of five shares).
-template <int DT, int WN, int TM, int TN>
-__global__ __launch_bounds__(256) void share_sum_kernel(MidArgs args, int tiles) {
-  typedef E16<DT> E;
-  constexpr int WM = 8 / WN, kWords = TM * TN * kMidThreads, BM = 16 * TM * WM, BN = 16 * TN * WN;
-  const MfmaArgs& a = args.a[0];
-  const int g = blockIdx.x * 256 + threadIdx.x, t = g / kWords, r = g - t * kWords;
-  const f32x4_t* part = reinterpret_cast<const f32x4_t*>(args.part) + (size_t)t * args.shares * kWords + r;
-  f32x4_t v = part[0];
-  int z = 1;
-  for (; z + 4 <= args.shares; z += 4) {               // four shares on their way at a time
-    f32x4_t w[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) w[u] = part[(size_t)(z + u) * kWords];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) v += w[u];
-  }
-  for (; z < args.shares; ++z) v += part[(size_t)z * kWords];
-  const int ij = r / kMidThreads, tid = r - ij * kMidThreads, i = ij / TN, j = ij - i * TN, wave = tid >> 6, lane = tid & 63;
-  const int MT = tiles / args.nt, tn = t / MT;
-  const int m = (t - tn * MT) * BM + (wave / WN) * 16 * TM + i * 16 + (lane & 15);
-  const int n = tn * BN + (wave % WN) * 16 * TN + j * 16 + (lane >> 4) * 4;
-  if (m >= a.B || n >= a.N) return;
-  const uint16_t* res = a.res ? a.res + (int64_t)m * a.ldres + n : nullptr;
-  uint16_t* y = a.y + (int64_t)m * a.ldy + n;
-  uint32_t o[2];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    if (a.bias && n + e < a.N) v[e] += E::val(a.bias[n + e]);
-  }
-  o[0] = E::pack2(v[0], v[1]);
-  o[1] = E::pack2(v[2], v[3]);
-  const bool whole = n + 3 < a.N;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    if (res && n + e < a.N) v[e] = E::val(res[e]) + E::val((o[e >> 1] >> (16 * (e & 1))) & 0xffffu);
-  }
-  if (res) {
-    o[0] = E::pack2(v[0], v[1]);
-    o[1] = E::pack2(v[2], v[3]);
-  }
-  if (whole && (reinterpret_cast<uintptr_t>(y) & 7) == 0) {
-    *reinterpret_cast<u32x2_t*>(y) = u32x2_t{o[0], o[1]};
-  } else {
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (n + e < a.N) y[e] = (uint16_t)(o[e >> 1] >> (16 * (e & 1)));
-  }
-}
-
-template <int DT, int WN, int TM, int TN, int NS>
-static int launch_share_t(MidArgs& m, hipStream_t st, const char* who) {
-  static bool granted = false;
-  constexpr int WM = 8 / WN, BM = 16 * TM * WM, BN = 16 * TN * WN;
-  constexpr size_t lds = (size_t)NS * (BM + BN) * kMidRow;
-  if (!granted) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_mid_kernel<DT, kMidShare, WM, WN, TM, TN, 1, NS>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) { set_last_error("%s: cannot reserve %zu bytes of LDS: %s", who, lds, hipGetErrorString(e)); return kErrLaunch; }
-    granted = true;
-  }
-  m.nt = (m.a[0].N + BN - 1) / BN;
-  const int tiles = m.nt * ((m.a[0].B + BM - 1) / BM);
-  static constexpr FormText form = form_text("shares ", BM, BN, "");
-  set_last_form(form.s);
-  hipLaunchKernelGGL((gemm_mid_kernel<DT, kMidShare, WM, WN, TM, TN, 1, NS>), dim3(tiles * m.shares), dim3(kMidThreads), lds, st, m);
-  hipLaunchKernelGGL((share_sum_kernel<DT, WN, TM, TN>), dim3(tiles * TM * TN * kMidThreads / 256), dim3(256), 0, st, m, tiles);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }
-  return kOk;
-}
-
 static int64_t mid_tiles(const MfmaArgs& a, int bm, int bn) { return (int64_t)((a.N + bn - 1) / bn) * ((a.B + bm - 1) / bm); }
 static int64_t mid_rounds(int64_t tiles) { return (tiles + compute_units() - 1) / compute_units(); }
 // true when a tiling fills `share` percent of its rounds of one tile per compute unit
@@ -502,73 +416,15 @@ static MidForm mid_form(const MfmaArgs& a, bool dual) {
   if (half * 2 > cu && half <= cu) return kMid128x64Halves;
   return small <= cu && (small * 2 > cu || (small * 4 >= cu && a.K <= 2048)) ? kMid64x64Halves : kMidNone;
 }
-// A long K in shares over workgroups, about one workgroup of the launch per compute unit, their sums in scratch of the call's own
-// (so that calls on different streams stay independent): tiles of 64 x 128 up to 192 rows, 256 x 128
-// from 385 on where they pad no more rows than 128 x 128 do (768 rows of 1536 x 11008 40 us against 45), else 128 x 128 (256 rows 24
-// against 27).  us with weights from HBM, what runs otherwise -> this:
-// K of 8192 and more, always: 1536 x 11008 (64-row tiles of two stages whose last workgroup adds the shares) at 128 / 154 / 256 / 333 /
-// 512 / 768 / 1024 rows 24 -> 20, 30 -> 24, 32 -> 24, 41 -> 28, 45 -> 36, 63 -> 45, 67 -> 47; 1536 x 8192 at 1536 / 2048 (ring of 128 x
-// 128) 71 -> 53, 74 -> 69; 2390 x 11008 at 2048 (128 x 64 tiles; one share) 194 -> 161.  Where no ring takes the shape and 64- or 128-row
-// tiles fill 70 percent of the compute units with it, K is cut as the 64 x 64 tiles cut it, whose bits those rows had before; as many shares
-// as the chip has room for took 19, 20, 23, 26, 32, 39 at the first six of these row counts.
-// K of 4096 to 8191: adding up the shares has to come out of the compute units that work here and not under the ring, i.e. out of
-// gain = shares * area(ring tile) / area(tile), where area counts a workgroup's outputs.
-//   gain 1.5: 128 x 4992 x 4096 22.1 -> 19.6, 333 x 3072 x 4096 25.2 -> 23.7, 768 x 3072 x 4096 38.7 -> 34.8, 1536 x 1500 x 5504 51 -> 41, 640 x 2048 x
-//     5504 36 -> 28.  Taken: from 1.4 on.
-//   gain 1.25, outputs for 90 percent of the compute units and more: 768 x 2048 x 5504 36 -> 32, 1024 x 1500 x 5504 37 -> 32; at a K of 4096, where
-//     the sum weighs more, only 4 percent (512 x 3072 x 4096 28.9 -> 27.7).  Taken: from 1.2 on with a K of 5120 and more.
-//   gain 1.25, a quarter of it padding: 420 x 3072 x 4096 24 -> 28, 200 x 3072 x 4096 17.0 -> 19.5; gain 1: 512 x 4096 x 4096 30.9 -> 31.8.  Not taken.
-//   no ring to compare with: from three shares over 3/16 of the compute units on: 128 x 3072 x 4096 21 -> 16, 154 x 2048 x 5504 22 -> 17.
-struct ShareForm { int bm, shares, per; };
-static ShareForm share_form(const MfmaArgs& a) {
-  const ShareForm none{0, 0, 0};
-  const int64_t cu = compute_units();
-  if (a.scratch_floats == 0 || a.B < 128 || cu <= 0 || a.K < 4096 || a.K % 64 || a.ldx % 8 || a.ldw % 8 || !aligned16(a.x) || !aligned16(a.W) ||
-      !below_4gib(a.B, a.ldx) || !below_4gib(a.N, a.ldw) || gemm_big_apply(a, false))
-    return none;
-  const auto pad = [&](int64_t r) { return (a.B + r - 1) / r * r; };
-  const int steps = a.K / 64;
-  const MidForm ring = mid_form(a, false);
-  // the cut of the 64 x 64 tiles, where a tile of this kernel fills 70 percent of the compute units with it: the same bits
-  if (a.K >= 8192 && ring == kMidNone) {
-    int unit = 1;
-    const int z = gemm_tiles_shares(a, &unit), per = z > 1 ? (steps / unit + z - 1) / z * unit : 0;
-    for (const int bm : {64, 128}) {
-      const int64_t t = mid_tiles(a, bm, 128) * (per ? (steps + per - 1) / per : 0);
-      if (t * 10 >= 7 * cu && t <= cu && (size_t)t * bm * 128 <= a.scratch_floats) return ShareForm{bm, (steps + per - 1) / per, per};
-    }
+bool gemm_mid_apply(const MfmaArgs& a, bool dual) { return mid_form(a, dual) != kMidNone; }
+RingRule gemm_mid_rule(const MfmaArgs& a) {
+  switch (mid_form(a, false)) {
+    case kMid128x128: return RingRule{128 * 128, false};
+    case kMid128x64Halves: return RingRule{128 * 64, true};
+    case kMid64x64Halves: return RingRule{64 * 64, true};
+    default: return RingRule{0, false};
   }
-  const int bm = a.B <= 192 ? 64 : (a.B > 384 && pad(256) <= pad(128) ? 256 : 128);
-  const int64_t tiles = mid_tiles(a, bm, 128), area = (int64_t)bm * 128;
-  int64_t shares = std::min<int64_t>(cu / tiles, steps / 8);                         // eight steps each at least
-  shares = std::min<int64_t>(shares, (int64_t)(a.scratch_floats / (size_t)(tiles * area)));
-  if (a.K < 8192) {
-    const int64_t ring_area = ring == kMid128x128 ? 128 * 128 : (ring == kMid128x64Halves ? 128 * 64 : 64 * 64);
-    const bool full = a.K >= 5120 && (int64_t)a.B * a.N * shares * 10 >= 9 * cu * area;
-    if (ring == kMidNone ? shares < 3 || tiles * 16 < 3 * cu : shares * ring_area * 100 < (full ? 120 : 140) * area) return none;
-  }
-  if (shares < 1) return none;
-  const int per = (steps + (int)shares - 1) / (int)shares;
-  return ShareForm{bm, (steps + per - 1) / per, per};
 }
-// floats of scratch that the call can use, out of at most `cap`
-size_t gemm_share_floats(MfmaArgs a, size_t cap) {
-  a.scratch_floats = cap;
-  const ShareForm f = share_form(a);
-  return f.shares > 0 ? (size_t)f.shares * mid_tiles(a, f.bm, 128) * f.bm * 128 : 0;
-}
-template <int DT>
-static int launch_share_dt(const MfmaArgs& a, const ShareForm& f, hipStream_t st, const char* who) {
-  MidArgs m{};
-  m.a[0] = a;
-  m.shares = f.shares;
-  m.per = f.per;
-  m.part = a.scratch;
-  if (f.bm == 64) return launch_share_t<DT, 4, 2, 2, 5>(m, st, who);
-  return f.bm == 128 ? launch_share_t<DT, 4, 4, 2, 4>(m, st, who) : launch_share_t<DT, 2, 4, 4, 3>(m, st, who);
-}
-
-bool gemm_mid_apply(const MfmaArgs& a, bool dual) { return (!dual && share_form(a).shares > 0) || mid_form(a, dual) != kMidNone; }
 
 template <int DT>
 static int launch_gemm_mid_dt(const MfmaArgs& a, bool dual, hipStream_t st, const char* who) {
@@ -583,8 +439,6 @@ static int launch_gemm_mid_dt(const MfmaArgs& a, bool dual, hipStream_t st, cons
   }
 }
 int launch_gemm_mid(const MfmaArgs& a, bool dual, hipStream_t st, const char* who) {
-  const ShareForm f = dual ? ShareForm{0, 0, 0} : share_form(a);
-  if (f.shares > 0) return a.dt == 1 ? launch_share_dt<1>(a, f, st, who) : launch_share_dt<0>(a, f, st, who);
   return a.dt == 1 ? launch_gemm_mid_dt<1>(a, dual, st, who) : launch_gemm_mid_dt<0>(a, dual, st, who);
 }
 

@@ -1,0 +1,273 @@
+// Projections of prompts on the four-wave tiles of mfma_quad.hpp: which tile a shape gets, the single matrices, the gate / up pair,
+// and long K in shares over workgroups.
+#include "mfma_quad.hpp"
+
+namespace fsvd {
+
+// What a round of workgroups costs in a form, us: f + s per K step of 64; 1: the compute units hold one workgroup each (or fewer), 2: as many
+// as fit.  Fitted to launches with weights from HBM over 195 / 51 / 68 shapes (128 to 16384 rows, 1024 to 4992 columns at K 512 to 4096; the
+// pair 5504 x 768 to 11008 x 2432; 48 and 96 heads at rank 512 to 1664): the form that they name is on average 1 % (worst 20 %, 7 %, 4 %)
+// behind the best of 35 tilings, and 18 / 23 / 17 % ahead of the rings, two-stage tiles and 256 x 256 tiles that ran before.
+struct QuadCost { float f1, s1, f2, s2; };
+static float quad_us(const QuadCost& c, int64_t tiles, int occ, float steps) {
+  const int64_t cu = compute_units(), full = tiles / (cu * occ), rest = tiles - full * cu * occ;
+  float us = (float)full * (c.f2 + c.s2 * steps);
+  if (rest > 0) us += occ == 2 && rest <= cu ? c.f1 + c.s1 * steps : c.f2 + c.s2 * steps;
+  return us;
+}
+static int64_t quad_tiles(const MfmaArgs& a, int tm, int tn) { return (int64_t)((a.N + 32 * tn - 1) / (32 * tn)) * ((a.B + 32 * tm - 1) / (32 * tm)); }
+
+//     form, TM, TN, stages of x and W, workgroups per compute unit, costs
+#define FSVD_QUAD_PLAIN(X) \
+  X(0, 8, 8, 2, 3, 1, 0.f, 0.f, 10.56f, 0.944f) X(1, 8, 6, 2, 3, 1, 0.f, 0.f, 8.22f, 0.757f) X(2, 6, 4, 3, 4, 1, 0.f, 0.f, 4.97f, 0.451f) \
+  X(3, 4, 4, 2, 3, 2, 1.96f, 0.425f, 6.73f, 0.754f) X(4, 4, 4, 4, 5, 1, 0.f, 0.f, 3.24f, 0.354f) X(5, 4, 2, 3, 4, 2, 1.32f, 0.249f, 2.24f, 0.570f) \
+  X(6, 2, 4, 3, 4, 1, 0.f, 0.f, 1.66f, 0.262f) X(7, 3, 2, 3, 4, 2, 0.88f, 0.218f, 1.78f, 0.448f) X(8, 2, 2, 4, 4, 2, 0.82f, 0.177f, 1.56f, 0.354f)
+#define FSVD_QUAD_PAIR(X) \
+  X(0, 4, 6, 3, 4, 1, 0.f, 0.f, 7.57f, 0.563f) X(1, 5, 4, 2, 2, 2, 1.88f, 0.697f, 10.04f, 0.892f) X(2, 4, 4, 2, 3, 2, 1.21f, 0.544f, 7.93f, 0.747f) \
+  X(3, 4, 4, 4, 5, 1, 0.f, 0.f, 5.57f, 0.410f) X(4, 3, 6, 2, 2, 2, 2.05f, 0.680f, 8.78f, 0.889f) X(5, 3, 6, 3, 4, 1, 0.f, 0.f, 5.59f, 0.463f) \
+  X(6, 3, 3, 3, 3, 2, 1.96f, 0.328f, 3.08f, 0.570f) X(7, 2, 3, 3, 4, 2, 0.96f, 0.268f, 1.43f, 0.463f)
+// ragged rows: tiles with two workgroups per compute unit
+#define FSVD_QUAD_PLAIN_ANY(X) X(3, 4, 4, 2, 3, 2, 0, 0, 0, 0) X(7, 3, 2, 3, 4, 2, 0, 0, 0, 0) X(8, 2, 2, 4, 4, 2, 0, 0, 0, 0)
+#define FSVD_QUAD_PAIR_ANY(X) X(2, 4, 4, 2, 3, 2, 0, 0, 0, 0) X(6, 3, 3, 3, 3, 2, 0, 0, 0, 0) X(7, 2, 3, 3, 4, 2, 0, 0, 0, 0)
+
+constexpr int kQuadNone = -1;
+struct QuadPick { int form; float us; };
+// The order of a single matrix's sums is the one that its shape had on the tiles before these (rings with K halved between waves, 64 x 64
+// tiles with K cut over workgroups), so that the bits stay: a model of 32 layers hands a flipped rounding on until another order of
+// the same sums ends 0.046 (relative) away.  Both cost nothing here: a second set of accumulators, a sum kept in registers.
+enum QuadOrder { kOrderPlain = 0, kOrderHalves = 1, kOrderCut = 2 };
+struct QuadSums { QuadOrder order; int per; };
+static QuadSums quad_sums(const MfmaArgs& a) {
+  if (gemm_big_apply(a, false)) return QuadSums{kOrderPlain, 0};
+  const RingRule r = gemm_mid_rule(a);
+  if (r.area > 0) return QuadSums{r.halves ? kOrderHalves : kOrderPlain, 0};
+  const int per = gemm_tiles_cut(a);
+  return per > 0 ? QuadSums{kOrderCut, per} : QuadSums{kOrderPlain, 0};
+}
+static QuadPick quad_pick(const MfmaArgs& a, bool dual, bool any, QuadOrder order = kOrderPlain) {
+  if (order == kOrderCut) return QuadPick{8, 0.f};                                   // few 64 x 64 tiles by that rule
+  QuadPick best{kQuadNone, 0.f};
+  const float steps = (float)((a.K + 63) / 64 * (dual ? 2 : 1));
+  const auto take = [&](int form, int tm, int tn, int occ, const QuadCost& c) {
+    const float us = quad_us(c, quad_tiles(a, tm, tn), occ, steps);
+    if (best.form == kQuadNone || us < best.us) best = QuadPick{form, us};
+  };
+  if (dual) {
+#define X(n, TM, TN, SX, SW, OCC, F1, S1, F2, S2) if (!any || (OCC == 2 && (n == 2 || n >= 6))) take(n, TM, TN, OCC, QuadCost{F1, S1, F2, S2});
+    FSVD_QUAD_PAIR(X)
+#undef X
+  } else {
+    // 96 x 64 is left out for a K of 4096 and more: 64 x 64 and 128 x 64 are within 6 % of it or ahead there (3072 columns at 154, 333,
+    // 420, 512 rows 22.4, 22.4, 22.2, 27.5 against 17.8, 22.0, 23.7, 27.1), below it is the best tile of 333 rows (4096 x 1536 9.7 against 10.5)
+#define X(n, TM, TN, SX, SW, OCC, F1, S1, F2, S2) if ((!any || n == 3 || n >= 7) && (n != 7 || a.K < 4096) && (order == kOrderPlain || n >= 3)) take(n, TM, TN, OCC, QuadCost{F1, S1, F2, S2});
+    FSVD_QUAD_PLAIN(X)
+#undef X
+  }
+  return best;
+}
+
+// rows of whole pieces that start on the 16-byte grid, K of whole steps
+static bool quad_grid(const MfmaArgs& a, bool dual) {
+  return a.K % 64 == 0 && a.ldx % 8 == 0 && a.ldw % 8 == 0 && a.up_off % 8 == 0 && aligned16(a.x) && aligned16(a.W) && (!dual || aligned16(a.W2));
+}
+// rows on the 4-byte grid, which is what a 16-byte load asks of its address
+static bool quad_words(const MfmaArgs& a, bool dual) {
+  const auto al4 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 3) == 0; };
+  return a.ldx % 2 == 0 && a.ldw % 2 == 0 && a.up_off % 2 == 0 && al4(a.x) && al4(a.W) && (!dual || al4(a.W2));
+}
+// From 128 rows and five K steps on (fewer steps than the stages hold are left to the tiles that were measured for them); N holds a whole
+// residual piece.  The pair in the rounding that keeps the gate in 32 bits goes to mfma_mid.hip.
+static bool quad_range(const MfmaArgs& a, bool dual) {
+  return a.B >= 128 && a.K >= 320 && a.N >= 8 && compute_units() > 0 && (!dual || a.mode == 0) && below_4gib(a.B, a.ldx) && below_4gib(a.N, a.ldw);
+}
+
+// A long K in shares over workgroups, about one workgroup of the launch per compute unit, their sums in scratch of the call's own
+// (so that calls on different streams stay independent): tiles of 64 x 128 up to 192 rows, 256 x 128
+// from 385 on where they pad no more rows than 128 x 128 do (768 rows of 1536 x 11008 40 us against 45), else 128 x 128 (256 rows 24
+// against 27).  us with weights from HBM, what runs otherwise -> this:
+// K of 8192 and more, always: 1536 x 11008 (64-row tiles of two stages whose last workgroup adds the shares) at 128 / 154 / 256 / 333 /
+// 512 / 768 / 1024 rows 24 -> 20, 30 -> 24, 32 -> 24, 41 -> 28, 45 -> 36, 63 -> 45, 67 -> 47; 1536 x 8192 at 1536 / 2048 (ring of 128 x
+// 128) 71 -> 53, 74 -> 69; 2390 x 11008 at 2048 (128 x 64 tiles; one share) 194 -> 161.  Where no ring takes the shape and 64- or 128-row
+// tiles fill 70 percent of the compute units with it, K is cut as the 64 x 64 tiles cut it, whose bits those rows had before; as many shares
+// as the chip has room for took 19, 20, 23, 26, 32, 39 at the first six of these row counts.
+// K of 4096 to 8191: adding up the shares has to come out of the compute units that work here and not under the ring, i.e. out of
+// gain = shares * area(ring tile) / area(tile), where area counts a workgroup's outputs.
+//   gain 1.5: 128 x 4992 x 4096 22.1 -> 19.6, 333 x 3072 x 4096 25.2 -> 23.7, 768 x 3072 x 4096 38.7 -> 34.8, 1536 x 1500 x 5504 51 -> 41, 640 x 2048 x
+//     5504 36 -> 28.  Taken: from 1.4 on.
+//   gain 1.25, outputs for 90 percent of the compute units and more: 768 x 2048 x 5504 36 -> 32, 1024 x 1500 x 5504 37 -> 32; at a K of 4096, where
+//     the sum weighs more, only 4 percent (512 x 3072 x 4096 28.9 -> 27.7).  Taken: from 1.2 on with a K of 5120 and more.
+//   gain 1.25, a quarter of it padding: 420 x 3072 x 4096 24 -> 28, 200 x 3072 x 4096 17.0 -> 19.5; gain 1: 512 x 4096 x 4096 30.9 -> 31.8.  Not taken.
+//   no ring to compare with: from three shares over 3/16 of the compute units on: 128 x 3072 x 4096 21 -> 16, 154 x 2048 x 5504 22 -> 17.
+struct ShareForm { int bm, shares, per; };
+static ShareForm share_form(const MfmaArgs& a) {
+  const ShareForm none{0, 0, 0};
+  const int64_t cu = compute_units();
+  if (a.scratch_floats == 0 || a.K < 4096 || !quad_range(a, false) || !quad_grid(a, false) || gemm_big_apply(a, false)) return none;
+  const auto pad = [&](int64_t r) { return (a.B + r - 1) / r * r; };
+  const int steps = a.K / 64;
+  const RingRule ring = gemm_mid_rule(a);
+  // the cut of the 64 x 64 tiles, where a tile of this kernel fills 70 percent of the compute units with it: the same bits
+  if (a.K >= 8192 && ring.area == 0) {
+    int unit = 1;
+    const int z = gemm_tiles_shares(a, &unit), per = z > 1 ? (steps / unit + z - 1) / z * unit : 0;
+    for (const int bm : {64, 128}) {
+      const int64_t t = quad_tiles(a, bm / 32, 4) * (per ? (steps + per - 1) / per : 0);
+      if (t * 10 >= 7 * cu && t <= cu && (size_t)t * bm * 128 <= a.scratch_floats) return ShareForm{bm, (steps + per - 1) / per, per};
+    }
+  }
+  const int bm = a.B <= 192 ? 64 : (a.B > 384 && pad(256) <= pad(128) ? 256 : 128);
+  const int64_t tiles = quad_tiles(a, bm / 32, 4), area = (int64_t)bm * 128;
+  int64_t shares = std::min<int64_t>(cu / tiles, steps / 8);                         // eight steps each at least
+  shares = std::min<int64_t>(shares, (int64_t)(a.scratch_floats / (size_t)(tiles * area)));
+  if (a.K < 8192) {
+    const bool full = a.K >= 5120 && (int64_t)a.B * a.N * shares * 10 >= 9 * cu * area;
+    if (ring.area == 0 ? shares < 3 || tiles * 16 < 3 * cu : shares * ring.area * 100 < (full ? 120 : 140) * area) return none;
+  }
+  if (shares < 1) return none;
+  const int per = (steps + (int)shares - 1) / (int)shares;
+  return ShareForm{bm, (steps + per - 1) / per, per};
+}
+// floats of scratch that the call can use, out of at most `cap`
+size_t gemm_share_floats(MfmaArgs a, size_t cap) {
+  a.scratch_floats = cap;
+  const ShareForm f = share_form(a);
+  return f.shares > 0 ? (size_t)f.shares * quad_tiles(a, f.bm / 32, 4) * f.bm * 128 : 0;
+}
+
+// The shares of every tile, added in their order, and the epilogue of a single matrix: one thread per four columns of a row, as the
+// accumulators hold them.  A launch of its own: the shares need no counters, and all compute units add.
+template <int DT, int TM, int TN>
+__global__ __launch_bounds__(256) void share_sum_kernel(QuadArgs args, int tiles) {
+  typedef E16<DT> E;
+  constexpr int kWords = TM * TN * kQuadThreads, BM = 32 * TM, BN = 32 * TN;
+  const MfmaArgs& a = args.a[0];
+  const int g = blockIdx.x * 256 + threadIdx.x, t = g / kWords, r = g - t * kWords;
+  const f32x4_t* part = reinterpret_cast<const f32x4_t*>(args.part) + (size_t)t * args.shares * kWords + r;
+  f32x4_t v = part[0];
+  int z = 1;
+  for (; z + 4 <= args.shares; z += 4) {               // four shares on their way at a time
+    f32x4_t w[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) w[u] = part[(size_t)(z + u) * kWords];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v += w[u];
+  }
+  for (; z < args.shares; ++z) v += part[(size_t)z * kWords];
+  const int ij = r / kQuadThreads, tid = r - ij * kQuadThreads, i = ij / TN, j = ij - i * TN, wave = tid >> 6, lane = tid & 63;
+  const int NT = args.nt, band = t / (8 * NT), tb = t - band * 8 * NT, bh = min(8, args.mt - band * 8), col = tb / bh;
+  const int m = (band * 8 + tb - col * bh) * BM + (wave >> 1) * 16 * TM + i * 16 + (lane & 15);
+  const int n = col * BN + (wave & 1) * 16 * TN + j * 16 + (lane >> 4) * 4;
+  if (m >= a.B || n >= a.N) return;
+  const uint16_t* res = a.res ? a.res + (int64_t)m * a.ldres + n : nullptr;
+  uint16_t* y = a.y + (int64_t)m * a.ldy + n;
+  uint32_t o[2];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (a.bias && n + e < a.N) v[e] += E::val(a.bias[n + e]);
+  }
+  o[0] = E::pack2(v[0], v[1]);
+  o[1] = E::pack2(v[2], v[3]);
+  const bool whole = n + 3 < a.N;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (res && n + e < a.N) v[e] = E::val(res[e]) + E::val((o[e >> 1] >> (16 * (e & 1))) & 0xffffu);
+  }
+  if (res) {
+    o[0] = E::pack2(v[0], v[1]);
+    o[1] = E::pack2(v[2], v[3]);
+  }
+  if (whole && (reinterpret_cast<uintptr_t>(y) & 7) == 0) {
+    *reinterpret_cast<u32x2_t*>(y) = u32x2_t{o[0], o[1]};
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < a.N) y[e] = (uint16_t)(o[e >> 1] >> (16 * (e & 1)));
+  }
+}
+template <int DT, int TM, int NSX, int NSW>
+static int launch_share_t(QuadArgs& q, hipStream_t st, const char* who) {
+  const int rc = launch_quad_t<DT, kQuadShare, TM, 4, NSX, NSW, 1>(q, st, who);
+  if (rc != kOk) return rc;
+  const int tiles = q.nt * q.mt;
+  hipLaunchKernelGGL((share_sum_kernel<DT, TM, 4>), dim3(tiles * TM * 4 * kQuadThreads / 256), dim3(256), 0, st, q, tiles);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }
+  return kOk;
+}
+template <int DT>
+static int launch_share_dt(QuadArgs& q, int bm, hipStream_t st, const char* who) {
+  if (bm == 64) return launch_share_t<DT, 2, 3, 4>(q, st, who);
+  return bm == 128 ? launch_share_t<DT, 4, 4, 5>(q, st, who) : launch_share_t<DT, 8, 3, 3>(q, st, who);
+}
+
+// The 256 x 256 pair of mfma_big.hip keeps what its larger tile still does better: 11008 x 2432 at 16384 rows 1602 us, here 1617 at best
+// (8192 rows 874 against 780); its cost in the same terms.
+static bool big_pair_is_ahead(const MfmaArgs& a, float us) {
+  return gemm_big_apply(a, true) && quad_us(QuadCost{0.f, 0.f, 26.7f, 1.564f}, quad_tiles(a, 8, 8), 1, (float)(a.K / 32)) < us;
+}
+
+bool gemm_quad_apply(const MfmaArgs& a, bool dual) {
+  if (!quad_range(a, dual)) return false;
+  if (quad_grid(a, dual)) return !dual || !big_pair_is_ahead(a, quad_pick(a, true, false).us);
+  return quad_words(a, dual);
+}
+
+template <int DT>
+static int launch_gemm_quad_dt(const MfmaArgs& a, bool dual, hipStream_t st, const char* who) {
+  QuadArgs q{};
+  q.a[0] = a;
+  const bool any = !quad_grid(a, dual);
+  if (!dual && !any) {
+    const ShareForm f = share_form(a);
+    if (f.shares > 0) {
+      q.shares = f.shares;
+      q.per = f.per;
+      q.part = a.scratch;
+      return launch_share_dt<DT>(q, f.bm, st, who);
+    }
+  }
+  const QuadSums sums = dual || any ? QuadSums{kOrderPlain, 0} : quad_sums(a);
+  const int form = quad_pick(a, dual, any, sums.order).form;
+#define FSVD_QUAD_CASE(EPI, RAG, n, TM, TN, SX, SW, OCC) case n: return launch_quad_t<DT, EPI, TM, TN, SX, SW, OCC, RAG>(q, st, who);
+  if (dual && any) {
+    switch (form) {
+#define X(n, TM, TN, SX, SW, OCC, ...) FSVD_QUAD_CASE(kQuadPair, true, n, TM, TN, SX, SW, OCC)
+      FSVD_QUAD_PAIR_ANY(X)
+#undef X
+    }
+  } else if (dual) {
+    switch (form) {
+#define X(n, TM, TN, SX, SW, OCC, ...) FSVD_QUAD_CASE(kQuadPair, false, n, TM, TN, SX, SW, OCC)
+      FSVD_QUAD_PAIR(X)
+#undef X
+    }
+  } else if (any) {
+    switch (form) {
+#define X(n, TM, TN, SX, SW, OCC, ...) FSVD_QUAD_CASE(kQuadPlain, true, n, TM, TN, SX, SW, OCC)
+      FSVD_QUAD_PLAIN_ANY(X)
+#undef X
+    }
+  } else if (sums.order == kOrderCut) {
+    q.per = sums.per;
+    return launch_quad_t<DT, kQuadPlain, 2, 2, 4, 4, 2, false, 1, true>(q, st, who);
+  } else if (sums.order == kOrderHalves) {
+    switch (form) {
+#define X(n, TM, TN, SX, SW, OCC, ...) case n: if constexpr (n >= 3) return launch_quad_t<DT, kQuadPlain, TM, TN, SX, SW, OCC, false, 2>(q, st, who); break;
+      FSVD_QUAD_PLAIN(X)
+#undef X
+    }
+  } else {
+    switch (form) {
+#define X(n, TM, TN, SX, SW, OCC, ...) FSVD_QUAD_CASE(kQuadPlain, false, n, TM, TN, SX, SW, OCC)
+      FSVD_QUAD_PLAIN(X)
+#undef X
+    }
+  }
+  set_last_error("%s: no tile for %d x %d x %d", who, a.B, a.N, a.K);
+  return kErrBadShape;
+}
+int launch_gemm_quad(const MfmaArgs& a, bool dual, hipStream_t st, const char* who) {
+  return a.dt == 1 ? launch_gemm_quad_dt<1>(a, dual, st, who) : launch_gemm_quad_dt<0>(a, dual, st, who);
+}
+
+}  // namespace fsvd
