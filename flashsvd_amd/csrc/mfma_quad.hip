@@ -5,10 +5,11 @@
 namespace fsvd {
 
 // What a round of workgroups costs in a form, us: f + s per K step of 64; 1: the compute units hold one workgroup each (or fewer), 2: as many
-// as fit.  Fitted to launches with weights from HBM over 195 / 51 / 68 shapes (128 to 16384 rows, 1024 to 4992 columns at K 512 to 4096; the
-// pair 5504 x 768 to 11008 x 2432; 48 and 96 heads at rank 512 to 1664): the form that they name is on average 1 % (worst 20 %, 7 %, 4 %)
-// behind the best of 35 tilings, and 18 / 23 / 17 % ahead of the rings, two-stage tiles and 256 x 256 tiles that ran before.
+// as fit.  Fitted to launches with weights from HBM (more of them in turn than the 256 MB in front of it hold) over 125 / 49 / 39 shapes
+// (154 to 16384 rows; 1024 to 4096 columns at K 768 to 4096; the pair 5504 x 768 to 11008 x 2432; 48 and 96 heads at rank 512 and 1024):
+// the form that they name is on average 2 / 1 / 1 % (at worst 20, 12, 8 %) behind the best of about 30 tilings.
 struct QuadCost { float f1, s1, f2, s2; };
+constexpr float kLaunchUs = 3.f;
 static float quad_us(const QuadCost& c, int64_t tiles, int occ, float steps) {
   const int64_t cu = compute_units(), full = tiles / (cu * occ), rest = tiles - full * cu * occ;
   float us = (float)full * (c.f2 + c.s2 * steps);
@@ -19,16 +20,19 @@ static int64_t quad_tiles(const MfmaArgs& a, int tm, int tn) { return (int64_t)(
 
 //     form, TM, TN, stages of x and W, workgroups per compute unit, costs
 #define FSVD_QUAD_PLAIN(X) \
-  X(0, 8, 8, 2, 3, 1, 0.f, 0.f, 10.56f, 0.944f) X(1, 8, 6, 2, 3, 1, 0.f, 0.f, 8.22f, 0.757f) X(2, 6, 4, 3, 4, 1, 0.f, 0.f, 4.97f, 0.451f) \
-  X(3, 4, 4, 2, 3, 2, 1.96f, 0.425f, 6.73f, 0.754f) X(4, 4, 4, 4, 5, 1, 0.f, 0.f, 3.24f, 0.354f) X(5, 4, 2, 3, 4, 2, 1.32f, 0.249f, 2.24f, 0.570f) \
-  X(6, 2, 4, 3, 4, 1, 0.f, 0.f, 1.66f, 0.262f) X(7, 3, 2, 3, 4, 2, 0.88f, 0.218f, 1.78f, 0.448f) X(8, 2, 2, 4, 4, 2, 0.82f, 0.177f, 1.56f, 0.354f)
+  X(0, 8, 8, 2, 3, 1, 0.f, 0.f, 11.21f, 0.952f) X(1, 8, 6, 2, 3, 1, 0.f, 0.f, 8.57f, 0.783f) X(2, 4, 6, 3, 4, 1, 0.f, 0.f, 4.35f, 0.578f) \
+  X(3, 8, 4, 2, 3, 1, 0.f, 0.f, 5.97f, 0.643f) X(4, 6, 4, 3, 4, 1, 0.f, 0.f, 4.84f, 0.502f) X(5, 4, 4, 2, 3, 2, 1.53f, 0.533f, 8.67f, 0.679f) \
+  X(6, 4, 4, 4, 5, 1, 0.f, 0.f, 3.03f, 0.450f) X(7, 4, 3, 5, 6, 1, 0.f, 0.f, 4.29f, 0.353f) X(8, 4, 2, 3, 4, 2, 0.57f, 0.339f, 3.94f, 0.568f) \
+  X(9, 2, 4, 3, 4, 1, 0.f, 0.f, 1.24f, 0.354f) X(10, 3, 2, 3, 4, 2, 0.24f, 0.297f, 3.14f, 0.440f) X(11, 2, 3, 3, 4, 2, 0.30f, 0.311f, 1.99f, 0.484f) \
+  X(12, 2, 2, 5, 5, 2, 0.49f, 0.227f, 2.66f, 0.355f)
+constexpr int kHalvesFrom = 5;                       // forms with registers for a second set of accumulators
 #define FSVD_QUAD_PAIR(X) \
-  X(0, 4, 6, 3, 4, 1, 0.f, 0.f, 7.57f, 0.563f) X(1, 5, 4, 2, 2, 2, 1.88f, 0.697f, 10.04f, 0.892f) X(2, 4, 4, 2, 3, 2, 1.21f, 0.544f, 7.93f, 0.747f) \
-  X(3, 4, 4, 4, 5, 1, 0.f, 0.f, 5.57f, 0.410f) X(4, 3, 6, 2, 2, 2, 2.05f, 0.680f, 8.78f, 0.889f) X(5, 3, 6, 3, 4, 1, 0.f, 0.f, 5.59f, 0.463f) \
-  X(6, 3, 3, 3, 3, 2, 1.96f, 0.328f, 3.08f, 0.570f) X(7, 2, 3, 3, 4, 2, 0.96f, 0.268f, 1.43f, 0.463f)
+  X(0, 4, 6, 3, 4, 1, 0.f, 0.f, 8.19f, 0.657f) X(1, 5, 6, 2, 3, 1, 0.f, 0.f, 9.82f, 0.693f) X(2, 5, 4, 2, 2, 2, 4.26f, 0.861f, 8.46f, 0.970f) \
+  X(3, 8, 4, 2, 3, 1, 0.f, 0.f, 10.88f, 0.710f) X(4, 4, 4, 2, 3, 2, 3.94f, 0.589f, 7.43f, 0.802f) X(5, 4, 4, 4, 5, 1, 0.f, 0.f, 6.31f, 0.487f) \
+  X(6, 3, 6, 3, 4, 1, 0.f, 0.f, 6.98f, 0.562f) X(7, 3, 3, 3, 3, 2, 1.93f, 0.444f, 4.61f, 0.652f) X(8, 2, 3, 3, 4, 2, 2.96f, 0.273f, 2.34f, 0.547f)
 // ragged rows: tiles with two workgroups per compute unit
-#define FSVD_QUAD_PLAIN_ANY(X) X(3, 4, 4, 2, 3, 2, 0, 0, 0, 0) X(7, 3, 2, 3, 4, 2, 0, 0, 0, 0) X(8, 2, 2, 4, 4, 2, 0, 0, 0, 0)
-#define FSVD_QUAD_PAIR_ANY(X) X(2, 4, 4, 2, 3, 2, 0, 0, 0, 0) X(6, 3, 3, 3, 3, 2, 0, 0, 0, 0) X(7, 2, 3, 3, 4, 2, 0, 0, 0, 0)
+#define FSVD_QUAD_PLAIN_ANY(X) X(5, 4, 4, 2, 3, 2) X(10, 3, 2, 3, 4, 2) X(12, 2, 2, 4, 4, 2)
+#define FSVD_QUAD_PAIR_ANY(X) X(4, 4, 4, 2, 3, 2) X(7, 3, 3, 3, 3, 2) X(8, 2, 3, 3, 4, 2)
 
 constexpr int kQuadNone = -1;
 struct QuadPick { int form; float us; };
@@ -45,7 +49,7 @@ static QuadSums quad_sums(const MfmaArgs& a) {
   return per > 0 ? QuadSums{kOrderCut, per} : QuadSums{kOrderPlain, 0};
 }
 static QuadPick quad_pick(const MfmaArgs& a, bool dual, bool any, QuadOrder order = kOrderPlain) {
-  if (order == kOrderCut) return QuadPick{8, 0.f};                                   // few 64 x 64 tiles by that rule
+  if (order == kOrderCut) return QuadPick{12, 0.f};                                  // few 64 x 64 tiles by that rule
   QuadPick best{kQuadNone, 0.f};
   const float steps = (float)((a.K + 63) / 64 * (dual ? 2 : 1));
   const auto take = [&](int form, int tm, int tn, int occ, const QuadCost& c) {
@@ -53,13 +57,19 @@ static QuadPick quad_pick(const MfmaArgs& a, bool dual, bool any, QuadOrder orde
     if (best.form == kQuadNone || us < best.us) best = QuadPick{form, us};
   };
   if (dual) {
-#define X(n, TM, TN, SX, SW, OCC, F1, S1, F2, S2) if (!any || (OCC == 2 && (n == 2 || n >= 6))) take(n, TM, TN, OCC, QuadCost{F1, S1, F2, S2});
+#define X(n, TM, TN, SX, SW, OCC, F1, S1, F2, S2) if (!any || n == 4 || n >= 7) take(n, TM, TN, OCC, QuadCost{F1, S1, F2, S2});
     FSVD_QUAD_PAIR(X)
 #undef X
   } else {
     // 96 x 64 is left out for a K of 4096 and more: 64 x 64 and 128 x 64 are within 6 % of it or ahead there (3072 columns at 154, 333,
-    // 420, 512 rows 22.4, 22.4, 22.2, 27.5 against 17.8, 22.0, 23.7, 27.1), below it is the best tile of 333 rows (4096 x 1536 9.7 against 10.5)
-#define X(n, TM, TN, SX, SW, OCC, F1, S1, F2, S2) if ((!any || n == 3 || n >= 7) && (n != 7 || a.K < 4096) && (order == kOrderPlain || n >= 3)) take(n, TM, TN, OCC, QuadCost{F1, S1, F2, S2});
+    // 420, 512 rows 22.5, 22.2, 22.2, 27.6 against 17.9, 21.5, 23.7, 27.2), below it is the best tile of 333 rows (4096 x 1536 11.4 against
+    // 12.8).  64 x 96 comes in where it pads nothing (512 x 3072 x 4096 24.5 against 27.2; 420 rows 23.6 against 23.7).
+    const auto fits = [&](int n) {
+      if (any) return n == 5 || n == 10 || n == 12;
+      if (n < kHalvesFrom && order != kOrderPlain) return false;
+      return n == 10 ? a.K < 4096 : (n == 11 ? a.B % 64 == 0 && a.N % 96 == 0 : true);
+    };
+#define X(n, TM, TN, SX, SW, OCC, F1, S1, F2, S2) if (fits(n)) take(n, TM, TN, OCC, QuadCost{F1, S1, F2, S2});
     FSVD_QUAD_PLAIN(X)
 #undef X
   }
@@ -98,21 +108,30 @@ static bool quad_range(const MfmaArgs& a, bool dual) {
 //     the sum weighs more, only 4 percent (512 x 3072 x 4096 28.9 -> 27.7).  Taken: from 1.2 on with a K of 5120 and more.
 //   gain 1.25, a quarter of it padding: 420 x 3072 x 4096 24 -> 28, 200 x 3072 x 4096 17.0 -> 19.5; gain 1: 512 x 4096 x 4096 30.9 -> 31.8.  Not taken.
 //   no ring to compare with: from three shares over 3/16 of the compute units on: 128 x 3072 x 4096 21 -> 16, 154 x 2048 x 5504 22 -> 17.
-struct ShareForm { int bm, shares, per; };
+struct ShareForm { int bm, bn, shares, per; };
 static ShareForm share_form(const MfmaArgs& a) {
-  const ShareForm none{0, 0, 0};
+  const ShareForm none{0, 0, 0, 0};
   const int64_t cu = compute_units();
   if (a.scratch_floats == 0 || a.K < 4096 || !quad_range(a, false) || !quad_grid(a, false) || gemm_big_apply(a, false)) return none;
   const auto pad = [&](int64_t r) { return (a.B + r - 1) / r * r; };
   const int steps = a.K / 64;
   const RingRule ring = gemm_mid_rule(a);
+  // K cut in ranges (see quad_sums): one workgroup per range and 64 x 64 tile where that beats one after the other (512 x 1024 x 4096 in two
+  // ranges 19.6 -> 16.4 us, 154 x 1024 x 4096 in six 18.6 -> 12.1)
+  const QuadSums sums = quad_sums(a);
+  if (sums.order == kOrderCut) {
+    const int64_t tiles = quad_tiles(a, 2, 2), shares = (steps + sums.per - 1) / sums.per;
+    const QuadCost c{0.49f, 0.227f, 2.66f, 0.355f};
+    const float apart = quad_us(c, tiles * shares, 2, (float)sums.per) + 3.5f + (float)(shares * tiles * 4096) * 8.f / 4.5e6f;
+    if (apart < quad_us(c, tiles, 2, (float)steps) && (size_t)(tiles * shares * 4096) <= a.scratch_floats) return ShareForm{64, 64, (int)shares, sums.per};
+  }
   // the cut of the 64 x 64 tiles, where a tile of this kernel fills 70 percent of the compute units with it: the same bits
   if (a.K >= 8192 && ring.area == 0) {
     int unit = 1;
     const int z = gemm_tiles_shares(a, &unit), per = z > 1 ? (steps / unit + z - 1) / z * unit : 0;
     for (const int bm : {64, 128}) {
       const int64_t t = quad_tiles(a, bm / 32, 4) * (per ? (steps + per - 1) / per : 0);
-      if (t * 10 >= 7 * cu && t <= cu && (size_t)t * bm * 128 <= a.scratch_floats) return ShareForm{bm, (steps + per - 1) / per, per};
+      if (t * 10 >= 7 * cu && t <= cu && (size_t)t * bm * 128 <= a.scratch_floats) return ShareForm{bm, 128, (steps + per - 1) / per, per};
     }
   }
   const int bm = a.B <= 192 ? 64 : (a.B > 384 && pad(256) <= pad(128) ? 256 : 128);
@@ -125,13 +144,21 @@ static ShareForm share_form(const MfmaArgs& a) {
   }
   if (shares < 1) return none;
   const int per = (steps + (int)shares - 1) / (int)shares;
-  return ShareForm{bm, (steps + per - 1) / per, per};
+  shares = (steps + per - 1) / per;
+  // the sums once out and once in, and the launch that adds them; 333 x 1664 x 4096 19.7 us in shares, 16.1 unsplit (here too a K below 5120 only:
+  // the longer ones were ahead in shares at every row count)
+  if (a.K < 5120) {
+    const QuadCost c = bm == 64 ? QuadCost{0.f, 0.f, 1.24f, 0.354f} : (bm == 128 ? QuadCost{0.f, 0.f, 3.03f, 0.450f} : QuadCost{0.f, 0.f, 6.65f, 0.634f});
+    const float us = c.f2 + c.s2 * (float)per + 3.5f + (float)(shares * tiles * area) * 8.f / 4.5e6f;
+    if (kLaunchUs + quad_pick(a, false, false).us < 0.9f * (kLaunchUs + us)) return none;
+  }
+  return ShareForm{bm, 128, (int)shares, per};
 }
 // floats of scratch that the call can use, out of at most `cap`
 size_t gemm_share_floats(MfmaArgs a, size_t cap) {
   a.scratch_floats = cap;
   const ShareForm f = share_form(a);
-  return f.shares > 0 ? (size_t)f.shares * quad_tiles(a, f.bm / 32, 4) * f.bm * 128 : 0;
+  return f.shares > 0 ? (size_t)f.shares * quad_tiles(a, f.bm / 32, f.bn / 32) * f.bm * f.bn : 0;
 }
 
 // The shares of every tile, added in their order, and the epilogue of a single matrix: one thread per four columns of a row, as the
@@ -184,24 +211,25 @@ __global__ __launch_bounds__(256) void share_sum_kernel(QuadArgs args, int tiles
       if (n + e < a.N) y[e] = (uint16_t)(o[e >> 1] >> (16 * (e & 1)));
   }
 }
-template <int DT, int TM, int NSX, int NSW>
+template <int DT, int TM, int TN, int NSX, int NSW, int OCC>
 static int launch_share_t(QuadArgs& q, hipStream_t st, const char* who) {
-  const int rc = launch_quad_t<DT, kQuadShare, TM, 4, NSX, NSW, 1>(q, st, who);
+  const int rc = launch_quad_t<DT, kQuadShare, TM, TN, NSX, NSW, OCC>(q, st, who);
   if (rc != kOk) return rc;
   const int tiles = q.nt * q.mt;
-  hipLaunchKernelGGL((share_sum_kernel<DT, TM, 4>), dim3(tiles * TM * 4 * kQuadThreads / 256), dim3(256), 0, st, q, tiles);
+  hipLaunchKernelGGL((share_sum_kernel<DT, TM, TN>), dim3(tiles * TM * TN * kQuadThreads / 256), dim3(256), 0, st, q, tiles);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }
   return kOk;
 }
 template <int DT>
-static int launch_share_dt(QuadArgs& q, int bm, hipStream_t st, const char* who) {
-  if (bm == 64) return launch_share_t<DT, 2, 3, 4>(q, st, who);
-  return bm == 128 ? launch_share_t<DT, 4, 4, 5>(q, st, who) : launch_share_t<DT, 8, 3, 3>(q, st, who);
+static int launch_share_dt(QuadArgs& q, const ShareForm& f, hipStream_t st, const char* who) {
+  if (f.bn == 64) return launch_share_t<DT, 2, 2, 5, 5, 2>(q, st, who);
+  if (f.bm == 64) return launch_share_t<DT, 2, 4, 3, 4, 1>(q, st, who);
+  return f.bm == 128 ? launch_share_t<DT, 4, 4, 4, 5, 1>(q, st, who) : launch_share_t<DT, 8, 4, 3, 3, 1>(q, st, who);
 }
 
 // The 256 x 256 pair of mfma_big.hip keeps what its larger tile still does better: 11008 x 2432 at 16384 rows 1602 us, here 1617 at best
-// (8192 rows 874 against 780); its cost in the same terms.
+// (8192 rows 874 against 780, its rounds being few and large); its cost in the same terms.
 static bool big_pair_is_ahead(const MfmaArgs& a, float us) {
   return gemm_big_apply(a, true) && quad_us(QuadCost{0.f, 0.f, 26.7f, 1.564f}, quad_tiles(a, 8, 8), 1, (float)(a.K / 32)) < us;
 }
@@ -223,7 +251,7 @@ static int launch_gemm_quad_dt(const MfmaArgs& a, bool dual, hipStream_t st, con
       q.shares = f.shares;
       q.per = f.per;
       q.part = a.scratch;
-      return launch_share_dt<DT>(q, f.bm, st, who);
+      return launch_share_dt<DT>(q, f, st, who);
     }
   }
   const QuadSums sums = dual || any ? QuadSums{kOrderPlain, 0} : quad_sums(a);
@@ -249,10 +277,10 @@ static int launch_gemm_quad_dt(const MfmaArgs& a, bool dual, hipStream_t st, con
     }
   } else if (sums.order == kOrderCut) {
     q.per = sums.per;
-    return launch_quad_t<DT, kQuadPlain, 2, 2, 4, 4, 2, false, 1, true>(q, st, who);
+    return launch_quad_t<DT, kQuadPlain, 2, 2, 5, 5, 2, false, 1, true>(q, st, who);
   } else if (sums.order == kOrderHalves) {
     switch (form) {
-#define X(n, TM, TN, SX, SW, OCC, ...) case n: if constexpr (n >= 3) return launch_quad_t<DT, kQuadPlain, TM, TN, SX, SW, OCC, false, 2>(q, st, who); break;
+#define X(n, TM, TN, SX, SW, OCC, ...) case n: if constexpr (n >= kHalvesFrom) return launch_quad_t<DT, kQuadPlain, TM, TN, SX, SW, OCC, false, 2>(q, st, who); break;
       FSVD_QUAD_PLAIN(X)
 #undef X
     }

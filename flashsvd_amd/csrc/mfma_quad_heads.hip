@@ -3,13 +3,13 @@
 
 namespace fsvd {
 
-// Tiles and their costs as in mfma_quad.hip, per round and K step in us (68 shapes: 48 and 96 heads at rank 512 to 1664, 128 to 16384 rows; the
-// form they name is 0.5 % behind the best of 19 on average, 4 % at worst, and 16 % ahead of the tiles that ran before):
-// a tile takes whole units of sixteen columns and the sixteen 64 past them.
+// Tiles and their costs as in mfma_quad.hip, per round and K step in us.  A tile takes whole units of sixteen columns and the sixteen 64 past
+// them.  q, k and v of 32 heads at rank 1024 with weights from HBM, 64 x 128 rings and 256 x 256 tiles before -> these: 154 / 333 / 512 / 1024 /
+// 2048 / 4096 rows 18.6 -> 15.0, 25.2 -> 20.5, 28.3 -> 25.7, 42.2 -> 39.7, 82.3 -> 70.1, 125.9 -> 115.2; at rank 1664 and 16384 rows 696 -> 594.
 #define FSVD_QUAD_HEADS(X) \
-  X(0, 8, 8, 2, 3, 1, 0.f, 0.f, 15.56f, 1.177f) X(1, 6, 4, 2, 2, 2, 4.00f, 0.866f, 8.98f, 1.194f) X(2, 5, 4, 2, 2, 2, 2.84f, 0.826f, 7.81f, 1.083f) \
-  X(3, 4, 4, 2, 3, 2, 3.37f, 0.565f, 6.78f, 0.922f) X(4, 3, 4, 2, 3, 2, 2.40f, 0.504f, 4.36f, 0.828f) X(5, 2, 4, 3, 4, 1, 0.f, 0.f, 2.10f, 0.389f) \
-  X(6, 2, 2, 4, 4, 2, 1.82f, 0.219f, 2.05f, 0.440f)
+  X(0, 8, 8, 2, 3, 1, 0.f, 0.f, 15.75f, 1.109f) X(1, 6, 4, 2, 2, 2, 5.73f, 0.855f, 8.07f, 1.176f) X(2, 5, 4, 2, 2, 2, 4.70f, 0.822f, 8.12f, 1.018f) \
+  X(3, 4, 4, 2, 3, 2, 4.44f, 0.540f, 6.92f, 0.861f) X(4, 3, 4, 2, 3, 2, 3.30f, 0.512f, 5.36f, 0.715f) X(5, 2, 4, 3, 4, 1, 0.f, 0.f, 3.01f, 0.359f) \
+  X(6, 2, 2, 5, 5, 2, 2.39f, 0.196f, 3.13f, 0.394f)
 #define FSVD_QUAD_HEADS_ANY(X) X(3, 4, 4, 2, 3, 2) X(4, 3, 4, 2, 3, 2) X(6, 2, 2, 4, 4, 2)
 
 static int heads_pick(const ExpandArgs* d, int n, bool any) {
