@@ -455,6 +455,73 @@ __global__ __launch_bounds__(kThreads) void qkv_rope_append_kernel(QkvArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------
+// Long outputs of one or two rows (the vocabulary): one workgroup per compute unit walks a slab of weight rows of its own.
+//
+// What a read stream reaches depends on how much of it is under way: 32 KB per compute unit 7.3 TB/s, 64 KB 7.0, 128 KB 6.0 (a plain
+// streaming kernel on this chip).  linear_kernel requests all it will read at once, four rows per wave and 2000 workgroups: 262 MB in 44.7 us.  Here
+// a wave keeps one window of P pieces (16 bytes per lane each) for R rows, eight pieces in all, and asks for a piece of its next row as soon
+// as it has consumed the one in its place; the activations sit in registers, so a piece costs its products and nothing else.  The sums
+// run in the order of linear_kernel: the same bits.
+// ---------------------------------------------------------------------------------------
+template <int DT, int BATCH, int P>
+__global__ __launch_bounds__(kThreads) void linear_slab_kernel(LinearArgs a) {
+  typedef E16<DT> E;
+  constexpr int R = 8 / P, K = P * kWave * 8;
+  __shared__ __align__(16) uint16_t xs[BATCH * K];
+  __shared__ float red[kWaves];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int per = a.N / (int)gridDim.x, rem = a.N - per * (int)gridDim.x, g = blockIdx.x;
+  const int row0 = g * per + min(g, rem) + wave, end = (g + 1) * per + min(g + 1, rem);      // this wave's rows: row0, row0 + 4, ...
+  u32x4_t w[R][P];
+#if defined(__HIP_DEVICE_COMPILE__)
+  // rows behind this workgroup's last one are out of the descriptor's range: asked for like any other, they move nothing
+  const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.W), 0, __builtin_amdgcn_readfirstlane((int)((int64_t)end * a.ldw * 2)), 0x00020000u);
+#endif
+  const auto request = [&](int r, int p, int row) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    w[r][p] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)((uint32_t)row * (uint32_t)(a.ldw * 2)) + lane * 16 + p * kWave * 16, 0, 2);
+#endif
+  };
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int p = 0; p < P; ++p) request(r, p, row0 + r * kWaves);
+  stage_x<DT, BATCH>(a.x, a.ldx, a.B, K, K, a.norm_w, a.eps, xs, red);
+  u32x4_t x[BATCH][P];
+#pragma unroll
+  for (int b = 0; b < BATCH; ++b)
+#pragma unroll
+    for (int p = 0; p < P; ++p) x[b][p] = *reinterpret_cast<const u32x4_t*>(xs + b * K + (p * kWave + lane) * 8);
+  for (int row = row0; row < end; row += R * kWaves) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int n = row + r * kWaves, next = n + R * kWaves;
+      float acc[BATCH];
+#pragma unroll
+      for (int b = 0; b < BATCH; ++b) acc[b] = 0.f;
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+#pragma unroll
+        for (int b = 0; b < BATCH; ++b) acc[b] = E::dot8(w[r][p], x[b][p], acc[b]);
+        __builtin_amdgcn_sched_barrier(0);
+        request(r, p, next);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int b = 0; b < BATCH; ++b) {
+        float v = wave_sum(acc[b]);
+        if (lane == b && b < a.B && n < end) {
+          if (a.bias) v += E::val(a.bias[n]);
+          v = E::rnd(v);
+          if (a.res) v = E::rnd(E::val(a.res[(int64_t)b * a.ldres + n]) + v);
+          a.y[(int64_t)b * a.ldy + n] = (uint16_t)E::bits(v);
+        }
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------
 // stand-alone RMSNorm (one block per row)
 // ---------------------------------------------------------------------------------------
 template <int DT>
@@ -494,12 +561,17 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_vec_kernel(const uint16_t* _
   const uint16_t* src = x + (int64_t)blockIdx.x * ldx;
   uint16_t* dst = y + (int64_t)blockIdx.x * ldy;
   const int nchunk = K >> 3;
-  u32x4_t v[NC];
-  float ss = 0.f;
+  // the weights are requested with the row: behind the reduction their way from memory came on top of the row's
+  u32x4_t v[NC], wv[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     const int ch = threadIdx.x + c * kThreads;
     v[c] = ch < nchunk ? *reinterpret_cast<const u32x4_t*>(src + ch * 8) : u32x4_t{0u, 0u, 0u, 0u};
+    wv[c] = ch < nchunk ? *reinterpret_cast<const u32x4_t*>(w + ch * 8) : u32x4_t{0u, 0u, 0u, 0u};
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
     const uint32_t e[4] = {v[c].x, v[c].y, v[c].z, v[c].w};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -519,8 +591,7 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_vec_kernel(const uint16_t* _
   for (int c = 0; c < NC; ++c) {
     const int ch = threadIdx.x + c * kThreads;
     if (ch >= nchunk) break;
-    const u32x4_t wv = *reinterpret_cast<const u32x4_t*>(w + ch * 8);
-    const uint32_t e[4] = {v[c].x, v[c].y, v[c].z, v[c].w}, g[4] = {wv.x, wv.y, wv.z, wv.w};
+    const uint32_t e[4] = {v[c].x, v[c].y, v[c].z, v[c].w}, g[4] = {wv[c].x, wv[c].y, wv[c].z, wv[c].w};
     uint32_t o[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -573,8 +644,25 @@ static int launch_linear_b(const LinearArgs& a, int cfg, hipStream_t st) {
   return kOk;
 }
 
+// long outputs whose rows are one window: 2048 or 4096 values, 64 rows and more per compute unit
+template <int DT>
+static int launch_linear_slab(const LinearArgs& a, hipStream_t st) {
+  const dim3 grid(2 * compute_units());
+  if (a.K == 4096) {
+    if (a.B == 1) hipLaunchKernelGGL((linear_slab_kernel<DT, 1, 8>), grid, dim3(kThreads), 0, st, a);
+    else hipLaunchKernelGGL((linear_slab_kernel<DT, 2, 8>), grid, dim3(kThreads), 0, st, a);
+  } else {
+    if (a.B == 1) hipLaunchKernelGGL((linear_slab_kernel<DT, 1, 4>), grid, dim3(kThreads), 0, st, a);
+    else hipLaunchKernelGGL((linear_slab_kernel<DT, 2, 4>), grid, dim3(kThreads), 0, st, a);
+  }
+  FSVD_CHECK_LAUNCH("fsvd_linear");
+  return kOk;
+}
 template <int DT>
 static int launch_linear_t(const LinearArgs& a, int cfg, hipStream_t st) {
+  if (cfg == 0 && a.B <= 2 && (a.K == 2048 || a.K == 4096) && a.positions == nullptr && compute_units() > 0 && a.N >= 64 * compute_units() &&
+      a.ldw % 8 == 0 && aligned16(a.W) && below_4gib(a.N, a.ldw))
+    return launch_linear_slab<DT>(a, st);
   const bool vec = (a.K % 8 == 0) && (a.ldw % 8 == 0) && aligned16(a.W);
   const int batch = a.B >= 4 && a.K <= 16384 ? 4 : (a.B >= 2 ? 2 : 1);
   if (vec) {

@@ -781,7 +781,7 @@ static int launch_mfma(const MfmaArgs& a0, hipStream_t st, const char* who) {
   int ks = 8;
   for (int c = 2; c <= 8; c *= 2)
     if ((tiles * c + 7) / 8 >= 256 && ksteps / c >= 4) { ks = c; break; }
-  // 128 rows and more (prompts): four-wave tiles, ragged K and rows on the 4-byte grid included
+  // prompts and large batches: four-wave tiles, ragged K and rows on the 4-byte grid included
   if (gemm_quad_apply(a0, DUAL)) return launch_gemm_quad(a0, DUAL, st, who);
   // any K, rows that start anywhere: in the kernel above without a workspace, or on tiles that are never split
   if (gemm_ragged_apply(a0)) {

@@ -10,8 +10,8 @@ namespace fsvd {
 // the form that they name is on average 2 / 1 / 1 % (at worst 20, 12, 8 %) behind the best of about 30 tilings.
 struct QuadCost { float f1, s1, f2, s2; };
 constexpr float kLaunchUs = 3.f;
-static float quad_us(const QuadCost& c, int64_t tiles, int occ, float steps) {
-  const int64_t cu = compute_units(), full = tiles / (cu * occ), rest = tiles - full * cu * occ;
+static float quad_us(const QuadCost& c, int64_t tiles, int occ, float steps, int64_t cu) {
+  const int64_t full = tiles / (cu * occ), rest = tiles - full * cu * occ;
   float us = (float)full * (c.f2 + c.s2 * steps);
   if (rest > 0) us += occ == 2 && rest <= cu ? c.f1 + c.s1 * steps : c.f2 + c.s2 * steps;
   return us;
@@ -29,10 +29,11 @@ constexpr int kHalvesFrom = 5;                       // forms with registers for
 #define FSVD_QUAD_PAIR(X) \
   X(0, 4, 6, 3, 4, 1, 0.f, 0.f, 8.19f, 0.657f) X(1, 5, 6, 2, 3, 1, 0.f, 0.f, 9.82f, 0.693f) X(2, 5, 4, 2, 2, 2, 4.26f, 0.861f, 8.46f, 0.970f) \
   X(3, 8, 4, 2, 3, 1, 0.f, 0.f, 10.88f, 0.710f) X(4, 4, 4, 2, 3, 2, 3.94f, 0.589f, 7.43f, 0.802f) X(5, 4, 4, 4, 5, 1, 0.f, 0.f, 6.31f, 0.487f) \
-  X(6, 3, 6, 3, 4, 1, 0.f, 0.f, 6.98f, 0.562f) X(7, 3, 3, 3, 3, 2, 1.93f, 0.444f, 4.61f, 0.652f) X(8, 2, 3, 3, 4, 2, 2.96f, 0.273f, 2.34f, 0.547f)
-// ragged rows: tiles with two workgroups per compute unit
-#define FSVD_QUAD_PLAIN_ANY(X) X(5, 4, 4, 2, 3, 2) X(10, 3, 2, 3, 4, 2) X(12, 2, 2, 4, 4, 2)
-#define FSVD_QUAD_PAIR_ANY(X) X(4, 4, 4, 2, 3, 2) X(7, 3, 3, 3, 3, 2) X(8, 2, 3, 3, 4, 2)
+  X(6, 3, 6, 3, 4, 1, 0.f, 0.f, 6.98f, 0.562f) X(7, 3, 3, 3, 3, 2, 1.93f, 0.444f, 4.61f, 0.652f) X(8, 2, 3, 3, 4, 2, 2.96f, 0.273f, 2.34f, 0.547f) \
+  X(9, 2, 2, 5, 5, 2, 1.50f, 0.330f, 1.50f, 0.490f)
+// ragged rows: some of them
+#define FSVD_QUAD_PLAIN_ANY(X) X(4, 6, 4, 3, 4, 1) X(5, 4, 4, 2, 3, 2) X(10, 3, 2, 3, 4, 2) X(12, 2, 2, 5, 5, 2)
+#define FSVD_QUAD_PAIR_ANY(X) X(0, 4, 6, 3, 4, 1) X(4, 4, 4, 2, 3, 2) X(6, 3, 6, 3, 4, 1) X(7, 3, 3, 3, 3, 2) X(8, 2, 3, 3, 4, 2)
 
 constexpr int kQuadNone = -1;
 struct QuadPick { int form; float us; };
@@ -42,7 +43,7 @@ struct QuadPick { int form; float us; };
 enum QuadOrder { kOrderPlain = 0, kOrderHalves = 1, kOrderCut = 2 };
 struct QuadSums { QuadOrder order; int per; };
 static QuadSums quad_sums(const MfmaArgs& a) {
-  if (gemm_big_apply(a, false)) return QuadSums{kOrderPlain, 0};
+  if (a.B < 128 || gemm_big_apply(a, false)) return QuadSums{kOrderPlain, 0};
   const RingRule r = gemm_mid_rule(a);
   if (r.area > 0) return QuadSums{r.halves ? kOrderHalves : kOrderPlain, 0};
   const int per = gemm_tiles_cut(a);
@@ -52,12 +53,13 @@ static QuadPick quad_pick(const MfmaArgs& a, bool dual, bool any, QuadOrder orde
   if (order == kOrderCut) return QuadPick{12, 0.f};                                  // few 64 x 64 tiles by that rule
   QuadPick best{kQuadNone, 0.f};
   const float steps = (float)((a.K + 63) / 64 * (dual ? 2 : 1));
+  const int64_t cu = compute_units();                // asked once: a small model's call is bound by what the host does per launch
   const auto take = [&](int form, int tm, int tn, int occ, const QuadCost& c) {
-    const float us = quad_us(c, quad_tiles(a, tm, tn), occ, steps);
+    const float us = quad_us(c, quad_tiles(a, tm, tn), occ, steps, cu);
     if (best.form == kQuadNone || us < best.us) best = QuadPick{form, us};
   };
   if (dual) {
-#define X(n, TM, TN, SX, SW, OCC, F1, S1, F2, S2) if (!any || n == 4 || n >= 7) take(n, TM, TN, OCC, QuadCost{F1, S1, F2, S2});
+#define X(n, TM, TN, SX, SW, OCC, F1, S1, F2, S2) if (!any || n == 0 || n == 4 || (n >= 6 && n <= 8)) take(n, TM, TN, OCC, QuadCost{F1, S1, F2, S2});
     FSVD_QUAD_PAIR(X)
 #undef X
   } else {
@@ -65,7 +67,7 @@ static QuadPick quad_pick(const MfmaArgs& a, bool dual, bool any, QuadOrder orde
     // 420, 512 rows 22.5, 22.2, 22.2, 27.6 against 17.9, 21.5, 23.7, 27.2), below it is the best tile of 333 rows (4096 x 1536 11.4 against
     // 12.8).  64 x 96 comes in where it pads nothing (512 x 3072 x 4096 24.5 against 27.2; 420 rows 23.6 against 23.7).
     const auto fits = [&](int n) {
-      if (any) return n == 5 || n == 10 || n == 12;
+      if (any) return n == 4 || n == 5 || n == 10 || n == 12;
       if (n < kHalvesFrom && order != kOrderPlain) return false;
       return n == 10 ? a.K < 4096 : (n == 11 ? a.B % 64 == 0 && a.N % 96 == 0 : true);
     };
@@ -86,9 +88,14 @@ static bool quad_words(const MfmaArgs& a, bool dual) {
   return a.ldx % 2 == 0 && a.ldw % 2 == 0 && a.up_off % 2 == 0 && al4(a.x) && al4(a.W) && (!dual || al4(a.W2));
 }
 // From 128 rows and five K steps on (fewer steps than the stages hold are left to the tiles that were measured for them); N holds a whole
-// residual piece.  The pair in the rounding that keeps the gate in 32 bits goes to mfma_mid.hip.
+// residual piece.  The pair in the rounding that keeps the gate in 32 bits goes to mfma_mid.hip.  From 33 rows on where there are 64 tiles of
+// 64 x 64 with a K below 4096, or 128 of them (us at 40 / 64 / 100 rows, 32-row tiles with K split over workgroups -> these: the pair 11008 x 1536 30.6 ->
+// 19.3, 31.9 -> 21.4, 34.5 -> 23.3, 32000 x 4096 65 -> 53, 72 -> 56, 99 -> 62, 4096 x 1024 8.7 -> 7.4, 8.9 -> 8.2, 10.9 -> 7.5); fewer tiles
+// need the split (3072 x 4096 16.1 against 18.5, 16.9 against 21.3; 1024 x 4096 9.4 against 17.8).
 static bool quad_range(const MfmaArgs& a, bool dual) {
-  return a.B >= 128 && a.K >= 320 && a.N >= 8 && compute_units() > 0 && (!dual || a.mode == 0) && below_4gib(a.B, a.ldx) && below_4gib(a.N, a.ldw);
+  if (a.B < 33 || a.K < 320 || a.N < 8 || compute_units() <= 0 || (dual && a.mode != 0) || !below_4gib(a.B, a.ldx) || !below_4gib(a.N, a.ldw)) return false;
+  const int64_t tiles = quad_tiles(a, 2, 2), cu = compute_units();
+  return a.B >= 128 || tiles * 2 >= cu || (tiles * 4 >= cu && a.K < 4096);
 }
 
 // A long K in shares over workgroups, about one workgroup of the launch per compute unit, their sums in scratch of the call's own
@@ -111,8 +118,8 @@ static bool quad_range(const MfmaArgs& a, bool dual) {
 struct ShareForm { int bm, bn, shares, per; };
 static ShareForm share_form(const MfmaArgs& a) {
   const ShareForm none{0, 0, 0, 0};
+  if (a.scratch_floats == 0 || a.B < 128 || a.K < 4096 || !quad_range(a, false) || !quad_grid(a, false) || gemm_big_apply(a, false)) return none;
   const int64_t cu = compute_units();
-  if (a.scratch_floats == 0 || a.K < 4096 || !quad_range(a, false) || !quad_grid(a, false) || gemm_big_apply(a, false)) return none;
   const auto pad = [&](int64_t r) { return (a.B + r - 1) / r * r; };
   const int steps = a.K / 64;
   const RingRule ring = gemm_mid_rule(a);
@@ -122,8 +129,8 @@ static ShareForm share_form(const MfmaArgs& a) {
   if (sums.order == kOrderCut) {
     const int64_t tiles = quad_tiles(a, 2, 2), shares = (steps + sums.per - 1) / sums.per;
     const QuadCost c{0.49f, 0.227f, 2.66f, 0.355f};
-    const float apart = quad_us(c, tiles * shares, 2, (float)sums.per) + 3.5f + (float)(shares * tiles * 4096) * 8.f / 4.5e6f;
-    if (apart < quad_us(c, tiles, 2, (float)steps) && (size_t)(tiles * shares * 4096) <= a.scratch_floats) return ShareForm{64, 64, (int)shares, sums.per};
+    const float apart = quad_us(c, tiles * shares, 2, (float)sums.per, cu) + 3.5f + (float)(shares * tiles * 4096) * 8.f / 4.5e6f;
+    if (apart < quad_us(c, tiles, 2, (float)steps, cu) && (size_t)(tiles * shares * 4096) <= a.scratch_floats) return ShareForm{64, 64, (int)shares, sums.per};
   }
   // the cut of the 64 x 64 tiles, where a tile of this kernel fills 70 percent of the compute units with it: the same bits
   if (a.K >= 8192 && ring.area == 0) {
@@ -230,14 +237,14 @@ static int launch_share_dt(QuadArgs& q, const ShareForm& f, hipStream_t st, cons
 
 // The 256 x 256 pair of mfma_big.hip keeps what its larger tile still does better: 11008 x 2432 at 16384 rows 1602 us, here 1617 at best
 // (8192 rows 874 against 780, its rounds being few and large); its cost in the same terms.
-static bool big_pair_is_ahead(const MfmaArgs& a, float us) {
-  return gemm_big_apply(a, true) && quad_us(QuadCost{0.f, 0.f, 26.7f, 1.564f}, quad_tiles(a, 8, 8), 1, (float)(a.K / 32)) < us;
+static bool big_pair_is_ahead(const MfmaArgs& a) {
+  return gemm_big_apply(a, true) && quad_us(QuadCost{0.f, 0.f, 26.7f, 1.564f}, quad_tiles(a, 8, 8), 1, (float)(a.K / 32), compute_units()) < quad_pick(a, true, false).us;
 }
 
 bool gemm_quad_apply(const MfmaArgs& a, bool dual) {
   if (!quad_range(a, dual)) return false;
-  if (quad_grid(a, dual)) return !dual || !big_pair_is_ahead(a, quad_pick(a, true, false).us);
-  return quad_words(a, dual);
+  if (quad_grid(a, dual)) return !dual || !big_pair_is_ahead(a);
+  return quad_words(a, dual) && (dual || a.B >= 128);
 }
 
 template <int DT>

@@ -5,7 +5,8 @@ namespace fsvd {
 
 // Tiles and their costs as in mfma_quad.hip, per round and K step in us.  A tile takes whole units of sixteen columns and the sixteen 64 past
 // them.  q, k and v of 32 heads at rank 1024 with weights from HBM, 64 x 128 rings and 256 x 256 tiles before -> these: 154 / 333 / 512 / 1024 /
-// 2048 / 4096 rows 18.6 -> 15.0, 25.2 -> 20.5, 28.3 -> 25.7, 42.2 -> 39.7, 82.3 -> 70.1, 125.9 -> 115.2; at rank 1664 and 16384 rows 696 -> 594.
+// 2048 / 4096 rows 18.6 -> 15.0, 25.2 -> 20.5, 28.3 -> 25.7, 42.2 -> 39.7, 82.3 -> 70.1, 125.9 -> 115.2; at rank 1664 and 16384 rows 696 -> 594;
+// 24 / 64 rows 12.3 -> 9.0, 13.5 -> 10.2.
 #define FSVD_QUAD_HEADS(X) \
   X(0, 8, 8, 2, 3, 1, 0.f, 0.f, 15.75f, 1.109f) X(1, 6, 4, 2, 2, 2, 5.73f, 0.855f, 8.07f, 1.176f) X(2, 5, 4, 2, 2, 2, 4.70f, 0.822f, 8.12f, 1.018f) \
   X(3, 4, 4, 2, 3, 2, 4.44f, 0.540f, 6.92f, 0.861f) X(4, 3, 4, 2, 3, 2, 3.30f, 0.512f, 5.36f, 0.715f) X(5, 2, 4, 3, 4, 1, 0.f, 0.f, 3.01f, 0.359f) \
@@ -34,7 +35,7 @@ static int heads_pick(const ExpandArgs* d, int n, bool any) {
 static bool heads_on_grid(const ExpandArgs& a) { return a.R % 64 == 0 && a.sp_b % 8 == 0 && a.sp_m % 8 == 0 && a.ldu % 8 == 0 && aligned16(a.p) && aligned16(a.u); }
 // the same rank in a launch where it is no whole number of steps (the tail is cleared by one rank)
 bool expand_quad_apply(const ExpandArgs* d, int n) {
-  if (compute_units() <= 0 || (int64_t)d[0].B * d[0].M < 128) return false;
+  if (compute_units() <= 0 || (int64_t)d[0].B * d[0].M < 17) return false;
   bool any = false;
   for (int k = 0; k < n; ++k) any = any || !heads_on_grid(d[k]);
   for (int k = 0; k < n; ++k) {
