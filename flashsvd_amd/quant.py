@@ -223,7 +223,10 @@ def pack_quant_rows(mods) -> Optional[tuple]:
 
 
 def is_quantized(*mods) -> bool:
-    return any(isinstance(m, PackedQuantLinear) for m in mods)
+    for m in mods:
+        if isinstance(m, PackedQuantLinear):
+            return True
+    return False
 
 
 # ---- model-level helpers (src/quant/common.py) ---------------------------------------------------------
