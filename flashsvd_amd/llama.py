@@ -60,8 +60,16 @@ class LlamaRMSNorm(nn.Module):
 
 # the factor modules of a half layer straight from the module's own table (asked for several times per layer and call: attribute by
 # attribute the fourteen of them took 7 us of a layer's host time)
-_ATTENTION_FACTORS = operator.itemgetter("q_v_proj", "q_u_proj", "k_v_proj", "k_u_proj", "v_v_proj", "v_u_proj", "o_v_proj", "o_u_proj")
-_MLP_FACTORS = operator.itemgetter("gate_v_proj", "gate_u_proj", "up_v_proj", "up_u_proj", "down_v_proj", "down_u_proj")
+_ATTENTION_NAMES = ("q_v_proj", "q_u_proj", "k_v_proj", "k_u_proj", "v_v_proj", "v_u_proj", "o_v_proj", "o_u_proj")
+_MLP_NAMES = ("gate_v_proj", "gate_u_proj", "up_v_proj", "up_u_proj", "down_v_proj", "down_u_proj")
+_ATTENTION_FACTORS, _MLP_FACTORS = operator.itemgetter(*_ATTENTION_NAMES), operator.itemgetter(*_MLP_NAMES)
+
+
+def _from_table(module: nn.Module, factors, names):
+    try:
+        return factors(module._modules)
+    except KeyError:                                   # a factor that is no registered module (a plain attribute, a property of a subclass)
+        return tuple(getattr(module, name) for name in names)
 
 
 class LlamaRotaryEmbedding(nn.Module):
@@ -156,7 +164,7 @@ class SVD_LlamaAttention(nn.Module):
         self._packed_qkv_v = None
 
     def _factor_modules(self):
-        return _ATTENTION_FACTORS(self._modules)
+        return _from_table(self, _ATTENTION_FACTORS, _ATTENTION_NAMES)
 
     def _ensure_runtime_state(self) -> None:
         """Idempotent.  Packs [q_v; k_v; v_v] into one row-contiguous buffer (the module weights
@@ -593,7 +601,7 @@ class SVD_LlamaMLP(nn.Module):
                 setattr(self, name, {})
 
     def _factor_modules(self):
-        return _MLP_FACTORS(self._modules)
+        return _from_table(self, _MLP_FACTORS, _MLP_NAMES)
 
     def _run_quantized(self, x: torch.Tensor, *, norm_weight=None, eps: float = 1e-6, residual=None, mode: Optional[int] = None):
         """The same four stages with int4 factors: each projection through the kernel that fits its module."""

@@ -330,3 +330,17 @@ def test_dual_split_config_pickers_honour_env():
     finally:
         del os.environ["FLASH_SVD_DUAL_SPLIT_V2_BD"], os.environ["FLASH_SVD_DUAL_SPLIT_V2_WARPS"]
     assert ds.flashsvd_ffn_dual_split_token_v3 is ds.flashsvd_mlp_dual_split_triton_v3
+
+
+def test_factor_modules_need_not_be_registered():
+    """A factor that was taken out of a half layer's modules and put back as a plain attribute is found, a missing one is an AttributeError."""
+    from flashsvd_amd import llama
+    model = llama.build_model(hidden_size=128, num_heads=2, num_kv_heads=2, head_dim=64, intermediate_size=128, num_layers=1, vocab_size=32,
+                              attn_rank=32, mlp_rank=32)
+    for half, name in ((model.model.layers[0].self_attn, "o_v_proj"), (model.model.layers[0].mlp, "down_v_proj")):
+        before, lin = half._factor_modules(), getattr(half, name)
+        delattr(half, name)
+        with pytest.raises(AttributeError):
+            half._factor_modules()
+        half.__dict__[name] = lin
+        assert all(a is b for a, b in zip(half._factor_modules(), before)) and len(half._factor_modules()) == len(before)
