@@ -25,7 +25,7 @@ static int64_t quad_tiles(const MfmaArgs& a, int tm, int tn) { return (int64_t)(
   X(6, 4, 4, 4, 5, 1, 0.f, 0.f, 3.03f, 0.450f) X(7, 4, 3, 5, 6, 1, 0.f, 0.f, 4.29f, 0.353f) X(8, 4, 2, 3, 4, 2, 0.57f, 0.339f, 3.94f, 0.568f) \
   X(9, 2, 4, 3, 4, 1, 0.f, 0.f, 1.24f, 0.354f) X(10, 3, 2, 3, 4, 2, 0.24f, 0.297f, 3.14f, 0.440f) X(11, 2, 3, 3, 4, 2, 0.30f, 0.311f, 1.99f, 0.484f) \
   X(12, 2, 2, 5, 5, 2, 0.49f, 0.227f, 2.66f, 0.355f)
-constexpr int kHalvesFrom = 5;                       // forms with registers for a second set of accumulators
+constexpr int kHalvesFrom = 8;                       // the forms that shapes with K halved get, with registers for a second set of accumulators
 #define FSVD_QUAD_PAIR(X) \
   X(0, 4, 6, 3, 4, 1, 0.f, 0.f, 8.19f, 0.657f) X(1, 5, 6, 2, 3, 1, 0.f, 0.f, 9.82f, 0.693f) X(2, 5, 4, 2, 2, 2, 4.26f, 0.861f, 8.46f, 0.970f) \
   X(3, 8, 4, 2, 3, 1, 0.f, 0.f, 10.88f, 0.710f) X(4, 4, 4, 2, 3, 2, 3.94f, 0.589f, 7.43f, 0.802f) X(5, 4, 4, 4, 5, 1, 0.f, 0.f, 6.31f, 0.487f) \
