@@ -109,7 +109,7 @@ __global__ __launch_bounds__(kPfThreads) void lowrank_expand_kernel(ExpandArgs a
 }
 
 // ---------------------------------------------------------------------------------------------
-// 2. causal flash attention, head_dim 128: 64 or 128 queries per workgroup (16 MI per wave), K and V tiles shared
+// 2. causal flash attention, head_dim 128: 32, 64 or 128 queries per workgroup (16 MI per wave), K and V tiles shared
 //     through LDS.  With every wave fetching its own K fragments a 64-key tile costs 80 KB of L2 traffic per 64
 //     queries and the kernel is bound by L2 requests; here a tile is read ONCE per workgroup, coalesced, one tile
 //     ahead into registers, and written to LDS (K row-major with a padded stride, V transposed: four adjacent keys
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(kPfThreads) void lowrank_expand_kernel(ExpandArgs a
 //     padding mask 215 -> 120; 512 tokens 19.0 -> 16.0.  Then, with every XCD starting the long tiles of all its heads first instead of
 //     head by head (on average 1.2 of two possible waves were resident per SIMD): 576 -> 506 us (543 TFLOP/s), 122 -> 85, padded
 //     121 -> 83; one sequence of 1024 / 2048 tokens 43 -> 36, 121 -> 97, 700 behind 1000 72 -> 63.  Below 128 rows a kernel without shared
-//     tiles ran: two chunks of 77 rows behind 1411 tokens (32 / 8 heads) 181 -> 31 us.  Two LDS stages instead of one, raised
+//     tiles ran: two chunks of 77 rows behind 1411 tokens (32 / 8 heads) 181 -> 31 us, with 32 rows per workgroup 25.6.  Two LDS stages instead of one, raised
 //     priority around the products and scalar address parts were built and gave nothing: two workgroups share a compute
 //     unit, and each covers the other's waits.
 // ---------------------------------------------------------------------------------------------
@@ -165,17 +165,19 @@ __device__ __forceinline__ float weight_of(float s, float scale, float m) {
 // statistics and outputs are merged through LDS at the end — for calls whose (query tile, head) pairs number no more than
 // the compute units, where a workgroup alone on its compute unit walks its key tiles with one wave per SIMD and waits out
 // every load and barrier.
-template <int DT, int MI, int NG>
-__global__ __launch_bounds__(kPfThreads * NG, NG == 1 ? 2 : 1) void attn_prefill_kernel(PrefillAttnArgs a) {
+// NW: waves of a group, 16 MI query rows each (see launch_prefill_attn_t).
+template <int DT, int MI, int NG, int NW>
+__global__ __launch_bounds__(kWave * NW * NG, NG == 1 ? 2 : 1) void attn_prefill_kernel(PrefillAttnArgs a) {
   typedef E16<DT> E;
   typedef typename E::frag_t frag_t;
-  constexpr int DH = 128, BN = 64, QW = 16 * MI, BM = 4 * QW, VSTR = BN;
+  constexpr int DH = 128, BN = 64, QW = 16 * MI, BM = NW * QW, VSTR = BN;
+  constexpr int TG = kWave * NW, SR = TG / 16, PASS = BN / 4 / SR;   // threads of a group; rows that it stages at a time; passes over V's 16 groups of four keys
   // K rows of 288 bytes: a 16-byte LDS read is served 16 lanes a cycle (lanes 0-3, 12-15, 20-27 / 4-11, 16-19, 28-31 of a
   // half wave); rows 16 r apart with r odd multiples of 32 bytes give those lanes 16 different bank groups
   constexpr int KSTR = DH + 16;
   extern __shared__ __align__(16) unsigned char pw_smem[];
   constexpr int kGroupBytes = BN * KSTR * 2 + DH * VSTR * 2;
-  const int grp = NG == 1 ? 0 : (int)(threadIdx.x >> 8);
+  const int grp = NG == 1 ? 0 : (int)threadIdx.x / TG;
   unsigned char* gsm = pw_smem + (size_t)grp * kGroupBytes;
   uint16_t (*Ks)[KSTR] = reinterpret_cast<uint16_t (*)[KSTR]>(gsm);                                   // [BN][KSTR]
   uint16_t (*Vt)[VSTR] = reinterpret_cast<uint16_t (*)[VSTR]>(gsm + (size_t)BN * KSTR * 2);            // [DH][VSTR]
@@ -198,7 +200,7 @@ __global__ __launch_bounds__(kPfThreads * NG, NG == 1 ? 2 : 1) void attn_prefill
   if (a.causal) mt = MT - 1 - mt;
   const int h = hb / (int)gridDim.z, b = hb - h * (int)gridDim.z;
   const int hk = h / (a.H / a.Hk);
-  const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;   // thread and wave within the group
+  const int tid = threadIdx.x % TG, lane = tid & 63, wave = tid >> 6;   // thread and wave within the group
   const int lr = lane & 15, lg = lane >> 4;
   const int q0 = a.q_pos0 ? a.q_pos0[b] : a.pos0;
   const int m_base = mt * BM + wave * QW;
@@ -230,20 +232,22 @@ __global__ __launch_bounds__(kPfThreads * NG, NG == 1 ? 2 : 1) void attn_prefill
   // the maximum is taken of the unscaled scores; an additive mask and a scale that does not keep the order take the long way
   const bool direct = a.add_mask == nullptr && a.scale > 0.f;
 
-  // staging roles: 16 lanes cover one 256-byte row; K: rows tid/16 + 16 j; V: the four adjacent keys 4 (tid/16) + j
+  // staging roles: 16 lanes cover one 256-byte row; K: rows tid/16 + SR j; V: the four adjacent keys 4 (tid/16 + SR p) + j
   const int srow = tid >> 4, d0 = (tid & 15) * 8;
   // column of this thread's four keys in the permuted order of V^T (see above), before the bank swizzle
-  const int vko = (srow * 4) & 31;
-  const int vcol = ((srow * 4) & 32) + 8 * ((vko & 15) >> 2) + 4 * (vko >> 4);
-  u32x4_t kreg[4], vreg[4];
+  const auto vcol_of = [](int row4) {
+    const int vko = (row4 * 4) & 31;
+    return ((row4 * 4) & 32) + 8 * ((vko & 15) >> 2) + 4 * (vko >> 4);
+  };
+  u32x4_t kreg[4 * PASS], vreg[4 * PASS];
   // the padding mask of a key tile travels with it: its bytes requested with the tile (the group's first wave, one key per
   // lane), parked in LDS beside it as one word, bit = key
   __shared__ uint64_t pms[NG];
   uint8_t pmreg = 1;
   auto request = [&](int n0) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int kkey = min(n0 + srow + 16 * j, n_keys_all - 1), vkey = min(n0 + srow * 4 + j, n_keys_all - 1);
+    for (int j = 0; j < 4 * PASS; ++j) {
+      const int kkey = min(n0 + srow + SR * j, n_keys_all - 1), vkey = min(n0 + (srow + SR * (j >> 2)) * 4 + (j & 3), n_keys_all - 1);
       kreg[j] = *reinterpret_cast<const u32x4_t*>(kb + (int64_t)kkey * a.sk_s + d0);
       vreg[j] = *reinterpret_cast<const u32x4_t*>(vb + (int64_t)vkey * a.sk_s + d0);
     }
@@ -261,10 +265,13 @@ __global__ __launch_bounds__(kPfThreads * NG, NG == 1 ? 2 : 1) void attn_prefill
       if (tid == 0) pms[grp] = seen;
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) *reinterpret_cast<u32x4_t*>(&Ks[srow + 16 * j][d0]) = kreg[j];
-    {
-      const uint32_t w[4][4] = {{vreg[0].x, vreg[0].y, vreg[0].z, vreg[0].w}, {vreg[1].x, vreg[1].y, vreg[1].z, vreg[1].w},
-                                {vreg[2].x, vreg[2].y, vreg[2].z, vreg[2].w}, {vreg[3].x, vreg[3].y, vreg[3].z, vreg[3].w}};
+    for (int j = 0; j < 4 * PASS; ++j) *reinterpret_cast<u32x4_t*>(&Ks[srow + SR * j][d0]) = kreg[j];
+#pragma unroll
+    for (int p = 0; p < PASS; ++p) {
+      const u32x4_t *v = vreg + 4 * p;
+      const int vcol = vcol_of(srow + SR * p);
+      const uint32_t w[4][4] = {{v[0].x, v[0].y, v[0].z, v[0].w}, {v[1].x, v[1].y, v[1].z, v[1].w},
+                                {v[2].x, v[2].y, v[2].z, v[2].w}, {v[3].x, v[3].y, v[3].z, v[3].w}};
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         u32x2_t lo, hi;   // dimensions d0 + 2c (low halves) and d0 + 2c + 1 (high halves) of the four keys
@@ -409,29 +416,29 @@ __global__ __launch_bounds__(kPfThreads * NG, NG == 1 ? 2 : 1) void attn_prefill
     f32x4_t* mb = reinterpret_cast<f32x4_t*>(pw_smem);
     __syncthreads();                   // all groups are done with their K / V tiles
     if (grp > 0) {
-      f32x4_t* mg = mb + (size_t)(grp - 1) * MI * 9 * 256;
+      f32x4_t* mg = mb + (size_t)(grp - 1) * MI * 9 * TG;
 #pragma unroll
       for (int mi = 0; mi < MI; ++mi) {
-        mg[(mi * 9) * 256 + tid] = f32x4_t{m_run[mi], l_run[mi], 0.f, 0.f};
+        mg[(mi * 9) * TG + tid] = f32x4_t{m_run[mi], l_run[mi], 0.f, 0.f};
 #pragma unroll
-        for (int t = 0; t < 8; ++t) mg[(mi * 9 + 1 + t) * 256 + tid] = o[mi][t];
+        for (int t = 0; t < 8; ++t) mg[(mi * 9 + 1 + t) * TG + tid] = o[mi][t];
       }
     }
     __syncthreads();
     if (grp > 0) return;
 #pragma unroll
     for (int g = 0; g < NG - 1; ++g) {
-      const f32x4_t* mg = mb + (size_t)g * MI * 9 * 256;
+      const f32x4_t* mg = mb + (size_t)g * MI * 9 * TG;
 #pragma unroll
       for (int mi = 0; mi < MI; ++mi) {
-        const f32x4_t st = mg[(mi * 9) * 256 + tid];
+        const f32x4_t st = mg[(mi * 9) * TG + tid];
         const float m1 = st[0], l1 = st[1];
         const float m = fmaxf(m_run[mi], m1);
         const float a0 = m_run[mi] == -INFINITY ? 0.f : __expf(m_run[mi] - m), a1 = m1 == -INFINITY ? 0.f : __expf(m1 - m);
         l_run[mi] = l_run[mi] * a0 + l1 * a1;
         m_run[mi] = m;
 #pragma unroll
-        for (int t = 0; t < 8; ++t) o[mi][t] = o[mi][t] * a0 + mg[(mi * 9 + 1 + t) * 256 + tid] * a1;
+        for (int t = 0; t < 8; ++t) o[mi][t] = o[mi][t] * a0 + mg[(mi * 9 + 1 + t) * TG + tid] * a1;
       }
     }
   }
@@ -502,19 +509,19 @@ int launch_expand(const ExpandArgs& a, hipStream_t st) {
   return kOk;
 }
 
-template <int DT, int MI, int NG>
+template <int DT, int MI, int NG, int NW = 4>
 static int launch_prefill_attn_form(const PrefillAttnArgs& a, hipStream_t st) {
   const char* fn = "fsvd_attn_prefill";
   constexpr size_t lds = (size_t)NG * ((size_t)64 * 144 * 2 + (size_t)128 * 64 * 2);
   if (NG > 1) {
     static bool granted = false;
     if (!granted) {
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_prefill_kernel<DT, MI, NG>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_prefill_kernel<DT, MI, NG, NW>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
       if (e != hipSuccess) { set_last_error("%s: cannot reserve %zu bytes of LDS: %s", fn, lds, hipGetErrorString(e)); return kErrLaunch; }
       granted = true;
     }
   }
-  hipLaunchKernelGGL((attn_prefill_kernel<DT, MI, NG>), dim3((a.M + 64 * MI - 1) / (64 * MI), a.H, a.B), dim3(NG * kPfThreads), lds, st, a);
+  hipLaunchKernelGGL((attn_prefill_kernel<DT, MI, NG, NW>), dim3((a.M + 16 * NW * MI - 1) / (16 * NW * MI), a.H, a.B), dim3(NG * NW * kWave), lds, st, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_last_error("%s: launch failed: %s", fn, hipGetErrorString(e)); return kErrLaunch; }
   return kOk;
@@ -525,10 +532,17 @@ static int launch_prefill_attn_t(const PrefillAttnArgs& a, hipStream_t st) {
   // 128 query rows per workgroup from 1.5 workgroups per compute unit on, else 64 (half the rows per wave)
   const int64_t cu = compute_units();
   if ((int64_t)((a.M + 127) / 128) * a.H * a.B * 2 >= cu * 3) return launch_prefill_attn_form<DT, 2, 1>(a, st);
-  // chunks of up to one 64-row workgroup per compute unit: three groups of waves share its key tiles (four spill); prompts of
-  // up to ~1.5: two.  us with one / two / three groups: 512 rows of 32 heads (256 workgroups) 17.1 / 15.3 / 15.7, the same behind 1000
-  // tokens 42.7 / 34.0 / 31.7, two chunks of 77 rows behind 1411 tokens (128) 42.0 / 33.4 / 30.5; 700 rows (352) 26.5 / 23.2 /
-  // 23.4, 1024 rows (512) 37.3 / 38.9 / 37.7
+  // Fewer 64-row workgroups than compute units leave part of the chip idle, and one that has a compute unit to itself waits out every load and
+  // barrier.  Where 32-row workgroups (two waves per group, the rest of the LDS for a fourth group) are one per compute unit at most, they:
+  // us per call, 64 rows in three groups (two from 128 rows on) -> this: two chunks of 77 rows of 32 / 8 heads behind 1411 tokens 32.0 -> 25.6, one of
+  // 40 behind 900 22.4 -> 18.9, 127 behind 1000 24.4 -> 19.0, 200 behind 1000 30.1 -> 22.6, two of 100 behind 500 17.3 -> 14.4, eight of 32 behind 400
+  // (256 workgroups) 17.3 -> 15.9; one more round of them loses: two of 130 behind 300 (320 workgroups) 14.4 -> 18.8.  Three groups of them 29.3,
+  // 20.4, 21.1, 25.3 at the first four; 16 rows and one wave per group no better at 40 rows, 46 at the first.
+  if ((int64_t)((a.M + 31) / 32) * a.H * a.B <= cu) return launch_prefill_attn_form<DT, 1, 4, 2>(a, st);
+  // Up to ~1.5 of 64 rows: three groups of waves share a workgroup's key tiles below 128 rows (four spill), two from there on: 512 rows of 32 heads
+  // (256 workgroups) 18.0 / 15.9 / 15.4 us with one / two / three groups, 700 rows (352) 23.7 / 20.3 / 19.1, 1024 rows (512) 37.3 / 38.9 / 37.7.  The
+  // half microsecond that the third would give there (0.2 % of a prompt pass of 32 layers) does not pay for another order of the sums: the
+  // layers hand a flipped rounding on until the logits of 512 rows end 0.04 (relative) from the present ones.
   const int64_t tiles = (int64_t)((a.M + 63) / 64) * a.H * a.B;
   if (tiles <= cu && a.M < 128) return launch_prefill_attn_form<DT, 1, 3>(a, st);
   if (tiles * 2 <= cu * 3) return launch_prefill_attn_form<DT, 1, 2>(a, st);

@@ -51,6 +51,14 @@ def test_chunks(dtype, B, M, H, Hk, start):
     _check(out[:, rows, :heads], ref, float(v.abs().max()), dtype)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,M,H,Hk,start", [(1, 31, 2, 2, 0), (1, 32, 8, 2, 33), (3, 33, 4, 2, 62), (2, 95, 4, 4, 161), (1, 97, 4, 1, 1), (1, 256, 32, 8, 70),
+                                            (8, 32, 32, 32, 225), (8, 40, 32, 8, 90), (1, 257, 32, 32, 0), (12, 30, 32, 8, 5), (13, 30, 32, 8, 500)])
+def test_chunks_around_the_rules(dtype, B, M, H, Hk, start):
+    """32 rows per workgroup up to 256 workgroups, 64 in groups up to 384, then without; fewer key tiles than groups, unequal shares of them."""
+    test_chunks(dtype, B, M, H, Hk, start)
+
+
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("M,H", [(77, 4), (200, 4), (512, 70)])
 def test_padding_masks(M, H, causal):
