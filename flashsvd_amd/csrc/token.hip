@@ -1,7 +1,7 @@
 // The few words of state between two decoded tokens: the greedy token of every row and its next position, and the state that a
 // caller sets before a step, one launch each instead of a chain of library launches.
 //   greedy token, one sequence of 32000 logits, on every token of the graph engine: the library's argmax took 13.0 us, the copy of its
-//     result and the position increment 6 with their gaps; this takes 5.9, bound by the one compute unit that reads the row.
+//     result and the position increment 6 with their gaps; this takes 3.8, bound by the one compute unit that reads the row.
 //   state, once per prompt in a generation: three 4-byte copies of 3 to 6 us each in front of the resident step, two in front of a
 //     graph -> one launch.  The steps advance their own state, so a generated token gains nothing from it; a program that sets the
 //     state before every token of the resident step saves 46 us on each.
@@ -21,46 +21,106 @@ __device__ __forceinline__ uint32_t order_key(uint32_t p) {
   return (p & 0x8000u) ? 0xffffu - p : p | 0x8000u;
 }
 
+// two 16-bit patterns as unsigned 16-bit integers in the order of their values (a NaN above everything of its sign, -0 next below +0)
+typedef short i16x2_t __attribute__((ext_vector_type(2)));
+typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ u16x2_t order_pair(uint32_t w) {
+  const i16x2_t p = __builtin_bit_cast(i16x2_t, w);
+  return __builtin_bit_cast(u16x2_t, (i16x2_t)(p ^ ((p >> 15) | (short)0x8000)));
+}
+
 // One workgroup per row: the row is requested in rounds of four 16-byte pieces per thread (32768 elements), so what it takes is
-// one round trip per round and the 60 GB/s of one compute unit.  Ties go to the lowest index and NaN counts as the largest value, as
-// torch.argmax has it.
+// one round trip per round and the 60 GB/s of one compute unit.  Beside that every instruction per element shows, 32 of them in a thread: a
+// first pass takes the maximum alone, two elements to an instruction; then the threads that hold it look for it in the round where they met
+// it.  us per launch in a graph, value and index carried along element by element -> this: 32000 logits of 1 / 16 / 64 rows 5.3 -> 3.8, 5.9 -> 4.2,
+// 6.1 -> 4.4, 128256 of 1 / 16 rows 14.7 -> 6.0, 15.2 -> 6.5.  Ties go to the lowest index and NaN counts as the largest value, as torch.argmax
+// has it: a row with a NaN (its largest magnitude tells), or whose largest value is a zero of either sign, is looked through element by element.
 template <int DT>
 __global__ __launch_bounds__(kPickThreads) void greedy_token_kernel(const uint16_t* __restrict__ logits, int64_t ld, int64_t* __restrict__ tokens,
                                                                    int64_t ldt, int32_t* __restrict__ positions, int V) {
   const uint16_t* row = logits + (int64_t)blockIdx.x * ld;
   const int tid = threadIdx.x, pieces = V >> 3;
-  uint32_t best = 0, at = 0x7fffffffu;
-  const auto take = [&](uint32_t p, uint32_t i) {
-    const uint32_t k = order_key<DT>(p);
-    if (k > best) { best = k; at = i; }                // a thread meets its elements in ascending order
-  };
-  for (int c0 = 0; c0 < pieces; c0 += kPickThreads * kPickLoads) {
-    u32x4_t v[kPickLoads];
+  __shared__ uint32_t top[kPickThreads / kWave], far[kPickThreads / kWave], first[kPickThreads / kWave];
+  const auto fetch = [&](int c0, u32x4_t (&v)[kPickLoads]) {
 #pragma unroll
     for (int j = 0; j < kPickLoads; ++j) v[j] = *reinterpret_cast<const u32x4_any_t*>(row + (int64_t)min(c0 + j * kPickThreads + tid, pieces - 1) * 8);
+  };
+  u32x4_t v[kPickLoads];
+  constexpr int kTail = -1;
+  uint32_t best = 0, mag = 0;                          // the largest of this thread and the largest magnitude
+  int where = 0;                                       // the first round with the largest
+  for (int c0 = 0; c0 < pieces; c0 += kPickThreads * kPickLoads) {
+    fetch(c0, v);
+    u16x2_t most = {0, 0}, wide = {0, 0};
 #pragma unroll
-    for (int j = 0; j < kPickLoads; ++j) {
-      const int c = c0 + j * kPickThreads + tid;
-      if (c >= pieces) break;
+    for (int j = 0; j < kPickLoads; ++j) {             // pieces past the end are the last one once more
       const uint32_t w[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
 #pragma unroll
-      for (int e = 0; e < 8; ++e) take((w[e >> 1] >> (16 * (e & 1))) & 0xffffu, c * 8 + e);
+      for (int e = 0; e < 4; ++e) {
+        most = __builtin_elementwise_max(most, order_pair(w[e]));
+        wide = __builtin_elementwise_max(wide, __builtin_bit_cast(u16x2_t, w[e] & 0x7fff7fffu));
+      }
+    }
+    const uint32_t k = max((uint32_t)most.x, (uint32_t)most.y);
+    if (k > best) { best = k; where = c0; }
+    mag = max(mag, max((uint32_t)wide.x, (uint32_t)wide.y));
+  }
+  const int t = pieces * 8 + tid;                      // at most seven elements behind the last piece
+  const uint32_t tail = t < V ? row[t] : 0xffffu;
+  if (t < V) {
+    const uint32_t k = order_pair(tail).x;
+    if (k > best) { best = k; where = kTail; }
+    mag = max(mag, tail & 0x7fffu);
+  }
+  const auto all_max = [&](uint32_t x, uint32_t* red) {
+#pragma unroll
+    for (int o = 32; o; o >>= 1) x = max(x, (uint32_t)__shfl_xor((int)x, o));
+    if ((tid & 63) == 0) red[tid >> 6] = x;
+  };
+  all_max(best, top);
+  all_max(mag, far);
+  __syncthreads();
+  uint32_t highest = 0, widest = 0;
+#pragma unroll
+  for (int i = 0; i < kPickThreads / kWave; ++i) { highest = max(highest, top[i]); widest = max(widest, far[i]); }
+  // the lowest index that holds the largest value
+  uint32_t at = 0xffffffffu;
+  const auto look = [&](int c0, auto hit) {
+#pragma unroll
+    for (int j = 0; j < kPickLoads; ++j) {
+      const uint32_t w[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
+      const int c = c0 + j * kPickThreads + tid;
+      if (c >= pieces) break;
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (hit((w[e >> 1] >> (16 * (e & 1))) & 0xffffu)) at = min(at, (uint32_t)(c * 8 + e));
+    }
+  };
+  constexpr int kRound = kPickThreads * kPickLoads;
+  if (widest > (DT == 1 ? 0x7c00u : 0x7f80u) || highest == 0x8000u) {      // a NaN, or zero, which -0 equals
+    const uint32_t least = highest == 0x8000u && widest <= (DT == 1 ? 0x7c00u : 0x7f80u) ? 0x8000u : 0x10000u;
+    const auto hit = [&](uint32_t p) { return order_key<DT>(p) >= least; };
+    for (int c0 = 0; c0 < pieces; c0 += kRound) {
+      fetch(c0, v);
+      look(c0, hit);
+    }
+    if (t < V && hit(tail)) at = min(at, (uint32_t)t);
+  } else if (best == highest) {
+    if (where == kTail) {
+      at = (uint32_t)t;
+    } else {
+      if (where + kRound < pieces) fetch(where, v);    // not the round that is still in registers
+      look(where, [&](uint32_t p) { return (uint32_t)order_pair(p).x == highest; });
     }
   }
-  if (pieces * 8 + tid < V) take(row[pieces * 8 + tid], pieces * 8 + tid);
-  unsigned long long m = ((unsigned long long)best << 32) | (0xffffffffu - at);
 #pragma unroll
-  for (int o = 32; o; o >>= 1) {
-    const unsigned long long other = __shfl_xor(m, o);
-    m = other > m ? other : m;
-  }
-  __shared__ unsigned long long red[kPickThreads / kWave];
-  if ((tid & 63) == 0) red[tid >> 6] = m;
+  for (int o = 32; o; o >>= 1) at = min(at, (uint32_t)__shfl_xor((int)at, o));
+  if ((tid & 63) == 0) first[tid >> 6] = at;
   __syncthreads();
   if (tid == 0) {
 #pragma unroll
-    for (int i = 1; i < kPickThreads / kWave; ++i) m = red[i] > m ? red[i] : m;
-    tokens[(int64_t)blockIdx.x * ldt] = (int64_t)(0xffffffffu - (uint32_t)m);
+    for (int i = 1; i < kPickThreads / kWave; ++i) at = min(at, first[i]);
+    tokens[(int64_t)blockIdx.x * ldt] = (int64_t)at;
     if (positions) positions[blockIdx.x] += 1;
   }
 }

@@ -34,6 +34,35 @@ def test_greedy_token_is_the_argmax(dtype, B, V, off):
         assert pos.tolist() == list(range(1, B + 1))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("V,off", [(5, 0), (32768, 0), (32769, 2), (65535, 1), (70007, 0)])
+def test_greedy_token_where_the_largest_lies(V, off, dtype):
+    """The largest value in the first piece, in the first and a later round, in the last round, behind the last whole piece; only zeros above the
+    rest, of either sign; a NaN of either sign; the lowest finite value."""
+    from flashsvd_amd import hip_ops
+    x = -torch.rand(14, V + off, generator=torch.Generator().manual_seed(V)).to(dtype)[:, off:] - 1
+    first, mid, last = 0, V // 2, V - 1
+    spots = [(first,), (mid,), (last,), (mid, last), (first, mid), (max(0, V - V % 8 - 1),), (min(V - 1, 32767), last)]
+    want = []
+    for r, s in enumerate(spots):
+        x[r, list(s)] = 3.0
+        want.append(min(s))
+    x[7, [mid, last]] = torch.tensor([-0.0, 0.0], dtype=dtype)
+    x[8, [mid, last]] = torch.tensor([0.0, -0.0], dtype=dtype)
+    x[9, [mid, last]] = -0.0
+    x[10, last] = float("nan")
+    x[11, first], x[12, mid] = float("inf"), float("nan")
+    x.view(torch.int16)[11:13, last] = -1               # a negative NaN
+    x[13] = torch.finfo(dtype).min
+    want += [mid, mid, mid, last, last, mid, 0]
+    rows = torch.empty(14, V + off, dtype=dtype, device="cuda")
+    got = rows[:, off:]
+    got.copy_(x.cuda())
+    tokens = torch.full((14, 1), -7, dtype=torch.long, device="cuda")
+    hip_ops.greedy_token_(got, tokens)
+    assert tokens[:, 0].tolist() == want
+
+
 def test_refusals_and_state_rows():
     from flashsvd_amd import hip_ops
     x = torch.zeros(2, 64, dtype=torch.bfloat16, device="cuda")
