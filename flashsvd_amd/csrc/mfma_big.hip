@@ -1,5 +1,6 @@
 // Projections of long prompts: 256 x 256 output tiles, one workgroup of eight waves per compute unit that walks its share of
-// the tiles.
+// the tiles.  They serve a K below 320 and the pair where the tiles of mfma_quad.hip cost more (see big_pair_is_ahead there); the rest runs there, whose
+// four waves are ahead (q, k and v of 32 heads at 16384 x 1664 696 -> 594 us).
 //
 // What bounds a large product on this chip is cycles and clock alike: under a stream of these products the clock stays at 1.95 to
 // 2.2 GHz (1.65 in the first milliseconds of a burst), the matrix cores are busy in 50 to 63 % of the cycles (counters), and
@@ -14,7 +15,8 @@
 // multiply theirs, then the other way round, a bare barrier between the turns (published as "ping-pong" scheduling for this
 // family of chips) and the multiplying wave at raised priority (12 % slower without).  A step, 2048
 // cycles of products, takes 3260 to 3340 with its share of the epilogue (a single matrix, K = 4096 and 1664; 4040 for the pair);
-// four waves of 128 x 128, which read a third less from LDS, were no faster.
+// four waves of 128 x 128, which read a third less from LDS, were no
+// faster in this turn-taking (with reads and loads laid out between their own products they are: mfma_quad.hpp).
 //
 // The walk over the tiles is one stream: the first stage of the next tile is requested during the last step of this one, and
 // a finished tile leaves from the accumulators (pairs of 8-byte pieces become 16-byte ones by a row swap between lanes)

@@ -1,5 +1,7 @@
 // Projections and head expansions of prompts of 128 to about 3000 rows (head expansions from 16): workgroups of eight waves, one
-// per output tile, operand rows straight into a ring of three to five LDS stages.
+// per output tile, operand rows straight into a ring of three to five LDS stages.  They serve a K below 320, the pair in the rounding that keeps the
+// gate in 32 bits and ragged rows off the 4-byte grid; everything else is ahead on the four-wave tiles of mfma_quad.hip (figures there).  Times below
+// at a longer K are those by which the rules were set.
 //
 // Up to a few tiles per compute unit neither form beside this one fits: the two-stage tiles of mfma_gemm.hip rely on a second
 // workgroup of the compute unit to cover a load distance of one step and wait out most of it, and the 256 x 256 tiles of
@@ -12,8 +14,7 @@
 //
 // LDS rows are 128 bytes (64 of K), their eight 16-byte pieces XOR-swizzled by row % 8.  KH = 2: waves 4-7 take the second half
 // of every 128 of K and hand their sums to waves 0-3 through LDS at the end; sums run over K in the order of the forms of
-// mfma_gemm.hip.  The gate / up pair runs its two products one after the other over the same tile.  A long K with few tiles runs in
-// shares of K over workgroups (kMidShare), added up by a launch of their own (share_sum_kernel).
+// mfma_gemm.hip.  The gate / up pair runs its two products one after the other over the same tile.
 #include <algorithm>
 
 #include "common.hpp"
