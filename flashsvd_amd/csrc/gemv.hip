@@ -462,7 +462,10 @@ __global__ __launch_bounds__(kThreads) void qkv_rope_append_kernel(QkvArgs a) {
 // a wave keeps one window of P pieces (16 bytes per lane each) for R rows, eight pieces in all, and asks for a piece of its next row as soon
 // as it has consumed the one in its place; the activations sit in registers, so a piece costs its products and nothing else.  The sums
 // run in the order of linear_kernel: the same bits.  32000 x 4096, weights from HBM: one row 44.6 -> 39.5 us (6.6 TB/s), with the norm 45.0 -> 40.8, two
-// rows 49.9 -> 42.5; 32000 x 2048 one row 25.7 -> 21.7.  Below 64 rows per compute unit (16 per wave) linear_kernel stays.
+// rows 49.9 -> 42.5; 32000 x 2048 one row 25.7 -> 21.7.  Shorter rows, several to a window, one row / one with the norm / two: 32000 x 512
+// 8.8 -> 8.0, 10.7 -> 8.6, 13.9 -> 10.0, 128256 x 512 25.3 -> 24.2, 30.0 -> 24.7, 46.6 -> 28.1, 32000 x 1024 12.9 -> 12.7, 14.6 -> 13.3, 17.8 -> 14.5, two rows of
+// 128256 x 1024 57.5 -> 45.3; one row of that 41.7 -> 42.8, which therefore stays with linear_kernel above 128 rows per compute unit, as everything
+// does below 64 (16 per wave).
 // ---------------------------------------------------------------------------------------
 template <int DT, int BATCH, int P>
 __global__ __launch_bounds__(kThreads) void linear_slab_kernel(LinearArgs a) {
@@ -645,25 +648,27 @@ static int launch_linear_b(const LinearArgs& a, int cfg, hipStream_t st) {
   return kOk;
 }
 
-// long outputs whose rows are one window: 2048 or 4096 values, 64 rows and more per compute unit
-template <int DT>
+// long outputs whose rows are a window or a part of one: 512, 1024, 2048 or 4096 values, 64 rows and more per compute unit
+template <int DT, int P>
 static int launch_linear_slab(const LinearArgs& a, hipStream_t st) {
   const dim3 grid(2 * compute_units());
-  if (a.K == 4096) {
-    if (a.B == 1) hipLaunchKernelGGL((linear_slab_kernel<DT, 1, 8>), grid, dim3(kThreads), 0, st, a);
-    else hipLaunchKernelGGL((linear_slab_kernel<DT, 2, 8>), grid, dim3(kThreads), 0, st, a);
-  } else {
-    if (a.B == 1) hipLaunchKernelGGL((linear_slab_kernel<DT, 1, 4>), grid, dim3(kThreads), 0, st, a);
-    else hipLaunchKernelGGL((linear_slab_kernel<DT, 2, 4>), grid, dim3(kThreads), 0, st, a);
-  }
+  if (a.B == 1) hipLaunchKernelGGL((linear_slab_kernel<DT, 1, P>), grid, dim3(kThreads), 0, st, a);
+  else hipLaunchKernelGGL((linear_slab_kernel<DT, 2, P>), grid, dim3(kThreads), 0, st, a);
   FSVD_CHECK_LAUNCH("fsvd_linear");
   return kOk;
 }
 template <int DT>
 static int launch_linear_t(const LinearArgs& a, int cfg, hipStream_t st) {
-  if (cfg == 0 && a.B <= 2 && (a.K == 2048 || a.K == 4096) && a.positions == nullptr && compute_units() > 0 && a.N >= 64 * compute_units() &&
-      a.ldw % 8 == 0 && aligned16(a.W) && below_4gib(a.N, a.ldw))
-    return launch_linear_slab<DT>(a, st);
+  if (cfg == 0 && a.B <= 2 && a.positions == nullptr && compute_units() > 0 && a.N >= 64 * compute_units() && a.ldw % 8 == 0 && aligned16(a.W) && below_4gib(a.N, a.ldw)) {
+    switch (a.K) {
+      case 512: return launch_linear_slab<DT, 1>(a, st);
+      case 1024:
+        if (a.B == 1 && a.N > 128 * compute_units()) break;
+        return launch_linear_slab<DT, 2>(a, st);
+      case 2048: return launch_linear_slab<DT, 4>(a, st);
+      case 4096: return launch_linear_slab<DT, 8>(a, st);
+    }
+  }
   const bool vec = (a.K % 8 == 0) && (a.ldw % 8 == 0) && aligned16(a.W);
   const int batch = a.B >= 4 && a.K <= 16384 ? 4 : (a.B >= 2 ? 2 : 1);
   if (vec) {

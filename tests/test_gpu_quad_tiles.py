@@ -87,7 +87,7 @@ def test_heads(B, T, H, Hk, R, form, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("N,K", [(16384, 4096), (16387, 2048), (32001, 4096), (128257, 2048)])
+@pytest.mark.parametrize("N,K", [(16384, 4096), (16387, 2048), (32001, 4096), (128257, 2048), (16385, 512), (32003, 1024), (32769, 1024), (50304, 512)])
 @pytest.mark.parametrize("B", [1, 2])
 def test_vocabulary_stream(B, N, K, dtype):
     """Slabs of unequal length, rows that are no multiple of the window, strided weight rows, norm, bias and residual."""
