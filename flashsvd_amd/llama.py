@@ -13,7 +13,6 @@ All compute goes through the HIP library; a module asked to run on CPU tensors r
 """
 from __future__ import annotations
 
-import operator
 import os
 from types import SimpleNamespace
 from typing import Optional
@@ -56,20 +55,6 @@ class LlamaRMSNorm(nn.Module):
     def forward(self, hidden_states: torch.Tensor) -> torch.Tensor:
         _require_gpu(hidden_states, "LlamaRMSNorm")
         return hip_ops.rmsnorm(hidden_states, self.weight, self.variance_epsilon)
-
-
-# the factor modules of a half layer straight from the module's own table (asked for several times per layer and call: attribute by
-# attribute the fourteen of them took 7 us of a layer's host time)
-_ATTENTION_NAMES = ("q_v_proj", "q_u_proj", "k_v_proj", "k_u_proj", "v_v_proj", "v_u_proj", "o_v_proj", "o_u_proj")
-_MLP_NAMES = ("gate_v_proj", "gate_u_proj", "up_v_proj", "up_u_proj", "down_v_proj", "down_u_proj")
-_ATTENTION_FACTORS, _MLP_FACTORS = operator.itemgetter(*_ATTENTION_NAMES), operator.itemgetter(*_MLP_NAMES)
-
-
-def _from_table(module: nn.Module, factors, names):
-    try:
-        return factors(module._modules)
-    except KeyError:                                   # a factor that is no registered module (a plain attribute, a property of a subclass)
-        return tuple(getattr(module, name) for name in names)
 
 
 class LlamaRotaryEmbedding(nn.Module):
@@ -164,7 +149,8 @@ class SVD_LlamaAttention(nn.Module):
         self._packed_qkv_v = None
 
     def _factor_modules(self):
-        return _from_table(self, _ATTENTION_FACTORS, _ATTENTION_NAMES)
+        return (self.q_v_proj, self.q_u_proj, self.k_v_proj, self.k_u_proj, self.v_v_proj, self.v_u_proj, self.o_v_proj,
+                self.o_u_proj)
 
     def _ensure_runtime_state(self) -> None:
         """Idempotent.  Packs [q_v; k_v; v_v] into one row-contiguous buffer (the module weights
@@ -601,7 +587,7 @@ class SVD_LlamaMLP(nn.Module):
                 setattr(self, name, {})
 
     def _factor_modules(self):
-        return _from_table(self, _MLP_FACTORS, _MLP_NAMES)
+        return (self.gate_v_proj, self.gate_u_proj, self.up_v_proj, self.up_u_proj, self.down_v_proj, self.down_u_proj)
 
     def _run_quantized(self, x: torch.Tensor, *, norm_weight=None, eps: float = 1e-6, residual=None, mode: Optional[int] = None):
         """The same four stages with int4 factors: each projection through the kernel that fits its module."""

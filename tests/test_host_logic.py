@@ -344,3 +344,20 @@ def test_factor_modules_need_not_be_registered():
             half._factor_modules()
         half.__dict__[name] = lin
         assert all(a is b for a, b in zip(half._factor_modules(), before)) and len(half._factor_modules()) == len(before)
+
+
+@pytest.mark.parametrize("half,name", [("self_attn", "q_u_proj"), ("mlp", "gate_u_proj")])
+def test_factor_modules_are_what_the_attributes_are(half, name):
+    """A factor that a subclass provides in place of the registered one, and one put over it on the instance, are the factors asked about."""
+    from flashsvd_amd import llama
+    model = llama.build_model(hidden_size=128, num_heads=2, num_kv_heads=2, head_dim=64, intermediate_size=128, num_layers=1, vocab_size=32,
+                              attn_rank=32, mlp_rank=32)
+    part = getattr(model.model.layers[0], half)
+    own, other = getattr(part, name), torch.nn.Identity()
+    part.__class__ = type("Provided", (type(part),), {name: property(lambda self: other)})
+    assert getattr(part, name) is other
+    assert any(m is other for m in part._factor_modules()) and not any(m is own for m in part._factor_modules())
+    part.__class__ = type(part).__mro__[1]
+    part.__dict__[name] = other
+    assert getattr(part, name) is other
+    assert any(m is other for m in part._factor_modules()) and not any(m is own for m in part._factor_modules())
