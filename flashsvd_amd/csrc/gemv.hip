@@ -652,6 +652,7 @@ static int launch_linear_b(const LinearArgs& a, int cfg, hipStream_t st) {
 template <int DT, int P>
 static int launch_linear_slab(const LinearArgs& a, hipStream_t st) {
   const dim3 grid(2 * compute_units());
+  set_last_form("rows in a window");
   if (a.B == 1) hipLaunchKernelGGL((linear_slab_kernel<DT, 1, P>), grid, dim3(kThreads), 0, st, a);
   else hipLaunchKernelGGL((linear_slab_kernel<DT, 2, P>), grid, dim3(kThreads), 0, st, a);
   FSVD_CHECK_LAUNCH("fsvd_linear");

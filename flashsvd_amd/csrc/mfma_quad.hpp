@@ -628,7 +628,10 @@ static int launch_quad_t(QuadArgs& q, hipStream_t st, const char* who) {
   q.mt = (q.a[0].B + BM - 1) / BM;
   const int64_t all = (int64_t)q.nt * q.mt * (EPI == kQuadShare ? q.shares : 1);
   const int64_t grid = quad_stream(TM, TN) ? std::min<int64_t>(all, (int64_t)OCC * compute_units()) : all;
-  static constexpr FormText form = form_text(EPI == kQuadShare ? "shares " : (RAG ? "any ring " : "ring "), BM, BN, EPI == kQuadPair ? " pair" : (EPI == kQuadHeads ? " heads" : ""));
+  constexpr bool kAlone = OCC == 1 && TM == 4 && TN == 4 && (EPI == kQuadPlain || EPI == kQuadPair);      // beside the form of two workgroups per compute unit
+  static constexpr FormText form = form_text(EPI == kQuadShare ? "shares " : (RAG ? "any quad " : "quad "), BM, BN,
+                                             EPI == kQuadHeads ? " heads" : (EPI == kQuadPair ? (kAlone ? " pair alone" : " pair") :
+                                             (H == 2 ? " halves" : (CUT ? " ranges" : (kAlone ? " alone" : "")))));
   set_last_form(form.s);
   hipLaunchKernelGGL((gemm_quad_kernel<DT, EPI, TM, TN, NSX, NSW, OCC, RAG, H, CUT>), dim3((unsigned)grid), dim3(kQuadThreads), lds, st, q);
   hipError_t e = hipGetLastError();

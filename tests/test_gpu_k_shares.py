@@ -1,4 +1,4 @@
-"""Projections of a long K in shares over workgroups (csrc/mfma_mid.hip) at the edges of their tilings: partial row and column
+"""Projections of a long K in shares over workgroups (csrc/mfma_quad.hip) at the edges of their tilings: partial row and column
 tiles, shares of unequal length, strided and odd rows, bias and residual, against the same product in fp32; and the two-stage
 ring of the head expansions at its shortest rank."""
 import os
@@ -18,7 +18,8 @@ pytestmark = pytest.mark.gpu
     (128, 1536, 11008, "shares 64 x 128"), (191, 1027, 8256, "shares 64 x 128"), (130, 3001, 4096, "shares 64 x 128"),
     (193, 1030, 8192, "shares 128 x 128"), (333, 3070, 4160, "shares 128 x 128"),
     (512, 1500, 5504, "shares 256 x 128"), (769, 1533, 8320, "shares 128 x 128"), (1000, 1533, 8320, "shares 256 x 128"), (2047, 2390, 8192, "shares 256 x 128"),
-    (512, 1536, 11008, "shares 128 x 128"), (420, 3072, 4096, "ring 128 x 64"), (512, 4096, 4096, "ring 128 x 64"), (127, 3072, 4096, "tiles 32 x 64"),
+    (150, 1027, 4096, "shares 64 x 64"), (200, 515, 4096, "shares 64 x 64"), (512, 1024, 4160, "shares 64 x 64"),
+    (512, 1536, 11008, "shares 128 x 128"), (420, 3072, 4096, "quad 128 x 64 halves"), (512, 4096, 4096, "quad 128 x 64 halves"), (127, 3072, 4096, "tiles 32 x 64"),
 ])
 def test_linear(B, N, K, form, dtype):
     from flashsvd_amd import hip_ops
@@ -34,6 +35,21 @@ def test_linear(B, N, K, form, dtype):
     _check(out[:B, 1:N + 1], ref, "bias, residual, odd output")
     assert bool((out[B] == 7).all()) and bool((out[:, 0] == 7).all()) and bool((out[:, N + 1:] == 7).all())
     assert torch.equal(y, hip_ops.linear(x, w)), "repeat differs"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,N,K", [(150, 1027, 4096), (200, 515, 4096), (333, 259, 6208)])
+def test_ranges_apart_and_in_a_row_give_the_same_bits(B, N, K, dtype):
+    """A K in ranges: one workgroup each with scratch of the call's own, without it as the registered buffer or one workgroup has them."""
+    from flashsvd_amd import _lib, hip_ops
+    x, w = _rand(B, K, seed=1, dtype=dtype), _rand(N, K, std=K ** -0.5, seed=2, dtype=dtype)
+    apart = hip_ops.linear(x, w)
+    assert form_taken() == "shares 64 x 64"
+    y = torch.empty_like(apart)
+    code = 1 if dtype == torch.float16 else 0
+    assert _lib.load().fsvd_linear(x.data_ptr(), K, w.data_ptr(), K, None, None, 0.0, None, 0, y.data_ptr(), N, B, N, K, 0, code, hip_ops._stream()) == 0
+    assert not form_taken().startswith("shares")
+    assert torch.equal(apart, y)
 
 
 def test_calls_on_two_streams_are_independent():

@@ -31,13 +31,14 @@ def _linear(B, N, K, dtype, any_grid=False):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,N,K,form", [
-    (1036, 11077, 320, "ring 256 x 256"), (706, 11209, 320, "ring 256 x 192"), (341, 12357, 320, "ring 128 x 192"),
-    (777, 7569, 320, "ring 256 x 128"), (514, 9972, 320, "ring 192 x 128"), (130, 11060, 320, "ring 128 x 128"),
-    (519, 11227, 320, "ring 128 x 128"), (69, 17004, 1024, "ring 128 x 96"), (99, 8635, 320, "ring 128 x 64"),
-    (133, 9272, 320, "ring 64 x 128"), (66, 8328, 320, "ring 96 x 64"), (3648, 1056, 320, "ring 64 x 96"),
-    (33, 4170, 320, "ring 64 x 64"),
-    (197, 5541, 384, "ring 128 x 64"), (132, 5545, 384, "ring 96 x 64"), (128, 8256, 384, "ring 64 x 96"), (135, 1362, 384, "ring 64 x 64"),   # K halved
-    (130, 259, 320, "ring 64 x 64"), (300, 517, 1088, "ring 64 x 64"), (301, 261, 2176, "ring 64 x 64"),                                       # K in ranges
+    (1036, 11077, 320, "quad 256 x 256"), (706, 11209, 320, "quad 256 x 192"), (341, 12357, 320, "quad 128 x 192"),
+    (777, 7569, 320, "quad 256 x 128"), (514, 9972, 320, "quad 192 x 128"), (130, 11060, 320, "quad 128 x 128"),
+    (519, 11227, 320, "quad 128 x 128 alone"), (69, 17004, 1024, "quad 128 x 96"), (99, 8635, 320, "quad 128 x 64"),
+    (133, 9272, 320, "quad 64 x 128"), (66, 8328, 320, "quad 96 x 64"), (3648, 1056, 320, "quad 64 x 96"),
+    (33, 4170, 320, "quad 64 x 64"),
+    (130, 259, 320, "quad 64 x 64"),
+    (197, 5541, 384, "quad 128 x 64 halves"), (132, 5545, 384, "quad 96 x 64 halves"), (128, 8256, 384, "quad 64 x 96 halves"), (135, 1362, 384, "quad 64 x 64 halves"),
+    (130, 259, 1088, "quad 64 x 64 ranges"), (300, 517, 1088, "quad 64 x 64 ranges"), (301, 261, 1920, "quad 64 x 64 ranges"),
 ])
 def test_linear(B, N, K, form, dtype):
     assert _linear(B, N, K, dtype) == form
@@ -45,8 +46,8 @@ def test_linear(B, N, K, form, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,N,K,form", [
-    (297, 12319, 323, "any ring 192 x 128"), (128, 8256, 322, "any ring 128 x 128"), (130, 5559, 383, "any ring 96 x 64"),
-    (130, 259, 321, "any ring 64 x 64"), (131, 8, 385, "any ring 64 x 64"), (128, 300, 320, "any ring 64 x 64"),
+    (297, 12319, 323, "any quad 192 x 128"), (128, 8256, 322, "any quad 128 x 128"), (130, 5559, 383, "any quad 96 x 64"),
+    (130, 259, 321, "any quad 64 x 64"), (131, 8, 385, "any quad 64 x 64"), (128, 300, 320, "any quad 64 x 64"),
 ])
 def test_linear_any_grid(B, N, K, form, dtype):
     assert _linear(B, N, K, dtype, any_grid=True) == form
@@ -54,12 +55,12 @@ def test_linear_any_grid(B, N, K, form, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,D,R,form", [
-    (341, 12357, 320, "ring 128 x 192 pair"), (783, 9447, 320, "ring 160 x 192 pair"), (409, 10404, 320, "ring 160 x 128 pair"),
-    (168, 27083, 1280, "ring 256 x 128 pair"), (261, 9918, 320, "ring 128 x 128 pair"), (67, 25091, 832, "ring 128 x 128 pair"),
-    (129, 17205, 896, "ring 96 x 192 pair"), (72, 12319, 320, "ring 96 x 96 pair"), (66, 8328, 320, "ring 64 x 96 pair"),
-    (130, 259, 320, "ring 64 x 64 pair"),
-    (341, 12357, 323, "any ring 128 x 192 pair"), (261, 9918, 322, "any ring 128 x 128 pair"), (129, 17205, 894, "any ring 96 x 192 pair"),
-    (130, 8954, 383, "any ring 96 x 96 pair"), (130, 259, 321, "any ring 64 x 96 pair"), (40, 8190, 330, "any ring 64 x 96 pair"),
+    (341, 12357, 320, "quad 128 x 192 pair"), (783, 9447, 320, "quad 160 x 192 pair"), (409, 10404, 320, "quad 160 x 128 pair"),
+    (168, 27083, 1280, "quad 256 x 128 pair"), (261, 9918, 320, "quad 128 x 128 pair"), (67, 25091, 832, "quad 128 x 128 pair alone"),
+    (129, 17205, 896, "quad 96 x 192 pair"), (72, 12319, 320, "quad 96 x 96 pair"), (66, 8328, 320, "quad 64 x 96 pair"),
+    (130, 259, 320, "quad 64 x 64 pair"),
+    (341, 12357, 323, "any quad 128 x 192 pair"), (261, 9918, 322, "any quad 128 x 128 pair"), (129, 17205, 894, "any quad 96 x 192 pair"),
+    (130, 8954, 383, "any quad 96 x 96 pair"), (130, 259, 321, "any quad 64 x 96 pair"), (40, 8190, 330, "any quad 64 x 96 pair"),
 ])
 def test_pair(B, D, R, form, dtype):
     from flashsvd_amd import hip_ops
@@ -76,10 +77,10 @@ def test_pair(B, D, R, form, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,T,H,Hk,R,form", [
-    (2, 866, 46, 9, 320, "ring 256 x 256 heads"), (2, 641, 48, 9, 320, "ring 192 x 128 heads"), (1, 650, 36, 7, 320, "ring 160 x 128 heads"),
-    (1, 391, 45, 9, 320, "ring 128 x 128 heads"), (2, 166, 36, 7, 320, "ring 96 x 128 heads"), (1, 130, 36, 7, 320, "ring 64 x 128 heads"),
-    (3, 11, 2, 1, 320, "ring 64 x 64 heads"), (1, 17, 3, 1, 384, "ring 64 x 64 heads"),
-    (1, 391, 45, 9, 322, "any ring 128 x 128 heads"), (2, 166, 36, 7, 322, "any ring 96 x 128 heads"), (3, 11, 2, 1, 382, "any ring 64 x 64 heads"),
+    (2, 866, 46, 9, 320, "quad 256 x 256 heads"), (2, 641, 48, 9, 320, "quad 192 x 128 heads"), (1, 650, 36, 7, 320, "quad 160 x 128 heads"),
+    (1, 391, 45, 9, 320, "quad 128 x 128 heads"), (2, 166, 36, 7, 320, "quad 96 x 128 heads"), (1, 130, 36, 7, 320, "quad 64 x 128 heads"),
+    (3, 11, 2, 1, 320, "quad 64 x 64 heads"), (1, 17, 3, 1, 384, "quad 64 x 64 heads"),
+    (1, 391, 45, 9, 322, "any quad 128 x 128 heads"), (2, 166, 36, 7, 322, "any quad 96 x 128 heads"), (3, 11, 2, 1, 382, "any quad 64 x 64 heads"),
 ])
 def test_heads(B, T, H, Hk, R, form, dtype):
     """Row tiles across sequences, rows past the cache dropped, tiles that straddle heads."""
@@ -95,11 +96,14 @@ def test_vocabulary_stream(B, N, K, dtype):
     x, w = _rand(B, K + 8, seed=1, dtype=dtype)[:, 8:], _rand(N, K + 8, std=K ** -0.5, seed=2, dtype=dtype)[:, :K]
     bias, res, nw = _rand(N, seed=3, dtype=dtype), _rand(B, N, seed=4, dtype=dtype), _rand(K, seed=5, dtype=dtype)
     ref = x.float() @ w.float().t()
-    _check(hip_ops.linear(x, w), ref.to(dtype), "plain")
+    y = hip_ops.linear(x, w)
+    assert form_taken() == ("vector" if (B, K) == (1, 1024) and N > 32768 else "rows in a window")
+    _check(y, ref.to(dtype), "plain")
+    assert torch.equal(y, hip_ops.linear(x, w, cfg=4)) and form_taken() == "vector"      # the same bits as four rows to a wave
     out = torch.full((B + 1, N + 3), 7.0, device="cuda", dtype=dtype)
     hip_ops.linear(x, w, bias, residual=res, out=out[:B, 1:N + 1])
     _check(out[:B, 1:N + 1], ((ref + bias.float()).to(dtype).float() + res.float()).to(dtype), "bias and residual")
     assert bool((out[B] == 7).all()) and bool((out[:, 0] == 7).all()) and bool((out[:, N + 1:] == 7).all())
     xn = hip_ops.rmsnorm(x, nw, 1e-6)
     _check(hip_ops.linear(x, w, norm_weight=nw), (xn.float() @ w.float().t()).to(dtype), "norm")
-    assert torch.equal(hip_ops.linear(x, w), torch.cat([hip_ops.linear(x[b:b + 1], w) for b in range(B)]))
+    assert torch.equal(y, torch.cat([hip_ops.linear(x[b:b + 1], w) for b in range(B)]))
