@@ -554,26 +554,16 @@ static int pick_ksplit_prompt(int64_t tiles, int ksteps, int K, size_t floats_pe
   return z > 1 ? fit_ksplit(z, tiles, ksteps, floats_per_share, ws, 8) : 1;
 }
 
-// how a K of 8192 and more would be cut over the 64 x 64 tiles with scratch at hand: shares, and the K steps of 64 in their unit (1 share:
-// another tile takes the shape)
-int gemm_tiles_shares(const MfmaArgs& a, int* unit) {
+// How the 64 x 64 tiles cut K where a buffer has room for the ranges' sums, whatever is registered: a caller that takes over their shapes adds
+// the ranges up in the same order, with and without a buffer.
+TilesCut gemm_tiles_cut(const MfmaArgs& a) {
   const auto count = [&](int bm, int bn) { return (int64_t)((a.N + bn - 1) / bn) * ((a.B + bm - 1) / bm); };
-  const int64_t big = count(128, 128), half = count(128, 64), small = count(64, 64);
-  if (big >= 144 || (half >= 160 && half <= 256 && a.K % 128 == 0)) return 1;
-  *unit = small < 320 && a.K % 128 == 0 ? 2 : 1;
-  const SplitWorkspace plenty{reinterpret_cast<float*>(16), ~(size_t)0, nullptr, 1 << 30};      // only counted with
-  return pick_ksplit_prompt(small, a.K / (64 * *unit), a.K, 0, plenty);
-}
-
-// Steps of 64 in a range of K where the 64 x 64 tiles cut a K below 8192 (0: they do not); a caller that takes over their shapes adds the
-// ranges up in the same order.
-int gemm_tiles_cut(const MfmaArgs& a) {
-  const auto count = [&](int bm, int bn) { return (int64_t)((a.N + bn - 1) / bn) * ((a.B + bm - 1) / bm); };
-  const int64_t small = count(64, 64);
-  if (count(128, 128) >= 144 || a.K >= 8192) return 0;
+  const int64_t half = count(128, 64), small = count(64, 64);
+  if (count(128, 128) >= 144 || (half >= 160 && half <= 256 && a.K % 128 == 0)) return TilesCut{0, 1, false};      // other tiles, unsplit
   const int unit = small < 320 && a.K % 128 == 0 ? 2 : 1, steps = a.K / (64 * unit);
-  const int z = pick_ksplit_prompt(small, steps, a.K, (size_t)64 * 64, split_workspace());
-  return z > 1 ? (steps + z - 1) / z * unit : 0;
+  const SplitWorkspace ws = split_workspace(), plenty{reinterpret_cast<float*>(16), ~(size_t)0, nullptr, 1 << 30};   // only counted with
+  const int z = pick_ksplit_prompt(small, steps, a.K, 0, plenty);
+  return TilesCut{z > 1 ? (steps + z - 1) / z * unit : 0, z, z > 1 && pick_ksplit_prompt(small, steps, a.K, (size_t)64 * 64, ws) == z};
 }
 
 template <int DT, bool DUAL, int WTM, int WT, int BK, int NW = 4, int PFSEL = 99, bool RAG = false>

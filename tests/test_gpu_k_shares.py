@@ -52,6 +52,49 @@ def test_ranges_apart_and_in_a_row_give_the_same_bits(B, N, K, dtype):
     assert torch.equal(apart, y)
 
 
+@pytest.mark.parametrize("B,N,K,form", [
+    (128, 1024, 4096, "tiles 64 x 64"), (128, 256, 8192, "tiles 64 x 64"), (150, 1027, 7168, "tiles 64 x 64"), (129, 1530, 11008, "tiles 64 x 64"),
+    (512, 1536, 11008, "tiles 64 x 64"), (333, 1536, 8192, "quad 64 x 64"), (333, 1024, 4096, "quad 64 x 64 ranges"),
+])
+def test_calls_without_scratch_split_in_the_registered_buffer(B, N, K, form):
+    """fsvd_linear, whose only scratch is the registered buffer; with that too small for the split, or with none, the same call runs unsplit."""
+    from flashsvd_amd import _lib, hip_ops
+    lib = _lib.load()
+    x, w = _rand(B, K, seed=1), _rand(N, K, std=K ** -0.5, seed=2)
+    y = torch.empty(B, N, device="cuda", dtype=torch.bfloat16)
+    ref = (x.float() @ w.float().t()).bfloat16()
+
+    def call():
+        y.fill_(7.0)
+        assert lib.fsvd_linear(x.data_ptr(), K, w.data_ptr(), K, None, None, 0.0, None, 0, y.data_ptr(), N, B, N, K, 0, 0, hip_ops._stream()) == 0
+        _check(y, ref, "without scratch")
+        return form_taken(), y.clone()
+
+    assert hip_ops.ensure_split_workspace(x.device)
+    taken, split = call()
+    assert taken == form
+    hip_ops.release_split_workspace(x.device)
+    small = torch.empty(1 << 20, dtype=torch.uint8, device="cuda")
+    try:
+        for buf, nbytes in ((small.data_ptr(), small.numel()), (None, 0)):
+            assert lib.fsvd_set_workspace(buf, nbytes, hip_ops._stream()) == 0
+            taken, y1 = call()
+            assert taken.startswith("quad")
+            assert K >= 8192 or torch.equal(y1, split)                                 # ranges of K are added up in the same order
+    finally:
+        assert hip_ops.ensure_split_workspace(x.device)
+
+
+@pytest.mark.parametrize("B,N,K,form", [(128, 1024, 3584, "tiles 64 x 64"), (130, 259, 2048, "tiles 64 x 64"), (512, 1024, 3328, "tiles 64 x 64"),
+                                        (512, 768, 3072, "quad 64 x 64 ranges"), (128, 1024, 1536, "quad 64 x 64 ranges")])
+def test_a_k_too_short_for_scratch(B, N, K, form):
+    from flashsvd_amd import hip_ops
+    x, w = _rand(B, K, seed=1), _rand(N, K, std=K ** -0.5, seed=2)
+    y = hip_ops.linear(x, w)
+    assert form_taken() == form
+    _check(y, (x.float() @ w.float().t()).bfloat16(), form)
+
+
 def test_calls_on_two_streams_are_independent():
     """Each call's sums lie in scratch of its own, the registered buffer stays as it is."""
     from flashsvd_amd import hip_ops
