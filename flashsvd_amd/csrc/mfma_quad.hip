@@ -116,30 +116,12 @@ static bool quad_range(const MfmaArgs& a, bool dual) {
 //   gain 1.25, a quarter of it padding: 420 x 3072 x 4096 24 -> 28, 200 x 3072 x 4096 17.0 -> 19.5; gain 1: 512 x 4096 x 4096 30.9 -> 31.8.  Not taken.
 //   no ring to compare with: from three shares over 3/16 of the compute units on: 128 x 3072 x 4096 21 -> 16, 154 x 2048 x 5504 22 -> 17.
 struct ShareForm { int bm, bn, shares, per; };
-static ShareForm share_form(const MfmaArgs& a) {
+// as many shares as there are compute units for
+static ShareForm filling_shares(const MfmaArgs& a, const RingRule& ring) {
   const ShareForm none{0, 0, 0, 0};
-  if (a.scratch_floats == 0 || a.B < 128 || a.K < 4096 || !quad_range(a, false) || !quad_grid(a, false) || gemm_big_apply(a, false)) return none;
   const int64_t cu = compute_units();
   const auto pad = [&](int64_t r) { return (a.B + r - 1) / r * r; };
   const int steps = a.K / 64;
-  const RingRule ring = gemm_mid_rule(a);
-  // K cut in ranges (see quad_sums): one workgroup per range and 64 x 64 tile where that beats one after the other (512 x 1024 x 4096 in two
-  // ranges 19.6 -> 16.4 us, 154 x 1024 x 4096 in six 18.6 -> 12.1)
-  const QuadSums sums = quad_sums(a);
-  if (sums.order == kOrderCut) {
-    const int64_t tiles = quad_tiles(a, 2, 2), shares = (steps + sums.per - 1) / sums.per;
-    const QuadCost c{0.49f, 0.227f, 2.66f, 0.355f};
-    const float apart = quad_us(c, tiles * shares, 2, (float)sums.per, cu) + 3.5f + (float)(shares * tiles * 4096) * 8.f / 4.5e6f;
-    if (apart < quad_us(c, tiles, 2, (float)steps, cu) && (size_t)(tiles * shares * 4096) <= a.scratch_floats) return ShareForm{64, 64, (int)shares, sums.per};
-  }
-  // the cut of the 64 x 64 tiles, where a tile of this kernel fills 70 percent of the compute units with it: the same bits
-  if (a.K >= 8192 && ring.area == 0) {
-    const int per = gemm_tiles_cut(a).per;
-    for (const int bm : {64, 128}) {
-      const int64_t t = quad_tiles(a, bm / 32, 4) * (per ? (steps + per - 1) / per : 0);
-      if (t * 10 >= 7 * cu && t <= cu && (size_t)t * bm * 128 <= a.scratch_floats) return ShareForm{bm, 128, (steps + per - 1) / per, per};
-    }
-  }
   const int bm = a.B <= 192 ? 64 : (a.B > 384 && pad(256) <= pad(128) ? 256 : 128);
   const int64_t tiles = quad_tiles(a, bm / 32, 4), area = (int64_t)bm * 128;
   int64_t shares = std::min<int64_t>(cu / tiles, steps / 8);                         // eight steps each at least
@@ -159,6 +141,32 @@ static ShareForm share_form(const MfmaArgs& a) {
     if (kLaunchUs + quad_pick(a, false, false).us < 0.9f * (kLaunchUs + us)) return none;
   }
   return ShareForm{bm, 128, (int)shares, per};
+}
+static ShareForm share_form(const MfmaArgs& a) {
+  const ShareForm none{0, 0, 0, 0};
+  if (a.scratch_floats == 0 || a.B < 128 || a.K < 4096 || !quad_range(a, false) || !quad_grid(a, false) || gemm_big_apply(a, false)) return none;
+  const int64_t cu = compute_units();
+  const int steps = a.K / 64;
+  const RingRule ring = gemm_mid_rule(a);
+  // the cut of the 64 x 64 tiles, where a tile of this kernel fills 70 percent of the compute units with it: the same bits
+  if (a.K >= 8192 && ring.area == 0) {
+    const int per = gemm_tiles_cut(a).per;
+    for (const int bm : {64, 128}) {
+      const int64_t t = quad_tiles(a, bm / 32, 4) * (per ? (steps + per - 1) / per : 0);
+      if (t * 10 >= 7 * cu && t <= cu && (size_t)t * bm * 128 <= a.scratch_floats) return ShareForm{bm, 128, (steps + per - 1) / per, per};
+    }
+  }
+  const ShareForm filling = filling_shares(a, ring);
+  if (filling.shares > 0) return filling;
+  // K cut in ranges (see quad_sums): one workgroup per range and 64 x 64 tile where that beats one after the other (512 x 1024 x 4096 in two
+  // ranges 19.6 -> 16.4 us, 154 x 1024 x 4096 in six 18.6 -> 12.1).  Shapes that fill the chip with shares of 64 x 128 do not come here (128 x 3072 x 5120
+  // 16.9 us there, 24.8 in ranges, 154 x 2048 x 8064 19.3 and 26.5).  A long walk takes up to 1.2 times its costs (384 x 1300 x 5120 26.3 us), hence the 1.1.
+  const QuadSums sums = quad_sums(a);
+  if (sums.order != kOrderCut) return none;
+  const int64_t tiles = quad_tiles(a, 2, 2), shares = (steps + sums.per - 1) / sums.per;
+  const QuadCost c{0.49f, 0.227f, 2.66f, 0.355f};
+  const float apart = quad_us(c, tiles * shares, 2, (float)sums.per, cu) + 3.5f + (float)(shares * tiles * 4096) * 8.f / 4.5e6f;
+  return apart < 1.1f * quad_us(c, tiles, 2, (float)steps, cu) && (size_t)(tiles * shares * 4096) <= a.scratch_floats ? ShareForm{64, 64, (int)shares, sums.per} : none;
 }
 // floats of scratch that the call can use, out of at most `cap`
 size_t gemm_share_floats(MfmaArgs a, size_t cap) {
