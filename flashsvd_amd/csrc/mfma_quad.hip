@@ -251,19 +251,20 @@ static bool big_pair_is_ahead(const MfmaArgs& a) {
 // A call of 128 rows and more that runs in no shares of its own is left to the 64 x 64 tiles of mfma_gemm.hip, K split over workgroups that add up in the
 // registered buffer, where that has room and the split is ahead of one workgroup per tile.  us in one workgroup / split, tiles x ranges in
 // brackets, weights from HBM:
-//   K of 2048 to 8191: up to one workgroup of the split per compute unit, 128 x 1024 x 4096 (32 x 8) 19.8 / 12.4, 256 x 1024 x 3584 (64 x 4) 17.4 / 12.0, 512 x
-//     1024 x 5504 (128 x 2) 26.4 / 20.5, and any split of 51 tiles, 128 x 1536 x 5504 (48 x 6) 26.8 / 18.7.  Not with more workgroups, where neighbours on
-//     a compute unit cover each other: 256 x 1536 x 4096 (96 x 3) 19.9 / 20.7, 333 x 704 x 3072 (66 x 4) 11.6 / 14.3; an eighth more from a K of 5120 on,
-//     256 x 1536 x 5504 26.5 / 24.3.  Shorter: 128 x 1024 x 2048 (32 x 4) 9.5 / 9.4, x 1536 (32 x 3) 8.0 / 9.0.
+//   K of 1536 to 8191: up to one workgroup of the split per compute unit, 128 x 1024 x 1536 (32 x 3) 10.3 / 9.4, x 4096 (32 x 8) 19.8 / 12.4, 256 x 1024 x
+//     3584 (64 x 4) 17.4 / 12.0, 512 x 1024 x 5504 (128 x 2) 26.4 / 20.5, and any split of 51 tiles, 128 x 1536 x 5504 (48 x 6) 26.8 / 18.7.  Not with more
+//     workgroups, where neighbours on a compute unit cover each other: 333 x 704 x 3072 (66 x 4) 13.4 / 14.6; a quarter more from a K of 3840 on, 128 x
+//     2560 x 3840 (80 x 4) 21.4 / 19.0, 512 x 768 x 3840 (96 x 3) 20.2 / 18.2, 256 x 1536 x 4096 (96 x 3) 19.9 / 20.7, x 5504 26.5 / 24.3.  Shorter: 128 x
+//     1024 x 1024 (32 x 2) 7.9 / 9.1.
 //   K of 8192 and more (a K below 4096 gets no scratch and these may come without): up to 128 tiles, 128 x 1536 x 11008 51.9 / 24.6, 512 x 1024 x 8192
 //     34.1 / 29.2, up to 192 from 10240 on, 512 x 1536 x 11008 50.9 / 46.4.  Not 200 x 2560 x 8192 (160 tiles) 28.5 / 37.4.
 static bool split_is_ahead(const MfmaArgs& a) {
-  if (a.B < 128 || a.K < 2048 || gemm_mid_rule(a).area > 0 || gemm_big_apply(a, false)) return false;
+  if (a.B < 128 || a.K < 1536 || gemm_mid_rule(a).area > 0 || gemm_big_apply(a, false)) return false;
   const int64_t tiles = quad_tiles(a, 2, 2), cu = compute_units();
   const TilesCut c = gemm_tiles_cut(a);
   if (!c.room) return false;
   const int64_t wgs = tiles * c.ranges;
-  const bool ahead = a.K < 8192 ? wgs <= cu || tiles * 5 <= cu || (a.K >= 5120 && wgs * 8 <= cu * 9) : tiles * 2 <= cu || (a.K >= 10240 && tiles * 4 <= cu * 3);
+  const bool ahead = a.K < 8192 ? wgs <= cu || tiles * 5 <= cu || (a.K >= 3840 && wgs * 4 <= cu * 5) : tiles * 2 <= cu || (a.K >= 10240 && tiles * 4 <= cu * 3);
   return ahead && share_form(a).shares == 0;
 }
 

@@ -43,7 +43,7 @@ const char* fsvd_last_error(void);
 const char* fsvd_last_form(void);
 
 /* Optional scratch for the projections (fsvd_linear, fsvd_swiglu_linear) of 17..127 rows, of 3..16 rows when the matrix has
- * fewer than 2048 rows, and of 128 rows and more where a single matrix has few output tiles and K >= 2048, each for K a
+ * fewer than 2048 rows, and of 128 rows and more where a single matrix has few output tiles and K >= 1536, each for K a
  * multiple of 64 and operand rows on the 16-byte grid: with it they split K over several workgroups per tile (fp32 partial
  * tiles and arrival counters live in this buffer; the sum is taken in a fixed order, so results do not depend on timing).
  * Other K and other rows never use it.

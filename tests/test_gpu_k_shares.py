@@ -55,7 +55,7 @@ def test_ranges_apart_and_in_a_row_give_the_same_bits(B, N, K, dtype):
 
 @pytest.mark.parametrize("B,N,K,form", [
     (128, 1024, 4096, "tiles 64 x 64"), (128, 256, 8192, "tiles 64 x 64"), (150, 1027, 7168, "tiles 64 x 64"), (129, 1530, 11008, "tiles 64 x 64"),
-    (512, 1536, 11008, "tiles 64 x 64"), (333, 1536, 8192, "quad 64 x 64"), (333, 1024, 4096, "quad 64 x 64 ranges"),
+    (512, 1536, 11008, "tiles 64 x 64"), (333, 1536, 8192, "quad 64 x 64"), (333, 1280, 4096, "quad 64 x 64 ranges"),
 ])
 def test_calls_without_scratch_split_in_the_registered_buffer(B, N, K, form):
     """fsvd_linear, whose only scratch is the registered buffer; with that too small for the split, or with none, the same call runs unsplit."""
@@ -87,7 +87,8 @@ def test_calls_without_scratch_split_in_the_registered_buffer(B, N, K, form):
 
 
 @pytest.mark.parametrize("B,N,K,form", [(128, 1024, 3584, "tiles 64 x 64"), (130, 259, 2048, "tiles 64 x 64"), (512, 1024, 3328, "tiles 64 x 64"),
-                                        (512, 768, 3072, "quad 64 x 64 ranges"), (128, 1024, 1536, "quad 64 x 64 ranges")])
+                                        (128, 1024, 1536, "tiles 64 x 64"), (128, 2559, 3840, "tiles 64 x 64"),
+                                        (512, 768, 3072, "quad 64 x 64 ranges"), (128, 1024, 1472, "quad 64 x 64 ranges")])
 def test_a_k_too_short_for_scratch(B, N, K, form):
     from flashsvd_amd import hip_ops
     x, w = _rand(B, K, seed=1), _rand(N, K, std=K ** -0.5, seed=2)

@@ -38,7 +38,7 @@ def _linear(B, N, K, dtype, any_grid=False):
     (33, 4170, 320, "quad 64 x 64"),
     (130, 259, 320, "quad 64 x 64"),
     (197, 5541, 384, "quad 128 x 64 halves"), (132, 5545, 384, "quad 96 x 64 halves"), (128, 8256, 384, "quad 64 x 96 halves"), (135, 1362, 384, "quad 64 x 64 halves"),
-    (130, 259, 1088, "quad 64 x 64 ranges"), (300, 517, 1088, "quad 64 x 64 ranges"), (301, 261, 1920, "quad 64 x 64 ranges"),
+    (130, 259, 1088, "quad 64 x 64 ranges"), (300, 517, 1088, "quad 64 x 64 ranges"), (301, 261, 1408, "quad 64 x 64 ranges"),
 ])
 def test_linear(B, N, K, form, dtype):
     assert _linear(B, N, K, dtype) == form
