@@ -268,8 +268,22 @@ static bool split_is_ahead(const MfmaArgs& a) {
   return ahead && share_form(a).shares == 0;
 }
 
+// 33 to 127 aligned rows whose 32 x 64 tiles are at most one per compute unit are left to those of mfma_gemm.hip, K split over workgroups in the registered
+// buffer, where K is long.  us here / split, weights from HBM: a single matrix of up to half as many tiles from a K of 2048 on, 64 x 4096 x 3072 18.4 / 14.3 (K
+// 1536 10.9 / 11.3), of more from 5120 on, 127 x 4096 x 5504 29.1 / 26.8, x 11008 54.8 / 45.8, 64 x 8192 x 8192 43.7 / 39.4 (127 x 4096 x 4096 21.6 / 21.0, 96
+// rows 18.6 / 23.0).  The pair by how many shares of K the tiles leave room for: up to half of them from 1024 on, 127 x 2048 x 1536 21.6 / 16.7, up to two
+// thirds from 1280 on, 64 x 5504 x 2752 38.1 / 29.1 (K 1024 16.0 / 19.2), else from 2048 on, 127 x 4096 x 4096 48.9 / 38.2.  With more tiles this is ahead at
+// any K: the pair 64 x 11008 x 4096 56.1 / 59.5.
+static bool narrow_split_is_ahead(const MfmaArgs& a, bool dual) {
+  const int64_t t = quad_tiles(a, 1, 2), cu = compute_units();
+  if (t > cu || !gemm_rows_apply(a)) return false;
+  if (!dual) return a.K >= (t * 2 <= cu ? 2048 : 5120);
+  return a.K >= (t * 2 <= cu ? 1024 : (t * 16 <= cu * 11 ? 1280 : 2048));
+}
+
 bool gemm_quad_apply(const MfmaArgs& a, bool dual) {
   if (!quad_range(a, dual)) return false;
+  if (a.B < 128 && quad_grid(a, dual)) return !narrow_split_is_ahead(a, dual);
   if (quad_grid(a, dual)) return dual ? !big_pair_is_ahead(a) : !split_is_ahead(a);
   return quad_words(a, dual) && (dual || a.B >= 128);
 }

@@ -44,6 +44,31 @@ def test_linear(B, N, K, form, dtype):
     assert _linear(B, N, K, dtype) == form
 
 
+@pytest.mark.parametrize("B,N,K,single,pair", [
+    (64, 4090, 3072, "tiles 32 x 64", "tiles 32 x 64 pair"), (33, 4096, 1984, "quad 64 x 64", "tiles 32 x 64 pair"), (100, 4096, 960, "quad 64 x 64", "quad 64 x 96 pair"),
+    (127, 4090, 5184, "tiles 32 x 64", "tiles 32 x 64 pair"), (127, 4096, 2048, "quad 64 x 64", "tiles 32 x 64 pair"), (64, 5500, 1280, "quad 64 x 64", "tiles 32 x 64 pair"),
+    (70, 8192, 5184, "quad 64 x 64", "quad 64 x 96 pair"),
+])
+def test_few_tiles_of_a_long_k_split(B, N, K, single, pair):
+    """33 to 127 rows: on either side of the lines, with the registered buffer; without it everything runs here."""
+    from flashsvd_amd import _lib, hip_ops
+    x, w, w2 = _rand(B, K, seed=1), _rand(N, K, std=K ** -0.5, seed=2), _rand(N, K, std=K ** -0.5, seed=3)
+    ref = x.float() @ w.float().t()
+    act = torch.nn.functional.silu(ref.bfloat16()) * (x.float() @ w2.float().t()).bfloat16()
+    _check(hip_ops.linear(x, w), ref.bfloat16(), "single")
+    assert form_taken() == single
+    _check(hip_ops.swiglu_linear(x, w, w2, up_off=0), act, "pair")
+    assert form_taken() == pair
+    hip_ops.release_split_workspace(x.device)
+    y = torch.empty(B, N, device="cuda", dtype=torch.bfloat16)
+    try:
+        rc = _lib.load().fsvd_linear(x.data_ptr(), K, w.data_ptr(), K, None, None, 0.0, None, 0, y.data_ptr(), N, B, N, K, 0, 0, hip_ops._stream())
+        assert rc == 0 and form_taken() == ("quad 64 x 64" if (N + 63) // 64 * ((B + 63) // 64) >= 128 or K < 4096 else "rows 16")
+        _check(y, ref.bfloat16(), "no buffer")
+    finally:
+        assert hip_ops.ensure_split_workspace(x.device)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,N,K,form", [
     (297, 12319, 323, "any quad 192 x 128"), (128, 8256, 322, "any quad 128 x 128"), (130, 5559, 383, "any quad 96 x 64"),
