@@ -418,6 +418,7 @@ static MidForm mid_form(const MfmaArgs& a, bool dual) {
   return small <= cu && (small * 2 > cu || (small * 4 >= cu && a.K <= 2048)) ? kMid64x64Halves : kMidNone;
 }
 bool gemm_mid_apply(const MfmaArgs& a, bool dual) { return mid_form(a, dual) != kMidNone; }
+bool gemm_mid_pair_of_64(const MfmaArgs& a) { return mid_form(a, true) == kMid64x192; }
 RingRule gemm_mid_rule(const MfmaArgs& a) {
   switch (mid_form(a, false)) {
     case kMid128x128: return RingRule{128 * 128, false};

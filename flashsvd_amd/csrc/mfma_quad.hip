@@ -281,10 +281,19 @@ static bool narrow_split_is_ahead(const MfmaArgs& a, bool dual) {
   return a.K >= (t * 2 <= cu ? 1024 : (t * 16 <= cu * 11 ? 1280 : 2048));
 }
 
+// The pair of 128 aligned rows and more with a K of 1152 and more is left to the 64 x 64 tiles of mfma_gemm.hip where these are at most one per compute
+// unit, and to the 64 x 192 ring of mfma_mid.hip where that takes the shape and 64 x 96 would serve it here.  us here / there, weights from HBM: 128 x 2752 x
+// 1536 21.8 / 20.1, 256 x 4096 x 2432 31.3 / 28.5 (K 1024 15.4 / 15.1, 768 11.2 / 13.1); 256 x 11008 x 1536 41.1 / 38.8, 575 x 4964 x 1536 39.1 / 35.7 (256 x
+// 11008 x 512 16.6 / 17.2).
+static bool pair_of_64_is_ahead(const MfmaArgs& a) {
+  if (a.B < 128 || a.K < 1152) return false;
+  return quad_tiles(a, 2, 2) <= compute_units() || (quad_pick(a, true, false).form == 8 && gemm_mid_pair_of_64(a));
+}
+
 bool gemm_quad_apply(const MfmaArgs& a, bool dual) {
   if (!quad_range(a, dual)) return false;
   if (a.B < 128 && quad_grid(a, dual)) return !narrow_split_is_ahead(a, dual);
-  if (quad_grid(a, dual)) return dual ? !big_pair_is_ahead(a) : !split_is_ahead(a);
+  if (quad_grid(a, dual)) return dual ? !big_pair_is_ahead(a) && !pair_of_64_is_ahead(a) : !split_is_ahead(a);
   return quad_words(a, dual) && (dual || a.B >= 128);
 }
 

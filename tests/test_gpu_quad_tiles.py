@@ -83,7 +83,8 @@ def test_linear_any_grid(B, N, K, form, dtype):
     (341, 12357, 320, "quad 128 x 192 pair"), (783, 9447, 320, "quad 160 x 192 pair"), (409, 10404, 320, "quad 160 x 128 pair"),
     (168, 27083, 1280, "quad 256 x 128 pair"), (261, 9918, 320, "quad 128 x 128 pair"), (67, 25091, 832, "quad 128 x 128 pair alone"),
     (129, 17205, 896, "quad 96 x 192 pair"), (72, 12319, 320, "quad 96 x 96 pair"), (66, 8328, 320, "quad 64 x 96 pair"),
-    (130, 259, 320, "quad 64 x 64 pair"),
+    (130, 259, 320, "quad 64 x 64 pair"), (250, 4090, 1088, "quad 64 x 96 pair"), (250, 4090, 1152, "tiles 64 x 64 pair"), (260, 4090, 1152, "quad 64 x 96 pair"),
+    (250, 11001, 1024, "quad 64 x 96 pair"), (250, 11001, 1536, "ring 64 x 192 pair"),
     (341, 12357, 323, "any quad 128 x 192 pair"), (261, 9918, 322, "any quad 128 x 128 pair"), (129, 17205, 894, "any quad 96 x 192 pair"),
     (130, 8954, 383, "any quad 96 x 96 pair"), (130, 259, 321, "any quad 64 x 96 pair"), (40, 8190, 330, "any quad 64 x 96 pair"),
 ])
