@@ -231,6 +231,7 @@ bool expand_quad_apply(const ExpandArgs* d, int n);                         // m
 int launch_expand_quad(const ExpandArgs* d, int n, hipStream_t st);
 struct RingRule { int area; bool halves; };                                  // outputs of a ring tile (0: no ring), K halved between waves
 RingRule gemm_mid_rule(const MfmaArgs& a);
+int gemm_mid_ragged_rows(const MfmaArgs& a);                                 // rows of the ring tile that a ragged single matrix gets there (0: none)
 bool gemm_mid_pair_of_64(const MfmaArgs& a);                                 // the pair on 64 x 192 tiles
 struct TilesCut { int per, ranges; bool room; };                             // steps of 64 in a range of K (0: not cut), the registered buffer holds the ranges' sums
 TilesCut gemm_tiles_cut(const MfmaArgs& a);                                 // mfma_gemm.hip

@@ -464,6 +464,10 @@ static RagForm mid_ragged_form(const MfmaArgs& a, bool dual) {
   return about_one(t) && (a.K <= 2048 || t * 8 >= cu * 7) ? kRag64x128 : kRagNone;
 }
 bool gemm_mid_ragged_apply(const MfmaArgs& a, bool dual) { return mid_ragged_form(a, dual) != kRagNone; }
+int gemm_mid_ragged_rows(const MfmaArgs& a) {
+  const RagForm f = mid_ragged_form(a, false);
+  return f == kRag64x128 ? 64 : (f == kRag128x128 ? 128 : 0);
+}
 template <int DT>
 static int launch_mid_ragged_dt(const MfmaArgs& a, bool dual, hipStream_t st, const char* who) {
   MidArgs m{};

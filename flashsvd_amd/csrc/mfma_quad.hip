@@ -281,20 +281,40 @@ static bool narrow_split_is_ahead(const MfmaArgs& a, bool dual) {
   return a.K >= (t * 2 <= cu ? 1024 : (t * 16 <= cu * 11 ? 1280 : 2048));
 }
 
-// The pair of 128 aligned rows and more with a K of 1152 and more is left to the 64 x 64 tiles of mfma_gemm.hip where these are at most one per compute
+// The pair of 128 aligned rows and more with a K of 1024 and more is left to the 64 x 64 tiles of mfma_gemm.hip where these are at most one per compute
 // unit, and to the 64 x 192 ring of mfma_mid.hip where that takes the shape and 64 x 96 would serve it here.  us here / there, weights from HBM: 128 x 2752 x
 // 1536 21.8 / 20.1, 256 x 4096 x 2432 31.3 / 28.5 (K 1024 15.4 / 15.1, 768 11.2 / 13.1); 256 x 11008 x 1536 41.1 / 38.8, 575 x 4964 x 1536 39.1 / 35.7 (256 x
 // 11008 x 512 16.6 / 17.2).
 static bool pair_of_64_is_ahead(const MfmaArgs& a) {
-  if (a.B < 128 || a.K < 1152) return false;
+  if (a.B < 128 || a.K < 1024) return false;
   return quad_tiles(a, 2, 2) <= compute_units() || (quad_pick(a, true, false).form == 8 && gemm_mid_pair_of_64(a));
+}
+
+// Ragged rows: the tiles here take up to twice their costs with them (256 x 4096 x 4098 34 us, 18 by the table), so that the register pipelines of mfma_gemm.hip
+// and mfma_mid.hip are ahead on few or small tiles.  us here / there, weights from HBM:
+//   a pair of up to 127 rows with at most one of the 32 x 64 tiles per compute unit, 64 x 5504 x 746 18.4 / 14.7, 33 x 4096 x 2050 38.6 / 25.8 (65 x 5504 x 746,
+//     one and a little, 14.8 / 15.4); of more rows with at most one 64 x 64 tile from a K of 1152 on, 154 x 1376 x 2050 35.9 / 30.8 (128 x 4096 x 1492 31.2 / 31.5);
+//   a single matrix with at most one 32 x 64 tile per compute unit, 128 x 4096 x 1492 15.7 / 11.5, 256 x 704 x 2050 18.2 / 12.5 (K 322 as fast);
+//   one that the 64 x 128 ring takes, unless 96 x 64 serves it here, 512 x 4096 x 1492 24.2 / 20.3 (1500 x 704 x 1492 on 96 x 64 15.3 / 18.2); one that
+//     the 128 x 128 ring takes and smaller or larger tiles would serve here, of up to 192 rows from 1280 on, 154 x 11008 x 4098 65.6 / 58.0, else from 6144 on;
+//   64 x 64 tiles here from a K of 2048 on, 256 x 4096 x 4098 34.2 / 28.9, or from 1280 on where no row tile is padded, 256 x 4096 x 1492 15.5 / 14.4 (200 x
+//     4096 x 1492 10.4 / 12.8); 96 x 64 that fill three quarters of the chip with up to 192 rows, 154 x 5504 x 4098 37.5 / 34.3.
+static bool ragged_is_ahead_elsewhere(const MfmaArgs& a, bool dual) {
+  const int64_t cu = compute_units();
+  if (dual) return a.B < 128 ? quad_tiles(a, 1, 2) <= cu : a.K >= 1152 && quad_tiles(a, 2, 2) <= cu;
+  if (quad_tiles(a, 1, 2) <= cu) return true;
+  const int ring = gemm_mid_ragged_rows(a), form = quad_pick(a, false, true).form;
+  if (ring == 64) return form != 10;
+  if (ring == 128) return form != 5 && a.K >= (a.B <= 192 ? 1280 : 6144);
+  if (form == 12) return a.K >= 2048 || (a.K >= 1280 && (int64_t)a.B * 16 >= (a.B + 63) / 64 * 64 * 15);
+  return form == 10 && a.B <= 192 && a.K >= 2048 && quad_tiles(a, 3, 2) * 4 <= 3 * cu;
 }
 
 bool gemm_quad_apply(const MfmaArgs& a, bool dual) {
   if (!quad_range(a, dual)) return false;
   if (a.B < 128 && quad_grid(a, dual)) return !narrow_split_is_ahead(a, dual);
   if (quad_grid(a, dual)) return dual ? !big_pair_is_ahead(a) && !pair_of_64_is_ahead(a) : !split_is_ahead(a);
-  return quad_words(a, dual) && (dual || a.B >= 128);
+  return quad_words(a, dual) && (dual || a.B >= 128) && !ragged_is_ahead_elsewhere(a, dual);
 }
 
 template <int DT>
