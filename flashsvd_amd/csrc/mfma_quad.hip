@@ -69,6 +69,10 @@ static QuadPick quad_pick(const MfmaArgs& a, bool dual, bool any, QuadOrder orde
     const auto fits = [&](int n) {
       if (any) return n == 4 || n == 5 || n == 10 || n == 12;
       if (n < kHalvesFrom && order != kOrderPlain) return false;
+      // two row tiles of 96 and more than a column of them per compute unit: 128 x 128 is ahead of its costs there (192 x 13260 x 1536 23.0 -> 19.7, 174 x 16384
+      // x 2048 30.2 -> 23.2, K 1024 as fast); 64 x 128 is a tile for one round (300 x 24000 x 320 20.5 -> 15.6, 700 x 11008 x 320 19.4 -> 14.3)
+      if (n == 10 && a.B >= 128 && a.B <= 192 && a.K >= 1280 && quad_tiles(a, 3, 2) > cu) return false;
+      if (n == 9 && quad_tiles(a, 2, 4) > cu) return false;
       return n == 10 ? a.K < 4096 : (n == 11 ? a.B % 64 == 0 && a.N % 96 == 0 : true);
     };
 #define X(n, TM, TN, SX, SW, OCC, F1, S1, F2, S2) if (fits(n)) take(n, TM, TN, OCC, QuadCost{F1, S1, F2, S2});
