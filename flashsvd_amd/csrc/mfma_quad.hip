@@ -65,7 +65,8 @@ static QuadPick quad_pick(const MfmaArgs& a, bool dual, bool any, QuadOrder orde
   } else {
     // 96 x 64 is left out for a K of 4096 and more: 64 x 64 and 128 x 64 are within 6 % of it or ahead there (3072 columns at 154, 333,
     // 420, 512 rows 22.5, 22.2, 22.2, 27.6 against 17.9, 21.5, 23.7, 27.2), below it is the best tile of 333 rows (4096 x 1536 11.4 against
-    // 12.8).  64 x 96 comes in where it pads nothing (512 x 3072 x 4096 24.5 against 27.2; 420 rows 23.6 against 23.7).
+    // 12.8).  64 x 96 is a tile for one per compute unit: 512 x 2238 x 4096 28.2 -> 24.6, 511 x 3072 x 4096 28.0 -> 25.4, 192 x 7717 x 8000 48.4 -> 50.3 (0.86 to
+    // 1.06 of 128 x 64 over 47 shapes); over more the others are up to 15 % ahead.
     const auto fits = [&](int n) {
       if (any) return n == 4 || n == 5 || n == 10 || n == 12;
       if (n < kHalvesFrom && order != kOrderPlain) return false;
@@ -73,7 +74,7 @@ static QuadPick quad_pick(const MfmaArgs& a, bool dual, bool any, QuadOrder orde
       // x 2048 30.2 -> 23.2, K 1024 as fast); 64 x 128 is a tile for one round (300 x 24000 x 320 20.5 -> 15.6, 700 x 11008 x 320 19.4 -> 14.3)
       if (n == 10 && a.B >= 128 && a.B <= 192 && a.K >= 1280 && quad_tiles(a, 3, 2) > cu) return false;
       if (n == 9 && quad_tiles(a, 2, 4) > cu) return false;
-      return n == 10 ? a.K < 4096 : (n == 11 ? a.B % 64 == 0 && a.N % 96 == 0 : true);
+      return n == 10 ? a.K < 4096 : (n == 11 ? quad_tiles(a, 2, 3) <= cu : true);
     };
 #define X(n, TM, TN, SX, SW, OCC, F1, S1, F2, S2) if (fits(n)) take(n, TM, TN, OCC, QuadCost{F1, S1, F2, S2});
     FSVD_QUAD_PLAIN(X)

@@ -20,7 +20,7 @@ pytestmark = pytest.mark.gpu
     (512, 1500, 5504, "shares 256 x 128"), (769, 1533, 8320, "shares 128 x 128"), (1000, 1533, 8320, "shares 256 x 128"), (2047, 2390, 8192, "shares 256 x 128"),
     (150, 1027, 4096, "shares 64 x 64"), (200, 515, 4096, "shares 64 x 64"), (512, 1024, 4160, "shares 64 x 64"),
     (128, 3070, 5120, "shares 64 x 128"), (191, 2050, 5504, "shares 64 x 128"),       # cut in ranges, but enough shares to fill the chip
-    (512, 1536, 11008, "shares 128 x 128"), (420, 3072, 4096, "quad 128 x 64 halves"), (512, 4096, 4096, "quad 128 x 64 halves"), (127, 3072, 4096, "tiles 32 x 64"),
+    (512, 1536, 11008, "shares 128 x 128"), (420, 3072, 4096, "quad 64 x 96 halves"), (520, 3072, 4096, "quad 128 x 64 halves"), (512, 4096, 4096, "quad 128 x 64 halves"), (127, 3072, 4096, "tiles 32 x 64"),
 ])
 def test_linear(B, N, K, form, dtype):
     from flashsvd_amd import hip_ops

@@ -33,11 +33,11 @@ def _linear(B, N, K, dtype, any_grid=False):
 @pytest.mark.parametrize("B,N,K,form", [
     (1036, 11077, 320, "quad 256 x 256"), (706, 11209, 320, "quad 256 x 192"), (341, 12357, 320, "quad 128 x 192"),
     (777, 7569, 320, "quad 256 x 128"), (514, 9972, 320, "quad 192 x 128"), (130, 11060, 320, "quad 128 x 128"),
-    (519, 11227, 320, "quad 128 x 128 alone"), (69, 17004, 1024, "quad 128 x 96"), (99, 8635, 320, "quad 128 x 64"),
-    (133, 9272, 320, "quad 64 x 128"), (66, 8328, 320, "quad 96 x 64"), (3648, 1056, 320, "quad 64 x 96"),
+    (519, 11227, 320, "quad 128 x 128 alone"), (69, 17004, 1024, "quad 128 x 96"), (99, 8635, 320, "quad 64 x 96"), (99, 12400, 320, "quad 128 x 64"),
+    (133, 9272, 320, "quad 64 x 128"), (66, 8328, 320, "quad 96 x 64"), (3648, 1056, 320, "quad 128 x 64"),
     (33, 4170, 320, "quad 64 x 64"), (190, 13257, 1280, "quad 128 x 128 alone"), (190, 13257, 1216, "quad 96 x 64"), (300, 24001, 320, "quad 256 x 192"),
     (130, 259, 320, "quad 64 x 64"),
-    (197, 5541, 384, "quad 128 x 64 halves"), (132, 5545, 384, "quad 96 x 64 halves"), (128, 8256, 384, "quad 64 x 96 halves"), (135, 1362, 384, "quad 64 x 64 halves"),
+    (197, 5541, 384, "quad 64 x 96 halves"), (197, 6201, 384, "quad 128 x 64 halves"), (132, 5545, 384, "quad 96 x 64 halves"), (128, 8256, 384, "quad 64 x 96 halves"), (135, 1362, 384, "quad 64 x 64 halves"),
     (130, 259, 1088, "quad 64 x 64 ranges"), (300, 517, 1088, "quad 64 x 64 ranges"), (301, 261, 1408, "quad 64 x 64 ranges"),
 ])
 def test_linear(B, N, K, form, dtype):
