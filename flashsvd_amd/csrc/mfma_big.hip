@@ -1,6 +1,6 @@
 // Projections of long prompts: 256 x 256 output tiles, one workgroup of eight waves per compute unit that walks its share of
-// the tiles.  They serve a K below 320 and the pair where the tiles of mfma_quad.hip cost more (see big_pair_is_ahead there); the rest runs there, whose
-// four waves are ahead (q, k and v of 32 heads at 16384 x 1664 696 -> 594 us).
+// the tiles.  They serve a K below 320; the rest runs on the tiles of mfma_quad.hip, whose four waves are ahead (q, k and v of 32 heads at 16384 x 1664
+// 696 -> 594 us) or as fast (the pair 16384 x 11008 x 2432 1602 and 1605).
 //
 // What bounds a large product on this chip is cycles and clock alike: under a stream of these products the clock stays at 1.95 to
 // 2.2 GHz (1.65 in the first milliseconds of a burst), the matrix cores are busy in 50 to 63 % of the cycles (counters), and

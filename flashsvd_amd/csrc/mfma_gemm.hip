@@ -620,7 +620,7 @@ static int launch_gemm_tiles_dt(const MfmaArgs& a, bool dual, hipStream_t st, co
   if (big >= 256) return launch_gemm_tiles_t<DT, false, 4, 2, 64>(a, st, who);
   // mfma_mid.hip takes these where its 32-bit offsets reach; operands past them stay on unsplit 128 x 128 tiles
   if (big >= 144) return launch_gemm_tiles_t<DT, false, 4, 4, 64, 4, 2, true>(a, st, who);
-  // K of 8192 and more with about one 128 x 64 tile per compute unit: eight waves, each half of them on half of the k slices
+  // (so far operands of 4 GiB and more, or a K below 320.)  About one 128 x 64 tile per compute unit: eight waves, each half of them on half of the k slices
   // of a step, so that a workgroup alone on its compute unit still runs two waves per SIMD (1536 x 11008 at 1024 rows 72 us,
   // three stages of loads straight into LDS 73)
   const int64_t half = (int64_t)((a.N + 63) / 64) * ((a.B + 127) / 128);

@@ -4,18 +4,6 @@
 
 namespace fsvd {
 
-// What a round of workgroups costs in a form, us: f + s per K step of 64; 1: the compute units hold one workgroup each (or fewer), 2: as many
-// as fit.  Fitted to launches with weights from HBM (more of them in turn than the 256 MB in front of it hold) over 125 / 49 / 39 shapes
-// (154 to 16384 rows; 1024 to 4096 columns at K 768 to 4096; the pair 5504 x 768 to 11008 x 2432; 48 and 96 heads at rank 512 and 1024):
-// the form that they name is on average 2 / 1 / 1 % (at worst 20, 12, 8 %) behind the best of about 30 tilings.
-struct QuadCost { float f1, s1, f2, s2; };
-constexpr float kLaunchUs = 3.f;
-static float quad_us(const QuadCost& c, int64_t tiles, int occ, float steps, int64_t cu) {
-  const int64_t full = tiles / (cu * occ), rest = tiles - full * cu * occ;
-  float us = (float)full * (c.f2 + c.s2 * steps);
-  if (rest > 0) us += occ == 2 && rest <= cu ? c.f1 + c.s1 * steps : c.f2 + c.s2 * steps;
-  return us;
-}
 static int64_t quad_tiles(const MfmaArgs& a, int tm, int tn) { return (int64_t)((a.N + 32 * tn - 1) / (32 * tn)) * ((a.B + 32 * tm - 1) / (32 * tm)); }
 
 //     form, TM, TN, stages of x and W, workgroups per compute unit, costs
@@ -25,7 +13,15 @@ static int64_t quad_tiles(const MfmaArgs& a, int tm, int tn) { return (int64_t)(
   X(6, 4, 4, 4, 5, 1, 0.f, 0.f, 3.03f, 0.450f) X(7, 4, 3, 5, 6, 1, 0.f, 0.f, 4.29f, 0.353f) X(8, 4, 2, 3, 4, 2, 0.57f, 0.339f, 3.94f, 0.568f) \
   X(9, 2, 4, 3, 4, 1, 0.f, 0.f, 1.24f, 0.354f) X(10, 3, 2, 3, 4, 2, 0.24f, 0.297f, 3.14f, 0.440f) X(11, 2, 3, 3, 4, 2, 0.30f, 0.311f, 1.99f, 0.484f) \
   X(12, 2, 2, 5, 5, 2, 0.49f, 0.227f, 2.66f, 0.355f)
-constexpr int kHalvesFrom = 8;                       // the forms that shapes with K halved get, with registers for a second set of accumulators
+constexpr bool quad_halves(int n) { return n >= 8 && n != 9; }      // the forms that shapes with K halved get, with registers for a second set of accumulators
+constexpr QuadCost kPlainCosts[] = {
+#define X(n, TM, TN, SX, SW, OCC, F1, S1, F2, S2) QuadCost{F1, S1, F2, S2},
+  FSVD_QUAD_PLAIN(X)
+#undef X
+};
+constexpr QuadCost kCost256x128Shares{0.f, 0.f, 6.65f, 0.634f};     // three stages of both operands, in shares only
+constexpr float kLaunchUs = 3.f, kShareSumUs = 3.5f, kShareBytesPerUs = 4.5e6f;      // of a launch; of the one that adds the shares, beside their way out and in
+static float share_sum_us(int64_t floats) { return kShareSumUs + (float)floats * 8.f / kShareBytesPerUs; }
 #define FSVD_QUAD_PAIR(X) \
   X(0, 4, 6, 3, 4, 1, 0.f, 0.f, 8.19f, 0.657f) X(1, 5, 6, 2, 3, 1, 0.f, 0.f, 9.82f, 0.693f) X(2, 5, 4, 2, 2, 2, 4.26f, 0.861f, 8.46f, 0.970f) \
   X(3, 8, 4, 2, 3, 1, 0.f, 0.f, 10.88f, 0.710f) X(4, 4, 4, 2, 3, 2, 3.94f, 0.589f, 7.43f, 0.802f) X(5, 4, 4, 4, 5, 1, 0.f, 0.f, 6.31f, 0.487f) \
@@ -69,7 +65,7 @@ static QuadPick quad_pick(const MfmaArgs& a, bool dual, bool any, QuadOrder orde
     // 1.06 of 128 x 64 over 47 shapes); over more the others are up to 15 % ahead.
     const auto fits = [&](int n) {
       if (any) return n == 4 || n == 5 || n == 10 || n == 12;
-      if (n < kHalvesFrom && order != kOrderPlain) return false;
+      if (order != kOrderPlain && !quad_halves(n)) return false;
       // two row tiles of 96 and more than a column of them per compute unit: 128 x 128 is ahead of its costs there (192 x 13260 x 1536 23.0 -> 19.7, 174 x 16384
       // x 2048 30.2 -> 23.2, K 1024 as fast); 64 x 128 is a tile for one round (300 x 24000 x 320 20.5 -> 15.6, 700 x 11008 x 320 19.4 -> 14.3)
       if (n == 10 && a.B >= 128 && a.B <= 192 && a.K >= 1280 && quad_tiles(a, 3, 2) > cu) return false;
@@ -141,8 +137,8 @@ static ShareForm filling_shares(const MfmaArgs& a, const RingRule& ring) {
   // the sums once out and once in, and the launch that adds them; 333 x 1664 x 4096 19.7 us in shares, 16.1 unsplit (here too a K below 5120 only:
   // the longer ones were ahead in shares at every row count)
   if (a.K < 5120) {
-    const QuadCost c = bm == 64 ? QuadCost{0.f, 0.f, 1.24f, 0.354f} : (bm == 128 ? QuadCost{0.f, 0.f, 3.03f, 0.450f} : QuadCost{0.f, 0.f, 6.65f, 0.634f});
-    const float us = c.f2 + c.s2 * (float)per + 3.5f + (float)(shares * tiles * area) * 8.f / 4.5e6f;
+    const QuadCost c = bm == 64 ? kPlainCosts[9] : (bm == 128 ? kPlainCosts[6] : kCost256x128Shares);
+    const float us = c.f2 + c.s2 * (float)per + share_sum_us(shares * tiles * area);
     if (kLaunchUs + quad_pick(a, false, false).us < 0.9f * (kLaunchUs + us)) return none;
   }
   return ShareForm{bm, 128, (int)shares, per};
@@ -169,9 +165,8 @@ static ShareForm share_form(const MfmaArgs& a) {
   const QuadSums sums = quad_sums(a);
   if (sums.order != kOrderCut) return none;
   const int64_t tiles = quad_tiles(a, 2, 2), shares = (steps + sums.per - 1) / sums.per;
-  const QuadCost c{0.49f, 0.227f, 2.66f, 0.355f};
-  const float apart = quad_us(c, tiles * shares, 2, (float)sums.per, cu) + 3.5f + (float)(shares * tiles * 4096) * 8.f / 4.5e6f;
-  return apart < 1.1f * quad_us(c, tiles, 2, (float)steps, cu) && (size_t)(tiles * shares * 4096) <= a.scratch_floats ? ShareForm{64, 64, (int)shares, sums.per} : none;
+  const float apart = quad_us(kPlainCosts[12], tiles * shares, 2, (float)sums.per, cu) + share_sum_us(shares * tiles * 4096);
+  return apart < 1.1f * quad_us(kPlainCosts[12], tiles, 2, (float)steps, cu) && (size_t)(tiles * shares * 4096) <= a.scratch_floats ? ShareForm{64, 64, (int)shares, sums.per} : none;
 }
 // floats of scratch that the call can use, out of at most `cap`
 size_t gemm_share_floats(MfmaArgs a, size_t cap) {
@@ -247,12 +242,6 @@ static int launch_share_dt(QuadArgs& q, const ShareForm& f, hipStream_t st, cons
   return f.bm == 128 ? launch_share_t<DT, 4, 4, 4, 5, 1>(q, st, who) : launch_share_t<DT, 8, 4, 3, 3, 1>(q, st, who);
 }
 
-// The 256 x 256 pair of mfma_big.hip keeps what its larger tile still does better: 11008 x 2432 at 16384 rows 1602 us, here 1617 at best
-// (8192 rows 874 against 780, its rounds being few and large); its cost in the same terms.
-static bool big_pair_is_ahead(const MfmaArgs& a) {
-  return gemm_big_apply(a, true) && quad_us(QuadCost{0.f, 0.f, 26.7f, 1.564f}, quad_tiles(a, 8, 8), 1, (float)(a.K / 32), compute_units()) < quad_pick(a, true, false).us;
-}
-
 // A call of 128 rows and more that runs in no shares of its own is left to the 64 x 64 tiles of mfma_gemm.hip, K split over workgroups that add up in the
 // registered buffer, where that has room and the split is ahead of one workgroup per tile.  us in one workgroup / split, tiles x ranges in
 // brackets, weights from HBM:
@@ -318,7 +307,7 @@ static bool ragged_is_ahead_elsewhere(const MfmaArgs& a, bool dual) {
 bool gemm_quad_apply(const MfmaArgs& a, bool dual) {
   if (!quad_range(a, dual)) return false;
   if (a.B < 128 && quad_grid(a, dual)) return !narrow_split_is_ahead(a, dual);
-  if (quad_grid(a, dual)) return dual ? !big_pair_is_ahead(a) && !pair_of_64_is_ahead(a) : !split_is_ahead(a);
+  if (quad_grid(a, dual)) return dual ? !pair_of_64_is_ahead(a) : !split_is_ahead(a);
   return quad_words(a, dual) && (dual || a.B >= 128) && !ragged_is_ahead_elsewhere(a, dual);
 }
 
@@ -362,7 +351,7 @@ static int launch_gemm_quad_dt(const MfmaArgs& a, bool dual, hipStream_t st, con
     return launch_quad_t<DT, kQuadPlain, 2, 2, 5, 5, 2, false, 1, true>(q, st, who);
   } else if (sums.order == kOrderHalves) {
     switch (form) {
-#define X(n, TM, TN, SX, SW, OCC, ...) case n: if constexpr (n >= kHalvesFrom) return launch_quad_t<DT, kQuadPlain, TM, TN, SX, SW, OCC, false, 2>(q, st, who); break;
+#define X(n, TM, TN, SX, SW, OCC, ...) case n: if constexpr (quad_halves(n)) return launch_quad_t<DT, kQuadPlain, TM, TN, SX, SW, OCC, false, 2>(q, st, who); break;
       FSVD_QUAD_PLAIN(X)
 #undef X
     }

@@ -53,6 +53,19 @@ __device__ __forceinline__ void quad_swap_rows(uint32_t& a, uint32_t& b) {
 // four elements at any element's address
 typedef uint32_t u32x2_any_t __attribute__((ext_vector_type(2), aligned(2)));
 
+// What a round of workgroups costs in a form, us: f + s per K step of 64; 1: the compute units hold one workgroup each (or fewer), 2: as many
+// as fit.  Fitted to launches with weights from HBM (more of them in turn than the 256 MB in front of it hold) over 125 / 49 / 39 shapes
+// (154 to 16384 rows; 1024 to 4096 columns at K 768 to 4096; the pair 5504 x 768 to 11008 x 2432; 48 and 96 heads at rank 512 and 1024):
+// the form that they name is on average 2 / 1 / 1 % (at worst 20, 12, 8 %) behind the best of about 30 tilings.  The largest launches take longer than
+// they say, whatever the tile (the pair 16384 x 11008 x 2432 1605 us, 1426 by them).
+struct QuadCost { float f1, s1, f2, s2; };
+static float quad_us(const QuadCost& c, int64_t tiles, int occ, float steps, int64_t cu) {
+  const int64_t full = tiles / (cu * occ), rest = tiles - full * cu * occ;
+  float us = (float)full * (c.f2 + c.s2 * steps);
+  if (rest > 0) us += occ == 2 && rest <= cu ? c.f1 + c.s1 * steps : c.f2 + c.s2 * steps;
+  return us;
+}
+
 constexpr bool quad_stream(int tm, int tn) { return tm * tn >= 24; }
 
 // H = 2: the first 64 of every 128 of K and the second 64 are added up apart and then together; CUT: K in ranges of args.per steps, their sums

@@ -18,16 +18,14 @@ static int heads_pick(const ExpandArgs* d, int n, bool any) {
   int best = -1;
   float best_us = 0.f, steps = 0.f;
   for (int k = 0; k < n; ++k) steps = std::max(steps, (float)((d[k].R + 63) / 64));
-  const auto take = [&](int form, int tm, int tn, int occ, float f1, float s1, float f2, float s2) {
+  const auto take = [&](int form, int tm, int tn, int occ, const QuadCost& c) {
     int64_t tiles = 0;
     for (int k = 0; k < n; ++k) tiles += ((int64_t)d[k].heads * 128 + 32 * tn - 1) / (32 * tn);
     tiles *= (rows + 32 * tm - 1) / (32 * tm);
-    const int64_t full = tiles / (cu * occ), rest = tiles - full * cu * occ;
-    float us = (float)full * (f2 + s2 * steps);
-    if (rest > 0) us += occ == 2 && rest <= cu ? f1 + s1 * steps : f2 + s2 * steps;
+    const float us = quad_us(c, tiles, occ, steps, cu);
     if (best < 0 || us < best_us) { best = form; best_us = us; }
   };
-#define X(n_, TM, TN, SX, SW, OCC, F1, S1, F2, S2) if (!any || n_ == 3 || n_ == 4 || n_ == 6) take(n_, TM, TN, OCC, F1, S1, F2, S2);
+#define X(n_, TM, TN, SX, SW, OCC, F1, S1, F2, S2) if (!any || n_ == 3 || n_ == 4 || n_ == 6) take(n_, TM, TN, OCC, QuadCost{F1, S1, F2, S2});
   FSVD_QUAD_HEADS(X)
 #undef X
   return best;
