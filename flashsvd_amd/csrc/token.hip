@@ -29,12 +29,57 @@ __device__ __forceinline__ u16x2_t order_pair(uint32_t w) {
   return __builtin_bit_cast(u16x2_t, (i16x2_t)(p ^ ((p >> 15) | (short)0x8000)));
 }
 
+// Rows of at most two 16-byte pieces per thread: value and index together, element by element, in one reduction.  What a launch takes is its two
+// round trips and the reductions, and the kernel below has three of those: us per launch in a graph there / here, 1000 logits of 1 / 64 rows 3.5 / 2.6, 4.0 /
+// 3.0, 8192 3.7 / 3.1, 4.1 / 3.6, 14336 3.7 / 3.6, 4.2 / 4.1; 16384 3.7 / 3.9, 4.2 / 4.4, hence the line.
+constexpr int kShortLoads = 2, kShortRow = 14336;
+static_assert(kShortRow <= kPickThreads * kShortLoads * 8, "two pieces per thread");
+template <int DT>
+__global__ __launch_bounds__(kPickThreads) void greedy_short_kernel(const uint16_t* __restrict__ logits, int64_t ld, int64_t* __restrict__ tokens,
+                                                                   int64_t ldt, int32_t* __restrict__ positions, int V) {
+  const uint16_t* row = logits + (int64_t)blockIdx.x * ld;
+  const int tid = threadIdx.x, pieces = V >> 3;
+  uint32_t best = 0, at = 0x7fffffffu;
+  const auto take = [&](uint32_t p, uint32_t i) {
+    const uint32_t k = order_key<DT>(p);
+    if (k > best) { best = k; at = i; }                // a thread meets its elements in ascending order
+  };
+  u32x4_t v[kShortLoads];
+#pragma unroll
+  for (int j = 0; j < kShortLoads; ++j)
+    if (j * kPickThreads + tid < pieces) v[j] = *reinterpret_cast<const u32x4_any_t*>(row + (j * kPickThreads + tid) * 8);
+#pragma unroll
+  for (int j = 0; j < kShortLoads; ++j) {
+    const int c = j * kPickThreads + tid;
+    if (c >= pieces) break;
+    const uint32_t w[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) take((w[e >> 1] >> (16 * (e & 1))) & 0xffffu, c * 8 + e);
+  }
+  if (pieces * 8 + tid < V) take(row[pieces * 8 + tid], pieces * 8 + tid);
+  unsigned long long m = ((unsigned long long)best << 32) | (0xffffffffu - at);
+#pragma unroll
+  for (int o = 32; o; o >>= 1) {
+    const unsigned long long other = __shfl_xor(m, o);
+    m = other > m ? other : m;
+  }
+  __shared__ unsigned long long red[kPickThreads / kWave];
+  if ((tid & 63) == 0) red[tid >> 6] = m;
+  __syncthreads();
+  if (tid == 0) {
+#pragma unroll
+    for (int i = 1; i < kPickThreads / kWave; ++i) m = red[i] > m ? red[i] : m;
+    tokens[(int64_t)blockIdx.x * ldt] = (int64_t)(0xffffffffu - (uint32_t)m);
+    if (positions) positions[blockIdx.x] += 1;
+  }
+}
+
 // One workgroup per row: the row is requested in rounds of four 16-byte pieces per thread (32768 elements), so what it takes is
 // one round trip per round and the 60 GB/s of one compute unit.  Beside that every instruction per element shows, 32 of them in a thread: a
 // first pass takes the maximum alone, two elements to an instruction; then the threads that hold it look for it in the round where they met
 // it.  us per launch in a graph, value and index carried along element by element -> this: 32000 logits of 1 / 16 / 64 rows 5.3 -> 3.8, 5.9 -> 4.2,
 // 6.1 -> 4.4, 128256 of 1 / 16 rows 14.7 -> 6.0, 15.2 -> 6.5.  Ties go to the lowest index and NaN counts as the largest value, as torch.argmax
-// has it: a row with a NaN (its largest magnitude tells), or whose largest value is a zero of either sign, is looked through element by element.
+// has it: a row with a NaN (its largest magnitude tells), or whose largest value is a zero of either sign, is looked through element by element (32000 zeros 6.4).
 template <int DT>
 __global__ __launch_bounds__(kPickThreads) void greedy_token_kernel(const uint16_t* __restrict__ logits, int64_t ld, int64_t* __restrict__ tokens,
                                                                    int64_t ldt, int32_t* __restrict__ positions, int V) {
@@ -159,7 +204,10 @@ int fsvd_greedy_token(const void* logits, int64_t ld, int64_t* tokens, int64_t l
   if ((reinterpret_cast<uintptr_t>(logits) & 1) != 0) { set_last_error("%s: logits must be 2-byte aligned", fn); return kErrBadAlign; }
   const auto* x = static_cast<const uint16_t*>(logits);
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  if (dtype == 1) hipLaunchKernelGGL(greedy_token_kernel<1>, dim3(B), dim3(kPickThreads), 0, st, x, ld, tokens, ldt, positions, V);
+  if (V <= kShortRow) {
+    if (dtype == 1) hipLaunchKernelGGL(greedy_short_kernel<1>, dim3(B), dim3(kPickThreads), 0, st, x, ld, tokens, ldt, positions, V);
+    else hipLaunchKernelGGL(greedy_short_kernel<0>, dim3(B), dim3(kPickThreads), 0, st, x, ld, tokens, ldt, positions, V);
+  } else if (dtype == 1) hipLaunchKernelGGL(greedy_token_kernel<1>, dim3(B), dim3(kPickThreads), 0, st, x, ld, tokens, ldt, positions, V);
   else hipLaunchKernelGGL(greedy_token_kernel<0>, dim3(B), dim3(kPickThreads), 0, st, x, ld, tokens, ldt, positions, V);
   return launched(fn);
 }

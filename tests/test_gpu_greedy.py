@@ -35,13 +35,13 @@ def test_greedy_token_is_the_argmax(dtype, B, V, off):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("V,off", [(5, 0), (32768, 0), (32769, 2), (65535, 1), (70007, 0)])
+@pytest.mark.parametrize("V,off", [(5, 0), (8191, 1), (8200, 0), (14336, 3), (14337, 0), (14343, 0), (32768, 0), (32769, 2), (65535, 1), (70007, 0)])
 def test_greedy_token_where_the_largest_lies(V, off, dtype):
     """The largest value in the first piece, in the first and a later round, in the last round, behind the last whole piece; only zeros above the
     rest, of either sign; a NaN of either sign; the lowest finite value."""
     from flashsvd_amd import hip_ops
     x = -torch.rand(14, V + off, generator=torch.Generator().manual_seed(V)).to(dtype)[:, off:] - 1
-    first, mid, last = 0, V // 2, V - 1
+    first, mid, last = 0, V // 2, V - 1               # up to 14336 logits in one pass, from there on in two
     spots = [(first,), (mid,), (last,), (mid, last), (first, mid), (max(0, V - V % 8 - 1),), (min(V - 1, 32767), last)]
     want = []
     for r, s in enumerate(spots):
