@@ -464,8 +464,9 @@ __global__ __launch_bounds__(kThreads) void qkv_rope_append_kernel(QkvArgs a) {
 // run in the order of linear_kernel: the same bits.  32000 x 4096, weights from HBM: one row 44.6 -> 39.5 us (6.6 TB/s), with the norm 45.0 -> 40.8, two
 // rows 49.9 -> 42.5; 32000 x 2048 one row 25.7 -> 21.7.  Shorter rows, several to a window, one row / one with the norm / two: 32000 x 512
 // 8.8 -> 8.0, 10.7 -> 8.6, 13.9 -> 10.0, 128256 x 512 25.3 -> 24.2, 30.0 -> 24.7, 46.6 -> 28.1, 32000 x 1024 12.9 -> 12.7, 14.6 -> 13.3, 17.8 -> 14.5, two rows of
-// 128256 x 1024 57.5 -> 45.3; one row of that 41.7 -> 42.8, which therefore stays with linear_kernel above 128 rows per compute unit, as everything
-// does below 64 (16 per wave).
+// 128256 x 1024 57.5 -> 45.3.  With linear_kernel stays everything below 64 rows per compute unit (16 per wave), one row of 512 below 80 of them (18000 x 512
+// 5.6 -> 6.2, with the norm 6.8 -> 7.1; 22000 x 512 7.1 -> 6.4), one row of 1024 above 128 (128256 x 1024 41.7 -> 42.8), and two rows of 4096 without the norm
+// above 400 (128256 x 4096 152.4 -> 158.1; 100000 x 4096 121.7 -> 123.5; with the norm 175.3 -> 160.0).
 // ---------------------------------------------------------------------------------------
 template <int DT, int BATCH, int P>
 __global__ __launch_bounds__(kThreads) void linear_slab_kernel(LinearArgs a) {
@@ -660,14 +661,19 @@ static int launch_linear_slab(const LinearArgs& a, hipStream_t st) {
 }
 template <int DT>
 static int launch_linear_t(const LinearArgs& a, int cfg, hipStream_t st) {
-  if (cfg == 0 && a.B <= 2 && a.positions == nullptr && compute_units() > 0 && a.N >= 64 * compute_units() && a.ldw % 8 == 0 && aligned16(a.W) && below_4gib(a.N, a.ldw)) {
+  const int64_t cu = compute_units();
+  if (cfg == 0 && a.B <= 2 && a.positions == nullptr && cu > 0 && a.N >= 64 * cu && a.ldw % 8 == 0 && aligned16(a.W) && below_4gib(a.N, a.ldw)) {
     switch (a.K) {
-      case 512: return launch_linear_slab<DT, 1>(a, st);
+      case 512:
+        if (a.B == 1 && a.N < 80 * cu) break;
+        return launch_linear_slab<DT, 1>(a, st);
       case 1024:
-        if (a.B == 1 && a.N > 128 * compute_units()) break;
+        if (a.B == 1 && a.N > 128 * cu) break;
         return launch_linear_slab<DT, 2>(a, st);
       case 2048: return launch_linear_slab<DT, 4>(a, st);
-      case 4096: return launch_linear_slab<DT, 8>(a, st);
+      case 4096:
+        if (a.B == 2 && a.norm_w == nullptr && a.N > 400 * cu) break;
+        return launch_linear_slab<DT, 8>(a, st);
     }
   }
   const bool vec = (a.K % 8 == 0) && (a.ldw % 8 == 0) && aligned16(a.W);
