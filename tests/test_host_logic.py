@@ -357,7 +357,18 @@ def test_factor_modules_are_what_the_attributes_are(half, name):
     part.__class__ = type("Provided", (type(part),), {name: property(lambda self: other)})
     assert getattr(part, name) is other
     assert any(m is other for m in part._factor_modules()) and not any(m is own for m in part._factor_modules())
-    part.__class__ = type(part).__mro__[1]
+    part.__class__ = cls = type(part).__mro__[1]
+    assert any(m is own for m in part._factor_modules())
     part.__dict__[name] = other
     assert getattr(part, name) is other
     assert any(m is other for m in part._factor_modules()) and not any(m is own for m in part._factor_modules())
+    del part.__dict__[name]
+    for attr, value in ((name, property(lambda self: other)), ("__getattr__", lambda self, n: other if n == name else torch.nn.Module.__getattr__(self, n)),
+                        ("__getattribute__", lambda self, n: other if n == name else object.__getattribute__(self, n))):
+        setattr(cls, attr, value)                       # put on the class itself
+        try:
+            assert getattr(part, name) is other
+            assert any(m is other for m in part._factor_modules()) and not any(m is own for m in part._factor_modules())
+        finally:
+            delattr(cls, attr)
+    assert any(m is own for m in part._factor_modules())
