@@ -218,14 +218,14 @@ struct SplitWorkspace { float* part; size_t part_floats; int32_t* count; int nco
 SplitWorkspace split_workspace();                                            // capi.hip
 bool gemm_tiles_apply(const MfmaArgs& a);                                   // mfma_gemm.hip: 128 rows and more
 int launch_gemm_tiles(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
-bool gemm_rows_apply(const MfmaArgs& a);                                    // mfma_gemm.hip: 5..127 rows, K split
+bool gemm_rows_apply(const MfmaArgs& a);                                    // mfma_gemm.hip: 3..127 rows, K split
 int launch_gemm_rows(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
 int compute_units();                                                         // of the current device, 0 when it cannot be asked
 bool gemm_big_apply(const MfmaArgs& a, bool dual);                          // mfma_big.hip: 256 x 256 tiles
 int launch_gemm_big(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
 bool expand_big_apply(const ExpandArgs* d, int n);
 int launch_expand_big(const ExpandArgs* d, int n, hipStream_t st);
-bool gemm_quad_apply(const MfmaArgs& a, bool dual);                         // mfma_quad.hip: prompts, K of five steps and more
+bool gemm_quad_apply(const MfmaArgs& a, bool dual);                         // mfma_quad.hip: 33 rows and more, K of five steps and more
 int launch_gemm_quad(const MfmaArgs& a, bool dual, hipStream_t st, const char* who);
 bool expand_quad_apply(const ExpandArgs* d, int n);                         // mfma_quad_heads.hip
 int launch_expand_quad(const ExpandArgs* d, int n, hipStream_t st);

@@ -546,7 +546,8 @@ static int pick_ksplit(int64_t tiles, int ksteps, size_t floats_per_share, const
 // units idle (up to 128 tiles: two workgroups per tile-starved pair of compute units) or walks a very long K with at
 // most two workgroups per compute unit (down_v of the 7B MLP, K = 11008).  Measured at 128..1024 rows with weights from
 // HBM: o_v 18 -> 12..15 us, down_v 51 -> 25 (128 rows), 32 (256), 46 (512), 92 -> 76 (1024); everything else is as fast
-// or faster unsplit.  (Calls with scratch of their own take the shares of mfma_quad.hip for such a K: 20, 24, 36, 47.)
+// or faster unsplit.  (Calls with scratch of their own take the shares of mfma_quad.hip for such a K: 20, 24, 36, 47; of calls without, the unsplit tiles
+// there take what their rule split_is_ahead does not leave here.)
 static int pick_ksplit_prompt(int64_t tiles, int ksteps, int K, size_t floats_per_share, const SplitWorkspace& ws) {
   int z = 1;
   if (tiles <= 128) z = (int)((256 + tiles - 1) / tiles);
@@ -667,8 +668,8 @@ bool gemm_ragged_apply(const MfmaArgs& a) {
 // rows 12.7 / 11.1, 13.6 / 12.0, 13.4 / 11.7, 1492 x 4104 27.4 / 19.4, 28.9 / 21.7, 28.1 / 21.0, 64 x 64 tiles alike: 4096 x 1492 at
 // 333, 500 rows 21.5 / 19.9, 23.7 / 22.0, 1492 x 4104 26.4 / 22.8, 32.5 / 26.1.  The pair at 3, 16, 64, 127 rows: 11008 x 1492
 // 24.7, 27.1, 43.4, 55.1 (with a split over three workgroups, which has to park partial tiles, 33.1, 34.6, 41.0, 54.8).
-// From 128 rows on the tiles of mfma_mid.hip take what gives about every compute unit one (or several rounds of the pair's); a K of 320 and more on
-// the 4-byte grid does not come here (mfma_quad.hip).
+// From 128 rows on the tiles of mfma_mid.hip take what gives about every compute unit one (or several rounds of the pair's).  Of a K of 320 and more on
+// the 4-byte grid comes what the rule of mfma_quad.hip leaves (ragged_is_ahead_elsewhere).
 template <int DT>
 static int launch_gemm_ragged_dt(const MfmaArgs& a, bool dual, hipStream_t st, const char* who) {
   if (gemm_mid_ragged_apply(a, dual)) return launch_mid_ragged(a, dual, st, who);

@@ -1,7 +1,7 @@
 // Projections and head expansions of prompts of 128 to about 3000 rows (head expansions from 16): workgroups of eight waves, one
 // per output tile, operand rows straight into a ring of three to five LDS stages.  They serve a K below 320, the pair in the rounding that keeps the
-// gate in 32 bits and ragged rows off the 4-byte grid; everything else is ahead on the four-wave tiles of mfma_quad.hip (figures there).  Times below
-// at a longer K are those by which the rules were set.
+// gate in 32 bits, ragged rows off the 4-byte grid, and the pairs and ragged rows that the rules of mfma_quad.hip leave here (figures there); everything
+// else is ahead on the four-wave tiles.  Times below at a longer K are those by which the rules were set.
 //
 // Up to a few tiles per compute unit neither form beside this one fits: the two-stage tiles of mfma_gemm.hip rely on a second
 // workgroup of the compute unit to cover a load distance of one step and wait out most of it, and the 256 x 256 tiles of

@@ -33,9 +33,12 @@ static float share_sum_us(int64_t floats) { return kShareSumUs + (float)floats *
 
 constexpr int kQuadNone = -1;
 struct QuadPick { int form; float us; };
-// The order of a single matrix's sums is the one that its shape had on the tiles before these (rings with K halved between waves, 64 x 64
-// tiles with K cut over workgroups), so that the bits stay: a model of 32 layers hands a flipped rounding on until another order of
-// the same sums ends 0.046 (relative) away.  Both cost nothing here: a second set of accumulators, a sum kept in registers.
+// The order of the sums of 128 aligned rows and more is the one that the shape had on the tiles before these (rings with K halved between waves, 64 x
+// 64 tiles with K cut over workgroups), so that the bits stay: a model of 32 layers hands a flipped rounding on until another order of the same
+// sums ends 0.046 (relative) away.  Both cost nothing here: a second set of accumulators, a sum kept in registers.  Other orders than before have 33
+// to 127 rows (one sum, no split), ragged single matrices (one sum; the tiles before halved K between waves), a K of 4096 to 5119 that filling_shares
+// declines by its costs, and a K of 8192 and more without scratch that split_is_ahead leaves here (133 such shapes: the error against
+// 64 bits, 0.0017 from the output's rounding, grows by at most 1.2e-7 of itself).
 enum QuadOrder { kOrderPlain = 0, kOrderHalves = 1, kOrderCut = 2 };
 struct QuadSums { QuadOrder order; int per; };
 static QuadSums quad_sums(const MfmaArgs& a) {
@@ -88,9 +91,9 @@ static bool quad_words(const MfmaArgs& a, bool dual) {
   const auto al4 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 3) == 0; };
   return a.ldx % 2 == 0 && a.ldw % 2 == 0 && a.up_off % 2 == 0 && al4(a.x) && al4(a.W) && (!dual || al4(a.W2));
 }
-// From 128 rows and five K steps on (fewer steps than the stages hold are left to the tiles that were measured for them); N holds a whole
-// residual piece.  The pair in the rounding that keeps the gate in 32 bits goes to mfma_mid.hip.  From 33 rows on where there are 64 tiles of
-// 64 x 64 with a K below 4096, or 128 of them (us at 40 / 64 / 100 rows, 32-row tiles with K split over workgroups -> these: the pair 11008 x 1536 30.6 ->
+// From 128 rows and five K steps on (fewer steps than the stages hold are left to the tiles that were measured for them), but for what the rules in
+// front of gemm_quad_apply leave to other kernels; N holds a whole residual piece.  The pair in the rounding that keeps the gate in 32 bits goes to
+// mfma_mid.hip.  From 33 rows on where there are 64 tiles of 64 x 64 with a K below 4096, or 128 of them (us at 40 / 64 / 100 rows, 32-row tiles with K split over workgroups -> these: the pair 11008 x 1536 30.6 ->
 // 19.3, 31.9 -> 21.4, 34.5 -> 23.3, 32000 x 4096 65 -> 53, 72 -> 56, 99 -> 62, 4096 x 1024 8.7 -> 7.4, 8.9 -> 8.2, 10.9 -> 7.5); fewer tiles
 // need the split (3072 x 4096 16.1 against 18.5, 16.9 against 21.3; 1024 x 4096 9.4 against 17.8).
 static bool quad_range(const MfmaArgs& a, bool dual) {
@@ -242,65 +245,79 @@ static int launch_share_dt(QuadArgs& q, const ShareForm& f, hipStream_t st, cons
   return f.bm == 128 ? launch_share_t<DT, 4, 4, 4, 5, 1>(q, st, who) : launch_share_t<DT, 8, 4, 3, 3, 1>(q, st, who);
 }
 
-// A call of 128 rows and more that runs in no shares of its own is left to the 64 x 64 tiles of mfma_gemm.hip, K split over workgroups that add up in the
-// registered buffer, where that has room and the split is ahead of one workgroup per tile.  us in one workgroup / split, tiles x ranges in
-// brackets, weights from HBM:
+// ---- what stays with the kernels before these because they are ahead there.  How full the row tiles are counts throughout: as many tiles take longer with
+// full ones (64 of 256 and of 200 rows, 1024 x 3584, one per compute unit: 18.0 and 14.7 us; why is not shown yet), and more so here than there.
+static bool rows_fill(const MfmaArgs& a) { return (int64_t)a.B * 16 >= (int64_t)((a.B + 63) / 64) * 64 * 15; }
+
+// A call of 128 rows and more that runs in no shares of its own: the 64 x 64 tiles of mfma_gemm.hip, K split over workgroups that add up in the registered
+// buffer, where that has room and the split is ahead of one workgroup per tile.  us in one workgroup / split, tiles x ranges in brackets,
+// weights from HBM:
 //   K of 1536 to 8191: up to one workgroup of the split per compute unit, 128 x 1024 x 1536 (32 x 3) 10.3 / 9.4, x 4096 (32 x 8) 19.8 / 12.4, 256 x 1024 x
-//     3584 (64 x 4) 17.4 / 12.0, 512 x 1024 x 5504 (128 x 2) 26.4 / 20.5, and any split of 51 tiles, 128 x 1536 x 5504 (48 x 6) 26.8 / 18.7.  Not with more
-//     workgroups, where neighbours on a compute unit cover each other: 333 x 704 x 3072 (66 x 4) 13.4 / 14.6; a quarter more from a K of 3840 on, 128 x
-//     2560 x 3840 (80 x 4) 21.4 / 19.0, 512 x 768 x 3840 (96 x 3) 20.2 / 18.2, 256 x 1536 x 4096 (96 x 3) 19.9 / 20.7, x 5504 26.5 / 24.3.  Shorter: 128 x
-//     1024 x 1024 (32 x 2) 7.9 / 9.1.
-//   K of 8192 and more (a K below 4096 gets no scratch and these may come without): up to 128 tiles, 128 x 1536 x 11008 51.9 / 24.6, 512 x 1024 x 8192
-//     34.1 / 29.2, up to 192 from 10240 on, 512 x 1536 x 11008 50.9 / 46.4.  Not 200 x 2560 x 8192 (160 tiles) 28.5 / 37.4.
+//     3584 (64 x 4) 17.4 / 12.0, 512 x 1024 x 5504 (128 x 2) 26.4 / 20.5; below 2048 with full row tiles and 512 columns only (185 x 812 x 1600 10.3 /
+//     11.1, 128 x 1024 x 1024 7.9 / 9.1).  More workgroups lose, as neighbours on a compute unit cover each other, 333 x 704 x 3072 (66 x 4) 13.4 / 14.6, 592 x
+//     267 x 1856 (50 x 6) 9.3 / 13.9, until K is long: 128 x 1536 x 5504 (48 x 6) 26.8 / 18.7, 128 x 2560 x 3840 (80 x 4) 21.4 / 19.0, 154 x 1536 x 5504 (72 x
+//     4) 22.2 / 20.2 (x 4096 18.5 / 18.7).
+//   K of 8192 and more: up to 128 tiles, 128 x 1536 x 11008 51.9 / 24.6, 512 x 1024 x 8192 34.1 / 29.2, up to 192 with full row tiles from 10240 on, 512 x 1536 x
+//     11008 50.9 / 46.4.  Not 200 x 2560 x 11008 (160 tiles) 39.7 / 46.6.
 static bool split_is_ahead(const MfmaArgs& a) {
   if (a.B < 128 || a.K < 1536 || gemm_mid_rule(a).area > 0 || gemm_big_apply(a, false)) return false;
   const int64_t tiles = quad_tiles(a, 2, 2), cu = compute_units();
   const TilesCut c = gemm_tiles_cut(a);
   if (!c.room) return false;
   const int64_t wgs = tiles * c.ranges;
-  const bool ahead = a.K < 8192 ? wgs <= cu || tiles * 5 <= cu || (a.K >= 3840 && wgs * 4 <= cu * 5) : tiles * 2 <= cu || (a.K >= 10240 && tiles * 4 <= cu * 3);
+  const bool full = rows_fill(a);
+  bool ahead;
+  if (a.K >= 8192) ahead = tiles * 2 <= cu || (full && a.K >= 10240 && tiles * 4 <= cu * 3);
+  else if (wgs <= cu) ahead = a.K >= 2048 || (full && a.N >= 512);
+  else if (tiles * 5 <= cu) ahead = a.K >= (full ? 3072 : 4096);
+  else ahead = a.N >= 320 && wgs * 3 <= cu * 4 && a.K >= (full ? 3584 : 5120);
   return ahead && share_form(a).shares == 0;
 }
 
-// 33 to 127 aligned rows whose 32 x 64 tiles are at most one per compute unit are left to those of mfma_gemm.hip, K split over workgroups in the registered
-// buffer, where K is long.  us here / split, weights from HBM: a single matrix of up to half as many tiles from a K of 2048 on, 64 x 4096 x 3072 18.4 / 14.3 (K
-// 1536 10.9 / 11.3), of more from 5120 on, 127 x 4096 x 5504 29.1 / 26.8, x 11008 54.8 / 45.8, 64 x 8192 x 8192 43.7 / 39.4 (127 x 4096 x 4096 21.6 / 21.0, 96
-// rows 18.6 / 23.0).  The pair by how many shares of K the tiles leave room for: up to half of them from 1024 on, 127 x 2048 x 1536 21.6 / 16.7, up to two
-// thirds from 1280 on, 64 x 5504 x 2752 38.1 / 29.1 (K 1024 16.0 / 19.2), else from 2048 on, 127 x 4096 x 4096 48.9 / 38.2.  With more tiles this is ahead at
-// any K: the pair 64 x 11008 x 4096 56.1 / 59.5.
+// 33 to 127 aligned rows with at most one 32 x 64 tile per compute unit: those of mfma_gemm.hip, K split over workgroups in the registered buffer, where K
+// is long.  The split gives every compute unit two workgroups, or a few more and with them a second round; from which K on it is ahead goes by that
+// and by how many ranges there are.  us here / split, weights from HBM: a single matrix of up to half as many tiles, 64 x 4096 x 3072 18.4 / 14.3 (K 1536
+// 10.9 / 11.3), of more 127 x 4096 x 5504 29.1 / 26.8, x 11008 54.8 / 45.8, 64 x 8192 x 8192 43.7 / 39.4 (127 x 4096 x 4096 21.6 / 21.0); with a second
+// round 65 x 4096 x 11008 40.1 / 43.6.  The pair of up to half as many tiles 64 x 4096 x 1536 23.6 / 17.7, two thirds 64 x 5504 x 2752 38.1 / 29.1 (K 1024 16.0 /
+// 19.2), more 127 x 4096 x 4096 48.9 / 38.2; with a second round 65 x 2048 x 1536 18.5 / 20.9, 96 x 4096 x 4096 44.7 / 38.3 (K 2048 25 / 27).
 static bool narrow_split_is_ahead(const MfmaArgs& a, bool dual) {
   const int64_t t = quad_tiles(a, 1, 2), cu = compute_units();
   if (t > cu || !gemm_rows_apply(a)) return false;
-  if (!dual) return a.K >= (t * 2 <= cu ? 2048 : 5120);
-  return a.K >= (t * 2 <= cu ? 1024 : (t * 16 <= cu * 11 ? 1280 : 2048));
+  const bool one_round = (2 * cu + t - 1) / t * t <= 2 * cu + 8, half = t * 2 <= cu;
+  if (!dual) return a.K >= (!one_round ? 9216 : (half ? 2048 : 5120));
+  return a.K >= (!one_round ? (half ? 1792 : 2432) : (half ? 1024 : (t * 16 <= cu * 11 ? 1280 : 1792)));
 }
 
-// The pair of 128 aligned rows and more with a K of 1024 and more is left to the 64 x 64 tiles of mfma_gemm.hip where these are at most one per compute
-// unit, and to the 64 x 192 ring of mfma_mid.hip where that takes the shape and 64 x 96 would serve it here.  us here / there, weights from HBM: 128 x 2752 x
-// 1536 21.8 / 20.1, 256 x 4096 x 2432 31.3 / 28.5 (K 1024 15.4 / 15.1, 768 11.2 / 13.1); 256 x 11008 x 1536 41.1 / 38.8, 575 x 4964 x 1536 39.1 / 35.7 (256 x
-// 11008 x 512 16.6 / 17.2).
+// The pair of 128 aligned rows and more with a K of 1024 and more: the 64 x 64 tiles of mfma_gemm.hip where these are at most one per compute unit, and the
+// 64 x 192 ring of mfma_mid.hip where that takes the shape with hardly a padded column and 64 x 96 would serve it here.  us here / there, weights from HBM:
+// 128 x 2752 x 1536 21.8 / 20.1, 256 x 4096 x 2432 31.3 / 28.5 (K 1024 15.4 / 15.1, 768 11.2 / 13.1); 256 x 11008 x 1536 41.1 / 38.8, 575 x 4964 x 1536 39.1 /
+// 35.7 (256 x 11008 x 512 16.6 / 17.2, 800 x 2752 x 1536, a twentieth of it padding, 32.1 / 33.5).
 static bool pair_of_64_is_ahead(const MfmaArgs& a) {
   if (a.B < 128 || a.K < 1024) return false;
-  return quad_tiles(a, 2, 2) <= compute_units() || (quad_pick(a, true, false).form == 8 && gemm_mid_pair_of_64(a));
+  if (quad_tiles(a, 2, 2) <= compute_units()) return true;
+  const int64_t wide = ((int64_t)a.N + 191) / 192 * 192;
+  return (int64_t)a.N * 29 >= wide * 28 && quad_pick(a, true, false).form == 8 && gemm_mid_pair_of_64(a);
 }
 
 // Ragged rows: the tiles here take up to twice their costs with them (256 x 4096 x 4098 34 us, 18 by the table), so that the register pipelines of mfma_gemm.hip
 // and mfma_mid.hip are ahead on few or small tiles.  us here / there, weights from HBM:
 //   a pair of up to 127 rows with at most one of the 32 x 64 tiles per compute unit, 64 x 5504 x 746 18.4 / 14.7, 33 x 4096 x 2050 38.6 / 25.8 (65 x 5504 x 746,
 //     one and a little, 14.8 / 15.4); of more rows with at most one 64 x 64 tile from a K of 1152 on, 154 x 1376 x 2050 35.9 / 30.8 (128 x 4096 x 1492 31.2 / 31.5);
-//   a single matrix with at most one 32 x 64 tile per compute unit, 128 x 4096 x 1492 15.7 / 11.5, 256 x 704 x 2050 18.2 / 12.5 (K 322 as fast);
-//   one that the 64 x 128 ring takes, unless 96 x 64 serves it here, 512 x 4096 x 1492 24.2 / 20.3 (1500 x 704 x 1492 on 96 x 64 15.3 / 18.2); one that
-//     the 128 x 128 ring takes and smaller or larger tiles would serve here, of up to 192 rows from 1280 on, 154 x 11008 x 4098 65.6 / 58.0, else from 6144 on;
-//   64 x 64 tiles here from a K of 2048 on, 256 x 4096 x 4098 34.2 / 28.9, or from 1280 on where no row tile is padded, 256 x 4096 x 1492 15.5 / 14.4 (200 x
-//     4096 x 1492 10.4 / 12.8); 96 x 64 that fill three quarters of the chip with up to 192 rows, 154 x 5504 x 4098 37.5 / 34.3.
+//   a single matrix with at most one 32 x 64 tile per compute unit, 128 x 4096 x 1492 15.7 / 11.5, 256 x 704 x 2050 18.2 / 12.5 (K 322 as fast); with padded row
+//     tiles from a K of 2048 on, or 1000 where they are few (200 x 1002 x 746 6.7 / 7.7, 154 x 256 x 1492 9.9 / 8.5);
+//   one that the 64 x 128 ring takes, unless 96 x 64 serves it here, 512 x 4096 x 1492 24.2 / 20.3 (1500 x 704 x 1492 on 96 x 64 15.3 / 18.2); one that the
+//     128 x 128 ring takes and 96 x 64 would serve here, of up to 192 rows from 1280 on, 154 x 11008 x 4098 65.6 / 58.0, else from 6144 on;
+//   64 x 64 tiles here without padded rows from 1280 on, 256 x 4096 x 4098 34.2 / 28.9, x 1492 15.5 / 14.4 (200 x 4096 x 1492 10.4 / 12.8, x 2050 12.8 / 14.8),
+//     with them from 2048 on and more than one per compute unit; 96 x 64 that fill three quarters of the chip with up to 192 rows, 154 x 5504 x 4098 37.5 / 34.3.
 static bool ragged_is_ahead_elsewhere(const MfmaArgs& a, bool dual) {
-  const int64_t cu = compute_units();
-  if (dual) return a.B < 128 ? quad_tiles(a, 1, 2) <= cu : a.K >= 1152 && quad_tiles(a, 2, 2) <= cu;
-  if (quad_tiles(a, 1, 2) <= cu) return true;
+  const int64_t cu = compute_units(), t32 = quad_tiles(a, 1, 2), t64 = quad_tiles(a, 2, 2);
+  if (dual) return a.B < 128 ? t32 <= cu : a.K >= 1152 && t64 <= cu;
+  const bool full = rows_fill(a);
+  if (t32 <= cu) return full || a.K >= 2048 || (t32 * 4 <= cu && a.K >= 1000);
   const int ring = gemm_mid_ragged_rows(a), form = quad_pick(a, false, true).form;
   if (ring == 64) return form != 10;
-  if (ring == 128) return form != 5 && a.K >= (a.B <= 192 ? 1280 : 6144);
-  if (form == 12) return a.K >= 2048 || (a.K >= 1280 && (int64_t)a.B * 16 >= (a.B + 63) / 64 * 64 * 15);
+  if (ring == 128) return form == 10 && a.K >= (a.B <= 192 ? 1280 : 6144);
+  if (form == 12) return full ? a.K >= 1280 : a.K >= 2048 && t64 > cu;
   return form == 10 && a.B <= 192 && a.K >= 2048 && quad_tiles(a, 3, 2) * 4 <= 3 * cu;
 }
 

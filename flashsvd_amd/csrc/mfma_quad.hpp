@@ -1,10 +1,10 @@
 // Projections and head expansions of prompts: the kernel (rules and launches: mfma_quad.hip and mfma_quad_heads.hip).
 //
 // A workgroup is four waves, one per SIMD, that own a quarter of the output tile each: (16 TM) x (16 TN) of (32 TM) x (32 TN).  What
-// bounds these products beside the matrix cores is the way of the operands into the registers: loads reach LDS at 93 to 104 bytes
-// per ns and compute unit whatever the pattern (loads alone, rows of 128 bytes), and a fragment read by every wave that shares it
-// costs LDS cycles and, under the chip's power limit, clock.  Four waves of 128 x 128 read two thirds of what eight of 128 x 64 do
-// for the same products: 8192 x 8192 x 8192 723 us (1.52 PFLOP/s; eight waves 1.31 PFLOP/s at 16384 x 4992 x 4096, this 1.43; products
+// bounds these products beside the matrix cores is the way of the operands into the registers: the loads of a walk reach LDS at 50 to 90 bytes
+// per ns and compute unit, products and reads taken out (512 x 3072 x 4096 18.6 of 20.0 us, 8192 x 8192 x 8192 490 of 717), and a fragment read by
+// every wave that shares it costs LDS cycles and, under the chip's power limit, clock.  Four waves of 128 x 128 read two thirds of what eight of 128 x
+// 64 do for the same products: 8192 x 8192 x 8192 723 us (1.52 PFLOP/s; eight waves 1.31 PFLOP/s at 16384 x 4992 x 4096, this 1.43; products
 // alone, operands fixed, 1.65 to 1.7 at the clock that the chip then keeps).
 //
 // One wave per SIMD has nobody to fill its gaps, so the order is laid down by hand: a K step of 64 is two slices of 32, a slice's

@@ -88,7 +88,7 @@ def test_calls_without_scratch_split_in_the_registered_buffer(B, N, K, form):
 
 @pytest.mark.parametrize("B,N,K,form", [(128, 1024, 3584, "tiles 64 x 64"), (130, 259, 2048, "tiles 64 x 64"), (512, 1024, 3328, "tiles 64 x 64"),
                                         (128, 1024, 1536, "tiles 64 x 64"), (128, 2559, 3840, "tiles 64 x 64"),
-                                        (512, 768, 3072, "quad 64 x 64 ranges"), (128, 1024, 1472, "quad 64 x 64 ranges")])
+                                        (512, 768, 3584, "tiles 64 x 64"), (512, 768, 3072, "quad 64 x 64 ranges"), (200, 1024, 1600, "quad 64 x 64 ranges"), (128, 1024, 1472, "quad 64 x 64 ranges")])
 def test_a_k_too_short_for_scratch(B, N, K, form):
     from flashsvd_amd import hip_ops
     x, w = _rand(B, K, seed=1), _rand(N, K, std=K ** -0.5, seed=2)

@@ -47,7 +47,7 @@ def test_linear(B, N, K, form, dtype):
 @pytest.mark.parametrize("B,N,K,single,pair", [
     (64, 4090, 3072, "tiles 32 x 64", "tiles 32 x 64 pair"), (33, 4096, 1984, "quad 64 x 64", "tiles 32 x 64 pair"), (100, 4096, 960, "quad 64 x 64", "quad 64 x 96 pair"),
     (127, 4090, 5184, "tiles 32 x 64", "tiles 32 x 64 pair"), (127, 4096, 2048, "quad 64 x 64", "tiles 32 x 64 pair"), (64, 5500, 1280, "quad 64 x 64", "tiles 32 x 64 pair"),
-    (70, 8192, 5184, "quad 64 x 64", "quad 64 x 96 pair"),
+    (70, 8192, 5184, "quad 64 x 64", "quad 64 x 96 pair"), (65, 4096, 5184, "quad 64 x 64", "tiles 32 x 64 pair"), (65, 4096, 2048, "quad 64 x 64", "quad 64 x 96 pair"),
 ])
 def test_few_tiles_of_a_long_k_split(B, N, K, single, pair):
     """33 to 127 rows: on either side of the lines, with the registered buffer; without it everything runs here."""
@@ -74,8 +74,10 @@ def test_few_tiles_of_a_long_k_split(B, N, K, single, pair):
     (297, 12319, 323, "any quad 192 x 128"), (128, 8256, 322, "any quad 128 x 128"), (130, 5559, 383, "any quad 96 x 64"),
     (131, 4103, 321, "any quad 64 x 64"), (8230, 8, 385, "any quad 64 x 64"), (200, 4096, 1281, "any quad 64 x 64"),
     # on either side of the lines to the other tiles
-    (130, 259, 321, "any rows 32 x 64"), (131, 8, 385, "any rows 32 x 64"), (128, 4096, 1490, "any rows 32 x 64"), (200, 4096, 2050, "any rows 64 x 64"),
-    (256, 4096, 1281, "any rows 64 x 64"), (500, 4090, 1490, "any ring 64 x 128"), (1500, 700, 1490, "any quad 96 x 64"), (154, 11008, 1282, "any ring 128 x 128"),
+    (128, 259, 321, "any rows 32 x 64"), (130, 259, 321, "any quad 64 x 64"), (130, 259, 1025, "any rows 32 x 64"), (131, 8, 385, "any quad 64 x 64"),
+    (200, 1002, 1025, "any quad 64 x 64"), (200, 1002, 2050, "any rows 32 x 64"), (128, 4096, 1490, "any rows 32 x 64"), (200, 4096, 2050, "any quad 64 x 64"),
+    (200, 5504, 2050, "any rows 64 x 64"), (256, 4096, 1281, "any rows 64 x 64"), (500, 4090, 1490, "any ring 64 x 128"), (1500, 700, 1490, "any quad 96 x 64"),
+    (154, 11008, 1282, "any ring 128 x 128"),
     (154, 11008, 1274, "any quad 96 x 64"), (154, 5500, 2050, "any rows 64 x 64"), (420, 5504, 1490, "any quad 96 x 64"),
 ])
 def test_linear_any_grid(B, N, K, form, dtype):
@@ -88,7 +90,7 @@ def test_linear_any_grid(B, N, K, form, dtype):
     (168, 27083, 1280, "quad 256 x 128 pair"), (261, 9918, 320, "quad 128 x 128 pair"), (67, 25091, 832, "quad 128 x 128 pair alone"),
     (129, 17205, 896, "quad 96 x 192 pair"), (72, 12319, 320, "quad 96 x 96 pair"), (66, 8328, 320, "quad 64 x 96 pair"),
     (130, 259, 320, "quad 64 x 64 pair"), (250, 4090, 960, "quad 64 x 96 pair"), (250, 4090, 1024, "tiles 64 x 64 pair"), (260, 4090, 1152, "quad 64 x 96 pair"),
-    (250, 11001, 960, "quad 64 x 96 pair"), (250, 11001, 1024, "ring 64 x 192 pair"),
+    (790, 2750, 1536, "quad 64 x 96 pair"), (250, 11001, 960, "quad 64 x 96 pair"), (250, 11001, 1024, "ring 64 x 192 pair"),
     (341, 12357, 323, "any quad 128 x 192 pair"), (261, 9918, 322, "any quad 128 x 128 pair"), (129, 17205, 894, "any quad 96 x 192 pair"),
     (130, 8954, 383, "any quad 96 x 96 pair"), (130, 259, 321, "any quad 64 x 96 pair"), (40, 8300, 330, "any quad 64 x 96 pair"),
     (40, 8190, 330, "any rows 32 x 64 pair"), (130, 2750, 1153, "any rows 64 x 64 pair"), (130, 2750, 1151, "any quad 64 x 96 pair"),
