@@ -256,7 +256,7 @@ static bool rows_fill(const MfmaArgs& a) { return (int64_t)a.B * 16 >= (int64_t)
 //     3584 (64 x 4) 17.4 / 12.0, 512 x 1024 x 5504 (128 x 2) 26.4 / 20.5; below 2048 with full row tiles and 512 columns only (185 x 812 x 1600 10.3 /
 //     11.1, 128 x 1024 x 1024 7.9 / 9.1).  More workgroups lose, as neighbours on a compute unit cover each other, 333 x 704 x 3072 (66 x 4) 13.4 / 14.6, 592 x
 //     267 x 1856 (50 x 6) 9.3 / 13.9, until K is long: 128 x 1536 x 5504 (48 x 6) 26.8 / 18.7, 128 x 2560 x 3840 (80 x 4) 21.4 / 19.0, 154 x 1536 x 5504 (72 x
-//     4) 22.2 / 20.2 (x 4096 18.5 / 18.7).
+//     4) 22.2 / 20.2 (x 4096 17.4 / 17.9).
 //   K of 8192 and more: up to 128 tiles, 128 x 1536 x 11008 51.9 / 24.6, 512 x 1024 x 8192 34.1 / 29.2, up to 192 with full row tiles from 10240 on, 512 x 1536 x
 //     11008 50.9 / 46.4.  Not 200 x 2560 x 11008 (160 tiles) 39.7 / 46.6.
 static bool split_is_ahead(const MfmaArgs& a) {
