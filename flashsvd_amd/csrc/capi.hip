@@ -629,7 +629,14 @@ int fsvd_lowrank_expand_heads_multi(const fsvd_expand_desc* desc, int n, const v
 int fsvd_rope_tables(const int64_t* positions, const float* inv_freq, void* cos_out, void* sin_out, int64_t rows, int half, int dtype, void* stream) {
   const char* fn = "fsvd_rope_tables";
   FSVD_REQUIRE_PTR(positions, fn); FSVD_REQUIRE_PTR(inv_freq, fn); FSVD_REQUIRE_PTR(cos_out, fn); FSVD_REQUIRE_PTR(sin_out, fn);
-  return launch_rope_tables(positions, inv_freq, u16(cos_out), u16(sin_out), rows, half, dtype, static_cast<hipStream_t>(stream));
+  return launch_rope_tables(positions, inv_freq, u16(cos_out), u16(sin_out), rows, half, nullptr, nullptr, 0, dtype, static_cast<hipStream_t>(stream));
+}
+int fsvd_rope_tables_mask(const int64_t* positions, const float* inv_freq, void* cos_out, void* sin_out, int64_t rows, int half, const int64_t* mask,
+                          uint8_t* pad_out, int64_t mask_count, int dtype, void* stream) {
+  const char* fn = "fsvd_rope_tables_mask";
+  FSVD_REQUIRE_PTR(positions, fn); FSVD_REQUIRE_PTR(inv_freq, fn); FSVD_REQUIRE_PTR(cos_out, fn); FSVD_REQUIRE_PTR(sin_out, fn);
+  if (mask_count != 0) { FSVD_REQUIRE_PTR(mask, fn); FSVD_REQUIRE_PTR(pad_out, fn); }
+  return launch_rope_tables(positions, inv_freq, u16(cos_out), u16(sin_out), rows, half, mask, pad_out, mask_count, dtype, static_cast<hipStream_t>(stream));
 }
 
 int fsvd_attn_prefill(const void* q, int64_t sq_b, int64_t sq_m, int64_t sq_h, const void* k, const void* v, int64_t sk_b,

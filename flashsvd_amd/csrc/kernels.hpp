@@ -168,7 +168,8 @@ int launch_expand_tiles(const ExpandArgs& a, hipStream_t st);
 bool expand_multi_apply(const ExpandArgs* d, int n);                        // two or three expansions in one launch
 int launch_expand_multi(const ExpandArgs* d, int n, hipStream_t st);
 int launch_prefill_attn(const PrefillAttnArgs& a, hipStream_t st);
-int launch_rope_tables(const int64_t* pos, const float* inv_freq, uint16_t* cos_out, uint16_t* sin_out, int64_t rows, int half, int dt, hipStream_t st);
+int launch_rope_tables(const int64_t* pos, const float* inv_freq, uint16_t* cos_out, uint16_t* sin_out, int64_t rows, int half, const int64_t* mask,
+                       uint8_t* pad, int64_t nmask, int dt, hipStream_t st);
 
 // matrix-core projections: y = epilogue(x . W^T) with the rounding points of the vector kernels
 struct MfmaArgs {

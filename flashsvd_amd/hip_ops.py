@@ -817,7 +817,13 @@ def rope_tables(position_ids: torch.Tensor, inv_freq: torch.Tensor, dtype: torch
     return _OPS.rope_tables.default(position_ids, inv_freq, dtype)
 
 
-def _rope_tables_impl(position_ids, inv_freq, dtype):
+def rope_tables_mask(position_ids: torch.Tensor, inv_freq: torch.Tensor, dtype: torch.dtype, mask: torch.Tensor):
+    """:func:`rope_tables` and ``(mask != 0)`` as the uint8 padding mask of :func:`attn_prefill` (mask: contiguous int64), in one
+    launch.  Custom operator flashsvd_hip::rope_tables_mask."""
+    return _OPS.rope_tables_mask.default(position_ids, inv_freq, dtype, mask)
+
+
+def _rope_tables_impl(position_ids, inv_freq, dtype, mask=None):
     code = _ELEM_CODES.get(dtype)
     if code is None:
         raise ValueError(f"rotation tables are torch.bfloat16 or torch.float16, got {dtype}")
@@ -829,9 +835,17 @@ def _rope_tables_impl(position_ids, inv_freq, dtype):
     rows, half = position_ids.numel(), inv_freq.numel()
     cos = torch.empty(rows, half, dtype=dtype, device=position_ids.device)
     sin = torch.empty_like(cos)
-    _lib.check("fsvd_rope_tables", _lib.load().fsvd_rope_tables(position_ids.data_ptr(), inv_freq.data_ptr(), cos.data_ptr(), sin.data_ptr(), rows,
-                                                                half, code, _stream()))
-    return cos, sin
+    if mask is None:
+        _lib.check("fsvd_rope_tables", _lib.load().fsvd_rope_tables(position_ids.data_ptr(), inv_freq.data_ptr(), cos.data_ptr(), sin.data_ptr(), rows,
+                                                                    half, code, _stream()))
+        return cos, sin
+    _need(mask, "mask", dtype=torch.long)
+    if not mask.is_contiguous() or mask.device != position_ids.device:
+        raise ValueError(f"mask must be contiguous and on {position_ids.device}, got strides {mask.stride()} on {mask.device}")
+    pad = torch.empty(mask.shape, dtype=torch.uint8, device=mask.device)
+    _lib.check("fsvd_rope_tables_mask", _lib.load().fsvd_rope_tables_mask(position_ids.data_ptr(), inv_freq.data_ptr(), cos.data_ptr(), sin.data_ptr(), rows,
+                                                                          half, mask.data_ptr(), pad.data_ptr(), mask.numel(), code, _stream()))
+    return cos, sin, pad
 
 
 def attn_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, q_pos0: Optional[torch.Tensor] = None, causal: bool = True,

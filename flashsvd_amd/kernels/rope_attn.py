@@ -54,8 +54,9 @@ class FlashSVDRoPEAttention(nn.Module):
         assert self.bdh == head_dim, "Kernel currently expects BDH == dh."
         self.causal = True   # decoder-only
 
-    def _tables(self, B: int, M: int, dh: int, position_ids, device, dtype):
-        """Per-token cos/sin rows [rows, dh/2] and the row offset of each batch entry (None: they share the rows)."""
+    def _tables(self, B: int, M: int, dh: int, position_ids, device, dtype, mask=None):
+        """Per-token cos/sin rows [rows, dh/2], the row offset of each batch entry (None: they share the rows), and the bytes of a 2-D
+        ``mask`` where the launch of the tables makes them, else None."""
         if position_ids is None:
             position_ids = torch.arange(M, device=device, dtype=torch.long).unsqueeze(0)
         if position_ids.dim() == 1:
@@ -67,8 +68,12 @@ class FlashSVDRoPEAttention(nn.Module):
         inv = getattr(self.rotary_emb, "inv_freq", None)
         if torch.is_tensor(inv) and inv.dim() == 1 and inv.numel() == dh // 2 and inv.dtype == torch.float32 and inv.is_contiguous() \
                 and position_ids.dtype == torch.long and position_ids.is_contiguous() and inv.device == position_ids.device == device:
+            offs = None if position_ids.shape[0] == 1 else torch.arange(B, dtype=torch.int32, device=device) * M
+            if mask is not None and mask.dim() == 2 and mask.dtype == torch.long and mask.is_contiguous() and mask.device == device and mask.numel():
+                cos, sin, pad = hip_ops.rope_tables_mask(position_ids, inv, dtype, mask)
+                return cos, sin, offs, pad
             cos, sin = hip_ops.rope_tables(position_ids, inv, dtype)
-            return cos, sin, None if position_ids.shape[0] == 1 else torch.arange(B, dtype=torch.int32, device=device) * M
+            return cos, sin, offs, None
         if inv is not None:
             ang = position_ids.to(device=device, dtype=torch.float32)[..., None] * inv.to(device=device, dtype=torch.float32)
             cos, sin = torch.cos(ang).to(dtype), torch.sin(ang).to(dtype)          # [Bpos, M, dh/2]
@@ -84,7 +89,7 @@ class FlashSVDRoPEAttention(nn.Module):
         shared = cos.shape[0] == 1
         offs = None if shared else \
             torch.arange(B, dtype=torch.int32, device=device) * M
-        return cos.reshape(-1, dh // 2).contiguous(), sin.reshape(-1, dh // 2).contiguous(), offs
+        return cos.reshape(-1, dh // 2).contiguous(), sin.reshape(-1, dh // 2).contiguous(), offs, None
 
     @torch.no_grad()
     def forward(self, qkv_factors: QKVFactors, attention_mask: Optional[torch.Tensor], position_ids: torch.Tensor,
@@ -105,7 +110,7 @@ class FlashSVDRoPEAttention(nn.Module):
         if (f.bk is not None or f.bv is not None) and Hk != H:
             raise NotImplementedError("key/value biases indexed by query head need H == Hk")
         dev, dt = f.Pq.device, f.Pq.dtype
-        cos, sin, offs = self._tables(B, M, dh, position_ids, dev, dt)
+        cos, sin, offs, pad = self._tables(B, M, dh, position_ids, dev, dt, attention_mask)
 
         def coeff(P):   # [B,h,M,R] -> view [B,M,h,R] without copying (head stride may be 0)
             P = P if P.stride(-1) == 1 else P.contiguous()
@@ -117,8 +122,8 @@ class FlashSVDRoPEAttention(nn.Module):
         uq, uk, uv = _as_linear_layout(f.Vq), _as_linear_layout(f.Vk), _as_linear_layout(f.Vv)
         Pq, Pk, Pv = coeff(f.Pq), coeff(f.Pk), coeff(f.Pv)
         bq, bk, bv = bias(f.bq, H), bias(f.bk, Hk), bias(f.bv, Hk)
-        pad = add = None
-        if attention_mask is not None:
+        add = None
+        if attention_mask is not None and pad is None:
             if attention_mask.dim() == 2:
                 pad = (attention_mask != 0).contiguous().view(torch.uint8)
             elif attention_mask.dim() == 4:

@@ -10,7 +10,7 @@ tensors.  ``flashsvd_amd.hip_ops`` and the modules under ``flashsvd_amd.kernels`
   rmsnorm / .out                      fsvd_rmsnorm
   lowrank_mlp                         fsvd_mlp_block_run     norm + rank projection + SwiGLU pair + down projection
   lowrank_attn_prefill                fsvd_attn_block_prefill   the attention half of a prompt pass over the dense cache
-  rope_tables                         fsvd_rope_tables
+  rope_tables, rope_tables_mask       fsvd_rope_tables, fsvd_rope_tables_mask   the latter with the padding mask as bytes
   greedy_token_                       fsvd_greedy_token      argmax of every row + position increment
   set_token_rows_                     fsvd_set_token_rows    token and position of every row
   qkv_rope_append / .out              fsvd_qkv_rope_append   head expansion + RoPE + dense-cache append
@@ -135,7 +135,18 @@ def _rope_tables_fake(position_ids, inv_freq, dtype):
     return inv_freq.new_empty(shape, dtype=dtype), inv_freq.new_empty(shape, dtype=dtype)
 
 
+def _rope_tables_mask(position_ids, inv_freq, dtype, mask):
+    from . import hip_ops
+    return hip_ops._rope_tables_impl(position_ids, inv_freq, dtype, mask)
+
+
+def _rope_tables_mask_fake(position_ids, inv_freq, dtype, mask):
+    return (*_rope_tables_fake(position_ids, inv_freq, dtype), mask.new_empty(mask.shape, dtype=torch.uint8))
+
+
 _define("rope_tables(Tensor position_ids, Tensor inv_freq, ScalarType dtype) -> (Tensor, Tensor)", _rope_tables, _rope_tables_fake)
+_define("rope_tables_mask(Tensor position_ids, Tensor inv_freq, ScalarType dtype, Tensor mask) -> (Tensor, Tensor, Tensor)", _rope_tables_mask,
+        _rope_tables_mask_fake)
 
 
 # ------------------------------------------------------------------ greedy token of every row
@@ -312,5 +323,5 @@ _define("mlp_dual_split(Tensor PUp, Tensor PGate, Tensor GateU, Tensor UpU, Tens
         PUp.new_empty((PUp.shape[0], DownU.shape[1])))
 
 ops = getattr(torch.ops, NS)
-OP_NAMES = ("linear", "swiglu_linear", "rmsnorm", "greedy_token_", "set_token_rows_", "lowrank_mlp", "lowrank_attn_prefill", "rope_tables", "qkv_rope_append", "attn_decode_densekv", "attn_decode_rankkv", "rankkv_append", "rankkv_fill", "linear_rankkv_append",
+OP_NAMES = ("linear", "swiglu_linear", "rmsnorm", "greedy_token_", "set_token_rows_", "lowrank_mlp", "lowrank_attn_prefill", "rope_tables", "rope_tables_mask", "qkv_rope_append", "attn_decode_densekv", "attn_decode_rankkv", "rankkv_append", "rankkv_fill", "linear_rankkv_append",
             "lowrank_expand_heads", "rope_attn_prefill", "reconstruct_qkv_token", "xw_linear", "mlp_dual_split")

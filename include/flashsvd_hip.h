@@ -322,6 +322,9 @@ int fsvd_lowrank_expand_heads_multi(const fsvd_expand_desc* desc, int n, const v
 /* cos_out / sin_out [rows, half] = cos / sin of (float)positions[row] * inv_freq[i], rounded once to `dtype`. */
 int fsvd_rope_tables(const int64_t* positions, const float* inv_freq, void* cos_out, void* sin_out, int64_t rows, int half, int dtype,
                      void* stream);
+/* fsvd_rope_tables and, in the same launch, pad_out[i] = mask[i] != 0 for i < mask_count: the padding mask of fsvd_attn_prefill. */
+int fsvd_rope_tables_mask(const int64_t* positions, const float* inv_freq, void* cos_out, void* sin_out, int64_t rows, int half, const int64_t* mask,
+                          uint8_t* pad_out, int64_t mask_count, int dtype, void* stream);
 int fsvd_attn_prefill(const void* q, int64_t sq_b, int64_t sq_m, int64_t sq_h,
                       const void* k, const void* v, int64_t sk_b, int64_t sk_s, int64_t sk_h,
                       const int32_t* q_pos0, const uint8_t* pad_mask, int64_t spm_b,
