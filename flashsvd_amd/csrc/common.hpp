@@ -160,6 +160,24 @@ __device__ __forceinline__ float wave_max(float v) {
   return fmaxf(fmaxf(a, b), fmaxf(c, d));
 }
 
+// Weights that the next launch reads, asked for by one that leaves the memory idle: they then come out of the 256 MB in front of HBM.
+struct Ahead { const unsigned char* p = nullptr; uint32_t bytes = 0; };
+// Workgroup `part` of `parts` reads its share of them, whole 16-byte pieces inside the range, and keeps nothing.
+template <int THREADS>
+__device__ __forceinline__ void request_ahead(const Ahead& a, int part, int parts, int tid) {
+  constexpr int U = 8;                                 // loads of a thread in flight
+  const uintptr_t p = reinterpret_cast<uintptr_t>(a.p), first = (p + 15) & ~(uintptr_t)15, end = (p + a.bytes) & ~(uintptr_t)15;
+  const int n = end > first ? (int)((end - first) >> 4) : 0;
+  const u32x4_t* q = reinterpret_cast<const u32x4_t*>(first);
+  for (int i = part * THREADS * U + tid; i < n; i += parts * THREADS * U) {
+    u32x4_t v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = q[min(i + u * THREADS, n - 1)];
+#pragma unroll
+    for (int u = 0; u < U; ++u) asm volatile("" ::"v"(v[u]));
+  }
+}
+
 // Eight consecutive 16-bit elements at any element's address as one 16-byte load (the hardware takes unaligned ones).
 typedef uint32_t u32x4_any_t __attribute__((ext_vector_type(4), aligned(2)));
 // The same for a piece that may reach past the end of its row: `left` elements of the row from `p` on, zero past them

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "common.hpp"
 #include "decode_map.hpp"
 
 namespace fsvd {
@@ -274,7 +275,7 @@ int launch_qkv(const QkvArgs& a, int cfg, hipStream_t st);
 bool qkv_mfma_applies(const QkvArgs& a);                                    // mfma_gemv.hip: 3..32 tokens
 int launch_qkv_mfma(const QkvArgs& a, hipStream_t st);
 int launch_rmsnorm(const uint16_t* x, int64_t ldx, const uint16_t* w, float eps, uint16_t* y, int64_t ldy, int rows,
-                   int K, int dt, hipStream_t st);
+                   int K, int dt, hipStream_t st, const Ahead& ahead = Ahead{});
 int launch_attn_decode(const AttnDecodeArgs& a, hipStream_t st);
 int launch_kv_append(const KvAppendArgs& a, hipStream_t st);
 size_t attn_decode_ws_floats(int B, int H, int nsplit, int Dh);

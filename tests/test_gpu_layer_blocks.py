@@ -31,6 +31,20 @@ def test_mlp_block(B, K, R, D, N, dtype):
     assert torch.equal(ops._mlp_from_coefficients(both[1], both[0], gu, uu, dv, du, bias, 1), want)
 
 
+@pytest.mark.parametrize("B,K,R,D,pad,off", [(239, 512, 128, 256, 0, 0), (240, 512, 128, 256, 0, 1), (256, 512, 130, 256, 64, 3), (1536, 8, 8, 64, 0, 7), (1537, 512, 128, 256, 0, 0),
+                                             (320, 512, 128, 256, 72, 0), (256, 16384, 64, 64, 8, 5)])
+def test_weights_asked_for_by_the_norm(B, K, R, D, pad, off):
+    """The norm's launch reads the rank projection's weights at 240 to 1536 rows: row strides up to an eighth over the row, weights at any element's
+    address, ranges with no whole piece beside them."""
+    from flashsvd_amd import hip_ops as ops
+    x, nw = _rand(B, K, seed=1), 1 + _rand(K, std=0.1, seed=7)
+    gu_v = _rand(2 * R * (K + pad) + off, std=K ** -0.5, seed=2)[off:].view(2 * R, K + pad)[:, :K]
+    gu, uu, dv, du = (_rand(*s, std=s[1] ** -0.5, seed=3 + i) for i, s in enumerate(((D, R), (D, R), (R, D), (K, R))))
+    p = ops.linear(x, gu_v, norm_weight=nw)
+    want = ops.linear(ops.linear(ops.swiglu_linear(p, gu, uu, up_off=R), dv), du, residual=x)
+    assert torch.equal(ops.lowrank_mlp(x, gu_v, gu, uu, dv, du, norm_weight=nw, residual=x), want)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,T,start,H,Hk,R", [(1, 16, 0, 4, 4, 128), (2, 77, 131, 8, 2, 128), (1, 333, 7, 4, 4, 122), (1, 700, 0, 32, 32, 64), (3, 512, 5, 16, 4, 192)])
 def test_attention_block(B, T, start, H, Hk, R, dtype):
