@@ -92,9 +92,9 @@ size_t fsvd_linear_scratch_bytes(const void* x, int64_t ldx, const void* W, int6
   return linear_scratch_floats(a, kShareScratchBytes / sizeof(float)) * sizeof(float);
 }
 
-int fsvd_linear_scratch(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* bias, const void* norm_w, float eps,
-                        const void* res, int64_t ldres, void* y, int64_t ldy, int B, int N, int K, int cfg, int dtype,
-                        void* scratch, size_t scratch_bytes, void* stream) {
+static int linear_call(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* bias, const void* norm_w, float eps,
+                       const void* res, int64_t ldres, void* y, int64_t ldy, int B, int N, int K, int cfg, int dtype,
+                       void* scratch, size_t scratch_bytes, const AheadList* next, void* stream) {
   const char* fn = "fsvd_linear";
   FSVD_REQUIRE_PTR(x, fn); FSVD_REQUIRE_PTR(W, fn); FSVD_REQUIRE_PTR(y, fn);
   LinearArgs a{cu16(x), ldx, cu16(W), ldw, cu16(bias), cu16(norm_w), eps, cu16(res), ldres, u16(y), ldy, B, N, K, dtype};
@@ -103,8 +103,14 @@ int fsvd_linear_scratch(const void* x, int64_t ldx, const void* W, int64_t ldw, 
     a.scratch = static_cast<float*>(scratch);
     a.scratch_floats = std::min(scratch_bytes, kShareScratchBytes) / sizeof(float);
   }
+  a.next = next;
   const int rc = linear_args(a, fn);
   return rc != kOk ? rc : launch_linear(a, cfg, static_cast<hipStream_t>(stream));
+}
+int fsvd_linear_scratch(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* bias, const void* norm_w, float eps,
+                        const void* res, int64_t ldres, void* y, int64_t ldy, int B, int N, int K, int cfg, int dtype,
+                        void* scratch, size_t scratch_bytes, void* stream) {
+  return linear_call(x, ldx, W, ldw, bias, norm_w, eps, res, ldres, y, ldy, B, N, K, cfg, dtype, scratch, scratch_bytes, nullptr, stream);
 }
 
 int fsvd_linear_rankkv_append(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* norm_w, float eps, void* y, int64_t ldy,
@@ -653,8 +659,18 @@ int fsvd_attn_prefill(const void* q, int64_t sq_b, int64_t sq_m, int64_t sq_h, c
 
 // one projection of a block: contiguous rows in and out unless said otherwise
 static int block_linear(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* bias, const void* norm_w, float eps, const void* res,
-                        int64_t ldres, void* y, int64_t ldy, int B, int N, int K, int dtype, void* scratch, size_t scratch_bytes, void* stream) {
-  return fsvd_linear_scratch(x, ldx, W, ldw, bias, norm_w, eps, res, ldres, y, ldy, B, N, K, 0, dtype, scratch, scratch_bytes, stream);
+                        int64_t ldres, void* y, int64_t ldy, int B, int N, int K, int dtype, void* scratch, size_t scratch_bytes, const AheadList* next, void* stream) {
+  return linear_call(x, ldx, W, ldw, bias, norm_w, eps, res, ldres, y, ldy, B, N, K, 0, dtype, scratch, scratch_bytes, next, stream);
+}
+// Weights [N, K] as a range to ask for ahead of their use: rows that lie (nearly) one behind the other, below 1 GiB.
+static Ahead weights_ahead(const void* W, int64_t ldw, int64_t N, int64_t K) {
+  Ahead a;
+  const int64_t bytes = ((N - 1) * ldw + K) * 2;
+  if (N > 0 && K > 0 && ldw >= K && ldw <= K + K / 8 && bytes < (int64_t)1 << 30) {
+    a.p = static_cast<const unsigned char*>(W);
+    a.bytes = (uint32_t)bytes;
+  }
+  return a;
 }
 // What the RMSNorm in front of a rank projection asks for on its behalf: 240 to 1536 rows that fill their tiles of 64 but for a sixteenth, up to 32 MB
 // of weights whose rows lie (nearly) one behind the other.  The tiles there take 7 of 25 us longer with weights from HBM than out of the 256 MB in front
@@ -667,24 +683,19 @@ static int block_linear(const void* x, int64_t ldx, const void* W, int64_t ldw, 
 // what the projection gains (16 / 32 / 208 rows 47.5 -> 49.1, 57.9 -> 59.6, 89.4 -> 90.2); more rows (2048 319.5 -> 326.7); 40 MB (rank 2432, 512 / 1024 rows
 // 171.4 -> 166.4, 272 -> 277).
 static Ahead norm_ahead(const void* W, int64_t ldw, int64_t B, int64_t N, int64_t K) {
-  Ahead a;
-  const int64_t bytes = ((N - 1) * ldw + K) * 2;
-  if (B >= 240 && B <= 1536 && B * 16 >= (B + 63) / 64 * 64 * 15 && N > 0 && ldw >= K && ldw <= K + K / 8 && bytes <= (int64_t)32 << 20) {
-    a.p = static_cast<const unsigned char*>(W);
-    a.bytes = (uint32_t)bytes;
-  }
-  return a;
+  const Ahead a = weights_ahead(W, ldw, N, K);
+  return B >= 240 && B <= 1536 && B * 16 >= (B + 63) / 64 * 64 * 15 && a.bytes <= 32u << 20 ? a : Ahead{};
 }
 // the rank projection in front of a block: three rows and more are normalised once up front, fewer in the projection's own launch
 static int block_input(const void* x, int64_t ldx, const void* norm_w, float eps, void* xn, const void* W, int64_t ldw, void* p, int64_t ldp, int B,
-                       int N, int K, int dtype, void* scratch, size_t scratch_bytes, const char* fn, void* stream) {
+                       int N, int K, int dtype, void* scratch, size_t scratch_bytes, const AheadList* next, const char* fn, void* stream) {
   if (norm_w != nullptr && B >= 3) {
     FSVD_REQUIRE_PTR(xn, fn);
     const int rc = launch_rmsnorm(cu16(x), ldx, cu16(norm_w), eps, u16(xn), K, B, K, dtype, static_cast<hipStream_t>(stream), norm_ahead(W, ldw, B, N, K));
     if (rc != kOk) return rc;
     x = xn; ldx = K; norm_w = nullptr;
   }
-  return block_linear(x, ldx, W, ldw, nullptr, norm_w, eps, nullptr, 0, p, ldp, B, N, K, dtype, scratch, scratch_bytes, stream);
+  return block_linear(x, ldx, W, ldw, nullptr, norm_w, eps, nullptr, 0, p, ldp, B, N, K, dtype, scratch, scratch_bytes, next, stream);
 }
 
 int fsvd_mlp_block_run(const fsvd_mlp_block* d, void* stream) {
@@ -697,21 +708,25 @@ int fsvd_mlp_block_run(const fsvd_mlp_block* d, void* stream) {
     set_last_error("%s: inconsistent layout (ldp=%lld R=%d ldu=%lld mode=%d)", fn, (long long)b.ldp, b.R, (long long)b.ldu, b.mode);
     return kErrBadShape;
   }
+  const Ahead down_u = weights_ahead(b.down_u, b.ldd, b.N, b.Rd);
+  const AheadList pair{{weights_ahead(b.gate_u, b.ldu, b.D, b.R), weights_ahead(b.up_u, b.ldu, b.D, b.R), Ahead{}}};
+  const AheadList down{{weights_ahead(b.down_v, b.ldv, b.Rd, b.D), down_u, Ahead{}}}, last{{down_u, Ahead{}, Ahead{}}};
   int rc;
   if (b.x != nullptr) {
     FSVD_REQUIRE_PTR(b.gu_v, fn);
-    rc = block_input(b.x, b.ldx, b.norm_w, b.eps, b.xn, b.gu_v, b.ldgv, b.p, b.ldp, b.B, 2 * b.R, b.K, b.dtype, b.scratch, b.scratch_bytes, fn, stream);
+    rc = block_input(b.x, b.ldx, b.norm_w, b.eps, b.xn, b.gu_v, b.ldgv, b.p, b.ldp, b.B, 2 * b.R, b.K, b.dtype, b.scratch, b.scratch_bytes, &pair, fn, stream);
     if (rc != kOk) return rc;
   }
   // the two sets of coefficients may be tensors of their own: a signed distance in elements
   const int64_t bytes = b.up ? (int64_t)(reinterpret_cast<intptr_t>(b.up) - reinterpret_cast<intptr_t>(b.p)) : 2 * (int64_t)b.R;
   if (bytes & 1) { set_last_error("%s: coefficients at an odd address", fn); return kErrBadAlign; }
   SwigluArgs a{cu16(b.p), b.ldp, bytes / 2, cu16(b.gate_u), cu16(b.up_u), b.ldu, u16(b.h), b.D, b.B, b.D, b.R, b.mode, b.dtype};
+  a.next = &down;
   rc = launch_swiglu(a, 0, static_cast<hipStream_t>(stream));
   if (rc != kOk) return rc;
-  rc = block_linear(b.h, b.D, b.down_v, b.ldv, nullptr, nullptr, 0.f, nullptr, 0, b.s, b.Rd, b.B, b.Rd, b.D, b.dtype, b.scratch, b.scratch_bytes, stream);
+  rc = block_linear(b.h, b.D, b.down_v, b.ldv, nullptr, nullptr, 0.f, nullptr, 0, b.s, b.Rd, b.B, b.Rd, b.D, b.dtype, b.scratch, b.scratch_bytes, &last, stream);
   if (rc != kOk) return rc;
-  return block_linear(b.s, b.Rd, b.down_u, b.ldd, b.bias, nullptr, 0.f, b.res, b.ldres, b.y, b.ldy, b.B, b.N, b.Rd, b.dtype, b.scratch, b.scratch_bytes, stream);
+  return block_linear(b.s, b.Rd, b.down_u, b.ldd, b.bias, nullptr, 0.f, b.res, b.ldres, b.y, b.ldy, b.B, b.N, b.Rd, b.dtype, b.scratch, b.scratch_bytes, nullptr, stream);
 }
 
 // (the normalised rows stand in for x: what counts is where they lie and how far apart)
@@ -753,12 +768,16 @@ int fsvd_attn_block_prefill(const fsvd_attn_block* d, void* stream) {
   }
   const int rows = (int)rows64, Rt = b.Rq + b.Rk + b.Rv, w = b.H * b.Dh;
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  int rc = block_input(b.x, b.ldx, b.norm_w, b.eps, b.xn, b.qkv_v, b.ldqkv, b.p, Rt, rows, Rt, b.K, b.dtype, b.scratch, b.scratch_bytes, fn, stream);
+  const AheadList heads{{weights_ahead(b.q_u, b.ldq, w, b.Rq), weights_ahead(b.k_u, b.ldk, (int64_t)b.Hk * b.Dh, b.Rk), weights_ahead(b.v_u, b.ldvu, (int64_t)b.Hk * b.Dh, b.Rv)}};
+  const Ahead o_u = weights_ahead(b.o_u, b.ldou, b.N, b.Ro);
+  const AheadList o{{weights_ahead(b.o_v, b.ldov, b.Ro, w), o_u, Ahead{}}}, last{{o_u, Ahead{}, Ahead{}}};
+  int rc = block_input(b.x, b.ldx, b.norm_w, b.eps, b.xn, b.qkv_v, b.ldqkv, b.p, Rt, rows, Rt, b.K, b.dtype, b.scratch, b.scratch_bytes, &heads, fn, stream);
   if (rc != kOk) return rc;
   const auto expansion = [&](int at, const void* u, int64_t ldu, int R, int heads, bool rotate, void* y, int64_t sy_b, int64_t sy_m, int64_t sy_h, int by_pos, int dst) {
     ExpandArgs e{cu16(b.p) + at, (int64_t)b.M * Rt, Rt, 0, cu16(u), ldu, nullptr, rotate ? cu16(b.cos) : nullptr, rotate ? cu16(b.sin) : nullptr, b.rope_len,
                  nullptr, u16(y), sy_b, sy_m, sy_h, by_pos, dst, b.B, b.M, heads, b.Dh, R, b.dtype};
     e.pos0 = b.start;
+    e.next = &o;
     return e;
   };
   const ExpandArgs e[3] = {expansion(0, b.q_u, b.ldq, b.Rq, b.H, true, b.q, (int64_t)b.M * w, w, b.Dh, 0, b.M),
@@ -778,9 +797,9 @@ int fsvd_attn_block_prefill(const fsvd_attn_block* d, void* stream) {
   t.pos0 = b.start;
   rc = launch_prefill_attn(t, st);
   if (rc != kOk) return rc;
-  rc = block_linear(b.a, w, b.o_v, b.ldov, b.o_v_bias, nullptr, 0.f, nullptr, 0, b.po, b.Ro, rows, b.Ro, w, b.dtype, b.scratch, b.scratch_bytes, stream);
+  rc = block_linear(b.a, w, b.o_v, b.ldov, b.o_v_bias, nullptr, 0.f, nullptr, 0, b.po, b.Ro, rows, b.Ro, w, b.dtype, b.scratch, b.scratch_bytes, &last, stream);
   if (rc != kOk) return rc;
-  return block_linear(b.po, b.Ro, b.o_u, b.ldou, b.o_u_bias, nullptr, 0.f, b.res, b.ldres, b.y, b.ldy, rows, b.N, b.Ro, b.dtype, b.scratch, b.scratch_bytes, stream);
+  return block_linear(b.po, b.Ro, b.o_u, b.ldou, b.o_u_bias, nullptr, 0.f, b.res, b.ldres, b.y, b.ldy, rows, b.N, b.Ro, b.dtype, b.scratch, b.scratch_bytes, nullptr, stream);
 }
 
 int fsvd_decode_step_workgroups(void) { return decode_step_workgroups(); }

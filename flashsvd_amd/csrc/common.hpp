@@ -162,6 +162,7 @@ __device__ __forceinline__ float wave_max(float v) {
 
 // Weights that the next launch reads, asked for by one that leaves the memory idle: they then come out of the 256 MB in front of HBM.
 struct Ahead { const unsigned char* p = nullptr; uint32_t bytes = 0; };
+struct AheadList { Ahead r[3]; };                      // in the order of their use
 // Workgroup `part` of `parts` reads its share of them, whole 16-byte pieces inside the range, and keeps nothing.
 template <int THREADS>
 __device__ __forceinline__ void request_ahead(const Ahead& a, int part, int parts, int tid) {

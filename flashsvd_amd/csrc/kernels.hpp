@@ -25,6 +25,7 @@ struct LinearArgs {
   int64_t app_sb[2] = {0, 0}, app_ss[2] = {0, 0};
   int app_n0[2] = {0, 0}, app_n[2] = {0, 0};
   int app_S = 0;
+  const AheadList* next = nullptr;       // weights of the launches behind this one, for compute units that it leaves idle
   float* scratch = nullptr; size_t scratch_floats = 0;   // this call's own, for the K shares of long prompt rows (fsvd_linear_scratch)
 };
 
@@ -35,6 +36,7 @@ struct SwigluArgs {
   int B, D, R;
   int mode;                              // 0 chain-of-linears rounding, 1 fused-kernel rounding
   int dt = 0;
+  const AheadList* next = nullptr;       // as in LinearArgs
 };
 
 struct QkvArgs {
@@ -150,6 +152,7 @@ struct ExpandArgs {
   int B, M, heads, Dh, R;
   int dt = 0;
   int pos0 = 0;                                     // position of token 0 of every row where positions is null
+  const AheadList* next = nullptr;                  // as in LinearArgs
 };
 struct PrefillAttnArgs {
   const uint16_t* q; int64_t sq_b, sq_m, sq_h;      // [B,M,H,Dh], rotated
@@ -185,6 +188,7 @@ struct MfmaArgs {
   int ksplit; float* ws_part; int32_t* ws_count;
   int dt = 0;
   float* scratch = nullptr; size_t scratch_floats = 0;   // this call's own (K shares of mfma_quad.hip)
+  const AheadList* next = nullptr;           // host only, as in LinearArgs
 };
 // epilogue of a head expansion (mfma_gemm.hip, mfma_mid.hip)
 struct ExpandEpi {

@@ -866,6 +866,7 @@ static MfmaArgs mfma_args(const LinearArgs& a) {
   m.dt = a.dt;
   m.scratch = a.scratch;
   m.scratch_floats = a.scratch_floats;
+  m.next = a.next;
   return m;
 }
 size_t linear_scratch_floats(const LinearArgs& a, size_t cap) {
@@ -880,6 +881,7 @@ bool mfma_swiglu_applies(const SwigluArgs& a) { return a.B >= 3; }
 int launch_swiglu_mfma(const SwigluArgs& a, hipStream_t st) {
   MfmaArgs m{a.p, a.ldp, a.up_off, a.gate_u, a.up_u, a.ldw, nullptr, nullptr, 0, a.h, a.ldh, a.B, a.D, a.R, a.mode};
   m.dt = a.dt;
+  m.next = a.next;
   return a.dt == 1 ? launch_mfma<1, true>(m, st, "fsvd_swiglu_linear") : launch_mfma<0, true>(m, st, "fsvd_swiglu_linear");
 }
 

@@ -339,11 +339,15 @@ static int launch_gemm_quad_dt(const MfmaArgs& a, bool dual, hipStream_t st, con
       q.shares = f.shares;
       q.per = f.per;
       q.part = a.scratch;
+      const QuadCost& c = f.bn == 64 ? kPlainCosts[12] : (f.bm == 64 ? kPlainCosts[9] : (f.bm == 128 ? kPlainCosts[6] : kCost256x128Shares));
+      q.us = c.f2 + c.s2 * (float)f.per;
       return launch_share_dt<DT>(q, f, st, who);
     }
   }
   const QuadSums sums = dual || any ? QuadSums{kOrderPlain, 0} : quad_sums(a);
-  const int form = quad_pick(a, dual, any, sums.order).form;
+  const QuadPick pick = quad_pick(a, dual, any, sums.order);
+  const int form = pick.form;
+  q.us = pick.us;
 #define FSVD_QUAD_CASE(EPI, RAG, n, TM, TN, SX, SW, OCC) case n: return launch_quad_t<DT, EPI, TM, TN, SX, SW, OCC, RAG>(q, st, who);
   if (dual && any) {
     switch (form) {

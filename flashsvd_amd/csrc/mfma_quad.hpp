@@ -40,6 +40,8 @@ struct QuadArgs {
   ExpandEpi ep[3];
   int first[4];                                      // heads: column tiles of problem i are [first[i], first[i + 1])
   int nt, mt;                                        // column and row tiles
+  float us;                                          // what the launch is expected to take
+  AheadList next;                                    // what workgroups without a tile ask for
   int shares, per; float* part;                      // kQuadShare: workgroups per tile, K steps of each (the last may have fewer), their sums; CUT: per
 };
 
@@ -64,6 +66,32 @@ static float quad_us(const QuadCost& c, int64_t tiles, int occ, float steps, int
   float us = (float)full * (c.f2 + c.s2 * steps);
   if (rest > 0) us += occ == 2 && rest <= cu ? c.f1 + c.s1 * steps : c.f2 + c.s2 * steps;
   return us;
+}
+
+// Workgroups for the compute units that a launch of `wgs` with `rows` rows in its row tiles leaves idle, and what they ask for: the ranges of
+// q.a[0].next, in their order, that they get through at 46 bytes per ns and compute unit while the launch is expected to last, padded row tiles
+// counted out (128 x 192 tiles over 400 rows end early: with down_v asked for all the same the MLP at rank 2432 went from 146 to 152 us).  A range in part gains
+// nothing, its launch takes as long as its slowest workgroups (ranges cut off at 15, 25, 40 bytes per ns: a prompt of 512 tokens 7027 -> 7014, 7010, 6880 us).
+// A compute unit reads about 60 from HBM; more than 46 outlasts some launches (54: rank 1024, 384 rows 83.7 -> 88.4, rank 2432, 512 rows 171 -> 177).
+// What it gives, us without -> with, weights from HBM: the pair 512 x 11008 x 1536 leaves 24 compute units to down_v, whose launches then take 26 instead of 36.  MLPs of 4096
+// x 11008 at rank 1536, 64 / 128 / 154 / 256 / 333 / 400 / 512 / 640 / 768 rows 80.8 -> 77.8, 75.8 -> 73.1, 79.0 -> 78.8, 94.2 -> 90.4, 106.7 -> 104.8, 110.4 -> 110.7, 124.5 -> 117.3, 139.3
+// -> 131.2, 162.8 -> 161.0, at rank 1492 384 / 768 rows 131.6 -> 125.5, 210.7 -> 191.1, 2048 x 5504 at rank 1024 192 / 300 / 400 / 700 rows 54.5 -> 48.1, 57.1 -> 52.5, 64.5 -> 64.4, 78.4
+// -> 72.1; over 100 of these (64 to 768 rows, rank 1024 to 2432) 0.977 of the time.  More tiles than compute units: nobody is idle, nothing is asked for.
+// The tiles of many rows are left out.
+constexpr float kAheadRate = 46.f;
+constexpr bool quad_asks(int tm, int tn) { return tm * tn < 32; }
+static int quad_ahead(QuadArgs& q, int64_t wgs, int64_t rows) {
+  q.next = AheadList{};
+  const int64_t idle = compute_units() - wgs;
+  if (q.a[0].next == nullptr || idle <= 0) return 0;
+  const int64_t room = (int64_t)(q.us * kAheadRate * 1000.f * (float)q.a[0].B / (float)rows) * idle;
+  int64_t sum = 0;
+  for (int i = 0; i < 3; ++i) {
+    if (sum + q.a[0].next->r[i].bytes > room) break;
+    q.next.r[i] = q.a[0].next->r[i];
+    sum += q.next.r[i].bytes;
+  }
+  return (int)std::min<int64_t>(idle, (sum + 32767) / 32768);
 }
 
 constexpr bool quad_stream(int tm, int tn) { return tm * tn >= 24; }
@@ -112,7 +140,13 @@ __global__ __launch_bounds__(kQuadThreads, OCC) void gemm_quad_kernel(QuadArgs a
     return w;
   };
   int ti = blockIdx.x >> 3;
-  if (ti >= run_n) return;
+  if (ti >= run_n) {
+    if constexpr (quad_asks(TM, TN)) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) request_ahead<kQuadThreads>(args.next.r[i], blockIdx.x - all, gridDim.x - all, tid);
+    }
+    return;
+  }
 
   // ---- load cursors.  Eight threads per row, rows tid / 8 + 32 j of each operand: a lane's byte offset holds its row and piece, the
   // base address the K step.  Offsets fit 32 bits (the launcher checks), rows past the end are clamped to the last one.
@@ -646,7 +680,8 @@ static int launch_quad_t(QuadArgs& q, hipStream_t st, const char* who) {
                                              EPI == kQuadHeads ? " heads" : (EPI == kQuadPair ? (kAlone ? " pair alone" : " pair") :
                                              (H == 2 ? " halves" : (CUT ? " ranges" : (kAlone ? " alone" : "")))));
   set_last_form(form.s);
-  hipLaunchKernelGGL((gemm_quad_kernel<DT, EPI, TM, TN, NSX, NSW, OCC, RAG, H, CUT>), dim3((unsigned)grid), dim3(kQuadThreads), lds, st, q);
+  const int parts = quad_asks(TM, TN) ? quad_ahead(q, all, (int64_t)q.mt * BM) : 0;
+  hipLaunchKernelGGL((gemm_quad_kernel<DT, EPI, TM, TN, NSX, NSW, OCC, RAG, H, CUT>), dim3((unsigned)(grid + parts)), dim3(kQuadThreads), lds, st, q);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_last_error("%s: launch failed: %s", who, hipGetErrorString(e)); return kErrLaunch; }
   return kOk;

@@ -13,7 +13,7 @@ namespace fsvd {
   X(6, 2, 2, 5, 5, 2, 2.39f, 0.196f, 3.13f, 0.394f)
 #define FSVD_QUAD_HEADS_ANY(X) X(3, 4, 4, 2, 3, 2) X(4, 3, 4, 2, 3, 2) X(6, 2, 2, 4, 4, 2)
 
-static int heads_pick(const ExpandArgs* d, int n, bool any) {
+static int heads_pick(const ExpandArgs* d, int n, bool any, float& us_out) {
   const int64_t rows = (int64_t)d[0].B * d[0].M, cu = compute_units();
   int best = -1;
   float best_us = 0.f, steps = 0.f;
@@ -28,6 +28,7 @@ static int heads_pick(const ExpandArgs* d, int n, bool any) {
 #define X(n_, TM, TN, SX, SW, OCC, F1, S1, F2, S2) if (!any || n_ == 3 || n_ == 4 || n_ == 6) take(n_, TM, TN, OCC, QuadCost{F1, S1, F2, S2});
   FSVD_QUAD_HEADS(X)
 #undef X
+  us_out = best_us;
   return best;
 }
 static bool heads_on_grid(const ExpandArgs& a) { return a.R % 64 == 0 && a.sp_b % 8 == 0 && a.sp_m % 8 == 0 && a.ldu % 8 == 0 && aligned16(a.p) && aligned16(a.u); }
@@ -64,7 +65,8 @@ static int launch_expand_quad_dt(const ExpandArgs* d, int n, hipStream_t st) {
     }
     q.nt = tiles;
   };
-  const int form = heads_pick(d, n, any);
+  q.a[0].next = d[0].next;
+  const int form = heads_pick(d, n, any, q.us);
   if (any) {
     switch (form) {
 #define X(n_, TM, TN, SX, SW, OCC) case n_: tile(32 * TN); return launch_quad_t<DT, kQuadHeads, TM, TN, SX, SW, OCC, true>(q, st, who);

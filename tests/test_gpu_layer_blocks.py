@@ -32,17 +32,22 @@ def test_mlp_block(B, K, R, D, N, dtype):
 
 
 @pytest.mark.parametrize("B,K,R,D,pad,off", [(239, 512, 128, 256, 0, 0), (240, 512, 128, 256, 0, 1), (256, 512, 130, 256, 64, 3), (1536, 8, 8, 64, 0, 7), (1537, 512, 128, 256, 0, 0),
-                                             (320, 512, 128, 256, 72, 0), (256, 16384, 64, 64, 8, 5)])
-def test_weights_asked_for_by_the_norm(B, K, R, D, pad, off):
-    """The norm's launch reads the rank projection's weights at 240 to 1536 rows: row strides up to an eighth over the row, weights at any element's
-    address, ranges with no whole piece beside them."""
+                                             (320, 512, 128, 256, 72, 0), (256, 16384, 64, 64, 8, 5), (64, 512, 384, 4096, 0, 0), (160, 1024, 384, 2816, 8, 8),
+                                             (512, 1024, 330, 2818, 2, 2), (512, 512, 320, 5504, 64, 0), (130, 512, 321, 1411, 0, 1)])
+def test_weights_asked_for_ahead(B, K, R, D, pad, off):
+    """The norm's launch and the compute units that a projection leaves idle read the weights of the launches behind them: row strides up to
+    an eighth over the row and more, weights at any element's address, ranges with no whole piece beside them, all compute units taken."""
     from flashsvd_amd import hip_ops as ops
+
+    def weight(n, k, seed):
+        return _rand(n * (k + pad) + off, std=k ** -0.5, seed=seed)[off:].view(n, k + pad)[:, :k]
+
     x, nw = _rand(B, K, seed=1), 1 + _rand(K, std=0.1, seed=7)
-    gu_v = _rand(2 * R * (K + pad) + off, std=K ** -0.5, seed=2)[off:].view(2 * R, K + pad)[:, :K]
-    gu, uu, dv, du = (_rand(*s, std=s[1] ** -0.5, seed=3 + i) for i, s in enumerate(((D, R), (D, R), (R, D), (K, R))))
+    gu_v, gu, uu, dv, du = weight(2 * R, K, 2), weight(D, R, 3), weight(D, R, 4), weight(R, D, 5), weight(K, R, 6)
     p = ops.linear(x, gu_v, norm_weight=nw)
     want = ops.linear(ops.linear(ops.swiglu_linear(p, gu, uu, up_off=R), dv), du, residual=x)
-    assert torch.equal(ops.lowrank_mlp(x, gu_v, gu, uu, dv, du, norm_weight=nw, residual=x), want)
+    for _ in range(2):
+        assert torch.equal(ops.lowrank_mlp(x, gu_v, gu, uu, dv, du, norm_weight=nw, residual=x), want)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
