@@ -6,8 +6,6 @@
 // form and p*V accumulates per lane.  The workgroup writes an un-normalised partial (acc, m, l)
 // with write-through stores; the last workgroup to arrive for a (b,h) merges the partials in
 // split order, so the result does not depend on arrival order.
-#include <type_traits>
-
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -152,27 +150,33 @@ __global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(1,
   float acc[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) acc[i] = 0.f;
+  const bool few = HALVES && k1 - k0 <= CH / 2;
   int it = 0;
-  const auto pass = [&](auto rows, int c0) {
-    constexpr int R = decltype(rows)::value;
+  for (int c0 = k0; c0 < k1; c0 += CH, ++it) {
     // all K and V rows of this pass are requested before anything is consumed
-    u32x4_t kv[R], vv[R];
+    u32x4_t kv[U], vv[U];
+    if constexpr (HALVES) {
 #pragma unroll
-    for (int u = 0; u < R; ++u) {
+      for (int u = U / 2; u < U; ++u) kv[u] = vv[u] = u32x4_t{0u, 0u, 0u, 0u};
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (few && u >= U / 2) break;
       const int key = min(c0 + u * KPB + slot, k1 - 1);
       kv[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(kbase + (int64_t)key * a.sc_s));
     }
 #pragma unroll
-    for (int u = 0; u < R; ++u) {
+    for (int u = 0; u < U; ++u) {
+      if (few && u >= U / 2) break;
       const int key = min(c0 + u * KPB + slot, k1 - 1);
       vv[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(vbase + (int64_t)key * a.sc_s));
     }
     if (it == 0) __syncthreads();  // qs ready
     const u32x4_t qv = *reinterpret_cast<const u32x4_t*>(qs + part * 8);
-    float sc[R];
+    float sc[U];
     float lmax = -INFINITY;
 #pragma unroll
-    for (int u = 0; u < R; ++u) {
+    for (int u = 0; u < U; ++u) {
       float d = E::dot8(kv[u], qv, 0.f);
       d += dpp_f32<0xB1>(d);
       d += dpp_f32<0x4E>(d);
@@ -192,7 +196,7 @@ __global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(1,
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[i] *= alpha;
 #pragma unroll
-    for (int u = 0; u < R; ++u) {
+    for (int u = 0; u < U; ++u) {
       const float p = (sc[u] == -INFINITY) ? 0.f : __expf(sc[u] - m_new);
       psum += p;
       acc[0] += p * E::lo(vv[u].x); acc[1] += p * E::hi(vv[u].x);
@@ -202,13 +206,6 @@ __global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(1,
     }
     l_thr = l_thr * alpha + (part == 0 ? psum : 0.f);
     m_run = m_new;
-  };
-  typedef std::integral_constant<int, U> all_t;
-  typedef std::integral_constant<int, (U + 1) / 2> half_t;
-  if (HALVES && k1 - k0 <= CH / 2) {
-    if (k0 < k1) { pass(half_t{}, k0); ++it; }
-  } else {
-    for (int c0 = k0; c0 < k1; c0 += CH, ++it) pass(all_t{}, c0);
   }
   if (it == 0) __syncthreads();
   // fold the key slots and the per-thread sums
@@ -512,7 +509,7 @@ static void launch_attn_decode_t(const AttnDecodeArgs& a, int G, hipStream_t st)
   else if (G == 2) hipLaunchKernelGGL((attn_decode_gqa_kernel<DT, 128, 8, 2>), grid, dim3(kAttnThreads), 0, st, a);
   else if (a.Dh == 128) hipLaunchKernelGGL((attn_decode_kernel<DT, 128, 8>), grid, dim3(kAttnThreads), 0, st, a);
   // one range of 129 to 256 rows of 64: 256 keys in flight instead of two passes of 128, or two workgroups that meet again in a merge.  us in two ranges of one
-  // pass / one range of two passes / this, 137 and 250 keys: 8 heads 5.6, 4.7, 4.3 and 5.7, 5.1, 4.8; 4 x 32 heads 6.2, 5.4, 4.8 and 6.6, 5.8, 5.5; 32 x 16 8.2, 8.0, 7.2 and 10.1, 10.1, 10.0
+  // pass / one range of two passes / this, 137 and 250 keys: 8 heads 5.6, 4.7, 4.4 and 5.7, 5.1, 5.2; 4 x 32 heads 6.2, 5.4, 5.1 and 6.6, 5.8, 5.8; 32 x 16 8.2, 8.0, 7.4 and 10.1, 10.1, 10.2
   else if (a.nsplit == 1 && a.S > 128 && a.S <= 256) hipLaunchKernelGGL((attn_decode_kernel<DT, 64, 8, true>), grid, dim3(kAttnThreads), 0, st, a);
   else hipLaunchKernelGGL((attn_decode_kernel<DT, 64, 4>), grid, dim3(kAttnThreads), 0, st, a);
 }

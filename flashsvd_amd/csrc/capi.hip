@@ -708,7 +708,8 @@ int fsvd_mlp_block_run(const fsvd_mlp_block* d, void* stream) {
     set_last_error("%s: inconsistent layout (ldp=%lld R=%d ldu=%lld mode=%d)", fn, (long long)b.ldp, b.R, (long long)b.ldu, b.mode);
     return kErrBadShape;
   }
-  const Ahead down_u = weights_ahead(b.down_u, b.ldd, b.N, b.Rd);
+  // (nothing is asked for on behalf of a projection that will be refused)
+  const Ahead down_u = b.ldy >= b.N && (b.res == nullptr || b.ldres >= b.N) ? weights_ahead(b.down_u, b.ldd, b.N, b.Rd) : Ahead{};
   const AheadList pair{{weights_ahead(b.gate_u, b.ldu, b.D, b.R), weights_ahead(b.up_u, b.ldu, b.D, b.R), Ahead{}}};
   const AheadList down{{weights_ahead(b.down_v, b.ldv, b.Rd, b.D), down_u, Ahead{}}}, last{{down_u, Ahead{}, Ahead{}}};
   int rc;
@@ -769,7 +770,8 @@ int fsvd_attn_block_prefill(const fsvd_attn_block* d, void* stream) {
   const int rows = (int)rows64, Rt = b.Rq + b.Rk + b.Rv, w = b.H * b.Dh;
   const hipStream_t st = static_cast<hipStream_t>(stream);
   const AheadList heads{{weights_ahead(b.q_u, b.ldq, w, b.Rq), weights_ahead(b.k_u, b.ldk, (int64_t)b.Hk * b.Dh, b.Rk), weights_ahead(b.v_u, b.ldvu, (int64_t)b.Hk * b.Dh, b.Rv)}};
-  const Ahead o_u = weights_ahead(b.o_u, b.ldou, b.N, b.Ro);
+  // (nothing is asked for on behalf of a projection that will be refused)
+  const Ahead o_u = b.ldy >= b.N && (b.res == nullptr || b.ldres >= b.N) ? weights_ahead(b.o_u, b.ldou, b.N, b.Ro) : Ahead{};
   const AheadList o{{weights_ahead(b.o_v, b.ldov, b.Ro, w), o_u, Ahead{}}}, last{{o_u, Ahead{}, Ahead{}}};
   int rc = block_input(b.x, b.ldx, b.norm_w, b.eps, b.xn, b.qkv_v, b.ldqkv, b.p, Rt, rows, Rt, b.K, b.dtype, b.scratch, b.scratch_bytes, &heads, fn, stream);
   if (rc != kOk) return rc;

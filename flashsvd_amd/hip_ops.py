@@ -395,7 +395,7 @@ def _qkv_rope_append_impl(p, q_u, k_u, v_u, cos, sin, positions, k_cache, v_cach
 def pick_nsplit(max_len: int, batch: int, heads: int, head_dim: int = 128) -> int:
     """Key-axis split: about 128 keys per workgroup (one pass of loads in flight), bounded so that
     batch*heads*nsplit stays within ~2048 workgroups.  Up to 256 rows in one range, which saves the merge, with head_dim 64 (8 heads,
-    137 keys 5.6 -> 4.3 us) and for 256 pairs and more (16 x 32 heads over 8 of 128 9.4 -> 8.0; fewer lose: 32 heads, 250 keys 6.4 -> 6.7)."""
+    137 keys 5.6 -> 4.4 us) and for 256 pairs and more (16 x 32 heads over 8 of 128 9.4 -> 8.0; fewer lose: 32 heads, 250 keys 6.4 -> 6.7)."""
     if max_len <= 256 and (head_dim < 128 or batch * heads >= 256):
         return 1
     n = max(1, math.ceil(max_len / 128))
