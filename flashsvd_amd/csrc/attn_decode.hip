@@ -92,7 +92,7 @@ __device__ __forceinline__ void append_pair(const Args& a, int half, int b, int 
 }
 
 // The new row of a sequence is its last key: the workgroup whose keys [k0, k1) end with it writes it before it reads them.
-// Only where no other workgroup reads the row (append_in_kernel).  Against a launch of its own for the append: 16 sequences of
+// Only where no other workgroup reads the row (launch_attn_decode).  Against a launch of its own for the append: 16 sequences of
 // up to 4001 keys, 32 heads over 8, 53.5 -> 50.1 us, 64 x 1000 49.8 -> 48.0, 16 x 1000 with 32 kv heads 49.6 -> 46.9.
 template <int DT, int DH>
 __device__ __forceinline__ void append_own_row(const AttnDecodeArgs& a, int b, int hk, int pos, int k0, int k1) {
@@ -514,11 +514,11 @@ static void launch_attn_decode_t(const AttnDecodeArgs& a, int G, hipStream_t st)
   else hipLaunchKernelGGL((attn_decode_kernel<DT, 64, 4>), grid, dim3(kAttnThreads), 0, st, a);
 }
 
-// true when the appended row of (b, hk) is read by one workgroup alone: all query heads of the kv head in one workgroup, and
-// cache rows of different sequences and heads that do not overlap (sequences bound to one cache row see each other's new
-// tokens, which takes a launch before this one)
-static bool append_in_kernel(const AttnDecodeArgs& a, int G) {
-  return a.H / a.Hk == G && a.sc_h >= a.Dh && a.sc_s >= (a.Hk - 1) * a.sc_h + a.Dh && (a.B == 1 || a.sc_b >= a.S * a.sc_s);
+// true when the appended row of (b, hk) may be written by the launch that reads it, where one workgroup takes all query heads of the kv head: cache
+// rows of different sequences and heads that do not overlap (sequences bound to one cache row see each other's new tokens, which takes a
+// launch before this one)
+static bool rows_apart(const AttnDecodeArgs& a) {
+  return a.sc_h >= a.Dh && a.sc_s >= (a.Hk - 1) * a.sc_h + a.Dh && (a.B == 1 || a.sc_b >= a.S * a.sc_s);
 }
 
 int launch_attn_decode(const AttnDecodeArgs& args, hipStream_t st) {
@@ -541,16 +541,10 @@ int launch_attn_decode(const AttnDecodeArgs& args, hipStream_t st) {
     return kErrBadAlign;
   }
   if (a.nsplit > 1 && (!a.ws_part || !a.ws_count)) { set_last_error("fsvd_attn_decode_densekv: workspace missing"); return kErrWorkspace; }
-  // grouped-query caches with enough work to fill the chip four (two) query heads at a time: the kv rows are read once
-  // per group of query heads
-  const int rep = a.H / a.Hk;
-  int G = 1;
-  if (rep % 4 == 0 && (int64_t)a.B * (a.H / 4) * a.nsplit >= 512) G = 4;
-  else if (a.Dh == 128) {
-    if (rep % 2 == 0 && (int64_t)a.B * (a.H / 2) * a.nsplit >= 512) G = 2;
-  }
+  const bool own = a.k_new != nullptr && rows_apart(a);
+  const int G = decode_group(a.Dh, a.B, a.H, a.Hk, a.S, a.nsplit, own);
   a.plan = decode_plan(a.Dh, G, a.B, a.H, a.Hk, a.nsplit);
-  if (a.k_new && !append_in_kernel(a, G)) {
+  if (a.k_new && !(own && a.H / a.Hk == G)) {
     const KvAppendArgs ka{a.k_new, a.v_new, a.sk_b, a.sk_h, a.sv_b, a.sv_h, const_cast<uint16_t*>(a.k_cache), const_cast<uint16_t*>(a.v_cache),
                           a.sc_b, a.sc_s, a.sc_h, a.seqlens, a.cos, a.sin, a.rope_len, a.B, a.Hk, a.Dh, a.S, a.dt};
     const int rc = launch_kv_append(ka, st);

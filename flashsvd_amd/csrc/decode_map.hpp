@@ -56,6 +56,27 @@ constexpr DecodePlan decode_plan(int head_dim, int group, int B, int H, int Hk, 
   return p;
 }
 
+// Query heads of a kv head that one workgroup takes: four (head_dim 128: four or two) where the workgroups then still are two per compute unit; groups read
+// the rows once and, where they are all heads of the kv head, append the new one themselves.  A cache of 129 to 256 rows and up to 1024 (sequence, head) pairs that
+// runs as one range counts as the two that there would be room for, with head_dim 64 and where the call appends (`appends`) and the group keeps that in the launch.
+// us at 137 / 248 keys, two ranges with the group, one range without, this; with an append 32 x 32 heads over 8 of 64 10.0, 10.8, 8.6 / 11.4, 13.1, 8.8, of 128
+// 13.5, 13.2, 12.4 / 15.5, 14.4, 13.0, 16 x 32 over 16 of 128 10.3, 11.9, 9.3 / 12.2, 13.8, 9.8, none appended 32 x 32 over 8 of 64 9.2, 8.3, 7.8 / 11.1, 10.4, 8.0.
+// Elsewhere smaller groups fill the chip better with one range: of 128 and none appended 32 x 32 over 8 12.9, 11.1, 11.5 / 14.9, 11.7, 12.2, 24 x 32 over 16 12.5, 11.3,
+// 12.1 / 15.3, 14.4, 13.5; 40 x 32 over 8 of 128, which has one range in any case, 13.9 in twos, 16.2 in fours.
+constexpr int decode_group_of(int head_dim, long pairs, int rep, int ranges) {
+  if (rep % 4 == 0 && pairs / 4 * ranges >= 512) return 4;
+  return head_dim == 128 && rep % 2 == 0 && pairs / 2 * ranges >= 512 ? 2 : 1;
+}
+constexpr int decode_group(int head_dim, int B, int H, int Hk, int S, int nsplit, bool appends) {
+  const int rep = H / Hk;
+  const long pairs = (long)B * H;
+  if (nsplit == 1 && S > 128 && S <= 256 && pairs <= 1024) {
+    const int two = decode_group_of(head_dim, pairs, rep, 2);
+    if (head_dim == 64 || (appends && two == rep)) return two;
+  }
+  return decode_group_of(head_dim, pairs, rep, nsplit);
+}
+
 // Key ranges that a sequence of n keys is cut into, at most nsplit (what the scratch holds): known from the length alone, so
 // the same launch serves a cache that is nearly empty and one that is full; the other workgroups of (b, h) leave at once.
 // A range holds at least one pass of 128 keys: one sequence of 300 keys in a cache of 4096 rows 13.0 us in 32 ranges, 6.6 in three.

@@ -95,3 +95,23 @@ def test_assignment_of_many_pairs_is_a_constant_expression(tmp_path):
                            f"constexpr auto p{len(asserts)} = decode_plan(64, 1, {B}, {H}, {H}, {nsplit});\n"
                            f"static_assert(t{len(asserts)}.s == {s} && t{len(asserts)}.h == {pair % H} && t{len(asserts)}.seq == {pair // H});")
     _build(tmp_path, '#include "decode_map.hpp"\nusing namespace fsvd;\n' + "\n".join(asserts) + "\nint main() { return 0; }\n")
+
+
+def test_one_range_keeps_the_group(tmp_path):
+    """Calls over 129 to 256 rows that run as one range keep the query heads together that a workgroup of two ranges takes where these are all heads of a
+    kv head, whose new row the launch then appends itself, and with head_dim 64; the group of all other calls goes by their ranges."""
+    from flashsvd_amd.hip_ops import pick_nsplit
+    asserts = []
+    for dh in (64, 128):
+        for B in (1, 8, 9, 15, 16, 24, 31, 32, 40, 63, 64, 100):
+            for H, hk in ((8, 8), (8, 2), (16, 8), (32, 32), (32, 16), (32, 8), (32, 1), (64, 8), (28, 4), (40, 8)):
+                for S in (1, 128, 129, 200, 256, 257):
+                    def group(n, rep=H // hk):
+                        return 4 if rep % 4 == 0 and B * (H // 4) * n >= 512 else (2 if dh == 128 and rep % 2 == 0 and B * (H // 2) * n >= 512 else 1)
+                    ranges, n = max(1, min((S + 127) // 128, max(1, 2048 // (B * H)))), pick_nsplit(S, B, H, dh)
+                    for appends in (0, 1):
+                        keeps = dh == 64 or (appends and group(ranges) == H // hk)
+                        want = group(ranges) if keeps else group(n)
+                        asserts.append(f"static_assert(decode_group({dh}, {B}, {H}, {hk}, {S}, {n}, {appends}) == {want});")
+                        asserts.append(f"static_assert(decode_group({dh}, {B}, {H}, {hk}, {S}, {ranges}, {appends}) == {group(ranges)});")
+    _build(tmp_path, '#include "decode_map.hpp"\nusing namespace fsvd;\n' + "\n".join(asserts) + "\nint main() { return 0; }\n")
