@@ -104,7 +104,7 @@ __device__ __forceinline__ void append_own_row(const AttnDecodeArgs& a, int b, i
 }
 
 // (head_dim 64 would fit eight waves on a SIMD, all of up to 2048 workgroups at once: 16 x 4000 keys of 32 heads 111.8 us, with seven 105.5)
-// HALVES: caches that one pass covers and that are a single range (head_dim 64, 129 to 256 rows): at most half a pass of keys takes half the loads.
+// HALVES: caches that one pass covers and that are a single range (decode_one_pass): at most half a pass of keys takes half the loads.
 template <int DT, int DH, int U, bool HALVES = false>
 __global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(1, DH == 64 ? 7 : 8))) void attn_decode_kernel(AttnDecodeArgs a) {
   typedef E16<DT> E;
@@ -508,9 +508,7 @@ static void launch_attn_decode_t(const AttnDecodeArgs& a, int G, hipStream_t st)
   else if (G == 4) hipLaunchKernelGGL((attn_decode_gqa_kernel<DT, 128, 8, 4>), grid, dim3(kAttnThreads), 0, st, a);
   else if (G == 2) hipLaunchKernelGGL((attn_decode_gqa_kernel<DT, 128, 8, 2>), grid, dim3(kAttnThreads), 0, st, a);
   else if (a.Dh == 128) hipLaunchKernelGGL((attn_decode_kernel<DT, 128, 8>), grid, dim3(kAttnThreads), 0, st, a);
-  // one range of 129 to 256 rows of 64: 256 keys in flight instead of two passes of 128, or two workgroups that meet again in a merge.  us in two ranges of one
-  // pass / one range of two passes / this, 137 and 250 keys: 8 heads 5.6, 4.7, 4.4 and 5.7, 5.1, 5.2; 4 x 32 heads 6.2, 5.4, 5.1 and 6.6, 5.8, 5.8; 32 x 16 8.2, 8.0, 7.4 and 10.1, 10.1, 10.2
-  else if (a.nsplit == 1 && a.S > 128 && a.S <= 256) hipLaunchKernelGGL((attn_decode_kernel<DT, 64, 8, true>), grid, dim3(kAttnThreads), 0, st, a);
+  else if (decode_one_pass(a.Dh, a.B, a.H, a.S, a.nsplit)) hipLaunchKernelGGL((attn_decode_kernel<DT, 64, 8, true>), grid, dim3(kAttnThreads), 0, st, a);
   else hipLaunchKernelGGL((attn_decode_kernel<DT, 64, 4>), grid, dim3(kAttnThreads), 0, st, a);
 }
 

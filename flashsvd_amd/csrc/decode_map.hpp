@@ -77,6 +77,14 @@ constexpr int decode_group(int head_dim, int B, int H, int Hk, int S, int nsplit
   return decode_group_of(head_dim, pairs, rep, nsplit);
 }
 
+// One range of 129 to 256 rows of 64, one head per workgroup: 256 keys in flight instead of two passes of 128, or two workgroups that meet again in a merge.
+// us in two ranges of one pass / one range of two passes / this, 137 and 248 keys: 8 heads 5.6, 4.7, 4.4 and 5.7, 5.1, 5.2; 4 x 32 heads 6.2, 5.4, 5.1 and 6.6, 5.8,
+// 5.8; 32 x 16 8.2, 8.0, 7.4 and 10.1, 10.1, 10.2.  Not for more than 1024 (sequence, head) pairs, which had one range before: two passes need half the registers
+// and sequences of one pass are ahead there, uneven ones of up to 137 keys, two passes / this: 56 x 32 heads over 4 7.7, 10.1, 64 x 32 13.1, 14.5.
+constexpr bool decode_one_pass(int head_dim, int B, int H, int S, int nsplit) {
+  return head_dim == 64 && nsplit == 1 && S > 128 && S <= 256 && (long)B * H <= 1024;
+}
+
 // Key ranges that a sequence of n keys is cut into, at most nsplit (what the scratch holds): known from the length alone, so
 // the same launch serves a cache that is nearly empty and one that is full; the other workgroups of (b, h) leave at once.
 // A range holds at least one pass of 128 keys: one sequence of 300 keys in a cache of 4096 rows 13.0 us in 32 ranges, 6.6 in three.

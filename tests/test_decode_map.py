@@ -115,3 +115,14 @@ def test_one_range_keeps_the_group(tmp_path):
                         asserts.append(f"static_assert(decode_group({dh}, {B}, {H}, {hk}, {S}, {n}, {appends}) == {want});")
                         asserts.append(f"static_assert(decode_group({dh}, {B}, {H}, {hk}, {S}, {ranges}, {appends}) == {group(ranges)});")
     _build(tmp_path, '#include "decode_map.hpp"\nusing namespace fsvd;\n' + "\n".join(asserts) + "\nint main() { return 0; }\n")
+
+
+def test_one_pass_of_256_keys_takes_few_pairs(tmp_path):
+    """More than 1024 pairs have one range whatever the cache's length and stay with passes of 128 keys, as other cache lengths and ranges do."""
+    _build(tmp_path, """#include "decode_map.hpp"
+using namespace fsvd;
+static_assert(decode_one_pass(64, 1, 8, 129, 1) && decode_one_pass(64, 32, 32, 256, 1) && decode_one_pass(64, 1, 1024, 200, 1));
+static_assert(!decode_one_pass(64, 33, 32, 256, 1) && !decode_one_pass(64, 64, 32, 137, 1) && !decode_one_pass(64, 65536, 65536, 200, 1));
+static_assert(!decode_one_pass(64, 1, 8, 128, 1) && !decode_one_pass(64, 1, 8, 257, 1) && !decode_one_pass(64, 1, 8, 200, 2) && !decode_one_pass(128, 1, 8, 200, 1));
+int main() { return 0; }
+""")
