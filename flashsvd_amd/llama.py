@@ -303,11 +303,12 @@ class SVD_LlamaAttention(nn.Module):
         kc, vc = cache.key_cache[self.layer_idx], cache.value_cache[self.layer_idx]
         if rope is None:
             rope = cache.get_rope_tables(seqlen=cache.max_cache_len, head_dim=Dh, device=x.device, dtype=x.dtype)
-        if nsplit is None:
-            nsplit = hip_ops.pick_nsplit(cache.max_cache_len, B, H, Dh)
         from .quant import apply_linear, is_quantized
         quantized = is_quantized(*self._factor_modules())
-        if quantized or self._dense_decode_backend(cache) == "exact":
+        by_module = quantized or self._dense_decode_backend(cache) == "exact"
+        if nsplit is None:
+            nsplit = hip_ops.pick_nsplit(cache.max_cache_len, B, H, Dh, own_row=by_module and H == Hk)
+        if by_module:
             # module by module: three rank projections, three head expansions, rotary + append inside attention
             # (the only form for int4 factors, whose bytes cannot be row-packed with their neighbours')
             pk = getattr(self, "_q4_qkv_v", None) if quantized else None

@@ -69,7 +69,8 @@ def flash_attn_with_kvcache(q, k_cache, v_cache, k=None, v=None, rotary_cos=None
     if not torch.is_tensor(cache_seqlens):
         cache_seqlens = torch.full((B,), int(cache_seqlens), dtype=torch.int32, device=q.device)
     cache_seqlens = cache_seqlens.to(torch.int32).contiguous()
-    nsplit = int(num_splits) if num_splits and num_splits > 0 else hip_ops.pick_nsplit(k_cache.shape[1], B, H, Dh)
+    nsplit = int(num_splits) if num_splits and num_splits > 0 else \
+        hip_ops.pick_nsplit(k_cache.shape[1], B, H, Dh, own_row=k is not None and k_cache.shape[-2] == H)
     key = (q.device, B, H, Dh, nsplit)
     ws = _WORKSPACES.get(key)
     if ws is None:

@@ -126,3 +126,17 @@ static_assert(!decode_one_pass(64, 33, 32, 256, 1) && !decode_one_pass(64, 64, 3
 static_assert(!decode_one_pass(64, 1, 8, 128, 1) && !decode_one_pass(64, 1, 8, 257, 1) && !decode_one_pass(64, 1, 8, 200, 2) && !decode_one_pass(128, 1, 8, 200, 1));
 int main() { return 0; }
 """)
+
+
+def test_ranges_of_calls_that_append_rows_of_their_own():
+    """head_dim 128 and a kv head per head: with an appended row, a second round of workgroups that is not two thirds full keeps two ranges."""
+    from flashsvd_amd.hip_ops import pick_nsplit
+    for batch, heads in ((17, 16), (24, 16), (36, 8), (9, 32), (12, 32), (257, 1), (415, 1)):
+        assert pick_nsplit(256, batch, heads, 128, own_row=True) == 2 and pick_nsplit(256, batch, heads, 128) == 1
+        assert pick_nsplit(128, batch, heads, 128, own_row=True) == 1 and pick_nsplit(200, batch, heads, 64, own_row=True) == 1
+    for batch, heads in ((8, 32), (16, 16), (26, 16), (13, 32), (416, 1), (32, 32), (64, 32)):
+        assert pick_nsplit(256, batch, heads, 128, own_row=True) == 1
+    for batch, heads in ((1, 32), (7, 32), (255, 1)):
+        assert pick_nsplit(256, batch, heads, 128, own_row=True) == pick_nsplit(256, batch, heads, 128) == 2
+    for length in (257, 4096):
+        assert pick_nsplit(length, 9, 32, 128, own_row=True) == pick_nsplit(length, 9, 32, 128)
