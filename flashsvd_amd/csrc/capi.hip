@@ -662,30 +662,6 @@ static int block_linear(const void* x, int64_t ldx, const void* W, int64_t ldw, 
                         int64_t ldres, void* y, int64_t ldy, int B, int N, int K, int dtype, void* scratch, size_t scratch_bytes, const AheadList* next, void* stream) {
   return linear_call(x, ldx, W, ldw, bias, norm_w, eps, res, ldres, y, ldy, B, N, K, 0, dtype, scratch, scratch_bytes, next, stream);
 }
-// Weights [N, K] as a range to ask for ahead of their use: rows that lie (nearly) one behind the other, below 1 GiB.
-static Ahead weights_ahead(const void* W, int64_t ldw, int64_t N, int64_t K) {
-  Ahead a;
-  const int64_t bytes = ((N - 1) * ldw + K) * 2;
-  if (N > 0 && K > 0 && ldw >= K && ldw <= K + K / 8 && bytes < (int64_t)1 << 30) {
-    a.p = static_cast<const unsigned char*>(W);
-    a.bytes = (uint32_t)bytes;
-  }
-  return a;
-}
-// What the RMSNorm in front of a rank projection asks for on its behalf: 240 to 1536 rows that fill their tiles of 64 but for a sixteenth, up to 32 MB
-// of weights whose rows lie (nearly) one behind the other.  The tiles there take 7 of 25 us longer with weights from HBM than out of the 256 MB in front
-// of it (512 x 3072 x 4096), which deeper stages, or a wave of the workgroup that requests lines 3 to 16 steps ahead, do not change: the loads of a
-// compute unit come back in order.  us of a whole MLP (norm, rank projection, pair, down projection), without -> with, all weights from HBM:
-//   4096 x 11008 at rank 1536: 240 / 256 / 320 / 448 / 512 / 640 / 768 / 1024 / 1536 rows 95.5 -> 93.7, 97.7 -> 95.0, 101.8 -> 97.5, 117.7 -> 113.3, 128.9 -> 124.9,
-//     142.1 -> 138.3, 169.6 -> 161.5, 195.0 -> 192.3, 270.5 -> 267.1; at rank 1024 320 / 512 / 1024 rows 81.3 -> 77.0, 98.1 -> 93.6, 156.6 -> 151.0;
-//   2048 x 5504 at rank 1024: 256 / 512 / 1024 rows 52.2 -> 49.7, 67.5 -> 65.6, 91.9 -> 89.1.
-// What it leaves out: padded row tiles, which wait less (rank 1536, 257 / 333 / 350 rows 98.0 -> 98.8, 105.5 -> 105.7, 108.4 -> 108.5); fewer rows, where the norm grows by
-// what the projection gains (16 / 32 / 208 rows 47.5 -> 49.1, 57.9 -> 59.6, 89.4 -> 90.2); more rows (2048 319.5 -> 326.7); 40 MB (rank 2432, 512 / 1024 rows
-// 171.4 -> 166.4, 272 -> 277).
-static Ahead norm_ahead(const void* W, int64_t ldw, int64_t B, int64_t N, int64_t K) {
-  const Ahead a = weights_ahead(W, ldw, N, K);
-  return B >= 240 && B <= 1536 && B * 16 >= (B + 63) / 64 * 64 * 15 && a.bytes <= 32u << 20 ? a : Ahead{};
-}
 // the rank projection in front of a block: three rows and more are normalised once up front, fewer in the projection's own launch
 static int block_input(const void* x, int64_t ldx, const void* norm_w, float eps, void* xn, const void* W, int64_t ldw, void* p, int64_t ldp, int B,
                        int N, int K, int dtype, void* scratch, size_t scratch_bytes, const AheadList* next, const char* fn, void* stream) {

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "ahead.hpp"
+
 namespace fsvd {
 
 constexpr int kWave = 64;
@@ -160,16 +162,12 @@ __device__ __forceinline__ float wave_max(float v) {
   return fmaxf(fmaxf(a, b), fmaxf(c, d));
 }
 
-// Weights that the next launch reads, asked for by one that leaves the memory idle: they then come out of the 256 MB in front of HBM.
-struct Ahead { const unsigned char* p = nullptr; uint32_t bytes = 0; };
-struct AheadList { Ahead r[3]; };                      // in the order of their use
 // Workgroup `part` of `parts` reads its share of them, whole 16-byte pieces inside the range, and keeps nothing.
 template <int THREADS>
 __device__ __forceinline__ void request_ahead(const Ahead& a, int part, int parts, int tid) {
   constexpr int U = 8;                                 // loads of a thread in flight
-  const uintptr_t p = reinterpret_cast<uintptr_t>(a.p), first = (p + 15) & ~(uintptr_t)15, end = (p + a.bytes) & ~(uintptr_t)15;
-  const int n = end > first ? (int)((end - first) >> 4) : 0;
-  const u32x4_t* q = reinterpret_cast<const u32x4_t*>(first);
+  const int n = ahead_pieces(reinterpret_cast<uintptr_t>(a.p), a.bytes);
+  const u32x4_t* q = reinterpret_cast<const u32x4_t*>(ahead_first(reinterpret_cast<uintptr_t>(a.p)));
   for (int i = part * THREADS * U + tid; i < n; i += parts * THREADS * U) {
     u32x4_t v[U];
 #pragma unroll

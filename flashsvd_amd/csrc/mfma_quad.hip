@@ -6,20 +6,6 @@ namespace fsvd {
 
 static int64_t quad_tiles(const MfmaArgs& a, int tm, int tn) { return (int64_t)((a.N + 32 * tn - 1) / (32 * tn)) * ((a.B + 32 * tm - 1) / (32 * tm)); }
 
-//     form, TM, TN, stages of x and W, workgroups per compute unit, costs
-#define FSVD_QUAD_PLAIN(X) \
-  X(0, 8, 8, 2, 3, 1, 0.f, 0.f, 11.21f, 0.952f) X(1, 8, 6, 2, 3, 1, 0.f, 0.f, 8.57f, 0.783f) X(2, 4, 6, 3, 4, 1, 0.f, 0.f, 4.35f, 0.578f) \
-  X(3, 8, 4, 2, 3, 1, 0.f, 0.f, 5.97f, 0.643f) X(4, 6, 4, 3, 4, 1, 0.f, 0.f, 4.84f, 0.502f) X(5, 4, 4, 2, 3, 2, 1.53f, 0.533f, 8.67f, 0.679f) \
-  X(6, 4, 4, 4, 5, 1, 0.f, 0.f, 3.03f, 0.450f) X(7, 4, 3, 5, 6, 1, 0.f, 0.f, 4.29f, 0.353f) X(8, 4, 2, 3, 4, 2, 0.57f, 0.339f, 3.94f, 0.568f) \
-  X(9, 2, 4, 3, 4, 1, 0.f, 0.f, 1.24f, 0.354f) X(10, 3, 2, 3, 4, 2, 0.24f, 0.297f, 3.14f, 0.440f) X(11, 2, 3, 3, 4, 2, 0.30f, 0.311f, 1.99f, 0.484f) \
-  X(12, 2, 2, 5, 5, 2, 0.49f, 0.227f, 2.66f, 0.355f)
-constexpr bool quad_halves(int n) { return n >= 8 && n != 9; }      // the forms that shapes with K halved get, with registers for a second set of accumulators
-constexpr QuadCost kPlainCosts[] = {
-#define X(n, TM, TN, SX, SW, OCC, F1, S1, F2, S2) QuadCost{F1, S1, F2, S2},
-  FSVD_QUAD_PLAIN(X)
-#undef X
-};
-constexpr QuadCost kCost256x128Shares{0.f, 0.f, 6.65f, 0.634f};     // three stages of both operands, in shares only
 constexpr float kLaunchUs = 3.f, kShareSumUs = 3.5f, kShareBytesPerUs = 4.5e6f;      // of a launch; of the one that adds the shares, beside their way out and in
 static float share_sum_us(int64_t floats) { return kShareSumUs + (float)floats * 8.f / kShareBytesPerUs; }
 #define FSVD_QUAD_PAIR(X) \

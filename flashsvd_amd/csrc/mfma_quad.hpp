@@ -29,6 +29,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "quad_costs.hpp"
 
 namespace fsvd {
 
@@ -55,43 +56,11 @@ __device__ __forceinline__ void quad_swap_rows(uint32_t& a, uint32_t& b) {
 // four elements at any element's address
 typedef uint32_t u32x2_any_t __attribute__((ext_vector_type(2), aligned(2)));
 
-// What a round of workgroups costs in a form, us: f + s per K step of 64; 1: the compute units hold one workgroup each (or fewer), 2: as many
-// as fit.  Fitted to launches with weights from HBM (more of them in turn than the 256 MB in front of it hold) over 125 / 49 / 39 shapes
-// (154 to 16384 rows; 1024 to 4096 columns at K 768 to 4096; the pair 5504 x 768 to 11008 x 2432; 48 and 96 heads at rank 512 and 1024):
-// the form that they name is on average 2 / 1 / 1 % (at worst 20, 12, 8 %) behind the best of about 30 tilings.  The largest launches take longer than
-// they say, whatever the tile (the pair 16384 x 11008 x 2432 1605 us, 1426 by them).
-struct QuadCost { float f1, s1, f2, s2; };
-static float quad_us(const QuadCost& c, int64_t tiles, int occ, float steps, int64_t cu) {
-  const int64_t full = tiles / (cu * occ), rest = tiles - full * cu * occ;
-  float us = (float)full * (c.f2 + c.s2 * steps);
-  if (rest > 0) us += occ == 2 && rest <= cu ? c.f1 + c.s1 * steps : c.f2 + c.s2 * steps;
-  return us;
-}
-
-// Workgroups for the compute units that a launch of `wgs` with `rows` rows in its row tiles leaves idle, and what they ask for: the ranges of
-// q.a[0].next, in their order, that they get through at 46 bytes per ns and compute unit while the launch is expected to last, padded row tiles
-// counted out (128 x 192 tiles over 400 rows end early: with down_v asked for all the same the MLP at rank 2432 went from 146 to 152 us).  A range in part gains
-// nothing, its launch takes as long as its slowest workgroups (ranges cut off at 15, 25, 40 bytes per ns: a prompt of 512 tokens 7027 -> 7014, 7010, 6880 us).
-// A compute unit reads about 60 from HBM; more than 46 outlasts some launches (54: rank 1024, 384 rows 83.7 -> 88.4, rank 2432, 512 rows 171 -> 177).
-// What it gives, us without -> with, weights from HBM: the pair 512 x 11008 x 1536 leaves 24 compute units to down_v, whose launches then take 26 instead of 36.  MLPs of 4096
-// x 11008 at rank 1536, 64 / 128 / 154 / 256 / 333 / 400 / 512 / 640 / 768 rows 80.8 -> 77.8, 75.8 -> 73.1, 79.0 -> 78.8, 94.2 -> 90.4, 106.7 -> 104.8, 110.4 -> 110.7, 124.5 -> 117.3, 139.3
-// -> 131.2, 162.8 -> 161.0, at rank 1492 384 / 768 rows 131.6 -> 125.5, 210.7 -> 191.1, 2048 x 5504 at rank 1024 192 / 300 / 400 / 700 rows 54.5 -> 48.1, 57.1 -> 52.5, 64.5 -> 64.4, 78.4
-// -> 72.1; over 100 of these (64 to 768 rows, rank 1024 to 2432) 0.977 of the time.  More tiles than compute units: nobody is idle, nothing is asked for.
-// The tiles of many rows are left out.
-constexpr float kAheadRate = 46.f;
-constexpr bool quad_asks(int tm, int tn) { return tm * tn < 32; }
+constexpr bool quad_asks(int tm, int tn) { return tm * tn < 32; }      // the tiles of many rows are left out
 static int quad_ahead(QuadArgs& q, int64_t wgs, int64_t rows) {
-  q.next = AheadList{};
-  const int64_t idle = compute_units() - wgs;
-  if (q.a[0].next == nullptr || idle <= 0) return 0;
-  const int64_t room = (int64_t)(q.us * kAheadRate * 1000.f * (float)q.a[0].B / (float)rows) * idle;
-  int64_t sum = 0;
-  for (int i = 0; i < 3; ++i) {
-    if (sum + q.a[0].next->r[i].bytes > room) break;
-    q.next.r[i] = q.a[0].next->r[i];
-    sum += q.next.r[i].bytes;
-  }
-  return (int)std::min<int64_t>(idle, (sum + 32767) / 32768);
+  const AheadChoice c = ahead_choice(q.a[0].next, q.us, q.a[0].B, rows, compute_units() - wgs);
+  q.next = c.ranges;
+  return c.workgroups;
 }
 
 constexpr bool quad_stream(int tm, int tn) { return tm * tn >= 24; }

@@ -107,3 +107,10 @@ def test_dual_split_operator_takes_rows_of_any_stride():
         pu, pg = base.as_strided((T, R), (size, 1), start), base.flip(0).as_strided((T, R), (size, 1), start)
         got, want = (registered.mlp_dual_split(u, g, *w, None, 2, 64, True, None) for u, g in ((pu, pg), (pu.clone(memory_format=torch.contiguous_format), pg.clone(memory_format=torch.contiguous_format))))
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,T,start,H,Hk,R", [(1, 17, 0, 4, 4, 320), (2, 77, 131, 8, 2, 384), (1, 333, 7, 4, 4, 330), (1, 128, 0, 32, 8, 320), (1, 257, 3, 8, 8, 576)])
+def test_attention_block_of_large_ranks(B, T, start, H, Hk, R, dtype):
+    """Ranks whose head expansions run on few four-wave tiles: the compute units that these leave idle read o_v and o_u."""
+    test_attention_block(B, T, start, H, Hk, R, dtype)
