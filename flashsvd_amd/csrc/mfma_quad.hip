@@ -126,8 +126,7 @@ static ShareForm filling_shares(const MfmaArgs& a, const RingRule& ring) {
   // the sums once out and once in, and the launch that adds them; 333 x 1664 x 4096 19.7 us in shares, 16.1 unsplit (here too a K below 5120 only:
   // the longer ones were ahead in shares at every row count)
   if (a.K < 5120) {
-    const QuadCost c = bm == 64 ? kPlainCosts[9] : (bm == 128 ? kPlainCosts[6] : kCost256x128Shares);
-    const float us = c.f2 + c.s2 * (float)per + share_sum_us(shares * tiles * area);
+    const float us = share_us(bm, 128, shares * tiles, per, cu) + share_sum_us(shares * tiles * area);
     if (kLaunchUs + quad_pick(a, false, false).us < 0.9f * (kLaunchUs + us)) return none;
   }
   return ShareForm{bm, 128, (int)shares, per};
@@ -154,7 +153,7 @@ static ShareForm share_form(const MfmaArgs& a) {
   const QuadSums sums = quad_sums(a);
   if (sums.order != kOrderCut) return none;
   const int64_t tiles = quad_tiles(a, 2, 2), shares = (steps + sums.per - 1) / sums.per;
-  const float apart = quad_us(kPlainCosts[12], tiles * shares, 2, (float)sums.per, cu) + share_sum_us(shares * tiles * 4096);
+  const float apart = share_us(64, 64, tiles * shares, sums.per, cu) + share_sum_us(shares * tiles * 4096);
   return apart < 1.1f * quad_us(kPlainCosts[12], tiles, 2, (float)steps, cu) && (size_t)(tiles * shares * 4096) <= a.scratch_floats ? ShareForm{64, 64, (int)shares, sums.per} : none;
 }
 // floats of scratch that the call can use, out of at most `cap`
@@ -325,8 +324,7 @@ static int launch_gemm_quad_dt(const MfmaArgs& a, bool dual, hipStream_t st, con
       q.shares = f.shares;
       q.per = f.per;
       q.part = a.scratch;
-      const QuadCost& c = f.bn == 64 ? kPlainCosts[12] : (f.bm == 64 ? kPlainCosts[9] : (f.bm == 128 ? kPlainCosts[6] : kCost256x128Shares));
-      q.us = c.f2 + c.s2 * (float)f.per;
+      q.us = share_us(f.bm, f.bn, quad_tiles(a, f.bm / 32, f.bn / 32) * f.shares, f.per, compute_units());
       return launch_share_dt<DT>(q, f, st, who);
     }
   }

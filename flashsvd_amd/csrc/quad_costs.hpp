@@ -31,5 +31,11 @@ constexpr QuadCost kPlainCosts[] = {
 #undef X
 };
 constexpr QuadCost kCost256x128Shares{0.f, 0.f, 6.65f, 0.634f};     // three stages of both operands, in shares only
+// A launch of `wgs` workgroups that take `per` K steps of a tile each, in shares; tiles of 64 x 64 fit twice on a compute unit and then, as elsewhere, take f1 and s1
+// where there are no more of them than compute units (16 steps 4.1 us, and 8.3 for two of them).
+constexpr const QuadCost& share_cost(int bm, int bn) {
+  return bn == 64 ? kPlainCosts[12] : (bm == 64 ? kPlainCosts[9] : (bm == 128 ? kPlainCosts[6] : kCost256x128Shares));
+}
+constexpr float share_us(int bm, int bn, int64_t wgs, int per, int64_t cu) { return quad_us(share_cost(bm, bn), wgs, bn == 64 ? 2 : 1, (float)per, cu); }
 
 }  // namespace fsvd

@@ -87,3 +87,18 @@ def test_whole_ranges_that_fit_into_the_launch(tmp_path):
   const AheadList hole = list(0, 32768, 32769);
   CHECK(ahead_choice(&hole, 10.f, 64, 64, 190).workgroups == 3 && took(ahead_choice(&hole, 10.f, 64, 64, 190)) == 6);
 """)
+
+
+def test_time_of_a_launch_in_shares(tmp_path):
+    """Tiles of 64 x 64 take the time of one per compute unit where there are no more of them; the other tiles are one per compute unit in any case."""
+    _run(tmp_path, r"""
+  CHECK(share_us(64, 64, 200, 16, 256) == kPlainCosts[12].f1 + kPlainCosts[12].s1 * 16 && share_us(64, 64, 256, 16, 256) == share_us(64, 64, 1, 16, 256));
+  CHECK(share_us(64, 64, 257, 16, 256) == kPlainCosts[12].f2 + kPlainCosts[12].s2 * 16 && share_us(64, 64, 512, 16, 256) == share_us(64, 64, 257, 16, 256));
+  for (int wgs : {1, 200, 256}) {
+    CHECK(share_us(64, 128, wgs, 12, 256) == kPlainCosts[9].f2 + kPlainCosts[9].s2 * 12 && share_us(128, 128, wgs, 12, 256) == kPlainCosts[6].f2 + kPlainCosts[6].s2 * 12);
+    CHECK(share_us(256, 128, wgs, 12, 256) == kCost256x128Shares.f2 + kCost256x128Shares.s2 * 12);
+  }
+  // 200 workgroups of 16 steps: 56 idle units get through 46 bytes per ns for 4.1 us, not for the 8.3 of two tiles on a unit
+  const AheadList l = list(12000000, 0, 0);
+  CHECK(ahead_choice(&l, share_us(64, 64, 200, 16, 256), 64, 64, 56).workgroups == 0 && ahead_choice(&l, share_us(64, 64, 257, 16, 256), 64, 64, 56).workgroups == 56);
+""")
