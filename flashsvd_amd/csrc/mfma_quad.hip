@@ -35,7 +35,7 @@ static QuadSums quad_sums(const MfmaArgs& a) {
   return per > 0 ? QuadSums{kOrderCut, per} : QuadSums{kOrderPlain, 0};
 }
 static QuadPick quad_pick(const MfmaArgs& a, bool dual, bool any, QuadOrder order = kOrderPlain) {
-  if (order == kOrderCut) return QuadPick{12, 0.f};                                  // few 64 x 64 tiles by that rule
+  if (order == kOrderCut) return QuadPick{12, ranges_us(quad_tiles(a, 2, 2), a.K, compute_units())};       // few 64 x 64 tiles by that rule
   QuadPick best{kQuadNone, 0.f};
   const float steps = (float)((a.K + 63) / 64 * (dual ? 2 : 1));
   const int64_t cu = compute_units();                // asked once: a small model's call is bound by what the host does per launch
@@ -154,7 +154,7 @@ static ShareForm share_form(const MfmaArgs& a) {
   if (sums.order != kOrderCut) return none;
   const int64_t tiles = quad_tiles(a, 2, 2), shares = (steps + sums.per - 1) / sums.per;
   const float apart = share_us(64, 64, tiles * shares, sums.per, cu) + share_sum_us(shares * tiles * 4096);
-  return apart < 1.1f * quad_us(kPlainCosts[12], tiles, 2, (float)steps, cu) && (size_t)(tiles * shares * 4096) <= a.scratch_floats ? ShareForm{64, 64, (int)shares, sums.per} : none;
+  return apart < 1.1f * ranges_us(tiles, a.K, cu) && (size_t)(tiles * shares * 4096) <= a.scratch_floats ? ShareForm{64, 64, (int)shares, sums.per} : none;
 }
 // floats of scratch that the call can use, out of at most `cap`
 size_t gemm_share_floats(MfmaArgs a, size_t cap) {

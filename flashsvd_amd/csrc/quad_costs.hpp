@@ -37,5 +37,7 @@ constexpr const QuadCost& share_cost(int bm, int bn) {
   return bn == 64 ? kPlainCosts[12] : (bm == 64 ? kPlainCosts[9] : (bm == 128 ? kPlainCosts[6] : kCost256x128Shares));
 }
 constexpr float share_us(int bm, int bn, int64_t wgs, int per, int64_t cu) { return quad_us(share_cost(bm, bn), wgs, bn == 64 ? 2 : 1, (float)per, cu); }
+// The same tiles with K in ranges one after the other (kOrderCut of mfma_quad.hip): the walk of one tile, whatever the ranges.
+constexpr float ranges_us(int64_t tiles, int K, int64_t cu) { return quad_us(kPlainCosts[12], tiles, 2, (float)((K + 63) / 64), cu); }
 
 }  // namespace fsvd

@@ -102,3 +102,12 @@ def test_time_of_a_launch_in_shares(tmp_path):
   const AheadList l = list(12000000, 0, 0);
   CHECK(ahead_choice(&l, share_us(64, 64, 200, 16, 256), 64, 64, 56).workgroups == 0 && ahead_choice(&l, share_us(64, 64, 257, 16, 256), 64, 64, 56).workgroups == 56);
 """)
+
+
+def test_tiles_with_k_in_ranges_ask(tmp_path):
+    """A launch whose tiles walk the ranges of K one after the other lasts that long and leaves most compute units idle: 333 x 704 x 3072, 66 tiles."""
+    _run(tmp_path, r"""
+  CHECK(ranges_us(66, 3072, 256) == kPlainCosts[12].f1 + kPlainCosts[12].s1 * 48 && ranges_us(300, 3072, 256) == kPlainCosts[12].f2 + kPlainCosts[12].s2 * 48);
+  const AheadList l = list(67000000, 33000000, 0);
+  CHECK(ahead_choice(&l, ranges_us(66, 3072, 256), 333, 384, 190).workgroups == 190 && ahead_choice(&l, ranges_us(66, 3072, 256), 333, 384, 190).ranges.r[1].bytes == 0);
+""")
