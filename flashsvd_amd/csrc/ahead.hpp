@@ -47,12 +47,17 @@ inline Ahead norm_ahead(const void* W, int64_t ldw, int64_t B, int64_t N, int64_
 // order, that they get through at 46 bytes per ns and compute unit while the launch is expected to last, the padding of its row tiles (`rows` in
 // `tile_rows`) counted out (128 x 192 tiles over 400 rows end early: with down_v asked for all the same the MLP at rank 2432 went from 146 to 152 us).  A range in part gains
 // nothing, its launch takes as long as its slowest workgroups (ranges cut off at 15, 25, 40 bytes per ns: a prompt of 512 tokens 7027 -> 7014, 7010, 6880 us).
-// A compute unit reads about 60 from HBM; more than 46 outlasts some launches (54: rank 1024, 384 rows 83.7 -> 88.4, rank 2432, 512 rows 171 -> 177).
-// What it gives, us without -> with, weights from HBM: the pair 512 x 11008 x 1536 leaves 24 compute units to down_v, whose launches then take 26 instead of 36.  MLPs of 4096
-// x 11008 at rank 1536, 64 / 128 / 154 / 256 / 333 / 400 / 512 / 640 / 768 rows 80.8 -> 77.8, 75.8 -> 73.1, 79.0 -> 78.8, 94.2 -> 90.4, 106.7 -> 104.8, 110.4 -> 110.7, 124.5 -> 117.3, 139.3
-// -> 131.2, 162.8 -> 161.0, at rank 1492 384 / 768 rows 131.6 -> 125.5, 210.7 -> 191.1, 2048 x 5504 at rank 1024 192 / 300 / 400 / 700 rows 54.5 -> 48.1, 57.1 -> 52.5, 64.5 -> 64.4, 78.4
-// -> 72.1; over 100 of these (64 to 768 rows, rank 1024 to 2432) 0.977 of the time.  More tiles than compute units: nobody is idle, nothing is asked for.
-// The tiles of many rows are left out.
+// A compute unit reads about 60 from HBM; more than 46 outlasts some launches (54: rank 1024, 384 rows 83.7 -> 88.4, rank 2432, 512 rows 171 -> 177), less
+// takes fewer ranges: 46 / 40 / 34 took 0.968, 0.970, 0.977 of the time without over 114 MLPs of 64 to 768 rows (4096 x 11008 at rank 1024, 1492, 1536, 2432, 2048 x 5504 at 704
+// and 1024) and 0.978, 0.980, 0.982 over 65 attention halves of 40 to 1024 rows (rank 512 to 1664, 16 and 32 heads over 8 to 32), weights from HBM.
+// us without -> with: the pair 512 x 11008 x 1536 leaves 24 compute units to down_v, whose launches then take 26 instead of 36.  MLPs of 4096 x 11008 at rank 1536, 64 / 128
+// / 154 / 256 / 333 / 384 / 400 / 512 / 640 / 700 / 768 rows 81.0 -> 77.8, 75.1 -> 73.1, 79.7 -> 79.0, 94.5 -> 90.3, 106.2 -> 105.7, 113.5 -> 107.9, 110.4 -> 110.3, 125.8 -> 116.9, 138.9 ->
+// 131.6, 156.5 -> 151.8, 166.5 -> 158.7, at rank 1492 384 / 768 rows 133.5 -> 126.2, 214.3 -> 191.1, 2048 x 5504 at rank 1024 192 / 300 / 400 / 700 rows 54.3 -> 48.2, 56.9 -> 51.9, 64.5 ->
+// 64.3, 78.8 -> 71.9; attention halves of 32 heads at rank 1024, 128 / 256 / 333 / 512 rows 56.8 -> 55.7, 67.2 -> 64.3, 81.5 -> 80.9, 93.5 -> 93.6, at rank 1664 512 rows 126.7 -> 119.0.
+// What loses: an MLP at rank 2432, 200 rows 117.2 -> 118.7, 2048 x 5504 at rank 1024, 64 rows 48.0 -> 48.4, attention of 32 heads at rank 1024, 200 rows 62.4 -> 62.8, at
+// rank 704, 700 rows 103.4 -> 105.0; the others are within 0.7 % of it or ahead.  Launches whose tiles walk K in ranges (ranges_us in quad_costs.hpp) are the idlest: MLPs of 3072 x
+// 8192 at rank 1152 / 704 / 512, 192 / 320 / 320 rows, whose rank projection asks for nothing -> asks as well, 63.7 -> 60.0, 57.6 -> 54.9, 51.1 -> 49.3.
+// More tiles than compute units: nobody is idle, nothing is asked for.
 constexpr float kAheadRate = 46.f;
 struct AheadChoice { AheadList ranges; int workgroups; };
 inline AheadChoice ahead_choice(const AheadList* next, float us, int64_t rows, int64_t tile_rows, int64_t idle) {

@@ -558,7 +558,7 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_kernel(const uint16_t* __res
 // the same with 16-byte accesses and the row kept in registers between the two passes (K a multiple of 8, at most
 // 8 * NC * kThreads, rows 16-byte aligned): a prompt of 512 rows x 4096 took 9.9 us with 2-byte accesses.  The launch is its
 // own start, two round trips and a reduction, and HBM has next to nothing to do meanwhile: workgroups behind those of the rows ask for the
-// weights of the projection that follows (see norm_ahead in capi.hip).
+// weights of the projection that follows (see norm_ahead in ahead.hpp).
 template <int DT, int NC>
 __global__ __launch_bounds__(kThreads) void rmsnorm_vec_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                               const uint16_t* __restrict__ w, float eps,
