@@ -397,7 +397,7 @@ def pick_nsplit(max_len: int, batch: int, heads: int, head_dim: int = 128, own_r
     batch*heads*nsplit stays within ~2048 workgroups.  Up to 256 rows in one range, which saves the merge, with head_dim 64 (8 heads,
     137 keys 5.6 -> 4.4 us) and for 256 pairs and more (16 x 32 heads over 8 of 128 9.4 -> 8.0; fewer lose: 32 heads, 250 keys 6.4 -> 6.7).
     ``own_row``: every head has a kv head of its own and the call appends its row.  The rows are then read behind the write's way to
-    memory, and a second round of workgroups that is not two thirds full waits for that once more: two ranges there (17 / 20 / 24 x 16 heads of up to 248 keys 10.1,
+    memory, and a second round of workgroups that is less than five eighths full waits for that once more: two ranges there (17 / 20 / 24 x 16 heads of up to 248 keys 10.1,
     10.9, 11.4 in two, 11.2, 11.7, 12.1 in one; 26 x 16 12.0 and 10.9).  It goes by the room in the cache: how many keys there are is not known here."""
     pairs = batch * heads
     if max_len <= 256 and (head_dim < 128 or (pairs >= 256 and not (own_row and 256 < pairs < 416))):

@@ -129,7 +129,7 @@ int main() { return 0; }
 
 
 def test_ranges_of_calls_that_append_rows_of_their_own():
-    """head_dim 128 and a kv head per head: with an appended row, a second round of workgroups that is not two thirds full keeps two ranges."""
+    """head_dim 128 and a kv head per head: with an appended row, a second round of workgroups that is less than five eighths full keeps two ranges."""
     from flashsvd_amd.hip_ops import pick_nsplit
     for batch, heads in ((17, 16), (24, 16), (36, 8), (9, 32), (12, 32), (257, 1), (415, 1)):
         assert pick_nsplit(256, batch, heads, 128, own_row=True) == 2 and pick_nsplit(256, batch, heads, 128) == 1
